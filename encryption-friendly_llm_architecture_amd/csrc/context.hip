@@ -124,10 +124,10 @@ hemm_context *hemm_context_build(int logN, int nQ, int nP, const u64 *primes, in
             ipw[j] = h_mulmod(ipw[j - 1], ipsi, q);
         }
         u64 *wt = w.data() + (size_t)i * N * 2, *iwt = iw.data() + (size_t)i * N * 2;
-        // Primes below 2^44 run the 2^16-point transform in double precision (exact: see ntt.hip); their
+        // Primes below 2^44 run the register-blocked transforms in double precision (exact: see ntt.hip); their
         // table is the N twiddles as doubles, packed into the first half of the prime's region (8 bytes per twiddle
         // instead of 16: the row passes read as many twiddle bytes as data, and the quotient w / q costs one multiply).
-        const bool fp = (logN == 16) && (q >> 44) == 0;
+        const bool fp = ring_has_fused_forms(c) && (q >> 44) == 0;
         auto as_bits = [](double d) {
             u64 b;
             memcpy(&b, &d, 8);
@@ -177,20 +177,21 @@ hemm_context *hemm_context_build(int logN, int nQ, int nP, const u64 *primes, in
     c->d_w = (u64 *)up(w.data(), w.size() * 8);
     c->d_iw = (u64 *)up(iw.data(), iw.size() * 8);
     c->d_rw = c->d_irw = nullptr;
-    if (logN == 16) {
+    if (ring_has_fused_forms(c)) {
         // per prime the same storage convention as the stage-ordered tables: 16-byte entries, or doubles packed into
         // the first half of the prime's region
+        const u32 R = (u32)N / 256;
         std::vector<u64> rw((size_t)T * N * 2, 0), irw((size_t)T * N * 2, 0);
         for (int i = 0; i < T; i++) {
             const bool fp = fpc[4 * i] != 0.0;
             const u64 *src[2] = {w.data() + (size_t)i * N * 2, iw.data() + (size_t)i * N * 2};
             u64 *dst[2] = {rw.data() + (size_t)i * N * 2, irw.data() + (size_t)i * N * 2};
             for (int dir = 0; dir < 2; dir++)
-                for (u32 r = 0; r < 256; r++)
+                for (u32 r = 0; r < R; r++)
                     for (u32 l = 0; l < 4; l++)
                         for (u32 g = 0; g < (1u << l); g++)
                             for (u32 cc = 0; cc < 16; cc++) {
-                                const size_t from = ((size_t)(16 * (256 + r) + cc) << l) + g;
+                                const size_t from = ((size_t)(16 * (R + r) + cc) << l) + g;
                                 const size_t to = ((size_t)r * 15 + (1u << l) - 1 + g) * 16 + cc;
                                 if (fp) {
                                     dst[dir][to] = src[dir][from];

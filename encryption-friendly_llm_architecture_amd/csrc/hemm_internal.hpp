@@ -26,9 +26,9 @@ struct hemm_context {
     std::vector<ModQ> modq;         // host copy
     // device tables, all [prime][N] unless noted
     u64 *d_w, *d_iw;                // (psi^bitrev(i), Shoup quotient), forward and inverse transform
-    u64 *d_rw, *d_irw;              // N = 2^16: the twiddles of the row passes' inner radix-16 blocks in the order their
+    u64 *d_rw, *d_irw;              // N >= 2^10: the twiddles of the row passes' inner radix-16 blocks in the order their
                                     // threads read them, entry (r * 15 + 2^l - 1 + g) * 16 + c = entry
-                                    // ((16 (256 + r) + c) << l) + g of d_w / d_iw (nullptr for other ring sizes)
+                                    // ((16 (N / 256 + r) + c) << l) + g of d_w / d_iw (nullptr for other ring sizes)
     u64 *d_ninv, *d_ninv_s;         // [prime]
     ModQ *d_modq;                   // [prime]
     double *d_fp;                   // [prime][4]: q, 1/q, 1/N mod q, that / q as doubles; q = 0 marks a prime of
@@ -63,6 +63,19 @@ inline void account(const hemm_context *c, int kind, size_t bytes, int n_launche
     m->launches[kind] += (unsigned long long)n_launches;
 }
 
+// Rings of 2^10 points and more run the register-blocked transforms, whose passes can begin in a basis conversion, end in
+// a subtraction and a constant, and read through an automorphism (primes below 2^44 in double precision, twiddle tables
+// laid out for it).
+inline bool ring_has_fused_forms(const hemm_context *c) { return c->logN >= 10; }
+// Whether a transform is one launch with a workgroup per limb: up to 2^12 points always.  A larger limb is slower in one
+// workgroup than spread over several in two launches (2^13 points: 11.5 against 11.0 us for one limb, 12.4 against 13.2
+// for 96; 2^14: 21 against 18.5 us for 64), until the limbs alone fill the CUs and the second trip through memory is what
+// counts (60-bit primes: 34.6 against 47.2 us for 768 limbs of 2^13; 2^14: 23 against 28 us for 128, 81 against 87 for 768).
+// plain: no conversion, tail or automorphism -- with them a workgroup of the 1024 threads a limb of 2^14 takes would spill.
+inline bool one_launch(const hemm_context *c, size_t limbs, bool plain) {
+    return c->logN >= 10 && (c->logN <= 12 || (c->logN == 13 && limbs >= 64) || (c->logN == 14 && plain && limbs >= 96));
+}
+
 // a constant and its Shoup quotient floor(w * 2^64 / q)
 struct __align__(16) Cst {
     u64 w, ws;
@@ -93,12 +106,12 @@ LimbList limbs_default(const hemm_context *c, int nq, int with_p);
 
 // kernel launchers (defined in the .hip files)
 // final_scale (device, one (constant, Shoup quotient) pair per limb of the launch, or nullptr): an inverse transform
-// of N = 2^16 ends with that constant in place of 1/N
+// of N >= 2^10 ends with that constant in place of 1/N
 void launch_ntt_slots(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs,
                       int n_polys, size_t poly_stride, bool inverse, hipStream_t s, const void *final_scale = nullptr);
 bool launch_ntt_sub_scale(const hemm_context *c, u64 *data, int n_limbs, int n_polys, const u64 *minuend,
                           size_t minuend_stride, u64 *out, size_t out_stride, const void *cst_dev, hipStream_t s);
-// A forward transform of N = 2^16 whose input is a fast basis conversion: limb l of the launch is the conversion of
+// A forward transform of N >= 2^10 whose input is a fast basis conversion: limb l of the launch is the conversion of
 // the coefficient-form sources of digit digit_of[l] (already carrying their (S/q_i)^-1 factors) to prime ll[l],
 // computed while the first pass loads its slab instead of being written by a conversion launch and read back.
 #define CONV_MAX_DIGITS 4
@@ -118,7 +131,7 @@ struct ConvSources {
     const u64 *copy_src;
     size_t copy_src_stride;
     int n_copy;
-    u32 copy_galois;            // != 0: the copies read their source through this automorphism (N = 2^16)
+    u32 copy_galois;            // != 0: the copies read their source through this automorphism
     uint8_t copy_src_slot[HEMM_MAX_PRIMES], copy_dst_slot[HEMM_MAX_PRIMES];
 };
 // data: [n_polys][.][N] (polynomial stride poly_stride), limb l written to slot sl[l].  With ep_* set the second pass
@@ -128,6 +141,14 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
                           int n_limbs, int n_polys, size_t poly_stride, hipStream_t s, const u64 *ep_minuend = nullptr,
                           size_t ep_minuend_stride = 0, u64 *ep_out = nullptr, size_t ep_out_stride = 0,
                           const void *ep_cst_dev = nullptr);
+// One-launch transforms (2^10 .. 2^14 points).  cs != nullptr: the inputs are its conversions; out != nullptr: out =
+// (minuend - transform) * cst[limb]; from != nullptr: the inverse reads there instead of data, through `galois` if != 0.
+void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
+                         size_t poly_stride, hipStream_t s, const ConvSources *cs, const u64 *minuend, size_t minuend_stride,
+                         u64 *out, size_t out_stride, const void *cst_dev);
+void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
+                         size_t poly_stride, hipStream_t s, const void *final_scale, const u64 *from, size_t from_stride,
+                         u32 galois);
 // out[p][j] = (y[p][j] - conversion of the n_src listed limbs of y[p] to prime j) * cst[j], j < nq_out, as inverse row
 // pass (in place on the listed limbs), one column-slab kernel (second inverse pass, conversion as lazy dot products, first
 // forward pass into conv[n_polys][nq_out][N]) and forward row pass with the fused tail.  final_scale / hat / cst: device
@@ -171,7 +192,7 @@ void launch_inner_product(hemm_context *c, const u64 *in, const u64 *ext, const 
                           hipStream_t s);
 void launch_moddown(hemm_context *c, u64 *acc, int nq, int n_polys, u64 *out, size_t out_stride, const u64 *add,
                     size_t add_stride, int add_polys, u64 *conv, hipStream_t s);
-// galois != 0 (N = 2^16): the key switch of the automorphism of `in`, which is read through it where the ModUp reads
+// galois != 0 (N >= 2^10): the key switch of the automorphism of `in`, which is read through it where the ModUp reads
 // it; b_rotates: add_b is read through the same automorphism where the key product adds it; add_a (N >= 512, with
 // add_b): out[1] = ks_a + add_a as well, both addends entering the sum in the extended basis
 void launch_keyswitch(hemm_context *c, const u64 *in, const u64 *evk, int nq, u64 *out, size_t out_stride,

@@ -582,7 +582,7 @@ struct KsTables {
     std::vector<std::vector<Cst>> dropinv;               // [nq][j<nq-1]  (P q_{nq-1})^-1 mod q_j
     size_t pinv_off = 0;                                 // device copies of pinv / dropinv[nq] / qlinv[l]
     std::vector<size_t> dropinv_off, qlinv_off;
-    // (1/N) (S/q_i)^-1 mod q_i in source order: the constant an inverse transform of N = 2^16 ends with when a basis
+    // (1/N) (S/q_i)^-1 mod q_i in source order: the constant an inverse transform of N >= 2^10 ends with when a basis
     // conversion follows it.  modup: per chain length nq, limbs 0 .. nq-1 (each limb in its own digit's basis).
     size_t p_invn_off = 0;
     std::vector<size_t> drop_invn_off, modup_invn_off;   // [nq]
@@ -927,7 +927,7 @@ static void rescale_with(hemm_context *c, KsTables *t, u64 *sc, const u64 *in, s
                                     hipMemcpyDeviceToDevice, s));
         launch_ntt(c, last, pl, 1, n_polys, N, true, s);
     }
-    if (c->logN == 16 && lazy_dot_ok(c)) {
+    if (ring_has_fused_forms(c) && lazy_dot_ok(c)) {
         // the reduction of the last limb's coefficients into every remaining prime is a one-source conversion with
         // the constant 1: computed inside the first pass of the forward transform
         ConvSources cs;
@@ -1081,7 +1081,7 @@ void launch_key_expand(const hemm_context *c, const u64 *compact, u64 *evk, hipS
 // launch (the first pass of the forward transform) is the one that can read its input through an automorphism.
 bool modup_through_automorphism_ok(const hemm_context *c, int nq) {
     const int K = c->nP, E = nq + K, alpha = c->alpha, beta = (nq + alpha - 1) / alpha;
-    return c->logN == 16 && alpha <= 8 && alpha <= CONV_MAX_SOURCES && beta <= BCONV_MAX_DIGITS &&
+    return ring_has_fused_forms(c) && alpha <= 8 && alpha <= CONV_MAX_SOURCES && beta <= BCONV_MAX_DIGITS &&
            beta <= CONV_MAX_DIGITS && beta * E <= 255 && beta * E - nq <= HEMM_MAX_PRIMES && lazy_dot_ok(c);
 }
 
@@ -1094,7 +1094,7 @@ void launch_modup_batch(hemm_context *c, const u64 *in, size_t in_stride, int nq
     const LimbList chain = limbs_default(c, nq, 0);
     LimbList ident;
     for (int j = 0; j < HEMM_MAX_PRIMES; j++) ident.idx[j] = (uint8_t)j;
-    const bool fold = c->logN == 16;
+    const bool fold = ring_has_fused_forms(c);
     if (galois != 0 && !modup_through_automorphism_ok(c, nq))
         throw std::invalid_argument("this ModUp shape has no form that reads its input through an automorphism");
     if (!launch_intt_from(c, in, in_stride, coef, chain, ident, nq, n_in, (size_t)nq * N, s,
@@ -1391,10 +1391,10 @@ void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop
         pl.idx[i] = a.src_prime[i];
         sl.idx[i] = a.src_slot[i];
     }
-    const bool fold = c->logN == 16;   // the inverse transform ends with (1/N)(S/q_i)^-1: no scaling pass in the conversion
+    const bool fold = ring_has_fused_forms(c);   // the inverse transform ends with (1/N)(S/q_i)^-1: no scaling pass in the conversion
     // the three-launch form with one column-slab kernel in the middle, only on request: it moves a fifth less data but
     // runs at two waves per SIMD and is slower on every batch size measured
-    if (slab && !(fold && lazy_dot_ok(c))) throw std::invalid_argument("the column-slab ModDown needs N = 2^16 and primes below 2^60");
+    if (slab && !(c->logN == 16 && lazy_dot_ok(c))) throw std::invalid_argument("the column-slab ModDown needs N = 2^16 and primes below 2^60");
     if (slab) {
         if (!launch_moddown_slab(c, y, (size_t)E * N, a.src_slot, a.src_prime, ns,
                             t->dev + (drop_last ? t->drop_invn_off[nq] : t->p_invn_off),

@@ -1,0 +1,396 @@
+// Device-side pieces shared by the transform kernels: butterflies, the two arithmetic back ends, register blocks of up
+// to four stages, and the row pass.
+#pragma once
+#include "hemm_internal.hpp"
+
+namespace {
+typedef u32 u32x2 __attribute__((ext_vector_type(2)));
+// Column passes address a limb through a buffer resource: the limb's base sits in scalar registers, the slab row
+// (a step of 2 KiB or 32 KiB) goes into the scalar offset of each access and a thread supplies one 32-bit byte offset
+// for all of its 16 accesses -- with 64-bit addresses in vector registers every access costs an add with carry.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t limb_rsrc(const void *p) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, -1, 0x00020000);   // raw, no range limit, 32-bit format
+}
+template <class E>
+__device__ __forceinline__ E buf_load(const __amdgpu_buffer_rsrc_t r, const u32 voff, const u32 soff) {
+    const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
+    const u64 u = ((u64)w.y << 32) | w.x;
+    E v;
+    __builtin_memcpy(&v, &u, 8);
+    return v;
+}
+template <class E>
+__device__ __forceinline__ void buf_store(const __amdgpu_buffer_rsrc_t r, const u32 voff, const u32 soff, const E v) {
+    u64 u;
+    __builtin_memcpy(&u, &v, 8);
+    u32x2 w;
+    w.x = (u32)u;
+    w.y = (u32)(u >> 32);
+    __builtin_amdgcn_raw_buffer_store_b64(w, r, voff, soff, 0);
+}
+
+struct __align__(16) Tw {
+    u64 w, ws;
+};
+
+// Lazy butterflies (q < 2^61, so 8q < 2^64): forward values stay in [0, 8q), inverse values in [0, 4q); q4 = 4q.
+// u -= 4q when u >= 4q, written as an addition of -4q and a select: no borrow chain
+__device__ __forceinline__ u64 csub(u64 u, const u64 m, const u64 neg_m) {
+    u64 t = u + neg_m;
+    asm("" : "+v"(t));          // keeps the compiler from turning this back into a subtraction of a selected 0 / m
+    return u >= m ? t : u;
+}
+// 2^64 - m as a value the compiler cannot see through (it would turn x + (2^64 - m) back into a subtraction)
+__device__ __forceinline__ u64 opaque_neg(u64 m) {
+    u64 n = 0 - m;
+    asm("" : "+s"(n));
+    return n;
+}
+__device__ __forceinline__ void ct_bfly(u64 &x, u64 &y, const Tw tw, const u64 q, const u64 q4, const u64 nq4) {
+    const u64 u = csub(x, q4, nq4);                        // < 4q
+    const u64 v = mul_shoup_lazy4(y, tw.w, tw.ws, q);      // < 4q
+    x = u + v;
+    y = u - v + q4;
+}
+__device__ __forceinline__ void gs_bfly(u64 &x, u64 &y, const Tw tw, const u64 q, const u64 q4, const u64 nq4) {
+    const u64 u = x, v = y;                                // < 4q each
+    x = csub(u + v, q4, nq4);
+    y = mul_shoup_lazy4(u - v + q4, tw.w, tw.ws, q);
+}
+
+// Two arithmetic back ends share the kernels below.
+//
+// IntField: 64-bit Shoup butterflies with values kept in [0, 4q) (Harvey), for primes up to 2^61.
+//
+// FpField: primes below 2^44 in double precision.  gfx950 issues one FP64 FMA per lane per clock but
+// has to assemble every 64-bit integer product from 32-bit pieces, so for residues that fit a double
+// exactly the floating-point butterfly is about a third of the instructions.  A product y*w mod q is
+//     c = rint(y * (w/q));  h = fl(y*w);  l = fma(y, w, -h)  [exact low part];  r = fma(-c, q, h) + l
+// Both h - c*q and the final sum are integers far below 2^53, so r is an exact residue of y*w, whatever c is.  The
+// quotient w/q is formed as fl(w * fl(1/q)): y * (w/q) is then off by at most |y| * 1.5 * 2^-52, so
+// |r| <= (0.5 + |y| * 1.5 * 2^-52) q -- 0.57 q for |y| < 2^47.5, 0.8 q for |y| < 2^49.7.  Values stay signed and
+// unreduced through the forward stages (growth 0.57 q per stage: below 11 q < 2^48 after all 16); the inverse
+// stages double the sums, so a radix-16 block first reduces its inputs.
+// The last pass maps to [0, q), which makes the stored result identical to the integer path's.
+// Between the two launches of one transform the buffer holds the raw doubles.
+#pragma clang fp contract(off)
+
+// LAZY16 (primes below 2^60, so 16q < 2^64; forward transforms only): forward values stay in [0, 16q) and only every
+// other stage corrects its first operand -- by 8q, which takes values below 16q to below 8q; the stage after it adds up
+// to 4q twice without a correction.  One conditional subtraction per two butterflies instead of one per butterfly.
+template <bool LAZY16>
+struct IntFieldT {
+    typedef u64 E;
+    typedef Tw W;
+    u64 q, q2, q4, nq8, nq4, nq2, nq1, ni, nis;
+    __device__ __forceinline__ IntFieldT(const ModQ *modq, const u64 *ninv, const u64 *ninv_s, const double *, int prime) {
+        q = modq[prime].q;
+        q2 = 2 * q;
+        q4 = 4 * q;
+        nq8 = opaque_neg(2 * q4);
+        nq4 = opaque_neg(q4);
+        nq2 = opaque_neg(q2);
+        nq1 = opaque_neg(q);
+        // a pass that does not end an inverse transform has no use for them and brings no table
+        ni = ninv != nullptr ? ninv[prime] : 0;
+        nis = ninv_s != nullptr ? ninv_s[prime] : 0;
+    }
+    __device__ __forceinline__ E from_canonical(u64 v) const { return v; }
+    __device__ __forceinline__ E from_dot(const Dot3 &d, const ModQ &m) const { return dot3_reduce(d, m); }
+    // odd: the stage's index within its radix-16 block is odd
+    __device__ __forceinline__ void ct(E &x, E &y, const W tw, const bool odd) const {
+        if (!LAZY16) {
+            ct_bfly(x, y, tw, q, q4, nq4);
+            return;
+        }
+        const u64 u = odd ? x : csub(x, 2 * q4, nq8);   // < 12q on odd stages, < 8q on even ones
+        const u64 v = mul_shoup_lazy4(y, tw.w, tw.ws, q);              // < 4q
+        x = u + v;
+        y = u - v + q4;
+    }
+    __device__ __forceinline__ void gs(E &x, E &y, const W tw) const { gs_bfly(x, y, tw, q, q4, nq4); }
+    template <int T>
+    __device__ __forceinline__ void after_inverse_block(E (&)[16]) const {}
+    __device__ __forceinline__ u64 to_canonical(E v) const {   // v < 8q (16q with LAZY16)
+        if (LAZY16) v = csub(v, 2 * q4, nq8);
+        return csub(csub(csub(v, q4, nq4), q2, nq2), q, nq1);
+    }
+    __device__ __forceinline__ u64 scale_to_canonical(E v) const {
+        return csub(mul_shoup_lazy(v, ni, nis, q), q, nq1);
+    }
+    // (y - v) * cst mod q for a transformed value v and a canonical minuend y
+    __device__ __forceinline__ u64 sub_scale(E v, u64 y, const Tw cst) const {
+        const u64 c = to_canonical(v);
+        const u64 d = y >= c ? y - c : y + q - c;
+        return csub(mul_shoup_lazy(d, cst.w, cst.ws, q), q, nq1);
+    }
+};
+
+typedef IntFieldT<false> IntField;
+
+
+struct FpField {
+    typedef double E;
+    typedef double W;   // the twiddle as a double; its quotient w / q is formed on the fly as w * (1 / q)
+    double q, qinv, ni, niinv;
+    __device__ __forceinline__ FpField(const ModQ *, const u64 *, const u64 *, const double *fp, int prime) {
+        q = fp[4 * prime];
+        qinv = fp[4 * prime + 1];
+        ni = fp[4 * prime + 2];
+        niinv = fp[4 * prime + 3];
+    }
+    __device__ __forceinline__ E mulmod(E y, E w, E winv) const {
+        const double c = __builtin_rint(y * winv);
+        const double h = y * w;
+        const double l = __builtin_fma(y, w, -h);
+        return __builtin_fma(-c, q, h) + l;
+    }
+    __device__ __forceinline__ E reduce(E x) const { return __builtin_fma(-__builtin_rint(x * qinv), q, x); }
+    __device__ __forceinline__ E from_canonical(u64 v) const {
+        return __longlong_as_double((long long)(v | 0x4330000000000000ull)) - 4503599627370496.0;
+    }
+    // A lazy dot product (three accumulators of weights 1, 2^32, 2^64 and a carry count of weight 2^64) as a residue of
+    // magnitude below q: regrouped into pieces of weights 1, 2^32, 2^64 below 2^32, 2^33 and 2^45 (constants below
+    // 2^44, residues below 2^60, 8 terms), each exact in a double; the two upper ones are multiplied by 2^32 and 2^64
+    // mod q.  No integer reduction and no conversion from canonical form.
+    __device__ __forceinline__ E from_dot(const Dot3 &d, const ModQ &) const {
+        const u64 p1 = (d.s0 >> 32) + (d.s1 & 0xffffffffull), p2 = (d.s1 >> 32) + d.s2 + d.c;
+        const double r32 = reduce(4294967296.0), r64 = reduce(18446744073709551616.0);
+        const double a = (double)(u32)d.s0 + mulmod(from_canonical(p1), r32, r32 * qinv) +
+                         mulmod(from_canonical(p2), r64, r64 * qinv);
+        return reduce(a);
+    }
+    __device__ __forceinline__ void ct(E &x, E &y, const W tw, const bool) const {
+        const double v = mulmod(y, tw, tw * qinv);
+        const double u = x;
+        x = u + v;
+        y = u - v;
+    }
+    __device__ __forceinline__ void gs(E &x, E &y, const W tw) const {
+        const double u = x, v = y;
+        x = u + v;
+        y = mulmod(u - v, tw, tw * qinv);
+    }
+    // A Gentleman-Sande block of T stages doubles the sums: from inputs bounded by B, element 0 of a sub-block of 2^T is
+    // bounded by 2^T B, element 1 by 2^(T-1) r, elements 2 and 3 by 2^(T-2) r, ... with r the bound of a product, and the
+    // largest value it multiplies is 2^T B.  With element 0 of every sub-block (and element 1 where T = 4) reduced after
+    // each block every block starts from B <= 4 r: r <= 0.8 q gives B <= 3.2 q and 16 B <= 51 q < 2^49.7 (q < 2^44), for
+    // which r <= 0.8 q holds again; products of values below 2^50 are still exact.
+    template <int T>
+    __device__ __forceinline__ void after_inverse_block(E (&x)[16]) const {
+#pragma unroll
+        for (int k = 0; k < 16; k += 1 << T) x[k] = reduce(x[k]);
+        if (T == 4) x[1] = reduce(x[1]);
+    }
+    __device__ __forceinline__ u64 centred_to_canonical(E r) const {
+        r += r < 0.0 ? q : 0.0;
+        return (u64)__double_as_longlong(r + 4503599627370496.0) & 0x000fffffffffffffull;
+    }
+    __device__ __forceinline__ u64 to_canonical(E v) const { return centred_to_canonical(reduce(v)); }
+    __device__ __forceinline__ u64 scale_to_canonical(E v) const { return centred_to_canonical(mulmod(v, ni, niinv)); }
+    __device__ __forceinline__ u64 sub_scale(E v, u64 y, const Tw cst) const {
+        const double w = (double)cst.w;
+        return centred_to_canonical(mulmod(from_canonical(y) - v, w, w * qinv));
+    }
+};
+
+// T Cooley-Tukey stages on 16 registers that hold 16 >> T sub-blocks of 2^T consecutive points; stage s, group g uses
+// twiddle (X << s) + g.  SAME: the sub-blocks are different columns of one block and share its twiddles.
+template <int T, bool SAME = false, class F>
+__device__ __forceinline__ void radix_fwd(const F &f, typename F::E (&x)[16], const typename F::W *__restrict__ tw,
+                                          const u32 X) {
+#pragma unroll
+    for (int s = 0; s < T; s++) {
+        const int d = 1 << (T - 1 - s);
+#pragma unroll
+        for (int g = 0; g < 8 / d; g++) {
+            const typename F::W w = tw[(X << s) + (SAME ? g & ((1 << s) - 1) : g)];
+#pragma unroll
+            for (int j = 0; j < d; j++) f.ct(x[g * 2 * d + j], x[g * 2 * d + j + d], w, (s & 1) != 0);
+        }
+    }
+}
+// T Gentleman-Sande stages; stage s (distance 1 << s), group g uses twiddle (X << (T - 1 - s)) + g.
+template <int T, bool SAME = false, class F>
+__device__ __forceinline__ void radix_inv(const F &f, typename F::E (&x)[16], const typename F::W *__restrict__ tw,
+                                          const u32 X) {
+#pragma unroll
+    for (int s = 0; s < T; s++) {
+        const int d = 1 << s;
+#pragma unroll
+        for (int g = 0; g < (8 >> s); g++) {
+            const typename F::W w = tw[(X << (T - 1 - s)) + (SAME ? g & ((1 << (T - 1 - s)) - 1) : g)];
+#pragma unroll
+            for (int j = 0; j < d; j++) f.gs(x[g * 2 * d + j], x[g * 2 * d + j + d], w);
+        }
+    }
+}
+
+// The inner radix-16 block of a row pass (X = 16 (R + r) + c: a different X for every thread) reads its 15 twiddles
+// from a table laid out for it: entry ((r * 15 + slot) * 16 + c), slot = 2^l - 1 + g for twiddle (X << l) + g, so that
+// the 16 threads of a row read 16 consecutive entries per (l, g) -- from the stage-ordered table they would read 16
+// entries 2^l apart, up to 64 cache lines per load instruction of a wavefront instead of 8.
+template <class F>
+__device__ __forceinline__ void radix16_fwd_rows(const F &f, typename F::E (&x)[16], const typename F::W *__restrict__ rt) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const int d = 8 >> s;
+#pragma unroll
+        for (int g = 0; g < (1 << s); g++) {
+            const typename F::W w = rt[((1 << s) - 1 + g) * 16];
+#pragma unroll
+            for (int j = 0; j < d; j++) f.ct(x[g * 2 * d + j], x[g * 2 * d + j + d], w, (s & 1) != 0);
+        }
+    }
+}
+template <class F>
+__device__ __forceinline__ void radix16_inv_rows(const F &f, typename F::E (&x)[16], const typename F::W *__restrict__ rt) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const int d = 1 << s;
+#pragma unroll
+        for (int g = 0; g < (8 >> s); g++) {
+            const typename F::W w = rt[((8 >> s) - 1 + g) * 16];
+#pragma unroll
+            for (int j = 0; j < d; j++) f.gs(x[g * 2 * d + j], x[g * 2 * d + j + d], w);
+        }
+    }
+}
+
+#define ROWPAD 272  // 256 residues of a row + one pad word per 16, so a 16-lane column read
+                    // (stride 17 words) hits 16 distinct bank pairs
+__device__ __forceinline__ int padc(int c) { return c + (c >> 4); }
+
+__device__ __forceinline__ int swz_row(int r) { return r ^ ((r >> 4) & 1); }
+
+// The 16 coefficients of a thread as a basis conversion computed on the fly: coefficient k is sum_i v_i * hat_i mod q
+// over the n_src <= NS source limbs (pre-scaled, the same lazy sums and reductions as the stand-alone conversion kernels,
+// so the residues are the same), read at voff + off(k) inside a limb; so[i]: byte offset of source limb i.
+template <int NS, class F, class OFF>
+__device__ __forceinline__ void converted_inputs(const F &f, typename F::E (&x)[16], const __amdgpu_buffer_rsrc_t src,
+                                                 const u32 voff, const u32 (&so)[NS], const u64 (&h)[NS], const int n_src,
+                                                 const ModQ m, const OFF off) {
+    // eight coefficients at a time (three accumulators each), source by source, so that the eight loads of one source
+    // limb are in flight together
+#pragma unroll
+    for (int half = 0; half < 2; half++) {
+        Dot3 d[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) dot3_clear(d[k]);
+#pragma unroll
+        for (int i = 0; i < NS; i++) {
+            if (i < n_src) {
+                u64 v[8];
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(src, voff, so[i] + off(8 * half + k), 0);
+                    v[k] = ((u64)w.y << 32) | w.x;
+                }
+#pragma unroll
+                for (int k = 0; k < 8; k++) dot3_add(d[k], v[k], h[i]);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++) x[8 * half + k] = f.from_dot(d[k], m);
+    }
+}
+
+// A row's 16 threads sit in one wavefront (thread = row * 16 + column group), so the LDS exchanges of
+// the row kernel never cross a wavefront: ordering them needs no workgroup barrier, only a fence that
+// keeps the compiler from moving LDS accesses across it.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Optional tail of a forward transform: instead of storing the transformed residues v in place, store
+// (minuend - v) * cst[limb] to `out` -- the last step of ModDown / rescale, folded into the pass that
+// already holds v in registers (saves one read and one write of every limb and a launch).
+struct NttEpilogue {
+    const u64 *minuend;
+    u64 *out;
+    const Tw *cst;  // per limb: constant and Shoup quotient
+    size_t minuend_stride, out_stride;
+    u32 galois;     // inverse transforms that read their input elsewhere: != 0 reads it through this automorphism
+};
+// An inverse transform may read its input elsewhere (same slot numbering, own polynomial stride) and leave the
+// result in `data`: the first pass then loads from `minuend` (stride `minuend_stride`) instead of `data`.
+
+// forward pass 2 / inverse pass 1 work on 16 whole rows (16 x 256 contiguous residues); r: the row of 2^log_r.
+// GAL (inverse only): ld is the base of the source limb and residue k of the input is ld[galois_index(k)] -- an aligned
+// group of 16 residues stays an aligned group under the automorphism, so the loads touch the same number of lines
+// IN_LDS: the row pass follows (forward) or precedes (inverse) a column pass over the same limb in the same workgroup: the
+// row is taken from, resp. left in, its padded LDS row instead of memory.
+template <bool INV, bool EPI, bool GAL, bool IN_LDS, class F>
+__device__ __forceinline__ void rows_body(u64 *__restrict__ row, const Tw *__restrict__ tw_int,
+                                          const Tw *__restrict__ rtw_int, const F f, u64 *lds_raw, const int log_r, const u32 r,
+                                          const u64 *__restrict__ mn, u64 *__restrict__ o, const Tw cst,
+                                          const u64 *__restrict__ ld, const u32 gal = 0) {
+    typedef typename F::E E;
+    const typename F::W *tw = (const typename F::W *)tw_int;
+    const int c = threadIdx.x & 15, rr = threadIdx.x >> 4;
+    const typename F::W *rt = (const typename F::W *)rtw_int + (r * 15u * 16u + (u32)c);
+    E *l = (E *)lds_raw + rr * ROWPAD;
+    u64 *lc = lds_raw + rr * ROWPAD;
+    E *mem = (E *)row;
+    E x[16];
+    if (!INV) {
+#pragma unroll
+        for (int k = 0; k < 16; k++) x[k] = IN_LDS ? l[padc(c + 16 * k)] : mem[c + 16 * k];
+        radix_fwd<4>(f, x, tw, (1u << log_r) + r);
+#pragma unroll
+        for (int k = 0; k < 16; k++) l[padc(c + 16 * k)] = x[k];
+        wave_sync();
+#pragma unroll
+        for (int k = 0; k < 16; k++) x[k] = l[padc(16 * c + k)];
+        // the minuend of the fused tail is fetched under the second radix-16 block instead of after it
+        u64 mv[EPI ? 16 : 1];
+        if (EPI) {
+#pragma unroll
+            for (int k = 0; k < 16; k++) mv[k] = __builtin_nontemporal_load(mn + c + 16 * k);
+        }
+        radix16_fwd_rows(f, x, rt);
+        wave_sync();
+#pragma unroll
+        for (int k = 0; k < 16; k++) l[padc(16 * c + k)] = x[k];
+        wave_sync();
+        if (EPI) {
+#pragma unroll
+            for (int k = 0; k < 16; k++) o[c + 16 * k] = f.sub_scale(l[padc(c + 16 * k)], mv[k], cst);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 16; k++) row[c + 16 * k] = f.to_canonical(l[padc(c + 16 * k)]);
+        }
+    } else {
+        if (GAL) {
+#pragma unroll
+            for (int k = 0; k < 16; k++) lc[padc(c + 16 * k)] = ld[galois_index((r << 8) + (u32)(c + 16 * k), gal, 8 + log_r)];
+        } else {
+#pragma unroll
+            for (int k = 0; k < 16; k++) lc[padc(c + 16 * k)] = ld[c + 16 * k];
+        }
+        wave_sync();
+#pragma unroll
+        for (int k = 0; k < 16; k++) x[k] = f.from_canonical(lc[padc(16 * c + k)]);
+        radix16_inv_rows(f, x, rt);
+        f.template after_inverse_block<4>(x);
+        wave_sync();
+#pragma unroll
+        for (int k = 0; k < 16; k++) l[padc(16 * c + k)] = x[k];
+        wave_sync();
+#pragma unroll
+        for (int k = 0; k < 16; k++) x[k] = l[padc(c + 16 * k)];
+        radix_inv<4>(f, x, tw, (1u << log_r) + r);
+        f.template after_inverse_block<4>(x);
+        if (IN_LDS) {   // the places this thread has just read
+#pragma unroll
+            for (int k = 0; k < 16; k++) l[padc(c + 16 * k)] = x[k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < 16; k++) mem[c + 16 * k] = x[k];
+        }
+    }
+}
+
+}  // namespace

@@ -1,0 +1,259 @@
+// Transforms in one launch, a workgroup per limb: rings of 2^10 .. 2^12 points, and batches of many limbs of 2^13 and 2^14.
+//
+// Such a limb (8 .. 128 KiB) fits the LDS of one CU, so the column pass and the row pass of the R x 256 view
+// (R = N / 256) meet in LDS instead of in memory, and a transform that the two-launch kernels would take as two dependent
+// launches is one.  What bounds a call on the small rings is the number of dependent launches, a few microseconds each
+// however little they do, not arithmetic or bytes: one transform of 2^12 points 7 us against 36 us with the butterflies
+// of every stage read from and written to LDS one by one, which these kernels replace.  A thread holds 16 residues: the log2 R
+// column stages in one block (R <= 16) or two, one exchange through LDS after each, then the row pass of the two-launch
+// kernels (two radix-16 blocks).  The first stages can read their input from a
+// basis conversion, the last ones can end in (minuend - v) * constant, and an inverse transform can read its input
+// elsewhere and through an automorphism, as in the two-launch kernels: same arithmetic, same residues.
+#include <algorithm>
+#include <cstring>
+
+#include "ntt_device.h"
+
+namespace {
+
+template <int LR>
+struct Limb {
+    static constexpr int R = 1 << LR, NT = 16 << LR;   // rows, threads
+    static constexpr int Q = LR > 4 ? R / 16 : 1;      // LR > 4: two column blocks, of four stages and of LR - 4
+    static constexpr int T1 = LR > 4 ? 4 : LR, T2 = LR - T1;
+    // R <= 16: element k of a thread is row k % R of column threadIdx.x + NT * (k / R); otherwise row rh + Q k of column
+    // threadIdx.x % 256 in the first block and row 16 rh + k in the second, rh = threadIdx.x / 256
+    static __device__ __forceinline__ int rh() { return LR > 4 ? (int)(threadIdx.x >> 8) : 0; }
+    static __device__ __forceinline__ int row(const int k) { return LR > 4 ? rh() + Q * k : k & (R - 1); }
+    static __device__ __forceinline__ int col(const int k) {
+        return LR > 4 ? (int)(threadIdx.x & 255) : (int)threadIdx.x + NT * (k / R);
+    }
+    // byte offset inside the limb: a thread's part and the step to element k
+    static __device__ __forceinline__ u32 voff() { return ((LR > 4 ? threadIdx.x & 255 : threadIdx.x) + ((u32)rh() << 8)) * 8u; }
+    static __device__ __forceinline__ constexpr u32 off(const int k) {
+        return LR > 4 ? (u32)(k * Q * 2048) : (u32)((k & (R - 1)) * 2048 + (k / R) * NT * 8);
+    }
+    static __device__ __forceinline__ int at(const int k) { return row(k) * ROWPAD + padc(col(k)); }
+    static __device__ __forceinline__ int at2(const int k) { return (16 * rh() + k) * ROWPAD + padc(col(k)); }
+};
+
+template <int LR, int NS, bool EPI, class F>
+__device__ __forceinline__ void limb_forward(u64 *__restrict__ limb, const Tw *__restrict__ tw_int, const Tw *__restrict__ rtw,
+                                             const F f, u64 *lds_raw, const __amdgpu_buffer_rsrc_t src,
+                                             const u32 (&so)[NS > 0 ? NS : 1], const u64 (&h)[NS > 0 ? NS : 1], const int n_src,
+                                             const ModQ m, const u64 *__restrict__ mn, u64 *__restrict__ o, const Tw cst) {
+    typedef typename F::E E;
+    typedef Limb<LR> S;
+    E *lds = (E *)lds_raw;
+    E x[16];
+    if (NS > 0) {
+        converted_inputs<(NS > 0 ? NS : 1)>(f, x, src, S::voff(), so, h, n_src, m,
+                                            [](const int k) { return S::off(k); });
+    } else {
+#pragma unroll
+        for (int k = 0; k < 16; k++) x[k] = f.from_canonical(buf_load<u64>(src, S::voff(), S::off(k)));
+    }
+    radix_fwd<S::T1, true>(f, x, (const typename F::W *)tw_int, 1u);
+#pragma unroll
+    for (int k = 0; k < 16; k++) lds[S::at(k)] = x[k];
+    __syncthreads();
+    if (S::T2 > 0) {
+#pragma unroll
+        for (int k = 0; k < 16; k++) x[k] = lds[S::at2(k)];
+        radix_fwd<S::T2>(f, x, (const typename F::W *)tw_int, 16u + (u32)S::rh() * (16 / S::Q));
+#pragma unroll
+        for (int k = 0; k < 16; k++) lds[S::at2(k)] = x[k];   // the places this thread has just read
+        __syncthreads();
+    }
+    const u32 r = threadIdx.x >> 4;
+    rows_body<false, EPI, false, true>(limb + (r << 8), tw_int, rtw, f, lds_raw, LR, r, EPI ? mn + (r << 8) : nullptr,
+                                       EPI ? o + (r << 8) : nullptr, cst, nullptr);
+}
+
+// data[n_polys][.][N] (polynomial stride poly_stride), limb l in slot sl[l]; NS > 0: the inputs are the conversions of
+// cs, whose plain copies follow the limbs of a polynomial; EPI: out = (minuend - transform) * cst[l].
+template <int LR, int NS, bool EPI>
+__global__ __launch_bounds__(16 << LR) void ntt_limb_forward_kernel(
+    u64 *__restrict__ data, const Tw *__restrict__ tw_all, const Tw *__restrict__ rtw_all, const ModQ *__restrict__ modq,
+    const double *__restrict__ fp, LimbList ll, LimbList sl, int n_limbs, size_t poly_stride, ConvSources cs, NttEpilogue ep) {
+    __shared__ u64 lds[(ROWPAD << LR)];
+    const int log_n = 8 + LR;
+    const int per_poly = n_limbs + (NS > 0 ? cs.n_copy : 0);
+    const int limb = blockIdx.x % per_poly, poly = blockIdx.x / per_poly;
+    if (NS > 0 && limb >= n_limbs) {   // a limb that is only copied into its slot
+        const u64 *from = cs.copy_src + (size_t)poly * cs.copy_src_stride + ((size_t)cs.copy_src_slot[limb - n_limbs] << log_n);
+        u64 *to = data + (size_t)poly * poly_stride + ((size_t)cs.copy_dst_slot[limb - n_limbs] << log_n);
+        u64 t[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) {
+            const u32 n = threadIdx.x + (u32)k * (16u << LR);
+            t[k] = from[cs.copy_galois != 0 ? galois_index(n, cs.copy_galois, log_n) : n];
+        }
+#pragma unroll
+        for (int k = 0; k < 16; k++) to[threadIdx.x + (u32)k * (16u << LR)] = t[k];
+        return;
+    }
+    const int prime = __builtin_amdgcn_readfirstlane((int)ll.idx[limb]);   // byte tables are read with vector loads
+    u64 *base = data + (size_t)poly * poly_stride + ((size_t)__builtin_amdgcn_readfirstlane((int)sl.idx[limb]) << log_n);
+    const Tw *tw = tw_all + ((size_t)prime << log_n), *rtw = rtw_all + ((size_t)prime << log_n);
+    const ModQ m = modq[prime];
+    __amdgpu_buffer_rsrc_t src = limb_rsrc(base);
+    u32 so[NS > 0 ? NS : 1];
+    u64 h[NS > 0 ? NS : 1];
+    int n_src = 0;
+    if (NS > 0) {
+        const int dg = __builtin_amdgcn_readfirstlane((int)cs.digit_of[limb]);
+        n_src = cs.d[dg].n_src;
+        src = limb_rsrc(cs.d[dg].src + (size_t)poly * cs.d[dg].src_poly_stride);
+        const Cst *hat = cs.d[dg].hat + prime;
+#pragma unroll
+        for (int i = 0; i < NS; i++) {
+            const int ii = i < n_src ? i : 0;
+            so[i] = __builtin_amdgcn_readfirstlane((u32)cs.d[dg].src_slot[ii]) << (log_n + 3);
+            h[i] = hat[(size_t)ii * cs.hat_ld].w;
+        }
+    }
+    const u64 *mn = nullptr;
+    u64 *o = nullptr;
+    Tw cst{0, 0};
+    if (EPI) {
+        mn = ep.minuend + (size_t)poly * ep.minuend_stride + ((size_t)limb << log_n);
+        o = ep.out + (size_t)poly * ep.out_stride + ((size_t)limb << log_n);
+        cst = ep.cst[limb];
+    }
+    if (fp[4 * prime] != 0.0)
+        limb_forward<LR, NS, EPI>(base, tw, rtw, FpField(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, mn, o, cst);
+    else if ((m.q >> 60) != 0)
+        limb_forward<LR, NS, EPI>(base, tw, rtw, IntField(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, mn, o, cst);
+    else
+        limb_forward<LR, NS, EPI>(base, tw, rtw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, mn,
+                                  o, cst);
+}
+
+template <int LR, bool GAL, class F>
+__device__ __forceinline__ void limb_inverse(u64 *__restrict__ limb, const Tw *__restrict__ tw_int, const Tw *__restrict__ rtw,
+                                             const F f, u64 *lds_raw, const u64 *__restrict__ ld, const u32 gal) {
+    typedef typename F::E E;
+    typedef Limb<LR> S;
+    E *lds = (E *)lds_raw;
+    const u32 r = threadIdx.x >> 4;
+    rows_body<true, false, GAL, true>(limb, tw_int, rtw, f, lds_raw, LR, r, nullptr, nullptr, Tw{0, 0}, GAL ? ld : ld + (r << 8), gal);
+    __syncthreads();
+    E x[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) x[k] = lds[S::T2 > 0 ? S::at2(k) : S::at(k)];
+    if (S::T2 > 0) {
+        radix_inv<S::T2>(f, x, (const typename F::W *)tw_int, 16u + (u32)S::rh() * (16 / S::Q));
+        f.template after_inverse_block<S::T2>(x);
+#pragma unroll
+        for (int k = 0; k < 16; k++) lds[S::at2(k)] = x[k];   // the places this thread has just read
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 16; k++) x[k] = lds[S::at(k)];
+    }
+    radix_inv<S::T1, true>(f, x, (const typename F::W *)tw_int, 1u);
+    const __amdgpu_buffer_rsrc_t to = limb_rsrc(limb);
+#pragma unroll
+    for (int k = 0; k < 16; k++) buf_store<u64>(to, S::voff(), S::off(k), f.scale_to_canonical(x[k]));
+}
+
+template <int LR, bool GAL>
+__global__ __launch_bounds__(16 << LR) void ntt_limb_inverse_kernel(
+    u64 *__restrict__ data, const Tw *__restrict__ tw_all, const Tw *__restrict__ rtw_all, const ModQ *__restrict__ modq,
+    const u64 *__restrict__ ninv, const u64 *__restrict__ ninv_s, const double *__restrict__ fp, LimbList ll, LimbList sl,
+    int n_limbs, size_t poly_stride, const Tw *__restrict__ final_scale, const u64 *__restrict__ from, size_t from_stride,
+    u32 gal) {
+    __shared__ u64 lds[(ROWPAD << LR)];
+    const int log_n = 8 + LR;
+    const int limb = blockIdx.x % n_limbs, poly = blockIdx.x / n_limbs;
+    const int prime = __builtin_amdgcn_readfirstlane((int)ll.idx[limb]);
+    const size_t slot = (size_t)__builtin_amdgcn_readfirstlane((int)sl.idx[limb]) << log_n;
+    u64 *base = data + (size_t)poly * poly_stride + slot;
+    const u64 *ld = from != nullptr ? from + (size_t)poly * from_stride + slot : base;
+    const Tw *tw = tw_all + ((size_t)prime << log_n), *rtw = rtw_all + ((size_t)prime << log_n);
+    if (fp[4 * prime] != 0.0) {
+        FpField f(modq, ninv, ninv_s, fp, prime);
+        if (final_scale != nullptr) {
+            f.ni = (double)final_scale[limb].w;
+            f.niinv = f.ni * f.qinv;
+        }
+        limb_inverse<LR, GAL>(base, tw, rtw, f, lds, ld, gal);
+    } else {
+        IntField f(modq, ninv, ninv_s, fp, prime);
+        if (final_scale != nullptr) {
+            f.ni = final_scale[limb].w;
+            f.nis = final_scale[limb].ws;
+        }
+        limb_inverse<LR, GAL>(base, tw, rtw, f, lds, ld, gal);
+    }
+}
+
+}  // namespace
+
+void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
+                         size_t poly_stride, hipStream_t s, const ConvSources *cs, const u64 *minuend, size_t minuend_stride,
+                         u64 *out, size_t out_stride, const void *cst_dev) {
+    const int LR = c->logN - 8;
+    int widest = 0;
+    ConvSources none;
+    if (cs == nullptr) {
+        memset(&none, 0, sizeof(none));
+        cs = &none;
+    } else {
+        for (int l = 0; l < n_limbs; l++) widest = std::max(widest, cs->d[cs->digit_of[l]].n_src);
+    }
+    const NttEpilogue ep{minuend, out, (const Tw *)cst_dev, minuend_stride, out_stride, 0};
+    const dim3 grid((unsigned)((n_limbs + cs->n_copy) * n_polys)), block(16u << LR);
+#define LIMB_FORWARD(L, K, EPI)                                                                                            \
+    hipLaunchKernelGGL((ntt_limb_forward_kernel<L, K, EPI>), grid, block, 0, s, data, (const Tw *)c->d_w,                  \
+                       (const Tw *)c->d_rw, c->d_modq, c->d_fp, ll, sl, n_limbs, poly_stride, *cs, ep)
+#define LIMB_SOURCES(L, EPI)                          \
+    do {                                              \
+        if (widest == 0) LIMB_FORWARD(L, 0, EPI);     \
+        else if (widest <= 2) LIMB_FORWARD(L, 2, EPI); \
+        else if (widest <= 5) LIMB_FORWARD(L, 5, EPI); \
+        else LIMB_FORWARD(L, 8, EPI);                 \
+    } while (0)
+#define LIMB_RING(L)                       \
+    do {                                   \
+        if (out != nullptr) LIMB_SOURCES(L, true); \
+        else LIMB_SOURCES(L, false);       \
+    } while (0)
+    switch (LR) {
+        case 2: LIMB_RING(2); break;
+        case 3: LIMB_RING(3); break;
+        case 4: LIMB_RING(4); break;
+        case 5: LIMB_RING(5); break;
+        case 6: LIMB_FORWARD(6, 0, false); break;
+        default: throw std::invalid_argument("no one-launch transform for this ring size");
+    }
+#undef LIMB_RING
+#undef LIMB_SOURCES
+#undef LIMB_FORWARD
+}
+
+void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
+                         size_t poly_stride, hipStream_t s, const void *final_scale, const u64 *from, size_t from_stride,
+                         u32 galois) {
+    const int LR = c->logN - 8;
+    const dim3 grid((unsigned)(n_limbs * n_polys)), block(16u << LR);
+#define LIMB_INVERSE(L, GAL)                                                                                          \
+    hipLaunchKernelGGL((ntt_limb_inverse_kernel<L, GAL>), grid, block, 0, s, data, (const Tw *)c->d_iw,               \
+                       (const Tw *)c->d_irw, c->d_modq, c->d_ninv, c->d_ninv_s, c->d_fp, ll, sl, n_limbs, poly_stride, \
+                       (const Tw *)final_scale, from, from_stride, galois)
+#define LIMB_RING(L)                        \
+    do {                                    \
+        if (galois != 0) LIMB_INVERSE(L, true); \
+        else LIMB_INVERSE(L, false);        \
+    } while (0)
+    switch (LR) {
+        case 2: LIMB_RING(2); break;
+        case 3: LIMB_RING(3); break;
+        case 4: LIMB_RING(4); break;
+        case 5: LIMB_RING(5); break;
+        case 6: LIMB_INVERSE(6, false); break;
+        default: throw std::invalid_argument("no one-launch transform for this ring size");
+    }
+#undef LIMB_RING
+#undef LIMB_INVERSE
+}

@@ -1,0 +1,94 @@
+"""GPU parity of the register-blocked transforms on every ring size they serve: whole key switches and rescales through
+their fused forms, and batches on both sides of the line between the one-launch and the two-launch kernels."""
+import numpy as np
+import pytest
+
+from __graft_entry__ import load_package
+from oracle import oracle as O
+from oracle.oracle import _p
+
+pytestmark = pytest.mark.gpu
+
+
+def dev(a):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a).view(np.int64)).cuda()
+
+
+def host(t):
+    return t.cpu().numpy().view(np.uint64)
+
+
+def top_and_random(rng, mods, lead, N):
+    """random residues, the largest one in the first polynomial's first half"""
+    out = np.empty(tuple(lead) + (len(mods), N), dtype=np.uint64)
+    for j, q in enumerate(mods):
+        out[..., j, :] = rng.integers(0, q, tuple(lead) + (N,), dtype=np.uint64)
+        out.reshape(-1, len(mods), N)[0, j, : N // 2] = q - 1
+    return out
+
+
+# digits of 1, 2, 5, 8 limbs take a kernel each; of 9 the forms without a fused conversion
+@pytest.mark.parametrize("log_n", [10, 11, 12, 13, 14, 15])
+@pytest.mark.parametrize("chain,special,dnum", [(3, 1, 3), (6, 2, 3), (10, 4, 2), (8, 5, 1), (9, 6, 1)])
+def test_keyswitch_forms(log_n, chain, special, dnum):
+    pkg = load_package()
+    qs, ps = O.ckks_chain(log_n, chain, special)
+    ctx, orc, N = pkg.Context(log_n, qs, ps, dnum), O.Oracle(log_n, qs, ps, dnum), 1 << log_n
+    rng = np.random.default_rng(log_n * 100 + chain)
+    key = top_and_random(rng, qs + ps, (dnum, 2), N)
+    for nq in (chain, max(2, chain - 1)):
+        ct = top_and_random(rng, qs[:nq], (3,), N)
+        g = pow(5, 3, 2 * N)
+        rot = np.empty((2, nq, N), dtype=np.uint64)
+        for p in range(2):
+            for j in range(nq):
+                orc.L.orc_automorphism_ntt(orc.h, _p(ct[p, j]), _p(rot[p, j]), g)
+        kb, ka = orc.keyswitch(rot[1], key)
+        want = np.stack([orc.add_residues(rot[0], kb), ka])
+        assert np.array_equal(host(ctx.rotate(dev(ct[:2]), dev(key), g, nq)), want)
+        kb, ka = orc.keyswitch(ct[2], key)
+        want = np.stack([orc.add_residues(ct[0], kb), orc.add_residues(ct[1], ka)])
+        assert np.array_equal(host(ctx.relinearize(dev(ct), dev(key), nq)), want)
+        want = np.empty((3, nq - 1, N), dtype=np.uint64)
+        for p in range(3):
+            orc.L.orc_rescale(orc.h, _p(ct[p]), nq, _p(want[p]))
+        assert np.array_equal(host(ctx.rescale(dev(ct), nq)), want)
+
+
+# limbs on both sides of where a ring goes over to one launch, and a run of polynomials that is cut
+@pytest.mark.parametrize("log_n,polys,limbs", [(11, 1, 1), (12, 3, 5), (13, 21, 3), (13, 32, 2), (14, 19, 5), (14, 16, 6), (15, 7, 3),
+                                               (15, 300, 3)])
+def test_batches(log_n, polys, limbs):
+    pkg = load_package()
+    mods = [O.primes_below(61, log_n, 1)[0], O.primes_below(60, log_n, 1)[0]] + O.primes_below(44, log_n, 4)
+    mods = mods[:limbs]
+    ctx, orc, N = pkg.Context(log_n, mods, [], 1), O.Oracle(log_n, mods, [], 1, threads=8), 1 << log_n
+    rng = np.random.default_rng(log_n + polys)
+    a = top_and_random(rng, mods, (polys,), N)
+    idx = list(range(len(mods)))
+    for inverse in (False, True):
+        d = dev(a)
+        ctx.ntt(d, idx, inverse=inverse)
+        got = host(d)
+        for p in sorted({0, polys // 2, polys - 1}):
+            want = a[p].copy()
+            orc.ntt(want, idx, inverse=inverse)
+            assert np.array_equal(got[p], want), (inverse, p)
+        ctx.ntt(d, idx, inverse=not inverse)
+        assert np.array_equal(host(d), a)
+
+
+@pytest.mark.parametrize("log_n,polys", [(12, 2), (13, 5), (13, 24), (14, 24), (15, 3)])
+@pytest.mark.parametrize("drop", [0, 1])
+def test_moddown_of_batches(log_n, polys, drop):
+    pkg = load_package()
+    qs, ps = O.ckks_chain(log_n, 6, 3)
+    ctx, orc, N, nq = pkg.Context(log_n, qs, ps, 2), O.Oracle(log_n, qs, ps, 2), 1 << log_n, 5
+    rng = np.random.default_rng(log_n + polys + drop)
+    y = top_and_random(rng, qs[:nq] + ps, (polys,), N)
+    got = host(ctx.moddown_batch(dev(y), nq, drop))
+    for p in sorted({0, polys // 2, polys - 1}):
+        want = np.empty((nq - drop, N), dtype=np.uint64)
+        orc.L.orc_moddown_drop(orc.h, _p(y[p].copy()), nq, drop, _p(want))
+        assert np.array_equal(got[p], want), p
