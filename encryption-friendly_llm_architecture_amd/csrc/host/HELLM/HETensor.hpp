@@ -43,9 +43,9 @@ public:
     HETensor(const Context &c, i64 rows, i64 cols) : shape_(rows, cols), data_(c) {}
     HETensor(const Context &c, i64 rows, i64 cols, i64 block_width) : shape_(rows, cols, block_width), data_(c) {}
     HETensor(const Context &c, const TileTensorShape &s) : shape_(s), data_(c) {}
-    HETensor(i64 rows, i64 cols, const T &d) : shape_(rows, cols), data_(d) {}
-    HETensor(i64 rows, i64 cols, const T &d, i64 block_width) : shape_(rows, cols, block_width), data_(d) {}
-    HETensor(const TileTensorShape &s, const T &d) : shape_(s), data_(d) {}
+    HETensor(i64 rows, i64 cols, T d) : shape_(rows, cols), data_(std::move(d)) {}
+    HETensor(i64 rows, i64 cols, T d, i64 block_width) : shape_(rows, cols, block_width), data_(std::move(d)) {}
+    HETensor(const TileTensorShape &s, T d) : shape_(s), data_(std::move(d)) {}
 
     T &get() { return data_; }
     const T &get() const { return data_; }

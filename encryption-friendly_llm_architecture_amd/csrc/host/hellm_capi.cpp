@@ -45,6 +45,8 @@ static Matrix mat(const double *p, uint32_t rows, uint32_t cols) {
     memcpy(m.v.data(), p, sizeof(double) * m.v.size());
     return m;
 }
+// an object for a result of the shape of `a`: the evaluator gives it its buffer, nothing is copied into it first
+static hellm_ct *like(const hellm_ct *a) { return new hellm_ct{CtxtTensor(a->t.get().getContext(), a->t.getShape())}; }
 static void need(bool ok, const char *msg) {
     if (!ok) throw std::invalid_argument(msg);
 }
@@ -324,7 +326,7 @@ int hellm_one_mat_rot_sum_inplace(hellm_hemmer *h, hellm_ct *a, hellm_ct *b) {
 int hellm_mask_right_left(hellm_hemmer *h, const hellm_ct *a, hellm_ct **out_left, hellm_ct **out_right) {
     FACADE_TRY
     need(h && a && out_left && out_right, "null argument");
-    hellm_ct *l = new hellm_ct{a->t}, *r = new hellm_ct{a->t};
+    hellm_ct *l = like(a), *r = like(a);
     h->m->maskRightLeft(a->t, l->t, r->t);
     *out_left = l;
     *out_right = r;
@@ -498,7 +500,7 @@ int hellm_ctvec_get(const hellm_ctvec *v, uint32_t i, uint32_t rows, uint32_t co
     int name(hellm_hemmer *h, const hellm_ct *a, hellm_ct **out) {    \
         FACADE_TRY                                                    \
         need(h && a && out, "null argument");                         \
-        hellm_ct *r = new hellm_ct{a->t};                             \
+        hellm_ct *r = like(a);                                         \
         try {                                                         \
             expr;                                                     \
         } catch (...) {                                               \
@@ -513,7 +515,7 @@ int hellm_left_rotate(hellm_hemmer *h, const hellm_ct *a, uint64_t rot, hellm_ct
     FACADE_TRY
     need(h && a && out, "null argument");
     h->m->ensureRotationKeys({rot});
-    hellm_ct *r = new hellm_ct{a->t};
+    hellm_ct *r = like(a);
     h->m->getEval().leftRotate(a->t.get(), rot, r->t.get());
     *out = r;
     FACADE_CATCH
@@ -526,7 +528,7 @@ UNARY_EVAL(hellm_diagonal_to_row, r->t = h->m->diagonalToRow(a->t))
 int hellm_mult(hellm_hemmer *h, const hellm_ct *a, const hellm_ct *b, hellm_ct **out) {
     FACADE_TRY
     need(h && a && b && out, "null argument");
-    hellm_ct *r = new hellm_ct{a->t};
+    hellm_ct *r = like(a);
     h->m->getEval().mult(a->t.get(), b->t.get(), r->t.get());
     *out = r;
     FACADE_CATCH
@@ -534,7 +536,7 @@ int hellm_mult(hellm_hemmer *h, const hellm_ct *a, const hellm_ct *b, hellm_ct *
 int hellm_mult_const(hellm_hemmer *h, const hellm_ct *a, double re, double im, hellm_ct **out) {
     FACADE_TRY
     need(h && a && out, "null argument");
-    hellm_ct *r = new hellm_ct{a->t};
+    hellm_ct *r = like(a);
     h->m->getEval().mult(a->t.get(), HEaaN::Complex(re, im), r->t.get());
     *out = r;
     FACADE_CATCH
@@ -542,7 +544,7 @@ int hellm_mult_const(hellm_hemmer *h, const hellm_ct *a, double re, double im, h
 int hellm_add_const(hellm_hemmer *h, const hellm_ct *a, double re, double im, hellm_ct **out) {
     FACADE_TRY
     need(h && a && out, "null argument");
-    hellm_ct *r = new hellm_ct{a->t};
+    hellm_ct *r = like(a);
     h->m->getEval().add(a->t.get(), HEaaN::Complex(re, im), r->t.get());
     *out = r;
     FACADE_CATCH
@@ -550,7 +552,7 @@ int hellm_add_const(hellm_hemmer *h, const hellm_ct *a, double re, double im, he
 int hellm_add(hellm_hemmer *h, const hellm_ct *a, const hellm_ct *b, hellm_ct **out) {
     FACADE_TRY
     need(h && a && b && out, "null argument");
-    hellm_ct *r = new hellm_ct{a->t};
+    hellm_ct *r = like(a);
     h->m->getEval().add(a->t.get(), b->t.get(), r->t.get());
     *out = r;
     FACADE_CATCH
@@ -558,7 +560,7 @@ int hellm_add(hellm_hemmer *h, const hellm_ct *a, const hellm_ct *b, hellm_ct **
 int hellm_level_down(hellm_hemmer *h, const hellm_ct *a, uint32_t target, hellm_ct **out) {
     FACADE_TRY
     need(h && a && out, "null argument");
-    hellm_ct *r = new hellm_ct{a->t};
+    hellm_ct *r = like(a);
     h->m->getEval().levelDown(a->t.get(), target, r->t.get());
     *out = r;
     FACADE_CATCH
@@ -599,7 +601,7 @@ int hellm_eval_chebyshev(hellm_hemmer *h, const hellm_ct *a, const double *coeff
                          double multiplier, hellm_ct **out) {
     FACADE_TRY
     need(h && a && coeffs && out, "null argument");
-    hellm_ct *r = new hellm_ct{a->t};
+    hellm_ct *r = like(a);
     r->t.get() = HEaaN::Math::evaluateChebyshevExpansion(
         h->m->getEval(), h->m->getBtp(), a->t.get(),
         HEaaN::Math::ChebyshevCoefficients(std::vector<HEaaN::Real>(coeffs, coeffs + n_coeffs), baby_steps), multiplier);
@@ -610,7 +612,7 @@ int hellm_eval_chebyshev(hellm_hemmer *h, const hellm_ct *a, const double *coeff
 int hellm_linear_transform(hellm_hemmer *h, const hellm_ct *a, double left, double right, hellm_ct **out) {
     FACADE_TRY
     need(h && a && out, "null argument");
-    hellm_ct *r = new hellm_ct{a->t};
+    hellm_ct *r = like(a);
     r->t.get() = HEaaN::Math::linearTransform(h->m->getEval(), h->m->getBtp(), a->t.get(),
                                               HEaaN::Math::InputInterval(left, right));
     *out = r;
@@ -801,7 +803,7 @@ int hellm_lora_rank2(hellm_hemmer *h, int up, const hellm_ct *const *cts, uint32
     }
     std::vector<HELLM::CtxtTensor> r =
         up ? h->m->loraRank2Up(v, weight->t, n_out, weight_level) : h->m->loraRank2Down(v, weight->t, weight_level);
-    for (size_t i = 0; i < r.size(); i++) out[i] = new hellm_ct{r[i]};
+    for (size_t i = 0; i < r.size(); i++) out[i] = new hellm_ct{std::move(r[i])};
     FACADE_CATCH
 }
 

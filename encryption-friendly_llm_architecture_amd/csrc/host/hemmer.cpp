@@ -388,7 +388,7 @@ void HEMMer::transposeInplace(CtxtTensor &t, u64 target_level) const {
         if (target_level > 0) eval_.levelDown(t.get(), 1 + target_level, t.get());
         const TileTensorShape shape(t.getWidth(), t.getHeight(), t.getBlockWidth());
         Ciphertext out = matrix_transformer.diagonalTransformFused(eval_, t.get(), MaskKind::DiagonalSigned, shape);
-        t = CtxtTensor(shape, out);
+        t = CtxtTensor(shape, std::move(out));
         return;
     }
     ensureRotationKeys(transformRotations(MaskKind::Diagonal, t.getBlockWidth()));
@@ -474,7 +474,7 @@ void HEMMer::splitInTwo(CtxtTensor &t, CtxtTensor &t1, CtxtTensor &t2) const {
 CtxtTensor HEMMer::diagonalToColumn(const CtxtTensor &a) const {
     ensureRotationKeys(transformRotations(MaskKind::Horizontal, a.getBlockWidth()));
     if (fused_) {   // one stage (the level contract: in at l, out at l - 1) through the batched launches
-        CtxtTensor res(a);
+        CtxtTensor res(context_, a.getShape());
         res.get() = matrix_transformer.diagonalTransformFused(eval_, a.get(), MaskKind::Horizontal, a.getShape());
         return res;
     }
@@ -483,7 +483,7 @@ CtxtTensor HEMMer::diagonalToColumn(const CtxtTensor &a) const {
 CtxtTensor HEMMer::diagonalToRow(const CtxtTensor &b) const {
     ensureRotationKeys(transformRotations(MaskKind::Vertical, b.getBlockWidth()));
     if (fused_) {
-        CtxtTensor res(b);
+        CtxtTensor res(context_, b.getShape());
         res.get() = matrix_transformer.diagonalTransformFused(eval_, b.get(), MaskKind::Vertical, b.getShape());
         return res;
     }
@@ -604,7 +604,7 @@ CtxtTensor HEMMer::packedMatMul(const CtxtTensor &a, const CtxtTensor &b, u64 T)
 CtxtTensor HEMMer::packedMatMulPre(const CtxtTensor &a, u64 T) const {
     ensureRotationKeys(transformRotations(MaskKind::PackedHorizontal, a.getBlockWidth()));
     if (fused_ && a.getLevel() >= T + 3) {   // sigma through the batched launches (two stages with a level to spare)
-        CtxtTensor res(a);
+        CtxtTensor res(context_, a.getShape());
         res.get() = matrix_transformer.lowerAndTransformFused(eval_, a.get(), MaskKind::PackedHorizontal, a.getShape(), T + 2);
         return res;
     }
@@ -625,7 +625,7 @@ void HEMMer::packedMatMulPreRot(const CtxtTensor &a, std::vector<Ciphertext> &tm
 CtxtTensor HEMMer::packedMatMulPreRev(const CtxtTensor &b, u64 T) const {
     ensureRotationKeys(transformRotations(MaskKind::PackedVertical, b.getBlockWidth()));
     if (fused_ && b.getLevel() >= T + 2) {   // tau through the batched launches (two stages with a level to spare)
-        CtxtTensor res(b);
+        CtxtTensor res(context_, b.getShape());
         res.setShape(pow2ceil(b.getHeight()), b.getWidth());
         res.get() = matrix_transformer.lowerAndTransformFused(eval_, b.get(), MaskKind::PackedVertical, res.getShape(), T + 1);
         return res;
@@ -660,7 +660,7 @@ CtxtTensor HEMMer::matMulReUse(const std::vector<Ciphertext> &tmp, const PtxtTen
 CtxtTensor HEMMer::matMulPreRev(const CtxtTensor &b, u64 T) const {
     ensureRotationKeys(transformRotations(MaskKind::Vertical, b.getBlockWidth()));
     if (fused_ && b.getLevel() >= T + 2) {
-        CtxtTensor res(b);
+        CtxtTensor res(context_, b.getShape());
         res.get() = matrix_transformer.lowerAndTransformFused(eval_, b.get(), MaskKind::Vertical, b.getShape(), T + 1);
         return res;
     }
@@ -838,7 +838,7 @@ CtxtTensor HEMMer::repackToMultiRow(const CtxtTensor &t, u64 out_row_block) cons
     return ret;
 }
 CtxtTensor HEMMer::getLowColBlock(const CtxtTensor &t, u64 col_block) const {
-    CtxtTensor res{t};
+    CtxtTensor res(context_, t.getShape());
     eval_.mult(t.get(),
                lowColBlockMask(log_slots_, (u64)t.getHeight(), (u64)t.getWidth(), (u64)t.getBlockWidth(), col_block,
                                LOW_DIM, true),
@@ -846,7 +846,7 @@ CtxtTensor HEMMer::getLowColBlock(const CtxtTensor &t, u64 col_block) const {
     return res;
 }
 CtxtTensor HEMMer::getLowRowBlock(const CtxtTensor &t, u64 row_block) const {
-    CtxtTensor res{t};
+    CtxtTensor res(context_, t.getShape());
     eval_.mult(t.get(), lowRowBlockMask(log_slots_, (u64)t.getBlockWidth(), row_block, LOW_DIM, (u64)t.getBlockWidth()),
                res.get());
     return res;
@@ -984,7 +984,7 @@ std::vector<CtxtTensor> HEMMer::loraRank2Up(const std::vector<CtxtTensor> &xa_in
 
 // x + conj(x) = 2 Re(x)
 CtxtTensor HEMMer::repackCC(CtxtTensor &t) const {
-    CtxtTensor out(t);
+    CtxtTensor out(context_, t.getShape());
     eval_.conjugate(t.get(), out.get());
     eval_.add(t.get(), out.get(), out.get());
     return out;
@@ -996,13 +996,13 @@ PtxtTensor HEMMer::complexPacking(const PtxtTensor &a, const PtxtTensor &b) cons
     return PtxtTensor(a.getShape(), endec_.encode(ma, std::min(a.getLevel(), b.getLevel())));
 }
 CtxtTensor HEMMer::complexPacking(const CtxtTensor &a, const CtxtTensor &b) const {
-    CtxtTensor res(b);
+    CtxtTensor res(context_, b.getShape());
     eval_.multImagUnit(b.get(), res.get());
     eval_.add(a.get(), res.get(), res.get());
     return res;
 }
 CtxtTensor HEMMer::complexPackingRev(const CtxtTensor &a, const CtxtTensor &b) const {
-    CtxtTensor res(b);
+    CtxtTensor res(context_, b.getShape());
     eval_.multImagUnit(b.get(), res.get());
     eval_.sub(a.get(), res.get(), res.get());
     return res;

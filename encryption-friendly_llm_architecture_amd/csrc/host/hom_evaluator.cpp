@@ -128,9 +128,10 @@ void HomEvaluator::add(const Ciphertext &a, const Plaintext &b, Ciphertext &out)
     const u64 occ = std::max(a.occupied_, b.occupied_);
     OutSlot o(ctx_, out, a.num_poly_, a.level_, a.rescale_counter_, true, {&a});
     Ciphertext &r = o.get();
-    if (r.buf_.data() != a.buf_.data())
-        (void)hipMemcpyAsync(r.buf_.data(), a.buf_.data(), a.buf_.words() * 8, hipMemcpyDeviceToDevice, ctx_->stream());
-    ck(hemm_pointwise(ctx_->dev, HEMM_ADD, r.buf_.data(), 0, b.buf_.data(), 0, r.buf_.data(), 0,
+    if (r.buf_.data() != a.buf_.data())   // the other polynomials pass through
+        (void)hipMemcpyAsync(r.buf_.data() + r.polyStride(), a.buf_.data() + a.polyStride(),
+                             (a.num_poly_ - 1) * a.polyStride() * 8, hipMemcpyDeviceToDevice, ctx_->stream());
+    ck(hemm_pointwise(ctx_->dev, HEMM_ADD, a.buf_.data(), 0, b.buf_.data(), 0, r.buf_.data(), 0,
                       (uint32_t)a.level_ + 1, 0, 1, nullptr));
     o.commit(occ);
 }
@@ -150,10 +151,11 @@ void HomEvaluator::add(const Ciphertext &a, const Complex &cst, Ciphertext &out)
     const u64 occ = (re != 0 || im != 0) ? (u64)ctx_->N / 2 : a.occupied_;
     OutSlot o(ctx_, out, a.num_poly_, a.level_, a.rescale_counter_, true, {&a});
     Ciphertext &r = o.get();
-    if (r.buf_.data() != a.buf_.data())
-        (void)hipMemcpyAsync(r.buf_.data(), a.buf_.data(), a.buf_.words() * 8, hipMemcpyDeviceToDevice, ctx_->stream());
+    if (r.buf_.data() != a.buf_.data())   // the other polynomials pass through
+        (void)hipMemcpyAsync(r.buf_.data() + r.polyStride(), a.buf_.data() + a.polyStride(),
+                             (a.num_poly_ - 1) * a.polyStride() * 8, hipMemcpyDeviceToDevice, ctx_->stream());
     const auto rr = int_residues(ctx_, re, a.level_ + 1), ri = int_residues(ctx_, im, a.level_ + 1);
-    ck(hemm_add_scalar(ctx_->dev, r.buf_.data(), rr.data(), im != 0 ? ri.data() : nullptr, r.buf_.data(),
+    ck(hemm_add_scalar(ctx_->dev, a.buf_.data(), rr.data(), im != 0 ? ri.data() : nullptr, r.buf_.data(),
                        (uint32_t)a.level_ + 1, 0, nullptr));
     o.commit(occ);
 }
@@ -366,11 +368,10 @@ void HomEvaluator::multRealBatch(const Ciphertext &a, const std::vector<Real> &c
                            0, 2, nullptr));
     }
     rescale_many(ctx_, t.data(), low.data(), nq, 2 * n);
+    auto parts = DeviceBuffer::split(std::move(low), n);
     for (size_t i = 0; i < n; i++) {
         res.emplace_back(ctx_);
-        res.back().allocate(2, lvl - 1, 0);
-        (void)hipMemcpyAsync(res.back().buf_.data(), low.data() + i * 2 * lvl * N, 2 * lvl * N * 8, hipMemcpyDeviceToDevice,
-                             ctx_->stream());
+        res.back().adopt(std::move(parts[i]), 2, lvl - 1, 0);
         res.back().occupied_ = a.occupied_;
     }
     out = std::move(res);
@@ -433,11 +434,10 @@ void HomEvaluator::multBatch(const std::vector<const Ciphertext *> &a, const std
     ck(hemm_hoisted_moddown(ctx_->dev, terms.data(), off.data(), (uint32_t)n, (uint32_t)nq, 0, 0, y.data(), r.data(), nq * N,
                             ws2.data(), nullptr));
     rescale_many(ctx_, r.data(), low.data(), nq, 2 * n);
+    auto parts = DeviceBuffer::split(std::move(low), n);
     for (size_t i = 0; i < n; i++) {
         res.emplace_back(ctx_);
-        res.back().allocate(2, lvl - 1, 0);
-        (void)hipMemcpyAsync(res.back().buf_.data(), low.data() + i * 2 * lvl * N, 2 * lvl * N * 8, hipMemcpyDeviceToDevice,
-                             ctx_->stream());
+        res.back().adopt(std::move(parts[i]), 2, lvl - 1, 0);
         res.back().occupied_ = std::min(a[i]->occupied_, b[i]->occupied_);
     }
     out = std::move(res);

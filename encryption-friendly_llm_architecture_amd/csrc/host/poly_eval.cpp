@@ -195,8 +195,8 @@ Value productTree(const HomEvaluator &eval, std::vector<Ciphertext> &pw, const R
         }
     }
     auto next_power = [&](const Ciphertext &square) {   // T_{2m} = 2 T_m^2 - 1
-        Ciphertext p(square);
-        eval.add(p, p, p);
+        Ciphertext p(ctx);
+        eval.add(square, square, p);
         eval.add(p, Complex(-1.0, 0.0), p);
         pw.push_back(std::move(p));
     };
@@ -289,7 +289,7 @@ Ciphertext evaluateChebyshevExpansion(const HomEvaluator &eval, const Bootstrapp
     pw.push_back(ctxt);
     Value v = productTree(eval, pw, e.data(), len);
     if (!v.has_ct) throw std::invalid_argument("[evaluateChebyshevExpansion] constant polynomial");
-    return v.ct;
+    return std::move(v.ct);
 }
 
 }  // namespace Math
