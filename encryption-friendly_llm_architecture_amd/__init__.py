@@ -63,6 +63,7 @@ def _declare(L):
     L.hemm_pointwise.argtypes = [vp, ci, vp, sz, vp, sz, vp, sz, u32, ci, u32, vp]
     L.hemm_mul_scalar.argtypes = [vp, vp, sz, u64p, vp, sz, u32, ci, u32, vp]
     L.hemm_encode.argtypes = [vp, vp, ctypes.c_double, u32, ci, u32, vp, vp]
+    L.hemm_encode_from.argtypes = [vp, vp, ctypes.c_double, u32, ci, u32, vp, vp, vp]
     L.hemm_decode.argtypes = [vp, vp, u32, ctypes.c_double, vp, vp, vp]
     L.hemm_mul_imag_unit.argtypes = [vp, vp, sz, vp, sz, u32, u32, vp]
     L.hemm_tensor.argtypes = [vp, vp, sz, vp, sz, vp, sz, u32, ci, vp]
@@ -152,11 +153,12 @@ class Context:
     def encode(self, slots, scale, nq, with_p=False):
         """slots: complex128 CUDA tensor [n_msgs][N/2] (or [N/2]) -> int64 [n_msgs][nq (+ n_p)][N] (NTT form)."""
         import torch
-        z = slots.reshape(-1, self.N // 2).clone().contiguous()
+        z = slots.reshape(-1, self.N // 2).contiguous()
         limbs = nq + (self.nP if with_p else 0)
         out = torch.empty((z.shape[0], limbs, self.N), dtype=torch.int64, device=z.device)
-        check(lib().hemm_encode(self.h, vp(z.data_ptr()), ctypes.c_double(scale), nq, int(with_p), z.shape[0],
-                                vp(out.data_ptr()), vp(0)))
+        ws = torch.empty((z.shape[0], self.N), dtype=torch.int64, device=z.device)
+        check(lib().hemm_encode_from(self.h, vp(z.data_ptr()), ctypes.c_double(scale), nq, int(with_p), z.shape[0],
+                                     vp(ws.data_ptr()), vp(out.data_ptr()), vp(0)))
         return out
 
     def decode(self, pt, scale, n_limbs=2):

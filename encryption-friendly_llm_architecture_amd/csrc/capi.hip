@@ -202,7 +202,45 @@ int hemm_encode(hemm_context *ctx, double *slots, double scale, uint32_t nq, int
     LimbList ll = chain_limbs(ctx, nq, with_p, &nl);
     need(slots && out && n_msgs >= 1, "null operand");
     need(scale > 0, "scale must be positive");
-    launch_encode(ctx, slots, scale, ll, nl, (int)n_msgs, (u64 *)out, on_stream(ctx, stream));
+    launch_encode(ctx, slots, nullptr, 0, scale, ll, nl, (int)n_msgs, (u64 *)slots, (u64 *)out, on_stream(ctx, stream));
+    check_launch();
+    HEMM_CATCH
+}
+int hemm_encode_from(hemm_context *ctx, const double *slots, double scale, uint32_t nq, int with_p, uint32_t n_msgs,
+                     uint64_t *workspace, uint64_t *out, void *stream) {
+    HEMM_TRY
+    int nl;
+    LimbList ll = chain_limbs(ctx, nq, with_p, &nl);
+    need(slots && workspace && out && n_msgs >= 1, "null operand");
+    need(scale > 0, "scale must be positive");
+    launch_encode(ctx, slots, nullptr, 0, scale, ll, nl, (int)n_msgs, (u64 *)workspace, (u64 *)out, on_stream(ctx, stream));
+    check_launch();
+    HEMM_CATCH
+}
+int hemm_encode_reals(hemm_context *ctx, const double *values, size_t count, double scale, uint32_t nq, int with_p,
+                      uint64_t *workspace, uint64_t *out, void *stream) {
+    HEMM_TRY
+    int nl;
+    LimbList ll = chain_limbs(ctx, nq, with_p, &nl);
+    need(values && workspace && out, "null operand");
+    need(ctx->logN >= 10 && count <= (size_t)ctx->N / 2, "needs N >= 1024 and at most N / 2 values");
+    need(scale > 0, "scale must be positive");
+    launch_encode(ctx, nullptr, values, count, scale, ll, nl, 1, (u64 *)workspace, (u64 *)out, on_stream(ctx, stream));
+    check_launch();
+    HEMM_CATCH
+}
+int hemm_encrypt_reals(hemm_context *ctx, const double *values, size_t count, double scale, uint32_t nq, const uint64_t *sk,
+                       uint64_t a_base, uint64_t error_key, uint64_t *workspace, uint64_t *ct, size_t ct_stride, void *stream) {
+    HEMM_TRY
+    int nl;
+    LimbList ll = chain_limbs(ctx, nq, 0, &nl);
+    need(values && sk && workspace && ct, "null operand");
+    need(ctx->logN >= 10 && count <= (size_t)ctx->N / 2, "needs N >= 1024 and at most N / 2 values");
+    need(ct_stride >= (size_t)nq * ctx->N, "the polynomials of the ciphertext overlap");
+    need(scale > 0, "scale must be positive");
+    const EncryptTail enc{(u64 *)ct, (u64 *)ct + ct_stride, (const u64 *)sk, a_base};
+    launch_encode(ctx, nullptr, values, count, scale, ll, nl, 1, (u64 *)workspace, (u64 *)ct, on_stream(ctx, stream), &enc,
+                  error_key);
     check_launch();
     HEMM_CATCH
 }
@@ -213,7 +251,20 @@ int hemm_decode(hemm_context *ctx, const uint64_t *pt, uint32_t n_limbs, double 
     need(pt && workspace && slots, "null operand");
     need(n_limbs >= 1 && n_limbs <= 2 && (int)n_limbs <= ctx->nQ, "decode reads one or two limbs");
     need(scale > 0, "scale must be positive");
-    launch_decode(ctx, (const u64 *)pt, (int)n_limbs, scale, (u64 *)workspace, slots, on_stream(ctx, stream));
+    launch_decode(ctx, (const u64 *)pt, nullptr, nullptr, (int)n_limbs, scale, (u64 *)workspace, slots, nullptr, 0,
+                  on_stream(ctx, stream));
+    check_launch();
+    HEMM_CATCH
+}
+int hemm_decrypt_reals(hemm_context *ctx, const uint64_t *ct, size_t ct_stride, const uint64_t *sk, uint32_t n_limbs,
+                       double scale, uint64_t *workspace, double *values, size_t count, void *stream) {
+    HEMM_TRY
+    need(ctx && ct && sk && workspace && values, "null operand");
+    need(n_limbs >= 1 && n_limbs <= 2 && (int)n_limbs <= ctx->nQ, "decode reads one or two limbs");
+    need(ctx->logN >= 10 && count <= (size_t)ctx->N / 2, "needs N >= 1024 and at most N / 2 values");
+    need(scale > 0, "scale must be positive");
+    launch_decode(ctx, (const u64 *)ct, (const u64 *)ct + ct_stride, (const u64 *)sk, (int)n_limbs, scale, (u64 *)workspace,
+                  (double *)(workspace + (size_t)n_limbs * ctx->N), values, count, on_stream(ctx, stream));
     check_launch();
     HEMM_CATCH
 }

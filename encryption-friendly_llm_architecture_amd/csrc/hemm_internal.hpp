@@ -141,14 +141,35 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
                           int n_limbs, int n_polys, size_t poly_stride, hipStream_t s, const u64 *ep_minuend = nullptr,
                           size_t ep_minuend_stride = 0, u64 *ep_out = nullptr, size_t ep_out_stride = 0,
                           const void *ep_cst_dev = nullptr);
-// One-launch transforms (2^10 .. 2^14 points).  cs != nullptr: the inputs are its conversions; out != nullptr: out =
-// (minuend - transform) * cst[limb]; from != nullptr: the inverse reads there instead of data, through `galois` if != 0.
-void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
-                         size_t poly_stride, hipStream_t s, const ConvSources *cs, const u64 *minuend, size_t minuend_stride,
-                         u64 *out, size_t out_stride, const void *cst_dev);
-void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
-                         size_t poly_stride, hipStream_t s, const void *final_scale, const u64 *from, size_t from_stride,
-                         u32 galois);
+// A forward transform of N >= 2^10 whose input is the rounded coefficients of an encoding (signed, [n_polys][stride >= N], the
+// same for every limb; plus, with_error, the error of a stream), reduced while the first pass loads them.  enc: the second
+// pass ends in an encryption instead of storing the transform (data is then only a workspace): a uniform from the streams
+// sm64(sm64(a_base + prime)), b = transform - a s, b and a laid out like data, sk [prime][N].  false: no such form.
+struct LiftSource {
+    const long long *coef;
+    size_t stride;
+    u64 error_key;
+    int with_error;
+};
+struct EncryptTail {
+    u64 *b, *a;
+    const u64 *sk;
+    u64 a_base;
+};
+bool launch_ntt_lifted(const hemm_context *c, const LiftSource &ls, u64 *data, const LimbList &ll, int n_limbs, int n_polys,
+                       size_t poly_stride, hipStream_t s, const EncryptTail *enc);
+// data[j] = inverse transform of b[j] + a[j] s for the first n_limbs chain primes (all [n_limbs][N])
+bool launch_intt_decrypt(const hemm_context *c, const u64 *b, const u64 *a, const u64 *sk, u64 *data, int n_limbs, hipStream_t s);
+// slots: [n_msgs][N/2] complex doubles, or re: the real parts of the first `count` slots of one message, in device memory or
+// in host memory the device reads; work: [n_msgs][N] words, may be `slots`; out: [n_msgs][n_limbs][N], with enc a
+// workspace (which may be enc->b).  re and enc need N >= 2^10.
+void launch_encode(const hemm_context *c, const double *slots, const double *re, size_t count, double scale, const LimbList &ll,
+                   int n_limbs, int n_msgs, u64 *work, u64 *out, hipStream_t s, const EncryptTail *enc = nullptr,
+                   u64 error_key = 0);
+// pt: [>= n_limbs][N]; a != nullptr: pt is the first polynomial of a ciphertext, a its second.  slots: [N/2] complex doubles; re
+// != nullptr: slots is a workspace and the real parts of the first `count` slots go to re.  a and re need N >= 2^10.
+void launch_decode(const hemm_context *c, const u64 *pt, const u64 *a, const u64 *sk, int n_limbs, double scale, u64 *work,
+                   double *slots, double *re, size_t count, hipStream_t s);
 // out[p][j] = (y[p][j] - conversion of the n_src listed limbs of y[p] to prime j) * cst[j], j < nq_out, as inverse row
 // pass (in place on the listed limbs), one column-slab kernel (second inverse pass, conversion as lazy dot products, first
 // forward pass into conv[n_polys][nq_out][N]) and forward row pass with the fused tail.  final_scale / hat / cst: device
@@ -171,9 +192,6 @@ void launch_mul_scalar(const hemm_context *c, const u64 *a, size_t a_stride, con
                        size_t out_stride, const LimbList &ll, int n_limbs, int n_polys, hipStream_t s);
 void launch_add_scalar(const hemm_context *c, const u64 *a, const u64 *re, const u64 *im, u64 *out, const LimbList &ll,
                        int n_limbs, hipStream_t s);
-void launch_encode(const hemm_context *c, double *slots, double scale, const LimbList &ll, int n_limbs, int n_msgs, u64 *out,
-                   hipStream_t s);
-void launch_decode(const hemm_context *c, const u64 *pt, int n_limbs, double scale, u64 *work, double *slots, hipStream_t s);
 void hemm_embedding_tables_free(const hemm_context *c);
 void launch_zero(const hemm_context *c, u64 *out, size_t words, hipStream_t s);
 void launch_mul_imag(const hemm_context *c, const u64 *a, size_t a_stride, u64 *out, size_t out_stride,

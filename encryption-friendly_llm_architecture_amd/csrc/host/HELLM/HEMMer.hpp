@@ -53,6 +53,7 @@ public:
     void save(const std::string &keys_path);
 
     Message message2(const Matrix &a, const Matrix &b) const;
+    void checkPair(i64 rows_a, i64 cols_a, i64 rows_b, i64 cols_b) const;
     PtxtTensor encode(const Matrix &data, u64 level = 0) const;
     PtxtTensor encode2(const Matrix &a, const Matrix &b, u64 level = 0) const;
     Message msgDiagonalToRow4(const Matrix &w1, const Matrix &w2, const Matrix &w3, const Matrix &w4) const;
@@ -89,6 +90,9 @@ public:
                                     u64 level = 0) const;
     CtxtTensor encrypt(const Matrix &data) const;
     CtxtTensor encrypt2(const Matrix &a, const Matrix &b) const;
+    // from and to row-major arrays; b: the second matrix of a pair, or nullptr
+    CtxtTensor encrypt(const double *a, const double *b, i64 rows, i64 cols) const;
+    void decrypt(const CtxtTensor &t, double *a, double *b) const;
     Matrix decrypt(const CtxtTensor &t) const;
     std::vector<Matrix> decrypt2(const CtxtTensor &t) const;
 

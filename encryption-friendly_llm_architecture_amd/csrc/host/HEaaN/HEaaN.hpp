@@ -271,6 +271,9 @@ public:
     Plaintext encode(const Message &msg, u64 level, u64 rescale_counter = 0) const;
     Plaintext encode(const Message &msg) const;
     Message decode(const Plaintext &pt) const;
+    // a message whose first `count` slots are these real numbers and whose others are zero; `values` is memory the device
+    // reads (device or pinned) and stays as it is until the queued work is done.  N >= 1024
+    Plaintext encodeReals(const Real *values, size_t count, u64 level) const;
     // plaintext over the extended basis (limbs q_0..q_level then the special primes), for masks that
     // are applied before ModDown
     Plaintext encodeExtended(const Message &msg, u64 level) const;
@@ -286,6 +289,8 @@ public:
     explicit Encryptor(const Context &c) : ctx_(c) {}
     void encrypt(const Plaintext &pt, const SecretKey &sk, Ciphertext &ct) const;
     void encrypt(const Message &msg, const SecretKey &sk, Ciphertext &ct) const;
+    // EnDecoder::encodeReals at the top level and its encryption in one chain of launches (same residues)
+    void encryptReals(const Real *values, size_t count, const SecretKey &sk, Ciphertext &ct) const;
 
 private:
     Context ctx_;
@@ -296,6 +301,9 @@ public:
     explicit Decryptor(const Context &c) : ctx_(c) {}
     void decrypt(const Ciphertext &ct, const SecretKey &sk, Message &msg) const;
     void decrypt(const Ciphertext &ct, const SecretKey &sk, Plaintext &pt) const;
+    // the real parts of the first `count` slots of a two-polynomial ciphertext to memory the device writes (complete when
+    // the context's stream is).  N >= 1024
+    void decryptReals(const Ciphertext &ct, const SecretKey &sk, Real *values, size_t count) const;
 
 private:
     Context ctx_;

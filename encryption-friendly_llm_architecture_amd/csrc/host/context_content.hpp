@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <condition_variable>
 #include <map>
 #include <mutex>
 #include <string>
@@ -99,6 +100,48 @@ struct ContextContent {
         trace_marks.clear();
     }
 
+    // Pinned host memory for the values of one message ([N/2] doubles), which kernels read and write in place: a transfer
+    // needs no copy command and no pageable staging.  At most STAGES of them, kept for the context's life.  A user holds one
+    // from takeStage() to giveStage(); `queued` says that work on `stream` still reads it, which the next user waits for.
+    struct Stage {
+        double *values = nullptr;
+        hipEvent_t done = nullptr;
+        bool pending = false;
+    };
+    static constexpr size_t STAGES = 8;
+    std::vector<Stage> stages;          // free ones, the longest unused first
+    size_t stages_made = 0;
+    std::condition_variable stage_free;
+    Stage takeStage() {
+        std::unique_lock<std::mutex> lk(mu);
+        if (stages.empty() && stages_made < STAGES) {
+            Stage s;
+            if (hipHostMalloc((void **)&s.values, N / 2 * sizeof(double)) != hipSuccess)
+                throw RuntimeException("hipHostMalloc failed");
+            if (hipEventCreateWithFlags(&s.done, hipEventDisableTiming) != hipSuccess) {
+                (void)hipHostFree(s.values);
+                throw RuntimeException("hipEventCreateWithFlags failed");
+            }
+            stages_made++;
+            return s;
+        }
+        stage_free.wait(lk, [&] { return !stages.empty(); });
+        Stage s = stages.front();
+        stages.erase(stages.begin());
+        lk.unlock();
+        if (s.pending) (void)hipEventSynchronize(s.done);
+        s.pending = false;
+        return s;
+    }
+    void giveStage(Stage s, bool queued) {
+        if (queued) s.pending = hipEventRecord(s.done, stream()) == hipSuccess;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            stages.push_back(s);
+        }
+        stage_free.notify_one();
+    }
+
     u64 prime(size_t i) const { return i < nQ ? q[i] : p[i - nQ]; }
     u64 *alloc(size_t words) {
         {
@@ -136,6 +179,10 @@ struct ContextContent {
         for (auto &kv : pool) (void)hipFree(kv.second);
         for (auto &kv : parked) (void)hipFree(kv.second);
         for (auto &kv : captured) (void)hipFree(kv.second);
+        for (auto &st : stages) {
+            (void)hipEventDestroy(st.done);
+            (void)hipHostFree(st.values);
+        }
         if (side) (void)hipStreamDestroy(side);
         if (ev_fork) (void)hipEventDestroy(ev_fork);
         if (ev_join) (void)hipEventDestroy(ev_join);
@@ -144,5 +191,24 @@ struct ContextContent {
         if (dev) hemm_context_destroy(dev);
     }
 };
+
+// a stage for as long as the object lives; read(): queued work reads it, so the next user has to wait for that
+class HostStage {
+  public:
+    explicit HostStage(const Context &c) : c_(c), s_(c->takeStage()) {}
+    ~HostStage() { c_->giveStage(s_, queued_); }
+    HostStage(const HostStage &) = delete;
+    HostStage &operator=(const HostStage &) = delete;
+    double *values() const { return s_.values; }
+    void read() { queued_ = true; }
+
+  private:
+    Context c_;
+    ContextContent::Stage s_;
+    bool queued_ = false;
+};
+// whether messages of this context go through a stage (a sequence being recorded reads its own copy: a replay would find
+// another message in the stage)
+inline bool stageable(const Context &c) { return c->logN >= 10 && !c->capture_open; }
 
 }  // namespace HEaaN

@@ -825,6 +825,25 @@ Message EnDecoder::decode(const Plaintext &pt) const {
     return m;
 }
 
+namespace {
+// slots up to the last one that is not zero
+u64 occupied_reals(const Real *v, size_t count) {
+    while (count > 0 && v[count - 1] == 0) count--;
+    return count;
+}
+}  // namespace
+
+Plaintext EnDecoder::encodeReals(const Real *values, size_t count, u64 level) const {
+    const Context &c = ctx_;
+    if (level >= c->nQ) throw RuntimeException("encode: level above the encryption level");
+    Plaintext pt(c);
+    pt.allocate(level, 0);
+    DeviceBuffer ws(c, c->N);
+    ck(hemm_encode_reals(c->dev, values, count, c->delta[level], (uint32_t)level + 1, 0, ws.data(), pt.buf_.data(), nullptr));
+    pt.occupied_ = occupied_reals(values, count);
+    return pt;
+}
+
 // ---- encrypt / decrypt -------------------------------------------------------------------------------
 void Encryptor::encrypt(const Plaintext &pt, const SecretKey &sk, Ciphertext &ct) const {
     const Context &c = ctx_;
@@ -849,6 +868,27 @@ void Encryptor::encrypt(const Plaintext &pt, const SecretKey &sk, Ciphertext &ct
 void Encryptor::encrypt(const Message &msg, const SecretKey &sk, Ciphertext &ct) const {
     EnDecoder ed(ctx_);
     encrypt(ed.encode(msg), sk, ct);
+}
+void Encryptor::encryptReals(const Real *values, size_t count, const SecretKey &sk, Ciphertext &ct) const {
+    const Context &c = ctx_;
+    const u64 level = c->nQ - 1, enc_id = g_enc_counter++;
+    Ciphertext out(c);
+    out.allocate(2, level, 0);
+    DeviceBuffer ws(c, c->N);
+    // limb i of a is drawn from stream_key(seed + id, TAG_ENC_A, i, 0) = sm64(sm64(a_base + i))
+    ck(hemm_encrypt_reals(c->dev, values, count, c->delta[level], (uint32_t)c->nQ, sk.ntt(), sm64(g_seed + enc_id + TAG_ENC_A),
+                          stream_key(g_seed + enc_id, TAG_ENC_E, 0, 0), ws.data(), out.buf_.data(), out.polyStride(), nullptr));
+    out.occupied_ = occupied_reals(values, count);
+    ct = std::move(out);
+}
+void Decryptor::decryptReals(const Ciphertext &ct, const SecretKey &sk, Real *values, size_t count) const {
+    const Context &c = ctx_;
+    if (ct.num_poly_ != 2) throw RuntimeException("decryptReals: the ciphertext must have two polynomials");
+    const uint32_t limbs = ct.level_ >= 1 ? 2 : 1;
+    Real scale = c->delta[ct.level_];
+    for (u64 k = 0; k < ct.rescale_counter_; k++) scale *= c->delta[ct.level_];
+    DeviceBuffer ws(c, (limbs + 1) * c->N);
+    ck(hemm_decrypt_reals(c->dev, ct.buf_.data(), ct.polyStride(), sk.ntt(), limbs, scale, ws.data(), values, count, nullptr));
 }
 void Decryptor::decrypt(const Ciphertext &ct, const SecretKey &sk, Plaintext &pt) const {
     const Context &c = ctx_;

@@ -279,14 +279,14 @@ int hellm_traffic(hellm_hemmer *h, uint64_t *bytes, uint64_t *launches, int rese
 
 int hellm_encrypt(hellm_hemmer *h, const double *m, uint32_t rows, uint32_t cols, hellm_ct **out) {
     FACADE_TRY
-    need(h && out, "null argument");
-    *out = new hellm_ct{h->m->encrypt(mat(m, rows, cols))};
+    need(h && out && m, "null argument");
+    *out = new hellm_ct{h->m->encrypt(m, nullptr, rows, cols)};
     FACADE_CATCH
 }
 int hellm_encrypt2(hellm_hemmer *h, const double *a, const double *b, uint32_t rows, uint32_t cols, hellm_ct **out) {
     FACADE_TRY
-    need(h && out, "null argument");
-    *out = new hellm_ct{h->m->encrypt2(mat(a, rows, cols), mat(b, rows, cols))};
+    need(h && out && a && b, "null argument");
+    *out = new hellm_ct{h->m->encrypt(a, b, rows, cols)};
     FACADE_CATCH
 }
 int hellm_encode(hellm_hemmer *h, const double *m, uint32_t rows, uint32_t cols, uint32_t level, hellm_pt **out) {
@@ -394,16 +394,13 @@ int hellm_ct_load(hellm_hemmer *h, const char *file, hellm_ct **out) {
 int hellm_decrypt(hellm_hemmer *h, const hellm_ct *ct, double *out) {
     FACADE_TRY
     need(h && ct && out, "null argument");
-    Matrix m = h->m->decrypt(ct->t);
-    memcpy(out, m.v.data(), m.v.size() * sizeof(double));
+    h->m->decrypt(ct->t, out, nullptr);
     FACADE_CATCH
 }
 int hellm_decrypt2(hellm_hemmer *h, const hellm_ct *ct, double *out) {
     FACADE_TRY
     need(h && ct && out, "null argument");
-    auto ms = h->m->decrypt2(ct->t);
-    memcpy(out, ms[0].v.data(), ms[0].v.size() * sizeof(double));
-    memcpy(out + ms[0].v.size(), ms[1].v.data(), ms[1].v.size() * sizeof(double));
+    h->m->decrypt(ct->t, out, out + ct->t.getHeight() * ct->t.getWidth());
     FACADE_CATCH
 }
 int hellm_decrypt_slots(hellm_hemmer *h, const hellm_ct *ct, double *re_im) {

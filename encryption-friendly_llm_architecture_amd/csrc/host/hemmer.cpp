@@ -1,10 +1,12 @@
 // HEMMer facade (reference: ciphertext/src/HEMMer.cpp, codec :232-416,:579-638, packing :764-831,
 // matmul entry points :833-880,:964-1124, transpose :1166-1172, masks :2336-2400).
 #include <cmath>
+#include <cstring>
 
 #include <fstream>
 
 #include "HELLM/HEMMer.hpp"
+#include "context_content.hpp"
 
 namespace HELLM {
 
@@ -152,10 +154,13 @@ std::vector<u64> HEMMer::transformRotations(MaskKind kind, i64 width) const {
 }
 
 // ---- codec ---------------------------------------------------------------------------------------------
+void HEMMer::checkPair(i64 rows_a, i64 cols_a, i64 rows_b, i64 cols_b) const {
+    if (rows_a != rows_b || cols_a != cols_b) throw RuntimeException("message2: shapes differ");
+    if ((u64)(2 * rows_a * cols_a) > (u64(1) << log_slots_)) throw RuntimeException("message2: matrices do not fit");
+}
 Message HEMMer::message2(const Matrix &a, const Matrix &b) const {
-    if (a.rows != b.rows || a.cols != b.cols) throw RuntimeException("message2: shapes differ");
+    checkPair(a.rows, a.cols, b.rows, b.cols);
     Message msg(log_slots_, 0);
-    if ((u64)(2 * a.rows * a.cols) > msg.getSize()) throw RuntimeException("message2: matrices do not fit");
     for (i64 r = 0; r < a.rows; r++)
         for (i64 c = 0; c < a.cols; c++) {
             msg[(u64)(r * 2 * a.cols + c)] = a.at(r, c);
@@ -163,17 +168,44 @@ Message HEMMer::message2(const Matrix &a, const Matrix &b) const {
         }
     return msg;
 }
+namespace {
+// the values of one matrix, or of two side by side in rows of twice their width (message2), in slot order
+size_t stageMatrices(double *to, const double *a, const double *b, i64 rows, i64 cols) {
+    const size_t w = (size_t)cols, n = (size_t)rows * w;
+    if (b == nullptr) {
+        memcpy(to, a, n * sizeof(double));
+        return n;
+    }
+    for (size_t r = 0; r < (size_t)rows; r++) {
+        memcpy(to + 2 * r * w, a + r * w, w * sizeof(double));
+        memcpy(to + (2 * r + 1) * w, b + r * w, w * sizeof(double));
+    }
+    return 2 * n;
+}
+}  // namespace
 PtxtTensor HEMMer::encode(const Matrix &data, u64 level) const {
-    Message msg(log_slots_, 0);
-    if (data.v.size() > msg.getSize()) throw RuntimeException("encode: matrix does not fit");
-    for (size_t i = 0; i < data.v.size(); i++) msg[i] = data.v[i];
+    if (data.v.size() > (size_t(1) << log_slots_)) throw RuntimeException("encode: matrix does not fit");
     if (level == 0) level = getEncryptionLevel(context_);
+    if (stageable(context_)) {
+        HostStage st(context_);
+        const size_t count = stageMatrices(st.values(), data.v.data(), nullptr, data.rows, data.cols);
+        st.read();
+        return PtxtTensor(data.rows, data.cols, endec_.encodeReals(st.values(), count, level));
+    }
+    Message msg(log_slots_, 0);
+    for (size_t i = 0; i < data.v.size(); i++) msg[i] = data.v[i];
     return PtxtTensor(data.rows, data.cols, endec_.encode(msg, level));
 }
 PtxtTensor HEMMer::encode2(const Matrix &a, const Matrix &b, u64 level) const {
-    Message msg = message2(a, b);
     if (level == 0) level = getEncryptionLevel(context_);
-    return PtxtTensor(a.rows, a.cols, endec_.encode(msg, level), a.cols * 2);
+    if (stageable(context_)) {
+        checkPair(a.rows, a.cols, b.rows, b.cols);
+        HostStage st(context_);
+        const size_t count = stageMatrices(st.values(), a.v.data(), b.v.data(), a.rows, a.cols);
+        st.read();
+        return PtxtTensor(a.rows, a.cols, endec_.encodeReals(st.values(), count, level), a.cols * 2);
+    }
+    return PtxtTensor(a.rows, a.cols, endec_.encode(message2(a, b), level), a.cols * 2);
 }
 // weight layout of the hoisted plaintext product: 0.5 (W1 - i W3) | 0.5 (W2 - i W4), column j of each
 // half rolled up by j (the tau layout)
@@ -337,36 +369,62 @@ CtxtTensor HEMMer::loadCtxtTensor(const std::string &file) const {
     return t;
 }
 
-CtxtTensor HEMMer::encrypt(const Matrix &data) const {
-    PtxtTensor p = encode(data);
-    CtxtTensor ret(context_, p.getShape());
-    enc_.encrypt(p.get(), sk_, ret.get());
-    return ret;
-}
+CtxtTensor HEMMer::encrypt(const Matrix &data) const { return encrypt(data.v.data(), nullptr, data.rows, data.cols); }
 CtxtTensor HEMMer::encrypt2(const Matrix &a, const Matrix &b) const {
-    PtxtTensor p = encode2(a, b);
-    CtxtTensor ret(context_, p.getShape());
-    enc_.encrypt(p.get(), sk_, ret.get());
+    checkPair(a.rows, a.cols, b.rows, b.cols);
+    return encrypt(a.v.data(), b.v.data(), a.rows, a.cols);
+}
+CtxtTensor HEMMer::encrypt(const double *a, const double *b, i64 rows, i64 cols) const {
+    if ((u64)(rows * cols * (b ? 2 : 1)) > (u64(1) << log_slots_)) throw RuntimeException("encode: matrix does not fit");
+    CtxtTensor ret(context_, b ? TileTensorShape(rows, cols, 2 * cols) : TileTensorShape(rows, cols));
+    if (stageable(context_)) {
+        HostStage st(context_);
+        const size_t count = stageMatrices(st.values(), a, b, rows, cols);
+        st.read();
+        enc_.encryptReals(st.values(), count, sk_, ret.get());
+        return ret;
+    }
+    Message msg(log_slots_, 0);
+    std::vector<double> v((size_t)(rows * cols * (b ? 2 : 1)));
+    stageMatrices(v.data(), a, b, rows, cols);
+    for (size_t i = 0; i < v.size(); i++) msg[i] = v[i];
+    enc_.encrypt(msg, sk_, ret.get());
     return ret;
 }
 Matrix HEMMer::decrypt(const CtxtTensor &t) const {
-    Message msg(log_slots_);
-    dec_.decrypt(t.get(), sk_, msg);
     Matrix m(t.getHeight(), t.getWidth());
-    for (size_t i = 0; i < m.v.size(); i++) m.v[i] = msg[i].real();
+    decrypt(t, m.v.data(), nullptr);
     return m;
 }
 std::vector<Matrix> HEMMer::decrypt2(const CtxtTensor &t) const {
+    std::vector<Matrix> out(2, Matrix(t.getHeight(), t.getWidth()));
+    decrypt(t, out[0].v.data(), out[1].v.data());
+    return out;
+}
+void HEMMer::decrypt(const CtxtTensor &t, double *a, double *b) const {
+    const size_t rows = (size_t)t.getHeight(), w = (size_t)t.getWidth(), count = rows * w * (b ? 2 : 1);
+    auto deal = [&](const double *v) {
+        if (b == nullptr) {
+            memcpy(a, v, count * sizeof(double));
+            return;
+        }
+        for (size_t r = 0; r < rows; r++) {
+            memcpy(a + r * w, v + 2 * r * w, w * sizeof(double));
+            memcpy(b + r * w, v + (2 * r + 1) * w, w * sizeof(double));
+        }
+    };
+    if (stageable(context_) && t.get().getNumPoly() == 2 && count <= (size_t(1) << log_slots_)) {
+        HostStage st(context_);
+        dec_.decryptReals(t.get(), sk_, st.values(), count);
+        if (hipStreamSynchronize(context_->stream()) != hipSuccess) throw RuntimeException("hipStreamSynchronize failed");
+        deal(st.values());
+        return;
+    }
     Message msg(log_slots_);
     dec_.decrypt(t.get(), sk_, msg);
-    const i64 h = t.getHeight(), w = t.getWidth();
-    std::vector<Matrix> out(2, Matrix(h, w));
-    for (i64 r = 0; r < h; r++)
-        for (i64 c = 0; c < w; c++) {
-            out[0].at(r, c) = msg[(u64)(r * 2 * w + c)].real();
-            out[1].at(r, c) = msg[(u64)(r * 2 * w + w + c)].real();
-        }
-    return out;
+    std::vector<double> v(count);
+    for (size_t i = 0; i < count; i++) v[i] = msg[i].real();
+    deal(v.data());
 }
 
 // ---- packing ---------------------------------------------------------------------------------------------

@@ -242,6 +242,39 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
         cols_converted_body<LR, NS>(base, tw, IntFieldT<true>(modq, ninv, ninv_s, fp, prime), lds, src, so, h, n_src, m);
 }
 
+// Forward pass 1 whose input is the rounded coefficients of an encoding, the same for every limb of a polynomial: reduced
+// as they are loaded instead of being written limb by limb and read back.
+template <int LR, class F>
+__device__ __forceinline__ void cols_lifted_body(const __amdgpu_buffer_rsrc_t limb, const Tw *__restrict__ tw_int, const F f,
+                                                 u64 *lds_raw, const LiftSource &ls, const long long *__restrict__ coef,
+                                                 const ModQ m) {
+    typedef Slab<LR> S;
+    typename F::E x[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) x[k] = f.from_canonical(lifted(ls, coef, ((S::rh() + S::Q * k) << 8) + S::col(), m));
+    cols_forward<LR>(limb, (const typename F::W *)tw_int, f, x, (typename F::E *)lds_raw);
+}
+template <int LR>
+__global__ __launch_bounds__(256) void ntt16_cols_lifted_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
+                                                                const ModQ *__restrict__ modq, const double *__restrict__ fp,
+                                                                LimbList ll, LimbList sl, int n_limbs, size_t poly_stride,
+                                                                LiftSource ls) {
+    __shared__ u64 lds[256 * 16];
+    const int limb = blockIdx.y % n_limbs, poly = blockIdx.y / n_limbs;
+    const int prime = ll.idx[limb];
+    const Tw *tw = tw_all + ((size_t)prime << (8 + LR));
+    const __amdgpu_buffer_rsrc_t base = limb_rsrc(
+        data + (size_t)poly * poly_stride + ((size_t)__builtin_amdgcn_readfirstlane((int)sl.idx[limb]) << (8 + LR)));
+    const long long *coef = ls.coef + (size_t)poly * ls.stride;
+    const ModQ m = modq[prime];
+    if (fp[4 * prime] != 0.0)
+        cols_lifted_body<LR>(base, tw, FpField(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
+    else if ((m.q >> 60) != 0)
+        cols_lifted_body<LR>(base, tw, IntField(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
+    else
+        cols_lifted_body<LR>(base, tw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
+}
+
 // ------------------------------------------------------------------------------------------
 // Column-slab kernel of a ModDown (or any conversion of a few source limbs): for one (polynomial, 16-column slab) a
 // workgroup runs the second pass of the inverse transform of every source limb, keeps the canonical coefficients on
@@ -390,7 +423,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 // LR: log2 of the rows of a limb, or 0: taken from the argument (the address arithmetic of N = 2^16 folds into constants:
 // 1 - 1.5 % of a single rotation or ciphertext product)
-template <int LR, bool INV, bool EPI, bool GAL>
+template <int LR, bool INV, int TAIL, int LOAD>
 __global__ __launch_bounds__(256) void ntt16_rows_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
                                                          const Tw *__restrict__ rtw_all,
                                                          const ModQ *__restrict__ modq, const double *__restrict__ fp,
@@ -422,26 +455,47 @@ __global__ __launch_bounds__(256) void ntt16_rows_kernel(u64 *__restrict__ data,
     const u64 *mn = nullptr;
     u64 *o = nullptr;
     Tw cst{0, 0};
-    if (EPI) {
+    RowSecond sec{};
+    if (TAIL != TAIL_NONE) {
         const size_t off = ((size_t)limb << log_n) + ((size_t)r << 8);
-        mn = ep.minuend + (size_t)poly * ep.minuend_stride + off;
         o = ep.out + (size_t)poly * ep.out_stride + off;
-        cst = ep.cst[limb];
+        if (TAIL == TAIL_SUB_SCALE) {
+            mn = ep.minuend + (size_t)poly * ep.minuend_stride + off;
+            cst = ep.cst[limb];
+        } else {
+            sec.out = ep.second_out + (size_t)poly * ep.out_stride + off;
+            sec.key = sm64(sm64(ep.a_base + (u64)prime));
+        }
     }
     const u64 *ld = row;
     if (INV && ep.minuend != nullptr)
-        ld = ep.minuend + (size_t)poly * ep.minuend_stride + ((size_t)sl.idx[limb] << log_n) + (GAL ? 0 : (size_t)r << 8);
-    const u32 gal = GAL ? ep.galois : 0u;
+        ld = ep.minuend + (size_t)poly * ep.minuend_stride + ((size_t)sl.idx[limb] << log_n) + (LOAD == LOAD_ROTATED ? 0 : (size_t)r << 8);
+    if (LOAD == LOAD_DECRYPT)
+        sec.in = ep.second_in + (size_t)poly * ep.minuend_stride + ((size_t)sl.idx[limb] << log_n) + ((size_t)r << 8);
+    if (TAIL == TAIL_ENCRYPT || LOAD == LOAD_DECRYPT) {
+        sec.sk = ep.sk + ((size_t)prime << log_n) + ((size_t)r << 8);
+        sec.m = modq[prime];
+    }
+    const u32 gal = LOAD == LOAD_ROTATED ? ep.galois : 0u;
     if (fp[4 * prime] != 0.0)
-        rows_body<INV, EPI, GAL, false>(row, tw, rtw, FpField(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld, gal);
+        rows_body<INV, TAIL, LOAD, false>(row, tw, rtw, FpField(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld, gal,
+                                            sec);
     else if (INV || (modq[prime].q >> 60) != 0)
-        rows_body<INV, EPI, GAL, false>(row, tw, rtw, IntField(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld, gal);
+        rows_body<INV, TAIL, LOAD, false>(row, tw, rtw, IntField(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld, gal,
+                                            sec);
     else
-        rows_body<INV, EPI, GAL, false>(row, tw, rtw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld,
-                                        gal);
+        rows_body<INV, TAIL, LOAD, false>(row, tw, rtw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld,
+                                            gal, sec);
 }
 
 }  // namespace
+
+// one-launch forms (ntt_limb.hip)
+void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
+                         size_t poly_stride, hipStream_t s, const ConvSources *cs, const LiftSource *ls, const NttEpilogue &ep,
+                         int tail);
+void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
+                         size_t poly_stride, hipStream_t s, const void *final_scale, const NttEpilogue &from, int load);
 
 // ---- launches of single passes (rings of 2^13 points and more) -------------------------------------------------------
 static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbList &ll, const LimbList &sl, int n_limbs,
@@ -465,29 +519,42 @@ static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
     }
 #undef COLS
 }
-// ep: a forward pass with ep.out ends in the fused tail, an inverse one with ep.minuend reads its input there
 static void rows_pass(const hemm_context *c, bool inverse, u64 *d, const LimbList &ll, const LimbList &sl, int n_limbs,
-                      int n_polys, size_t poly_stride, hipStream_t s, const NttEpilogue &ep) {
+                      int n_polys, size_t poly_stride, hipStream_t s, const NttEpilogue &ep, int tail = TAIL_NONE,
+                      int load = LOAD_PLAIN) {
     const dim3 grid((unsigned)(c->N >> 12) * (unsigned)(n_limbs * n_polys)), block(256);
     const int log_r = c->logN - 8;
-#define ROWS(LR, INV, EPI, GAL)                                                                                          \
-    hipLaunchKernelGGL((ntt16_rows_kernel<LR, INV, EPI, GAL>), grid, block, 0, s, d, (const Tw *)(INV ? c->d_iw : c->d_w), \
+#define ROWS(LR, INV, TAIL, LOAD)                                                                                          \
+    hipLaunchKernelGGL((ntt16_rows_kernel<LR, INV, TAIL, LOAD>), grid, block, 0, s, d, (const Tw *)(INV ? c->d_iw : c->d_w), \
                        (const Tw *)(INV ? c->d_irw : c->d_rw), c->d_modq, c->d_fp, ll, sl, n_limbs, poly_stride, ep, log_r)
-#define ROWS_RING(INV, EPI, GAL)                          \
-    do {                                                  \
-        if (log_r == 8) ROWS(8, INV, EPI, GAL);           \
-        else ROWS(0, INV, EPI, GAL);                      \
+#define ROWS_RING(INV, TAIL, LOAD)                          \
+    do {                                                    \
+        if (log_r == 8) ROWS(8, INV, TAIL, LOAD);           \
+        else ROWS(0, INV, TAIL, LOAD);                      \
     } while (0)
-    if (inverse && ep.galois != 0)
-        ROWS_RING(true, false, true);
+    if (inverse && load == LOAD_ROTATED)
+        ROWS_RING(true, TAIL_NONE, LOAD_ROTATED);
+    else if (inverse && load == LOAD_DECRYPT)
+        ROWS_RING(true, TAIL_NONE, LOAD_DECRYPT);
     else if (inverse)
-        ROWS_RING(true, false, false);
-    else if (ep.out != nullptr)
-        ROWS_RING(false, true, false);
+        ROWS_RING(true, TAIL_NONE, LOAD_PLAIN);
+    else if (tail == TAIL_SUB_SCALE)
+        ROWS_RING(false, TAIL_SUB_SCALE, LOAD_PLAIN);
+    else if (tail == TAIL_ENCRYPT)
+        ROWS_RING(false, TAIL_ENCRYPT, LOAD_PLAIN);
     else
-        ROWS_RING(false, false, false);
+        ROWS_RING(false, TAIL_NONE, LOAD_PLAIN);
 #undef ROWS_RING
 #undef ROWS
+}
+static NttEpilogue sub_scale_tail(const u64 *minuend, size_t minuend_stride, u64 *out, size_t out_stride, const void *cst) {
+    NttEpilogue ep{};
+    ep.minuend = minuend;
+    ep.minuend_stride = minuend_stride;
+    ep.out = out;
+    ep.out_stride = out_stride;
+    ep.cst = (const Tw *)cst;
+    return ep;
 }
 
 // A transform is two launches, and the second reads what the first wrote.  On a large batch the first launch has
@@ -523,18 +590,19 @@ bool launch_ntt_sub_scale(const hemm_context *c, u64 *data, int n_limbs, int n_p
     for (int j = 0; j < HEMM_MAX_PRIMES; j++) ll.idx[j] = sl.idx[j] = (uint8_t)j;
     const size_t poly_stride = (size_t)n_limbs * c->N;
     if (one) {
-        launch_limb_forward(c, data, ll, sl, n_limbs, n_polys, poly_stride, s, nullptr, minuend, minuend_stride, out, out_stride,
-                            cst_dev);
+        launch_limb_forward(c, data, ll, sl, n_limbs, n_polys, poly_stride, s, nullptr, nullptr,
+                            sub_scale_tail(minuend, minuend_stride, out, out_stride, cst_dev), TAIL_SUB_SCALE);
         return true;
     }
     const int run = polys_per_run(c, n_limbs, n_polys, false);
     for (int p0 = 0; p0 < n_polys; p0 += run) {
         const int np = n_polys - p0 < run ? n_polys - p0 : run;
         u64 *d = data + (size_t)p0 * poly_stride;
-        const NttEpilogue ep{minuend + (size_t)p0 * minuend_stride, out + (size_t)p0 * out_stride, (const Tw *)cst_dev,
-                             minuend_stride, out_stride, 0};
         cols_pass(c, false, d, ll, sl, n_limbs, np, poly_stride, s);
-        rows_pass(c, false, d, ll, sl, n_limbs, np, poly_stride, s, ep);
+        rows_pass(c, false, d, ll, sl, n_limbs, np, poly_stride, s,
+                  sub_scale_tail(minuend + (size_t)p0 * minuend_stride, minuend_stride, out + (size_t)p0 * out_stride, out_stride,
+                                 cst_dev),
+                  TAIL_SUB_SCALE);
     }
     return true;
 }
@@ -567,8 +635,9 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
     const bool one = one_launch(c, (size_t)n_limbs * n_polys, false);
     account(c, TR_NTT, (size_t)(tail ? 2 : 1) * n_limbs * n_polys * c->N * 8, one ? 1 : 2);
     if (one) {
-        launch_limb_forward(c, data, ll, sl, n_limbs, n_polys, poly_stride, s, &cs, ep_minuend, ep_minuend_stride, ep_out,
-                            ep_out_stride, ep_cst_dev);
+        launch_limb_forward(c, data, ll, sl, n_limbs, n_polys, poly_stride, s, &cs, nullptr,
+                            sub_scale_tail(ep_minuend, ep_minuend_stride, ep_out, ep_out_stride, ep_cst_dev),
+                            tail ? TAIL_SUB_SCALE : TAIL_NONE);
         return true;
     }
     const dim3 block(256), grid((unsigned)(c->N >> 12), (n_limbs + cs.n_copy) * n_polys);
@@ -590,7 +659,7 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
 #undef CONV_RING
 #undef CONV_CASE
     rows_pass(c, false, data, ll, sl, n_limbs, n_polys, poly_stride, s,
-              tail ? NttEpilogue{ep_minuend, ep_out, (const Tw *)ep_cst_dev, ep_minuend_stride, ep_out_stride, 0} : NttEpilogue{});
+              sub_scale_tail(ep_minuend, ep_minuend_stride, ep_out, ep_out_stride, ep_cst_dev), tail ? TAIL_SUB_SCALE : TAIL_NONE);
     return true;
 }
 
@@ -648,7 +717,7 @@ bool launch_moddown_slab(const hemm_context *c, u64 *y, size_t y_stride, const u
             SLAB_CASE(4, false);
 #undef SLAB_CASE
         rows_pass(c, false, cp, cl, ident, nq_out, np, conv_stride, s,
-                  NttEpilogue{yp, out + (size_t)p0 * out_stride, (const Tw *)cst_dev, y_stride, out_stride, 0});
+                  sub_scale_tail(yp, y_stride, out + (size_t)p0 * out_stride, out_stride, cst_dev), TAIL_SUB_SCALE);
     }
     return true;
 }
@@ -664,7 +733,12 @@ bool launch_intt_from(const hemm_context *c, const u64 *src, size_t src_poly_str
     const bool one = one_launch(c, (size_t)n_limbs * n_polys, galois == 0);
     account(c, TR_NTT, (size_t)2 * n_limbs * n_polys * c->N * 8, one ? 1 : 2);
     if (one) {
-        launch_limb_inverse(c, data, ll, sl, n_limbs, n_polys, poly_stride, s, final_scale, src, src_poly_stride, galois);
+        NttEpilogue from{};
+        from.minuend = src;
+        from.minuend_stride = src_poly_stride;
+        from.galois = galois;
+        launch_limb_inverse(c, data, ll, sl, n_limbs, n_polys, poly_stride, s, final_scale, from,
+                            galois != 0 ? LOAD_ROTATED : LOAD_PLAIN);
         return true;
     }
     const int run = polys_per_run(c, n_limbs, n_polys, true);
@@ -675,9 +749,75 @@ bool launch_intt_from(const hemm_context *c, const u64 *src, size_t src_poly_str
         from.minuend = src + (size_t)p0 * src_poly_stride;
         from.minuend_stride = src_poly_stride;
         from.galois = galois;
-        rows_pass(c, true, d, ll, sl, n_limbs, np, poly_stride, s, from);
+        rows_pass(c, true, d, ll, sl, n_limbs, np, poly_stride, s, from, TAIL_NONE, galois != 0 ? LOAD_ROTATED : LOAD_PLAIN);
         cols_pass(c, true, d, ll, sl, n_limbs, np, poly_stride, s, final_scale);
     }
+    return true;
+}
+
+bool launch_ntt_lifted(const hemm_context *c, const LiftSource &ls, u64 *data, const LimbList &ll, int n_limbs, int n_polys,
+                       size_t poly_stride, hipStream_t s, const EncryptTail *enc) {
+    if (!ring_has_fused_forms(c)) return false;
+    LimbList sl;
+    for (int j = 0; j < HEMM_MAX_PRIMES; j++) sl.idx[j] = (uint8_t)j;
+    const bool one = one_launch(c, (size_t)n_limbs * n_polys, false);
+    account(c, TR_NTT, (size_t)(n_limbs + 1) * n_polys * c->N * 8 + (enc ? (size_t)2 * n_limbs * n_polys * c->N * 8 : 0), one ? 1 : 2);
+    NttEpilogue ep{};
+    if (enc != nullptr) {
+        ep.out = enc->b;
+        ep.second_out = enc->a;
+        ep.out_stride = poly_stride;
+        ep.sk = enc->sk;
+        ep.a_base = enc->a_base;
+    }
+    const int tail = enc != nullptr ? TAIL_ENCRYPT : TAIL_NONE;
+    if (one) {
+        launch_limb_forward(c, data, ll, sl, n_limbs, n_polys, poly_stride, s, nullptr, &ls, ep, tail);
+        return true;
+    }
+    const int run = polys_per_run(c, n_limbs, n_polys, false);
+    for (int p0 = 0; p0 < n_polys; p0 += run) {
+        const int np = n_polys - p0 < run ? n_polys - p0 : run;
+        u64 *d = data + (size_t)p0 * poly_stride;
+        LiftSource l = ls;
+        l.coef += (size_t)p0 * ls.stride;
+        const dim3 grid((unsigned)(c->N >> 12), (unsigned)(n_limbs * np)), block(256);
+#define LIFTED(LR)                                                                                                       \
+    hipLaunchKernelGGL(ntt16_cols_lifted_kernel<LR>, grid, block, 0, s, d, (const Tw *)c->d_w, c->d_modq, c->d_fp, ll, sl, \
+                       n_limbs, poly_stride, l)
+        switch (c->logN) {
+            case 13: LIFTED(5); break;
+            case 14: LIFTED(6); break;
+            case 15: LIFTED(7); break;
+            default: LIFTED(8); break;
+        }
+#undef LIFTED
+        rows_pass(c, false, d, ll, sl, n_limbs, np, poly_stride, s, ep, tail);
+        if (enc != nullptr) {
+            ep.out += (size_t)np * poly_stride;
+            ep.second_out += (size_t)np * poly_stride;
+        }
+    }
+    return true;
+}
+
+bool launch_intt_decrypt(const hemm_context *c, const u64 *b, const u64 *a, const u64 *sk, u64 *data, int n_limbs, hipStream_t s) {
+    if (!ring_has_fused_forms(c)) return false;
+    LimbList ll;
+    for (int j = 0; j < HEMM_MAX_PRIMES; j++) ll.idx[j] = (uint8_t)j;
+    const bool one = one_launch(c, (size_t)n_limbs, false);
+    account(c, TR_NTT, (size_t)4 * n_limbs * c->N * 8, one ? 1 : 2);
+    NttEpilogue from{};
+    from.minuend = b;
+    from.second_in = a;
+    from.sk = sk;
+    const size_t poly_stride = (size_t)n_limbs * c->N;
+    if (one) {
+        launch_limb_inverse(c, data, ll, ll, n_limbs, 1, poly_stride, s, nullptr, from, LOAD_DECRYPT);
+        return true;
+    }
+    rows_pass(c, true, data, ll, ll, n_limbs, 1, poly_stride, s, from, TAIL_NONE, LOAD_DECRYPT);
+    cols_pass(c, true, data, ll, ll, n_limbs, 1, poly_stride, s);
     return true;
 }
 
@@ -700,9 +840,9 @@ void launch_ntt_slots(const hemm_context *c, u64 *data, const LimbList &ll, cons
     }
     if (one) {
         if (inverse)
-            launch_limb_inverse(c, data, ll, sl, n_limbs, n_polys, poly_stride, s, final_scale, nullptr, 0, 0);
+            launch_limb_inverse(c, data, ll, sl, n_limbs, n_polys, poly_stride, s, final_scale, NttEpilogue{}, LOAD_PLAIN);
         else
-            launch_limb_forward(c, data, ll, sl, n_limbs, n_polys, poly_stride, s, nullptr, nullptr, 0, nullptr, 0, nullptr);
+            launch_limb_forward(c, data, ll, sl, n_limbs, n_polys, poly_stride, s, nullptr, nullptr, NttEpilogue{}, TAIL_NONE);
         return;
     }
     const int run = polys_per_run(c, n_limbs, n_polys, inverse, true);

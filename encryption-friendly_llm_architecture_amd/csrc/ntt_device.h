@@ -2,6 +2,24 @@
 // to four stages, and the row pass.
 #pragma once
 #include "hemm_internal.hpp"
+#include "sampling.h"
+
+// a twiddle and its Shoup quotient
+struct __align__(16) Tw {
+    u64 w, ws;
+};
+// what a pass does at its far end (see TAIL_*, LOAD_* below)
+struct NttEpilogue {
+    const u64 *minuend;
+    u64 *out;
+    const Tw *cst;  // per limb: constant and Shoup quotient
+    size_t minuend_stride, out_stride;
+    u32 galois;
+    const u64 *second_in;   // strides as minuend / out
+    u64 *second_out;
+    const u64 *sk;          // [prime][N]
+    u64 a_base;             // the stream of prime i has key sm64(sm64(a_base + i))
+};
 
 namespace {
 typedef u32 u32x2 __attribute__((ext_vector_type(2)));
@@ -29,9 +47,6 @@ __device__ __forceinline__ void buf_store(const __amdgpu_buffer_rsrc_t r, const 
     __builtin_amdgcn_raw_buffer_store_b64(w, r, voff, soff, 0);
 }
 
-struct __align__(16) Tw {
-    u64 w, ws;
-};
 
 // Lazy butterflies (q < 2^61, so 8q < 2^64): forward values stay in [0, 8q), inverse values in [0, 4q); q4 = 4q.
 // u -= 4q when u >= 4q, written as an addition of -4q and a select: no borrow chain
@@ -263,6 +278,17 @@ __device__ __forceinline__ int padc(int c) { return c + (c >> 4); }
 
 __device__ __forceinline__ int swz_row(int r) { return r ^ ((r >> 4) & 1); }
 
+// A signed coefficient of an encoding, plus an error coefficient where one is drawn, as a residue
+__device__ __forceinline__ u64 lift_residue(const long long v, const ModQ &m) {
+    const u64 r = reduce64((u64)(v < 0 ? -v : v), m), n = m.q - r;
+    return (v < 0) & (r != 0) ? n : r;
+}
+__device__ __forceinline__ u64 lifted(const LiftSource &ls, const long long *__restrict__ coef, const u32 n, const ModQ &m) {
+    const u64 r = lift_residue(coef[n], m);
+    if (!ls.with_error) return r;
+    const int e = sample_error(ls.error_key, n);
+    return addmod(r, e >= 0 ? (u64)e : m.q - (u64)(-e), m.q);
+}
 // The 16 coefficients of a thread as a basis conversion computed on the fly: coefficient k is sum_i v_i * hat_i mod q
 // over the n_src <= NS source limbs (pre-scaled, the same lazy sums and reductions as the stand-alone conversion kernels,
 // so the residues are the same), read at voff + off(k) inside a limb; so[i]: byte offset of source limb i.
@@ -304,29 +330,35 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Optional tail of a forward transform: instead of storing the transformed residues v in place, store
-// (minuend - v) * cst[limb] to `out` -- the last step of ModDown / rescale, folded into the pass that
-// already holds v in registers (saves one read and one write of every limb and a launch).
-struct NttEpilogue {
-    const u64 *minuend;
+// Optional tail of a forward transform (TAIL), on the values v that the last pass already holds in registers, instead of
+// storing them in place:
+//   TAIL_SUB_SCALE: (minuend - v) * cst[limb] to `out` -- the last step of ModDown / rescale (saves one read and one write of
+//                   every limb and a launch);
+//   TAIL_ENCRYPT:   v is an encoded message plus an error: a sampled from a stream of the limb's prime to `second_out`,
+//                   v - a s to `out`.
+// Optional origin of an inverse transform's input (LOAD): `data` itself or `minuend` (same slot numbering, own polynomial
+// stride; nullptr: data), LOAD_ROTATED: `minuend` through the automorphism `galois`, LOAD_DECRYPT: minuend + second_in * s.
+enum { TAIL_NONE = 0, TAIL_SUB_SCALE = 1, TAIL_ENCRYPT = 2 };
+enum { LOAD_PLAIN = 0, LOAD_ROTATED = 1, LOAD_DECRYPT = 2 };
+// what TAIL_ENCRYPT and LOAD_DECRYPT need for one row
+struct RowSecond {
+    const u64 *in;
     u64 *out;
-    const Tw *cst;  // per limb: constant and Shoup quotient
-    size_t minuend_stride, out_stride;
-    u32 galois;     // inverse transforms that read their input elsewhere: != 0 reads it through this automorphism
+    const u64 *sk;
+    u64 key;
+    ModQ m;
 };
-// An inverse transform may read its input elsewhere (same slot numbering, own polynomial stride) and leave the
-// result in `data`: the first pass then loads from `minuend` (stride `minuend_stride`) instead of `data`.
 
 // forward pass 2 / inverse pass 1 work on 16 whole rows (16 x 256 contiguous residues); r: the row of 2^log_r.
-// GAL (inverse only): ld is the base of the source limb and residue k of the input is ld[galois_index(k)] -- an aligned
+// LOAD_ROTATED: ld is the base of the source limb and residue k of the input is ld[galois_index(k)] -- an aligned
 // group of 16 residues stays an aligned group under the automorphism, so the loads touch the same number of lines
 // IN_LDS: the row pass follows (forward) or precedes (inverse) a column pass over the same limb in the same workgroup: the
 // row is taken from, resp. left in, its padded LDS row instead of memory.
-template <bool INV, bool EPI, bool GAL, bool IN_LDS, class F>
+template <bool INV, int TAIL, int LOAD, bool IN_LDS, class F>
 __device__ __forceinline__ void rows_body(u64 *__restrict__ row, const Tw *__restrict__ tw_int,
                                           const Tw *__restrict__ rtw_int, const F f, u64 *lds_raw, const int log_r, const u32 r,
                                           const u64 *__restrict__ mn, u64 *__restrict__ o, const Tw cst,
-                                          const u64 *__restrict__ ld, const u32 gal = 0) {
+                                          const u64 *__restrict__ ld, const u32 gal, const RowSecond &sec) {
     typedef typename F::E E;
     const typename F::W *tw = (const typename F::W *)tw_int;
     const int c = threadIdx.x & 15, rr = threadIdx.x >> 4;
@@ -345,8 +377,8 @@ __device__ __forceinline__ void rows_body(u64 *__restrict__ row, const Tw *__res
 #pragma unroll
         for (int k = 0; k < 16; k++) x[k] = l[padc(16 * c + k)];
         // the minuend of the fused tail is fetched under the second radix-16 block instead of after it
-        u64 mv[EPI ? 16 : 1];
-        if (EPI) {
+        u64 mv[TAIL == TAIL_SUB_SCALE ? 16 : 1];
+        if (TAIL == TAIL_SUB_SCALE) {
 #pragma unroll
             for (int k = 0; k < 16; k++) mv[k] = __builtin_nontemporal_load(mn + c + 16 * k);
         }
@@ -355,15 +387,26 @@ __device__ __forceinline__ void rows_body(u64 *__restrict__ row, const Tw *__res
 #pragma unroll
         for (int k = 0; k < 16; k++) l[padc(16 * c + k)] = x[k];
         wave_sync();
-        if (EPI) {
+        if (TAIL == TAIL_SUB_SCALE) {
 #pragma unroll
             for (int k = 0; k < 16; k++) o[c + 16 * k] = f.sub_scale(l[padc(c + 16 * k)], mv[k], cst);
+        } else if (TAIL == TAIL_ENCRYPT) {
+#pragma unroll 4
+            for (int k = 0; k < 16; k++) {
+                const u64 a = sample_uniform(sec.key, (r << 8) + (u32)(c + 16 * k), sec.m);
+                o[c + 16 * k] = submod(f.to_canonical(l[padc(c + 16 * k)]), mulmod(a, sec.sk[c + 16 * k], sec.m), sec.m.q);
+                sec.out[c + 16 * k] = a;
+            }
         } else {
 #pragma unroll
             for (int k = 0; k < 16; k++) row[c + 16 * k] = f.to_canonical(l[padc(c + 16 * k)]);
         }
     } else {
-        if (GAL) {
+        if (LOAD == LOAD_DECRYPT) {
+#pragma unroll 4
+            for (int k = 0; k < 16; k++)
+                lc[padc(c + 16 * k)] = addmod(ld[c + 16 * k], mulmod(sec.in[c + 16 * k], sec.sk[c + 16 * k], sec.m), sec.m.q);
+        } else if (LOAD == LOAD_ROTATED) {
 #pragma unroll
             for (int k = 0; k < 16; k++) lc[padc(c + 16 * k)] = ld[galois_index((r << 8) + (u32)(c + 16 * k), gal, 8 + log_r)];
         } else {

@@ -37,11 +37,14 @@ struct Limb {
     static __device__ __forceinline__ int at2(const int k) { return (16 * rh() + k) * ROWPAD + padc(col(k)); }
 };
 
-template <int LR, int NS, bool EPI, class F>
+// NS > 0: the input is a conversion of up to NS sources, LIFTED: the coefficients of an encoding
+enum { LIFTED = -1 };
+template <int LR, int NS, int TAIL, class F>
 __device__ __forceinline__ void limb_forward(u64 *__restrict__ limb, const Tw *__restrict__ tw_int, const Tw *__restrict__ rtw,
                                              const F f, u64 *lds_raw, const __amdgpu_buffer_rsrc_t src,
                                              const u32 (&so)[NS > 0 ? NS : 1], const u64 (&h)[NS > 0 ? NS : 1], const int n_src,
-                                             const ModQ m, const u64 *__restrict__ mn, u64 *__restrict__ o, const Tw cst) {
+                                             const ModQ m, const LiftSource &ls, const long long *__restrict__ coef,
+                                             const u64 *__restrict__ mn, u64 *__restrict__ o, const Tw cst, RowSecond sec) {
     typedef typename F::E E;
     typedef Limb<LR> S;
     E *lds = (E *)lds_raw;
@@ -49,6 +52,9 @@ __device__ __forceinline__ void limb_forward(u64 *__restrict__ limb, const Tw *_
     if (NS > 0) {
         converted_inputs<(NS > 0 ? NS : 1)>(f, x, src, S::voff(), so, h, n_src, m,
                                             [](const int k) { return S::off(k); });
+    } else if (NS == LIFTED) {
+#pragma unroll
+        for (int k = 0; k < 16; k++) x[k] = f.from_canonical(lifted(ls, coef, (S::voff() + S::off(k)) >> 3, m));
     } else {
 #pragma unroll
         for (int k = 0; k < 16; k++) x[k] = f.from_canonical(buf_load<u64>(src, S::voff(), S::off(k)));
@@ -66,16 +72,22 @@ __device__ __forceinline__ void limb_forward(u64 *__restrict__ limb, const Tw *_
         __syncthreads();
     }
     const u32 r = threadIdx.x >> 4;
-    rows_body<false, EPI, false, true>(limb + (r << 8), tw_int, rtw, f, lds_raw, LR, r, EPI ? mn + (r << 8) : nullptr,
-                                       EPI ? o + (r << 8) : nullptr, cst, nullptr);
+    if (TAIL == TAIL_ENCRYPT) {
+        sec.out += r << 8;
+        sec.sk += r << 8;
+    }
+    rows_body<false, TAIL, LOAD_PLAIN, true>(limb + (r << 8), tw_int, rtw, f, lds_raw, LR, r,
+                                             TAIL == TAIL_SUB_SCALE ? mn + (r << 8) : nullptr,
+                                             TAIL != TAIL_NONE ? o + (r << 8) : nullptr, cst, nullptr, 0, sec);
 }
 
-// data[n_polys][.][N] (polynomial stride poly_stride), limb l in slot sl[l]; NS > 0: the inputs are the conversions of
-// cs, whose plain copies follow the limbs of a polynomial; EPI: out = (minuend - transform) * cst[l].
-template <int LR, int NS, bool EPI>
+// data[n_polys][.][N] (polynomial stride poly_stride), limb l in slot sl[l]; the plain copies of cs follow the limbs of a
+// polynomial.
+template <int LR, int NS, int TAIL>
 __global__ __launch_bounds__(16 << LR) void ntt_limb_forward_kernel(
     u64 *__restrict__ data, const Tw *__restrict__ tw_all, const Tw *__restrict__ rtw_all, const ModQ *__restrict__ modq,
-    const double *__restrict__ fp, LimbList ll, LimbList sl, int n_limbs, size_t poly_stride, ConvSources cs, NttEpilogue ep) {
+    const double *__restrict__ fp, LimbList ll, LimbList sl, int n_limbs, size_t poly_stride, ConvSources cs,
+    LiftSource ls, NttEpilogue ep) {
     __shared__ u64 lds[(ROWPAD << LR)];
     const int log_n = 8 + LR;
     const int per_poly = n_limbs + (NS > 0 ? cs.n_copy : 0);
@@ -116,28 +128,42 @@ __global__ __launch_bounds__(16 << LR) void ntt_limb_forward_kernel(
     const u64 *mn = nullptr;
     u64 *o = nullptr;
     Tw cst{0, 0};
-    if (EPI) {
+    RowSecond sec{};
+    if (TAIL != TAIL_NONE) o = ep.out + (size_t)poly * ep.out_stride + ((size_t)limb << log_n);
+    if (TAIL == TAIL_SUB_SCALE) {
         mn = ep.minuend + (size_t)poly * ep.minuend_stride + ((size_t)limb << log_n);
-        o = ep.out + (size_t)poly * ep.out_stride + ((size_t)limb << log_n);
         cst = ep.cst[limb];
+    } else if (TAIL == TAIL_ENCRYPT) {
+        sec.out = ep.second_out + (size_t)poly * ep.out_stride + ((size_t)limb << log_n);
+        sec.sk = ep.sk + ((size_t)prime << log_n);
+        sec.key = sm64(sm64(ep.a_base + (u64)prime));
+        sec.m = m;
     }
+    const long long *coef = NS == LIFTED ? ls.coef + (size_t)poly * ls.stride : nullptr;
     if (fp[4 * prime] != 0.0)
-        limb_forward<LR, NS, EPI>(base, tw, rtw, FpField(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, mn, o, cst);
+        limb_forward<LR, NS, TAIL>(base, tw, rtw, FpField(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, ls,
+                                   coef, mn, o, cst, sec);
     else if ((m.q >> 60) != 0)
-        limb_forward<LR, NS, EPI>(base, tw, rtw, IntField(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, mn, o, cst);
+        limb_forward<LR, NS, TAIL>(base, tw, rtw, IntField(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, ls,
+                                   coef, mn, o, cst, sec);
     else
-        limb_forward<LR, NS, EPI>(base, tw, rtw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, mn,
-                                  o, cst);
+        limb_forward<LR, NS, TAIL>(base, tw, rtw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, ls,
+                                   coef, mn, o, cst, sec);
 }
 
-template <int LR, bool GAL, class F>
+template <int LR, int LOAD, class F>
 __device__ __forceinline__ void limb_inverse(u64 *__restrict__ limb, const Tw *__restrict__ tw_int, const Tw *__restrict__ rtw,
-                                             const F f, u64 *lds_raw, const u64 *__restrict__ ld, const u32 gal) {
+                                             const F f, u64 *lds_raw, const u64 *__restrict__ ld, const u32 gal, RowSecond sec) {
     typedef typename F::E E;
     typedef Limb<LR> S;
     E *lds = (E *)lds_raw;
     const u32 r = threadIdx.x >> 4;
-    rows_body<true, false, GAL, true>(limb, tw_int, rtw, f, lds_raw, LR, r, nullptr, nullptr, Tw{0, 0}, GAL ? ld : ld + (r << 8), gal);
+    if (LOAD == LOAD_DECRYPT) {
+        sec.in += r << 8;
+        sec.sk += r << 8;
+    }
+    rows_body<true, TAIL_NONE, LOAD, true>(limb, tw_int, rtw, f, lds_raw, LR, r, nullptr, nullptr, Tw{0, 0},
+                                           LOAD == LOAD_ROTATED ? ld : ld + (r << 8), gal, sec);
     __syncthreads();
     E x[16];
 #pragma unroll
@@ -157,19 +183,24 @@ __device__ __forceinline__ void limb_inverse(u64 *__restrict__ limb, const Tw *_
     for (int k = 0; k < 16; k++) buf_store<u64>(to, S::voff(), S::off(k), f.scale_to_canonical(x[k]));
 }
 
-template <int LR, bool GAL>
+template <int LR, int LOAD>
 __global__ __launch_bounds__(16 << LR) void ntt_limb_inverse_kernel(
     u64 *__restrict__ data, const Tw *__restrict__ tw_all, const Tw *__restrict__ rtw_all, const ModQ *__restrict__ modq,
     const u64 *__restrict__ ninv, const u64 *__restrict__ ninv_s, const double *__restrict__ fp, LimbList ll, LimbList sl,
-    int n_limbs, size_t poly_stride, const Tw *__restrict__ final_scale, const u64 *__restrict__ from, size_t from_stride,
-    u32 gal) {
+    int n_limbs, size_t poly_stride, const Tw *__restrict__ final_scale, NttEpilogue from) {
     __shared__ u64 lds[(ROWPAD << LR)];
     const int log_n = 8 + LR;
     const int limb = blockIdx.x % n_limbs, poly = blockIdx.x / n_limbs;
     const int prime = __builtin_amdgcn_readfirstlane((int)ll.idx[limb]);
     const size_t slot = (size_t)__builtin_amdgcn_readfirstlane((int)sl.idx[limb]) << log_n;
     u64 *base = data + (size_t)poly * poly_stride + slot;
-    const u64 *ld = from != nullptr ? from + (size_t)poly * from_stride + slot : base;
+    const u64 *ld = from.minuend != nullptr ? from.minuend + (size_t)poly * from.minuend_stride + slot : base;
+    RowSecond sec{};
+    if (LOAD == LOAD_DECRYPT) {
+        sec.in = from.second_in + (size_t)poly * from.minuend_stride + slot;
+        sec.sk = from.sk + ((size_t)prime << log_n);
+        sec.m = modq[prime];
+    }
     const Tw *tw = tw_all + ((size_t)prime << log_n), *rtw = rtw_all + ((size_t)prime << log_n);
     if (fp[4 * prime] != 0.0) {
         FpField f(modq, ninv, ninv_s, fp, prime);
@@ -177,54 +208,56 @@ __global__ __launch_bounds__(16 << LR) void ntt_limb_inverse_kernel(
             f.ni = (double)final_scale[limb].w;
             f.niinv = f.ni * f.qinv;
         }
-        limb_inverse<LR, GAL>(base, tw, rtw, f, lds, ld, gal);
+        limb_inverse<LR, LOAD>(base, tw, rtw, f, lds, ld, from.galois, sec);
     } else {
         IntField f(modq, ninv, ninv_s, fp, prime);
         if (final_scale != nullptr) {
             f.ni = final_scale[limb].w;
             f.nis = final_scale[limb].ws;
         }
-        limb_inverse<LR, GAL>(base, tw, rtw, f, lds, ld, gal);
+        limb_inverse<LR, LOAD>(base, tw, rtw, f, lds, ld, from.galois, sec);
     }
 }
 
 }  // namespace
 
 void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
-                         size_t poly_stride, hipStream_t s, const ConvSources *cs, const u64 *minuend, size_t minuend_stride,
-                         u64 *out, size_t out_stride, const void *cst_dev) {
+                         size_t poly_stride, hipStream_t s, const ConvSources *cs, const LiftSource *ls, const NttEpilogue &ep,
+                         int tail) {
     const int LR = c->logN - 8;
     int widest = 0;
-    ConvSources none;
-    if (cs == nullptr) {
-        memset(&none, 0, sizeof(none));
-        cs = &none;
-    } else {
+    ConvSources conv;
+    LiftSource lift{};
+    memset(&conv, 0, sizeof(conv));
+    if (cs != nullptr) {
+        conv = *cs;
         for (int l = 0; l < n_limbs; l++) widest = std::max(widest, cs->d[cs->digit_of[l]].n_src);
     }
-    const NttEpilogue ep{minuend, out, (const Tw *)cst_dev, minuend_stride, out_stride, 0};
-    const dim3 grid((unsigned)((n_limbs + cs->n_copy) * n_polys)), block(16u << LR);
-#define LIMB_FORWARD(L, K, EPI)                                                                                            \
-    hipLaunchKernelGGL((ntt_limb_forward_kernel<L, K, EPI>), grid, block, 0, s, data, (const Tw *)c->d_w,                  \
-                       (const Tw *)c->d_rw, c->d_modq, c->d_fp, ll, sl, n_limbs, poly_stride, *cs, ep)
-#define LIMB_SOURCES(L, EPI)                          \
-    do {                                              \
-        if (widest == 0) LIMB_FORWARD(L, 0, EPI);     \
-        else if (widest <= 2) LIMB_FORWARD(L, 2, EPI); \
-        else if (widest <= 5) LIMB_FORWARD(L, 5, EPI); \
-        else LIMB_FORWARD(L, 8, EPI);                 \
+    if (ls != nullptr) lift = *ls;
+    const dim3 grid((unsigned)((n_limbs + conv.n_copy) * n_polys)), block(16u << LR);
+#define LIMB_FORWARD(L, K, TAIL)                                                                                           \
+    hipLaunchKernelGGL((ntt_limb_forward_kernel<L, K, TAIL>), grid, block, 0, s, data, (const Tw *)c->d_w,                 \
+                       (const Tw *)c->d_rw, c->d_modq, c->d_fp, ll, sl, n_limbs, poly_stride, conv, lift, ep)
+#define LIMB_SOURCES(L, TAIL)                          \
+    do {                                               \
+        if (widest == 0) LIMB_FORWARD(L, 0, TAIL);     \
+        else if (widest <= 2) LIMB_FORWARD(L, 2, TAIL); \
+        else if (widest <= 5) LIMB_FORWARD(L, 5, TAIL); \
+        else LIMB_FORWARD(L, 8, TAIL);                 \
     } while (0)
-#define LIMB_RING(L)                       \
-    do {                                   \
-        if (out != nullptr) LIMB_SOURCES(L, true); \
-        else LIMB_SOURCES(L, false);       \
+#define LIMB_RING(L)                                                       \
+    do {                                                                   \
+        if (ls != nullptr && tail == TAIL_ENCRYPT) LIMB_FORWARD(L, LIFTED, TAIL_ENCRYPT); \
+        else if (ls != nullptr) LIMB_FORWARD(L, LIFTED, TAIL_NONE);        \
+        else if (tail == TAIL_SUB_SCALE) LIMB_SOURCES(L, TAIL_SUB_SCALE);  \
+        else LIMB_SOURCES(L, TAIL_NONE);                                   \
     } while (0)
     switch (LR) {
         case 2: LIMB_RING(2); break;
         case 3: LIMB_RING(3); break;
         case 4: LIMB_RING(4); break;
         case 5: LIMB_RING(5); break;
-        case 6: LIMB_FORWARD(6, 0, false); break;
+        case 6: LIMB_FORWARD(6, 0, TAIL_NONE); break;
         default: throw std::invalid_argument("no one-launch transform for this ring size");
     }
 #undef LIMB_RING
@@ -233,25 +266,25 @@ void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, c
 }
 
 void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
-                         size_t poly_stride, hipStream_t s, const void *final_scale, const u64 *from, size_t from_stride,
-                         u32 galois) {
+                         size_t poly_stride, hipStream_t s, const void *final_scale, const NttEpilogue &from, int load) {
     const int LR = c->logN - 8;
     const dim3 grid((unsigned)(n_limbs * n_polys)), block(16u << LR);
-#define LIMB_INVERSE(L, GAL)                                                                                          \
-    hipLaunchKernelGGL((ntt_limb_inverse_kernel<L, GAL>), grid, block, 0, s, data, (const Tw *)c->d_iw,               \
+#define LIMB_INVERSE(L, LOAD)                                                                                         \
+    hipLaunchKernelGGL((ntt_limb_inverse_kernel<L, LOAD>), grid, block, 0, s, data, (const Tw *)c->d_iw,              \
                        (const Tw *)c->d_irw, c->d_modq, c->d_ninv, c->d_ninv_s, c->d_fp, ll, sl, n_limbs, poly_stride, \
-                       (const Tw *)final_scale, from, from_stride, galois)
-#define LIMB_RING(L)                        \
-    do {                                    \
-        if (galois != 0) LIMB_INVERSE(L, true); \
-        else LIMB_INVERSE(L, false);        \
+                       (const Tw *)final_scale, from)
+#define LIMB_RING(L)                                                   \
+    do {                                                               \
+        if (load == LOAD_ROTATED) LIMB_INVERSE(L, LOAD_ROTATED);       \
+        else if (load == LOAD_DECRYPT) LIMB_INVERSE(L, LOAD_DECRYPT);  \
+        else LIMB_INVERSE(L, LOAD_PLAIN);                              \
     } while (0)
     switch (LR) {
         case 2: LIMB_RING(2); break;
         case 3: LIMB_RING(3); break;
         case 4: LIMB_RING(4); break;
         case 5: LIMB_RING(5); break;
-        case 6: LIMB_INVERSE(6, false); break;
+        case 6: LIMB_INVERSE(6, LOAD_PLAIN); break;
         default: throw std::invalid_argument("no one-launch transform for this ring size");
     }
 #undef LIMB_RING

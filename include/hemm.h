@@ -100,6 +100,25 @@ int hemm_mul_scalar(hemm_context *ctx, const uint64_t *a, size_t a_stride, const
  * with one IEEE operation per step in a fixed order: the same bits as a host loop over the same butterflies. */
 int hemm_encode(hemm_context *ctx, double *slots, double scale, uint32_t nq, int with_p, uint32_t n_msgs, uint64_t *out,
                 void *stream);
+/* the same from slots that stay as they are; workspace: [n_msgs][N] words */
+int hemm_encode_from(hemm_context *ctx, const double *slots, double scale, uint32_t nq, int with_p, uint32_t n_msgs,
+                     uint64_t *workspace, uint64_t *out, void *stream);
+/* One message whose first `count` slots are the real numbers `values` and whose others are zero (a matrix in its tile; N >=
+ * 1024).  `values` may be device memory or pinned host memory, which the first launch reads in place: it has to stay as it
+ * is until the work queued on `stream` here is done.  workspace: N words.  hemm_encrypt_reals encrypts it as well
+ * (Encryptor::encrypt(Message), Encryptor.hpp:32-49): ct = (pt + e - a s, a) with polynomial stride ct_stride, limb i of a
+ * uniform from stream sm64(sm64(a_base + i)) and e from stream error_key (the samplers above); sk: the secret in NTT form
+ * [n_q + n_p][N].  Same residues as the separate steps. */
+int hemm_encode_reals(hemm_context *ctx, const double *values, size_t count, double scale, uint32_t nq, int with_p,
+                      uint64_t *workspace, uint64_t *out, void *stream);
+int hemm_encrypt_reals(hemm_context *ctx, const double *values, size_t count, double scale, uint32_t nq, const uint64_t *sk,
+                       uint64_t a_base, uint64_t error_key, uint64_t *workspace, uint64_t *ct, size_t ct_stride,
+                       void *stream);
+/* Decryptor::decrypt + decode of a two-polynomial ciphertext (Decryptor.hpp:27-60): the real parts of its first `count` slots
+ * to `values`, device memory or pinned host memory (complete when `stream` is).  n_limbs as for hemm_decode; workspace:
+ * (n_limbs + 1) * N words; N >= 1024. */
+int hemm_decrypt_reals(hemm_context *ctx, const uint64_t *ct, size_t ct_stride, const uint64_t *sk, uint32_t n_limbs,
+                       double scale, uint64_t *workspace, double *values, size_t count, void *stream);
 /* EnDecoder::decode (EnDecoder.hpp:66): plaintext pt [>= n_limbs][N] (NTT form, limbs of chain primes 0 .. n_limbs-1,
  * n_limbs = 1 or 2: the centred value is recovered from that many limbs) -> slots [N/2][2] doubles on the device;
  * workspace: n_limbs * N words. */
