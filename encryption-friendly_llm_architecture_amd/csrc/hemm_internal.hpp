@@ -68,8 +68,8 @@ inline void account(const hemm_context *c, int kind, size_t bytes, int n_launche
 // laid out for it).
 inline bool ring_has_fused_forms(const hemm_context *c) { return c->logN >= 10; }
 // Whether a transform is one launch with a workgroup per limb: up to 2^12 points always.  A larger limb is slower in one
-// workgroup than spread over several in two launches (2^13 points: 11.5 against 11.0 us for one limb, 12.4 against 13.2
-// for 96; 2^14: 21 against 18.5 us for 64), until the limbs alone fill the CUs and the second trip through memory is what
+// workgroup than spread over several in two launches (2^13 points: 11.3 against 9.0 us for one limb, 12.0 against 11.8
+// for 48 of 60 bits; 2^14: 21 against 18.5 us for 64), until the limbs alone fill the CUs and the second trip through memory is what
 // counts (60-bit primes: 34.6 against 47.2 us for 768 limbs of 2^13; 2^14: 23 against 28 us for 128, 81 against 87 for 768).
 // plain: no conversion, tail or automorphism -- with them a workgroup of the 1024 threads a limb of 2^14 takes would spill.
 inline bool one_launch(const hemm_context *c, size_t limbs, bool plain) {

@@ -8,9 +8,9 @@
 // points, 512 KiB, does not fit a CU's LDS, and a smaller one spread over R / 16 workgroups keeps more CUs busy):
 //   forward pass 1: stages 0 .. log2 R - 1  act down columns  (butterfly distance >= 256)
 //   forward pass 2: the last eight stages   act inside rows   (distance <= 128)
-// and mirrored for the inverse.  Each workgroup (256 threads = 4 wavefronts) owns 4096 points, R rows of 4096 / R columns
-// (or 16 rows); a thread keeps 16 residues in registers, runs a block of up to four stages
-// on them, swaps through LDS once and runs the second block.  All global accesses
+// and mirrored for the inverse.  Each workgroup owns 4096 points, R rows of 4096 / R columns (or 16 rows, 8 with eight points
+// per thread); a thread keeps 16 residues in registers, or two lanes of a wavefront 8 each, runs a block of up to four
+// stages on them, swaps through LDS once and runs the second block.  All global accesses
 // are segments of at least 128 bytes shared by adjacent lanes.
 //
 // Rings of 2^10 .. 2^12 points, and large batches of 2^13 and 2^14, take one launch (ntt_limb.hip), the smallest rings
@@ -71,13 +71,14 @@ __global__ __launch_bounds__(256) void ntt_small_kernel(u64 *__restrict__ data, 
 // ------------------------------------------------------------------------------------------
 // two-launch kernels (N = 2^13 .. 2^16)
 // ------------------------------------------------------------------------------------------
-// Column passes work on a slab of R = 2^LR rows and CW = 4096 / R columns (R = 256: 16 columns): a thread's 16 residues
+// Column passes work on a slab of R = 2^LR rows and CW = 4096 / R columns (R = 256: 16 columns): the 16 residues of a thread or lane pair
 // are rows rh + (R / 16) k for the block of the four widest stages and rows 16 rh + k for the LR - 4 others.
-template <int LR>
+template <int LR, int P>
 struct Slab {
+    typedef Lanes<P> L;
     static constexpr int R = 1 << LR, Q = R / 16, CW = 4096 / R, T = LR - 4;
-    static __device__ __forceinline__ u32 cc() { return threadIdx.x & (CW - 1); }
-    static __device__ __forceinline__ u32 rh() { return threadIdx.x >> (12 - LR); }
+    static __device__ __forceinline__ u32 cc() { return L::t() & (CW - 1); }
+    static __device__ __forceinline__ u32 rh() { return L::t() >> (12 - LR); }
     static __device__ __forceinline__ u32 col() { return blockIdx.x * CW + cc(); }
     // twiddle group of the second block: 16 / Q sub-blocks per thread
     static __device__ __forceinline__ u32 group() { return 16u + rh() * (16 / Q); }
@@ -87,60 +88,64 @@ struct Slab {
     // conflicts: 9.7 against 8.8 us for 10 limbs of 42-bit primes)
     template <bool INV>
     static __device__ __forceinline__ int at(const int r) { return (CW == 16 && !INV ? swz_row(r) : r) * CW + (int)cc(); }
-    // byte offsets of (row rh, col) and (row 16 rh, col) inside a limb; the step from k to k + 1 goes into the scalar offset
-    static __device__ __forceinline__ u32 v_outer() { return (col() + (rh() << 8)) * 8u; }
-    static __device__ __forceinline__ u32 v_inner() { return (col() + (rh() << 12)) * 8u; }
-    static __device__ __forceinline__ constexpr u32 outer(const int k) { return (u32)k * (Q << 11); }
+    // rows of a thread's register k: of the four widest stages (split, whole), of the others (split, whole)
+    static __device__ __forceinline__ int r_outer_s(const int k) { return (int)(rh() + Q * L::template h_split<4>()) + Q * L::template split<4>(k); }
+    static __device__ __forceinline__ int r_outer_w(const int k) { return (int)(rh() + Q * L::h_whole()) + Q * k; }
+    static __device__ __forceinline__ int r_inner_s(const int k) { return (int)(16 * rh() + L::template h_split<T>()) + L::template split<T>(k); }
+    static __device__ __forceinline__ int r_inner_w(const int k) { return (int)(16 * rh() + L::h_whole()) + k; }
+    // byte offsets inside a limb of the widest stages' points (split) and of the others' (whole): a thread's part, and the
+    // step to register k, which goes into the scalar offset
+    static __device__ __forceinline__ u32 v_outer() { return (col() + ((u32)r_outer_s(0) << 8)) * 8u; }
+    static __device__ __forceinline__ u32 v_inner() { return (col() + ((u32)r_inner_w(0) << 8)) * 8u; }
+    static __device__ __forceinline__ constexpr u32 outer(const int k) { return (u32)L::template split<4>(k) * (Q << 11); }
     static __device__ __forceinline__ constexpr u32 inner(const int k) { return (u32)k << 11; }
 };
 // the exchange and the second block of a forward column pass, results to memory
-template <int LR, class F>
+template <int LR, int P, class F>
 __device__ __forceinline__ void cols_forward(const __amdgpu_buffer_rsrc_t limb, const typename F::W *__restrict__ tw,
-                                             const F f, typename F::E (&x)[16], typename F::E *lds) {
+                                             const F f, typename F::E (&x)[P], typename F::E *lds) {
     typedef typename F::E E;
-    typedef Slab<LR> S;
-    const int rh = (int)S::rh();
+    typedef Slab<LR, P> S;
     radix_fwd<4>(f, x, tw, 1u);
 #pragma unroll
-    for (int k = 0; k < 16; k++) lds[S::template at<false>(rh + S::Q * k)] = x[k];
+    for (int k = 0; k < P; k++) lds[S::template at<false>(S::r_outer_w(k))] = x[k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = lds[S::template at<false>(16 * rh + k)];
+    for (int k = 0; k < P; k++) x[k] = lds[S::template at<false>(S::r_inner_s(k))];
     radix_fwd<S::T>(f, x, tw, S::group());
 #pragma unroll
-    for (int k = 0; k < 16; k++) buf_store<E>(limb, S::v_inner(), S::inner(k), x[k]);
+    for (int k = 0; k < P; k++) buf_store<E>(limb, S::v_inner(), S::inner(k), x[k]);
 }
-template <int LR, bool INV, class F>
+template <int LR, int P, bool INV, class F>
 __device__ __forceinline__ void cols_body(const __amdgpu_buffer_rsrc_t limb, const Tw *__restrict__ tw_int, const F f,
                                           u64 *lds_raw) {
     typedef typename F::E E;
-    typedef Slab<LR> S;
+    typedef Slab<LR, P> S;
     const typename F::W *tw = (const typename F::W *)tw_int;
     E *lds = (E *)lds_raw;
-    const int rh = (int)S::rh();
-    E x[16];
+    E x[P];
     if (!INV) {
 #pragma unroll
-        for (int k = 0; k < 16; k++) x[k] = f.from_canonical(buf_load<u64>(limb, S::v_outer(), S::outer(k)));
+        for (int k = 0; k < P; k++) x[k] = f.from_canonical(buf_load<u64>(limb, S::v_outer(), S::outer(k)));
         cols_forward<LR>(limb, tw, f, x, lds);
     } else {
 #pragma unroll
-        for (int k = 0; k < 16; k++) x[k] = buf_load<E>(limb, S::v_inner(), S::inner(k));
+        for (int k = 0; k < P; k++) x[k] = buf_load<E>(limb, S::v_inner(), S::inner(k));
         radix_inv<S::T>(f, x, tw, S::group());
         f.template after_inverse_block<S::T>(x);
 #pragma unroll
-        for (int k = 0; k < 16; k++) lds[S::template at<true>(16 * rh + k)] = x[k];
+        for (int k = 0; k < P; k++) lds[S::template at<true>(S::r_inner_s(k))] = x[k];
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < 16; k++) x[k] = lds[S::template at<true>(rh + S::Q * k)];
+        for (int k = 0; k < P; k++) x[k] = lds[S::template at<true>(S::r_outer_w(k))];
         radix_inv<4>(f, x, tw, 1u);
 #pragma unroll
-        for (int k = 0; k < 16; k++) buf_store<u64>(limb, S::v_outer(), S::outer(k), f.scale_to_canonical(x[k]));
+        for (int k = 0; k < P; k++) buf_store<u64>(limb, S::v_outer(), S::outer(k), f.scale_to_canonical(x[k]));
     }
 }
 
-template <int LR, bool INV>
-__global__ __launch_bounds__(256) void ntt16_cols_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
+template <int LR, int P, bool INV>
+__global__ __launch_bounds__(4096 / P) void ntt16_cols_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
                                                          const ModQ *__restrict__ modq,
                                                          const u64 *__restrict__ ninv, const u64 *__restrict__ ninv_s,
                                                          const double *__restrict__ fp, LimbList ll, LimbList sl,
@@ -159,16 +164,16 @@ __global__ __launch_bounds__(256) void ntt16_cols_kernel(u64 *__restrict__ data,
             f.ni = (double)final_scale[limb].w;
             f.niinv = f.ni * f.qinv;
         }
-        cols_body<LR, INV>(base, tw, f, lds);
+        cols_body<LR, P, INV>(base, tw, f, lds);
     } else if (INV || (modq[prime].q >> 60) != 0) {
         IntField f(modq, ninv, ninv_s, fp, prime);
         if (INV && final_scale != nullptr) {
             f.ni = final_scale[limb].w;
             f.nis = final_scale[limb].ws;
         }
-        cols_body<LR, INV>(base, tw, f, lds);
+        cols_body<LR, P, INV>(base, tw, f, lds);
     } else {
-        cols_body<LR, INV>(base, tw, IntFieldT<true>(modq, ninv, ninv_s, fp, prime), lds);
+        cols_body<LR, P, INV>(base, tw, IntFieldT<true>(modq, ninv, ninv_s, fp, prime), lds);
     }
 }
 
@@ -179,40 +184,39 @@ template <int LR, int NS, class F>
 __device__ __forceinline__ void cols_converted_body(const __amdgpu_buffer_rsrc_t limb, const Tw *__restrict__ tw_int,
                                                     const F f, u64 *lds_raw, const __amdgpu_buffer_rsrc_t src,
                                                     const u32 (&so)[NS], const u64 (&h)[NS], const int n_src, const ModQ m) {
-    typedef Slab<LR> S;
-    typename F::E x[16];
-    // row rh + Q k of the slab: the row step goes into the scalar offset
+    typedef Slab<LR, 8> S;
+    typename F::E x[8];
+    // the row step goes into the scalar offset
     converted_inputs<NS>(f, x, src, S::v_outer(), so, h, n_src, m, [](const int k) { return S::outer(k); });
     cols_forward<LR>(limb, (const typename F::W *)tw_int, f, x, (typename F::E *)lds_raw);
 }
 
-// Register budget of three waves per SIMD (168): left alone the compiler takes 170 - 176 registers, which leaves two
-// waves (measured 15 % slower); four waves (128 registers) only with about 86 spilled ones (18 % slower).
+// Eight points per thread: 96 - 108 registers, four waves per SIMD (sixteen points: 154 - 166, three waves).  1200 workgroups
+// (24 primes of 60 bits, level 20) 38 -> 35 us, 64 polynomials x 6 limbs 2 % less of the whole projection.
 template <int LR, int NS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void ntt16_cols_converted_kernel(
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void ntt16_cols_converted_kernel(
     u64 *__restrict__ data, const Tw *__restrict__ tw_all, const ModQ *__restrict__ modq, const u64 *__restrict__ ninv,
     const u64 *__restrict__ ninv_s, const double *__restrict__ fp, LimbList ll, LimbList sl, int n_limbs,
     size_t poly_stride, ConvSources cs) {
     __shared__ u64 lds[256 * 16];
     const int per_poly = n_limbs + cs.n_copy;
     const int limb = blockIdx.y % per_poly, poly = blockIdx.y / per_poly;
-    typedef Slab<LR> S;
+    typedef Slab<LR, 8> S;
     if (limb >= n_limbs) {   // a limb that is only copied into its slot
         const u64 *from = cs.copy_src + (size_t)poly * cs.copy_src_stride +
                           ((size_t)cs.copy_src_slot[limb - n_limbs] << (8 + LR));
         u64 *base = data + (size_t)poly * poly_stride + ((size_t)cs.copy_dst_slot[limb - n_limbs] << (8 + LR)) + S::col();
-        const u32 rh = S::rh();
-        u64 t[16];
+        u64 t[8];
         if (cs.copy_galois != 0) {   // the copy of the source's automorphism
 #pragma unroll
-            for (int k = 0; k < 16; k++)
-                t[k] = from[galois_index(((rh + S::Q * k) << 8) + S::col(), cs.copy_galois, 8 + LR)];
+            for (int k = 0; k < 8; k++)
+                t[k] = from[galois_index(((u32)S::r_outer_w(k) << 8) + S::col(), cs.copy_galois, 8 + LR)];
         } else {
 #pragma unroll
-            for (int k = 0; k < 16; k++) t[k] = from[((rh + S::Q * k) << 8) + S::col()];
+            for (int k = 0; k < 8; k++) t[k] = from[((u32)S::r_outer_w(k) << 8) + S::col()];
         }
 #pragma unroll
-        for (int k = 0; k < 16; k++) base[(rh + S::Q * k) << 8] = t[k];
+        for (int k = 0; k < 8; k++) base[(u32)S::r_outer_w(k) << 8] = t[k];
         return;
     }
     const __amdgpu_buffer_rsrc_t base = limb_rsrc(
@@ -248,14 +252,14 @@ template <int LR, class F>
 __device__ __forceinline__ void cols_lifted_body(const __amdgpu_buffer_rsrc_t limb, const Tw *__restrict__ tw_int, const F f,
                                                  u64 *lds_raw, const LiftSource &ls, const long long *__restrict__ coef,
                                                  const ModQ m) {
-    typedef Slab<LR> S;
-    typename F::E x[16];
+    typedef Slab<LR, 8> S;
+    typename F::E x[8];
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = f.from_canonical(lifted(ls, coef, ((S::rh() + S::Q * k) << 8) + S::col(), m));
+    for (int k = 0; k < 8; k++) x[k] = f.from_canonical(lifted(ls, coef, ((u32)S::r_outer_s(k) << 8) + S::col(), m));
     cols_forward<LR>(limb, (const typename F::W *)tw_int, f, x, (typename F::E *)lds_raw);
 }
 template <int LR>
-__global__ __launch_bounds__(256) void ntt16_cols_lifted_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
+__global__ __launch_bounds__(512) void ntt16_cols_lifted_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
                                                                 const ModQ *__restrict__ modq, const double *__restrict__ fp,
                                                                 LimbList ll, LimbList sl, int n_limbs, size_t poly_stride,
                                                                 LiftSource ls) {
@@ -423,19 +427,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 // LR: log2 of the rows of a limb, or 0: taken from the argument (the address arithmetic of N = 2^16 folds into constants:
 // 1 - 1.5 % of a single rotation or ciphertext product)
-template <int LR, bool INV, int TAIL, int LOAD>
+template <int LR, int P, bool INV, int TAIL, int LOAD>
 __global__ __launch_bounds__(256) void ntt16_rows_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
                                                          const Tw *__restrict__ rtw_all,
                                                          const ModQ *__restrict__ modq, const double *__restrict__ fp,
                                                          LimbList ll, LimbList sl, int n_limbs, size_t poly_stride,
                                                          NttEpilogue ep, const int log_r_arg) {
-    __shared__ u64 lds[16 * ROWPAD];
+    constexpr int RB = P == 16 ? 4 : 3;   // log2 of the rows of a workgroup
+    __shared__ u64 lds[ROWPAD << RB];
     const int log_r = LR != 0 ? LR : log_r_arg;
     // The second radix-16 block of a row pass walks 1/16 of the prime's twiddle table per 16-row slab (as
     // many bytes as the slab's data), identical for every polynomial of the batch.  Workgroups are dealt
     // round-robin to the 8 XCDs, so the polynomials of one (limb, slab) pair are placed back to back on
     // one XCD and share those twiddles through its L2 instead of fetching them from HBM once each.
-    const u32 groups = (u32)n_limbs << (log_r - 4), n_polys = gridDim.x / groups;
+    const u32 groups = (u32)n_limbs << (log_r - RB), n_polys = gridDim.x / groups;
     u32 poly, group;
     if ((groups & 7u) == 0) {
         const u32 xcd = blockIdx.x & 7u, slot = blockIdx.x >> 3;
@@ -445,12 +450,12 @@ __global__ __launch_bounds__(256) void ntt16_rows_kernel(u64 *__restrict__ data,
         poly = blockIdx.x % n_polys;
         group = blockIdx.x / n_polys;
     }
-    const int limb = (int)(group >> (log_r - 4));
-    const u32 slab = group & ((1u << (log_r - 4)) - 1u);
+    const int limb = (int)(group >> (log_r - RB));
+    const u32 slab = group & ((1u << (log_r - RB)) - 1u);
     const int log_n = 8 + log_r;
     const int prime = ll.idx[limb];
     const Tw *tw = tw_all + ((size_t)prime << log_n), *rtw = rtw_all + ((size_t)prime << log_n);
-    const u32 r = slab * 16 + (threadIdx.x >> 4);  // global row
+    const u32 r = (slab << RB) + (Lanes<P>::t() >> 4);  // global row
     u64 *row = data + (size_t)poly * poly_stride + ((size_t)sl.idx[limb] << log_n) + ((size_t)r << 8);
     const u64 *mn = nullptr;
     u64 *o = nullptr;
@@ -478,13 +483,13 @@ __global__ __launch_bounds__(256) void ntt16_rows_kernel(u64 *__restrict__ data,
     }
     const u32 gal = LOAD == LOAD_ROTATED ? ep.galois : 0u;
     if (fp[4 * prime] != 0.0)
-        rows_body<INV, TAIL, LOAD, false>(row, tw, rtw, FpField(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld, gal,
+        rows_body<P, INV, TAIL, LOAD, false>(row, tw, rtw, FpField(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld, gal,
                                             sec);
     else if (INV || (modq[prime].q >> 60) != 0)
-        rows_body<INV, TAIL, LOAD, false>(row, tw, rtw, IntField(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld, gal,
+        rows_body<P, INV, TAIL, LOAD, false>(row, tw, rtw, IntField(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld, gal,
                                             sec);
     else
-        rows_body<INV, TAIL, LOAD, false>(row, tw, rtw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld,
+        rows_body<P, INV, TAIL, LOAD, false>(row, tw, rtw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld,
                                             gal, sec);
 }
 
@@ -498,18 +503,33 @@ void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, c
                          size_t poly_stride, hipStream_t s, const void *final_scale, const NttEpilogue &from, int load);
 
 // ---- launches of single passes (rings of 2^13 points and more) -------------------------------------------------------
+// Which passes give a thread eight points instead of sixteen (ntt_device.h, Lanes).  Passes that begin in a basis conversion
+// or a lift, and inverse row passes, always do: they fit four waves per SIMD instead of three resp. eight instead of four.
+// The others only where the launch leaves the chip part empty, since in a full one the second twiddle and address of each
+// pair of lanes is work for nothing (workgroups of 4096 points, 60-bit primes):
+//   columns: 64 workgroups 13.9 -> 13.5 us a forward transform, 15.0 -> 14.1 an inverse one; 384: 25.6 -> 25.5; 768: 31.5 -> 32.5;
+//            6144: 171 -> 180
+//   forward rows: up to the 640 that are resident at once with 87 registers (five waves): 64: 13.9 -> 12.0 us, 384: 25.6 -> 24.3,
+//            672 with the fused tail +5 us (a second round), 6144: 171 -> 179
+// Together, with the conversions: rotation at 24 primes of 60 bits, level 20: 172 -> 162 us, level 7: 100 -> 81; product at level 9
+// 153 -> 134; rotation at N = 2^13 66 -> 53.
+static bool few_for_columns(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 512; }
+static bool few_for_rows(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 640; }
+
 static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbList &ll, const LimbList &sl, int n_limbs,
                       int n_polys, size_t poly_stride, hipStream_t s, const void *final_scale = nullptr) {
-    const dim3 grid((unsigned)(c->N >> 12), (unsigned)(n_limbs * n_polys)), block(256);
+    const dim3 grid((unsigned)(c->N >> 12), (unsigned)(n_limbs * n_polys));
+    const bool few = few_for_columns(c, n_limbs * n_polys);
     const Tw *tw = (const Tw *)(inverse ? c->d_iw : c->d_w);
-#define COLS(LR)                                                                                                            \
-    do {                                                                                                                    \
-        if (inverse)                                                                                                        \
-            hipLaunchKernelGGL((ntt16_cols_kernel<LR, true>), grid, block, 0, s, d, tw, c->d_modq, c->d_ninv, c->d_ninv_s,  \
-                               c->d_fp, ll, sl, n_limbs, poly_stride, (const Tw *)final_scale);                             \
-        else                                                                                                                \
-            hipLaunchKernelGGL((ntt16_cols_kernel<LR, false>), grid, block, 0, s, d, tw, c->d_modq, c->d_ninv, c->d_ninv_s, \
-                               c->d_fp, ll, sl, n_limbs, poly_stride, (const Tw *)nullptr);                                 \
+#define COLS_FORM(LR, P, INV)                                                                                             \
+    hipLaunchKernelGGL((ntt16_cols_kernel<LR, P, INV>), grid, dim3(4096 / P), 0, s, d, tw, c->d_modq, c->d_ninv,          \
+                       c->d_ninv_s, c->d_fp, ll, sl, n_limbs, poly_stride, (const Tw *)(INV ? final_scale : nullptr))
+#define COLS(LR)                                    \
+    do {                                            \
+        if (inverse && few) COLS_FORM(LR, 8, true); \
+        else if (inverse) COLS_FORM(LR, 16, true);  \
+        else if (few) COLS_FORM(LR, 8, false);      \
+        else COLS_FORM(LR, 16, false);              \
     } while (0)
     switch (c->logN) {
         case 13: COLS(5); break;
@@ -518,32 +538,40 @@ static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
         default: COLS(8); break;
     }
 #undef COLS
+#undef COLS_FORM
 }
 static void rows_pass(const hemm_context *c, bool inverse, u64 *d, const LimbList &ll, const LimbList &sl, int n_limbs,
                       int n_polys, size_t poly_stride, hipStream_t s, const NttEpilogue &ep, int tail = TAIL_NONE,
                       int load = LOAD_PLAIN) {
-    const dim3 grid((unsigned)(c->N >> 12) * (unsigned)(n_limbs * n_polys)), block(256);
+    const bool few = inverse || few_for_rows(c, n_limbs * n_polys);
+    const dim3 grid((unsigned)(c->N >> (few ? 11 : 12)) * (unsigned)(n_limbs * n_polys)), block(256);
     const int log_r = c->logN - 8;
-#define ROWS(LR, INV, TAIL, LOAD)                                                                                          \
-    hipLaunchKernelGGL((ntt16_rows_kernel<LR, INV, TAIL, LOAD>), grid, block, 0, s, d, (const Tw *)(INV ? c->d_iw : c->d_w), \
+#define ROWS(LR, P, INV, TAIL, LOAD)                                                                                          \
+    hipLaunchKernelGGL((ntt16_rows_kernel<LR, P, INV, TAIL, LOAD>), grid, block, 0, s, d, (const Tw *)(INV ? c->d_iw : c->d_w), \
                        (const Tw *)(INV ? c->d_irw : c->d_rw), c->d_modq, c->d_fp, ll, sl, n_limbs, poly_stride, ep, log_r)
-#define ROWS_RING(INV, TAIL, LOAD)                          \
-    do {                                                    \
-        if (log_r == 8) ROWS(8, INV, TAIL, LOAD);           \
-        else ROWS(0, INV, TAIL, LOAD);                      \
+#define ROWS_RING(P, INV, TAIL, LOAD)                  \
+    do {                                               \
+        if (log_r == 8) ROWS(8, P, INV, TAIL, LOAD);   \
+        else ROWS(0, P, INV, TAIL, LOAD);              \
+    } while (0)
+#define ROWS_FORWARD(TAIL)                                   \
+    do {                                                     \
+        if (few) ROWS_RING(8, false, TAIL, LOAD_PLAIN);      \
+        else ROWS_RING(16, false, TAIL, LOAD_PLAIN);         \
     } while (0)
     if (inverse && load == LOAD_ROTATED)
-        ROWS_RING(true, TAIL_NONE, LOAD_ROTATED);
+        ROWS_RING(8, true, TAIL_NONE, LOAD_ROTATED);
     else if (inverse && load == LOAD_DECRYPT)
-        ROWS_RING(true, TAIL_NONE, LOAD_DECRYPT);
+        ROWS_RING(8, true, TAIL_NONE, LOAD_DECRYPT);
     else if (inverse)
-        ROWS_RING(true, TAIL_NONE, LOAD_PLAIN);
+        ROWS_RING(8, true, TAIL_NONE, LOAD_PLAIN);
     else if (tail == TAIL_SUB_SCALE)
-        ROWS_RING(false, TAIL_SUB_SCALE, LOAD_PLAIN);
+        ROWS_FORWARD(TAIL_SUB_SCALE);
     else if (tail == TAIL_ENCRYPT)
-        ROWS_RING(false, TAIL_ENCRYPT, LOAD_PLAIN);
+        ROWS_FORWARD(TAIL_ENCRYPT);
     else
-        ROWS_RING(false, TAIL_NONE, LOAD_PLAIN);
+        ROWS_FORWARD(TAIL_NONE);
+#undef ROWS_FORWARD
 #undef ROWS_RING
 #undef ROWS
 }
@@ -640,9 +668,9 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
                             tail ? TAIL_SUB_SCALE : TAIL_NONE);
         return true;
     }
-    const dim3 block(256), grid((unsigned)(c->N >> 12), (n_limbs + cs.n_copy) * n_polys);
-#define CONV_CASE(LR, K)                                                                                               \
-    hipLaunchKernelGGL((ntt16_cols_converted_kernel<LR, K>), grid, block, 0, s, data, (const Tw *)c->d_w, c->d_modq, \
+    const dim3 grid((unsigned)(c->N >> 12), (n_limbs + cs.n_copy) * n_polys);
+#define CONV_CASE(LR, K)                                                                                                     \
+    hipLaunchKernelGGL((ntt16_cols_converted_kernel<LR, K>), grid, dim3(512), 0, s, data, (const Tw *)c->d_w, c->d_modq, \
                        c->d_ninv, c->d_ninv_s, c->d_fp, ll, sl, n_limbs, poly_stride, cs)
 #define CONV_RING(LR)                      \
     do {                                   \
@@ -781,9 +809,9 @@ bool launch_ntt_lifted(const hemm_context *c, const LiftSource &ls, u64 *data, c
         u64 *d = data + (size_t)p0 * poly_stride;
         LiftSource l = ls;
         l.coef += (size_t)p0 * ls.stride;
-        const dim3 grid((unsigned)(c->N >> 12), (unsigned)(n_limbs * np)), block(256);
-#define LIFTED(LR)                                                                                                       \
-    hipLaunchKernelGGL(ntt16_cols_lifted_kernel<LR>, grid, block, 0, s, d, (const Tw *)c->d_w, c->d_modq, c->d_fp, ll, sl, \
+        const dim3 grid((unsigned)(c->N >> 12), (unsigned)(n_limbs * np));
+#define LIFTED(LR)                                                                                                         \
+    hipLaunchKernelGGL(ntt16_cols_lifted_kernel<LR>, grid, dim3(512), 0, s, d, (const Tw *)c->d_w, c->d_modq, c->d_fp, ll, sl, \
                        n_limbs, poly_stride, l)
         switch (c->logN) {
             case 13: LIFTED(5); break;

@@ -124,8 +124,8 @@ struct IntFieldT {
         y = u - v + q4;
     }
     __device__ __forceinline__ void gs(E &x, E &y, const W tw) const { gs_bfly(x, y, tw, q, q4, nq4); }
-    template <int T>
-    __device__ __forceinline__ void after_inverse_block(E (&)[16]) const {}
+    template <int T, int P>
+    __device__ __forceinline__ void after_inverse_block(E (&)[P]) const {}
     __device__ __forceinline__ u64 to_canonical(E v) const {   // v < 8q (16q with LAZY16)
         if (LAZY16) v = csub(v, 2 * q4, nq8);
         return csub(csub(csub(v, q4, nq4), q2, nq2), q, nq1);
@@ -191,10 +191,11 @@ struct FpField {
     // largest value it multiplies is 2^T B.  With element 0 of every sub-block (and element 1 where T = 4) reduced after
     // each block every block starts from B <= 4 r: r <= 0.8 q gives B <= 3.2 q and 16 B <= 51 q < 2^49.7 (q < 2^44), for
     // which r <= 0.8 q holds again; products of values below 2^50 are still exact.
-    template <int T>
-    __device__ __forceinline__ void after_inverse_block(E (&x)[16]) const {
+    // (Eight registers per thread: the upper half of a block of four stages has its elements 4 and 5 reduced as well.)
+    template <int T, int P>
+    __device__ __forceinline__ void after_inverse_block(E (&x)[P]) const {
 #pragma unroll
-        for (int k = 0; k < 16; k += 1 << T) x[k] = reduce(x[k]);
+        for (int k = 0; k < P; k += 1 << T) x[k] = reduce(x[k]);
         if (T == 4) x[1] = reduce(x[1]);
     }
     __device__ __forceinline__ u64 centred_to_canonical(E r) const {
@@ -209,67 +210,118 @@ struct FpField {
     }
 };
 
-// T Cooley-Tukey stages on 16 registers that hold 16 >> T sub-blocks of 2^T consecutive points; stage s, group g uses
-// twiddle (X << s) + g.  SAME: the sub-blocks are different columns of one block and share its twiddles.
-template <int T, bool SAME = false, class F>
-__device__ __forceinline__ void radix_fwd(const F &f, typename F::E (&x)[16], const typename F::W *__restrict__ tw,
-                                          const u32 X) {
+// How a block of up to four stages on 16 points lies in registers.  P = 16: one thread holds the block.  P = 8: two lanes of a
+// wavefront 32 apart hold eight points each, h = 0 and 1; the threads that share a block are otherwise numbered as with
+// P = 16 (t).  Two layouts: `whole`, lane h holds points 8h .. 8h + 7, in which every stage of a distance below 8 is local,
+// and `split`, lane h holds points 4h .. 4h + 3 and 8 + 4h .. 8 + 4h + 3, in which the stage of distance 8 is; one
+// v_permlane32_swap_b32 per register pair turns one into the other.  T < 4 stages only ever use `whole`.
+// A thread of 16 points is one wavefront per SIMD in a launch of up to 256 workgroups, and then its load latencies and the
+// dependences of 64-bit products are what the launch takes; eight points per thread put two wavefronts there with half
+// the instructions each.  The arithmetic of every point, and with it the residues, is the same.
+template <int P>
+struct Lanes {
+    static __device__ __forceinline__ u32 t() { return P == 16 ? threadIdx.x : (threadIdx.x & 31u) | ((threadIdx.x >> 6) << 5); }
+    static __device__ __forceinline__ u32 h() { return P == 16 ? 0u : (threadIdx.x >> 5) & 1u; }
+    // point of register k: a constant and the lane's part
+    template <int T>
+    static __device__ __forceinline__ constexpr int split(const int k) { return P == 16 || T < 4 ? k : (k & 3) + 8 * (k >> 2); }
+    template <int T>
+    static __device__ __forceinline__ u32 h_split() { return (P == 16 || T < 4 ? 8u : 4u) * h(); }
+    static __device__ __forceinline__ u32 h_whole() { return 8u * h(); }
+};
+// split <-> whole
+__device__ __forceinline__ void swap_halves(u64 &a, u64 &b) {
+    const u32x2 lo = __builtin_amdgcn_permlane32_swap((u32)a, (u32)b, false, false);
+    const u32x2 hi = __builtin_amdgcn_permlane32_swap((u32)(a >> 32), (u32)(b >> 32), false, false);
+    a = ((u64)hi.x << 32) | lo.x;
+    b = ((u64)hi.y << 32) | lo.y;
+}
+template <class E>
+__device__ __forceinline__ void swap_layout(E (&x)[8]) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        u64 a, b;
+        __builtin_memcpy(&a, &x[k], 8);
+        __builtin_memcpy(&b, &x[k + 4], 8);
+        swap_halves(a, b);
+        __builtin_memcpy(&x[k], &a, 8);
+        __builtin_memcpy(&x[k + 4], &b, 8);
+    }
+}
+template <class E>
+__device__ __forceinline__ void swap_layout(E (&)[16]) {}
+
+// T Cooley-Tukey stages on 16 points that are 16 >> T sub-blocks of 2^T consecutive ones; stage s, group g uses twiddle
+// tw(s, g).  Points come in as `split` and leave as `whole`.
+template <int T, int P, class F, class TW>
+__device__ __forceinline__ void stages_fwd(const F &f, typename F::E (&x)[P], const TW tw) {
+    const u32 h = Lanes<P>::h();
 #pragma unroll
     for (int s = 0; s < T; s++) {
         const int d = 1 << (T - 1 - s);
+        if (P == 8 && d == 8) {   // the first stage of four, in the split layout
+            const typename F::W w = tw(0, 0u);
 #pragma unroll
-        for (int g = 0; g < 8 / d; g++) {
-            const typename F::W w = tw[(X << s) + (SAME ? g & ((1 << s) - 1) : g)];
+            for (int j = 0; j < 4; j++) f.ct(x[j], x[j + 4], w, false);
+            swap_layout(x);
+        } else {
 #pragma unroll
-            for (int j = 0; j < d; j++) f.ct(x[g * 2 * d + j], x[g * 2 * d + j + d], w, (s & 1) != 0);
+            for (int g = 0; g < P / 2 / d; g++) {
+                const typename F::W w = tw(s, h * (u32)(8 / 2 / d) + (u32)g);
+#pragma unroll
+                for (int j = 0; j < d; j++) f.ct(x[g * 2 * d + j], x[g * 2 * d + j + d], w, (s & 1) != 0);
+            }
         }
     }
 }
-// T Gentleman-Sande stages; stage s (distance 1 << s), group g uses twiddle (X << (T - 1 - s)) + g.
-template <int T, bool SAME = false, class F>
-__device__ __forceinline__ void radix_inv(const F &f, typename F::E (&x)[16], const typename F::W *__restrict__ tw,
-                                          const u32 X) {
+// T Gentleman-Sande stages, the other way round: `whole` in, `split` out; stage s has distance 1 << s.
+template <int T, int P, class F, class TW>
+__device__ __forceinline__ void stages_inv(const F &f, typename F::E (&x)[P], const TW tw) {
+    const u32 h = Lanes<P>::h();
 #pragma unroll
     for (int s = 0; s < T; s++) {
         const int d = 1 << s;
+        if (P == 8 && d == 8) {
+            swap_layout(x);
+            const typename F::W w = tw(3, 0u);
 #pragma unroll
-        for (int g = 0; g < (8 >> s); g++) {
-            const typename F::W w = tw[(X << (T - 1 - s)) + (SAME ? g & ((1 << (T - 1 - s)) - 1) : g)];
+            for (int j = 0; j < 4; j++) f.gs(x[j], x[j + 4], w);
+        } else {
 #pragma unroll
-            for (int j = 0; j < d; j++) f.gs(x[g * 2 * d + j], x[g * 2 * d + j + d], w);
+            for (int g = 0; g < P / 2 / d; g++) {
+                const typename F::W w = tw(s, h * (u32)(8 / 2 / d) + (u32)g);
+#pragma unroll
+                for (int j = 0; j < d; j++) f.gs(x[g * 2 * d + j], x[g * 2 * d + j + d], w);
+            }
         }
     }
+}
+// Blocks on the stage-ordered table: forward stage s, group g: entry (X << s) + g; inverse: (X << (T - 1 - s)) + g.  SAME: the
+// sub-blocks are different columns of one block and share its twiddles.
+template <int T, bool SAME = false, int P, class F>
+__device__ __forceinline__ void radix_fwd(const F &f, typename F::E (&x)[P], const typename F::W *__restrict__ tw,
+                                          const u32 X) {
+    stages_fwd<T>(f, x, [&](const int s, const u32 g) { return tw[(X << s) + (SAME ? g & ((1u << s) - 1u) : g)]; });
+}
+template <int T, bool SAME = false, int P, class F>
+__device__ __forceinline__ void radix_inv(const F &f, typename F::E (&x)[P], const typename F::W *__restrict__ tw,
+                                          const u32 X) {
+    stages_inv<T>(f, x, [&](const int s, const u32 g) {
+        return tw[(X << (T - 1 - s)) + (SAME ? g & ((1u << (T - 1 - s)) - 1u) : g)];
+    });
 }
 
 // The inner radix-16 block of a row pass (X = 16 (R + r) + c: a different X for every thread) reads its 15 twiddles
 // from a table laid out for it: entry ((r * 15 + slot) * 16 + c), slot = 2^l - 1 + g for twiddle (X << l) + g, so that
 // the 16 threads of a row read 16 consecutive entries per (l, g) -- from the stage-ordered table they would read 16
 // entries 2^l apart, up to 64 cache lines per load instruction of a wavefront instead of 8.
-template <class F>
-__device__ __forceinline__ void radix16_fwd_rows(const F &f, typename F::E (&x)[16], const typename F::W *__restrict__ rt) {
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-        const int d = 8 >> s;
-#pragma unroll
-        for (int g = 0; g < (1 << s); g++) {
-            const typename F::W w = rt[((1 << s) - 1 + g) * 16];
-#pragma unroll
-            for (int j = 0; j < d; j++) f.ct(x[g * 2 * d + j], x[g * 2 * d + j + d], w, (s & 1) != 0);
-        }
-    }
+template <int P, class F>
+__device__ __forceinline__ void radix16_fwd_rows(const F &f, typename F::E (&x)[P], const typename F::W *__restrict__ rt) {
+    stages_fwd<4>(f, x, [&](const int s, const u32 g) { return rt[((1u << s) - 1u + g) * 16u]; });
 }
-template <class F>
-__device__ __forceinline__ void radix16_inv_rows(const F &f, typename F::E (&x)[16], const typename F::W *__restrict__ rt) {
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-        const int d = 1 << s;
-#pragma unroll
-        for (int g = 0; g < (8 >> s); g++) {
-            const typename F::W w = rt[((8 >> s) - 1 + g) * 16];
-#pragma unroll
-            for (int j = 0; j < d; j++) f.gs(x[g * 2 * d + j], x[g * 2 * d + j + d], w);
-        }
-    }
+template <int P, class F>
+__device__ __forceinline__ void radix16_inv_rows(const F &f, typename F::E (&x)[P], const typename F::W *__restrict__ rt) {
+    stages_inv<4>(f, x, [&](const int s, const u32 g) { return rt[((8u >> s) - 1u + g) * 16u]; });
 }
 
 #define ROWPAD 272  // 256 residues of a row + one pad word per 16, so a 16-lane column read
@@ -289,17 +341,17 @@ __device__ __forceinline__ u64 lifted(const LiftSource &ls, const long long *__r
     const int e = sample_error(ls.error_key, n);
     return addmod(r, e >= 0 ? (u64)e : m.q - (u64)(-e), m.q);
 }
-// The 16 coefficients of a thread as a basis conversion computed on the fly: coefficient k is sum_i v_i * hat_i mod q
+// The P coefficients of a thread as a basis conversion computed on the fly: coefficient k is sum_i v_i * hat_i mod q
 // over the n_src <= NS source limbs (pre-scaled, the same lazy sums and reductions as the stand-alone conversion kernels,
 // so the residues are the same), read at voff + off(k) inside a limb; so[i]: byte offset of source limb i.
-template <int NS, class F, class OFF>
-__device__ __forceinline__ void converted_inputs(const F &f, typename F::E (&x)[16], const __amdgpu_buffer_rsrc_t src,
+template <int NS, int P, class F, class OFF>
+__device__ __forceinline__ void converted_inputs(const F &f, typename F::E (&x)[P], const __amdgpu_buffer_rsrc_t src,
                                                  const u32 voff, const u32 (&so)[NS], const u64 (&h)[NS], const int n_src,
                                                  const ModQ m, const OFF off) {
     // eight coefficients at a time (three accumulators each), source by source, so that the eight loads of one source
     // limb are in flight together
 #pragma unroll
-    for (int half = 0; half < 2; half++) {
+    for (int half = 0; half < P / 8; half++) {
         Dot3 d[8];
 #pragma unroll
         for (int k = 0; k < 8; k++) dot3_clear(d[k]);
@@ -321,7 +373,7 @@ __device__ __forceinline__ void converted_inputs(const F &f, typename F::E (&x)[
     }
 }
 
-// A row's 16 threads sit in one wavefront (thread = row * 16 + column group), so the LDS exchanges of
+// A row's 16 threads (32 with eight points each) sit in one wavefront, so the LDS exchanges of
 // the row kernel never cross a wavefront: ordering them needs no workgroup barrier, only a fence that
 // keeps the compiler from moving LDS accesses across it.
 __device__ __forceinline__ void wave_sync() {
@@ -354,84 +406,98 @@ struct RowSecond {
 // group of 16 residues stays an aligned group under the automorphism, so the loads touch the same number of lines
 // IN_LDS: the row pass follows (forward) or precedes (inverse) a column pass over the same limb in the same workgroup: the
 // row is taken from, resp. left in, its padded LDS row instead of memory.
-template <bool INV, int TAIL, int LOAD, bool IN_LDS, class F>
+template <int P, bool INV, int TAIL, int LOAD, bool IN_LDS, class F>
 __device__ __forceinline__ void rows_body(u64 *__restrict__ row, const Tw *__restrict__ tw_int,
                                           const Tw *__restrict__ rtw_int, const F f, u64 *lds_raw, const int log_r, const u32 r,
                                           const u64 *__restrict__ mn, u64 *__restrict__ o, const Tw cst,
                                           const u64 *__restrict__ ld, const u32 gal, const RowSecond &sec) {
     typedef typename F::E E;
+    typedef Lanes<P> L;
     const typename F::W *tw = (const typename F::W *)tw_int;
-    const int c = threadIdx.x & 15, rr = threadIdx.x >> 4;
+    const int c = L::t() & 15, rr = L::t() >> 4;
     const typename F::W *rt = (const typename F::W *)rtw_int + (r * 15u * 16u + (u32)c);
     E *l = (E *)lds_raw + rr * ROWPAD;
     u64 *lc = lds_raw + rr * ROWPAD;
     E *mem = (E *)row;
-    E x[16];
+    // residues of a thread: c + 16 e for the points e of the outer block, 16 c + e for the inner one, and from and to
+    // memory in canonical form c + 16 e with the lanes of a pair side by side (e = 2 k + h)
+    const int cs = c + 16 * (int)L::template h_split<4>(), cw = c + 16 * (int)L::h_whole();
+    const int is = 16 * c + (int)L::template h_split<4>(), iw = 16 * c + (int)L::h_whole();
+    const int cm = c + 16 * (int)L::h();
+    constexpr int step = 256 / P;
+    E x[P];
     if (!INV) {
 #pragma unroll
-        for (int k = 0; k < 16; k++) x[k] = IN_LDS ? l[padc(c + 16 * k)] : mem[c + 16 * k];
+        for (int k = 0; k < P; k++) {
+            const int e = cs + 16 * L::template split<4>(k);
+            x[k] = IN_LDS ? l[padc(e)] : mem[e];
+        }
         radix_fwd<4>(f, x, tw, (1u << log_r) + r);
+        if (IN_LDS && P == 8) wave_sync();   // both lanes of a pair have read before either writes
 #pragma unroll
-        for (int k = 0; k < 16; k++) l[padc(c + 16 * k)] = x[k];
+        for (int k = 0; k < P; k++) l[padc(cw + 16 * k)] = x[k];
         wave_sync();
 #pragma unroll
-        for (int k = 0; k < 16; k++) x[k] = l[padc(16 * c + k)];
+        for (int k = 0; k < P; k++) x[k] = l[padc(is + L::template split<4>(k))];
         // the minuend of the fused tail is fetched under the second radix-16 block instead of after it
-        u64 mv[TAIL == TAIL_SUB_SCALE ? 16 : 1];
+        u64 mv[TAIL == TAIL_SUB_SCALE ? P : 1];
         if (TAIL == TAIL_SUB_SCALE) {
 #pragma unroll
-            for (int k = 0; k < 16; k++) mv[k] = __builtin_nontemporal_load(mn + c + 16 * k);
+            for (int k = 0; k < P; k++) mv[k] = __builtin_nontemporal_load(mn + cm + step * k);
         }
         radix16_fwd_rows(f, x, rt);
         wave_sync();
 #pragma unroll
-        for (int k = 0; k < 16; k++) l[padc(16 * c + k)] = x[k];
+        for (int k = 0; k < P; k++) l[padc(iw + k)] = x[k];
         wave_sync();
         if (TAIL == TAIL_SUB_SCALE) {
 #pragma unroll
-            for (int k = 0; k < 16; k++) o[c + 16 * k] = f.sub_scale(l[padc(c + 16 * k)], mv[k], cst);
+            for (int k = 0; k < P; k++) o[cm + step * k] = f.sub_scale(l[padc(cm + step * k)], mv[k], cst);
         } else if (TAIL == TAIL_ENCRYPT) {
 #pragma unroll 4
-            for (int k = 0; k < 16; k++) {
-                const u64 a = sample_uniform(sec.key, (r << 8) + (u32)(c + 16 * k), sec.m);
-                o[c + 16 * k] = submod(f.to_canonical(l[padc(c + 16 * k)]), mulmod(a, sec.sk[c + 16 * k], sec.m), sec.m.q);
-                sec.out[c + 16 * k] = a;
+            for (int k = 0; k < P; k++) {
+                const int e = cm + step * k;
+                const u64 a = sample_uniform(sec.key, (r << 8) + (u32)e, sec.m);
+                o[e] = submod(f.to_canonical(l[padc(e)]), mulmod(a, sec.sk[e], sec.m), sec.m.q);
+                sec.out[e] = a;
             }
         } else {
 #pragma unroll
-            for (int k = 0; k < 16; k++) row[c + 16 * k] = f.to_canonical(l[padc(c + 16 * k)]);
+            for (int k = 0; k < P; k++) row[cm + step * k] = f.to_canonical(l[padc(cm + step * k)]);
         }
     } else {
         if (LOAD == LOAD_DECRYPT) {
 #pragma unroll 4
-            for (int k = 0; k < 16; k++)
-                lc[padc(c + 16 * k)] = addmod(ld[c + 16 * k], mulmod(sec.in[c + 16 * k], sec.sk[c + 16 * k], sec.m), sec.m.q);
+            for (int k = 0; k < P; k++) {
+                const int e = cm + step * k;
+                lc[padc(e)] = addmod(ld[e], mulmod(sec.in[e], sec.sk[e], sec.m), sec.m.q);
+            }
         } else if (LOAD == LOAD_ROTATED) {
 #pragma unroll
-            for (int k = 0; k < 16; k++) lc[padc(c + 16 * k)] = ld[galois_index((r << 8) + (u32)(c + 16 * k), gal, 8 + log_r)];
+            for (int k = 0; k < P; k++) lc[padc(cm + step * k)] = ld[galois_index((r << 8) + (u32)(cm + step * k), gal, 8 + log_r)];
         } else {
 #pragma unroll
-            for (int k = 0; k < 16; k++) lc[padc(c + 16 * k)] = ld[c + 16 * k];
+            for (int k = 0; k < P; k++) lc[padc(cm + step * k)] = ld[cm + step * k];
         }
         wave_sync();
 #pragma unroll
-        for (int k = 0; k < 16; k++) x[k] = f.from_canonical(lc[padc(16 * c + k)]);
+        for (int k = 0; k < P; k++) x[k] = f.from_canonical(lc[padc(iw + k)]);
         radix16_inv_rows(f, x, rt);
         f.template after_inverse_block<4>(x);
         wave_sync();
 #pragma unroll
-        for (int k = 0; k < 16; k++) l[padc(16 * c + k)] = x[k];
+        for (int k = 0; k < P; k++) l[padc(is + L::template split<4>(k))] = x[k];
         wave_sync();
 #pragma unroll
-        for (int k = 0; k < 16; k++) x[k] = l[padc(c + 16 * k)];
+        for (int k = 0; k < P; k++) x[k] = l[padc(cw + 16 * k)];
         radix_inv<4>(f, x, tw, (1u << log_r) + r);
         f.template after_inverse_block<4>(x);
-        if (IN_LDS) {   // the places this thread has just read
+        if (IN_LDS && P == 8) wave_sync();
 #pragma unroll
-            for (int k = 0; k < 16; k++) l[padc(c + 16 * k)] = x[k];
-        } else {
-#pragma unroll
-            for (int k = 0; k < 16; k++) mem[c + 16 * k] = x[k];
+        for (int k = 0; k < P; k++) {   // IN_LDS: the places this thread, or the other one of its pair, has just read
+            const int e = cs + 16 * L::template split<4>(k);
+            if (IN_LDS) l[padc(e)] = x[k];
+            else mem[e] = x[k];
         }
     }
 }

@@ -4,7 +4,9 @@
 // (R = N / 256) meet in LDS instead of in memory, and a transform that the two-launch kernels would take as two dependent
 // launches is one.  What bounds a call on the small rings is the number of dependent launches, a few microseconds each
 // however little they do, not arithmetic or bytes: one transform of 2^12 points 7 us against 36 us with the butterflies
-// of every stage read from and written to LDS one by one, which these kernels replace.  A thread holds 16 residues: the log2 R
+// of every stage read from and written to LDS one by one, which these kernels replace.  A thread holds eight residues (16 at 2^14 points, where
+// eight would take 2048 threads; with eight a CU has two wavefronts per SIMD on a limb of 2^12 points instead of one: product
+// of two encrypted 32 x 32 tiles 687 -> 595 us): the log2 R
 // column stages in one block (R <= 16) or two, one exchange through LDS after each, then the row pass of the two-launch
 // kernels (two radix-16 blocks).  The first stages can read their input from a
 // basis conversion, the last ones can end in (minuend - v) * constant, and an inverse transform can read its input
@@ -16,75 +18,82 @@
 
 namespace {
 
-template <int LR>
+template <int LR, int P>
 struct Limb {
+    typedef Lanes<P> L;
     static constexpr int R = 1 << LR, NT = 16 << LR;   // rows, threads
     static constexpr int Q = LR > 4 ? R / 16 : 1;      // LR > 4: two column blocks, of four stages and of LR - 4
     static constexpr int T1 = LR > 4 ? 4 : LR, T2 = LR - T1;
     // R <= 16: element k of a thread is row k % R of column threadIdx.x + NT * (k / R); otherwise row rh + Q k of column
     // threadIdx.x % 256 in the first block and row 16 rh + k in the second, rh = threadIdx.x / 256
-    static __device__ __forceinline__ int rh() { return LR > 4 ? (int)(threadIdx.x >> 8) : 0; }
-    static __device__ __forceinline__ int row(const int k) { return LR > 4 ? rh() + Q * k : k & (R - 1); }
-    static __device__ __forceinline__ int col(const int k) {
-        return LR > 4 ? (int)(threadIdx.x & 255) : (int)threadIdx.x + NT * (k / R);
+    static __device__ __forceinline__ u32 t() { return L::t(); }
+    static __device__ __forceinline__ int rh() { return LR > 4 ? (int)(t() >> 8) : 0; }
+    // row and column of point e of the first block
+    static __device__ __forceinline__ int row(const int e) { return LR > 4 ? rh() + Q * e : e & (R - 1); }
+    static __device__ __forceinline__ int col(const int e) { return LR > 4 ? (int)(t() & 255) : (int)t() + NT * (e / R); }
+    // byte offset inside the limb of the first block's points (split): a thread's part and the step to register k
+    static __device__ __forceinline__ constexpr u32 step(const u32 e) {
+        return LR > 4 ? e * (u32)(Q * 2048) : (e & (R - 1)) * 2048u + (e / R) * (u32)(NT * 8);
     }
-    // byte offset inside the limb: a thread's part and the step to element k
-    static __device__ __forceinline__ u32 voff() { return ((LR > 4 ? threadIdx.x & 255 : threadIdx.x) + ((u32)rh() << 8)) * 8u; }
-    static __device__ __forceinline__ constexpr u32 off(const int k) {
-        return LR > 4 ? (u32)(k * Q * 2048) : (u32)((k & (R - 1)) * 2048 + (k / R) * NT * 8);
+    static __device__ __forceinline__ u32 voff() {
+        return ((LR > 4 ? t() & 255 : t()) + ((u32)rh() << 8)) * 8u + step(L::template h_split<T1>());
     }
-    static __device__ __forceinline__ int at(const int k) { return row(k) * ROWPAD + padc(col(k)); }
-    static __device__ __forceinline__ int at2(const int k) { return (16 * rh() + k) * ROWPAD + padc(col(k)); }
+    static __device__ __forceinline__ constexpr u32 off(const int k) { return step((u32)L::template split<T1>(k)); }
+    // places in LDS of register k: of the first block (split, whole) and of the second, which has less than four stages
+    static __device__ __forceinline__ int place(const int e) { return row(e) * ROWPAD + padc(col(e)); }
+    static __device__ __forceinline__ int at_s(const int k) { return place((int)L::template h_split<T1>() + L::template split<T1>(k)); }
+    static __device__ __forceinline__ int at_w(const int k) { return place((int)L::h_whole() + k); }
+    static __device__ __forceinline__ int at2(const int k) { return (16 * rh() + (int)L::h_whole() + k) * ROWPAD + padc(col(0)); }
 };
 
 // NS > 0: the input is a conversion of up to NS sources, LIFTED: the coefficients of an encoding
 enum { LIFTED = -1 };
-template <int LR, int NS, int TAIL, class F>
+template <int LR, int P, int NS, int TAIL, class F>
 __device__ __forceinline__ void limb_forward(u64 *__restrict__ limb, const Tw *__restrict__ tw_int, const Tw *__restrict__ rtw,
                                              const F f, u64 *lds_raw, const __amdgpu_buffer_rsrc_t src,
                                              const u32 (&so)[NS > 0 ? NS : 1], const u64 (&h)[NS > 0 ? NS : 1], const int n_src,
                                              const ModQ m, const LiftSource &ls, const long long *__restrict__ coef,
                                              const u64 *__restrict__ mn, u64 *__restrict__ o, const Tw cst, RowSecond sec) {
     typedef typename F::E E;
-    typedef Limb<LR> S;
+    typedef Limb<LR, P> S;
     E *lds = (E *)lds_raw;
-    E x[16];
+    E x[P];
     if (NS > 0) {
         converted_inputs<(NS > 0 ? NS : 1)>(f, x, src, S::voff(), so, h, n_src, m,
                                             [](const int k) { return S::off(k); });
     } else if (NS == LIFTED) {
 #pragma unroll
-        for (int k = 0; k < 16; k++) x[k] = f.from_canonical(lifted(ls, coef, (S::voff() + S::off(k)) >> 3, m));
+        for (int k = 0; k < P; k++) x[k] = f.from_canonical(lifted(ls, coef, (S::voff() + S::off(k)) >> 3, m));
     } else {
 #pragma unroll
-        for (int k = 0; k < 16; k++) x[k] = f.from_canonical(buf_load<u64>(src, S::voff(), S::off(k)));
+        for (int k = 0; k < P; k++) x[k] = f.from_canonical(buf_load<u64>(src, S::voff(), S::off(k)));
     }
     radix_fwd<S::T1, true>(f, x, (const typename F::W *)tw_int, 1u);
 #pragma unroll
-    for (int k = 0; k < 16; k++) lds[S::at(k)] = x[k];
+    for (int k = 0; k < P; k++) lds[S::at_w(k)] = x[k];
     __syncthreads();
     if (S::T2 > 0) {
 #pragma unroll
-        for (int k = 0; k < 16; k++) x[k] = lds[S::at2(k)];
+        for (int k = 0; k < P; k++) x[k] = lds[S::at2(k)];
         radix_fwd<S::T2>(f, x, (const typename F::W *)tw_int, 16u + (u32)S::rh() * (16 / S::Q));
 #pragma unroll
-        for (int k = 0; k < 16; k++) lds[S::at2(k)] = x[k];   // the places this thread has just read
+        for (int k = 0; k < P; k++) lds[S::at2(k)] = x[k];   // the places this thread has just read
         __syncthreads();
     }
-    const u32 r = threadIdx.x >> 4;
+    const u32 r = Lanes<P>::t() >> 4;
     if (TAIL == TAIL_ENCRYPT) {
         sec.out += r << 8;
         sec.sk += r << 8;
     }
-    rows_body<false, TAIL, LOAD_PLAIN, true>(limb + (r << 8), tw_int, rtw, f, lds_raw, LR, r,
+    rows_body<P, false, TAIL, LOAD_PLAIN, true>(limb + (r << 8), tw_int, rtw, f, lds_raw, LR, r,
                                              TAIL == TAIL_SUB_SCALE ? mn + (r << 8) : nullptr,
                                              TAIL != TAIL_NONE ? o + (r << 8) : nullptr, cst, nullptr, 0, sec);
 }
 
 // data[n_polys][.][N] (polynomial stride poly_stride), limb l in slot sl[l]; the plain copies of cs follow the limbs of a
 // polynomial.
-template <int LR, int NS, int TAIL>
-__global__ __launch_bounds__(16 << LR) void ntt_limb_forward_kernel(
+template <int LR, int P, int NS, int TAIL>
+__global__ __launch_bounds__((256 / P) << LR) void ntt_limb_forward_kernel(
     u64 *__restrict__ data, const Tw *__restrict__ tw_all, const Tw *__restrict__ rtw_all, const ModQ *__restrict__ modq,
     const double *__restrict__ fp, LimbList ll, LimbList sl, int n_limbs, size_t poly_stride, ConvSources cs,
     LiftSource ls, NttEpilogue ep) {
@@ -95,14 +104,14 @@ __global__ __launch_bounds__(16 << LR) void ntt_limb_forward_kernel(
     if (NS > 0 && limb >= n_limbs) {   // a limb that is only copied into its slot
         const u64 *from = cs.copy_src + (size_t)poly * cs.copy_src_stride + ((size_t)cs.copy_src_slot[limb - n_limbs] << log_n);
         u64 *to = data + (size_t)poly * poly_stride + ((size_t)cs.copy_dst_slot[limb - n_limbs] << log_n);
-        u64 t[16];
+        u64 t[P];
 #pragma unroll
-        for (int k = 0; k < 16; k++) {
-            const u32 n = threadIdx.x + (u32)k * (16u << LR);
+        for (int k = 0; k < P; k++) {
+            const u32 n = threadIdx.x + (u32)k * (u32)((256 / P) << LR);
             t[k] = from[cs.copy_galois != 0 ? galois_index(n, cs.copy_galois, log_n) : n];
         }
 #pragma unroll
-        for (int k = 0; k < 16; k++) to[threadIdx.x + (u32)k * (16u << LR)] = t[k];
+        for (int k = 0; k < P; k++) to[threadIdx.x + (u32)k * (u32)((256 / P) << LR)] = t[k];
         return;
     }
     const int prime = __builtin_amdgcn_readfirstlane((int)ll.idx[limb]);   // byte tables are read with vector loads
@@ -141,50 +150,50 @@ __global__ __launch_bounds__(16 << LR) void ntt_limb_forward_kernel(
     }
     const long long *coef = NS == LIFTED ? ls.coef + (size_t)poly * ls.stride : nullptr;
     if (fp[4 * prime] != 0.0)
-        limb_forward<LR, NS, TAIL>(base, tw, rtw, FpField(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, ls,
+        limb_forward<LR, P, NS, TAIL>(base, tw, rtw, FpField(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, ls,
                                    coef, mn, o, cst, sec);
     else if ((m.q >> 60) != 0)
-        limb_forward<LR, NS, TAIL>(base, tw, rtw, IntField(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, ls,
+        limb_forward<LR, P, NS, TAIL>(base, tw, rtw, IntField(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, ls,
                                    coef, mn, o, cst, sec);
     else
-        limb_forward<LR, NS, TAIL>(base, tw, rtw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, ls,
+        limb_forward<LR, P, NS, TAIL>(base, tw, rtw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, ls,
                                    coef, mn, o, cst, sec);
 }
 
-template <int LR, int LOAD, class F>
+template <int LR, int P, int LOAD, class F>
 __device__ __forceinline__ void limb_inverse(u64 *__restrict__ limb, const Tw *__restrict__ tw_int, const Tw *__restrict__ rtw,
                                              const F f, u64 *lds_raw, const u64 *__restrict__ ld, const u32 gal, RowSecond sec) {
     typedef typename F::E E;
-    typedef Limb<LR> S;
+    typedef Limb<LR, P> S;
     E *lds = (E *)lds_raw;
-    const u32 r = threadIdx.x >> 4;
+    const u32 r = Lanes<P>::t() >> 4;
     if (LOAD == LOAD_DECRYPT) {
         sec.in += r << 8;
         sec.sk += r << 8;
     }
-    rows_body<true, TAIL_NONE, LOAD, true>(limb, tw_int, rtw, f, lds_raw, LR, r, nullptr, nullptr, Tw{0, 0},
+    rows_body<P, true, TAIL_NONE, LOAD, true>(limb, tw_int, rtw, f, lds_raw, LR, r, nullptr, nullptr, Tw{0, 0},
                                            LOAD == LOAD_ROTATED ? ld : ld + (r << 8), gal, sec);
     __syncthreads();
-    E x[16];
+    E x[P];
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = lds[S::T2 > 0 ? S::at2(k) : S::at(k)];
+    for (int k = 0; k < P; k++) x[k] = lds[S::T2 > 0 ? S::at2(k) : S::at_w(k)];
     if (S::T2 > 0) {
         radix_inv<S::T2>(f, x, (const typename F::W *)tw_int, 16u + (u32)S::rh() * (16 / S::Q));
         f.template after_inverse_block<S::T2>(x);
 #pragma unroll
-        for (int k = 0; k < 16; k++) lds[S::at2(k)] = x[k];   // the places this thread has just read
+        for (int k = 0; k < P; k++) lds[S::at2(k)] = x[k];   // the places this thread has just read
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < 16; k++) x[k] = lds[S::at(k)];
+        for (int k = 0; k < P; k++) x[k] = lds[S::at_w(k)];
     }
     radix_inv<S::T1, true>(f, x, (const typename F::W *)tw_int, 1u);
     const __amdgpu_buffer_rsrc_t to = limb_rsrc(limb);
 #pragma unroll
-    for (int k = 0; k < 16; k++) buf_store<u64>(to, S::voff(), S::off(k), f.scale_to_canonical(x[k]));
+    for (int k = 0; k < P; k++) buf_store<u64>(to, S::voff(), S::off(k), f.scale_to_canonical(x[k]));
 }
 
-template <int LR, int LOAD>
-__global__ __launch_bounds__(16 << LR) void ntt_limb_inverse_kernel(
+template <int LR, int P, int LOAD>
+__global__ __launch_bounds__((256 / P) << LR) void ntt_limb_inverse_kernel(
     u64 *__restrict__ data, const Tw *__restrict__ tw_all, const Tw *__restrict__ rtw_all, const ModQ *__restrict__ modq,
     const u64 *__restrict__ ninv, const u64 *__restrict__ ninv_s, const double *__restrict__ fp, LimbList ll, LimbList sl,
     int n_limbs, size_t poly_stride, const Tw *__restrict__ final_scale, NttEpilogue from) {
@@ -208,17 +217,19 @@ __global__ __launch_bounds__(16 << LR) void ntt_limb_inverse_kernel(
             f.ni = (double)final_scale[limb].w;
             f.niinv = f.ni * f.qinv;
         }
-        limb_inverse<LR, LOAD>(base, tw, rtw, f, lds, ld, from.galois, sec);
+        limb_inverse<LR, P, LOAD>(base, tw, rtw, f, lds, ld, from.galois, sec);
     } else {
         IntField f(modq, ninv, ninv_s, fp, prime);
         if (final_scale != nullptr) {
             f.ni = final_scale[limb].w;
             f.nis = final_scale[limb].ws;
         }
-        limb_inverse<LR, LOAD>(base, tw, rtw, f, lds, ld, from.galois, sec);
+        limb_inverse<LR, P, LOAD>(base, tw, rtw, f, lds, ld, from.galois, sec);
     }
 }
 
+// points per thread
+#define POINTS(LR) ((LR) <= 5 ? 8 : 16)
 }  // namespace
 
 void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
@@ -234,9 +245,9 @@ void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, c
         for (int l = 0; l < n_limbs; l++) widest = std::max(widest, cs->d[cs->digit_of[l]].n_src);
     }
     if (ls != nullptr) lift = *ls;
-    const dim3 grid((unsigned)((n_limbs + conv.n_copy) * n_polys)), block(16u << LR);
+    const dim3 grid((unsigned)((n_limbs + conv.n_copy) * n_polys)), block((unsigned)((256 / POINTS(LR)) << LR));
 #define LIMB_FORWARD(L, K, TAIL)                                                                                           \
-    hipLaunchKernelGGL((ntt_limb_forward_kernel<L, K, TAIL>), grid, block, 0, s, data, (const Tw *)c->d_w,                 \
+    hipLaunchKernelGGL((ntt_limb_forward_kernel<L, POINTS(L), K, TAIL>), grid, block, 0, s, data, (const Tw *)c->d_w,                 \
                        (const Tw *)c->d_rw, c->d_modq, c->d_fp, ll, sl, n_limbs, poly_stride, conv, lift, ep)
 #define LIMB_SOURCES(L, TAIL)                          \
     do {                                               \
@@ -268,9 +279,9 @@ void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, c
 void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
                          size_t poly_stride, hipStream_t s, const void *final_scale, const NttEpilogue &from, int load) {
     const int LR = c->logN - 8;
-    const dim3 grid((unsigned)(n_limbs * n_polys)), block(16u << LR);
+    const dim3 grid((unsigned)(n_limbs * n_polys)), block((unsigned)((256 / POINTS(LR)) << LR));
 #define LIMB_INVERSE(L, LOAD)                                                                                         \
-    hipLaunchKernelGGL((ntt_limb_inverse_kernel<L, LOAD>), grid, block, 0, s, data, (const Tw *)c->d_iw,              \
+    hipLaunchKernelGGL((ntt_limb_inverse_kernel<L, POINTS(L), LOAD>), grid, block, 0, s, data, (const Tw *)c->d_iw,              \
                        (const Tw *)c->d_irw, c->d_modq, c->d_ninv, c->d_ninv_s, c->d_fp, ll, sl, n_limbs, poly_stride, \
                        (const Tw *)final_scale, from)
 #define LIMB_RING(L)                                                   \

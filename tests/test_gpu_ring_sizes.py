@@ -92,3 +92,25 @@ def test_moddown_of_batches(log_n, polys, drop):
         want = np.empty((nq - drop, N), dtype=np.uint64)
         orc.L.orc_moddown_drop(orc.h, _p(y[p].copy()), nq, drop, _p(want))
         assert np.array_equal(got[p], want), p
+
+
+# limbs on both sides of where a pass gives a thread eight points instead of sixteen (2^16 points: 32 limbs for columns, 40 for
+# rows; 2^13: 256 and 320, out of a launch that would be one), primes of all three arithmetic forms, extreme residues
+@pytest.mark.parametrize("log_n,polys,limbs", [(16, 1, 1), (16, 2, 16), (16, 3, 11), (16, 4, 10), (16, 1, 41), (15, 3, 27), (14, 5, 19)])
+@pytest.mark.parametrize("bits", [42, 60, 61])
+def test_points_per_thread(log_n, polys, limbs, bits):
+    import torch
+    pkg = load_package()
+    primes = O.primes_below(bits, log_n, limbs)
+    ctx, orc, N = pkg.Context(log_n, primes, [], 1), O.Oracle(log_n, primes, [], 1), 1 << log_n
+    rng = np.random.default_rng(log_n * 1000 + polys * limbs + bits)
+    a = top_and_random(rng, primes, (polys,), N)
+    d = dev(a)
+    ctx.ntt(d, list(range(limbs)))
+    got = host(d)
+    for p in {0, polys - 1}:   # the oracle takes its time: the first and the last polynomial, the others by the way back
+        want = a[p].copy()
+        orc.ntt(want, list(range(limbs)))
+        assert np.array_equal(got[p], want)
+    ctx.ntt(d, list(range(limbs)), inverse=True)
+    assert torch.equal(d, dev(a))
