@@ -33,22 +33,28 @@ struct RotTermDev {
 // Accesses to data that is touched once per launch (keys, masks, results): marked non-temporal so they do
 // not push the rotation sources, which every output gathers from, out of the L2.
 typedef u64 u64x2 __attribute__((ext_vector_type(2)));
+// Pointers that a kernel reads from a term record in memory are of no known address space, and loads through them would be
+// flat ones, for which every wait is a wait for all loads in flight: the address space is said here.
+typedef const u64x2 __attribute__((address_space(1))) *global_u64x2;
 __device__ __forceinline__ ulonglong2 stream_load2(const u64 *p) {
-    const u64x2 v = __builtin_nontemporal_load((const u64x2 *)p);
+    const u64x2 v = __builtin_nontemporal_load((global_u64x2)p);
     return make_ulonglong2(v.x, v.y);
 }
-__device__ __forceinline__ u64 stream_load1(const u64 *p) { return __builtin_nontemporal_load(p); }
+__device__ __forceinline__ ulonglong2 load2(const u64 *p) {
+    const u64x2 v = *(global_u64x2)p;
+    return make_ulonglong2(v.x, v.y);
+}
 // mask residues of the pair (n, n+1) of limb j: streamed from a full mask, or one value of a run table (every
 // lane of the workgroup reads the same one or two entries, which stay in cache).  A run table holds pairs
 // (value, floor(value * 2^64 / q)): the second word lets integer limbs multiply by the value as by a constant.
 __device__ __forceinline__ ulonglong2 load_mask2(const u64 *mask, const u32 shift, const int j, const u32 n, const int logN) {
     if (shift == 0) return stream_load2(mask + ((size_t)j << logN) + n);
-    const u64 v = mask[(((size_t)j << (logN - shift)) + (n >> shift)) * 2];
+    const u64 v = *(const u64 __attribute__((address_space(1))) *)(mask + (((size_t)j << (logN - shift)) + (n >> shift)) * 2);
     return make_ulonglong2(v, v);
 }
 // (value, Shoup companion) of the run that holds the pair (n, n+1)
 __device__ __forceinline__ ulonglong2 load_mask_run(const u64 *mask, const u32 shift, const int j, const u32 n, const int logN) {
-    return *(const ulonglong2 *)(mask + (((size_t)j << (logN - shift)) + (n >> shift)) * 2);
+    return load2(mask + (((size_t)j << (logN - shift)) + (n >> shift)) * 2);
 }
 // x1 * w1 + x2 * w2 mod q for run-table constants, canonical
 __device__ __forceinline__ u64 shoup_pair(u64 x1, const ulonglong2 w1, u64 x2, const ulonglong2 w2, u64 q) {
@@ -59,7 +65,7 @@ __device__ __forceinline__ u64 shoup_pair(u64 x1, const ulonglong2 w1, u64 x2, c
 // pair, possibly swapped)
 __device__ __forceinline__ ulonglong2 load_rotated2(const u64 *pt, const u32 g, const int j, const u32 n, const int logN) {
     const u32 np = g == 1u ? n : galois_index(n, g, logN);
-    ulonglong2 v = *(const ulonglong2 *)(pt + ((size_t)j << logN) + (np & ~1u));
+    ulonglong2 v = load2(pt + ((size_t)j << logN) + (np & ~1u));
     if (np & 1u) {
         const u64 t = v.x;
         v.x = v.y;
@@ -168,8 +174,8 @@ __device__ __forceinline__ void two_source_int(const RotTermDev &T, const u32 *_
     }
     u128_t pb[2] = {{0, 0}, {0, 0}}, pa[2] = {{0, 0}, {0, 0}};
     for (int d = 0; d < beta; d++) {
-        ulonglong2 x1 = *(const ulonglong2 *)(T.ext + ((size_t)d * E + j) * N + base);
-        ulonglong2 x2 = *(const ulonglong2 *)(T.ext2 + ((size_t)d * E + j) * N + base);
+        ulonglong2 x1 = load2(T.ext + ((size_t)d * E + j) * N + base);
+        ulonglong2 x2 = load2(T.ext2 + ((size_t)d * E + j) * N + base);
         if (swap) {
             u64 tmp = x1.x;
             x1.x = x1.y;
@@ -208,8 +214,8 @@ __device__ __forceinline__ void two_source_int(const RotTermDev &T, const u32 *_
         ra[1] = barrett128_u(pa[1], m);
     }
     if (j < nq) {
-        ulonglong2 b1 = *(const ulonglong2 *)(T.b + (size_t)j * N + base);
-        ulonglong2 b2 = *(const ulonglong2 *)(T.b2 + (size_t)j * N + base);
+        ulonglong2 b1 = load2(T.b + (size_t)j * N + base);
+        ulonglong2 b2 = load2(T.b2 + (size_t)j * N + base);
         if (swap) {
             u64 tmp = b1.x;
             b1.x = b1.y;
@@ -286,7 +292,7 @@ __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ 
         const bool keyless = T.evk == nullptr;
         const bool ext_as_is = !COMPACT && (T.flags & ROT_TERM_EXT_ROTATED) != 0;
         for (int d = 0; d < (keyless ? 0 : beta); d++) {
-            ulonglong2 x = *(const ulonglong2 *)(T.ext + ((size_t)d * E + j) * N + (ext_as_is ? n : base));
+            ulonglong2 x = load2(T.ext + ((size_t)d * E + j) * N + (ext_as_is ? n : base));
             if (swap && !ext_as_is) {
                 const u64 tmp = x.x;
                 x.x = x.y;
@@ -312,7 +318,7 @@ __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ 
             ra[1] = barrett128_u(sa[1], m);
         }
         if (j < nq && T.b != nullptr) {
-            ulonglong2 bv = *(const ulonglong2 *)(T.b + (size_t)j * N + base);
+            ulonglong2 bv = load2(T.b + (size_t)j * N + base);
             if (swap) {
                 const u64 tmp = bv.x;
                 bv.x = bv.y;
@@ -326,7 +332,7 @@ __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ 
             rb[1] = addmod_u(rb[1], bv.y, m.q);
         }
         if (keyless) {   // the a-polynomial enters as it is (times P): no key product above (j < nq here)
-            ulonglong2 av = *(const ulonglong2 *)(T.ext + (size_t)j * N + base);
+            ulonglong2 av = load2(T.ext + (size_t)j * N + base);
             if (swap) {
                 const u64 tmp = av.x;
                 av.x = av.y;
@@ -391,7 +397,7 @@ __device__ __forceinline__ D2 to_d2(const ulonglong2 v) {
     return r;
 }
 __device__ __forceinline__ D2 gather_d2(const u64 *p, const bool swap) {
-    ulonglong2 v = *(const ulonglong2 *)p;
+    ulonglong2 v = load2(p);
     if (swap) {
         const u64 tmp = v.x;
         v.x = v.y;

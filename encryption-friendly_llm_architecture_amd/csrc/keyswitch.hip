@@ -349,7 +349,11 @@ struct LinTermDev {
 // out[o][p][j] = sum_{t in group o} mask_t[j] * ct_t[p][j], p < n_polys (<= 3).  A thread owns the residue pair
 // (n, n+1) of one limb for every polynomial (16-byte accesses; under an automorphism an aligned pair stays an
 // aligned pair, possibly swapped), so each mask residue is read once; integer products are summed as 128-bit
-// values and reduced every 4 terms.
+// values and reduced every 4 terms.  What bounds it is the trip to memory of each term: its loads are the only ones a
+// wavefront has in flight, so nothing may wait between them.  64 terms of 6 limbs over 768 workgroups 199 us with flat loads and a
+// branch on a missing mask between the mask's load and the ciphertext's, 146 us without; 24576 workgroups 445 -> 417 us.
+// Four or eight terms in flight per wavefront: 156 and 151 us, and 472 us on the 24576 workgroups, which lose wavefronts to
+// the registers.
 template <int n_polys>
 __device__ __forceinline__ void masked_sum_body(const LinTermDev *__restrict__ terms, const u32 *__restrict__ group_off,
                                                 u64 *__restrict__ out, const ModQ *__restrict__ modq,
@@ -373,18 +377,34 @@ __device__ __forceinline__ void masked_sum_body(const LinTermDev *__restrict__ t
     const u32 n = ((tile & ((1u << (logN - 9)) - 1)) * 256 + threadIdx.x) * 2;
     const size_t e = (size_t)j * N + n;
     const double fq = fp[4 * j];
-    // mask residues of the pair (n, n+1), read through the term's automorphism if it has one
-    auto load_mask = [&](const LinTermDev &T) -> ulonglong2 {
-        if (T.galois == 0) return stream_load2(T.mask + e);
-        const u32 np = galois_index(n, (u32)T.galois, logN);
-        ulonglong2 v = *(const ulonglong2 *)(T.mask + (size_t)j * N + (np & ~1u));
-        if (np & 1u) {
-            const u64 tmp = v.x;
-            v.x = v.y;
-            v.y = tmp;
+    struct Loaded {
+        ulonglong2 mask, ct[n_polys];
+        bool has, swap;
+    };
+    // All loads of a term, nothing between them that waits for one: a mask read through an automorphism is put in order, and
+    // that of a term without one replaced by 1, only where it is used (such a term reads its ciphertext in the mask's place).
+    auto load = [&](const u32 t) {
+        const LinTermDev T = terms[t];
+        Loaded v;
+        v.has = T.mask != nullptr;
+        v.swap = false;
+        const u64 *mask = v.has ? T.mask : T.ct;
+        if (T.galois != 0) {   // kept in the caches: another term may read the same mask through another automorphism
+            const u32 np = v.has ? galois_index(n, (u32)T.galois, logN) : n;
+            v.swap = (np & 1u) != 0;
+            v.mask = load2(mask + (size_t)j * N + (np & ~1u));
+        } else {
+            v.mask = stream_load2(mask + e);
         }
+#pragma unroll
+        for (int p = 0; p < n_polys; p++) v.ct[p] = load2(T.ct + p * T.stride + e);
         return v;
     };
+    auto mask_of = [](const Loaded &v) {
+        const u64 x = v.swap ? v.mask.y : v.mask.x, y = v.swap ? v.mask.x : v.mask.y;
+        return make_ulonglong2(v.has ? x : 1ull, v.has ? y : 1ull);
+    };
+    const u32 end = group_off[o + 1];
     if (fq != 0.0) {
         // primes below 2^44: exact double-precision products (6 FP64 operations each)
         const FpMod f{fq, fp[4 * j + 1]};
@@ -392,26 +412,16 @@ __device__ __forceinline__ void masked_sum_body(const LinTermDev *__restrict__ t
 #pragma unroll
         for (int p = 0; p < n_polys; p++) facc[p][0] = facc[p][1] = 0.0;
         int since = 0;
-        for (u32 t = group_off[o]; t < group_off[o + 1]; t++) {
-            const LinTermDev T = terms[t];
-            if (T.mask != nullptr) {
-                const ulonglong2 mk = load_mask(T);
-                const double dm0 = u64_to_double(mk.x), dm1 = u64_to_double(mk.y);
+        for (u32 t = group_off[o]; t < end; t++) {
+            const Loaded v = load(t);
+            const ulonglong2 mk = mask_of(v);
+            const double dm0 = u64_to_double(mk.x), dm1 = u64_to_double(mk.y);
 #pragma unroll
-                for (int p = 0; p < n_polys; p++) {
-                    const ulonglong2 cv = *(const ulonglong2 *)(T.ct + p * T.stride + e);
-                    facc[p][0] += f.mul(u64_to_double(cv.x), dm0);
-                    facc[p][1] += f.mul(u64_to_double(cv.y), dm1);
-                }
-            } else {
-#pragma unroll
-                for (int p = 0; p < n_polys; p++) {
-                    const ulonglong2 cv = *(const ulonglong2 *)(T.ct + p * T.stride + e);
-                    facc[p][0] += u64_to_double(cv.x);
-                    facc[p][1] += u64_to_double(cv.y);
-                }
+            for (int p = 0; p < n_polys; p++) {
+                facc[p][0] += f.mul(u64_to_double(v.ct[p].x), dm0);
+                facc[p][1] += f.mul(u64_to_double(v.ct[p].y), dm1);
             }
-            if (++since == 64) {  // a term adds at most q: keep the running sums far below 2^52
+            if (++since == 64) {  // a term adds at most 0.54 q: keep the running sums far below 2^52
 #pragma unroll
                 for (int p = 0; p < n_polys; p++) {
                     facc[p][0] = f.reduce(facc[p][0]);
@@ -434,32 +444,22 @@ __device__ __forceinline__ void masked_sum_body(const LinTermDev *__restrict__ t
             lazy[p][h].lo = lazy[p][h].hi = 0;
         }
     int pending = 0;
-    for (u32 t = group_off[o]; t < group_off[o + 1]; t++) {
-        const LinTermDev T = terms[t];
-        if (T.mask != nullptr) {
-            const ulonglong2 mk = load_mask(T);
+    for (u32 t = group_off[o]; t < end; t++) {
+        const Loaded v = load(t);
+        const ulonglong2 mk = mask_of(v);
 #pragma unroll
-            for (int p = 0; p < n_polys; p++) {
-                const ulonglong2 cv = *(const ulonglong2 *)(T.ct + p * T.stride + e);
-                add128(lazy[p][0], mul64wide(cv.x, mk.x));
-                add128(lazy[p][1], mul64wide(cv.y, mk.y));
-            }
-            if (++pending == 4) {
+        for (int p = 0; p < n_polys; p++) {
+            add128(lazy[p][0], mul64wide(v.ct[p].x, mk.x));
+            add128(lazy[p][1], mul64wide(v.ct[p].y, mk.y));
+        }
+        if (++pending == 4) {
 #pragma unroll
-                for (int p = 0; p < n_polys; p++)
-                    for (int h = 0; h < 2; h++) {
-                        acc[p][h] = addmod(acc[p][h], barrett128(lazy[p][h], m), m.q);
-                        lazy[p][h].lo = lazy[p][h].hi = 0;
-                    }
-                pending = 0;
-            }
-        } else {
-#pragma unroll
-            for (int p = 0; p < n_polys; p++) {
-                const ulonglong2 cv = *(const ulonglong2 *)(T.ct + p * T.stride + e);
-                acc[p][0] = addmod(acc[p][0], cv.x, m.q);
-                acc[p][1] = addmod(acc[p][1], cv.y, m.q);
-            }
+            for (int p = 0; p < n_polys; p++)
+                for (int h = 0; h < 2; h++) {
+                    acc[p][h] = addmod(acc[p][h], barrett128(lazy[p][h], m), m.q);
+                    lazy[p][h].lo = lazy[p][h].hi = 0;
+                }
+            pending = 0;
         }
     }
 #pragma unroll

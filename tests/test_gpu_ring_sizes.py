@@ -114,3 +114,28 @@ def test_points_per_thread(log_n, polys, limbs, bits):
         assert np.array_equal(got[p], want)
     ctx.ntt(d, list(range(limbs)), inverse=True)
     assert torch.equal(d, dev(a))
+
+
+# term counts around the four products between reductions and the 64 terms of the double-precision sums, in the lists that
+# travel in the kernel arguments (up to 32 terms) and in those that do not; unmasked terms, masks through an automorphism
+@pytest.mark.parametrize("n_terms", [1, 3, 4, 5, 32, 33, 64, 65, 129])
+def test_masked_sum_lengths(n_terms):
+    pkg = load_package()
+    log_n, g = 10, 25
+    mods = [O.primes_below(60, log_n, 1)[0], O.primes_below(44, log_n, 1)[0]]
+    ctx, orc, N = pkg.Context(log_n, mods, [], 1), O.Oracle(log_n, mods, [], 1), 1 << log_n
+    rng = np.random.default_rng(n_terms)
+    cts, masks = top_and_random(rng, mods, (3, 2), N), top_and_random(rng, mods, (2,), N)
+    masks[0, :, : N // 2] = np.array(mods, dtype=np.uint64)[:, None] - np.uint64(1)
+    turned = np.empty_like(masks)
+    for i in range(2):
+        for j in range(2):
+            orc.L.orc_automorphism_ntt(orc.h, _p(masks[i, j]), _p(turned[i, j]), g)
+    dct, dmask = [dev(c) for c in cts], [dev(m) for m in masks]
+    spec = [(t % 3, None if t % 7 == 3 else t % 2, g if t % 5 == 4 else 0) for t in range(n_terms)]
+    got = host(ctx.masked_sum_batch([[(dct[c], None if m is None else dmask[m], gal if m is not None else 0) for c, m, gal in spec]], 2, 2))
+    want = np.zeros((2, 2, N), dtype=object)
+    for c, m, gal in spec:
+        want += cts[c].astype(object) * (1 if m is None else (turned if gal else masks)[m].astype(object))
+    want %= np.array(mods, dtype=object)[:, None]
+    assert np.array_equal(got[0], want.astype(np.uint64))
