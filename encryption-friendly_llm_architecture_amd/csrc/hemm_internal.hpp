@@ -233,7 +233,7 @@ void launch_hoisted_terms_args(hemm_context *c, const void *terms_host, int n_te
 void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop_last, u64 *out, size_t out_stride,
                           u64 *conv, hipStream_t s, bool slab = false);
 void launch_masked_sum(hemm_context *c, const void *terms_dev, const u32 *group_off_dev, int n_out, int nq, int n_polys,
-                       u64 *out, hipStream_t s, const void *terms_host = nullptr, int n_terms = 0);
+                       u64 *out, hipStream_t s, const void *terms_host, int n_terms);
 // y[o][p][j] = sum_{q < parts} part[o * parts + q][p][j] over the extended basis, y / part: [.][2][nq+K][N]
 void launch_sum_parts(hemm_context *c, const u64 *part, int parts, int n_out, int nq, u64 *y, hipStream_t s);
 size_t key_compact_words(const hemm_context *c);

@@ -354,7 +354,10 @@ struct LinTermDev {
 // branch on a missing mask between the mask's load and the ciphertext's, 146 us without; 24576 workgroups 445 -> 417 us.
 // Four or eight terms in flight per wavefront: 156 and 151 us, and 472 us on the 24576 workgroups, which lose wavefronts to
 // the registers.
-template <int n_polys>
+// ALL_MASKED: no term of the launch is without a mask.  The branch on it keeps the next term's loads behind this one's products
+// (128 masks of their own, 6 limbs of 60 bits: 213 - 220 us with it, 206 without), so only lists that hold such a term pay for it;
+// there the term is an addition (128 of them 138 us; as a product by one, its first polynomial read again in the mask's place, 167).
+template <int n_polys, bool ALL_MASKED>
 __device__ __forceinline__ void masked_sum_body(const LinTermDev *__restrict__ terms, const u32 *__restrict__ group_off,
                                                 u64 *__restrict__ out, const ModQ *__restrict__ modq,
                                                 const double *__restrict__ fp, int nq, int logN, int n_out) {
@@ -377,32 +380,35 @@ __device__ __forceinline__ void masked_sum_body(const LinTermDev *__restrict__ t
     const u32 n = ((tile & ((1u << (logN - 9)) - 1)) * 256 + threadIdx.x) * 2;
     const size_t e = (size_t)j * N + n;
     const double fq = fp[4 * j];
-    struct Loaded {
-        ulonglong2 mask, ct[n_polys];
-        bool has, swap;
-    };
-    // All loads of a term, nothing between them that waits for one: a mask read through an automorphism is put in order, and
-    // that of a term without one replaced by 1, only where it is used (such a term reads its ciphertext in the mask's place).
-    auto load = [&](const u32 t) {
-        const LinTermDev T = terms[t];
-        Loaded v;
-        v.has = T.mask != nullptr;
-        v.swap = false;
-        const u64 *mask = v.has ? T.mask : T.ct;
-        if (T.galois != 0) {   // kept in the caches: another term may read the same mask through another automorphism
-            const u32 np = v.has ? galois_index(n, (u32)T.galois, logN) : n;
-            v.swap = (np & 1u) != 0;
-            v.mask = load2(mask + (size_t)j * N + (np & ~1u));
-        } else {
-            v.mask = stream_load2(mask + e);
-        }
+    auto load_ct = [&](const LinTermDev &T, ulonglong2 (&ct)[n_polys]) {
 #pragma unroll
-        for (int p = 0; p < n_polys; p++) v.ct[p] = load2(T.ct + p * T.stride + e);
-        return v;
+        for (int p = 0; p < n_polys; p++) ct[p] = load2(T.ct + p * T.stride + e);
     };
-    auto mask_of = [](const Loaded &v) {
-        const u64 x = v.swap ? v.mask.y : v.mask.x, y = v.swap ? v.mask.x : v.mask.y;
-        return make_ulonglong2(v.has ? x : 1ull, v.has ? y : 1ull);
+    auto load_mask = [&](const LinTermDev &T, ulonglong2 &mask, bool &swap) {
+        if (T.galois != 0) {   // kept in the caches: another term may read the same mask through another automorphism
+            const u32 np = galois_index(n, (u32)T.galois, logN);
+            swap = (np & 1u) != 0;
+            mask = load2(T.mask + (size_t)j * N + (np & ~1u));
+            if (ALL_MASKED) asm volatile("");   // or the two loads become one that is not non-temporal
+        } else {
+            mask = stream_load2(T.mask + e);
+        }
+    };
+    // The loads of a term, nothing between them that waits for one: a mask read through an automorphism is put in order behind
+    // them all.  false: a term without a mask.
+    auto load = [&](const u32 t, ulonglong2 (&ct)[n_polys], ulonglong2 &mask) {
+        const LinTermDev T = terms[t];
+        bool swap = false;
+        if (ALL_MASKED) {
+            load_mask(T, mask, swap);
+            load_ct(T, ct);
+        } else {
+            load_ct(T, ct);
+            if (T.mask == nullptr) return false;
+            load_mask(T, mask, swap);
+        }
+        if (swap) mask = make_ulonglong2(mask.y, mask.x);
+        return true;
     };
     const u32 end = group_off[o + 1];
     if (fq != 0.0) {
@@ -413,15 +419,22 @@ __device__ __forceinline__ void masked_sum_body(const LinTermDev *__restrict__ t
         for (int p = 0; p < n_polys; p++) facc[p][0] = facc[p][1] = 0.0;
         int since = 0;
         for (u32 t = group_off[o]; t < end; t++) {
-            const Loaded v = load(t);
-            const ulonglong2 mk = mask_of(v);
-            const double dm0 = u64_to_double(mk.x), dm1 = u64_to_double(mk.y);
+            ulonglong2 ct[n_polys], mk;
+            if (load(t, ct, mk)) {
+                const double dm0 = u64_to_double(mk.x), dm1 = u64_to_double(mk.y);
 #pragma unroll
-            for (int p = 0; p < n_polys; p++) {
-                facc[p][0] += f.mul(u64_to_double(v.ct[p].x), dm0);
-                facc[p][1] += f.mul(u64_to_double(v.ct[p].y), dm1);
+                for (int p = 0; p < n_polys; p++) {
+                    facc[p][0] += f.mul(u64_to_double(ct[p].x), dm0);
+                    facc[p][1] += f.mul(u64_to_double(ct[p].y), dm1);
+                }
+            } else {
+#pragma unroll
+                for (int p = 0; p < n_polys; p++) {
+                    facc[p][0] += u64_to_double(ct[p].x);
+                    facc[p][1] += u64_to_double(ct[p].y);
+                }
             }
-            if (++since == 64) {  // a term adds at most 0.54 q: keep the running sums far below 2^52
+            if (++since == 64) {  // a term adds at most q: keep the running sums far below 2^52
 #pragma unroll
                 for (int p = 0; p < n_polys; p++) {
                     facc[p][0] = f.reduce(facc[p][0]);
@@ -445,12 +458,19 @@ __device__ __forceinline__ void masked_sum_body(const LinTermDev *__restrict__ t
         }
     int pending = 0;
     for (u32 t = group_off[o]; t < end; t++) {
-        const Loaded v = load(t);
-        const ulonglong2 mk = mask_of(v);
+        ulonglong2 ct[n_polys], mk;
+        if (!load(t, ct, mk)) {
+#pragma unroll
+            for (int p = 0; p < n_polys; p++) {
+                acc[p][0] = addmod(acc[p][0], ct[p].x, m.q);
+                acc[p][1] = addmod(acc[p][1], ct[p].y, m.q);
+            }
+            continue;
+        }
 #pragma unroll
         for (int p = 0; p < n_polys; p++) {
-            add128(lazy[p][0], mul64wide(v.ct[p].x, mk.x));
-            add128(lazy[p][1], mul64wide(v.ct[p].y, mk.y));
+            add128(lazy[p][0], mul64wide(ct[p].x, mk.x));
+            add128(lazy[p][1], mul64wide(ct[p].y, mk.y));
         }
         if (++pending == 4) {
 #pragma unroll
@@ -479,18 +499,18 @@ struct MaskedArgs {
     LinTermDev t[MASKED_ARG_TERMS];
     u32 off[MASKED_ARG_TERMS + 1];
 };
-template <int n_polys>
+template <int n_polys, bool ALL_MASKED>
 __global__ __launch_bounds__(256) void masked_sum_kernel(const MaskedArgs args, u64 *__restrict__ out,
                                                          const ModQ *__restrict__ modq, const double *__restrict__ fp,
                                                          int nq, int logN, int n_out) {
-    masked_sum_body<n_polys>(args.t, args.off, out, modq, fp, nq, logN, n_out);
+    masked_sum_body<n_polys, ALL_MASKED>(args.t, args.off, out, modq, fp, nq, logN, n_out);
 }
-template <int n_polys>
+template <int n_polys, bool ALL_MASKED>
 __global__ __launch_bounds__(256) void masked_sum_list_kernel(const LinTermDev *__restrict__ terms,
                                                               const u32 *__restrict__ group_off, u64 *__restrict__ out,
                                                               const ModQ *__restrict__ modq, const double *__restrict__ fp,
                                                               int nq, int logN, int n_out) {
-    masked_sum_body<n_polys>(terms, group_off, out, modq, fp, nq, logN, n_out);
+    masked_sum_body<n_polys, ALL_MASKED>(terms, group_off, out, modq, fp, nq, logN, n_out);
 }
 
 // acc3 (+)= sum_{g < G} (b1 b2, a1 b2 + a2 b1, a1 a2) of t1[g], t2[g], each [2][nq][N]
@@ -1470,22 +1490,29 @@ static size_t masked_bytes(const hemm_context *c, const LinTermDev *t, int n_ter
     return bytes;
 }
 
+static bool all_masked(const LinTermDev *t, int n_terms) {
+    for (int i = 0; i < n_terms; i++)
+        if (t[i].mask == nullptr) return false;
+    return true;
+}
+#define MASKED_SUM(KERNEL, ALL, ...)                                                                           \
+    do {                                                                                                       \
+        if (n_polys == 1) hipLaunchKernelGGL((KERNEL<1, ALL>), grid, block, 0, s, __VA_ARGS__, out, c->d_modq, c->d_fp, nq, c->logN, n_out); \
+        else if (n_polys == 2) hipLaunchKernelGGL((KERNEL<2, ALL>), grid, block, 0, s, __VA_ARGS__, out, c->d_modq, c->d_fp, nq, c->logN, n_out); \
+        else hipLaunchKernelGGL((KERNEL<3, ALL>), grid, block, 0, s, __VA_ARGS__, out, c->d_modq, c->d_fp, nq, c->logN, n_out); \
+    } while (0)
+// terms_dev: the list terms_host on the device
 void launch_masked_sum(hemm_context *c, const void *terms_dev, const u32 *group_off_dev, int n_out, int nq, int n_polys,
                        u64 *out, hipStream_t s, const void *terms_host, int n_terms) {
     if (n_polys > 3) throw std::invalid_argument("masked sums take at most 3 polynomials");
-    if (terms_host != nullptr) account(c, TR_MASKED, masked_bytes(c, (const LinTermDev *)terms_host, n_terms, n_out, nq, n_polys));
     if (c->N < 512) throw std::invalid_argument("masked sums need N >= 512");
+    account(c, TR_MASKED, masked_bytes(c, (const LinTermDev *)terms_host, n_terms, n_out, nq, n_polys));
     dim3 grid((unsigned)(c->N / 512) * nq * n_out), block(256);
     const LinTermDev *td = (const LinTermDev *)terms_dev;
-    if (n_polys == 1)
-        hipLaunchKernelGGL(masked_sum_list_kernel<1>, grid, block, 0, s, td, group_off_dev, out, c->d_modq, c->d_fp, nq,
-                           c->logN, n_out);
-    else if (n_polys == 2)
-        hipLaunchKernelGGL(masked_sum_list_kernel<2>, grid, block, 0, s, td, group_off_dev, out, c->d_modq, c->d_fp, nq,
-                           c->logN, n_out);
+    if (all_masked((const LinTermDev *)terms_host, n_terms))
+        MASKED_SUM(masked_sum_list_kernel, true, td, group_off_dev);
     else
-        hipLaunchKernelGGL(masked_sum_list_kernel<3>, grid, block, 0, s, td, group_off_dev, out, c->d_modq, c->d_fp, nq,
-                           c->logN, n_out);
+        MASKED_SUM(masked_sum_list_kernel, false, td, group_off_dev);
 }
 // table[run] = (value, floor(value * 2^64 / q)) of each run of a mask over the extended basis; *differs is set when
 // some run is not constant
@@ -1566,13 +1593,12 @@ void launch_masked_sum_args(hemm_context *c, const void *terms_host, int n_terms
     memcpy(a.t, terms_host, (size_t)n_terms * sizeof(LinTermDev));
     memcpy(a.off, group_off_host, (size_t)(n_out + 1) * sizeof(u32));
     dim3 grid((unsigned)(c->N / 512) * nq * n_out), block(256);
-    if (n_polys == 1)
-        hipLaunchKernelGGL(masked_sum_kernel<1>, grid, block, 0, s, a, out, c->d_modq, c->d_fp, nq, c->logN, n_out);
-    else if (n_polys == 2)
-        hipLaunchKernelGGL(masked_sum_kernel<2>, grid, block, 0, s, a, out, c->d_modq, c->d_fp, nq, c->logN, n_out);
+    if (all_masked(a.t, n_terms))
+        MASKED_SUM(masked_sum_kernel, true, a);
     else
-        hipLaunchKernelGGL(masked_sum_kernel<3>, grid, block, 0, s, a, out, c->d_modq, c->d_fp, nq, c->logN, n_out);
+        MASKED_SUM(masked_sum_kernel, false, a);
 }
+#undef MASKED_SUM
 
 int tensor_max_groups() { return TENSOR_MAX_GROUPS; }
 void launch_tensor_groups(hemm_context *c, const TensorGroupHost *g, int n_groups, int nq, size_t acc_stride,
