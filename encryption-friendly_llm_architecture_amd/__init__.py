@@ -75,6 +75,7 @@ def _declare(L):
     L.hemm_rotate.argtypes = [vp, vp, sz, vp, u64, u32, vp, sz, vp]
     L.hemm_relinearize.argtypes = [vp, vp, sz, vp, u32, vp, sz, vp]
     L.hemm_rescale.argtypes = [vp, vp, sz, vp, sz, u32, u32, vp]
+    L.hemm_rescale_to.argtypes = [vp, vp, sz, ctypes.POINTER(vp), sz, u32, u32, vp]
     L.hemm_rescale_static.argtypes = [vp, vp, sz, vp, sz, u32, u32, vp]
     L.hemm_sample_uniform.argtypes = [vp, u64p, u32p, u32, vp, vp]
     L.hemm_sample_error.argtypes = [vp, u64, u32p, u32, vp, vp]
@@ -82,6 +83,7 @@ def _declare(L):
     L.hemm_hoisted_terms.argtypes = [vp, ctypes.POINTER(RotTerm), u32p, u32, u32, vp, ci, vp]
     L.hemm_moddown_batch.argtypes = [vp, vp, u32, u32, ci, vp, sz, vp, vp]
     L.hemm_hoisted_moddown.argtypes = [vp, ctypes.POINTER(RotTerm), u32p, u32, u32, ci, ci, vp, vp, sz, vp, vp]
+    L.hemm_hoisted_moddown_to.argtypes = [vp, ctypes.POINTER(RotTerm), u32p, u32, u32, ci, ci, vp, ctypes.POINTER(vp), sz, vp, vp]
     L.hemm_masked_sum_batch.argtypes = [vp, ctypes.POINTER(LinTerm), u32p, u32, u32, u32, vp, vp]
     L.hemm_tensor_batch.argtypes = [vp, vp, vp, u32, u32, vp, ci, vp]
     L.hemm_tensor_batch_groups.argtypes = [vp, ctypes.POINTER(TensorGroup), u32, u32, sz, vp]

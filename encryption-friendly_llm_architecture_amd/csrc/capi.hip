@@ -1,4 +1,5 @@
 // extern "C" boundary (declared in include/hemm.h).
+#include <algorithm>
 #include <cstring>
 #include <vector>
 
@@ -40,6 +41,11 @@ static void need(bool ok, const char *msg) {
     if (!ok) throw std::invalid_argument(msg);
 }
 static void check_launch() { HEMM_HIP(hipGetLastError()); }
+static ResultList results_in(uint64_t *const *outs, uint32_t n) {
+    ResultList list{};
+    for (uint32_t i = 0; i < n; i++) list.at[i] = (u64 *)outs[i];
+    return list;
+}
 
 extern "C" {
 
@@ -583,6 +589,27 @@ int hemm_hoisted_moddown(hemm_context *ctx, const hemm_rot_term *terms, const ui
     HEMM_CATCH
 }
 
+int hemm_hoisted_moddown_to(hemm_context *ctx, const hemm_rot_term *terms, const uint32_t *group_offsets, uint32_t n_out,
+                            uint32_t nq, int b_premultiplied, int drop_last, uint64_t *y_workspace, uint64_t *const *outs,
+                            size_t out_stride, uint64_t *workspace, void *stream) {
+    HEMM_TRY
+    int nl;
+    chain_limbs(ctx, nq, 1, &nl);
+    need(terms && group_offsets && y_workspace && outs && workspace && n_out >= 1, "null operand");
+    need(ctx->nP >= 1, "key switching needs special primes");
+    for (uint32_t o = 0; o < n_out; o++) need(outs[o] != nullptr, "null output");
+    run_hoisted_terms(ctx, terms, group_offsets, n_out, nq, (u64 *)y_workspace, b_premultiplied != 0, on_stream(ctx, stream));
+    const size_t y_words = 2 * (size_t)(nq + ctx->nP) * ctx->N, ws_words = 2 * (size_t)(drop_last ? nq - 1 : nq) * ctx->N;
+    for (uint32_t o = 0; o < n_out; o += RESULT_PARTS) {
+        const uint32_t n = std::min<uint32_t>(n_out - o, RESULT_PARTS);
+        const ResultList list = results_in(outs + o, n);
+        launch_moddown_batch(ctx, (u64 *)y_workspace + o * y_words, (int)nq, (int)(2 * n), drop_last != 0, nullptr, out_stride,
+                             (u64 *)workspace + o * ws_words, on_stream(ctx, stream), false, &list);
+    }
+    check_launch();
+    HEMM_CATCH
+}
+
 int hemm_moddown_batch(hemm_context *ctx, uint64_t *y, uint32_t nq, uint32_t n_polys, int drop_last, uint64_t *out,
                        size_t out_stride, uint64_t *workspace, void *stream) {
     HEMM_TRY
@@ -749,6 +776,33 @@ int hemm_rescale(hemm_context *ctx, const uint64_t *in, size_t in_stride, uint64
     check_rescale_layout(ctx, in, in_stride, out, out_stride, nq, n_polys);
     launch_rescale(ctx, (const u64 *)in, in_stride, (u64 *)out, out_stride, (int)nq, (int)n_polys,
                    on_stream(ctx, stream));
+    check_launch();
+    HEMM_CATCH
+}
+
+int hemm_rescale_to(hemm_context *ctx, const uint64_t *in, size_t in_stride, uint64_t *const *outs, size_t out_stride, uint32_t nq,
+                    uint32_t n_out, void *stream) {
+    HEMM_TRY
+    int nl;
+    chain_limbs(ctx, nq, 0, &nl);
+    need(in && outs, "null operand");
+    need(nq >= 2, "rescale needs at least two limbs");
+    const size_t in_words = (size_t)nq * ctx->N, out_words = (size_t)(nq - 1) * ctx->N;
+    need(n_out >= 1 && 2 * (size_t)n_out * in_words <= hemm_scratch_words(ctx),
+         "2 * n_out * nq limbs must fit the context's scratch ((dnum + 7) * (nQ + nP) limbs)");
+    need(in_stride >= in_words, "in_stride is shorter than a polynomial of nq limbs");
+    need(out_stride >= out_words, "out_stride is shorter than a polynomial of nq - 1 limbs");
+    const uint64_t *in_end = in + (size_t)(2 * n_out - 1) * in_stride + in_words;
+    for (uint32_t o = 0; o < n_out; o++) {
+        need(outs[o] != nullptr, "null output");
+        need(outs[o] >= in_end || outs[o] + out_stride + out_words <= in, "an output overlaps in");
+    }
+    for (uint32_t o = 0; o < n_out; o += RESULT_PARTS) {
+        const uint32_t n = std::min<uint32_t>(n_out - o, RESULT_PARTS);
+        const ResultList list = results_in(outs + o, n);
+        launch_rescale(ctx, (const u64 *)in + (size_t)2 * o * in_stride, in_stride, nullptr, out_stride, (int)nq, (int)(2 * n),
+                       on_stream(ctx, stream), &list);
+    }
     check_launch();
     HEMM_CATCH
 }

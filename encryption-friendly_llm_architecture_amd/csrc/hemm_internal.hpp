@@ -90,6 +90,13 @@ __device__ __forceinline__ u32 galois_index(u32 k, u32 g, int logN) {
 
 void hemm_set_error(const std::string &msg);
 
+// Where a chain over several ciphertexts leaves its results when they do not lie back to back: polynomials 2 i and 2 i + 1 in
+// at[i] (a chain's output stride apart).  Travels in the kernel arguments.
+#define RESULT_PARTS 32
+struct ResultList {
+    u64 *at[RESULT_PARTS];
+};
+
 #define HEMM_HIP(call)                                                                       \
     do {                                                                                     \
         hipError_t e_ = (call);                                                              \
@@ -110,7 +117,8 @@ LimbList limbs_default(const hemm_context *c, int nq, int with_p);
 void launch_ntt_slots(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs,
                       int n_polys, size_t poly_stride, bool inverse, hipStream_t s, const void *final_scale = nullptr);
 bool launch_ntt_sub_scale(const hemm_context *c, u64 *data, int n_limbs, int n_polys, const u64 *minuend,
-                          size_t minuend_stride, u64 *out, size_t out_stride, const void *cst_dev, hipStream_t s);
+                          size_t minuend_stride, u64 *out, size_t out_stride, const void *cst_dev, hipStream_t s,
+                          const ResultList *list = nullptr);
 // A forward transform of N >= 2^10 whose input is a fast basis conversion: limb l of the launch is the conversion of
 // the coefficient-form sources of digit digit_of[l] (already carrying their (S/q_i)^-1 factors) to prime ll[l],
 // computed while the first pass loads its slab instead of being written by a conversion launch and read back.
@@ -135,12 +143,13 @@ struct ConvSources {
     uint8_t copy_src_slot[HEMM_MAX_PRIMES], copy_dst_slot[HEMM_MAX_PRIMES];
 };
 // data: [n_polys][.][N] (polynomial stride poly_stride), limb l written to slot sl[l].  With ep_* set the second pass
-// ends with out = (minuend - transform) * cst[l] (slots of minuend / out = l) and data is only a workspace.
+// ends with out = (minuend - transform) * cst[l] (slots of minuend / out = l) and data is only a workspace; ep_list: the
+// polynomials of `out` lie where the list says.
 // false when the ring size or the source counts have no such form (nothing was launched).
 bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *data, const LimbList &ll, const LimbList &sl,
                           int n_limbs, int n_polys, size_t poly_stride, hipStream_t s, const u64 *ep_minuend = nullptr,
                           size_t ep_minuend_stride = 0, u64 *ep_out = nullptr, size_t ep_out_stride = 0,
-                          const void *ep_cst_dev = nullptr);
+                          const void *ep_cst_dev = nullptr, const ResultList *ep_list = nullptr);
 // A forward transform of N >= 2^10 whose input is the rounded coefficients of an encoding (signed, [n_polys][stride >= N], the
 // same for every limb; plus, with_error, the error of a stream), reduced while the first pass loads them.  enc: the second
 // pass ends in an encryption instead of storing the transform (data is then only a workspace): a uniform from the streams
@@ -217,7 +226,7 @@ void launch_keyswitch(hemm_context *c, const u64 *in, const u64 *evk, int nq, u6
                       const u64 *add_b, hipStream_t s, u32 galois = 0, bool b_rotates = false,
                       const u64 *add_a = nullptr);
 void launch_rescale(hemm_context *c, const u64 *in, size_t in_stride, u64 *out, size_t out_stride, int nq,
-                    int n_polys, hipStream_t s);
+                    int n_polys, hipStream_t s, const ResultList *list = nullptr);
 void launch_modup_batch(hemm_context *c, const u64 *in, size_t in_stride, int nq, int n_in, u64 *ext, u64 *coef,
                         hipStream_t s, u32 galois = 0);
 // whether launch_modup_batch at this level takes a non-zero `galois` (its input read through that automorphism)
@@ -231,7 +240,7 @@ int hoisted_arg_capacity();
 void launch_hoisted_terms_args(hemm_context *c, const void *terms_host, int n_terms, const u32 *group_off_host, int n_out,
                                int nq, u64 *y, bool b_premultiplied, hipStream_t s);
 void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop_last, u64 *out, size_t out_stride,
-                          u64 *conv, hipStream_t s, bool slab = false);
+                          u64 *conv, hipStream_t s, bool slab = false, const ResultList *list = nullptr);
 void launch_masked_sum(hemm_context *c, const void *terms_dev, const u32 *group_off_dev, int n_out, int nq, int n_polys,
                        u64 *out, hipStream_t s, const void *terms_host, int n_terms);
 // y[o][p][j] = sum_{q < parts} part[o * parts + q][p][j] over the extended basis, y / part: [.][2][nq+K][N]

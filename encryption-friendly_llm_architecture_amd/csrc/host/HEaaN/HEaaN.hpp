@@ -89,15 +89,11 @@ public:
     size_t words() const { return words_; }
     void resize(const Context &c, size_t words);  // contents undefined afterwards
     void release();
-    // `whole` as `parts` buffers of equal size: the results of one batched launch become objects of their own without
-    // being copied out of it.  The memory goes back to the pool with the last part.
-    static std::vector<DeviceBuffer> split(DeviceBuffer &&whole, size_t parts);
 
 private:
     Context ctx_;
     u64 *ptr_ = nullptr;
     size_t words_ = 0, cap_ = 0;
-    std::shared_ptr<DeviceBuffer> whole_;   // set: ptr_ points into this buffer, which is the one to release
 };
 
 // ---- value types -----------------------------------------------------------------------------
@@ -173,7 +169,6 @@ public:
     const Context &getContext() const { return ctx_; }
     // internal
     void allocate(u64 num_poly, u64 level, u64 rescale_counter);
-    void adopt(DeviceBuffer &&b, u64 num_poly, u64 level, u64 rescale_counter);   // b: [num_poly][level+1][N]
     size_t polyStride() const;
     Context ctx_;
     DeviceBuffer buf_;  // [num_poly][level+1][N], NTT form

@@ -216,17 +216,13 @@ DeviceBuffer &DeviceBuffer::operator=(DeviceBuffer &&o) noexcept {
     ptr_ = o.ptr_;
     words_ = o.words_;
     cap_ = o.cap_;
-    whole_ = std::move(o.whole_);
     o.ptr_ = nullptr;
     o.words_ = o.cap_ = 0;
     return *this;
 }
 DeviceBuffer::~DeviceBuffer() { release(); }
 void DeviceBuffer::release() {
-    if (whole_)
-        whole_.reset();
-    else if (ptr_ && ctx_)
-        ctx_->release(ptr_, cap_);
+    if (ptr_ && ctx_) ctx_->release(ptr_, cap_);
     ptr_ = nullptr;
     words_ = cap_ = 0;
     ctx_.reset();
@@ -240,18 +236,6 @@ void DeviceBuffer::resize(const Context &c, size_t words) {
     ctx_ = c;
     ptr_ = c->alloc(words);
     words_ = cap_ = words;
-}
-
-std::vector<DeviceBuffer> DeviceBuffer::split(DeviceBuffer &&whole, size_t parts) {
-    std::vector<DeviceBuffer> r(parts);
-    const auto w = std::make_shared<DeviceBuffer>(std::move(whole));
-    for (size_t i = 0; i < parts; i++) {
-        r[i].ctx_ = w->ctx_;
-        r[i].words_ = r[i].cap_ = w->words_ / parts;
-        r[i].ptr_ = w->ptr_ + i * r[i].words_;
-        r[i].whole_ = w;
-    }
-    return r;
 }
 
 // ---- value types -------------------------------------------------------------------------------
@@ -317,14 +301,6 @@ void Ciphertext::allocate(u64 num_poly, u64 level, u64 rc) {
     log_slots_ = ctx_->logN - 1;
     occupied_ = ~u64(0);
     buf_.resize(ctx_, num_poly * (level + 1) * ctx_->N);
-}
-void Ciphertext::adopt(DeviceBuffer &&b, u64 num_poly, u64 level, u64 rc) {
-    num_poly_ = num_poly;
-    level_ = level;
-    rescale_counter_ = rc;
-    log_slots_ = ctx_->logN - 1;
-    occupied_ = ~u64(0);
-    buf_ = std::move(b);
 }
 size_t Ciphertext::polyStride() const { return (size_t)(level_ + 1) * ctx_->N; }
 u64 *Ciphertext::getPolyData(u64 i, u64 level) const {

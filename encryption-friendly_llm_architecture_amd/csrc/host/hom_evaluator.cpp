@@ -336,16 +336,20 @@ void HomEvaluator::mult(const Ciphertext &a, const Ciphertext &b, Ciphertext &ou
 void HomEvaluator::square(const Ciphertext &a, Ciphertext &out) const { mult(a, a, out); }
 
 namespace {
-// hemm_rescale of n_polys polynomials stored back to back, in as few calls as the context's scratch region allows
-// ((dnum + 7) (nQ + nP) limbs per call)
-void rescale_many(const Context &c, const u64 *in, u64 *out, u64 nq, size_t n_polys) {
+// n ciphertexts of two polynomials stored back to back, rescaled into buffers of their own (appended to `res`) in as few calls
+// as the context's scratch region allows ((dnum + 7) (nQ + nP) limbs per call)
+void rescale_many(const Context &c, const u64 *in, u64 nq, size_t n, std::vector<Ciphertext> &res) {
     const u64 N = c->N;
-    const size_t per_call = std::max<size_t>(1, (size_t)((c->dnum + 7) * (c->nQ + c->nP) / nq));
-    for (size_t p0 = 0; p0 < n_polys; p0 += per_call) {
-        const size_t np = std::min(per_call, n_polys - p0);
-        ck(hemm_rescale(c->dev, in + p0 * nq * N, nq * N, out + p0 * (nq - 1) * N, (nq - 1) * N, (uint32_t)nq, (uint32_t)np,
-                        nullptr));
+    std::vector<uint64_t *> outs;
+    for (size_t i = 0; i < n; i++) {
+        res.emplace_back(c);
+        res.back().allocate(2, nq - 2, 0);
+        outs.push_back(res.back().buf_.data());
     }
+    const size_t per_call = std::max<size_t>(1, (size_t)((c->dnum + 7) * (c->nQ + c->nP) / nq / 2));
+    for (size_t i = 0; i < n; i += per_call)
+        ck(hemm_rescale_to(c->dev, in + i * 2 * nq * N, nq * N, outs.data() + i, (nq - 1) * N, (uint32_t)nq,
+                           (uint32_t)std::min(per_call, n - i), nullptr));
 }
 }  // namespace
 
@@ -361,19 +365,14 @@ void HomEvaluator::multRealBatch(const Ciphertext &a, const std::vector<Real> &c
         out = std::move(res);
         return;
     }
-    DeviceBuffer t(ctx_, n * 2 * nq * N), low(ctx_, n * 2 * lvl * N);
+    DeviceBuffer t(ctx_, n * 2 * nq * N);
     for (size_t i = 0; i < n; i++) {
         const auto sc = int_residues(ctx_, (i64)llround(csts[i] * delta), nq);
         ck(hemm_mul_scalar(ctx_->dev, a.buf_.data(), a.polyStride(), sc.data(), t.data() + i * 2 * nq * N, nq * N, (uint32_t)nq,
                            0, 2, nullptr));
     }
-    rescale_many(ctx_, t.data(), low.data(), nq, 2 * n);
-    auto parts = DeviceBuffer::split(std::move(low), n);
-    for (size_t i = 0; i < n; i++) {
-        res.emplace_back(ctx_);
-        res.back().adopt(std::move(parts[i]), 2, lvl - 1, 0);
-        res.back().occupied_ = a.occupied_;
-    }
+    rescale_many(ctx_, t.data(), nq, n, res);
+    for (Ciphertext &r : res) r.occupied_ = a.occupied_;
     out = std::move(res);
 }
 
@@ -430,16 +429,11 @@ void HomEvaluator::multBatch(const std::vector<const Ciphertext *> &a, const std
         terms.push_back(d1);
         off.push_back((uint32_t)terms.size());
     }
-    DeviceBuffer y(ctx_, n * 2 * E * N), r(ctx_, n * ctw), ws2(ctx_, n * ctw), low(ctx_, n * 2 * lvl * N);
+    DeviceBuffer y(ctx_, n * 2 * E * N), r(ctx_, n * ctw), ws2(ctx_, n * ctw);
     ck(hemm_hoisted_moddown(ctx_->dev, terms.data(), off.data(), (uint32_t)n, (uint32_t)nq, 0, 0, y.data(), r.data(), nq * N,
                             ws2.data(), nullptr));
-    rescale_many(ctx_, r.data(), low.data(), nq, 2 * n);
-    auto parts = DeviceBuffer::split(std::move(low), n);
-    for (size_t i = 0; i < n; i++) {
-        res.emplace_back(ctx_);
-        res.back().adopt(std::move(parts[i]), 2, lvl - 1, 0);
-        res.back().occupied_ = std::min(a[i]->occupied_, b[i]->occupied_);
-    }
+    rescale_many(ctx_, r.data(), nq, n, res);
+    for (size_t i = 0; i < n; i++) res[i].occupied_ = std::min(a[i]->occupied_, b[i]->occupied_);
     out = std::move(res);
 }
 

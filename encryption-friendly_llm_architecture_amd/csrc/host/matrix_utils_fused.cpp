@@ -782,7 +782,7 @@ void MatrixTransformer::packingStageOne(const HomEvaluator &eval, const u64 *in,
 // i.e. Z = m +- i m', M_+ = +- i m, M_- = m' with m'[s] = m[s - step].  One hoisted sum with three terms per job: the two
 // rotations and Z x, which needs no key switch (a term without a key).
 void MatrixTransformer::complexPackingBatch(const HomEvaluator &eval, const u64 *in, size_t n_jobs, u64 level,
-                                            const bool *rows, i64 w, u64 *out, const u64 *scale_levels) {
+                                            const bool *rows, i64 w, u64 *const *out, const u64 *scale_levels) {
     const Context &c = eval.getContext();
     if (level < 1) throw std::invalid_argument("[complexPacking] level >= 1 is needed.");
     const u64 nq = level + 1, N = c->N, E = nq + c->nP, ctw = 2 * nq * N;
@@ -815,8 +815,8 @@ void MatrixTransformer::complexPackingBatch(const HomEvaluator &eval, const u64 
         off.push_back((uint32_t)terms.size());
     }
     DeviceBuffer y(c, n_jobs * 2 * E * N), ws(c, n_jobs * 2 * (nq - 1) * N);
-    ck(hemm_hoisted_moddown(c->dev, terms.data(), off.data(), (uint32_t)n_jobs, (uint32_t)nq, x.premultiplied(), 1, y.data(),
-                            out, (nq - 1) * N, ws.data(), nullptr));
+    ck(hemm_hoisted_moddown_to(c->dev, terms.data(), off.data(), (uint32_t)n_jobs, (uint32_t)nq, x.premultiplied(), 1, y.data(),
+                               out, (nq - 1) * N, ws.data(), nullptr));
 }
 
 namespace {
@@ -1424,8 +1424,8 @@ namespace {
 // per hoisted sum and ModDown (merged with the rescale of the mask product).  Such chains do not depend on one another and
 // go to the context's stream and the side stream in turn, each with buffers of its own, so that the launches of one fill
 // the part-empty last rounds of workgroups of the other's (a projection of 3 x 127 shifts: 12.9 ms in chains of 16 on two
-// streams, 13.4 on one; chains of 32 13.2 and 13.05).  The results stay where the ModDown leaves them (DeviceBuffer::split); copying them
-// out took 5.4 us per shift, a seventh of a hoisted projection.
+// streams, 13.4 on one; chains of 32 13.2 and 13.05).  The ModDown leaves every shift in its ciphertext; copying them out of a
+// common buffer took 5.4 us per shift, a seventh of a hoisted projection.
 void hoistedShifts(const HomEvaluator &eval, const Sources &x, const Sources &x2, const std::vector<Shift> &shifts, u64 T,
                    u64 batch, std::vector<Ciphertext> &tmp) {
     const Context &c = eval.getContext();
@@ -1438,7 +1438,12 @@ void hoistedShifts(const HomEvaluator &eval, const Sources &x, const Sources &x2
         const Context &c;
         ~JoinOnExit() { c->joinSide(); }   // also when a launch below throws
     };
-    std::vector<std::pair<DeviceBuffer, size_t>> results;
+    std::vector<Ciphertext> results(n, Ciphertext(c));
+    std::vector<uint64_t *> outs;
+    for (Ciphertext &r : results) {
+        r.allocate(2, T + 1, 0);
+        outs.push_back(r.buf_.data());
+    }
     {
         JoinOnExit join_on_exit{c};
         DeviceBuffer y[2], ws[2];
@@ -1452,16 +1457,11 @@ void hoistedShifts(const HomEvaluator &eval, const Sources &x, const Sources &x2
             std::vector<hemm_rot_term> terms;
             std::vector<uint32_t> off{0};
             pushShifts(eval, x, 0, x2, 0, shifts, first, cnt, terms, off);
-            results.emplace_back(DeviceBuffer(c, cnt * 2 * lo * N), cnt);
-            ck(hemm_hoisted_moddown(c->dev, terms.data(), off.data(), (uint32_t)cnt, (uint32_t)nq, 1, 1, y[lane].data(),
-                                    results.back().first.data(), lo * N, ws[lane].data(), lane ? side : nullptr));
+            ck(hemm_hoisted_moddown_to(c->dev, terms.data(), off.data(), (uint32_t)cnt, (uint32_t)nq, 1, 1, y[lane].data(),
+                                       outs.data() + first, lo * N, ws[lane].data(), lane ? side : nullptr));
         }
     }
-    for (auto &r : results)
-        for (DeviceBuffer &b : DeviceBuffer::split(std::move(r.first), r.second)) {
-            tmp.emplace_back(c);
-            tmp.back().adopt(std::move(b), 2, T + 1, 0);
-        }
+    for (Ciphertext &r : results) tmp.push_back(std::move(r));
 }
 }  // namespace
 
@@ -1527,15 +1527,14 @@ void complexPackingPair(const HomEvaluator &eval, MatrixTransformer &tr, const C
         throw std::invalid_argument("[complexPacking] operands must be rescaled.");
     // operands above pack_level are lowered first (both at once): the packing then runs on fewer limbs
     const u64 L = std::min<u64>(std::min(a.getLevel(), b.getLevel()), pack_level);
-    const u64 N = c->N, ctw = 2 * (L + 1) * N, half = 2 * L * N;
-    DeviceBuffer joint(c, 2 * ctw), packed(c, 2 * half);
+    DeviceBuffer joint(c, 2 * 2 * (L + 1) * c->N);
     jointLevelDown(eval, a, b, L, joint.data());
     const bool by_rows[2] = {false, true};
-    tr.complexPackingBatch(eval, joint.data(), 2, L, by_rows, w, packed.data());
     Ciphertext ra(c), rb(c);
-    auto parts = DeviceBuffer::split(std::move(packed), 2);
-    ra.adopt(std::move(parts[0]), 2, L - 1, 0);
-    rb.adopt(std::move(parts[1]), 2, L - 1, 0);
+    ra.allocate(2, L - 1, 0);
+    rb.allocate(2, L - 1, 0);
+    u64 *const out[2] = {ra.buf_.data(), rb.buf_.data()};
+    tr.complexPackingBatch(eval, joint.data(), 2, L, by_rows, w, out);
     pa = std::move(ra);
     pb = std::move(rb);
 }
@@ -1591,7 +1590,8 @@ CtxtTensor multMatMatComplexPackedFused(const HomEvaluator &eval, const Bootstra
                     const DeviceBuffer jb = truncated(b.get(), Lb);
                     DeviceBuffer pk(c, 2 * Lb * N);
                     const bool by_rows = true;
-                    tr.complexPackingBatch(eval, jb.data(), 1, Lb, &by_rows, w, pk.data(), &lb);
+                    u64 *const out = pk.data();
+                    tr.complexPackingBatch(eval, jb.data(), 1, Lb, &by_rows, w, &out, &lb);
                     tr.diagonalTransformTwoStage(eval, pk.data(), 1, Lb - 1, &kind, &shape_b, tb.data());
                 } else {          // truncated to T+3, packing + first stage (T+2), second stage (T+1)
                     const u64 Lb = T + 3;
@@ -1608,7 +1608,8 @@ CtxtTensor multMatMatComplexPackedFused(const HomEvaluator &eval, const Bootstra
                 DeviceBuffer pk(c, 2 * La * N);
                 const bool by_rows = false;
                 const MaskKind kind = MaskKind::PackedHorizontal;
-                tr.complexPackingBatch(eval, ja.data(), 1, La, &by_rows, w, pk.data(), &la);
+                u64 *const out = pk.data();
+                tr.complexPackingBatch(eval, ja.data(), 1, La, &by_rows, w, &out, &la);
                 tr.diagonalTransformTwoStage(eval, pk.data(), 1, La - 1, &kind, &shape_a, sa.data());
             } else if (la >= T + 4) {   // truncated to T+4, packing + first stage (T+3), second stage (T+2)
                 const u64 La = T + 4;
@@ -1653,7 +1654,8 @@ CtxtTensor multMatMatComplexPackedFused(const HomEvaluator &eval, const Bootstra
         tr.packingStageOne(eval, joint.data(), 2, L, kinds, shapes, packed.data(), from);
         return ccmmFused(eval, btp, a, b, T, tr, batch, single_tile, true, packed.data(), L - 1, false, add_conj, 2);
     }
-    tr.complexPackingBatch(eval, joint.data(), 2, L, by_rows, a.getBlockWidth(), packed.data(), from);
+    u64 *const out[2] = {packed.data(), packed.data() + 2 * L * N};
+    tr.complexPackingBatch(eval, joint.data(), 2, L, by_rows, a.getBlockWidth(), out, from);
     c->mark("complex packing");
     return ccmmFused(eval, btp, a, b, T, tr, batch, single_tile, true, packed.data(), L - 1, false, add_conj);
 }
@@ -1693,18 +1695,28 @@ void rotateSumFused(const HomEvaluator &eval, const std::vector<RotateSumJob> &j
         if (j.in == nullptr || j.out == nullptr || j.in->getNumPoly() != 2 || j.in->getLevel() != level ||
             j.in->getRescaleCounter() != rc)
             throw std::invalid_argument("[rotateSum] the operands must share one level and have two polynomials.");
-    const auto stages = rotateSumStages(count);
+    auto stages = rotateSumStages(count);
+    stages.erase(std::remove_if(stages.begin(), stages.end(), [](const auto &st) { return st.first <= 1; }), stages.end());
+    std::vector<Ciphertext> res(n, Ciphertext(c));   // (occupied slots: unknown, as allocate leaves them)
+    std::vector<uint64_t *> outs;
+    for (Ciphertext &r : res) {
+        r.allocate(2, level, rc);
+        outs.push_back(r.buf_.data());
+    }
+    if (stages.empty())   // one term: a copy
+        for (size_t q = 0; q < n; q++)
+            (void)hipMemcpyAsync(outs[q], jobs[q].in->buf_.data(), ctw * 8, hipMemcpyDeviceToDevice, c->stream());
     // one operand is read where it is, several are laid side by side
     DeviceBuffer cur;
     const u64 *in = jobs[0].in->buf_.data();
-    if (n > 1 || count == 1) {
+    if (n > 1 && !stages.empty()) {
         cur = DeviceBuffer(c, n * ctw);
         for (size_t q = 0; q < n; q++)
             (void)hipMemcpyAsync(cur.data() + q * ctw, jobs[q].in->buf_.data(), ctw * 8, hipMemcpyDeviceToDevice, c->stream());
         in = cur.data();
     }
-    for (const auto &st : stages) {
-        if (st.first <= 1) continue;
+    for (size_t s = 0; s < stages.size(); s++) {
+        const auto &st = stages[s];
         // raw b polynomials: the launch multiplies them by P itself (one launch less than premultiplied sources)
         const Sources x = extendSources(c, in, n, nq, nullptr, false);
         std::vector<hemm_rot_term> terms;
@@ -1721,18 +1733,19 @@ void rotateSumFused(const HomEvaluator &eval, const std::vector<RotateSumJob> &j
             terms.push_back(keylessTerm(b, a, nullptr));   // i = 0: no key switch
             off.push_back((uint32_t)terms.size());
         }
-        DeviceBuffer y(c, n * 2 * E * N), ws(c, n * ctw), nxt(c, n * ctw);
-        ck(hemm_hoisted_moddown(c->dev, terms.data(), off.data(), (uint32_t)n, (uint32_t)nq, x.premultiplied(), 0, y.data(),
-                                nxt.data(), nq * N, ws.data(), nullptr));
-        cur = std::move(nxt);
-        in = cur.data();
+        DeviceBuffer y(c, n * 2 * E * N), ws(c, n * ctw);
+        if (s + 1 == stages.size()) {
+            ck(hemm_hoisted_moddown_to(c->dev, terms.data(), off.data(), (uint32_t)n, (uint32_t)nq, x.premultiplied(), 0, y.data(),
+                                       outs.data(), nq * N, ws.data(), nullptr));
+        } else {
+            DeviceBuffer nxt(c, n * ctw);
+            ck(hemm_hoisted_moddown(c->dev, terms.data(), off.data(), (uint32_t)n, (uint32_t)nq, x.premultiplied(), 0, y.data(),
+                                    nxt.data(), nq * N, ws.data(), nullptr));
+            cur = std::move(nxt);
+            in = cur.data();
+        }
     }
-    auto parts = DeviceBuffer::split(std::move(cur), n);
-    for (size_t q = 0; q < n; q++) {
-        Ciphertext res(c);
-        res.adopt(std::move(parts[q]), 2, level, rc);
-        *jobs[q].out = std::move(res);   // (occupied slots: unknown, as adopt leaves them)
-    }
+    for (size_t q = 0; q < n; q++) *jobs[q].out = std::move(res[q]);
 }
 
 // Ciphertext x ciphertext re-use product: sum_k tmp[k] (x) rho^(k step)(b) with tmp from multMatMatPre(Fused) and

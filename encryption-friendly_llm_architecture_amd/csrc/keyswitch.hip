@@ -930,10 +930,22 @@ void launch_keyswitch(hemm_context *c, const u64 *in, const u64 *evk, int nq, u6
     launch_moddown(c, acc, nq, 2, out, out_stride, add_b, 0, add_b ? 1 : 0, coef, s);
 }
 
+// sub_scale_kernel without an addend, the results back to back or where a list says (rings without fused tails)
+static void sub_scale(const hemm_context *c, const u64 *a, size_t a_stride, const u64 *t, const CstList &cl, int n_limbs, int n_polys,
+                      u64 *out, size_t out_stride, const ResultList *list, hipStream_t s) {
+    const size_t N = c->N, t_stride = (size_t)n_limbs * N;
+    account(c, TR_POINTWISE, (size_t)3 * n_polys * n_limbs * N * 8);
+    const int run = list != nullptr ? 2 : n_polys;
+    for (int p0 = 0; p0 < n_polys; p0 += run)
+        hipLaunchKernelGGL(sub_scale_kernel, dim3(N / 256, n_limbs * std::min(run, n_polys - p0)), dim3(256), 0, s,
+                           a + p0 * a_stride, a_stride, t + p0 * t_stride, t_stride, (const u64 *)nullptr, (size_t)0, 0,
+                           list != nullptr ? list->at[p0 / 2] : out, out_stride, c->d_modq, cl, n_limbs, c->logN);
+}
+
 // in: [n_polys][nq][N] -> out: [n_polys][nq-1][N]; sc: scratch of n_polys * nq * N words, fully written before it
 // is read
 static void rescale_with(hemm_context *c, KsTables *t, u64 *sc, const u64 *in, size_t in_stride, u64 *out,
-                         size_t out_stride, int nq, int n_polys, hipStream_t s) {
+                         size_t out_stride, int nq, int n_polys, hipStream_t s, const ResultList *list = nullptr) {
     const size_t N = c->N;
     u64 *last = sc;                               // [n_polys][N]
     u64 *tt = sc + (size_t)n_polys * N;           // [n_polys][nq-1][N]
@@ -958,26 +970,24 @@ static void rescale_with(hemm_context *c, KsTables *t, u64 *sc, const u64 *in, s
         cs.d[0].n_src = 1;
         cs.hat_ld = c->nQ + c->nP;
         if (launch_ntt_converted(c, cs, tt, limbs_default(c, nq - 1, 0), ident, nq - 1, n_polys, (size_t)(nq - 1) * N, s,
-                                 in, in_stride, out, out_stride, t->dev + t->qlinv_off[nq - 1]))
+                                 in, in_stride, out, out_stride, t->dev + t->qlinv_off[nq - 1], list))
             return;
     }
     dim3 grid(N / 256, (nq - 1) * n_polys), block(256);
     account(c, TR_POINTWISE, (size_t)n_polys * nq * N * 8);
     hipLaunchKernelGGL(spread_kernel, grid, block, 0, s, last, tt, (size_t)(nq - 1) * N, c->d_modq, nq - 1, c->logN);
-    if (launch_ntt_sub_scale(c, tt, nq - 1, n_polys, in, in_stride, out, out_stride, t->dev + t->qlinv_off[nq - 1], s))
+    if (launch_ntt_sub_scale(c, tt, nq - 1, n_polys, in, in_stride, out, out_stride, t->dev + t->qlinv_off[nq - 1], s, list))
         return;
     launch_ntt(c, tt, limbs_default(c, nq - 1, 0), nq - 1, n_polys, (size_t)(nq - 1) * N, false, s);
     CstList cl;
     for (int j = 0; j < nq - 1; j++) cl.c[j] = t->qlinv[nq - 1][j];
-    account(c, TR_POINTWISE, (size_t)3 * n_polys * (nq - 1) * N * 8);
-    hipLaunchKernelGGL(sub_scale_kernel, grid, block, 0, s, in, in_stride, tt, (size_t)(nq - 1) * N,
-                       (const u64 *)nullptr, (size_t)0, 0, out, out_stride, c->d_modq, cl, nq - 1, c->logN);
+    sub_scale(c, in, in_stride, tt, cl, nq - 1, n_polys, out, out_stride, list, s);
 }
 
 void launch_rescale(hemm_context *c, const u64 *in, size_t in_stride, u64 *out, size_t out_stride, int nq,
-                    int n_polys, hipStream_t s) {
+                    int n_polys, hipStream_t s, const ResultList *list) {
     if (nq < 2) throw std::invalid_argument("rescale needs at least two limbs");
-    rescale_with(c, g_tables_of(c), hemm_scratch(c), in, in_stride, out, out_stride, nq, n_polys, s);
+    rescale_with(c, g_tables_of(c), hemm_scratch(c), in, in_stride, out, out_stride, nq, n_polys, s, list);
 }
 
 // ---- rescale for callers that cannot allocate ----------------------------------------------------
@@ -1383,9 +1393,9 @@ void launch_hoisted_terms_args(hemm_context *c, const void *terms_host, int n_te
 
 // y: [n_polys][nq+K][N] NTT (dropped limbs are clobbered).  drop_last = 0: out[p] = y[p] / P over nq limbs;
 // drop_last = 1: out[p] = y[p] / (P q_{nq-1}) over nq-1 limbs (ModDown and rescale in one conversion).
-// conv: workspace [n_polys][nq_out][N].
+// conv: workspace [n_polys][nq_out][N].  list: the results lie where it says.
 void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop_last, u64 *out, size_t out_stride,
-                          u64 *conv, hipStream_t s, bool slab) {
+                          u64 *conv, hipStream_t s, bool slab, const ResultList *list) {
     KsTables *t = g_tables_of(c);
     const int K = c->nP, E = nq + K, nq_out = drop_last ? nq - 1 : nq;
     const size_t N = c->N;
@@ -1414,6 +1424,7 @@ void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop
     const bool fold = ring_has_fused_forms(c);   // the inverse transform ends with (1/N)(S/q_i)^-1: no scaling pass in the conversion
     // the three-launch form with one column-slab kernel in the middle, only on request: it moves a fifth less data but
     // runs at two waves per SIMD and is slower on every batch size measured
+    if (slab && list != nullptr) throw std::invalid_argument("the column-slab ModDown leaves its results back to back");
     if (slab && !(c->logN == 16 && lazy_dot_ok(c))) throw std::invalid_argument("the column-slab ModDown needs N = 2^16 and primes below 2^60");
     if (slab) {
         if (!launch_moddown_slab(c, y, (size_t)E * N, a.src_slot, a.src_prime, ns,
@@ -1440,7 +1451,6 @@ void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop
         a.dst_slot[j] = (uint8_t)j;
         a.dst_prime[j] = (uint8_t)j;
     }
-    const dim3 block(256);
     const Cst *cst_dev = t->dev + (drop_last ? t->dropinv_off[nq] : t->pinv_off);
     if (fold && ns <= CONV_MAX_SOURCES && lazy_dot_ok(c)) {
         // the conversion is computed inside the first pass of the forward transform: no conversion launch, and the
@@ -1456,18 +1466,15 @@ void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop
         LimbList cl = limbs_default(c, nq_out, 0), ident;
         for (int j = 0; j < HEMM_MAX_PRIMES; j++) ident.idx[j] = (uint8_t)j;
         if (launch_ntt_converted(c, cs, conv, cl, ident, nq_out, n_polys, (size_t)nq_out * N, s, y, (size_t)E * N, out,
-                                 out_stride, cst_dev))
+                                 out_stride, cst_dev, list))
             return;
     }
     launch_bconv(c, a, c->d_modq, (int)N, n_polys, s);
-    if (launch_ntt_sub_scale(c, conv, nq_out, n_polys, y, (size_t)E * N, out, out_stride, cst_dev, s)) return;
+    if (launch_ntt_sub_scale(c, conv, nq_out, n_polys, y, (size_t)E * N, out, out_stride, cst_dev, s, list)) return;
     launch_ntt(c, conv, limbs_default(c, nq_out, 0), nq_out, n_polys, (size_t)nq_out * N, false, s);
     CstList cl;
     for (int j = 0; j < nq_out; j++) cl.c[j] = drop_last ? t->dropinv[nq][j] : t->pinv[j];
-    dim3 g2(N / 256, nq_out * n_polys);
-    account(c, TR_POINTWISE, (size_t)3 * n_polys * nq_out * N * 8);
-    hipLaunchKernelGGL(sub_scale_kernel, g2, block, 0, s, y, (size_t)E * N, conv, (size_t)nq_out * N,
-                       (const u64 *)nullptr, (size_t)0, 0, out, out_stride, c->d_modq, cl, nq_out, c->logN);
+    sub_scale(c, y, (size_t)E * N, conv, cl, nq_out, n_polys, out, out_stride, list, s);
 }
 
 

@@ -427,12 +427,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
 // LR: log2 of the rows of a limb, or 0: taken from the argument (the address arithmetic of N = 2^16 folds into constants:
 // 1 - 1.5 % of a single rotation or ciphertext product)
-template <int LR, int P, bool INV, int TAIL, int LOAD>
+template <int LR, int P, bool INV, int KTAIL, int LOAD>
 __global__ __launch_bounds__(256) void ntt16_rows_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
                                                          const Tw *__restrict__ rtw_all,
                                                          const ModQ *__restrict__ modq, const double *__restrict__ fp,
                                                          LimbList ll, LimbList sl, int n_limbs, size_t poly_stride,
-                                                         NttEpilogue ep, const int log_r_arg) {
+                                                         typename EpilogueOf<KTAIL>::T ep, const int log_r_arg) {
+    constexpr int TAIL = tail_of(KTAIL);
     constexpr int RB = P == 16 ? 4 : 3;   // log2 of the rows of a workgroup
     __shared__ u64 lds[ROWPAD << RB];
     const int log_r = LR != 0 ? LR : log_r_arg;
@@ -463,7 +464,7 @@ __global__ __launch_bounds__(256) void ntt16_rows_kernel(u64 *__restrict__ data,
     RowSecond sec{};
     if (TAIL != TAIL_NONE) {
         const size_t off = ((size_t)limb << log_n) + ((size_t)r << 8);
-        o = ep.out + (size_t)poly * ep.out_stride + off;
+        o = ep.result((int)poly) + off;
         if (TAIL == TAIL_SUB_SCALE) {
             mn = ep.minuend + (size_t)poly * ep.minuend_stride + off;
             cst = ep.cst[limb];
@@ -498,7 +499,7 @@ __global__ __launch_bounds__(256) void ntt16_rows_kernel(u64 *__restrict__ data,
 // one-launch forms (ntt_limb.hip)
 void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
                          size_t poly_stride, hipStream_t s, const ConvSources *cs, const LiftSource *ls, const NttEpilogue &ep,
-                         int tail);
+                         int tail, const ResultList *list = nullptr);
 void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
                          size_t poly_stride, hipStream_t s, const void *final_scale, const NttEpilogue &from, int load);
 
@@ -542,35 +543,38 @@ static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
 }
 static void rows_pass(const hemm_context *c, bool inverse, u64 *d, const LimbList &ll, const LimbList &sl, int n_limbs,
                       int n_polys, size_t poly_stride, hipStream_t s, const NttEpilogue &ep, int tail = TAIL_NONE,
-                      int load = LOAD_PLAIN) {
+                      int load = LOAD_PLAIN, const ResultList *list = nullptr, int first = 0) {
     const bool few = inverse || few_for_rows(c, n_limbs * n_polys);
     const dim3 grid((unsigned)(c->N >> (few ? 11 : 12)) * (unsigned)(n_limbs * n_polys)), block(256);
     const int log_r = c->logN - 8;
-#define ROWS(LR, P, INV, TAIL, LOAD)                                                                                          \
+#define ROWS(LR, P, INV, TAIL, LOAD, EP)                                                                                      \
     hipLaunchKernelGGL((ntt16_rows_kernel<LR, P, INV, TAIL, LOAD>), grid, block, 0, s, d, (const Tw *)(INV ? c->d_iw : c->d_w), \
-                       (const Tw *)(INV ? c->d_irw : c->d_rw), c->d_modq, c->d_fp, ll, sl, n_limbs, poly_stride, ep, log_r)
-#define ROWS_RING(P, INV, TAIL, LOAD)                  \
-    do {                                               \
-        if (log_r == 8) ROWS(8, P, INV, TAIL, LOAD);   \
-        else ROWS(0, P, INV, TAIL, LOAD);              \
+                       (const Tw *)(INV ? c->d_irw : c->d_rw), c->d_modq, c->d_fp, ll, sl, n_limbs, poly_stride, EP, log_r)
+#define ROWS_RING(P, INV, TAIL, LOAD, EP)                  \
+    do {                                                   \
+        if (log_r == 8) ROWS(8, P, INV, TAIL, LOAD, EP);   \
+        else ROWS(0, P, INV, TAIL, LOAD, EP);              \
     } while (0)
-#define ROWS_FORWARD(TAIL)                                   \
-    do {                                                     \
-        if (few) ROWS_RING(8, false, TAIL, LOAD_PLAIN);      \
-        else ROWS_RING(16, false, TAIL, LOAD_PLAIN);         \
+#define ROWS_FORWARD(TAIL, EP)                                   \
+    do {                                                         \
+        if (few) ROWS_RING(8, false, TAIL, LOAD_PLAIN, EP);      \
+        else ROWS_RING(16, false, TAIL, LOAD_PLAIN, EP);         \
     } while (0)
     if (inverse && load == LOAD_ROTATED)
-        ROWS_RING(8, true, TAIL_NONE, LOAD_ROTATED);
+        ROWS_RING(8, true, TAIL_NONE, LOAD_ROTATED, ep);
     else if (inverse && load == LOAD_DECRYPT)
-        ROWS_RING(8, true, TAIL_NONE, LOAD_DECRYPT);
+        ROWS_RING(8, true, TAIL_NONE, LOAD_DECRYPT, ep);
     else if (inverse)
-        ROWS_RING(8, true, TAIL_NONE, LOAD_PLAIN);
-    else if (tail == TAIL_SUB_SCALE)
-        ROWS_FORWARD(TAIL_SUB_SCALE);
+        ROWS_RING(8, true, TAIL_NONE, LOAD_PLAIN, ep);
+    else if (tail == TAIL_SUB_SCALE && list != nullptr) {
+        const NttEpilogueList epl{ep, (u32)first, *list};
+        ROWS_FORWARD(TAIL_SUB_SCALE_LIST, epl);
+    } else if (tail == TAIL_SUB_SCALE)
+        ROWS_FORWARD(TAIL_SUB_SCALE, ep);
     else if (tail == TAIL_ENCRYPT)
-        ROWS_FORWARD(TAIL_ENCRYPT);
+        ROWS_FORWARD(TAIL_ENCRYPT, ep);
     else
-        ROWS_FORWARD(TAIL_NONE);
+        ROWS_FORWARD(TAIL_NONE, ep);
 #undef ROWS_FORWARD
 #undef ROWS_RING
 #undef ROWS
@@ -610,8 +614,10 @@ static int polys_per_run(const hemm_context *c, int n_limbs, int n_polys, bool i
 // out = (minuend - NTT(data)) * cst[j]; returns false when this ring size has no fused tail (the caller
 // then runs the transform and the subtraction separately).
 bool launch_ntt_sub_scale(const hemm_context *c, u64 *data, int n_limbs, int n_polys, const u64 *minuend,
-                          size_t minuend_stride, u64 *out, size_t out_stride, const void *cst_dev, hipStream_t s) {
+                          size_t minuend_stride, u64 *out, size_t out_stride, const void *cst_dev, hipStream_t s,
+                          const ResultList *list) {
     if (!ring_has_fused_forms(c)) return false;
+    if (list != nullptr && n_polys > 2 * RESULT_PARTS) throw std::invalid_argument("too many results for one list");
     const bool one = one_launch(c, (size_t)n_limbs * n_polys, false);
     account(c, TR_NTT, (size_t)3 * n_limbs * n_polys * c->N * 8, one ? 1 : 2);   // limbs in, minuend in, result out
     LimbList ll, sl;
@@ -619,7 +625,7 @@ bool launch_ntt_sub_scale(const hemm_context *c, u64 *data, int n_limbs, int n_p
     const size_t poly_stride = (size_t)n_limbs * c->N;
     if (one) {
         launch_limb_forward(c, data, ll, sl, n_limbs, n_polys, poly_stride, s, nullptr, nullptr,
-                            sub_scale_tail(minuend, minuend_stride, out, out_stride, cst_dev), TAIL_SUB_SCALE);
+                            sub_scale_tail(minuend, minuend_stride, out, out_stride, cst_dev), TAIL_SUB_SCALE, list);
         return true;
     }
     const int run = polys_per_run(c, n_limbs, n_polys, false);
@@ -628,16 +634,17 @@ bool launch_ntt_sub_scale(const hemm_context *c, u64 *data, int n_limbs, int n_p
         u64 *d = data + (size_t)p0 * poly_stride;
         cols_pass(c, false, d, ll, sl, n_limbs, np, poly_stride, s);
         rows_pass(c, false, d, ll, sl, n_limbs, np, poly_stride, s,
-                  sub_scale_tail(minuend + (size_t)p0 * minuend_stride, minuend_stride, out + (size_t)p0 * out_stride, out_stride,
-                                 cst_dev),
-                  TAIL_SUB_SCALE);
+                  sub_scale_tail(minuend + (size_t)p0 * minuend_stride, minuend_stride,
+                                 list != nullptr ? nullptr : out + (size_t)p0 * out_stride, out_stride, cst_dev),
+                  TAIL_SUB_SCALE, LOAD_PLAIN, list, p0);
     }
     return true;
 }
 
 bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *data, const LimbList &ll, const LimbList &sl,
                           int n_limbs, int n_polys, size_t poly_stride, hipStream_t s, const u64 *ep_minuend,
-                          size_t ep_minuend_stride, u64 *ep_out, size_t ep_out_stride, const void *ep_cst_dev) {
+                          size_t ep_minuend_stride, u64 *ep_out, size_t ep_out_stride, const void *ep_cst_dev,
+                          const ResultList *ep_list) {
     if (!ring_has_fused_forms(c)) return false;
     if (n_limbs > HEMM_MAX_PRIMES || cs.n_copy < 0 || cs.n_copy > HEMM_MAX_PRIMES)
         throw std::invalid_argument("too many limbs in one converted transform");
@@ -648,7 +655,8 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
     }
     if (widest < 1 || widest > CONV_MAX_SOURCES) return false;
     if (n_limbs <= 0 || n_polys <= 0) return true;
-    const bool tail = ep_out != nullptr;
+    if (ep_list != nullptr && n_polys > 2 * RESULT_PARTS) throw std::invalid_argument("too many results for one list");
+    const bool tail = ep_out != nullptr || ep_list != nullptr;
     // sources of every digit in use once, limbs out (through the tail: minuend in, result out)
     size_t src_limbs = 0;
     bool seen[CONV_MAX_DIGITS] = {false, false, false, false};
@@ -665,7 +673,7 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
     if (one) {
         launch_limb_forward(c, data, ll, sl, n_limbs, n_polys, poly_stride, s, &cs, nullptr,
                             sub_scale_tail(ep_minuend, ep_minuend_stride, ep_out, ep_out_stride, ep_cst_dev),
-                            tail ? TAIL_SUB_SCALE : TAIL_NONE);
+                            tail ? TAIL_SUB_SCALE : TAIL_NONE, ep_list);
         return true;
     }
     const dim3 grid((unsigned)(c->N >> 12), (n_limbs + cs.n_copy) * n_polys);
@@ -687,7 +695,8 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
 #undef CONV_RING
 #undef CONV_CASE
     rows_pass(c, false, data, ll, sl, n_limbs, n_polys, poly_stride, s,
-              sub_scale_tail(ep_minuend, ep_minuend_stride, ep_out, ep_out_stride, ep_cst_dev), tail ? TAIL_SUB_SCALE : TAIL_NONE);
+              sub_scale_tail(ep_minuend, ep_minuend_stride, ep_out, ep_out_stride, ep_cst_dev), tail ? TAIL_SUB_SCALE : TAIL_NONE,
+              LOAD_PLAIN, ep_list);
     return true;
 }
 

@@ -19,6 +19,17 @@ struct NttEpilogue {
     u64 *second_out;
     const u64 *sk;          // [prime][N]
     u64 a_base;             // the stream of prime i has key sm64(sm64(a_base + i))
+    __device__ __forceinline__ u64 *result(const int poly) const { return out + (size_t)poly * out_stride; }
+};
+// the same with the results where a list says, the launch's first polynomial being number `first` of it: a type of its own, since
+// the list in the arguments of every launch made single key switches 0.4 % slower
+struct NttEpilogueList : NttEpilogue {
+    u32 first;
+    ResultList list;
+    __device__ __forceinline__ u64 *result(const int poly) const {
+        const u32 p = first + (u32)poly;
+        return list.at[p >> 1] + (p & 1 ? out_stride : 0);
+    }
 };
 
 namespace {
@@ -390,7 +401,17 @@ __device__ __forceinline__ void wave_sync() {
 //                   v - a s to `out`.
 // Optional origin of an inverse transform's input (LOAD): `data` itself or `minuend` (same slot numbering, own polynomial
 // stride; nullptr: data), LOAD_ROTATED: `minuend` through the automorphism `galois`, LOAD_DECRYPT: minuend + second_in * s.
-enum { TAIL_NONE = 0, TAIL_SUB_SCALE = 1, TAIL_ENCRYPT = 2 };
+//   TAIL_SUB_SCALE_LIST: TAIL_SUB_SCALE with results where a list says (a kernel's choice of NttEpilogueList; not of rows_body).
+enum { TAIL_NONE = 0, TAIL_SUB_SCALE = 1, TAIL_ENCRYPT = 2, TAIL_SUB_SCALE_LIST = 3 };
+constexpr int tail_of(const int tail) { return tail == TAIL_SUB_SCALE_LIST ? (int)TAIL_SUB_SCALE : tail; }
+template <int TAIL>
+struct EpilogueOf {
+    typedef NttEpilogue T;
+};
+template <>
+struct EpilogueOf<TAIL_SUB_SCALE_LIST> {
+    typedef NttEpilogueList T;
+};
 enum { LOAD_PLAIN = 0, LOAD_ROTATED = 1, LOAD_DECRYPT = 2 };
 // what TAIL_ENCRYPT and LOAD_DECRYPT need for one row
 struct RowSecond {

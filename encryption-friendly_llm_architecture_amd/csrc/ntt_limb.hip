@@ -92,11 +92,12 @@ __device__ __forceinline__ void limb_forward(u64 *__restrict__ limb, const Tw *_
 
 // data[n_polys][.][N] (polynomial stride poly_stride), limb l in slot sl[l]; the plain copies of cs follow the limbs of a
 // polynomial.
-template <int LR, int P, int NS, int TAIL>
+template <int LR, int P, int NS, int KTAIL>
 __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_forward_kernel(
     u64 *__restrict__ data, const Tw *__restrict__ tw_all, const Tw *__restrict__ rtw_all, const ModQ *__restrict__ modq,
     const double *__restrict__ fp, LimbList ll, LimbList sl, int n_limbs, size_t poly_stride, ConvSources cs,
-    LiftSource ls, NttEpilogue ep) {
+    LiftSource ls, typename EpilogueOf<KTAIL>::T ep) {
+    constexpr int TAIL = tail_of(KTAIL);
     __shared__ u64 lds[(ROWPAD << LR)];
     const int log_n = 8 + LR;
     const int per_poly = n_limbs + (NS > 0 ? cs.n_copy : 0);
@@ -138,7 +139,7 @@ __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_forward_kernel(
     u64 *o = nullptr;
     Tw cst{0, 0};
     RowSecond sec{};
-    if (TAIL != TAIL_NONE) o = ep.out + (size_t)poly * ep.out_stride + ((size_t)limb << log_n);
+    if (TAIL != TAIL_NONE) o = ep.result(poly) + ((size_t)limb << log_n);
     if (TAIL == TAIL_SUB_SCALE) {
         mn = ep.minuend + (size_t)poly * ep.minuend_stride + ((size_t)limb << log_n);
         cst = ep.cst[limb];
@@ -234,7 +235,7 @@ __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_inverse_kernel(
 
 void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
                          size_t poly_stride, hipStream_t s, const ConvSources *cs, const LiftSource *ls, const NttEpilogue &ep,
-                         int tail) {
+                         int tail, const ResultList *list) {
     const int LR = c->logN - 8;
     int widest = 0;
     ConvSources conv;
@@ -245,30 +246,33 @@ void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, c
         for (int l = 0; l < n_limbs; l++) widest = std::max(widest, cs->d[cs->digit_of[l]].n_src);
     }
     if (ls != nullptr) lift = *ls;
+    NttEpilogueList epl{ep, 0, {}};
+    if (list != nullptr) epl.list = *list;
     const dim3 grid((unsigned)((n_limbs + conv.n_copy) * n_polys)), block((unsigned)((256 / POINTS(LR)) << LR));
-#define LIMB_FORWARD(L, K, TAIL)                                                                                           \
+#define LIMB_FORWARD(L, K, TAIL, EP)                                                                                       \
     hipLaunchKernelGGL((ntt_limb_forward_kernel<L, POINTS(L), K, TAIL>), grid, block, 0, s, data, (const Tw *)c->d_w,                 \
-                       (const Tw *)c->d_rw, c->d_modq, c->d_fp, ll, sl, n_limbs, poly_stride, conv, lift, ep)
-#define LIMB_SOURCES(L, TAIL)                          \
-    do {                                               \
-        if (widest == 0) LIMB_FORWARD(L, 0, TAIL);     \
-        else if (widest <= 2) LIMB_FORWARD(L, 2, TAIL); \
-        else if (widest <= 5) LIMB_FORWARD(L, 5, TAIL); \
-        else LIMB_FORWARD(L, 8, TAIL);                 \
+                       (const Tw *)c->d_rw, c->d_modq, c->d_fp, ll, sl, n_limbs, poly_stride, conv, lift, EP)
+#define LIMB_SOURCES(L, TAIL, EP)                          \
+    do {                                                   \
+        if (widest == 0) LIMB_FORWARD(L, 0, TAIL, EP);     \
+        else if (widest <= 2) LIMB_FORWARD(L, 2, TAIL, EP); \
+        else if (widest <= 5) LIMB_FORWARD(L, 5, TAIL, EP); \
+        else LIMB_FORWARD(L, 8, TAIL, EP);                 \
     } while (0)
 #define LIMB_RING(L)                                                       \
     do {                                                                   \
-        if (ls != nullptr && tail == TAIL_ENCRYPT) LIMB_FORWARD(L, LIFTED, TAIL_ENCRYPT); \
-        else if (ls != nullptr) LIMB_FORWARD(L, LIFTED, TAIL_NONE);        \
-        else if (tail == TAIL_SUB_SCALE) LIMB_SOURCES(L, TAIL_SUB_SCALE);  \
-        else LIMB_SOURCES(L, TAIL_NONE);                                   \
+        if (ls != nullptr && tail == TAIL_ENCRYPT) LIMB_FORWARD(L, LIFTED, TAIL_ENCRYPT, ep); \
+        else if (ls != nullptr) LIMB_FORWARD(L, LIFTED, TAIL_NONE, ep);    \
+        else if (tail == TAIL_SUB_SCALE && list != nullptr) LIMB_SOURCES(L, TAIL_SUB_SCALE_LIST, epl); \
+        else if (tail == TAIL_SUB_SCALE) LIMB_SOURCES(L, TAIL_SUB_SCALE, ep);  \
+        else LIMB_SOURCES(L, TAIL_NONE, ep);                               \
     } while (0)
     switch (LR) {
         case 2: LIMB_RING(2); break;
         case 3: LIMB_RING(3); break;
         case 4: LIMB_RING(4); break;
         case 5: LIMB_RING(5); break;
-        case 6: LIMB_FORWARD(6, 0, TAIL_NONE); break;
+        case 6: LIMB_FORWARD(6, 0, TAIL_NONE, ep); break;
         default: throw std::invalid_argument("no one-launch transform for this ring size");
     }
 #undef LIMB_RING

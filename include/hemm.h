@@ -245,6 +245,11 @@ int hemm_hoisted_terms(hemm_context *ctx, const hemm_rot_term *terms, const uint
 int hemm_hoisted_moddown(hemm_context *ctx, const hemm_rot_term *terms, const uint32_t *group_offsets,
                          uint32_t n_out, uint32_t nq, int b_premultiplied, int drop_last, uint64_t *y_workspace,
                          uint64_t *out, size_t out_stride, uint64_t *workspace, void *stream);
+/* the same with every result in a buffer of its own: outs (host array of device pointers) [n_out], outs[o]: [2][nq_out][N] with
+ * polynomial stride out_stride, none overlapping another or the operands */
+int hemm_hoisted_moddown_to(hemm_context *ctx, const hemm_rot_term *terms, const uint32_t *group_offsets,
+                            uint32_t n_out, uint32_t nq, int b_premultiplied, int drop_last, uint64_t *y_workspace,
+                            uint64_t *const *outs, size_t out_stride, uint64_t *workspace, void *stream);
 
 /* y [n_polys][nq+n_p][N] (clobbered) -> out [n_polys][nq - drop_last][N]: division by P (drop_last = 0)
  * or by P*q_{nq-1} (drop_last = 1, ModDown and rescale in one basis conversion);
@@ -292,7 +297,11 @@ int hemm_tensor_batch_groups(hemm_context *ctx, const hemm_tensor_group *groups,
  * out == in with equal strides (each result then takes the place of its own input); anything else is refused. */
 int hemm_rescale(hemm_context *ctx, const uint64_t *in, size_t in_stride, uint64_t *out,
                  size_t out_stride, uint32_t nq, uint32_t n_polys, void *stream);
-
+/* the same for n_out ciphertexts of two polynomials each, in: [n_out][2][nq][N], every result in a buffer of its own: outs (host
+ * array of device pointers) [n_out], outs[o]: [2][nq-1][N] with polynomial stride out_stride.  No output may overlap `in`
+ * or another one. */
+int hemm_rescale_to(hemm_context *ctx, const uint64_t *in, size_t in_stride, uint64_t *const *outs, size_t out_stride,
+                    uint32_t nq, uint32_t n_out, void *stream);
 
 /* hemm_rescale for callers that cannot allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  It has no counterpart in the reference.  Same arguments, same kernels and same
