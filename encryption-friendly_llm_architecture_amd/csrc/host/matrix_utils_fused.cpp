@@ -1421,18 +1421,20 @@ CtxtTensor multPackedMatMatFused(const HomEvaluator &eval, const Bootstrapper &b
 
 namespace {
 // The column shifts of a pair of sources at level T + 2 as ciphertexts of level T + 1, appended to `tmp`: `batch` shifts
-// per hoisted sum and ModDown (merged with the rescale of the mask product).  Such chains do not depend on one another and
-// go to the context's stream and the side stream in turn, each with buffers of its own, so that the launches of one fill
-// the part-empty last rounds of workgroups of the other's (a projection of 3 x 127 shifts: 12.9 ms in chains of 16 on two
-// streams, 13.4 on one; chains of 32 13.2 and 13.05).  The ModDown leaves every shift in its ciphertext; copying them out of a
-// common buffer took 5.4 us per shift, a seventh of a hoisted projection.
+// at a time through hoisted sums and ModDowns (merged with the rescale of the mask product).  More than `batch` shifts go to the
+// context's stream and the side stream in turn, in chains of half as many that do not depend on one another, so that the launches
+// of one fill the part-empty last rounds of workgroups of the other's and the two workspaces together are no larger than one for
+// `batch` shifts (285 MB for 16 at the preset).  A projection of 3 x 127 shifts: 11.95 ms so, 11.90 with two whole workspaces, 0.5 ms
+// more on one stream; batches of 32 12.15.  The ModDown leaves every shift in its ciphertext; copying them out of a common buffer took
+// 5.4 us per shift, a seventh of a hoisted projection.
 void hoistedShifts(const HomEvaluator &eval, const Sources &x, const Sources &x2, const std::vector<Shift> &shifts, u64 T,
                    u64 batch, std::vector<Ciphertext> &tmp) {
     const Context &c = eval.getContext();
     const u64 nq = T + 3, N = c->N, E = nq + c->nP, lo = nq - 1;
-    const size_t n = shifts.size(), G = std::max<u64>(1, std::min<u64>(batch, (u64)n));
+    const size_t n = shifts.size(), whole = std::max<u64>(1, std::min<u64>(batch, (u64)n));
     // longer term lists are staged from pageable memory, which waits for the stream: no second stream for them
-    const bool two = n > G && G <= 32;
+    const bool two = n > whole && whole >= 2 && whole <= 32;
+    const size_t G = two ? whole / 2 : whole;
     const hipStream_t side = two ? c->forkSide() : nullptr;
     struct JoinOnExit {
         const Context &c;

@@ -127,3 +127,28 @@ def test_one_of_two_results_keeps_only_its_own_memory():
     taken = (free - torch.cuda.mem_get_info()[0]) / count
     assert taken < 1.5 * own, (taken, own)       # a shared buffer holds two; allocations are rounded up a little
     assert np.array_equal(kept[0].residues(), kept[-1].residues())
+
+
+def test_shifts_on_two_streams_share_one_workspace():
+    """The column shifts of an activation run in two chains side by side; their workspaces together are one for `batch` shifts."""
+    import torch
+    pkg = load_package()
+    from efla_amd import hellm
+    log_n, target, special = 14, 4, 4
+    qs, ps = O.ckks_chain(log_n, 9, special)
+    H = hellm.HEMMer(log_n, qs, ps, dnum=3, min_bootstrap_level=0, seed=5)
+    x = H.encrypt(np.random.default_rng(1).normal(size=(H.dim, H.dim)))
+    H.set_schedule(True, 4)
+    a = H.matmul_pre(x, target)                  # keys, masks, and as many results as the call below takes from the pool
+    first = a.get(H.dim - 1, H.dim, H.dim, H.dim).residues()
+    a.free()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    H.set_schedule(True, 16)
+    b = H.matmul_pre(x, target)
+    torch.cuda.synchronize()
+    taken = free - torch.cuda.mem_get_info()[0]
+    nq = target + 3
+    workspace = 16 * 2 * ((nq + special) + (nq - 1)) * 8 << log_n
+    assert taken < 1.25 * workspace, (taken, workspace)
+    assert np.array_equal(first, b.get(H.dim - 1, H.dim, H.dim, H.dim).residues())
