@@ -114,7 +114,16 @@ struct ContextContent {
     std::condition_variable stage_free;
     Stage takeStage() {
         std::unique_lock<std::mutex> lk(mu);
-        if (stages.empty() && stages_made < STAGES) {
+        // another one while work that has not run yet reads the longest unused: a queue of messages does not wait for the GPU
+        // before it holds STAGES of them
+        const auto idle = [&] {
+            if (stages.empty()) return false;
+            if (!stages.front().pending) return true;
+            if (hipEventQuery(stages.front().done) == hipSuccess) stages.front().pending = false;
+            else (void)hipGetLastError();   // "not ready" is an answer here, not an error for the next launch to report
+            return !stages.front().pending;
+        };
+        if (stages_made < STAGES && !idle()) {
             Stage s;
             if (hipHostMalloc((void **)&s.values, N / 2 * sizeof(double)) != hipSuccess)
                 throw RuntimeException("hipHostMalloc failed");
