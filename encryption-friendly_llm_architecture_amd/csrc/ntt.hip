@@ -767,7 +767,8 @@ bool launch_intt_from(const hemm_context *c, const u64 *src, size_t src_poly_str
         return false;
     }
     if (n_limbs <= 0 || n_polys <= 0) return true;
-    const bool one = one_launch(c, (size_t)n_limbs * n_polys, galois == 0);
+    // (through an automorphism: the input of a single key switch, less than the 64 limbs of the line of 2^13 points)
+    const bool one = galois == 0 ? one_launch(c, (size_t)n_limbs * n_polys, true) : c->logN <= 12;
     account(c, TR_NTT, (size_t)2 * n_limbs * n_polys * c->N * 8, one ? 1 : 2);
     if (one) {
         NttEpilogue from{};
@@ -797,7 +798,9 @@ bool launch_ntt_lifted(const hemm_context *c, const LiftSource &ls, u64 *data, c
     if (!ring_has_fused_forms(c)) return false;
     LimbList sl;
     for (int j = 0; j < HEMM_MAX_PRIMES; j++) sl.idx[j] = (uint8_t)j;
-    const bool one = one_launch(c, (size_t)n_limbs * n_polys, false);
+    // (an encryption has a limb per chain prime, 64 at most: the line of 2^13 points is reached by one chain length, without
+    // special primes, which is not worth a kernel)
+    const bool one = one_launch(c, (size_t)n_limbs * n_polys, false) && (enc == nullptr || c->logN <= 12);
     account(c, TR_NTT, (size_t)(n_limbs + 1) * n_polys * c->N * 8 + (enc ? (size_t)2 * n_limbs * n_polys * c->N * 8 : 0), one ? 1 : 2);
     NttEpilogue ep{};
     if (enc != nullptr) {
@@ -842,7 +845,7 @@ bool launch_intt_decrypt(const hemm_context *c, const u64 *b, const u64 *a, cons
     if (!ring_has_fused_forms(c)) return false;
     LimbList ll;
     for (int j = 0; j < HEMM_MAX_PRIMES; j++) ll.idx[j] = (uint8_t)j;
-    const bool one = one_launch(c, (size_t)n_limbs, false);
+    const bool one = c->logN <= 12;   // one or two limbs
     account(c, TR_NTT, (size_t)4 * n_limbs * c->N * 8, one ? 1 : 2);
     NttEpilogue from{};
     from.minuend = b;

@@ -271,7 +271,13 @@ void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, c
         case 2: LIMB_RING(2); break;
         case 3: LIMB_RING(3); break;
         case 4: LIMB_RING(4); break;
-        case 5: LIMB_RING(5); break;
+        case 5:
+            if (tail == TAIL_ENCRYPT) throw std::invalid_argument("no one-launch encryption for this ring size");
+            if (ls != nullptr) LIMB_FORWARD(5, LIFTED, TAIL_NONE, ep);
+            else if (tail == TAIL_SUB_SCALE && list != nullptr) LIMB_SOURCES(5, TAIL_SUB_SCALE_LIST, epl);
+            else if (tail == TAIL_SUB_SCALE) LIMB_SOURCES(5, TAIL_SUB_SCALE, ep);
+            else LIMB_SOURCES(5, TAIL_NONE, ep);
+            break;
         case 6: LIMB_FORWARD(6, 0, TAIL_NONE, ep); break;
         default: throw std::invalid_argument("no one-launch transform for this ring size");
     }
@@ -298,7 +304,10 @@ void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, c
         case 2: LIMB_RING(2); break;
         case 3: LIMB_RING(3); break;
         case 4: LIMB_RING(4); break;
-        case 5: LIMB_RING(5); break;
+        case 5:
+            if (load != LOAD_PLAIN) throw std::invalid_argument("no such one-launch transform for this ring size");
+            LIMB_INVERSE(5, LOAD_PLAIN);
+            break;
         case 6: LIMB_INVERSE(6, LOAD_PLAIN); break;
         default: throw std::invalid_argument("no one-launch transform for this ring size");
     }

@@ -1,4 +1,8 @@
-"""Matrices on their way to the GPU through pinned host memory."""
+"""Encoding, encryption, decryption and decoding on every ring that runs the register-blocked passes (2^10 .. 2^16), against the CPU
+oracle: residues and decoded doubles bit for bit.  The embedding has a kernel per number of rows, the reduction of rounded
+coefficients inside the transform a one-launch and a two-launch form."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -6,6 +10,98 @@ from __graft_entry__ import load_package
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
+
+
+def dev(a):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(a).view(np.int64)).cuda()
+
+
+def host(t):
+    return t.cpu().numpy().view(np.uint64)
+
+
+def moduli(log_n, limbs):
+    """primes of 61, 60 and 44 bits: the three forms of arithmetic"""
+    return ([O.primes_below(61, log_n, 1)[0], O.primes_below(60, log_n, 1)[0]] + O.primes_below(44, log_n, max(1, limbs - 2)))[:limbs]
+
+
+def make(log_n, limbs):
+    pkg = load_package()
+    mods = moduli(log_n, limbs)
+    return pkg, pkg.Context(log_n, mods, [], 1), O.Oracle(log_n, mods, [], 1, threads=8)
+
+
+def slots(orc, count, seed):
+    rng = np.random.default_rng(seed)
+    z = rng.uniform(-1, 1, (count, orc.slots)) + 1j * rng.uniform(-1, 1, (count, orc.slots))
+    z[0, orc.slots // 3:] = 0
+    z[-1, 0] = -1.0
+    return z
+
+
+# the widest scale leaves coefficients of about 2^58, beyond the primes of 44 bits
+@pytest.mark.parametrize("log_n", [10, 11, 12, 13, 14, 15, 16])
+@pytest.mark.parametrize("log_scale", [42, 57])
+def test_encode_and_decode(log_n, log_scale):
+    import torch
+    pkg, ctx, orc = make(log_n, 4)
+    z, scale = slots(orc, 3, log_n), 2.0 ** log_scale * 1.0009765625
+    got = host(ctx.encode(torch.from_numpy(z).cuda(), scale, 4))
+    want = [orc.encode(m, 3, scale) for m in z]
+    for m in range(3):
+        assert np.array_equal(got[m], want[m].data), m
+    for limbs in (1, 2):
+        if limbs == 1 and log_scale > 50:
+            continue   # beyond the first prime
+        d = ctx.decode(dev(want[1].data[:limbs]), scale, n_limbs=limbs).cpu().numpy()
+        assert np.array_equal(d.view(np.float64), orc.decode(O.Pt(want[1].data[:limbs], scale)).view(np.float64)), limbs
+
+
+# limbs on both sides of the 64 from which a ring of 2^13 points takes one launch; a batch that is cut into runs (2^16: 448 limbs)
+@pytest.mark.parametrize("log_n,messages,limbs,check", [(13, 21, 3, (0, 20)), (13, 16, 4, (0, 7, 15)), (13, 13, 5, (0, 12)), (14, 20, 5, (0, 19)),
+                                                        (16, 90, 5, (0, 37, 38, 89))])
+def test_encode_of_batches(log_n, messages, limbs, check):
+    import torch
+    pkg, ctx, orc = make(log_n, limbs)
+    z, scale = slots(orc, messages, messages), 2.0 ** 42
+    got = host(ctx.encode(torch.from_numpy(z).cuda(), scale, limbs))
+    for m in check:
+        assert np.array_equal(got[m], orc.encode(z[m], limbs - 1, scale).data), m
+
+
+# (2^13 points, 64 limbs: the longest chain there is, and no special primes)
+@pytest.mark.parametrize("log_n,limbs,count", [(10, 4, 512), (11, 3, 1021), (12, 4, 1), (13, 4, 4095), (13, 64, 4096), (14, 3, 8192), (15, 4, 9999),
+                                               (16, 4, 32768)])
+def test_encrypt_and_decrypt(log_n, limbs, count):
+    import torch
+    pkg, ctx, orc = make(log_n, limbs)
+    L, N, seed, scale = pkg.lib(), 1 << log_n, 17 + log_n, 2.0 ** 42
+    f64, u64, vp, sz, u32 = ctypes.c_double, ctypes.c_uint64, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_uint32
+    L.hemm_encrypt_reals.argtypes = [vp, vp, sz, f64, u32, vp, u64, u64, vp, vp, sz, vp]
+    L.hemm_decrypt_reals.argtypes = [vp, vp, sz, vp, u32, f64, vp, vp, sz, vp]
+    orc.gen_secret(3)
+    sk = dev(orc.sk)
+    v = np.random.default_rng(seed).uniform(-1, 1, count)
+    values = torch.from_numpy(v).cuda()
+    for nq in sorted({limbs, 2}):
+        stride = nq * N + 2
+        ct = torch.full((2, stride), -1, dtype=torch.int64, device="cuda")
+        ws = torch.empty(N, dtype=torch.int64, device="cuda")
+        pkg.check(L.hemm_encrypt_reals(ctx.h, values.data_ptr(), count, scale, nq, sk.data_ptr(),
+                                       O.lib().orc_sm64((seed + O.TAG_ENC_A) % 2 ** 64), orc.stream(seed, O.TAG_ENC_E), ws.data_ptr(),
+                                       ct.data_ptr(), stride, None))
+        want = orc.encrypt(orc.encode(v, nq - 1, scale), seed)
+        assert np.array_equal(host(ct[:, : nq * N].reshape(2, nq, N)), want.data), nq
+        assert bool((ct[:, nq * N:] == -1).all())
+        for n in (1, 2):
+            out = torch.full((count + 1,), -7.0, dtype=torch.float64, device="cuda")
+            ws = torch.empty((n + 1) * N, dtype=torch.int64, device="cuda")
+            pkg.check(L.hemm_decrypt_reals(ctx.h, ct.data_ptr(), stride, sk.data_ptr(), n, scale, ws.data_ptr(), out.data_ptr(), count, None))
+            ref = orc.decode(orc.decrypt_pt(O.Ct(np.ascontiguousarray(want.data[:, :n]), scale))).real[:count]
+            assert np.array_equal(out.cpu().numpy()[:count].view(np.uint64), np.ascontiguousarray(ref).view(np.uint64)), (nq, n)
+            assert float(out[count]) == -7.0
+            assert np.abs(ref - v).max() < 1e-6
 
 
 @pytest.mark.parametrize("log_n", [10, 16])
