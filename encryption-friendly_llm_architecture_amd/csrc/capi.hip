@@ -603,8 +603,8 @@ int hemm_hoisted_moddown_to(hemm_context *ctx, const hemm_rot_term *terms, const
     for (uint32_t o = 0; o < n_out; o += RESULT_PARTS) {
         const uint32_t n = std::min<uint32_t>(n_out - o, RESULT_PARTS);
         const ResultList list = results_in(outs + o, n);
-        launch_moddown_batch(ctx, (u64 *)y_workspace + o * y_words, (int)nq, (int)(2 * n), drop_last != 0, nullptr, out_stride,
-                             (u64 *)workspace + o * ws_words, on_stream(ctx, stream), false, &list);
+        launch_moddown_batch(ctx, (u64 *)y_workspace + o * y_words, (int)nq, (int)(2 * n), drop_last != 0, list.at[0], out_stride,
+                             (u64 *)workspace + o * ws_words, on_stream(ctx, stream), false, n > 1 ? &list : nullptr);
     }
     check_launch();
     HEMM_CATCH
@@ -800,8 +800,8 @@ int hemm_rescale_to(hemm_context *ctx, const uint64_t *in, size_t in_stride, uin
     for (uint32_t o = 0; o < n_out; o += RESULT_PARTS) {
         const uint32_t n = std::min<uint32_t>(n_out - o, RESULT_PARTS);
         const ResultList list = results_in(outs + o, n);
-        launch_rescale(ctx, (const u64 *)in + (size_t)2 * o * in_stride, in_stride, nullptr, out_stride, (int)nq, (int)(2 * n),
-                       on_stream(ctx, stream), &list);
+        launch_rescale(ctx, (const u64 *)in + (size_t)2 * o * in_stride, in_stride, list.at[0], out_stride, (int)nq, (int)(2 * n),
+                       on_stream(ctx, stream), n > 1 ? &list : nullptr);
     }
     check_launch();
     HEMM_CATCH
