@@ -230,7 +230,7 @@ def gpu_ntt(args, out):
     # launches moves that much, so the pair cannot exceed half of the HBM roofline on this figure)
     alg_bytes = limbs * 2 * LIMB_BYTES
     out["roofline_ntt"] = {
-        "kernel": "ntt16_cols_kernel<false> + ntt16_rows_kernel<false> (one forward transform of "
+        "kernel": "ntt16_cols_kernel<8, 16, false> + ntt16_rows_kernel<8, 16, false, 0, 0> (one forward transform of "
                   "32x24 limbs = 2 launches), 60-bit primes / 42-bit primes",
         "bound": "hbm", "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "achieved": alg_bytes / (fwd_ms * 1e-3) / 1e9, "frac": alg_bytes / (fwd_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
@@ -354,8 +354,8 @@ def gpu_hoisted(args, out):
         ctx.moddown_batch(y, nq, True, column_slab=True)
     ms3_slab = timer.stop() / iters
     out["roofline"] = {
-        "kernel": "ntt16_rows_kernel<true,false> + ntt16_cols_kernel<true> + ntt16_cols_converted_kernel<5> + "
-                  "ntt16_rows_kernel<false,true> (ModDown + rescale of one main-loop batch, 64 polynomials, 7+4 -> 6 limbs: "
+        "kernel": "ntt16_rows_kernel<8, 8, true, 0, 0> + ntt16_cols_kernel<8, 16, true> + ntt16_cols_converted_kernel<8, 5> + "
+                  "ntt16_rows_kernel<8, 16, false, 1, 0> (ModDown + rescale of one main-loop batch, 64 polynomials, 7+4 -> 6 limbs: "
                   "the largest kernel family of the CCMM; the basis conversion runs inside the first forward pass)",
         "bound": "hbm", "achieved": md_bytes / (ms3 * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "frac": md_bytes / (ms3 * 1e-3) / 1e9 / HBM_PEAK_GBS, "traffic": MODDOWN_TRAFFIC_BYTES,

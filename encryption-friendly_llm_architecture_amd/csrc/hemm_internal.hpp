@@ -67,10 +67,17 @@ inline void account(const hemm_context *c, int kind, size_t bytes, int n_launche
 // a subtraction and a constant, and read through an automorphism (primes below 2^44 in double precision, twiddle tables
 // laid out for it).
 inline bool ring_has_fused_forms(const hemm_context *c) { return c->logN >= 10; }
-// Whether a transform is one launch with a workgroup per limb: up to 2^12 points always.  A larger limb is slower in one
-// workgroup than spread over several in two launches (2^13 points: 11.3 against 9.0 us for one limb, 12.0 against 11.8
-// for 48 of 60 bits; 2^14: 21 against 18.5 us for 64), until the limbs alone fill the CUs and the second trip through memory is what
-// counts (60-bit primes: 34.6 against 47.2 us for 768 limbs of 2^13; 2^14: 23 against 28 us for 128, 81 against 87 for 768).
+// Whether a transform is one launch with a workgroup per limb: up to 2^12 points always.  A larger limb of 60 bits is slower in
+// one workgroup than spread over several in two launches, until the limbs alone fill the CUs and the second trip through memory is
+// what counts; one of 42 bits has fewer instructions to spread and gains earlier.  A launch may hold limbs of both, so the lines
+// lie where 60-bit ones have crossed over.  Forward, us in one launch / in two:
+//   2^13 points, limbs    1          8         48         64        128         768
+//     60 bits     11.2/ 9.3  11.6/ 9.8  12.2/12.3  12.2/13.1  12.9/19.0   36.9/46.7
+//     42 bits      8.0/ 8.1   8.1/ 9.7   8.2/10.4   8.6/11.3   9.0/16.8   24.5/37.6
+//   2^14 points, limbs    8         48         64         80         96        128        768
+//     60 bits     20.3/10.3  21.6/16.4  21.5/18.4  21.6/23.2  21.8/25.5  23.5/30.0  78.0/82.8
+//     42 bits     12.1/ 8.8  13.2/14.0  13.1/16.0  13.3/19.3  13.4/21.3  14.3/25.3  54.4/67.3
+// (inverse ones alike: 60 bits cross over at 48 to 64 resp. 64 to 96 limbs; 768 of 2^14 points and 60 bits 86.3/85.6).
 // plain: no conversion, tail or automorphism -- with them a workgroup of the 1024 threads a limb of 2^14 takes would spill.
 inline bool one_launch(const hemm_context *c, size_t limbs, bool plain) {
     return c->logN >= 10 && (c->logN <= 12 || (c->logN == 13 && limbs >= 64) || (c->logN == 14 && plain && limbs >= 96));

@@ -317,9 +317,8 @@ struct HoistedArgs {
     RotTermDev t[HOISTED_ARG_TERMS];
     u32 off[HOISTED_ARG_TERMS + 1];
 };
-// Register budget for five waves per SIMD (96 registers): the double-precision form needs 72 (74 on compact keys) and
-// the integer form 93 - 96; the mixed form would take 109 and run at four waves, capped it spills two or three registers
-// and gains a wave.  COMPACT: the key layout of the launch (hoisted.h, key_limb).
+// Register budget for five waves per SIMD (96 registers): the double-precision form needs 70, the integer and the mixed form
+// 94 - 95, none of them spills.  COMPACT: the key layout of the launch (hoisted.h, key_limb).
 #define HOISTED_KERNEL __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void
 template <int MODE, bool COMPACT>
 HOISTED_KERNEL hoisted_terms_kernel(const HoistedArgs args, u64 *__restrict__ y, const ModQ *__restrict__ modq,
@@ -349,11 +348,11 @@ struct LinTermDev {
 // out[o][p][j] = sum_{t in group o} mask_t[j] * ct_t[p][j], p < n_polys (<= 3).  A thread owns the residue pair
 // (n, n+1) of one limb for every polynomial (16-byte accesses; under an automorphism an aligned pair stays an
 // aligned pair, possibly swapped), so each mask residue is read once; integer products are summed as 128-bit
-// values and reduced every 4 terms.  What bounds it is the trip to memory of each term: its loads are the only ones a
-// wavefront has in flight, so nothing may wait between them.  64 terms of 6 limbs over 768 workgroups 199 us with flat loads and a
-// branch on a missing mask between the mask's load and the ciphertext's, 146 us without; 24576 workgroups 445 -> 417 us.
-// Four or eight terms in flight per wavefront: 156 and 151 us, and 472 us on the 24576 workgroups, which lose wavefronts to
-// the registers.
+// values and reduced every 4 terms.  A term's loads are the only ones a wavefront has in flight, so nothing may wait between
+// them: 128 ciphertexts of 6 limbs under one mask (768 workgroups; 805 MB read once) took 199 us with flat loads and a branch on a
+// missing mask between the mask's load and the ciphertext's, and take 146 us without, 5.6 TB/s, the rate of a large copy, which
+// is what bounds it; 24576 workgroups 445 -> 417 us.  Four or eight terms in flight per wavefront: 156 and 151 us, and 472 us on the
+// 24576 workgroups, which lose wavefronts to the registers.
 // ALL_MASKED: no term of the launch is without a mask.  The branch on it keeps the next term's loads behind this one's products
 // (128 masks of their own, 6 limbs of 60 bits: 213 - 220 us with it, 206 without), so only lists that hold such a term pay for it;
 // there the term is an addition (128 of them 138 us; as a product by one, its first polynomial read again in the mask's place, 167).

@@ -507,11 +507,18 @@ void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, c
 // Which passes give a thread eight points instead of sixteen (ntt_device.h, Lanes).  Passes that begin in a basis conversion
 // or a lift, and inverse row passes, always do: they fit four waves per SIMD instead of three resp. eight instead of four.
 // The others only where the launch leaves the chip part empty, since in a full one the second twiddle and address of each
-// pair of lanes is work for nothing (workgroups of 4096 points, 60-bit primes):
-//   columns: 64 workgroups 13.9 -> 13.5 us a forward transform, 15.0 -> 14.1 an inverse one; 384: 25.6 -> 25.5; 768: 31.5 -> 32.5;
-//            6144: 171 -> 180
-//   forward rows: up to the 640 that are resident at once with 87 registers (five waves): 64: 13.9 -> 12.0 us, 384: 25.6 -> 24.3,
-//            672 with the fused tail +5 us (a second round), 6144: 171 -> 179
+// pair of lanes is work for nothing.  Transforms of 2^16 points, us with sixteen / with eight in that pass (workgroups of 4096
+// points); both arithmetics are level between 400 and 1500 workgroups, the lines lie where rows with 87 registers are all resident:
+//   workgroups                  64        256        384        640        768       1024       3072
+//   columns, forward, 60 bits   12.7/11.8  19.6/19.4  26.2/26.3  28.7/29.2  31.8/31.8  38.3/38.0  90.3/93.8
+//                     42 bits    9.6/ 9.4  16.5/16.2  21.6/21.5  23.4/23.6  23.3/22.9  27.3/27.0  70.1/68.4
+//            inverse, 60 bits   13.1/12.3  20.2/19.2  28.0/27.3  31.8/30.7  32.6/31.9  39.5/39.1  92.9/95.4
+//                     42 bits    9.7/ 9.5  16.5/16.1  22.1/21.9  24.0/24.0  23.8/23.7  27.4/28.3  68.2/66.7
+//   forward rows,     60 bits   13.4/11.7  19.6/18.7  26.5/25.4  29.8/27.5  30.0/29.2  35.8/35.4  88.6/91.3
+//                     42 bits   10.1/ 9.4  17.3/15.9  21.9/21.1  23.6/22.6  22.5/23.1  26.2/27.1  68.4/67.3
+//   in a rescale (the fused tail: 110 registers, four waves, with sixteen points, 87 and five with eight; whole rescale)
+//                     60 bits   27.6/25.1  33.6/32.5  42.6/40.7  53.0/50.2  53.7/53.9  61.6/62.6
+//                     42 bits   20.0/18.7  24.8/24.5  31.5/30.4  41.1/37.5  42.5/40.4  46.6/46.2
 // Together, with the conversions: rotation at 24 primes of 60 bits, level 20: 172 -> 162 us, level 7: 100 -> 81; product at level 9
 // 153 -> 134; rotation at N = 2^13 66 -> 53.
 static bool few_for_columns(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 512; }
