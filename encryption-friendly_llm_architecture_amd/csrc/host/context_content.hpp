@@ -100,50 +100,50 @@ struct ContextContent {
         trace_marks.clear();
     }
 
-    // Pinned host memory for the values of one message ([N/2] doubles), which kernels read and write in place: a transfer
-    // needs no copy command and no pageable staging.  At most STAGES of them, kept for the context's life.  A user holds one
-    // from takeStage() to giveStage(); `queued` says that work on `stream` still reads it, which the next user waits for.
+    // Pinned host memory for the values of STAGES messages ([N/2] doubles each), which kernels read and write in place: a
+    // transfer needs no copy command and no pageable staging.  One allocation on first use (it costs what one for a single message
+    // does), kept for the context's life.  A user holds a stage from takeStage() to giveStage(); `queued` says that work on
+    // `stream` still reads it, which the next user waits for: a queue of messages waits for the GPU once it holds STAGES of them.
     struct Stage {
         double *values = nullptr;
         hipEvent_t done = nullptr;
         bool pending = false;
     };
     static constexpr size_t STAGES = 8;
+    double *stage_memory = nullptr;
     std::vector<Stage> stages;          // free ones, the longest unused first
-    size_t stages_made = 0;
     std::condition_variable stage_free;
     Stage takeStage() {
         std::unique_lock<std::mutex> lk(mu);
-        // another one while work that has not run yet reads the longest unused: a queue of messages does not wait for the GPU
-        // before it holds STAGES of them
-        const auto idle = [&] {
-            if (stages.empty()) return false;
-            if (!stages.front().pending) return true;
-            if (hipEventQuery(stages.front().done) == hipSuccess) stages.front().pending = false;
-            else (void)hipGetLastError();   // "not ready" is an answer here, not an error for the next launch to report
-            return !stages.front().pending;
-        };
-        if (stages_made < STAGES && !idle()) {
-            Stage s;
-            if (hipHostMalloc((void **)&s.values, N / 2 * sizeof(double)) != hipSuccess)
-                throw RuntimeException("hipHostMalloc failed");
-            if (hipEventCreateWithFlags(&s.done, hipEventDisableTiming) != hipSuccess) {
-                (void)hipHostFree(s.values);
-                throw RuntimeException("hipEventCreateWithFlags failed");
+        if (stage_memory == nullptr) {
+            std::vector<Stage> made(STAGES);
+            bool ok = hipHostMalloc((void **)&stage_memory, STAGES * (N / 2) * sizeof(double)) == hipSuccess;
+            for (size_t i = 0; ok && i < STAGES; i++) {
+                made[i].values = stage_memory + i * (N / 2);
+                ok = hipEventCreateWithFlags(&made[i].done, hipEventDisableTiming) == hipSuccess;
             }
-            stages_made++;
-            return s;
+            if (!ok) {
+                for (Stage &s : made)
+                    if (s.done) (void)hipEventDestroy(s.done);
+                if (stage_memory) (void)hipHostFree(stage_memory);
+                stage_memory = nullptr;
+                throw RuntimeException("no pinned memory for the values of messages");
+            }
+            stages = std::move(made);
         }
         stage_free.wait(lk, [&] { return !stages.empty(); });
         Stage s = stages.front();
         stages.erase(stages.begin());
         lk.unlock();
-        if (s.pending) (void)hipEventSynchronize(s.done);
+        if (s.pending && hipEventQuery(s.done) != hipSuccess) {   // (a query of one long since reached is cheaper than a wait)
+            (void)hipGetLastError();   // "not ready" is an answer here, not an error for the next launch to report
+            (void)hipEventSynchronize(s.done);
+        }
         s.pending = false;
         return s;
     }
     void giveStage(Stage s, bool queued) {
-        if (queued) s.pending = hipEventRecord(s.done, stream()) == hipSuccess;
+        if (queued && !(s.pending = hipEventRecord(s.done, stream()) == hipSuccess)) (void)hipStreamSynchronize(stream());
         {
             std::lock_guard<std::mutex> lk(mu);
             stages.push_back(s);
@@ -188,10 +188,8 @@ struct ContextContent {
         for (auto &kv : pool) (void)hipFree(kv.second);
         for (auto &kv : parked) (void)hipFree(kv.second);
         for (auto &kv : captured) (void)hipFree(kv.second);
-        for (auto &st : stages) {
-            (void)hipEventDestroy(st.done);
-            (void)hipHostFree(st.values);
-        }
+        for (auto &st : stages) (void)hipEventDestroy(st.done);
+        if (stage_memory) (void)hipHostFree(stage_memory);
         if (side) (void)hipStreamDestroy(side);
         if (ev_fork) (void)hipEventDestroy(ev_fork);
         if (ev_join) (void)hipEventDestroy(ev_join);
