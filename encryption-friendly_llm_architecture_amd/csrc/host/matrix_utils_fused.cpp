@@ -1435,18 +1435,18 @@ void hoistedShifts(const HomEvaluator &eval, const Sources &x, const Sources &x2
     // longer term lists are staged from pageable memory, which waits for the stream: no second stream for them
     const bool two = n > whole && whole >= 2 && whole <= 32;
     const size_t G = two ? whole / 2 : whole;
-    const hipStream_t side = two ? c->forkSide() : nullptr;
-    struct JoinOnExit {
-        const Context &c;
-        ~JoinOnExit() { c->joinSide(); }   // also when a launch below throws
-    };
     std::vector<Ciphertext> results(n, Ciphertext(c));
     std::vector<uint64_t *> outs;
     for (Ciphertext &r : results) {
         r.allocate(2, T + 1, 0);
         outs.push_back(r.buf_.data());
     }
+    struct JoinOnExit {
+        const Context &c;
+        ~JoinOnExit() { c->joinSide(); }   // also when a launch below throws
+    };
     {
+        const hipStream_t side = two ? c->forkSide() : nullptr;
         JoinOnExit join_on_exit{c};
         DeviceBuffer y[2], ws[2];
         size_t chain = 0;
