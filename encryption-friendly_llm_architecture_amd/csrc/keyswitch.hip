@@ -349,9 +349,9 @@ struct LinTermDev {
 // (n, n+1) of one limb for every polynomial (16-byte accesses; under an automorphism an aligned pair stays an
 // aligned pair, possibly swapped), so each mask residue is read once; integer products are summed as 128-bit
 // values and reduced every 4 terms.  A term's loads are the only ones a wavefront has in flight, so nothing may wait between
-// them: 128 ciphertexts of 6 limbs under one mask (768 workgroups; 805 MB read once) took 199 us with flat loads and a branch on a
-// missing mask between the mask's load and the ciphertext's, and take 146 us without, 5.6 TB/s, the rate of a large copy, which
-// is what bounds it; 24576 workgroups 445 -> 417 us.  Four or eight terms in flight per wavefront: 156 and 151 us, and 472 us on the
+// them: 128 ciphertexts of 6 limbs under one mask (768 workgroups; 805 MB read once) took 199 us with a branch on a missing mask
+// between the mask's load and the ciphertext's (flat or global loads alike), and take 146 us without, 5.6 TB/s, the rate of a large
+// copy, which is what bounds it; 24576 workgroups 445 -> 417 us.  Four or eight terms in flight per wavefront: 156 and 151 us, and 472 us on the
 // 24576 workgroups, which lose wavefronts to the registers.
 // ALL_MASKED: no term of the launch is without a mask.  The branch on it keeps the next term's loads behind this one's products
 // (128 masks of their own, 6 limbs of 60 bits: 213 - 220 us with it, 206 without), so only lists that hold such a term pay for it;
