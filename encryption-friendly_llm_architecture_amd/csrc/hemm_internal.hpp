@@ -134,7 +134,7 @@ bool launch_ntt_sub_scale(const hemm_context *c, u64 *data, int n_limbs, int n_p
 struct ConvSources {
     struct Digit {
         const u64 *src;             // coefficient form, [n_polys][.][N]
-        const Cst *hat;             // [n_src][hat_ld]  (S/q_i) mod prime, indexed by prime
+        const Cst *hat;             // [n_src][hat_ld]  (S/q_i) mod prime and 2^30 times that, indexed by prime
         size_t src_poly_stride;
         int n_src;
         uint8_t src_slot[CONV_MAX_SOURCES];
@@ -189,7 +189,7 @@ void launch_decode(const hemm_context *c, const u64 *pt, const u64 *a, const u64
 // out[p][j] = (y[p][j] - conversion of the n_src listed limbs of y[p] to prime j) * cst[j], j < nq_out, as inverse row
 // pass (in place on the listed limbs), one column-slab kernel (second inverse pass, conversion as lazy dot products, first
 // forward pass into conv[n_polys][nq_out][N]) and forward row pass with the fused tail.  final_scale / hat / cst: device
-// tables in source order, [n_src][hat_ld] by prime, by target limb.  false when the shape has no such form.
+// tables in source order, [n_src][hat_ld] by prime (as in ConvSources), by target limb.  false when the shape has no such form.
 bool launch_moddown_slab(const hemm_context *c, u64 *y, size_t y_stride, const uint8_t *src_slot, const uint8_t *src_prime,
                          int n_src, const void *final_scale_dev, const void *hat_dev, int hat_ld, u64 *conv, int nq_out,
                          int n_polys, u64 *out, size_t out_stride, const void *cst_dev, hipStream_t s);

@@ -22,6 +22,7 @@ struct BConvArgs {
     size_t src_poly_stride, dst_poly_stride;
     const Cst *inv;        // [n_src]  (S/q_i)^-1 mod q_i
     const Cst *hat;        // [n_src][hat_ld]  (S/q_i) mod prime, indexed by prime
+    const Cst *dot;        // ... and 2^30 times that in place of the Shoup quotient (modarith.h, DotCst)
     int n_src, n_dst, hat_ld, logN;
     int pre_scaled;        // the source residues already carry their (S/q_i)^-1 factor (folded into the inverse transform)
     int split;             // register kernels: the target limbs are dealt to this many workgroups per coefficient block
@@ -58,7 +59,7 @@ __global__ __launch_bounds__(256) void bconv_kernel(BConvArgs a, const ModQ *__r
 
 // Register form of the same conversion for up to 8 source limbs and primes below 2^60: a thread owns two adjacent
 // coefficients (16-byte accesses), keeps the scaled source residues in registers and takes every target residue as a
-// lazy dot product (four 32-bit multiply-adds per term) with one reduction at the end.
+// lazy dot product (four multiply-adds per term) with one reduction at the end.
 template <int NS>
 __global__ __launch_bounds__(256) void bconv_reg_kernel(BConvArgs a, const ModQ *__restrict__ modq) {
     const int S = a.split > 1 ? a.split : 1;
@@ -79,16 +80,17 @@ __global__ __launch_bounds__(256) void bconv_reg_kernel(BConvArgs a, const ModQ 
     for (int j = j_lo; j < j_hi; j++) {
         const int pj = a.dst_prime[j];
         const ModQ m = modq[pj];
-        Dot3 d0, d1;
-        dot3_clear(d0);
-        dot3_clear(d1);
+        Dot2 d0, d1;
+        dot_clear(d0);
+        dot_clear(d1);
 #pragma unroll
         for (int i = 0; i < NS; i++) {
-            const u64 h = a.hat[i * a.hat_ld + pj].w;
-            dot3_add(d0, v0[i], h);
-            dot3_add(d1, v1[i], h);
+            const Cst hg = a.dot[i * a.hat_ld + pj];
+            const DotCst h = dot_cst(hg.w, hg.ws);
+            dot_add(d0, v0[i], h);
+            dot_add(d1, v1[i], h);
         }
-        *(ulonglong2 *)(dst + ((size_t)a.dst_slot[j] << a.logN) + n) = make_ulonglong2(dot3_reduce(d0, m), dot3_reduce(d1, m));
+        *(ulonglong2 *)(dst + ((size_t)a.dst_slot[j] << a.logN) + n) = make_ulonglong2(dot_reduce(d0, m), dot_reduce(d1, m));
     }
 }
 
@@ -125,18 +127,19 @@ __global__ __launch_bounds__(256) void bconv_digits_kernel(BConvDigits g, const 
     for (int j = j_lo; j < j_hi; j++) {
         const int pj = a.dst_prime[j];
         const ModQ m = modq[pj];
-        Dot3 d0, d1;
-        dot3_clear(d0);
-        dot3_clear(d1);
+        Dot2 d0, d1;
+        dot_clear(d0);
+        dot_clear(d1);
 #pragma unroll
         for (int i = 0; i < NS; i++) {
             if (i < a.n_src) {
-                const u64 h = a.hat[i * a.hat_ld + pj].w;
-                dot3_add(d0, v0[i], h);
-                dot3_add(d1, v1[i], h);
+                const Cst hg = a.dot[i * a.hat_ld + pj];
+                const DotCst h = dot_cst(hg.w, hg.ws);
+                dot_add(d0, v0[i], h);
+                dot_add(d1, v1[i], h);
             }
         }
-        *(ulonglong2 *)(dst + ((size_t)a.dst_slot[j] << a.logN) + n) = make_ulonglong2(dot3_reduce(d0, m), dot3_reduce(d1, m));
+        *(ulonglong2 *)(dst + ((size_t)a.dst_slot[j] << a.logN) + n) = make_ulonglong2(dot_reduce(d0, m), dot_reduce(d1, m));
     }
     const u64 *own = g.own + poly * g.own_stride;
     for (int j = g.own_lo[blockIdx.z] + part; j < g.own_hi[blockIdx.z]; j += S)
@@ -592,6 +595,7 @@ __global__ __launch_bounds__(256) void tensor_groups_kernel(TensorGroups gr, siz
 struct KsTables {
     std::vector<Cst> host;
     Cst *dev = nullptr;
+    const Cst *dot = nullptr;                            // the hat entries (and `ones`) at the same offsets as (w, 2^30 w mod q)
     std::vector<std::vector<size_t>> inv_off, hat_off;  // [nq][d]
     size_t p_inv_off = 0, p_hat_off = 0;
     std::vector<Cst> pinv;                               // P^-1 mod q_j
@@ -613,6 +617,12 @@ static KsTables *g_tables_of(const hemm_context *c);
 
 static void build_tables(const hemm_context *c, KsTables &t) {
     const int nQ = c->nQ, K = c->nP, T = nQ + K, alpha = c->alpha;
+    std::vector<Cst> dot;
+    auto dot_entry = [&](const size_t at, const int prime) {
+        const u64 w = t.host[at].w, q = c->primes[prime];
+        if (dot.size() <= at) dot.resize(at + 1, Cst{0, 0});
+        dot[at] = Cst{w, h_mulmod(w, (1ull << 30) % q, q)};
+    };
     auto push_basis = [&](const std::vector<int> &src, size_t &inv_off, size_t &hat_off) {
         inv_off = t.host.size();
         for (size_t i = 0; i < src.size(); i++) {
@@ -629,6 +639,7 @@ static void build_tables(const hemm_context *c, KsTables &t) {
                 for (size_t k = 0; k < src.size(); k++)
                     if (k != i) prod = h_mulmod(prod, c->primes[src[k]] % tq, tq);
                 t.host.push_back(Cst{prod, shoup_h(prod, tq)});
+                dot_entry(t.host.size() - 1, pj);
             }
     };
     t.inv_off.assign(nQ + 1, {});
@@ -725,8 +736,13 @@ static void build_tables(const hemm_context *c, KsTables &t) {
     }
     t.ones_off = t.host.size();
     for (int pj = 0; pj < T; pj++) t.host.push_back(Cst{1, 0});
-    HEMM_HIP(hipMalloc((void **)&t.dev, t.host.size() * sizeof(Cst)));
-    HEMM_HIP(hipMemcpy(t.dev, t.host.data(), t.host.size() * sizeof(Cst), hipMemcpyHostToDevice));
+    for (int pj = 0; pj < T; pj++) dot_entry(t.ones_off + pj, pj);
+    const size_t n = t.host.size();
+    dot.resize(n, Cst{0, 0});
+    HEMM_HIP(hipMalloc((void **)&t.dev, 2 * n * sizeof(Cst)));
+    HEMM_HIP(hipMemcpy(t.dev, t.host.data(), n * sizeof(Cst), hipMemcpyHostToDevice));
+    HEMM_HIP(hipMemcpy(t.dev + n, dot.data(), n * sizeof(Cst), hipMemcpyHostToDevice));
+    t.dot = t.dev + n;
 }
 
 // tables live beside the context (created on first use, destroyed with it)
@@ -793,6 +809,7 @@ void launch_modup(hemm_context *c, const u64 *in, int nq, u64 *ext, u64 *coef, b
         a.dst = ext + (size_t)d * E * N;
         a.inv = t->dev + t->inv_off[nq][d];
         a.hat = t->dev + t->hat_off[nq][d];
+        a.dot = t->dot + t->hat_off[nq][d];
         a.n_src = hi - lo;
         a.hat_ld = c->nQ + c->nP;
         a.logN = c->logN;
@@ -857,6 +874,7 @@ void launch_moddown(hemm_context *c, u64 *acc, int nq, int n_polys, u64 *out, si
     a.dst_poly_stride = (size_t)nq * N;
     a.inv = t->dev + t->p_inv_off;
     a.hat = t->dev + t->p_hat_off;
+    a.dot = t->dot + t->p_hat_off;
     a.n_src = K;
     a.n_dst = nq;
     a.hat_ld = c->nQ + c->nP;
@@ -964,7 +982,7 @@ static void rescale_with(hemm_context *c, KsTables *t, u64 *sc, const u64 *in, s
         ConvSources cs;
         memset(&cs, 0, sizeof(cs));
         cs.d[0].src = last;
-        cs.d[0].hat = t->dev + t->ones_off;
+        cs.d[0].hat = t->dot + t->ones_off;
         cs.d[0].src_poly_stride = N;
         cs.d[0].n_src = 1;
         cs.hat_ld = c->nQ + c->nP;
@@ -1154,6 +1172,7 @@ void launch_modup_batch(hemm_context *c, const u64 *in, size_t in_stride, int nq
         a.dst_poly_stride = (size_t)beta * E * N;
         a.inv = t->dev + t->inv_off[nq][d];
         a.hat = t->dev + t->hat_off[nq][d];
+        a.dot = t->dot + t->hat_off[nq][d];
         a.n_src = hi - lo;
         a.hat_ld = c->nQ + c->nP;
         a.logN = c->logN;
@@ -1203,7 +1222,7 @@ void launch_modup_batch(hemm_context *c, const u64 *in, size_t in_stride, int nq
         int l = 0;
         for (int d = 0; d < beta; d++) {
             cs.d[d].src = g.d[d].src;
-            cs.d[d].hat = g.d[d].hat;
+            cs.d[d].hat = g.d[d].dot;
             cs.d[d].src_poly_stride = g.d[d].src_poly_stride;
             cs.d[d].n_src = g.d[d].n_src;
             for (int i = 0; i < g.d[d].n_src; i++) cs.d[d].src_slot[i] = g.d[d].src_slot[i];
@@ -1428,7 +1447,7 @@ void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop
     if (slab) {
         if (!launch_moddown_slab(c, y, (size_t)E * N, a.src_slot, a.src_prime, ns,
                             t->dev + (drop_last ? t->drop_invn_off[nq] : t->p_invn_off),
-                            t->dev + (drop_last ? t->drop_hat_off[nq] : t->p_hat_off), c->nQ + c->nP, conv, nq_out, n_polys,
+                            t->dot + (drop_last ? t->drop_hat_off[nq] : t->p_hat_off), c->nQ + c->nP, conv, nq_out, n_polys,
                             out, out_stride, t->dev + (drop_last ? t->dropinv_off[nq] : t->pinv_off), s))
             throw std::invalid_argument("the column-slab ModDown takes 4 or 5 dropped limbs");
         return;
@@ -1442,6 +1461,7 @@ void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop
     a.dst_poly_stride = (size_t)nq_out * N;
     a.inv = t->dev + (drop_last ? t->drop_inv_off[nq] : t->p_inv_off);
     a.hat = t->dev + (drop_last ? t->drop_hat_off[nq] : t->p_hat_off);
+    a.dot = t->dot + (drop_last ? t->drop_hat_off[nq] : t->p_hat_off);
     a.n_src = ns;
     a.n_dst = nq_out;
     a.hat_ld = c->nQ + c->nP;
@@ -1457,7 +1477,7 @@ void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop
         ConvSources cs;
         memset(&cs, 0, sizeof(cs));
         cs.d[0].src = y;
-        cs.d[0].hat = a.hat;
+        cs.d[0].hat = a.dot;
         cs.d[0].src_poly_stride = a.src_poly_stride;
         cs.d[0].n_src = ns;
         for (int i = 0; i < ns; i++) cs.d[0].src_slot[i] = a.src_slot[i];

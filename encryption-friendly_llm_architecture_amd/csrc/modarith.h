@@ -35,9 +35,8 @@ struct ModQ {
     u64 q;     // the prime
     u64 mu;    // floor(2^(2k) / q), k = bit length of q
     u32 k;     // bit length of q (q < 2^k, k <= 61)
-    u32 pad;
+    u32 mdot;  // floor(2^(k+31) / q) (dot_reduce_lazy)
     u64 mu3;   // floor(2^(2k+3) / q) for k = 59 or 60, else 0 (barrett_tight)
-    u64 r64;   // 2^64 mod q
 };
 
 // x * w mod q for a constant w with ws = floor(w * 2^64 / q); result in [0, 2q).
@@ -109,44 +108,45 @@ __device__ __forceinline__ u64 reduce64(u64 a, const ModQ &m) {
     t.hi = 0;
     return barrett128(t, m);
 }
-// Lazy dot product sum_i v_i * h_i of up to 8 residues v_i < 2^60 with constants h_i < 2^60 (a target residue of a
-// fast basis conversion).  The 32-bit halves are multiplied into three 64-bit accumulators -- s0 (weight 1, with a
-// carry count), s1 (weight 2^32: 16 terms below 2^60 cannot overflow), s2 (weight 2^64) -- four multiply-adds per
-// term and no reduction until the end, against a Shoup product with its own quotient per term.
-struct Dot3 {
-    u64 s0, s1, s2;
-    u32 c;
+// Lazy dot product sum_i v_i * h_i of up to 8 residues v_i < 2^60 with constants h_i < 2^60 (a target residue of a fast basis
+// conversion).  With v = v0 + 2^30 v1 and g = 2^30 h mod q kept beside h, the term is v0 h + v1 g: products of 30-bit
+// pieces of v with 30-bit pieces of h and g, four multiply-adds into two 64-bit accumulators of weights 1 and 2^30 that 16
+// products below 2^60 cannot overflow -- no carries, and a sum 34 bits longer than q instead of 64 to reduce.
+struct DotCst {
+    u32 h0, h1, g0, g1;
 };
-__device__ __forceinline__ void dot3_clear(Dot3 &d) {
-    d.s0 = d.s1 = d.s2 = 0;
-    d.c = 0;
+__device__ __forceinline__ DotCst dot_cst(const u64 h, const u64 g) {
+    return DotCst{(u32)h & 0x3fffffffu, (u32)(h >> 30), (u32)g & 0x3fffffffu, (u32)(g >> 30)};
 }
-__device__ __forceinline__ void dot3_add(Dot3 &d, const u64 v, const u64 h) {
-    const u32 vl = (u32)v, vh = (u32)(v >> 32), hl = (u32)h, hh = (u32)(h >> 32);
-    const u64 p = (u64)vl * hl;
-    d.s0 += p;
-    d.c += d.s0 < p ? 1u : 0u;
-    d.s1 += (u64)vl * hh;
-    d.s1 += (u64)vh * hl;
-    d.s2 += (u64)vh * hh;
+struct Dot2 {
+    u64 s0, s1;
+};
+__device__ __forceinline__ void dot_clear(Dot2 &d) { d.s0 = d.s1 = 0; }
+__device__ __forceinline__ void dot_add(Dot2 &d, const u64 v, const DotCst &c) {
+    const u32 v0 = (u32)v & 0x3fffffffu, v1 = (u32)(v >> 30);
+    d.s0 += (u64)v0 * c.h0;
+    d.s0 += (u64)v1 * c.g0;
+    d.s1 += (u64)v0 * c.h1;
+    d.s1 += (u64)v1 * c.g1;
 }
-// the sum as a 128-bit value (below 8 * 2^(60 + k) for constants below 2^k)
-__device__ __forceinline__ u128_t dot3_value(const Dot3 &d) {
+// the sum as a 128-bit value, below 2^(k + 34) for constants below 2^k
+__device__ __forceinline__ u128_t dot_value(const Dot2 &d) {
     u128_t t;
-    const u64 mid = d.s1 << 32;
-    t.lo = d.s0 + mid;
-    t.hi = d.s2 + d.c + (d.s1 >> 32) + (t.lo < mid ? 1ull : 0ull);
+    t.lo = d.s0 + (d.s1 << 30);
+    t.hi = (d.s1 >> 34) + (t.lo < d.s0 ? 1ull : 0ull);
     return t;
 }
-// ... reduced to [0, q): the high word (below 2^(k-1)) is folded with 2^64 mod q, which leaves a value below
-// 2^(2k-1) + 2^64 < 6 * 2^(2k) for k >= 31, then one Barrett step
-__device__ __forceinline__ u64 dot3_reduce(const Dot3 &d, const ModQ &m) {
-    const u128_t t = dot3_value(d);
-    u128_t u = mul64wide(t.hi, m.r64);
-    const u64 lo = u.lo + t.lo;
-    u.hi += lo < t.lo ? 1ull : 0ull;
-    u.lo = lo;
-    return barrett128(u, m);
+// ... reduced to [0, q): k >= 32 (primes of 2^31 and more), so it lies below 6 * 2^(2k)
+__device__ __forceinline__ u64 dot_reduce(const Dot2 &d, const ModQ &m) { return barrett3(dot_value(d), m); }
+// ... to [0, 13q), for butterflies that take values below 16q (q < 2^60).  The sum is below 16 * 2^30 q, so that t = sum / 2^(k+2)
+// fits 32 bits and t * (2^(k+31) / q) / 2^29 misses the quotient by less than 2^(k+2) / q for the cut of the sum, t / 2^29 for the
+// cut of the constant and 1: 4 + 8 + 1 for q near 2^k, 8 + 4 + 1 for q near 2^(k-1).
+__device__ __forceinline__ u64 dot_reduce_lazy(const Dot2 &d, const ModQ &m) {
+    const u32 t = (u32)((d.s1 + (d.s0 >> 30)) >> (m.k - 28));
+    const u64 qhat = ((u64)t * m.mdot) >> 29, nq = 0 - m.q;
+    const u32 hl = (u32)qhat, hh = (u32)(qhat >> 32), nl = (u32)nq, nh = (u32)(nq >> 32);
+    const u64 r = (u64)hl * nl + (d.s0 + (d.s1 << 30));
+    return r + ((u64)(hl * nh + hh * nl) << 32);
 }
 __device__ __forceinline__ u64 addmod(u64 a, u64 b, u64 q) {
     u64 s = a + b;

@@ -183,7 +183,7 @@ __global__ __launch_bounds__(4096 / P) void ntt16_cols_kernel(u64 *__restrict__ 
 template <int LR, int NS, class F>
 __device__ __forceinline__ void cols_converted_body(const __amdgpu_buffer_rsrc_t limb, const Tw *__restrict__ tw_int,
                                                     const F f, u64 *lds_raw, const __amdgpu_buffer_rsrc_t src,
-                                                    const u32 (&so)[NS], const u64 (&h)[NS], const int n_src, const ModQ m) {
+                                                    const u32 (&so)[NS], const DotCst (&h)[NS], const int n_src, const ModQ m) {
     typedef Slab<LR, 8> S;
     typename F::E x[8];
     // the row step goes into the scalar offset
@@ -191,10 +191,13 @@ __device__ __forceinline__ void cols_converted_body(const __amdgpu_buffer_rsrc_t
     cols_forward<LR>(limb, (const typename F::W *)tw_int, f, x, (typename F::E *)lds_raw);
 }
 
-// Eight points per thread: 96 - 108 registers, four waves per SIMD (sixteen points: 154 - 166, three waves).  1200 workgroups
-// (24 primes of 60 bits, level 20) 38 -> 35 us, 64 polynomials x 6 limbs 2 % less of the whole projection.
+// What bounds it is the work of a column pass and the trips to memory in front of it.  Eight points per thread and 20 source
+// residues in flight fit 80 registers, six waves per SIMD (sixteen points: 154 - 166 registers, three waves; 40 residues: four).  1536
+// workgroups (16 polynomials x 6 limbs, 5 sources) 42 -> 37 us alone, 1002 -> 789 vector instructions per wave, with sums that carry
+// nothing (modarith.h, DotCst) and loads that wait once; rotation at 24 primes of 60 bits, level 20 161 -> 154 us, projection of a
+// 768-wide layer 2.5 % less.
 template <int LR, int NS>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void ntt16_cols_converted_kernel(
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) void ntt16_cols_converted_kernel(
     u64 *__restrict__ data, const Tw *__restrict__ tw_all, const ModQ *__restrict__ modq, const u64 *__restrict__ ninv,
     const u64 *__restrict__ ninv_s, const double *__restrict__ fp, LimbList ll, LimbList sl, int n_limbs,
     size_t poly_stride, ConvSources cs) {
@@ -225,24 +228,23 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const Tw *tw = tw_all + ((size_t)prime << (8 + LR));
     const int dg = __builtin_amdgcn_readfirstlane((int)cs.digit_of[limb]), n_src = cs.d[dg].n_src;
     // The sources are read through a buffer resource: base (the polynomial's source limbs; far below 4 GiB), source slot
-    // and slab row sit in scalar registers, a thread supplies one 32-bit offset for all of its 16 n_src loads.
+    // and slab row sit in scalar registers, a thread supplies one 32-bit offset for all of its 8 n_src loads.
     const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(cs.d[dg].src + (size_t)poly * cs.d[dg].src_poly_stride), 0, -1, 0x00020000);
     const Cst *hat = cs.d[dg].hat + prime;
     const ModQ m = modq[prime];
     u32 so[NS];
-    u64 h[NS];
+    DotCst h[NS];
 #pragma unroll
     for (int i = 0; i < NS; i++) {
         const int ii = i < n_src ? i : 0;
         so[i] = __builtin_amdgcn_readfirstlane((u32)cs.d[dg].src_slot[ii]) << (11 + LR);
-        h[i] = hat[(size_t)ii * cs.hat_ld].w;
+        const Cst hg = hat[(size_t)ii * cs.hat_ld];
+        h[i] = dot_cst(hg.w, hg.ws);
     }
     if (fp[4 * prime] != 0.0)
         cols_converted_body<LR, NS>(base, tw, FpField(modq, ninv, ninv_s, fp, prime), lds, src, so, h, n_src, m);
-    else if ((m.q >> 60) != 0)
-        cols_converted_body<LR, NS>(base, tw, IntField(modq, ninv, ninv_s, fp, prime), lds, src, so, h, n_src, m);
-    else
+    else   // (the sums take primes below 2^60)
         cols_converted_body<LR, NS>(base, tw, IntFieldT<true>(modq, ninv, ninv_s, fp, prime), lds, src, so, h, n_src, m);
 }
 
@@ -293,7 +295,7 @@ __global__ __launch_bounds__(512) void ntt16_cols_lifted_kernel(u64 *__restrict_
 struct SlabSources {
     const u64 *src;            // first-pass output of the inverse transform (raw field values), [n_polys][.][N]
     size_t src_poly_stride;
-    const Cst *hat;            // [n_src][hat_ld]  (S/q_i) mod prime, indexed by prime
+    const Cst *hat;            // [n_src][hat_ld]  (S/q_i) mod prime and 2^30 times that, indexed by prime
     const Tw *final_scale;     // [n_src]  (1/N)(S/q_i)^-1 mod q_i
     int hat_ld, n_src, n_dst;
     uint8_t src_slot[SLAB_REG_SOURCES + 1], src_prime[SLAB_REG_SOURCES + 1];
@@ -326,8 +328,8 @@ __device__ __forceinline__ void slab_inverse(const __amdgpu_buffer_rsrc_t limb, 
 template <int NREG, bool LDS, class F>
 __device__ __forceinline__ void slab_forward(const __amdgpu_buffer_rsrc_t limb, const u32 v_inner,
                                              const Tw *__restrict__ tw_int, const F f, u64 *lds_raw,
-                                             const u64 *__restrict__ lsrc, const u64 hl,
-                                             const u64 (&c)[SLAB_REG_SOURCES][16], const u64 (&h)[SLAB_REG_SOURCES],
+                                             const u64 *__restrict__ lsrc, const DotCst &hl,
+                                             const u64 (&c)[SLAB_REG_SOURCES][16], const DotCst (&h)[SLAB_REG_SOURCES],
                                              const ModQ m) {
     typedef typename F::E E;
     const typename F::W *tw = (const typename F::W *)tw_int;
@@ -336,11 +338,11 @@ __device__ __forceinline__ void slab_forward(const __amdgpu_buffer_rsrc_t limb, 
     E x[16];
 #pragma unroll
     for (int k = 0; k < 16; k++) {
-        Dot3 d;
-        dot3_clear(d);
-        if (LDS) dot3_add(d, lsrc[k * 256 + threadIdx.x], hl);
+        Dot2 d;
+        dot_clear(d);
+        if (LDS) dot_add(d, lsrc[k * 256 + threadIdx.x], hl);
 #pragma unroll
-        for (int j = SLAB_REG_SOURCES - NREG; j < SLAB_REG_SOURCES; j++) dot3_add(d, c[j][k], h[j]);
+        for (int j = SLAB_REG_SOURCES - NREG; j < SLAB_REG_SOURCES; j++) dot_add(d, c[j][k], h[j]);
         x[k] = f.from_dot(d, m);
     }
     radix_fwd<4>(f, x, tw, 1u);
@@ -411,13 +413,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         const Tw *tw = tw_all + ((size_t)prime << 16);
         const ModQ m = modq[prime];
         const Cst *hat = ss.hat + prime;
-        u64 h[SLAB_REG_SOURCES];
+        DotCst h[SLAB_REG_SOURCES];
 #pragma unroll
         for (int j = 0; j < SLAB_REG_SOURCES; j++) {
             const int i = n_lds + j - first_reg;
-            h[j] = j >= first_reg ? hat[(size_t)i * ss.hat_ld].w : 0;
+            const Cst hg = j >= first_reg ? hat[(size_t)i * ss.hat_ld] : Cst{0, 0};
+            h[j] = dot_cst(hg.w, hg.ws);
         }
-        const u64 hl = LDS ? hat[0].w : 0;
+        const DotCst hl = dot_cst(LDS ? hat[0].w : 0, LDS ? hat[0].ws : 0);
         if (fp[4 * prime] != 0.0)
             slab_forward<NREG, LDS>(limb, v_inner, tw, FpField(modq, ninv, ninv_s, fp, prime), lds, lsrc, hl, c, h, m);
         else

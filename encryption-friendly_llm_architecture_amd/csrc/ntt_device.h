@@ -122,7 +122,8 @@ struct IntFieldT {
         nis = ninv_s != nullptr ? ninv_s[prime] : 0;
     }
     __device__ __forceinline__ E from_canonical(u64 v) const { return v; }
-    __device__ __forceinline__ E from_dot(const Dot3 &d, const ModQ &m) const { return dot3_reduce(d, m); }
+    // < 13q: primes below 2^60 only, whose butterflies take inputs below 16q
+    __device__ __forceinline__ E from_dot(const Dot2 &d, const ModQ &m) const { return dot_reduce_lazy(d, m); }
     // odd: the stage's index within its radix-16 block is odd
     __device__ __forceinline__ void ct(E &x, E &y, const W tw, const bool odd) const {
         if (!LAZY16) {
@@ -175,16 +176,12 @@ struct FpField {
     __device__ __forceinline__ E from_canonical(u64 v) const {
         return __longlong_as_double((long long)(v | 0x4330000000000000ull)) - 4503599627370496.0;
     }
-    // A lazy dot product (three accumulators of weights 1, 2^32, 2^64 and a carry count of weight 2^64) as a residue of
-    // magnitude below q: regrouped into pieces of weights 1, 2^32, 2^64 below 2^32, 2^33 and 2^45 (constants below
-    // 2^44, residues below 2^60, 8 terms), each exact in a double; the two upper ones are multiplied by 2^32 and 2^64
-    // mod q.  No integer reduction and no conversion from canonical form.
-    __device__ __forceinline__ E from_dot(const Dot3 &d, const ModQ &) const {
-        const u64 p1 = (d.s0 >> 32) + (d.s1 & 0xffffffffull), p2 = (d.s1 >> 32) + d.s2 + d.c;
-        const double r32 = reduce(4294967296.0), r64 = reduce(18446744073709551616.0);
-        const double a = (double)(u32)d.s0 + mulmod(from_canonical(p1), r32, r32 * qinv) +
-                         mulmod(from_canonical(p2), r64, r64 * qinv);
-        return reduce(a);
+    // A lazy dot product as a residue of magnitude below 1.3 q: regrouped into pieces of weights 1 and 2^30, below 2^30 and 2^49
+    // (constants below 2^44), both exact in a double; the upper one is multiplied by 2^30 (below q, as every prime is).  No
+    // integer reduction and no conversion from canonical form; a forward transform then ends below 11 q as from canonical residues.
+    __device__ __forceinline__ E from_dot(const Dot2 &d, const ModQ &) const {
+        const u64 p1 = (d.s0 >> 30) + d.s1;
+        return (double)((u32)d.s0 & 0x3fffffffu) + mulmod(from_canonical(p1), 1073741824.0, 1073741824.0 * qinv);
     }
     __device__ __forceinline__ void ct(E &x, E &y, const W tw, const bool) const {
         const double v = mulmod(y, tw, tw * qinv);
@@ -352,36 +349,41 @@ __device__ __forceinline__ u64 lifted(const LiftSource &ls, const long long *__r
     const int e = sample_error(ls.error_key, n);
     return addmod(r, e >= 0 ? (u64)e : m.q - (u64)(-e), m.q);
 }
-// The P coefficients of a thread as a basis conversion computed on the fly: coefficient k is sum_i v_i * hat_i mod q
-// over the n_src <= NS source limbs (pre-scaled, the same lazy sums and reductions as the stand-alone conversion kernels,
-// so the residues are the same), read at voff + off(k) inside a limb; so[i]: byte offset of source limb i.
-template <int NS, int P, class F, class OFF>
-__device__ __forceinline__ void converted_inputs(const F &f, typename F::E (&x)[P], const __amdgpu_buffer_rsrc_t src,
-                                                 const u32 voff, const u32 (&so)[NS], const u64 (&h)[NS], const int n_src,
-                                                 const ModQ m, const OFF off) {
-    // eight coefficients at a time (three accumulators each), source by source, so that the eight loads of one source
-    // limb are in flight together
+// The eight coefficients of a thread as a basis conversion computed on the fly: coefficient k is sum_i v_i * hat_i mod q over
+// the n_src <= NS source limbs (pre-scaled, the same sums as the stand-alone conversion kernels), read at voff + off(k) inside a
+// limb; so[i]: byte offset of source limb i.
+// The loads of the next coefficients, about CONV_LOADS residues, are in flight while the present one's products are taken: one
+// wait for the first of them instead of one per source limb behind a branch of its own.  More in flight cost wavefronts: ModDown
+// of 64 / 16 polynomials of 7 + 4 limbs 389 / 108 us with 20 residues and six waves per SIMD, 400 / 110 with 40 and four.
+#define CONV_LOADS 20
+template <int N_SRC, int NS, class F, class OFF>
+__device__ __forceinline__ void converted_exact(const F &f, typename F::E (&x)[8], const __amdgpu_buffer_rsrc_t src, const u32 voff,
+                                                const u32 (&so)[NS], const DotCst (&h)[NS], const ModQ m, const OFF off) {
+    constexpr int AHEAD = CONV_LOADS / N_SRC < 8 ? CONV_LOADS / N_SRC : 8;   // coefficients whose sources are in flight together
+    u32x2 v[8][N_SRC];
+    auto load = [&](const int k) {
 #pragma unroll
-    for (int half = 0; half < P / 8; half++) {
-        Dot3 d[8];
+        for (int i = 0; i < N_SRC; i++) v[k][i] = __builtin_amdgcn_raw_buffer_load_b64(src, voff, so[i] + off(k), 0);
+    };
 #pragma unroll
-        for (int k = 0; k < 8; k++) dot3_clear(d[k]);
+    for (int k = 0; k < AHEAD; k++) load(k);
 #pragma unroll
-        for (int i = 0; i < NS; i++) {
-            if (i < n_src) {
-                u64 v[8];
+    for (int k = 0; k < 8; k++) {
+        Dot2 d;
+        dot_clear(d);
 #pragma unroll
-                for (int k = 0; k < 8; k++) {
-                    const u32x2 w = __builtin_amdgcn_raw_buffer_load_b64(src, voff, so[i] + off(8 * half + k), 0);
-                    v[k] = ((u64)w.y << 32) | w.x;
-                }
-#pragma unroll
-                for (int k = 0; k < 8; k++) dot3_add(d[k], v[k], h[i]);
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < 8; k++) x[8 * half + k] = f.from_dot(d[k], m);
+        for (int i = 0; i < N_SRC; i++) dot_add(d, ((u64)v[k][i].y << 32) | v[k][i].x, h[i]);
+        if (k + AHEAD < 8) load(k + AHEAD);
+        x[k] = f.from_dot(d, m);
     }
+}
+template <int K, int NS, class F, class OFF>
+__device__ __forceinline__ void converted_inputs(const F &f, typename F::E (&x)[8], const __amdgpu_buffer_rsrc_t src,
+                                                 const u32 voff, const u32 (&so)[NS], const DotCst (&h)[NS], const int n_src,
+                                                 const ModQ m, const OFF off) {
+    if constexpr (K > 1)
+        if (n_src < K) return converted_inputs<K - 1>(f, x, src, voff, so, h, n_src, m, off);
+    converted_exact<K>(f, x, src, voff, so, h, m, off);
 }
 
 // A row's 16 threads (32 with eight points each) sit in one wavefront, so the LDS exchanges of

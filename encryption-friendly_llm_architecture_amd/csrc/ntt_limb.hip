@@ -51,16 +51,16 @@ enum { LIFTED = -1 };
 template <int LR, int P, int NS, int TAIL, class F>
 __device__ __forceinline__ void limb_forward(u64 *__restrict__ limb, const Tw *__restrict__ tw_int, const Tw *__restrict__ rtw,
                                              const F f, u64 *lds_raw, const __amdgpu_buffer_rsrc_t src,
-                                             const u32 (&so)[NS > 0 ? NS : 1], const u64 (&h)[NS > 0 ? NS : 1], const int n_src,
+                                             const u32 (&so)[NS > 0 ? NS : 1], const DotCst (&h)[NS > 0 ? NS : 1], const int n_src,
                                              const ModQ m, const LiftSource &ls, const long long *__restrict__ coef,
                                              const u64 *__restrict__ mn, u64 *__restrict__ o, const Tw cst, RowSecond sec) {
     typedef typename F::E E;
     typedef Limb<LR, P> S;
     E *lds = (E *)lds_raw;
     E x[P];
-    if (NS > 0) {
-        converted_inputs<(NS > 0 ? NS : 1)>(f, x, src, S::voff(), so, h, n_src, m,
-                                            [](const int k) { return S::off(k); });
+    if constexpr (NS > 0) {
+        converted_inputs<NS>(f, x, src, S::voff(), so, h, n_src, m,
+                             [](const int k) { return S::off(k); });
     } else if (NS == LIFTED) {
 #pragma unroll
         for (int k = 0; k < P; k++) x[k] = f.from_canonical(lifted(ls, coef, (S::voff() + S::off(k)) >> 3, m));
@@ -121,7 +121,7 @@ __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_forward_kernel(
     const ModQ m = modq[prime];
     __amdgpu_buffer_rsrc_t src = limb_rsrc(base);
     u32 so[NS > 0 ? NS : 1];
-    u64 h[NS > 0 ? NS : 1];
+    DotCst h[NS > 0 ? NS : 1];
     int n_src = 0;
     if (NS > 0) {
         const int dg = __builtin_amdgcn_readfirstlane((int)cs.digit_of[limb]);
@@ -132,7 +132,8 @@ __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_forward_kernel(
         for (int i = 0; i < NS; i++) {
             const int ii = i < n_src ? i : 0;
             so[i] = __builtin_amdgcn_readfirstlane((u32)cs.d[dg].src_slot[ii]) << (log_n + 3);
-            h[i] = hat[(size_t)ii * cs.hat_ld].w;
+            const Cst hg = hat[(size_t)ii * cs.hat_ld];
+            h[i] = dot_cst(hg.w, hg.ws);
         }
     }
     const u64 *mn = nullptr;
@@ -153,7 +154,7 @@ __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_forward_kernel(
     if (fp[4 * prime] != 0.0)
         limb_forward<LR, P, NS, TAIL>(base, tw, rtw, FpField(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, ls,
                                    coef, mn, o, cst, sec);
-    else if ((m.q >> 60) != 0)
+    else if (NS <= 0 && (m.q >> 60) != 0)   // (the sums of a conversion take primes below 2^60)
         limb_forward<LR, P, NS, TAIL>(base, tw, rtw, IntField(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, ls,
                                    coef, mn, o, cst, sec);
     else
