@@ -262,7 +262,7 @@ __global__ __launch_bounds__(256) void emb_lift_kernel(const double2 *__restrict
     const long long c0 = round_half_away(v.x * inv_n * scale), c1 = round_half_away(v.y * inv_n * scale);
     u64 *o = out + (size_t)blockIdx.y * n_limbs * 2 * n;
     for (int j = 0; j < n_limbs; j++) {
-        const ModQ m = modq[ll.idx[j]];
+        const ModQ m = modq[table_byte(ll.idx, j)];
         const u64 r0 = reduce64((u64)(c0 < 0 ? -c0 : c0), m), r1 = reduce64((u64)(c1 < 0 ? -c1 : c1), m);
         o[(size_t)j * 2 * n + i] = c0 < 0 && r0 ? m.q - r0 : r0;
         o[(size_t)j * 2 * n + n + i] = c1 < 0 && r1 ? m.q - r1 : r1;

@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256) void inner_product_kernel(const u64 *__restric
                                                             const ModQ *__restrict__ modq, LimbList ll, DigitMap dm,
                                                             int beta, int n_ext, int n_full, int logN) {
     const int j = blockIdx.y;
-    const int prime = ll.idx[j];
+    const int prime = (int)table_byte(ll.idx, j);
     const ModQ m = modq[prime];
     const size_t n = (size_t)blockIdx.x * 256 + threadIdx.x;
     const size_t N = (size_t)1 << logN;
@@ -266,7 +266,7 @@ __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict_
         // limits overlap instead of alternating.
         const u32 rest = slot / (u32)n_out;
         const u32 s = (rest / (u32)n_j) * 8u + xcd;
-        j = jmap.idx[rest % (u32)n_j];
+        j = table_byte(jmap.idx, rest % (u32)n_j);
         (void)per;
         // output chunk whose gather lands in source chunk s: the low cbits+1 bits of the exponent 2 br(i) + 1
         // are fixed by the chunk; multiply them by g^-1 (mod 2^(cbits+1))
@@ -283,14 +283,14 @@ __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict_
         o = blockIdx.x % (u32)n_out;
         const u32 rest = blockIdx.x / (u32)n_out;
         chunk = rest % chunks;
-        j = jmap.idx[rest / chunks];
+        j = table_byte(jmap.idx, rest / chunks);
     }
     // output, limb and chunk are the same for the whole workgroup; the byte tables above are read with vector loads,
     // so say it: everything derived from them (the bases of all streams) then lives in scalar registers
     o = __builtin_amdgcn_readfirstlane(o);
     j = __builtin_amdgcn_readfirstlane(j);
     chunk = __builtin_amdgcn_readfirstlane(chunk);
-    const int prime = __builtin_amdgcn_readfirstlane((int)ll.idx[j]);
+    const int prime = (int)table_byte(ll.idx, j);
     const u32 n = (chunk * 256 + threadIdx.x) * 2;
     const double fq = fp[4 * prime];
     const size_t N = (size_t)1 << logN;

@@ -33,10 +33,10 @@ __global__ __launch_bounds__(256) void ntt_small_kernel(u64 *__restrict__ data, 
     __shared__ u64 lds[512];
     const int N = 1 << logN;
     const int limb = blockIdx.y % n_limbs, poly = blockIdx.y / n_limbs;
-    const int prime = ll.idx[limb];
+    const int prime = (int)table_byte(ll.idx, limb);
     const Tw *tw = tw_all + (size_t)prime * N;
     const u64 q = modq[prime].q, q2 = 2 * q, q4 = 4 * q, nq4 = opaque_neg(q4);
-    u64 *base = data + (size_t)poly * poly_stride + (size_t)sl.idx[limb] * N;
+    u64 *base = data + (size_t)poly * poly_stride + (size_t)table_byte(sl.idx, limb) * N;
     for (int e = threadIdx.x; e < N; e += blockDim.x) lds[e] = base[e];
     __syncthreads();
     for (int step = 0; step < logN; step++) {
@@ -152,10 +152,10 @@ __global__ __launch_bounds__(4096 / P) void ntt16_cols_kernel(u64 *__restrict__ 
                                                          int n_limbs, size_t poly_stride, const Tw *__restrict__ final_scale) {
     __shared__ u64 lds[256 * 16];
     const int limb = blockIdx.y % n_limbs, poly = blockIdx.y / n_limbs;
-    const int prime = ll.idx[limb];
+    const int prime = (int)table_byte(ll.idx, limb);
     const Tw *tw = tw_all + ((size_t)prime << (8 + LR));
     const __amdgpu_buffer_rsrc_t base = limb_rsrc(
-        data + (size_t)poly * poly_stride + ((size_t)__builtin_amdgcn_readfirstlane((int)sl.idx[limb]) << (8 + LR)));
+        data + (size_t)poly * poly_stride + ((size_t)table_byte(sl.idx, limb) << (8 + LR)));
     // final_scale (inverse transforms only): limb i ends with the constant final_scale[i] in place of 1/N -- a basis
     // conversion folds its (S/q_i)^-1 factor in here (the caller supplies (1/N)(S/q_i)^-1), at no cost
     if (fp[4 * prime] != 0.0) {
@@ -207,8 +207,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
     typedef Slab<LR, 8> S;
     if (limb >= n_limbs) {   // a limb that is only copied into its slot
         const u64 *from = cs.copy_src + (size_t)poly * cs.copy_src_stride +
-                          ((size_t)cs.copy_src_slot[limb - n_limbs] << (8 + LR));
-        u64 *base = data + (size_t)poly * poly_stride + ((size_t)cs.copy_dst_slot[limb - n_limbs] << (8 + LR)) + S::col();
+                          ((size_t)table_byte(cs.copy_src_slot, limb - n_limbs) << (8 + LR));
+        u64 *base = data + (size_t)poly * poly_stride + ((size_t)table_byte(cs.copy_dst_slot, limb - n_limbs) << (8 + LR)) + S::col();
         u64 t[8];
         if (cs.copy_galois != 0) {   // the copy of the source's automorphism
 #pragma unroll
@@ -223,10 +223,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
         return;
     }
     const __amdgpu_buffer_rsrc_t base = limb_rsrc(
-        data + (size_t)poly * poly_stride + ((size_t)__builtin_amdgcn_readfirstlane((int)sl.idx[limb]) << (8 + LR)));
-    const int prime = ll.idx[limb];
+        data + (size_t)poly * poly_stride + ((size_t)table_byte(sl.idx, limb) << (8 + LR)));
+    const int prime = (int)table_byte(ll.idx, limb);
     const Tw *tw = tw_all + ((size_t)prime << (8 + LR));
-    const int dg = __builtin_amdgcn_readfirstlane((int)cs.digit_of[limb]), n_src = cs.d[dg].n_src;
+    const int dg = (int)table_byte(cs.digit_of, limb), n_src = cs.d[dg].n_src;
     // The sources are read through a buffer resource: base (the polynomial's source limbs; far below 4 GiB), source slot
     // and slab row sit in scalar registers, a thread supplies one 32-bit offset for all of its 8 n_src loads.
     const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
 #pragma unroll
     for (int i = 0; i < NS; i++) {
         const int ii = i < n_src ? i : 0;
-        so[i] = __builtin_amdgcn_readfirstlane((u32)cs.d[dg].src_slot[ii]) << (11 + LR);
+        so[i] = table_byte(cs.d[dg].src_slot, ii) << (11 + LR);
         const Cst hg = hat[(size_t)ii * cs.hat_ld];
         h[i] = dot_cst(hg.w, hg.ws);
     }
@@ -267,10 +267,10 @@ __global__ __launch_bounds__(512) void ntt16_cols_lifted_kernel(u64 *__restrict_
                                                                 LiftSource ls) {
     __shared__ u64 lds[256 * 16];
     const int limb = blockIdx.y % n_limbs, poly = blockIdx.y / n_limbs;
-    const int prime = ll.idx[limb];
+    const int prime = (int)table_byte(ll.idx, limb);
     const Tw *tw = tw_all + ((size_t)prime << (8 + LR));
     const __amdgpu_buffer_rsrc_t base = limb_rsrc(
-        data + (size_t)poly * poly_stride + ((size_t)__builtin_amdgcn_readfirstlane((int)sl.idx[limb]) << (8 + LR)));
+        data + (size_t)poly * poly_stride + ((size_t)table_byte(sl.idx, limb) << (8 + LR)));
     const long long *coef = ls.coef + (size_t)poly * ls.stride;
     const ModQ m = modq[prime];
     if (fp[4 * prime] != 0.0)
@@ -457,10 +457,10 @@ __global__ __launch_bounds__(256) void ntt16_rows_kernel(u64 *__restrict__ data,
     const int limb = (int)(group >> (log_r - RB));
     const u32 slab = group & ((1u << (log_r - RB)) - 1u);
     const int log_n = 8 + log_r;
-    const int prime = ll.idx[limb];
+    const int prime = (int)table_byte(ll.idx, limb);
     const Tw *tw = tw_all + ((size_t)prime << log_n), *rtw = rtw_all + ((size_t)prime << log_n);
     const u32 r = (slab << RB) + (Lanes<P>::t() >> 4);  // global row
-    u64 *row = data + (size_t)poly * poly_stride + ((size_t)sl.idx[limb] << log_n) + ((size_t)r << 8);
+    u64 *row = data + (size_t)poly * poly_stride + ((size_t)table_byte(sl.idx, limb) << log_n) + ((size_t)r << 8);
     const u64 *mn = nullptr;
     u64 *o = nullptr;
     Tw cst{0, 0};
@@ -478,9 +478,9 @@ __global__ __launch_bounds__(256) void ntt16_rows_kernel(u64 *__restrict__ data,
     }
     const u64 *ld = row;
     if (INV && ep.minuend != nullptr)
-        ld = ep.minuend + (size_t)poly * ep.minuend_stride + ((size_t)sl.idx[limb] << log_n) + (LOAD == LOAD_ROTATED ? 0 : (size_t)r << 8);
+        ld = ep.minuend + (size_t)poly * ep.minuend_stride + ((size_t)table_byte(sl.idx, limb) << log_n) + (LOAD == LOAD_ROTATED ? 0 : (size_t)r << 8);
     if (LOAD == LOAD_DECRYPT)
-        sec.in = ep.second_in + (size_t)poly * ep.minuend_stride + ((size_t)sl.idx[limb] << log_n) + ((size_t)r << 8);
+        sec.in = ep.second_in + (size_t)poly * ep.minuend_stride + ((size_t)table_byte(sl.idx, limb) << log_n) + ((size_t)r << 8);
     if (TAIL == TAIL_ENCRYPT || LOAD == LOAD_DECRYPT) {
         sec.sk = ep.sk + ((size_t)prime << log_n) + ((size_t)r << 8);
         sec.m = modq[prime];

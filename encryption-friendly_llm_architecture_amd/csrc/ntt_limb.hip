@@ -103,8 +103,8 @@ __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_forward_kernel(
     const int per_poly = n_limbs + (NS > 0 ? cs.n_copy : 0);
     const int limb = blockIdx.x % per_poly, poly = blockIdx.x / per_poly;
     if (NS > 0 && limb >= n_limbs) {   // a limb that is only copied into its slot
-        const u64 *from = cs.copy_src + (size_t)poly * cs.copy_src_stride + ((size_t)cs.copy_src_slot[limb - n_limbs] << log_n);
-        u64 *to = data + (size_t)poly * poly_stride + ((size_t)cs.copy_dst_slot[limb - n_limbs] << log_n);
+        const u64 *from = cs.copy_src + (size_t)poly * cs.copy_src_stride + ((size_t)table_byte(cs.copy_src_slot, limb - n_limbs) << log_n);
+        u64 *to = data + (size_t)poly * poly_stride + ((size_t)table_byte(cs.copy_dst_slot, limb - n_limbs) << log_n);
         u64 t[P];
 #pragma unroll
         for (int k = 0; k < P; k++) {
@@ -115,8 +115,8 @@ __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_forward_kernel(
         for (int k = 0; k < P; k++) to[threadIdx.x + (u32)k * (u32)((256 / P) << LR)] = t[k];
         return;
     }
-    const int prime = __builtin_amdgcn_readfirstlane((int)ll.idx[limb]);   // byte tables are read with vector loads
-    u64 *base = data + (size_t)poly * poly_stride + ((size_t)__builtin_amdgcn_readfirstlane((int)sl.idx[limb]) << log_n);
+    const int prime = (int)table_byte(ll.idx, limb);
+    u64 *base = data + (size_t)poly * poly_stride + ((size_t)table_byte(sl.idx, limb) << log_n);
     const Tw *tw = tw_all + ((size_t)prime << log_n), *rtw = rtw_all + ((size_t)prime << log_n);
     const ModQ m = modq[prime];
     __amdgpu_buffer_rsrc_t src = limb_rsrc(base);
@@ -124,14 +124,14 @@ __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_forward_kernel(
     DotCst h[NS > 0 ? NS : 1];
     int n_src = 0;
     if (NS > 0) {
-        const int dg = __builtin_amdgcn_readfirstlane((int)cs.digit_of[limb]);
+        const int dg = (int)table_byte(cs.digit_of, limb);
         n_src = cs.d[dg].n_src;
         src = limb_rsrc(cs.d[dg].src + (size_t)poly * cs.d[dg].src_poly_stride);
         const Cst *hat = cs.d[dg].hat + prime;
 #pragma unroll
         for (int i = 0; i < NS; i++) {
             const int ii = i < n_src ? i : 0;
-            so[i] = __builtin_amdgcn_readfirstlane((u32)cs.d[dg].src_slot[ii]) << (log_n + 3);
+            so[i] = table_byte(cs.d[dg].src_slot, ii) << (log_n + 3);
             const Cst hg = hat[(size_t)ii * cs.hat_ld];
             h[i] = dot_cst(hg.w, hg.ws);
         }
@@ -202,8 +202,8 @@ __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_inverse_kernel(
     __shared__ u64 lds[(ROWPAD << LR)];
     const int log_n = 8 + LR;
     const int limb = blockIdx.x % n_limbs, poly = blockIdx.x / n_limbs;
-    const int prime = __builtin_amdgcn_readfirstlane((int)ll.idx[limb]);
-    const size_t slot = (size_t)__builtin_amdgcn_readfirstlane((int)sl.idx[limb]) << log_n;
+    const int prime = (int)table_byte(ll.idx, limb);
+    const size_t slot = (size_t)table_byte(sl.idx, limb) << log_n;
     u64 *base = data + (size_t)poly * poly_stride + slot;
     const u64 *ld = from.minuend != nullptr ? from.minuend + (size_t)poly * from.minuend_stride + slot : base;
     RowSecond sec{};

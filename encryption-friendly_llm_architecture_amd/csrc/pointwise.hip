@@ -20,7 +20,7 @@ __global__ __launch_bounds__(256) void binary_kernel(Operand a, Operand b, u64 *
                                                      const ModQ *__restrict__ modq, LimbList ll, int n_limbs,
                                                      int logN) {
     const int limb = blockIdx.y % n_limbs, poly = blockIdx.y / n_limbs;
-    const ModQ m = modq[ll.idx[limb]];
+    const ModQ m = modq[table_byte(ll.idx, limb)];
     const size_t e = ((size_t)limb << logN) + ((size_t)blockIdx.x * 256 + threadIdx.x) * 2;
     const ulonglong2 x = *(const ulonglong2 *)(a.p + poly * a.poly_stride + e);
     ulonglong2 y = make_ulonglong2(0, 0);
@@ -58,7 +58,7 @@ __global__ __launch_bounds__(256) void scalar_kernel(Operand a, u64 *__restrict_
                                                      const ModQ *__restrict__ modq, LimbList ll, ScalarList sc,
                                                      int n_limbs, int logN) {
     const int limb = blockIdx.y % n_limbs, poly = blockIdx.y / n_limbs;
-    const u64 q = modq[ll.idx[limb]].q;
+    const u64 q = modq[table_byte(ll.idx, limb)].q;
     const size_t k = ((size_t)blockIdx.x * 256 + threadIdx.x) * 2;
     const size_t e = ((size_t)limb << logN) + k;
     const ulonglong2 x = *(const ulonglong2 *)(a.p + poly * a.poly_stride + e);
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256) void scalar_add_kernel(Operand a, u64 *__restr
                                                          const ModQ *__restrict__ modq, LimbList ll, ScalarList sc,
                                                          int n_limbs, int logN) {
     const int limb = blockIdx.y;
-    const u64 q = modq[ll.idx[limb]].q;
+    const u64 q = modq[table_byte(ll.idx, limb)].q;
     const size_t k = ((size_t)blockIdx.x * 256 + threadIdx.x) * 2;
     const size_t e = ((size_t)limb << logN) + k;
     const ulonglong2 x = *(const ulonglong2 *)(a.p + e);

@@ -13,7 +13,7 @@ __global__ __launch_bounds__(256) void sample_uniform_kernel(KeyList keys, LimbL
                                                              u64 *__restrict__ out, int logN) {
     const int limb = blockIdx.y;
     const u64 i = (u64)blockIdx.x * 256 + threadIdx.x;
-    out[((size_t)limb << logN) + i] = sample_uniform(keys.key[limb], i, modq[ll.idx[limb]]);
+    out[((size_t)limb << logN) + i] = sample_uniform(keys.key[limb], i, modq[table_byte(ll.idx, limb)]);
 }
 
 // out[limb][i] = e_i mod q_limb for the centred-binomial error e of stream `key`
@@ -21,7 +21,7 @@ __global__ __launch_bounds__(256) void sample_error_kernel(u64 key, LimbList ll,
                                                            u64 *__restrict__ out, int logN) {
     const int limb = blockIdx.y;
     const u64 i = (u64)blockIdx.x * 256 + threadIdx.x;
-    const u64 q = modq[ll.idx[limb]].q;
+    const u64 q = modq[table_byte(ll.idx, limb)].q;
     const int e = sample_error(key, i);
     out[((size_t)limb << logN) + i] = e >= 0 ? (u64)e : q - (u64)(-e);
 }
