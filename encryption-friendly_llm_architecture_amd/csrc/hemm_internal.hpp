@@ -209,6 +209,9 @@ bool launch_moddown_slab(const hemm_context *c, u64 *y, size_t y_stride, const u
 bool launch_intt_from(const hemm_context *c, const u64 *src, size_t src_poly_stride, u64 *data, const LimbList &ll,
                       const LimbList &sl, int n_limbs, int n_polys, size_t poly_stride, hipStream_t s,
                       const void *final_scale = nullptr, u32 galois = 0);
+// the second pass of an inverse transform of two launches (N >= 2^13), in place
+void launch_intt_cols(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
+                      size_t poly_stride, hipStream_t s, const void *final_scale);
 void launch_ntt(const hemm_context *c, u64 *data, const LimbList &ll, int n_limbs, int n_polys,
                 size_t poly_stride, bool inverse, hipStream_t s);
 void launch_binary(const hemm_context *c, int op, const u64 *a, size_t a_stride, const u64 *b, size_t b_stride,
@@ -251,12 +254,15 @@ bool modup_through_automorphism_ok(const hemm_context *c, int nq);
 // compact: every term's key is in the compact layout (all terms of a launch use the same layout)
 void launch_hoisted_terms(hemm_context *c, const void *terms_dev, const u32 *group_off_dev, int n_out, int nq, u64 *y,
                           bool b_premultiplied, hipStream_t s, const void *terms_host = nullptr, int n_terms = 0,
-                          bool compact = false);
+                          bool compact = false, u64 inverse_rows = 0);
 int hoisted_arg_capacity();
 void launch_hoisted_terms_args(hemm_context *c, const void *terms_host, int n_terms, const u32 *group_off_host, int n_out,
-                               int nq, u64 *y, bool b_premultiplied, hipStream_t s);
+                               int nq, u64 *y, bool b_premultiplied, hipStream_t s, u64 inverse_rows = 0);
+// inverse_rows (bit j: limb j of the extended basis; N >= 2^9): these limbs of y are left as the first pass of their inverse
+// transform; rows_done: y comes so, for all limbs that the ModDown drops
+u64 moddown_rows_in_sum(const hemm_context *c, int nq, int n_out, int drop_last);
 void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop_last, u64 *out, size_t out_stride,
-                          u64 *conv, hipStream_t s, bool slab = false, const ResultList *list = nullptr);
+                          u64 *conv, hipStream_t s, bool slab = false, const ResultList *list = nullptr, bool rows_done = false);
 void launch_masked_sum(hemm_context *c, const void *terms_dev, const u32 *group_off_dev, int n_out, int nq, int n_polys,
                        u64 *out, hipStream_t s, const void *terms_host, int n_terms);
 // y[o][p][j] = sum_{q < parts} part[o * parts + q][p][j] over the extended basis, y / part: [.][2][nq+K][N]

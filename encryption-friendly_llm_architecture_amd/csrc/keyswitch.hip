@@ -12,7 +12,7 @@
 
 #include "hemm_internal.hpp"
 #include "hoisted.h"
-
+#include "ntt_device.h"
 
 namespace {
 
@@ -232,22 +232,100 @@ __global__ __launch_bounds__(256) void spread_kernel(const u64 *__restrict__ las
 
 u64 shoup_h(u64 w, u64 q) { return (u64)((((unsigned __int128)w) << 64) / q); }
 
+// ---- the first pass of an inverse transform on results that are still on chip -----------------------------------------------
+// The limbs that a ModDown drops are read by its inverse transform only, whose first pass stays inside rows of 256 residues: a
+// workgroup of a hoisted sum holds two whole rows of both polynomials, runs the eight stages on them and stores what the column
+// pass reads.  Written and read back as plain residues they cost a launch of their own and two trips through memory.
+// Four residues per thread: two stages on quads of neighbours, which two adjacent lanes make of their pairs of both polynomials
+// by an exchange, then a wavefront per row and two stages at a time, the row meeting in LDS in between.  Twiddles come from the
+// stage-ordered table, which adjacent lanes read side by side.
+// What bounds the sum stays its loads; 8 outputs of 7 + 4 limbs, five of them dropped: 72 -> 80 us (217 instead of 193 MB fetched, the
+// rest twiddles) for a launch of 26 us less.  Rotation on 24 primes of 60 bits, level 20 152.6 -> 147.1 us, at N = 2^13 48.5 -> 45.1, product
+// at level 9 126.8 -> 121.2, product of two encrypted matrices 2766 -> 2680, projection of a 768-wide layer 11.44 -> 10.95 ms.
+__device__ __forceinline__ u64 from_next_lane(const u64 v) {   // lane ^ 1
+    const u32 lo = (u32)__builtin_amdgcn_mov_dpp((int)(u32)v, 0xb1, 0xf, 0xf, true);
+    const u32 hi = (u32)__builtin_amdgcn_mov_dpp((int)(u32)(v >> 32), 0xb1, 0xf, 0xf, true);
+    return ((u64)hi << 32) | lo;
+}
+// two stages, distances d and 2 d, on points 0, d, 2 d, 3 d of group g of 2^l
+template <class F>
+__device__ __forceinline__ void two_stages_inv(const F &f, typename F::E (&x)[4], const typename F::W *__restrict__ tw, const u32 group) {
+    const typename F::W w0 = tw[2 * group], w1 = tw[2 * group + 1], w = tw[group];
+    f.gs(x[0], x[1], w0);
+    f.gs(x[2], x[3], w1);
+    f.gs(x[0], x[2], w);
+    f.gs(x[1], x[3], w);
+}
+// rb, ra: residues (2 t, 2 t + 1) of the workgroup's 512 of both polynomials; yb, ya: their places; row: the first of the two
+template <class F>
+__device__ __forceinline__ void rows_of_products(const F f, const u64 (&rb)[2], const u64 (&ra)[2], u64 *yb, u64 *ya, u64 *lds_raw,
+                                                 const Tw *__restrict__ tw_int, const int log_r, const u32 row) {
+    typedef typename F::E E;
+    const typename F::W *tw = (const typename F::W *)tw_int;
+    E *lds = (E *)lds_raw;
+    const u32 t = threadIdx.x, odd = t & 1u, R = 1u << log_r;
+    E x[4];
+    {   // even lanes go on with the quad of the first polynomial, odd ones with that of the second
+        const u64 r0 = from_next_lane(odd ? rb[0] : ra[0]), r1 = from_next_lane(odd ? rb[1] : ra[1]);
+        x[0] = f.from_canonical(odd ? r0 : rb[0]);
+        x[1] = f.from_canonical(odd ? r1 : rb[1]);
+        x[2] = f.from_canonical(odd ? ra[0] : r0);
+        x[3] = f.from_canonical(odd ? ra[1] : r1);
+        const u32 quad = (t & 127u) >> 1, r = t >> 7;
+        two_stages_inv(f, x, tw, 64u * (R + row + r) + quad);
+        E *l = lds + (2u * odd + r) * ROWPAD;
+#pragma unroll
+        for (int k = 0; k < 4; k++) l[padc((int)(4u * quad) + k)] = x[k];
+    }
+    __syncthreads();
+    const u32 wave = (u32)__builtin_amdgcn_readfirstlane((int)(t >> 6)), lane = t & 63u;
+    const u32 X = R + row + (wave & 1u);
+    E *l = lds + wave * ROWPAD;
+    const int b = (int)(16u * (lane >> 2) + (lane & 3u)), c = (int)(64u * (lane >> 4) + (lane & 15u));
+#pragma unroll
+    for (int k = 0; k < 4; k++) x[k] = l[padc(b + 4 * k)];
+    two_stages_inv(f, x, tw, 16u * X + (lane >> 2));
+    f.template after_inverse_block<2>(x);
+#pragma unroll
+    for (int k = 0; k < 4; k++) l[padc(b + 4 * k)] = x[k];
+    wave_sync();
+#pragma unroll
+    for (int k = 0; k < 4; k++) x[k] = l[padc(c + 16 * k)];
+    two_stages_inv(f, x, tw, 4u * X + (lane >> 4));
+#pragma unroll
+    for (int k = 0; k < 4; k++) l[padc(c + 16 * k)] = x[k];
+    wave_sync();
+#pragma unroll
+    for (int k = 0; k < 4; k++) x[k] = l[padc((int)lane + 64 * k)];
+    two_stages_inv(f, x, tw, X);
+    f.template after_inverse_block<2>(x);
+    E *to = (E *)(wave & 2u ? ya : yb) + 256u * (wave & 1u) + lane;
+#pragma unroll
+    for (int k = 0; k < 4; k++) to[64 * k] = x[k];
+}
+
 // Hoisted rotations, several per output, combined with masks in the extended basis:
 //   y[o][pol][j][n] = sum_{t in group o} mask_t[j][n] * ( sum_d ext_t[d][j][pi_t(n)] * evk_t[d][pol][j][n]
 //                                                         + [pol = 0, j < nq] (P mod q_j) * b_t[j][pi_t(n)] )
 // The automorphism is an index map on the reads (aligned 2^m-blocks map to aligned 2^m-blocks in the
 // bit-reversed order, so a wavefront still reads whole 512-byte runs); the key is streamed once.
+// Limbs in ir.limbs leave as the first pass of their inverse transform (rows_of_products).
 // MODE 1: the launch covers only limbs of primes below 2^44 (double-precision path); MODE 2: only the others
 // (integer path); MODE 0: any limb, path chosen per workgroup.  jmap lists the n_j limbs of the launch.  The integer
 // path keeps 128-bit accumulators and needs more registers, so on large launches the double-precision limbs get a
 // kernel of their own and run at a higher occupancy; small launches stay whole (two part-filled launches cost more).
+struct InverseRows {
+    u64 limbs;       // bit j: limb j of the extended basis
+    const Tw *tw;    // stage-ordered twiddles of the inverse transforms, [prime][N]
+};
 template <int MODE, bool COMPACT>
 __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict__ terms,
                                                    const u32 *__restrict__ group_off, u64 *__restrict__ y,
                                                    const ModQ *__restrict__ modq, const double *__restrict__ fp,
                                                    const LimbList &ll, const CstList &pmod, int nq, int E, int beta,
                                                    int n_full, int logN, int b_premultiplied, int n_out,
-                                                   const LimbList &jmap, int n_j, const u32 *__restrict__ koff) {
+                                                   const LimbList &jmap, int n_j, const u32 *__restrict__ koff,
+                                                   const InverseRows ir) {
     // A thread owns the residue pair (n, n+1): the automorphism maps an aligned pair to an aligned pair
     // (possibly swapped), so every access is a 16-byte load or store.
     // Work is dealt out by SOURCE chunk.  The automorphism maps aligned 512-coefficient chunks onto aligned
@@ -308,8 +386,19 @@ __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict_
         hoisted_pair_int<COMPACT>(terms, group_off, koff, modq[prime], pmod, j, o, prime, n, nq, E, beta, n_full, logN,
                                   b_premultiplied, rb, ra);
     }
-    stream_store2(y + (((size_t)o * 2 + 0) * E + j) * N + n, rb[0], rb[1]);
-    stream_store2(y + (((size_t)o * 2 + 1) * E + j) * N + n, ra[0], ra[1]);
+    u64 *yb = y + (((size_t)o * 2 + 0) * E + j) * N, *ya = y + (((size_t)o * 2 + 1) * E + j) * N;
+    if ((ir.limbs >> j) & 1ull) {
+        __shared__ u64 lds[4 * ROWPAD];
+        const u32 first = chunk * 512;
+        const Tw *tw = ir.tw + ((size_t)prime << logN);
+        if (MODE == 1 || (MODE == 0 && fq != 0.0))
+            rows_of_products(FpField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
+        else
+            rows_of_products(IntField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
+        return;
+    }
+    stream_store2(yb + n, rb[0], rb[1]);
+    stream_store2(ya + n, ra[0], ra[1]);
 }
 
 // Term lists of up to HOISTED_ARG_TERMS terms and outputs travel in the kernel arguments (no staging copy before
@@ -327,18 +416,18 @@ template <int MODE, bool COMPACT>
 HOISTED_KERNEL hoisted_terms_kernel(const HoistedArgs args, u64 *__restrict__ y, const ModQ *__restrict__ modq,
                                     const double *__restrict__ fp, LimbList ll, CstList pmod, int nq, int E, int beta,
                                     int n_full, int logN, int b_premultiplied, int n_out, LimbList jmap, int n_j,
-                                    const u32 *__restrict__ koff) {
+                                    const u32 *__restrict__ koff, const InverseRows ir) {
     hoisted_terms_body<MODE, COMPACT>(args.t, args.off, y, modq, fp, ll, pmod, nq, E, beta, n_full, logN,
-                                      b_premultiplied, n_out, jmap, n_j, koff);
+                                      b_premultiplied, n_out, jmap, n_j, koff, ir);
 }
 template <int MODE, bool COMPACT>
 HOISTED_KERNEL hoisted_terms_list_kernel(const RotTermDev *__restrict__ terms, const u32 *__restrict__ group_off,
                                          u64 *__restrict__ y, const ModQ *__restrict__ modq,
                                          const double *__restrict__ fp, LimbList ll, CstList pmod, int nq, int E,
                                          int beta, int n_full, int logN, int b_premultiplied, int n_out, LimbList jmap,
-                                         int n_j, const u32 *__restrict__ koff) {
+                                         int n_j, const u32 *__restrict__ koff, const InverseRows ir) {
     hoisted_terms_body<MODE, COMPACT>(terms, group_off, y, modq, fp, ll, pmod, nq, E, beta, n_full, logN,
-                                      b_premultiplied, n_out, jmap, n_j, koff);
+                                      b_premultiplied, n_out, jmap, n_j, koff, ir);
 }
 #undef HOISTED_KERNEL
 
@@ -939,8 +1028,9 @@ void launch_keyswitch(hemm_context *c, const u64 *in, const u64 *evk, int nq, u6
             n_terms = 2;
         }
         const u32 off[2] = {0, (u32)n_terms};
-        launch_hoisted_terms_args(c, term, n_terms, off, 1, nq, acc, false, s);
-        launch_moddown_batch(c, acc, nq, 2, 0, out, out_stride, coef, s);
+        const u64 rows = moddown_rows_in_sum(c, nq, 1, 0);
+        launch_hoisted_terms_args(c, term, n_terms, off, 1, nq, acc, false, s, rows);
+        launch_moddown_batch(c, acc, nq, 2, 0, out, out_stride, coef, s, false, nullptr, rows != 0);
         return;
     }
     launch_inner_product(c, in, ext, evk, nq, acc, s);
@@ -1325,7 +1415,8 @@ static bool split_limbs(const hemm_context *c, int nq, int beta, int n_out, Limb
 }
 
 void launch_hoisted_terms(hemm_context *c, const void *terms_dev, const u32 *group_off_dev, int n_out, int nq, u64 *y,
-                          bool b_premultiplied, hipStream_t s, const void *terms_host, int n_terms, bool compact) {
+                          bool b_premultiplied, hipStream_t s, const void *terms_host, int n_terms, bool compact, u64 inverse_rows) {
+    const InverseRows ir{inverse_rows, (const Tw *)c->d_iw};
     const int K = c->nP, E = nq + K, beta = (nq + c->alpha - 1) / c->alpha;
     if (terms_host != nullptr) account(c, TR_KEYPROD, hoisted_bytes(c, (const RotTermDev *)terms_host, n_terms, n_out, nq));
     const CstList pm = p_mod_chain(c, nq);
@@ -1346,7 +1437,7 @@ void launch_hoisted_terms(hemm_context *c, const void *terms_dev, const u32 *gro
 #define HOISTED_LIST(MODE, COMPACT, GRID, JM, NJ)                                                                  \
     hipLaunchKernelGGL((hoisted_terms_list_kernel<MODE, COMPACT>), dim3((unsigned)(GRID)), block, 0, s, td,        \
                        group_off_dev, y, c->d_modq, c->d_fp, ll, pm, nq, E, beta, n_full, c->logN, pre, n_out, JM, \
-                       NJ, c->d_key_off)
+                       NJ, c->d_key_off, ir)
     if (!split) {
         if (compact)
             HOISTED_LIST(0, true, per_limb * E, all, E);
@@ -1367,7 +1458,8 @@ void launch_hoisted_terms(hemm_context *c, const void *terms_dev, const u32 *gro
 // passed in the kernel arguments
 int hoisted_arg_capacity() { return HOISTED_ARG_TERMS; }
 void launch_hoisted_terms_args(hemm_context *c, const void *terms_host, int n_terms, const u32 *group_off_host, int n_out,
-                               int nq, u64 *y, bool b_premultiplied, hipStream_t s) {
+                               int nq, u64 *y, bool b_premultiplied, hipStream_t s, u64 inverse_rows) {
+    const InverseRows ir{inverse_rows, (const Tw *)c->d_iw};
     const int K = c->nP, E = nq + K, beta = (nq + c->alpha - 1) / c->alpha;
     const CstList pm = p_mod_chain(c, nq);
     if (c->N < 512) throw std::invalid_argument("hoisted terms need N >= 512");
@@ -1391,7 +1483,7 @@ void launch_hoisted_terms_args(hemm_context *c, const void *terms_host, int n_te
         throw std::invalid_argument("hoisted terms need keys below 4 GiB");
 #define HOISTED_ARGS(MODE, COMPACT, GRID, JM, NJ)                                                                  \
     hipLaunchKernelGGL((hoisted_terms_kernel<MODE, COMPACT>), dim3((unsigned)(GRID)), block, 0, s, a, y, c->d_modq, \
-                       c->d_fp, ll, pm, nq, E, beta, n_full, c->logN, pre, n_out, JM, NJ, c->d_key_off)
+                       c->d_fp, ll, pm, nq, E, beta, n_full, c->logN, pre, n_out, JM, NJ, c->d_key_off, ir)
     if (!split) {
         if (compact)
             HOISTED_ARGS(0, true, per_limb * E, all, E);
@@ -1409,11 +1501,22 @@ void launch_hoisted_terms_args(hemm_context *c, const void *terms_host, int n_te
 #undef HOISTED_ARGS
 }
 
+// The limbs of the extended basis whose inverse row pass belongs into the hoisted sum in front of a ModDown of n_out results (0: none):
+// all that it drops, where their inverse transform is two launches.
+u64 moddown_rows_in_sum(const hemm_context *c, int nq, int n_out, int drop_last) {
+    const int first = drop_last ? nq - 1 : nq, E = nq + c->nP;
+    if (first < 0 || E > 64 || c->logN < 13 || one_launch(c, (size_t)2 * n_out * (E - first), true)) return 0;
+    u64 limbs = 0;
+    for (int j = first; j < E; j++) limbs |= 1ull << j;
+    return limbs;
+}
+
 // y: [n_polys][nq+K][N] NTT (dropped limbs are clobbered).  drop_last = 0: out[p] = y[p] / P over nq limbs;
 // drop_last = 1: out[p] = y[p] / (P q_{nq-1}) over nq-1 limbs (ModDown and rescale in one conversion).
 // conv: workspace [n_polys][nq_out][N].  list: the results lie where it says.
+// rows_done: the dropped limbs are what rows_of_products leaves.
 void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop_last, u64 *out, size_t out_stride,
-                          u64 *conv, hipStream_t s, bool slab, const ResultList *list) {
+                          u64 *conv, hipStream_t s, bool slab, const ResultList *list, bool rows_done) {
     KsTables *t = g_tables_of(c);
     const int K = c->nP, E = nq + K, nq_out = drop_last ? nq - 1 : nq;
     const size_t N = c->N;
@@ -1442,6 +1545,7 @@ void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop
     const bool fold = ring_has_fused_forms(c);   // the inverse transform ends with (1/N)(S/q_i)^-1: no scaling pass in the conversion
     // the three-launch form with one column-slab kernel in the middle, only on request: it moves a fifth less data but
     // runs at two waves per SIMD and is slower on every batch size measured
+    if (slab && rows_done) throw std::invalid_argument("the column-slab ModDown begins with its own row pass");
     if (slab && list != nullptr) throw std::invalid_argument("the column-slab ModDown leaves its results back to back");
     if (slab && !(c->logN == 16 && lazy_dot_ok(c))) throw std::invalid_argument("the column-slab ModDown needs N = 2^16 and primes below 2^60");
     if (slab) {
@@ -1452,7 +1556,10 @@ void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop
             throw std::invalid_argument("the column-slab ModDown takes 4 or 5 dropped limbs");
         return;
     }
-    launch_ntt_slots(c, y, pl, sl, ns, n_polys, (size_t)E * N, true, s,
+    if (rows_done)
+        launch_intt_cols(c, y, pl, sl, ns, n_polys, (size_t)E * N, s, t->dev + (drop_last ? t->drop_invn_off[nq] : t->p_invn_off));
+    else
+        launch_ntt_slots(c, y, pl, sl, ns, n_polys, (size_t)E * N, true, s,
                      fold ? t->dev + (drop_last ? t->drop_invn_off[nq] : t->p_invn_off) : nullptr);
     a.pre_scaled = fold ? 1 : 0;
     a.src = y;

@@ -929,6 +929,14 @@ void launch_ntt_slots(const hemm_context *c, u64 *data, const LimbList &ll, cons
     }
 }
 
+void launch_intt_cols(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
+                      size_t poly_stride, hipStream_t s, const void *final_scale) {
+    account(c, TR_NTT, (size_t)2 * n_limbs * n_polys * c->N * 8, 1);
+    const int run = std::min(n_polys, 65535 / n_limbs);   // rows of workgroups of a launch
+    for (int p0 = 0; p0 < n_polys; p0 += run)
+        cols_pass(c, true, data + (size_t)p0 * poly_stride, ll, sl, n_limbs, std::min(run, n_polys - p0), poly_stride, s, final_scale);
+}
+
 void launch_ntt(const hemm_context *c, u64 *data, const LimbList &ll, int n_limbs, int n_polys,
                 size_t poly_stride, bool inverse, hipStream_t s) {
     LimbList sl;
