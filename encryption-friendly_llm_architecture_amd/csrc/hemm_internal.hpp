@@ -24,7 +24,7 @@ struct __align__(4) LimbList {
 __device__ __forceinline__ u32 table_byte(const uint8_t *t, const u32 i) {
     u32 w;
     __builtin_memcpy(&w, __builtin_assume_aligned(t + (i & ~3u), 4), 4);
-    return (w >> (8u * (i & 3u))) & 255u;
+    return (u32)__builtin_amdgcn_readfirstlane((int)((w >> (8u * (i & 3u))) & 255u));   // i may come out of a division in vector registers
 }
 
 struct hemm_context {
