@@ -525,25 +525,23 @@ static void build_rot_terms(hemm_context *ctx, const hemm_rot_term *terms, const
     for (RotDev &t : d)
         if (t.evk == nullptr) t.flags = layout;
 }
-// hoisted sums of a validated, merged term list: short lists travel in the kernel arguments, long ones through the
-// staging region
-static void run_hoisted_terms(hemm_context *ctx, const hemm_rot_term *terms, const uint32_t *group_offsets, uint32_t n_out,
-                              uint32_t nq, u64 *y, bool b_premultiplied, hipStream_t stream, u64 inverse_rows = 0) {
+// a validated, merged term list: short lists travel in the kernel arguments, long ones through the staging region
+struct Terms {
     std::vector<RotDev> d;
     std::vector<uint32_t> off;
-    build_rot_terms(ctx, terms, group_offsets, n_out, d, off);
-    for (const RotDev &t : d)
-        need(t.flags == d[0].flags, "all terms of a hoisted sum must use the same key layout");
-    if ((int)d.size() <= hoisted_arg_capacity() && (int)n_out <= hoisted_arg_capacity()) {
-        launch_hoisted_terms_args(ctx, d.data(), (int)d.size(), off.data(), (int)n_out, (int)nq, y, b_premultiplied, stream, inverse_rows);
-        return;
+    HoistedList list;
+    Terms(hemm_context *ctx, const hemm_rot_term *terms, const uint32_t *group_offsets, uint32_t n_out, hipStream_t stream) {
+        build_rot_terms(ctx, terms, group_offsets, n_out, d, off);
+        for (const RotDev &t : d)
+            need(t.flags == d[0].flags, "all terms of a hoisted sum must use the same key layout");
+        list = HoistedList{d.data(), off.data(), nullptr, nullptr, (int)d.size()};
+        if ((int)d.size() <= hoisted_arg_capacity() && (int)n_out <= hoisted_arg_capacity()) return;
+        void *off_dev = nullptr;
+        list.terms_dev = upload_desc(ctx, d.data(), d.size() * sizeof(RotDev), off.data(), (n_out + 1) * sizeof(uint32_t), &off_dev,
+                                     stream);
+        list.offsets_dev = (const u32 *)off_dev;
     }
-    void *off_dev = nullptr;
-    void *terms_dev = upload_desc(ctx, d.data(), d.size() * sizeof(RotDev), off.data(), (n_out + 1) * sizeof(uint32_t),
-                                  &off_dev, stream);
-    launch_hoisted_terms(ctx, terms_dev, (const u32 *)off_dev, (int)n_out, (int)nq, y, b_premultiplied, stream, d.data(),
-                         (int)d.size(), !d.empty() && (d[0].flags & HEMM_ROT_COMPACT_KEY) != 0, inverse_rows);
-}
+};
 
 size_t hemm_key_compact_words(const hemm_context *ctx) { return ctx ? key_compact_words(ctx) : 0; }
 int hemm_key_compact(hemm_context *ctx, const uint64_t *evk, uint64_t *out, void *stream) {
@@ -569,7 +567,8 @@ int hemm_hoisted_terms(hemm_context *ctx, const hemm_rot_term *terms, const uint
     chain_limbs(ctx, nq, 1, &nl);
     need(terms && group_offsets && y && n_out >= 1, "null operand");
     need(ctx->nP >= 1, "key switching needs special primes");
-    run_hoisted_terms(ctx, terms, group_offsets, n_out, nq, (u64 *)y, b_premultiplied != 0, on_stream(ctx, stream));
+    const Terms t(ctx, terms, group_offsets, n_out, on_stream(ctx, stream));
+    launch_hoisted_terms(ctx, t.list, (int)n_out, (int)nq, (u64 *)y, b_premultiplied != 0, on_stream(ctx, stream));
     check_launch();
     HEMM_CATCH
 }
@@ -582,10 +581,9 @@ int hemm_hoisted_moddown(hemm_context *ctx, const hemm_rot_term *terms, const ui
     chain_limbs(ctx, nq, 1, &nl);
     need(terms && group_offsets && y_workspace && out && workspace && n_out >= 1, "null operand");
     need(ctx->nP >= 1, "key switching needs special primes");
-    const u64 rows = moddown_rows_in_sum(ctx, (int)nq, (int)n_out, drop_last != 0);
-    run_hoisted_terms(ctx, terms, group_offsets, n_out, nq, (u64 *)y_workspace, b_premultiplied != 0, on_stream(ctx, stream), rows);
-    launch_moddown_batch(ctx, (u64 *)y_workspace, (int)nq, (int)(2 * n_out), drop_last != 0, (u64 *)out, out_stride,
-                         (u64 *)workspace, on_stream(ctx, stream), false, nullptr, rows != 0);
+    const Terms t(ctx, terms, group_offsets, n_out, on_stream(ctx, stream));
+    launch_hoisted_moddown(ctx, t.list, (int)n_out, (int)nq, (u64 *)y_workspace, b_premultiplied != 0, drop_last != 0, (u64 *)out,
+                           out_stride, nullptr, (u64 *)workspace, on_stream(ctx, stream));
     check_launch();
     HEMM_CATCH
 }
@@ -599,15 +597,9 @@ int hemm_hoisted_moddown_to(hemm_context *ctx, const hemm_rot_term *terms, const
     need(terms && group_offsets && y_workspace && outs && workspace && n_out >= 1, "null operand");
     need(ctx->nP >= 1, "key switching needs special primes");
     for (uint32_t o = 0; o < n_out; o++) need(outs[o] != nullptr, "null output");
-    const u64 rows = moddown_rows_in_sum(ctx, (int)nq, (int)std::min<uint32_t>(n_out, RESULT_PARTS), drop_last != 0);
-    run_hoisted_terms(ctx, terms, group_offsets, n_out, nq, (u64 *)y_workspace, b_premultiplied != 0, on_stream(ctx, stream), rows);
-    const size_t y_words = 2 * (size_t)(nq + ctx->nP) * ctx->N, ws_words = 2 * (size_t)(drop_last ? nq - 1 : nq) * ctx->N;
-    for (uint32_t o = 0; o < n_out; o += RESULT_PARTS) {
-        const uint32_t n = std::min<uint32_t>(n_out - o, RESULT_PARTS);
-        const ResultList list = results_in(outs + o, n);
-        launch_moddown_batch(ctx, (u64 *)y_workspace + o * y_words, (int)nq, (int)(2 * n), drop_last != 0, list.at[0], out_stride,
-                             (u64 *)workspace + o * ws_words, on_stream(ctx, stream), false, n > 1 ? &list : nullptr, rows != 0);
-    }
+    const Terms t(ctx, terms, group_offsets, n_out, on_stream(ctx, stream));
+    launch_hoisted_moddown(ctx, t.list, (int)n_out, (int)nq, (u64 *)y_workspace, b_premultiplied != 0, drop_last != 0, nullptr,
+                           out_stride, (u64 *const *)outs, (u64 *)workspace, on_stream(ctx, stream));
     check_launch();
     HEMM_CATCH
 }

@@ -160,12 +160,12 @@ struct ConvSources {
 };
 // data: [n_polys][.][N] (polynomial stride poly_stride), limb l written to slot sl[l].  With ep_* set the second pass
 // ends with out = (minuend - transform) * cst[l] (slots of minuend / out = l) and data is only a workspace; ep_list: the
-// polynomials of `out` lie where the list says.
+// polynomials of `out` lie where the list says.  cols_only: the first of two passes, left in data.
 // false when the ring size or the source counts have no such form (nothing was launched).
 bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *data, const LimbList &ll, const LimbList &sl,
                           int n_limbs, int n_polys, size_t poly_stride, hipStream_t s, const u64 *ep_minuend = nullptr,
                           size_t ep_minuend_stride = 0, u64 *ep_out = nullptr, size_t ep_out_stride = 0,
-                          const void *ep_cst_dev = nullptr, const ResultList *ep_list = nullptr);
+                          const void *ep_cst_dev = nullptr, const ResultList *ep_list = nullptr, bool cols_only = false);
 // A forward transform of N >= 2^10 whose input is the rounded coefficients of an encoding (signed, [n_polys][stride >= N], the
 // same for every limb; plus, with_error, the error of a stream), reduced while the first pass loads them.  enc: the second
 // pass ends in an encryption instead of storing the transform (data is then only a workspace): a uniform from the streams
@@ -250,19 +250,23 @@ void launch_modup_batch(hemm_context *c, const u64 *in, size_t in_stride, int nq
                         hipStream_t s, u32 galois = 0);
 // whether launch_modup_batch at this level takes a non-zero `galois` (its input read through that automorphism)
 bool modup_through_automorphism_ok(const hemm_context *c, int nq);
-// terms_host / n_terms: the host copy of the list (only read for the byte accounting; may be nullptr)
-// compact: every term's key is in the compact layout (all terms of a launch use the same layout)
-void launch_hoisted_terms(hemm_context *c, const void *terms_dev, const u32 *group_off_dev, int n_out, int nq, u64 *y,
-                          bool b_premultiplied, hipStream_t s, const void *terms_host = nullptr, int n_terms = 0,
-                          bool compact = false, u64 inverse_rows = 0);
+// A list of rotation terms (merged; RotTermDev) and the offsets of its groups: in host memory, and in device memory as well where it
+// is too long for the kernel arguments (terms_dev, then the only copy the kernels read).  All keys in one layout.
+struct HoistedList {
+    const void *terms;
+    const u32 *offsets;
+    const void *terms_dev;
+    const u32 *offsets_dev;
+    int n_terms;
+};
 int hoisted_arg_capacity();
-void launch_hoisted_terms_args(hemm_context *c, const void *terms_host, int n_terms, const u32 *group_off_host, int n_out,
-                               int nq, u64 *y, bool b_premultiplied, hipStream_t s, u64 inverse_rows = 0);
-// inverse_rows (bit j: limb j of the extended basis; N >= 2^9): these limbs of y are left as the first pass of their inverse
-// transform; rows_done: y comes so, for all limbs that the ModDown drops
-u64 moddown_rows_in_sum(const hemm_context *c, int nq, int n_out, int drop_last);
+void launch_hoisted_terms(hemm_context *c, const HoistedList &l, int n_out, int nq, u64 *y, bool b_premultiplied, hipStream_t s);
+// outs: the two polynomials of result o at outs[o], out_stride apart (nullptr: back to back at out)
+void launch_hoisted_moddown(hemm_context *c, const HoistedList &l, int n_out, int nq, u64 *y, bool b_premultiplied, int drop_last, u64 *out,
+                            size_t out_stride, u64 *const *outs, u64 *conv, hipStream_t s);
 void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop_last, u64 *out, size_t out_stride,
-                          u64 *conv, hipStream_t s, bool slab = false, const ResultList *list = nullptr, bool rows_done = false);
+                          u64 *conv, hipStream_t s, bool slab = false, const ResultList *list = nullptr, bool rows_done = false,
+                          bool cols_only = false);
 void launch_masked_sum(hemm_context *c, const void *terms_dev, const u32 *group_off_dev, int n_out, int nq, int n_polys,
                        u64 *out, hipStream_t s, const void *terms_host, int n_terms);
 // y[o][p][j] = sum_{q < parts} part[o * parts + q][p][j] over the extended basis, y / part: [.][2][nq+K][N]

@@ -124,12 +124,16 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t key_rsrc(const RotTermDev &T) 
     // raw buffer (stride 0), no range limit, 32-bit data format
     return __builtin_amdgcn_make_buffer_rsrc((void *)T.evk, 0, -1, 0x00020000);
 }
-// byte offset of limb `prime` of polynomial pol of digit d inside the key (keys are far below 4 GiB)
+// byte offsets inside a key (far below 4 GiB) of one limb: of polynomial 0 of digit 0, and the step to each next (digit, polynomial);
+// read once per workgroup, not in front of every load of a key
+struct KeyLimb {
+    u32 at, slice;
+    __device__ __forceinline__ u32 of(const int d, const int pol) const { return at + (u32)(d * 2 + pol) * slice; }
+};
 template <bool COMPACT>
-__device__ __forceinline__ u32 key_limb(const u32 *__restrict__ koff, const int d, const int pol, const int prime,
-                                        const int logN, const int n_full) {
-    if (COMPACT) return (((u32)(d * 2 + pol) * koff[n_full] + koff[prime]) << (logN + 1));
-    return ((u32)((d * 2 + pol) * n_full + prime)) << (logN + 3);
+__device__ __forceinline__ KeyLimb key_limb(const u32 *__restrict__ koff, const int prime, const int logN, const int n_full) {
+    if (COMPACT) return KeyLimb{koff[prime] << (logN + 1), koff[n_full] << (logN + 1)};
+    return KeyLimb{(u32)prime << (logN + 3), (u32)n_full << (logN + 3)};
 }
 // residues (n, n+1) of a limb of any prime (compact keys: of a prime of 2^44 or more); streamed (non-temporal)
 __device__ __forceinline__ ulonglong2 key_pair_u64(const __amdgpu_buffer_rsrc_t key, const u32 limb, const u32 n) {
@@ -138,12 +142,8 @@ __device__ __forceinline__ ulonglong2 key_pair_u64(const __amdgpu_buffer_rsrc_t 
 }
 // The integer path keeps plain pointers: it is short of scalar registers (106 of 102 usable with a resource per term,
 // which spilled 18 vector registers), not of vector registers.
-template <bool COMPACT>
-__device__ __forceinline__ ulonglong2 key_pair_ptr(const RotTermDev &T, const u32 *__restrict__ koff, const int d,
-                                                   const int pol, const int prime, const int logN, const int n_full,
-                                                   const u32 n) {
-    const char *limb = (const char *)T.evk + key_limb<COMPACT>(koff, d, pol, prime, logN, n_full);
-    return stream_load2((const u64 *)limb + n);
+__device__ __forceinline__ ulonglong2 key_pair_ptr(const RotTermDev &T, const u32 limb, const u32 n) {
+    return stream_load2((const u64 *)((const char *)T.evk + limb) + n);
 }
 typedef u32 u32x3 __attribute__((ext_vector_type(3), aligned(4)));
 
@@ -151,11 +151,11 @@ typedef u32 u32x3 __attribute__((ext_vector_type(3), aligned(4)));
 // <z, evk> + P (mask b + mask2 b2) with z_d = mask * x_d + mask2 * x2_d, canonical.  RUNS: the masks are run tables,
 // i.e. constants with a Shoup companion: no wide product and no Barrett step for z_d; a plaintext factor of the term is
 // then left to the caller, which multiplies the finished pair by it.
-template <bool RUNS, bool COMPACT>
-__device__ __forceinline__ void two_source_int(const RotTermDev &T, const u32 *__restrict__ koff, const ModQ m,
-                                               const CstList &pmod, const int j,
-                                               const int prime, const u32 n, const u32 base, const bool swap, int nq,
-                                               int E, int beta, int n_full, int logN, int b_premultiplied,
+template <bool RUNS>
+__device__ __forceinline__ void two_source_int(const RotTermDev &T, const KeyLimb kl, const ModQ m,
+                                               const Cst *__restrict__ pmod, const int j,
+                                               const u32 n, const u32 base, const bool swap, int nq,
+                                               int E, int beta, int logN, int b_premultiplied,
                                                u64 (&rb)[2], u64 (&ra)[2]) {
     const size_t N = (size_t)1 << logN;
     ulonglong2 m1, m2;   // RUNS: (value, companion) of each mask; otherwise the mask residues of the pair
@@ -196,8 +196,8 @@ __device__ __forceinline__ void two_source_int(const RotTermDev &T, const u32 *_
             z0 = barrett3_u(t0, m);
             z1 = barrett3_u(t1, m);
         }
-        const ulonglong2 kb = key_pair_ptr<COMPACT>(T, koff, d, 0, prime, logN, n_full, n);
-        const ulonglong2 ka = key_pair_ptr<COMPACT>(T, koff, d, 1, prime, logN, n_full, n);
+        const ulonglong2 kb = key_pair_ptr(T, kl.of(d, 0), n);
+        const ulonglong2 ka = key_pair_ptr(T, kl.of(d, 1), n);
         add128(pb[0], mul64wide(z0, kb.x));
         add128(pb[1], mul64wide(z1, kb.y));
         add128(pa[0], mul64wide(z0, ka.x));
@@ -226,10 +226,10 @@ __device__ __forceinline__ void two_source_int(const RotTermDev &T, const u32 *_
             b2.y = tmp;
         }
         if (!b_premultiplied) {
-            b1.x = mul_shoup_u(b1.x, pmod.c[j].w, pmod.c[j].ws, m.q);
-            b1.y = mul_shoup_u(b1.y, pmod.c[j].w, pmod.c[j].ws, m.q);
-            b2.x = mul_shoup_u(b2.x, pmod.c[j].w, pmod.c[j].ws, m.q);
-            b2.y = mul_shoup_u(b2.y, pmod.c[j].w, pmod.c[j].ws, m.q);
+            b1.x = mul_shoup_u(b1.x, pmod[j].w, pmod[j].ws, m.q);
+            b1.y = mul_shoup_u(b1.y, pmod[j].w, pmod[j].ws, m.q);
+            b2.x = mul_shoup_u(b2.x, pmod[j].w, pmod[j].ws, m.q);
+            b2.y = mul_shoup_u(b2.y, pmod[j].w, pmod[j].ws, m.q);
         }
         if (RUNS) {
             rb[0] = addmod_u(rb[0], shoup_pair(b1.x, m1, b2.x, m2, m.q), m.q);
@@ -247,10 +247,10 @@ __device__ __forceinline__ void two_source_int(const RotTermDev &T, const u32 *_
 // Residues (n, n+1) of limb j of both polynomials of output o (integer path), canonical.
 template <bool COMPACT>
 __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ terms,
-                                                 const u32 *__restrict__ group_off, const u32 *__restrict__ koff,
-                                                 const ModQ m, const CstList &pmod,
-                                                 const int j, const int o, const int prime, const u32 n, int nq, int E,
-                                                 int beta, int n_full, int logN, int b_premultiplied, u64 (&out_b)[2],
+                                                 const u32 *__restrict__ group_off, const KeyLimb kl,
+                                                 const ModQ m, const Cst *__restrict__ pmod,
+                                                 const int j, const int o, const u32 n, int nq, int E,
+                                                 int beta, int logN, int b_premultiplied, u64 (&out_b)[2],
                                                  u64 (&out_a)[2]) {
     const size_t N = (size_t)1 << logN;
     u64 acc_b[2] = {0, 0}, acc_a[2] = {0, 0};
@@ -270,7 +270,7 @@ __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ 
             if (T.mask_shift != 0) {
                 // run-table masks are constants: the plaintext factor of the term, if it has one, is common to both
                 // sources and multiplies the finished pair once (same residues as masks multiplied by it beforehand)
-                two_source_int<true, COMPACT>(T, koff, m, pmod, j, prime, n, base, swap, nq, E, beta, n_full, logN,
+                two_source_int<true>(T, kl, m, pmod, j, n, base, swap, nq, E, beta, logN,
                                               b_premultiplied, rb, ra);
                 if (T.pt != nullptr) {
                     const ulonglong2 pv = load_rotated2(T.pt, T.pt_galois, j, n, logN);
@@ -280,7 +280,7 @@ __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ 
                     ra[1] = mulmod_u(ra[1], pv.y, m);
                 }
             } else {
-                two_source_int<false, COMPACT>(T, koff, m, pmod, j, prime, n, base, swap, nq, E, beta, n_full, logN,
+                two_source_int<false>(T, kl, m, pmod, j, n, base, swap, nq, E, beta, logN,
                                                b_premultiplied, rb, ra);
             }
             acc_b[0] = addmod_u(acc_b[0], rb[0], m.q);
@@ -299,8 +299,8 @@ __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ 
                 x.x = x.y;
                 x.y = tmp;
             }
-            const ulonglong2 kb = key_pair_ptr<COMPACT>(T, koff, d, 0, prime, logN, n_full, n);
-            const ulonglong2 ka = key_pair_ptr<COMPACT>(T, koff, d, 1, prime, logN, n_full, n);
+            const ulonglong2 kb = key_pair_ptr(T, kl.of(d, 0), n);
+            const ulonglong2 ka = key_pair_ptr(T, kl.of(d, 1), n);
             add128(sb[0], mul64wide(x.x, kb.x));
             add128(sb[1], mul64wide(x.y, kb.y));
             add128(sa[0], mul64wide(x.x, ka.x));
@@ -326,8 +326,8 @@ __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ 
                 bv.y = tmp;
             }
             if (!b_premultiplied) {
-                bv.x = mul_shoup_u(bv.x, pmod.c[j].w, pmod.c[j].ws, m.q);
-                bv.y = mul_shoup_u(bv.y, pmod.c[j].w, pmod.c[j].ws, m.q);
+                bv.x = mul_shoup_u(bv.x, pmod[j].w, pmod[j].ws, m.q);
+                bv.y = mul_shoup_u(bv.y, pmod[j].w, pmod[j].ws, m.q);
             }
             rb[0] = addmod_u(rb[0], bv.x, m.q);
             rb[1] = addmod_u(rb[1], bv.y, m.q);
@@ -339,8 +339,8 @@ __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ 
                 av.x = av.y;
                 av.y = tmp;
             }
-            av.x = mul_shoup_u(av.x, pmod.c[j].w, pmod.c[j].ws, m.q);   // never premultiplied, whatever b is
-            av.y = mul_shoup_u(av.y, pmod.c[j].w, pmod.c[j].ws, m.q);
+            av.x = mul_shoup_u(av.x, pmod[j].w, pmod[j].ws, m.q);   // never premultiplied, whatever b is
+            av.y = mul_shoup_u(av.y, pmod[j].w, pmod[j].ws, m.q);
             ra[0] = av.x;
             ra[1] = av.y;
         }
@@ -420,10 +420,10 @@ __device__ __forceinline__ D2 key_pair_fp(const __amdgpu_buffer_rsrc_t key, cons
 // The same residues in double precision (primes below 2^44); out_* are unreduced centred doubles.
 template <bool COMPACT>
 __device__ __forceinline__ void hoisted_pair_fp(const RotTermDev *__restrict__ terms,
-                                                const u32 *__restrict__ group_off, const u32 *__restrict__ koff,
+                                                const u32 *__restrict__ group_off, const KeyLimb kl,
                                                 const FpMod f, const double p_mod_q,
-                                                const int j, const int o, const int prime, const u32 n, int nq, int E,
-                                                int beta, int n_full, int logN, int b_premultiplied, double (&out_b)[2],
+                                                const int j, const int o, const u32 n, int nq, int E,
+                                                int beta, int logN, int b_premultiplied, double (&out_b)[2],
                                                 double (&out_a)[2]) {
     const size_t N = (size_t)1 << logN;
     double acc_b0 = 0, acc_b1 = 0, acc_a0 = 0, acc_a1 = 0;
@@ -451,8 +451,8 @@ __device__ __forceinline__ void hoisted_pair_fp(const RotTermDev *__restrict__ t
                 const D2 x2 = gather_d2(T.ext2 + ((size_t)d * E + j) * N + base, swap);
                 const double z0 = f.mul(m1.x, x1.x) + f.mul(m2.x, x2.x);
                 const double z1 = f.mul(m1.y, x1.y) + f.mul(m2.y, x2.y);
-                const D2 kb = key_pair_fp<COMPACT>(kr, key_limb<COMPACT>(koff, d, 0, prime, logN, n_full), n);
-                const D2 ka = key_pair_fp<COMPACT>(kr, key_limb<COMPACT>(koff, d, 1, prime, logN, n_full), n);
+                const D2 kb = key_pair_fp<COMPACT>(kr, kl.of(d, 0), n);
+                const D2 ka = key_pair_fp<COMPACT>(kr, kl.of(d, 1), n);
                 sb0 += f.mul(z0, kb.x);
                 sb1 += f.mul(z1, kb.y);
                 sa0 += f.mul(z0, ka.x);
@@ -475,8 +475,8 @@ __device__ __forceinline__ void hoisted_pair_fp(const RotTermDev *__restrict__ t
             const bool ext_as_is = !COMPACT && (T.flags & ROT_TERM_EXT_ROTATED) != 0;
             for (int d = 0; d < (keyless ? 0 : beta); d++) {
                 const D2 x = gather_d2(T.ext + ((size_t)d * E + j) * N + (ext_as_is ? n : base), swap && !ext_as_is);
-                const D2 kb = key_pair_fp<COMPACT>(kr, key_limb<COMPACT>(koff, d, 0, prime, logN, n_full), n);
-                const D2 ka = key_pair_fp<COMPACT>(kr, key_limb<COMPACT>(koff, d, 1, prime, logN, n_full), n);
+                const D2 kb = key_pair_fp<COMPACT>(kr, kl.of(d, 0), n);
+                const D2 ka = key_pair_fp<COMPACT>(kr, kl.of(d, 1), n);
                 sb0 += f.mul(x.x, kb.x);
                 sb1 += f.mul(x.y, kb.y);
                 sa0 += f.mul(x.x, ka.x);

@@ -8,7 +8,9 @@
 //   ModDown  : INTT of the special limbs, basis conversion P -> Q, NTT, (acc - conv) * P^-1.
 //   rescale  : INTT of the last limb, reduce into every remaining prime, NTT, (c - t) * q_l^-1.
 // Basis conversion is the float-free form  y_j = sum_i [x_i * (S/q_i)^-1]_{q_i} * (S/q_i) mod q_j.
+#include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "hemm_internal.hpp"
 #include "hoisted.h"
@@ -238,7 +240,7 @@ u64 shoup_h(u64 w, u64 q) { return (u64)((((unsigned __int128)w) << 64) / q); }
 // pass reads.  Written and read back as plain residues they cost a launch of their own and two trips through memory.
 // Four residues per thread: two stages on quads of neighbours, which two adjacent lanes make of their pairs of both polynomials
 // by an exchange, then a wavefront per row and two stages at a time, the row meeting in LDS in between.  Twiddles come from the
-// stage-ordered table, which adjacent lanes read side by side.
+// stage-ordered table, which adjacent lanes read side by side, all of them in one trip in front of the first stage.
 // What bounds the sum stays its loads; 8 outputs of 7 + 4 limbs, five of them dropped: 72 -> 80 us (217 instead of 193 MB fetched, the
 // rest twiddles) for a launch of 26 us less.  Rotation on 24 primes of 60 bits, level 20 152.6 -> 147.1 us, at N = 2^13 48.5 -> 45.1, product
 // at level 9 126.8 -> 121.2, product of two encrypted matrices 2766 -> 2680, projection of a 768-wide layer 11.44 -> 10.95 ms.
@@ -247,15 +249,24 @@ __device__ __forceinline__ u64 from_next_lane(const u64 v) {   // lane ^ 1
     const u32 hi = (u32)__builtin_amdgcn_mov_dpp((int)(u32)(v >> 32), 0xb1, 0xf, 0xf, true);
     return ((u64)hi << 32) | lo;
 }
-// two stages, distances d and 2 d, on points 0, d, 2 d, 3 d of group g of 2^l
+// the twiddles of two stages, distances d and 2 d, on points 0, d, 2 d, 3 d of a group
 template <class F>
-__device__ __forceinline__ void two_stages_inv(const F &f, typename F::E (&x)[4], const typename F::W *__restrict__ tw, const u32 group) {
-    const typename F::W w0 = tw[2 * group], w1 = tw[2 * group + 1], w = tw[group];
-    f.gs(x[0], x[1], w0);
-    f.gs(x[2], x[3], w1);
-    f.gs(x[0], x[2], w);
-    f.gs(x[1], x[3], w);
-}
+struct TwoStages {
+    typename F::W w0, w1, w;
+    __device__ __forceinline__ TwoStages(const typename F::W *__restrict__ tw, const u32 group) : w0(tw[2 * group]), w1(tw[2 * group + 1]), w(tw[group]) {}
+    __device__ __forceinline__ void inverse(const F &f, typename F::E (&x)[4]) const {
+        f.gs(x[0], x[1], w0);
+        f.gs(x[2], x[3], w1);
+        f.gs(x[0], x[2], w);
+        f.gs(x[1], x[3], w);
+    }
+    __device__ __forceinline__ void forward(const F &f, typename F::E (&x)[4]) const {
+        f.ct(x[0], x[2], w, false);
+        f.ct(x[1], x[3], w, false);
+        f.ct(x[0], x[1], w0, true);
+        f.ct(x[2], x[3], w1, true);
+    }
+};
 // rb, ra: residues (2 t, 2 t + 1) of the workgroup's 512 of both polynomials; yb, ya: their places; row: the first of the two
 template <class F>
 __device__ __forceinline__ void rows_of_products(const F f, const u64 (&rb)[2], const u64 (&ra)[2], u64 *yb, u64 *ya, u64 *lds_raw,
@@ -264,6 +275,9 @@ __device__ __forceinline__ void rows_of_products(const F f, const u64 (&rb)[2], 
     const typename F::W *tw = (const typename F::W *)tw_int;
     E *lds = (E *)lds_raw;
     const u32 t = threadIdx.x, odd = t & 1u, R = 1u << log_r;
+    const u32 wave = (u32)__builtin_amdgcn_readfirstlane((int)(t >> 6)), lane = t & 63u;
+    const u32 quad = (t & 127u) >> 1, r = t >> 7, X = R + row + (wave & 1u);
+    const TwoStages<F> s1(tw, 64u * (R + row + r) + quad), s4(tw, 16u * X + (lane >> 2)), s16(tw, 4u * X + (lane >> 4)), s64(tw, X);
     E x[4];
     {   // even lanes go on with the quad of the first polynomial, odd ones with that of the second
         const u64 r0 = from_next_lane(odd ? rb[0] : ra[0]), r1 = from_next_lane(odd ? rb[1] : ra[1]);
@@ -271,37 +285,95 @@ __device__ __forceinline__ void rows_of_products(const F f, const u64 (&rb)[2], 
         x[1] = f.from_canonical(odd ? r1 : rb[1]);
         x[2] = f.from_canonical(odd ? ra[0] : r0);
         x[3] = f.from_canonical(odd ? ra[1] : r1);
-        const u32 quad = (t & 127u) >> 1, r = t >> 7;
-        two_stages_inv(f, x, tw, 64u * (R + row + r) + quad);
+        s1.inverse(f, x);
         E *l = lds + (2u * odd + r) * ROWPAD;
 #pragma unroll
         for (int k = 0; k < 4; k++) l[padc((int)(4u * quad) + k)] = x[k];
     }
     __syncthreads();
-    const u32 wave = (u32)__builtin_amdgcn_readfirstlane((int)(t >> 6)), lane = t & 63u;
-    const u32 X = R + row + (wave & 1u);
     E *l = lds + wave * ROWPAD;
     const int b = (int)(16u * (lane >> 2) + (lane & 3u)), c = (int)(64u * (lane >> 4) + (lane & 15u));
 #pragma unroll
     for (int k = 0; k < 4; k++) x[k] = l[padc(b + 4 * k)];
-    two_stages_inv(f, x, tw, 16u * X + (lane >> 2));
+    s4.inverse(f, x);
     f.template after_inverse_block<2>(x);
 #pragma unroll
     for (int k = 0; k < 4; k++) l[padc(b + 4 * k)] = x[k];
     wave_sync();
 #pragma unroll
     for (int k = 0; k < 4; k++) x[k] = l[padc(c + 16 * k)];
-    two_stages_inv(f, x, tw, 4u * X + (lane >> 4));
+    s16.inverse(f, x);
 #pragma unroll
     for (int k = 0; k < 4; k++) l[padc(c + 16 * k)] = x[k];
     wave_sync();
 #pragma unroll
     for (int k = 0; k < 4; k++) x[k] = l[padc((int)lane + 64 * k)];
-    two_stages_inv(f, x, tw, X);
+    s64.inverse(f, x);
     f.template after_inverse_block<2>(x);
     E *to = (E *)(wave & 2u ? ya : yb) + 256u * (wave & 1u) + lane;
 #pragma unroll
     for (int k = 0; k < 4; k++) to[64 * k] = x[k];
+}
+
+// The other way round for the limbs that a ModDown keeps: the second pass of the converted limbs' forward transform, on the rows
+// that the sum's products belong to, and its tail (products - transform) * cst.  The sum is neither written nor read back (100 of
+// 740 MB for 8 outputs of 7 + 4 limbs): sum, row pass and tail 80 + 34 us as two launches, 48 + 56 us as the two halves of the sum with the
+// row passes in them.  Product of two encrypted matrices 2655 -> 2530 us, projection of a 768-wide layer 10.92 -> 10.33 ms,
+// rotation on 24 primes of 60 bits, level 20 147.7 -> 145.0 us.
+template <class E>
+__device__ __forceinline__ E value_from_next_lane(const E v) {
+    u64 u;
+    __builtin_memcpy(&u, &v, 8);
+    u = from_next_lane(u);
+    E r;
+    __builtin_memcpy(&r, &u, 8);
+    return r;
+}
+// cb, ca: what the column pass left of the workgroup's rows of both polynomials; ob, oa: the results' places
+template <class F>
+__device__ __forceinline__ void rows_under_products(const F f, const u64 (&rb)[2], const u64 (&ra)[2], const u64 *__restrict__ cb,
+                                                    const u64 *__restrict__ ca, u64 *ob, u64 *oa, u64 *lds_raw,
+                                                    const Tw *__restrict__ tw_int, const int log_r, const u32 row, const Tw cst) {
+    typedef typename F::E E;
+    const typename F::W *tw = (const typename F::W *)tw_int;
+    E *lds = (E *)lds_raw;
+    const u32 t = threadIdx.x, odd = t & 1u, R = 1u << log_r;
+    const u32 wave = (u32)__builtin_amdgcn_readfirstlane((int)(t >> 6)), lane = t & 63u;
+    const u32 quad = (t & 127u) >> 1, r = t >> 7, X = R + row + (wave & 1u);
+    const TwoStages<F> s64(tw, X), s16(tw, 4u * X + (lane >> 4)), s4(tw, 16u * X + (lane >> 2)), s1(tw, 64u * (R + row + r) + quad);
+    E x[4];
+    {
+        E *l = lds + wave * ROWPAD;
+        const int b = (int)(16u * (lane >> 2) + (lane & 3u)), c = (int)(64u * (lane >> 4) + (lane & 15u));
+        const E *from = (const E *)(wave & 2u ? ca : cb) + 256u * (wave & 1u) + lane;
+#pragma unroll
+        for (int k = 0; k < 4; k++) x[k] = from[64 * k];
+        s64.forward(f, x);
+#pragma unroll
+        for (int k = 0; k < 4; k++) l[padc((int)lane + 64 * k)] = x[k];
+        wave_sync();
+#pragma unroll
+        for (int k = 0; k < 4; k++) x[k] = l[padc(c + 16 * k)];
+        s16.forward(f, x);
+#pragma unroll
+        for (int k = 0; k < 4; k++) l[padc(c + 16 * k)] = x[k];
+        wave_sync();
+#pragma unroll
+        for (int k = 0; k < 4; k++) x[k] = l[padc(b + 4 * k)];
+        s4.forward(f, x);
+#pragma unroll
+        for (int k = 0; k < 4; k++) l[padc(b + 4 * k)] = x[k];
+    }
+    __syncthreads();
+    E *l = lds + (2u * odd + r) * ROWPAD;
+#pragma unroll
+    for (int k = 0; k < 4; k++) x[k] = l[padc((int)(4u * quad) + k)];
+    s1.forward(f, x);
+    // even lanes have a quad of the first polynomial, odd ones of the second: back to a pair of both
+    const E r0 = value_from_next_lane(odd ? x[0] : x[2]), r1 = value_from_next_lane(odd ? x[1] : x[3]);
+    const E b0 = odd ? r0 : x[0], b1 = odd ? r1 : x[1], a0 = odd ? x[2] : r0, a1 = odd ? x[3] : r1;
+    *(ulonglong2 *)(ob + 2 * t) = make_ulonglong2(f.sub_scale(b0, rb[0], cst), f.sub_scale(b1, rb[1], cst));
+    *(ulonglong2 *)(oa + 2 * t) = make_ulonglong2(f.sub_scale(a0, ra[0], cst), f.sub_scale(a1, ra[1], cst));
 }
 
 // Hoisted rotations, several per output, combined with masks in the extended basis:
@@ -309,23 +381,34 @@ __device__ __forceinline__ void rows_of_products(const F f, const u64 (&rb)[2], 
 //                                                         + [pol = 0, j < nq] (P mod q_j) * b_t[j][pi_t(n)] )
 // The automorphism is an index map on the reads (aligned 2^m-blocks map to aligned 2^m-blocks in the
 // bit-reversed order, so a wavefront still reads whole 512-byte runs); the key is streamed once.
-// Limbs in ir.limbs leave as the first pass of their inverse transform (rows_of_products).
+// Limbs in rows.inverse leave as the first pass of their inverse transform (rows_of_products), with a SumTail as results of the
+// ModDown (rows_under_products).
 // MODE 1: the launch covers only limbs of primes below 2^44 (double-precision path); MODE 2: only the others
 // (integer path); MODE 0: any limb, path chosen per workgroup.  jmap lists the n_j limbs of the launch.  The integer
 // path keeps 128-bit accumulators and needs more registers, so on large launches the double-precision limbs get a
 // kernel of their own and run at a higher occupancy; small launches stay whole (two part-filled launches cost more).
-struct InverseRows {
-    u64 limbs;       // bit j: limb j of the extended basis
-    const Tw *tw;    // stage-ordered twiddles of the inverse transforms, [prime][N]
+// what becomes of the sums of a launch's limbs
+struct SumRows {
+    u64 inverse;       // bit j: limb j of the extended basis leaves as the first pass of its inverse transform; the others as they are
+    const Tw *tw;      // stage-ordered twiddles of the inverse transforms, [prime][N]
 };
-template <int MODE, bool COMPACT>
+struct SumTail {       // all limbs of the launch end in the ModDown's tail
+    const u64 *conv;   // [n_out][2][nq_out][N]
+    const Tw *tw;      // stage-ordered twiddles of the forward transforms
+    const Tw *cst;     // per limb: constant and Shoup quotient
+    u64 *out;          // polynomials out_stride apart, or with `listed` two of them at each entry of the list
+    size_t out_stride;
+    int nq_out, listed;
+    ResultList list;
+};
+template <int MODE, bool COMPACT, class ROWS>
 __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict__ terms,
                                                    const u32 *__restrict__ group_off, u64 *__restrict__ y,
                                                    const ModQ *__restrict__ modq, const double *__restrict__ fp,
-                                                   const LimbList &ll, const CstList &pmod, int nq, int E, int beta,
+                                                   const LimbList &ll, const Cst *__restrict__ pmod, int nq, int E, int beta,
                                                    int n_full, int logN, int b_premultiplied, int n_out,
                                                    const LimbList &jmap, int n_j, const u32 *__restrict__ koff,
-                                                   const InverseRows ir) {
+                                                   const ROWS &rows) {
     // A thread owns the residue pair (n, n+1): the automorphism maps an aligned pair to an aligned pair
     // (possibly swapped), so every access is a 16-byte load or store.
     // Work is dealt out by SOURCE chunk.  The automorphism maps aligned 512-coefficient chunks onto aligned
@@ -371,34 +454,46 @@ __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict_
     const int prime = (int)table_byte(ll.idx, j);
     const u32 n = (chunk * 256 + threadIdx.x) * 2;
     const double fq = fp[4 * prime];
+    const KeyLimb kl = key_limb<COMPACT>(koff, prime, logN, n_full);
     const size_t N = (size_t)1 << logN;
     u64 rb[2], ra[2];
     if (MODE == 1 || (MODE == 0 && fq != 0.0 && beta <= 6)) {
         const FpMod f{fq, fp[4 * prime + 1]};
         double fb[2], fa[2];
-        hoisted_pair_fp<COMPACT>(terms, group_off, koff, f, j < nq ? (double)pmod.c[j].w : 0.0, j, o, prime, n, nq, E,
-                                 beta, n_full, logN, b_premultiplied, fb, fa);
+        hoisted_pair_fp<COMPACT>(terms, group_off, kl, f, j < nq ? (double)pmod[j].w : 0.0, j, o, n, nq, E, beta, logN, b_premultiplied,
+                                 fb, fa);
         rb[0] = f.canonical(fb[0]);
         rb[1] = f.canonical(fb[1]);
         ra[0] = f.canonical(fa[0]);
         ra[1] = f.canonical(fa[1]);
     } else {
-        hoisted_pair_int<COMPACT>(terms, group_off, koff, modq[prime], pmod, j, o, prime, n, nq, E, beta, n_full, logN,
-                                  b_premultiplied, rb, ra);
+        hoisted_pair_int<COMPACT>(terms, group_off, kl, modq[prime], pmod, j, o, n, nq, E, beta, logN, b_premultiplied, rb, ra);
     }
-    u64 *yb = y + (((size_t)o * 2 + 0) * E + j) * N, *ya = y + (((size_t)o * 2 + 1) * E + j) * N;
-    if ((ir.limbs >> j) & 1ull) {
-        __shared__ u64 lds[4 * ROWPAD];
-        const u32 first = chunk * 512;
-        const Tw *tw = ir.tw + ((size_t)prime << logN);
-        if (MODE == 1 || (MODE == 0 && fq != 0.0))
-            rows_of_products(FpField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
+    __shared__ u64 lds[4 * ROWPAD];
+    const u32 first = chunk * 512;
+    const bool fp_limb = MODE == 1 || (MODE == 0 && fq != 0.0);
+    if constexpr (std::is_same<ROWS, SumTail>::value) {
+        const u64 *cb = rows.conv + ((size_t)o * 2 * rows.nq_out + j) * N + first, *ca = cb + (size_t)rows.nq_out * N;
+        u64 *ob = (rows.listed ? rows.list.at[o] : rows.out + (size_t)o * 2 * rows.out_stride) + (size_t)j * N + first;
+        u64 *oa = ob + rows.out_stride;
+        const Tw *tw = rows.tw + ((size_t)prime << logN), cst = rows.cst[j];
+        if (fp_limb)
+            rows_under_products(FpField(modq, nullptr, nullptr, fp, prime), rb, ra, cb, ca, ob, oa, lds, tw, logN - 8, 2 * chunk, cst);
         else
-            rows_of_products(IntField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
-        return;
+            rows_under_products(IntFieldT<true>(modq, nullptr, nullptr, fp, prime), rb, ra, cb, ca, ob, oa, lds, tw, logN - 8, 2 * chunk, cst);
+    } else {
+        u64 *yb = y + (((size_t)o * 2 + 0) * E + j) * N, *ya = y + (((size_t)o * 2 + 1) * E + j) * N;
+        if ((rows.inverse >> j) & 1ull) {
+            const Tw *tw = rows.tw + ((size_t)prime << logN);
+            if (fp_limb)
+                rows_of_products(FpField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
+            else
+                rows_of_products(IntField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
+            return;
+        }
+        stream_store2(yb + n, rb[0], rb[1]);
+        stream_store2(ya + n, ra[0], ra[1]);
     }
-    stream_store2(yb + n, rb[0], rb[1]);
-    stream_store2(ya + n, ra[0], ra[1]);
 }
 
 // Term lists of up to HOISTED_ARG_TERMS terms and outputs travel in the kernel arguments (no staging copy before
@@ -409,25 +504,26 @@ struct HoistedArgs {
     RotTermDev t[HOISTED_ARG_TERMS];
     u32 off[HOISTED_ARG_TERMS + 1];
 };
-// Register budget for five waves per SIMD (96 registers): the double-precision form needs 70, the integer and the mixed form
-// 94 - 95, none of them spills.  COMPACT: the key layout of the launch (hoisted.h, key_limb).
+// Register budget for five waves per SIMD (96 registers): the double-precision form needs 72, the integer and the mixed form
+// all 96.  The mixed form under a ModDown's tail spills three; with four waves and none a product at level 9 takes 122.1 instead of
+// 120.2 us, the projection of a 768-wide layer 10.46 instead of 10.33 ms.  COMPACT: the key layout of the launch (hoisted.h, key_limb).
 #define HOISTED_KERNEL __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void
-template <int MODE, bool COMPACT>
+template <int MODE, bool COMPACT, class ROWS>
 HOISTED_KERNEL hoisted_terms_kernel(const HoistedArgs args, u64 *__restrict__ y, const ModQ *__restrict__ modq,
-                                    const double *__restrict__ fp, LimbList ll, CstList pmod, int nq, int E, int beta,
+                                    const double *__restrict__ fp, LimbList ll, const Cst *__restrict__ pmod, int nq, int E, int beta,
                                     int n_full, int logN, int b_premultiplied, int n_out, LimbList jmap, int n_j,
-                                    const u32 *__restrict__ koff, const InverseRows ir) {
+                                    const u32 *__restrict__ koff, const ROWS rows) {
     hoisted_terms_body<MODE, COMPACT>(args.t, args.off, y, modq, fp, ll, pmod, nq, E, beta, n_full, logN,
-                                      b_premultiplied, n_out, jmap, n_j, koff, ir);
+                                      b_premultiplied, n_out, jmap, n_j, koff, rows);
 }
-template <int MODE, bool COMPACT>
+template <int MODE, bool COMPACT, class ROWS>
 HOISTED_KERNEL hoisted_terms_list_kernel(const RotTermDev *__restrict__ terms, const u32 *__restrict__ group_off,
                                          u64 *__restrict__ y, const ModQ *__restrict__ modq,
-                                         const double *__restrict__ fp, LimbList ll, CstList pmod, int nq, int E,
+                                         const double *__restrict__ fp, LimbList ll, const Cst *__restrict__ pmod, int nq, int E,
                                          int beta, int n_full, int logN, int b_premultiplied, int n_out, LimbList jmap,
-                                         int n_j, const u32 *__restrict__ koff, const InverseRows ir) {
+                                         int n_j, const u32 *__restrict__ koff, const ROWS rows) {
     hoisted_terms_body<MODE, COMPACT>(terms, group_off, y, modq, fp, ll, pmod, nq, E, beta, n_full, logN,
-                                      b_premultiplied, n_out, jmap, n_j, koff, ir);
+                                      b_premultiplied, n_out, jmap, n_j, koff, rows);
 }
 #undef HOISTED_KERNEL
 
@@ -698,6 +794,7 @@ struct KsTables {
     // conversion follows it.  modup: per chain length nq, limbs 0 .. nq-1 (each limb in its own digit's basis).
     size_t p_invn_off = 0;
     std::vector<size_t> drop_invn_off, modup_invn_off;   // [nq]
+    size_t pmod_off = 0;                                 // P mod q_j for the chain primes
     size_t ones_off = 0;                                 // the constant 1 for every prime (a one-source conversion
                                                          // with it is a plain reduction into the target prime)
 };
@@ -822,6 +919,12 @@ static void build_tables(const hemm_context *c, KsTables &t) {
             for (int j = d * alpha; j < std::min(nq, (d + 1) * alpha); j++) src.push_back(j);
             invn(t.inv_off[nq][d], src);
         }
+    }
+    t.pmod_off = t.host.size();
+    for (int j = 0; j < nQ; j++) {
+        u64 q = c->primes[j], P = 1;
+        for (int k = 0; k < K; k++) P = h_mulmod(P, c->primes[nQ + k] % q, q);
+        t.host.push_back(Cst{P, shoup_h(P, q)});
     }
     t.ones_off = t.host.size();
     for (int pj = 0; pj < T; pj++) t.host.push_back(Cst{1, 0});
@@ -1028,9 +1131,8 @@ void launch_keyswitch(hemm_context *c, const u64 *in, const u64 *evk, int nq, u6
             n_terms = 2;
         }
         const u32 off[2] = {0, (u32)n_terms};
-        const u64 rows = moddown_rows_in_sum(c, nq, 1, 0);
-        launch_hoisted_terms_args(c, term, n_terms, off, 1, nq, acc, false, s, rows);
-        launch_moddown_batch(c, acc, nq, 2, 0, out, out_stride, coef, s, false, nullptr, rows != 0);
+        launch_hoisted_moddown(c, HoistedList{term, off, nullptr, nullptr, n_terms}, 1, nq, acc, false, 0, out, out_stride, nullptr,
+                               coef, s);
         return;
     }
     launch_inner_product(c, in, ext, evk, nq, acc, s);
@@ -1382,141 +1484,79 @@ static size_t hoisted_bytes(const hemm_context *c, const RotTermDev *t, int n_te
     return bytes;
 }
 
-// terms / group_off are DEVICE arrays (n_out + 1 offsets); y: [n_out][2][nq+K][N]
-// P mod q_j (and Shoup quotient) for the chain limbs j < nq
-static CstList p_mod_chain(const hemm_context *c, int nq) {
-    CstList pm;
-    memset(&pm, 0, sizeof(pm));
-    for (int j = 0; j < nq; j++) {
-        u64 q = c->primes[j], P = 1;
-        for (int k = 0; k < c->nP; k++) P = h_mulmod(P, c->primes[c->nQ + k] % q, q);
-        pm.c[j] = Cst{P, shoup_h(P, q)};
-    }
-    return pm;
-}
-
-// Limbs of the extended basis handled in double precision (primes below 2^44, at most 6 digits) and the others;
-// true when the launch is large enough (in workgroups) for one kernel per kind to pay.
-static bool split_limbs(const hemm_context *c, int nq, int beta, int n_out, LimbList &fpl, int &n_fp, LimbList &il,
-                        int &n_int, LimbList &all) {
-    const LimbList ll = limbs_default(c, nq, 1);
-    const int E = nq + c->nP;
-    memset(&fpl, 0, sizeof(fpl));
-    memset(&il, 0, sizeof(il));
-    n_fp = n_int = 0;
-    for (int j = 0; j < HEMM_MAX_PRIMES; j++) all.idx[j] = (uint8_t)j;
-    for (int j = 0; j < E; j++) {
-        if (c->primes[ll.idx[j]] < (1ull << 44) && beta <= 6)
-            fpl.idx[n_fp++] = (uint8_t)j;
-        else
-            il.idx[n_int++] = (uint8_t)j;
-    }
-    return n_fp > 0 && n_int > 0 && (size_t)n_out * E * (c->N / 512) >= 16384;
-}
-
-void launch_hoisted_terms(hemm_context *c, const void *terms_dev, const u32 *group_off_dev, int n_out, int nq, u64 *y,
-                          bool b_premultiplied, hipStream_t s, const void *terms_host, int n_terms, bool compact, u64 inverse_rows) {
-    const InverseRows ir{inverse_rows, (const Tw *)c->d_iw};
-    const int K = c->nP, E = nq + K, beta = (nq + c->alpha - 1) / c->alpha;
-    if (terms_host != nullptr) account(c, TR_KEYPROD, hoisted_bytes(c, (const RotTermDev *)terms_host, n_terms, n_out, nq));
-    const CstList pm = p_mod_chain(c, nq);
+int hoisted_arg_capacity() { return HOISTED_ARG_TERMS; }
+// The sums of outputs first .. first + n_out for the n_j limbs in jl of the extended basis.  Limbs handled in double precision (primes
+// below 2^44, at most 6 digits) and the others take a kernel each where the launch is large enough (in workgroups) for that to pay.
+template <class ROWS>
+static void sum_limbs(hemm_context *c, const HoistedList &l, int first, int n_out, int nq, u64 *y, bool b_premultiplied,
+                      const LimbList &jl, int n_j, const ROWS &rows, hipStream_t s) {
+    const int E = nq + c->nP, beta = (nq + c->alpha - 1) / c->alpha, n_full = c->nQ + c->nP, pre = b_premultiplied ? 1 : 0;
+    const bool compact = l.n_terms > 0 && (((const RotTermDev *)l.terms)[0].flags & ROT_TERM_COMPACT_KEY) != 0;
     if (c->N < 512) throw std::invalid_argument("hoisted terms need N >= 512");
     // with more than 6 digits the limbs of primes below 2^44 go through the integer path, which reads whole words
     if (compact && beta > 6) throw std::invalid_argument("compact keys need at most 6 digits");
     // the kernels address a key by 32-bit byte offsets
     if ((size_t)c->dnum * 2 * (c->nQ + c->nP) * c->N * 8 >= ((size_t)1 << 32))
         throw std::invalid_argument("hoisted terms need keys below 4 GiB");
-    LimbList fpl, il, all;
-    int n_fp, n_int;
-    const bool split = split_limbs(c, nq, beta, n_out, fpl, n_fp, il, n_int, all);
-    const dim3 block(256);
-    const size_t per_limb = (size_t)n_out * (c->N / 512);
-    const LimbList ll = limbs_default(c, nq, 1);
-    const RotTermDev *td = (const RotTermDev *)terms_dev;
-    const int n_full = c->nQ + c->nP, pre = b_premultiplied ? 1 : 0;
-#define HOISTED_LIST(MODE, COMPACT, GRID, JM, NJ)                                                                  \
-    hipLaunchKernelGGL((hoisted_terms_list_kernel<MODE, COMPACT>), dim3((unsigned)(GRID)), block, 0, s, td,        \
-                       group_off_dev, y, c->d_modq, c->d_fp, ll, pm, nq, E, beta, n_full, c->logN, pre, n_out, JM, \
-                       NJ, c->d_key_off, ir)
-    if (!split) {
-        if (compact)
-            HOISTED_LIST(0, true, per_limb * E, all, E);
-        else
-            HOISTED_LIST(0, false, per_limb * E, all, E);
-        return;
-    }
-    if (compact) {
-        HOISTED_LIST(1, true, per_limb * n_fp, fpl, n_fp);
-        HOISTED_LIST(2, true, per_limb * n_int, il, n_int);
-    } else {
-        HOISTED_LIST(1, false, per_limb * n_fp, fpl, n_fp);
-        HOISTED_LIST(2, false, per_limb * n_int, il, n_int);
-    }
-#undef HOISTED_LIST
-}
-// the same with the term list (host memory, already merged: n_terms <= HOISTED_ARG_TERMS, n_out <= HOISTED_ARG_TERMS)
-// passed in the kernel arguments
-int hoisted_arg_capacity() { return HOISTED_ARG_TERMS; }
-void launch_hoisted_terms_args(hemm_context *c, const void *terms_host, int n_terms, const u32 *group_off_host, int n_out,
-                               int nq, u64 *y, bool b_premultiplied, hipStream_t s, u64 inverse_rows) {
-    const InverseRows ir{inverse_rows, (const Tw *)c->d_iw};
-    const int K = c->nP, E = nq + K, beta = (nq + c->alpha - 1) / c->alpha;
-    const CstList pm = p_mod_chain(c, nq);
-    if (c->N < 512) throw std::invalid_argument("hoisted terms need N >= 512");
-    if (n_terms > HOISTED_ARG_TERMS || n_out > HOISTED_ARG_TERMS)
-        throw std::invalid_argument("term list too long for the argument path");
-    account(c, TR_KEYPROD, hoisted_bytes(c, (const RotTermDev *)terms_host, n_terms, n_out, nq));
     HoistedArgs a;
-    memset(&a, 0, sizeof(a));
-    memcpy(a.t, terms_host, (size_t)n_terms * sizeof(RotTermDev));
-    memcpy(a.off, group_off_host, (size_t)(n_out + 1) * sizeof(u32));
-    LimbList fpl, il, all;
-    int n_fp, n_int;
-    const bool split = split_limbs(c, nq, beta, n_out, fpl, n_fp, il, n_int, all);
-    const dim3 block(256);
-    const size_t per_limb = (size_t)n_out * (c->N / 512);
+    if (l.terms_dev == nullptr) {
+        if (first != 0 || l.n_terms > HOISTED_ARG_TERMS || n_out > HOISTED_ARG_TERMS)
+            throw std::invalid_argument("term list too long for the argument path");
+        memset(&a, 0, sizeof(a));
+        memcpy(a.t, l.terms, (size_t)l.n_terms * sizeof(RotTermDev));
+        memcpy(a.off, l.offsets, (size_t)(n_out + 1) * sizeof(u32));
+    }
     const LimbList ll = limbs_default(c, nq, 1);
-    const int n_full = c->nQ + c->nP, pre = b_premultiplied ? 1 : 0;
-    const bool compact = n_terms > 0 && (((const RotTermDev *)terms_host)[0].flags & ROT_TERM_COMPACT_KEY) != 0;
-    if (compact && beta > 6) throw std::invalid_argument("compact keys need at most 6 digits");
-    if ((size_t)c->dnum * 2 * (c->nQ + c->nP) * c->N * 8 >= ((size_t)1 << 32))
-        throw std::invalid_argument("hoisted terms need keys below 4 GiB");
-#define HOISTED_ARGS(MODE, COMPACT, GRID, JM, NJ)                                                                  \
-    hipLaunchKernelGGL((hoisted_terms_kernel<MODE, COMPACT>), dim3((unsigned)(GRID)), block, 0, s, a, y, c->d_modq, \
-                       c->d_fp, ll, pm, nq, E, beta, n_full, c->logN, pre, n_out, JM, NJ, c->d_key_off, ir)
-    if (!split) {
-        if (compact)
-            HOISTED_ARGS(0, true, per_limb * E, all, E);
-        else
-            HOISTED_ARGS(0, false, per_limb * E, all, E);
-        return;
+    const Cst *pm = g_tables_of(c)->dev + g_tables_of(c)->pmod_off;
+    LimbList kind[2];   // double precision, integers
+    int n_kind[2] = {0, 0};
+    memset(kind, 0, sizeof(kind));
+    for (int i = 0; i < n_j; i++) {
+        const int k = c->primes[ll.idx[jl.idx[i]]] < (1ull << 44) && beta <= 6 ? 0 : 1;
+        kind[k].idx[n_kind[k]++] = jl.idx[i];
     }
-    if (compact) {
-        HOISTED_ARGS(1, true, per_limb * n_fp, fpl, n_fp);
-        HOISTED_ARGS(2, true, per_limb * n_int, il, n_int);
+    const size_t per_limb = (size_t)n_out * (c->N / 512);
+#define SUM_FORM(MODE, COMPACT, JM, NJ)                                                                                        \
+    do {                                                                                                                       \
+        const dim3 grid((unsigned)(per_limb * (NJ)));                                                                          \
+        if (l.terms_dev != nullptr)                                                                                            \
+            hipLaunchKernelGGL((hoisted_terms_list_kernel<MODE, COMPACT, ROWS>), grid, dim3(256), 0, s,                        \
+                               (const RotTermDev *)l.terms_dev, l.offsets_dev + first, y, c->d_modq, c->d_fp, ll, pm, nq, E,   \
+                               beta, n_full, c->logN, pre, n_out, JM, NJ, c->d_key_off, rows);                                 \
+        else                                                                                                                   \
+            hipLaunchKernelGGL((hoisted_terms_kernel<MODE, COMPACT, ROWS>), grid, dim3(256), 0, s, a, y, c->d_modq, c->d_fp,   \
+                               ll, pm, nq, E, beta, n_full, c->logN, pre, n_out, JM, NJ, c->d_key_off, rows);                  \
+    } while (0)
+#define SUM_LIMBS(MODE, JM, NJ)                   \
+    do {                                          \
+        if (compact) SUM_FORM(MODE, true, JM, NJ); \
+        else SUM_FORM(MODE, false, JM, NJ);       \
+    } while (0)
+    if (n_kind[0] == 0 || n_kind[1] == 0 || per_limb * n_j < 16384) {
+        SUM_LIMBS(0, jl, n_j);
     } else {
-        HOISTED_ARGS(1, false, per_limb * n_fp, fpl, n_fp);
-        HOISTED_ARGS(2, false, per_limb * n_int, il, n_int);
+        SUM_LIMBS(1, kind[0], n_kind[0]);
+        SUM_LIMBS(2, kind[1], n_kind[1]);
     }
-#undef HOISTED_ARGS
+#undef SUM_LIMBS
+#undef SUM_FORM
 }
 
-// The limbs of the extended basis whose inverse row pass belongs into the hoisted sum in front of a ModDown of n_out results (0: none):
-// all that it drops, where their inverse transform is two launches.
-u64 moddown_rows_in_sum(const hemm_context *c, int nq, int n_out, int drop_last) {
-    const int first = drop_last ? nq - 1 : nq, E = nq + c->nP;
-    if (first < 0 || E > 64 || c->logN < 13 || one_launch(c, (size_t)2 * n_out * (E - first), true)) return 0;
-    u64 limbs = 0;
-    for (int j = first; j < E; j++) limbs |= 1ull << j;
-    return limbs;
+// y: [n_out][2][nq+K][N]
+void launch_hoisted_terms(hemm_context *c, const HoistedList &l, int n_out, int nq, u64 *y, bool b_premultiplied, hipStream_t s) {
+    account(c, TR_KEYPROD, hoisted_bytes(c, (const RotTermDev *)l.terms, l.n_terms, n_out, nq));
+    LimbList all;
+    for (int j = 0; j < HEMM_MAX_PRIMES; j++) all.idx[j] = (uint8_t)j;
+    sum_limbs(c, l, 0, n_out, nq, y, b_premultiplied, all, nq + c->nP, SumRows{0, nullptr}, s);
 }
 
 // y: [n_polys][nq+K][N] NTT (dropped limbs are clobbered).  drop_last = 0: out[p] = y[p] / P over nq limbs;
 // drop_last = 1: out[p] = y[p] / (P q_{nq-1}) over nq-1 limbs (ModDown and rescale in one conversion).
 // conv: workspace [n_polys][nq_out][N].  list: the results lie where it says.
-// rows_done: the dropped limbs are what rows_of_products leaves.
+// rows_done: the dropped limbs are what rows_of_products leaves; cols_only: stop after the first pass of the converted limbs' transform,
+// for rows_under_products.
 void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop_last, u64 *out, size_t out_stride,
-                          u64 *conv, hipStream_t s, bool slab, const ResultList *list, bool rows_done) {
+                          u64 *conv, hipStream_t s, bool slab, const ResultList *list, bool rows_done, bool cols_only) {
     KsTables *t = g_tables_of(c);
     const int K = c->nP, E = nq + K, nq_out = drop_last ? nq - 1 : nq;
     const size_t N = c->N;
@@ -1592,15 +1632,107 @@ void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop
         LimbList cl = limbs_default(c, nq_out, 0), ident;
         for (int j = 0; j < HEMM_MAX_PRIMES; j++) ident.idx[j] = (uint8_t)j;
         if (launch_ntt_converted(c, cs, conv, cl, ident, nq_out, n_polys, (size_t)nq_out * N, s, y, (size_t)E * N, out,
-                                 out_stride, cst_dev, list))
+                                 out_stride, cst_dev, list, cols_only))
             return;
     }
+    if (cols_only) throw std::invalid_argument("this ModDown's conversion has a pass of its own");
     launch_bconv(c, a, c->d_modq, (int)N, n_polys, s);
     if (launch_ntt_sub_scale(c, conv, nq_out, n_polys, y, (size_t)E * N, out, out_stride, cst_dev, s, list)) return;
     launch_ntt(c, conv, limbs_default(c, nq_out, 0), nq_out, n_polys, (size_t)nq_out * N, false, s);
     CstList cl;
     for (int j = 0; j < nq_out; j++) cl.c[j] = drop_last ? t->dropinv[nq][j] : t->pinv[j];
     sub_scale(c, y, (size_t)E * N, conv, cl, nq_out, n_polys, out, out_stride, list, s);
+}
+
+
+// Whether a sum that a ModDown follows can leave the limbs it keeps to the end: nothing it reads may lie where the ModDown writes
+// before then (a result that replaces an operand), and results are written as pairs of residues.
+static bool tail_may_sum(const HoistedList &l, int n_out, size_t N, int nq, int E, int beta, size_t key_words, const u64 *out,
+                         size_t out_stride, u64 *const *outs, const u64 *conv, size_t conv_words, int nq_out) {
+    typedef std::pair<uintptr_t, uintptr_t> Range;
+    std::vector<Range> written;
+    written.reserve(n_out + 1);
+    auto range = [](const u64 *p, size_t words) { return Range((uintptr_t)p, (uintptr_t)(p + words)); };
+    if (out_stride % 2 != 0) return false;
+    for (int o = 0; o < n_out; o++) {
+        const u64 *at = outs != nullptr ? outs[o] : out + (size_t)o * 2 * out_stride;
+        if ((uintptr_t)at % 16 != 0) return false;
+        written.push_back(range(at, out_stride + (size_t)nq_out * N));
+    }
+    written.push_back(range(conv, conv_words));
+    std::sort(written.begin(), written.end());
+    auto apart = [&](const u64 *p, size_t words) {
+        if (p == nullptr) return true;
+        const Range r = range(p, words);
+        auto it = std::upper_bound(written.begin(), written.end(), Range(r.first, UINTPTR_MAX));
+        if (it != written.end() && it->first < r.second) return false;
+        // ranges written may not overlap each other, so only the last one that begins before can reach into this one
+        return it == written.begin() || std::prev(it)->second <= r.first;
+    };
+    for (size_t i = 1; i < written.size(); i++)
+        if (written[i].first < written[i - 1].second) return false;
+    const RotTermDev *t = (const RotTermDev *)l.terms, none{};
+    for (int i = 0; i < l.n_terms; i++) {
+        const RotTermDev &last = i > 0 ? t[i - 1] : none;   // terms share most of what they read
+        const size_t mask_words = t[i].mask_shift ? (size_t)E * 2 * (N >> t[i].mask_shift) : (size_t)E * N;
+        const size_t ext_words = (size_t)(t[i].evk == nullptr ? nq : beta * E) * N;
+        if ((t[i].ext != last.ext || t[i].evk == nullptr || last.evk == nullptr) && !apart(t[i].ext, ext_words)) return false;
+        if (t[i].ext2 != last.ext2 && !apart(t[i].ext2, (size_t)beta * E * N)) return false;
+        if (t[i].b != last.b && !apart(t[i].b, (size_t)nq * N)) return false;
+        if (t[i].b2 != last.b2 && !apart(t[i].b2, (size_t)nq * N)) return false;
+        if (!apart(t[i].evk, key_words) || !apart(t[i].mask, mask_words) || !apart(t[i].mask2, mask_words)) return false;
+        if (!apart(t[i].pt, (size_t)E * N)) return false;
+    }
+    return true;
+}
+
+// A hoisted sum and the ModDown of its results.  Where the transforms are two launches each, the sum is split between the passes at
+// either end of the ModDown: the limbs it drops leave as the first pass of their inverse transform (rows_of_products), those it
+// keeps are summed under the last pass of the converted limbs' (rows_under_products).
+void launch_hoisted_moddown(hemm_context *c, const HoistedList &l, int n_out, int nq, u64 *y, bool b_premultiplied, int drop_last, u64 *out,
+                            size_t out_stride, u64 *const *outs, u64 *conv, hipStream_t s) {
+    const int K = c->nP, E = nq + K, nq_out = drop_last ? nq - 1 : nq, ns = E - nq_out, beta = (nq + c->alpha - 1) / c->alpha;
+    const size_t N = c->N;
+    const int group = outs != nullptr ? std::min(n_out, RESULT_PARTS) : n_out;
+    const bool rows = nq_out > 0 && E <= HEMM_MAX_PRIMES && c->logN >= 13 && !one_launch(c, (size_t)2 * group * ns, true);
+    // What the split costs is a second wait for the terms, one after the other, in a launch that has less to fill it with.  One launch
+    // / split, us (7 + 4 limbs of 42 bits, and 9 + 4 of 60, one dropped with the special ones; workgroups of the whole sum):
+    //   1 term an output    160   704        1408        1664        2816        5632        11264       22528
+    //                 26.5/26.7   32.6/32.8  41.9/40.9   47.4/46.5   57.2/56.3   87.7/83.3   148.7/146.8 276/248
+    //   7 terms             320   704        1408        1664        2816        3328        5632        11264
+    //                 46.3/63.8   55.5/54.6  79.8/82.0   98.3/103    128.5/127.5 158/162     225/217     435/418
+    // (rotation at N = 2^13, 128 workgroups: 45.0/47.4; on 24 primes of 60 bits, level 20, 3200: 147.2/144.1)
+    const size_t wgs = (size_t)n_out * E * (N / 512);
+    const bool tail = rows && (wgs >= 4096 || (wgs >= 1024 && l.n_terms <= 2 * n_out)) && ns <= CONV_MAX_SOURCES && lazy_dot_ok(c) && !one_launch(c, (size_t)2 * group * nq_out, false) &&
+                      (size_t)2 * group * nq_out <= 65535 &&
+                      tail_may_sum(l, n_out, N, nq, E, beta, (size_t)c->dnum * 2 * (c->nQ + K) * N, out, out_stride, outs, conv,
+                                   (size_t)n_out * 2 * nq_out * N, nq_out);
+    account(c, TR_KEYPROD, hoisted_bytes(c, (const RotTermDev *)l.terms, l.n_terms, n_out, nq));
+    LimbList all, dropped, kept;
+    memset(&dropped, 0, sizeof(dropped));
+    for (int j = 0; j < HEMM_MAX_PRIMES; j++) all.idx[j] = kept.idx[j] = (uint8_t)j;
+    SumRows sr{0, (const Tw *)c->d_iw};
+    for (int i = 0; i < ns; i++) dropped.idx[i] = (uint8_t)(nq_out + i);
+    for (int j = nq_out; rows && j < E; j++) sr.inverse |= 1ull << j;
+    if (tail)
+        sum_limbs(c, l, 0, n_out, nq, y, b_premultiplied, dropped, ns, sr, s);
+    else
+        sum_limbs(c, l, 0, n_out, nq, y, b_premultiplied, all, E, sr, s);
+    for (int o = 0; o < n_out; o += group) {
+        const int n = std::min(n_out - o, group);
+        ResultList list{};
+        for (int i = 0; outs != nullptr && i < n; i++) list.at[i] = outs[o + i];
+        u64 *yo = y + (size_t)o * 2 * E * N, *co = conv + (size_t)o * 2 * nq_out * N;
+        const bool listed = outs != nullptr && n > 1;
+        u64 *to = outs != nullptr ? outs[o] : out;
+        launch_moddown_batch(c, yo, nq, 2 * n, drop_last, to, out_stride, co, s, false, listed ? &list : nullptr, rows, tail);
+        if (!tail) continue;
+        KsTables *t = g_tables_of(c);
+        SumTail st{co, (const Tw *)c->d_w, (const Tw *)(t->dev + (drop_last ? t->dropinv_off[nq] : t->pinv_off)), to, out_stride, nq_out,
+                   listed ? 1 : 0, list};
+        account(c, TR_KEYPROD, 0);
+        sum_limbs(c, l, o, n, nq, nullptr, b_premultiplied, kept, nq_out, st, s);
+    }
 }
 
 

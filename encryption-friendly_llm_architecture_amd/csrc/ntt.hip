@@ -654,7 +654,7 @@ bool launch_ntt_sub_scale(const hemm_context *c, u64 *data, int n_limbs, int n_p
 bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *data, const LimbList &ll, const LimbList &sl,
                           int n_limbs, int n_polys, size_t poly_stride, hipStream_t s, const u64 *ep_minuend,
                           size_t ep_minuend_stride, u64 *ep_out, size_t ep_out_stride, const void *ep_cst_dev,
-                          const ResultList *ep_list) {
+                          const ResultList *ep_list, bool cols_only) {
     if (!ring_has_fused_forms(c)) return false;
     if (n_limbs > HEMM_MAX_PRIMES || cs.n_copy < 0 || cs.n_copy > HEMM_MAX_PRIMES)
         throw std::invalid_argument("too many limbs in one converted transform");
@@ -679,7 +679,8 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
         return false;   // more workgroup rows than one launch holds: the caller converts and transforms separately
     account(c, TR_BCONV, (src_limbs + 2 * (size_t)cs.n_copy) * n_polys * c->N * 8, 0);
     const bool one = one_launch(c, (size_t)n_limbs * n_polys, false);
-    account(c, TR_NTT, (size_t)(tail ? 2 : 1) * n_limbs * n_polys * c->N * 8, one ? 1 : 2);
+    if (one && cols_only) throw std::invalid_argument("a transform in one launch has no passes");
+    account(c, TR_NTT, (size_t)(tail ? 2 : 1) * n_limbs * n_polys * c->N * 8, one || cols_only ? 1 : 2);
     if (one) {
         launch_limb_forward(c, data, ll, sl, n_limbs, n_polys, poly_stride, s, &cs, nullptr,
                             sub_scale_tail(ep_minuend, ep_minuend_stride, ep_out, ep_out_stride, ep_cst_dev),
@@ -704,6 +705,7 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
     }
 #undef CONV_RING
 #undef CONV_CASE
+    if (cols_only) return true;
     rows_pass(c, false, data, ll, sl, n_limbs, n_polys, poly_stride, s,
               sub_scale_tail(ep_minuend, ep_minuend_stride, ep_out, ep_out_stride, ep_cst_dev), tail ? TAIL_SUB_SCALE : TAIL_NONE,
               LOAD_PLAIN, ep_list);
