@@ -147,104 +147,257 @@ __device__ __forceinline__ ulonglong2 key_pair_ptr(const RotTermDev &T, const u3
 }
 typedef u32 u32x3 __attribute__((ext_vector_type(3), aligned(4)));
 
-// One term with two masked sources under one key (integer path): residues (n, n+1) of limb j of
-// <z, evk> + P (mask b + mask2 b2) with z_d = mask * x_d + mask2 * x2_d, canonical.  RUNS: the masks are run tables,
-// i.e. constants with a Shoup companion: no wide product and no Barrett step for z_d; a plaintext factor of the term is
-// then left to the caller, which multiplies the finished pair by it.
-template <bool RUNS>
-__device__ __forceinline__ void two_source_int(const RotTermDev &T, const KeyLimb kl, const ModQ m,
-                                               const Cst *__restrict__ pmod, const int j,
-                                               const u32 n, const u32 base, const bool swap, int nq,
-                                               int E, int beta, int logN, int b_premultiplied,
-                                               u64 (&rb)[2], u64 (&ra)[2]) {
-    const size_t N = (size_t)1 << logN;
-    ulonglong2 m1, m2;   // RUNS: (value, companion) of each mask; otherwise the mask residues of the pair
-    if (RUNS) {
-        m1 = load_mask_run(T.mask, T.mask_shift, j, n, logN);
-        m2 = load_mask_run(T.mask2, T.mask_shift, j, n, logN);
-    } else {
-        m1 = load_mask2(T.mask, T.mask_shift, j, n, logN);
-        m2 = load_mask2(T.mask2, T.mask_shift, j, n, logN);
-        if (T.pt != nullptr) {
-            const ulonglong2 pv = load_rotated2(T.pt, T.pt_galois, j, n, logN);
-            m1.x = mulmod_u(m1.x, pv.x, m);
-            m1.y = mulmod_u(m1.y, pv.y, m);
-            m2.x = mulmod_u(m2.x, pv.x, m);
-            m2.y = mulmod_u(m2.y, pv.y, m);
+__device__ __forceinline__ void swap_if(const bool swap, ulonglong2 &v) {
+    if (swap) {
+        const u64 t = v.x;
+        v.x = v.y;
+        v.y = t;
+    }
+}
+// The integer path for primes below 2^60 and B = 1, 2, 3 digits, the usual case.  The 60-bit half of a sum with a plaintext factor per
+// term is bound by instructions, every other one by the trips to memory of its loads.  Products in pieces (modarith.h, Acc3) and
+// values that stay below a few multiples of q until something needs less take 590 instead of 680 vector instructions per
+// two-source term and pair of residues; that alone gained nothing (440 -> 424 us for this sum, 1 - 2 % lost elsewhere).  With all loads of
+// a term in front of its first product, which the registers of the pieces' sums leave room for: pair-layout plaintext product
+// 1513 -> 1428 us, product of two encrypted matrices 2530 -> 2478, projection of a 768-wide layer 10.33 -> 10.08 ms, rotation on 24
+// primes of 60 bits, level 20 144 -> 141.4 us.  (The same order of loads in the double-precision path below: 0.5 % of the projection
+// won, 0.5 % of an attention block and 3 us of the rotation, whose code it is not, lost; not taken.)  Sums of terms lie below 8q.
+struct TermAt {      // where a thread finds what a term reads
+    size_t N;
+    u32 n, base;
+    int j, E;
+    bool swap;
+    __device__ __forceinline__ ulonglong2 source(const u64 *ext, const int d) const { return load2(ext + ((size_t)d * E + j) * N + base); }
+    __device__ __forceinline__ ulonglong2 chain(const u64 *b) const { return load2(b + (size_t)j * N + base); }
+};
+// two masked sources under one key: z_d = mask * x_d + mask2 * x2_d, then one pass over the key.  RUNS: the masks are run tables, i.e.
+// constants with a Shoup companion.  rb < 7q, ra < 3q.
+template <int B, bool RUNS>
+__device__ __forceinline__ void pieces_two(const RotTermDev &T, const KeyLimb kl, const ModQ m, const Cst pmod, const TermAt at, const int nq,
+                                           const int logN, const int b_premultiplied, u64 (&rb)[2], u64 (&ra)[2]) {
+    const u64 q = m.q;
+    ulonglong2 x[B], x2[B], kb[B], ka[B], b, b2;
+    const ulonglong2 m1 = RUNS ? load_mask_run(T.mask, T.mask_shift, at.j, at.n, logN) : load_mask2(T.mask, 0, at.j, at.n, logN);
+    const ulonglong2 m2 = RUNS ? load_mask_run(T.mask2, T.mask_shift, at.j, at.n, logN) : load_mask2(T.mask2, 0, at.j, at.n, logN);
+#pragma unroll
+    for (int d = 0; d < B; d++) {
+        x[d] = at.source(T.ext, d);
+        x2[d] = at.source(T.ext2, d);
+        kb[d] = key_pair_ptr(T, kl.of(d, 0), at.n);
+        ka[d] = key_pair_ptr(T, kl.of(d, 1), at.n);
+    }
+    // mask * v + mask2 * v2 for v < 2q, below 4q
+    auto masked = [&](const u64 v, const u64 v2, const int h) -> u64 {
+        if (RUNS) return mul_shoup_lazy_u(v, m1.x, m1.y, q) + mul_shoup_lazy_u(v2, m2.x, m2.y, q);
+        Acc3 z{0, 0, 0};
+        acc_mul(z, pieces(v), pieces(h ? m1.y : m1.x));
+        acc_mul(z, pieces(v2), pieces(h ? m2.y : m2.x));
+        return acc_reduce(z, m);
+    };
+    Acc3 sb[2] = {{0, 0, 0}, {0, 0, 0}}, sa[2] = {{0, 0, 0}, {0, 0, 0}};
+#pragma unroll
+    for (int d = 0; d < B; d++) {
+        swap_if(at.swap, x[d]);
+        swap_if(at.swap, x2[d]);
+        u64 z[2] = {cond_sub_u(masked(x[d].x, x2[d].x, 0), 2 * q), cond_sub_u(masked(x[d].y, x2[d].y, 1), 2 * q)};
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            if (B > 2) z[h] = cond_sub_u(z[h], q);   // products of two digits sum to less than 4 q^2 as they are
+            acc_mul(sb[h], pieces(z[h]), pieces(h ? kb[d].y : kb[d].x));
+            acc_mul(sa[h], pieces(z[h]), pieces(h ? ka[d].y : ka[d].x));
         }
     }
+    if (at.j < nq) {
+        b = at.chain(T.b);
+        b2 = at.chain(T.b2);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        rb[h] = acc_reduce(sb[h], m);
+        ra[h] = acc_reduce(sa[h], m);
+    }
+    if (at.j < nq) {
+        swap_if(at.swap, b);
+        swap_if(at.swap, b2);
+        if (!b_premultiplied) {
+            b.x = mul_shoup_lazy_u(b.x, pmod.w, pmod.ws, q);
+            b.y = mul_shoup_lazy_u(b.y, pmod.w, pmod.ws, q);
+            b2.x = mul_shoup_lazy_u(b2.x, pmod.w, pmod.ws, q);
+            b2.y = mul_shoup_lazy_u(b2.y, pmod.w, pmod.ws, q);
+        }
+        rb[0] += masked(b.x, b2.x, 0);
+        rb[1] += masked(b.y, b2.y, 1);
+    }
+}
+// one source: rb < 5q, ra < 3q
+template <int B>
+__device__ __forceinline__ void pieces_one(const RotTermDev &T, const KeyLimb kl, const ModQ m, const Cst pmod, const TermAt at, const int nq,
+                                           const bool ext_as_is, const int b_premultiplied, u64 (&rb)[2], u64 (&ra)[2]) {
+    const u64 q = m.q;
+    ulonglong2 x[B], kb[B], ka[B], b;
+    const u32 from = ext_as_is ? at.n : at.base;
+    const bool swap = at.swap && !ext_as_is, with_b = at.j < nq && T.b != nullptr;
+#pragma unroll
+    for (int d = 0; d < B; d++) {
+        x[d] = load2(T.ext + ((size_t)d * at.E + at.j) * at.N + from);
+        kb[d] = key_pair_ptr(T, kl.of(d, 0), at.n);
+        ka[d] = key_pair_ptr(T, kl.of(d, 1), at.n);
+    }
+    if (with_b) b = at.chain(T.b);
+    Acc3 sb[2] = {{0, 0, 0}, {0, 0, 0}}, sa[2] = {{0, 0, 0}, {0, 0, 0}};
+#pragma unroll
+    for (int d = 0; d < B; d++) {
+        swap_if(swap, x[d]);
+        const Pieces px = pieces(x[d].x), py = pieces(x[d].y);
+        acc_mul(sb[0], px, pieces(kb[d].x));
+        acc_mul(sb[1], py, pieces(kb[d].y));
+        acc_mul(sa[0], px, pieces(ka[d].x));
+        acc_mul(sa[1], py, pieces(ka[d].y));
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        rb[h] = acc_reduce(sb[h], m);
+        ra[h] = acc_reduce(sa[h], m);
+    }
+    if (with_b) {
+        swap_if(at.swap, b);
+        if (!b_premultiplied) {
+            b.x = mul_shoup_lazy_u(b.x, pmod.w, pmod.ws, q);
+            b.y = mul_shoup_lazy_u(b.y, pmod.w, pmod.ws, q);
+        }
+        rb[0] += b.x;
+        rb[1] += b.y;
+    }
+}
+// no key: P (b, a), below 2q
+__device__ __forceinline__ void pieces_keyless(const RotTermDev &T, const u64 q, const Cst pmod, const TermAt at, const int b_premultiplied,
+                                               u64 (&rb)[2], u64 (&ra)[2]) {
+    ulonglong2 a = at.chain(T.ext), b = make_ulonglong2(0, 0);
+    if (T.b != nullptr) b = at.chain(T.b);
+    swap_if(at.swap, a);
+    swap_if(at.swap, b);
+    ra[0] = mul_shoup_lazy_u(a.x, pmod.w, pmod.ws, q);   // never premultiplied, whatever b is
+    ra[1] = mul_shoup_lazy_u(a.y, pmod.w, pmod.ws, q);
+    rb[0] = b_premultiplied ? b.x : mul_shoup_lazy_u(b.x, pmod.w, pmod.ws, q);
+    rb[1] = b_premultiplied ? b.y : mul_shoup_lazy_u(b.y, pmod.w, pmod.ws, q);
+}
+template <bool COMPACT, int B>
+__device__ __forceinline__ void hoisted_pair_pieces(const RotTermDev *__restrict__ terms, const u32 *__restrict__ group_off, const KeyLimb kl,
+                                                    const ModQ m, const Cst *__restrict__ pmods, const int j, const int o, const u32 n,
+                                                    int nq, int E, int logN, int b_premultiplied, u64 (&out_b)[2], u64 (&out_a)[2]) {
+    const u64 q = m.q;
+    u64 acc_b[2] = {0, 0}, acc_a[2] = {0, 0};
+    Cst pmod{0, 0};
+    if (j < nq) pmod = pmods[j];
+    for (u32 t = group_off[o]; t < group_off[o + 1]; t++) {
+        const RotTermDev T = terms[t];
+        // a term without a key lives on the chain limbs: its polynomials and its mask have nq limbs, nothing of it
+        // is read for a special limb
+        if (T.evk == nullptr && j >= nq) continue;
+        const u32 np = galois_index(n, T.galois, logN);
+        const TermAt at{(size_t)1 << logN, n, np & ~1u, j, E, (np & 1u) != 0};
+        u64 rb[2], ra[2];
+        const bool two = T.ext2 != nullptr;
+        if (two && T.mask_shift != 0)
+            pieces_two<B, true>(T, kl, m, pmod, at, nq, logN, b_premultiplied, rb, ra);
+        else if (two)
+            pieces_two<B, false>(T, kl, m, pmod, at, nq, logN, b_premultiplied, rb, ra);
+        else if (T.evk != nullptr)
+            pieces_one<B>(T, kl, m, pmod, at, nq, !COMPACT && (T.flags & ROT_TERM_EXT_ROTATED) != 0, b_premultiplied, rb, ra);
+        else
+            pieces_keyless(T, q, pmod, at, b_premultiplied, rb, ra);
+        const bool mask = !two && T.mask != nullptr;
+        if (mask || T.pt != nullptr) {   // factors below q, values below 4q
+            ulonglong2 f = make_ulonglong2(0, 0);
+            if (mask) f = load_mask2(T.mask, T.mask_shift, j, n, logN);
+            if (T.pt != nullptr) {
+                const ulonglong2 pv = load_rotated2(T.pt, T.pt_galois, j, n, logN);
+                f = mask ? make_ulonglong2(mulmod_u(f.x, pv.x, m), mulmod_u(f.y, pv.y, m)) : pv;
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const Pieces y = pieces(h ? f.y : f.x);
+                Acc3 p{0, 0, 0};
+                acc_mul(p, pieces(cond_sub_u(rb[h], 4 * q)), y);
+                rb[h] = acc_reduce(p, m);
+                p = Acc3{0, 0, 0};
+                acc_mul(p, pieces(ra[h]), y);
+                ra[h] = acc_reduce(p, m);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {   // < 8q + 7q
+            acc_b[h] = cond_sub_u(acc_b[h] + rb[h], 8 * q);
+            acc_a[h] = cond_sub_u(acc_a[h] + ra[h], 8 * q);
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        out_b[h] = cond_sub_u(cond_sub_u(cond_sub_u(acc_b[h], 4 * q), 2 * q), q);
+        out_a[h] = cond_sub_u(cond_sub_u(cond_sub_u(acc_a[h], 4 * q), 2 * q), q);
+    }
+}
+
+// One term with two masked sources under one key (general integer path): residues (n, n+1) of limb j of
+// <z, evk> + P (mask b + mask2 b2) with z_d = mask * x_d + mask2 * x2_d, canonical.  RUNS: the masks are run tables, i.e. constants with a
+// Shoup companion; a plaintext factor of the term is then left to the caller, which multiplies the finished pair by it.
+template <bool RUNS>
+__device__ __forceinline__ void two_source_int(const RotTermDev &T, const KeyLimb kl, const ModQ m, const Cst *__restrict__ pmod, const int j,
+                                               const u32 n, const u32 base, const bool swap, int nq, int E, int beta, int logN,
+                                               int b_premultiplied, u64 (&rb)[2], u64 (&ra)[2]) {
+    const size_t N = (size_t)1 << logN;
+    ulonglong2 m1 = RUNS ? load_mask_run(T.mask, T.mask_shift, j, n, logN) : load_mask2(T.mask, 0, j, n, logN);
+    ulonglong2 m2 = RUNS ? load_mask_run(T.mask2, T.mask_shift, j, n, logN) : load_mask2(T.mask2, 0, j, n, logN);
+    if (!RUNS && T.pt != nullptr) {
+        const ulonglong2 pv = load_rotated2(T.pt, T.pt_galois, j, n, logN);
+        m1.x = mulmod_u(m1.x, pv.x, m);
+        m1.y = mulmod_u(m1.y, pv.y, m);
+        m2.x = mulmod_u(m2.x, pv.x, m);
+        m2.y = mulmod_u(m2.y, pv.y, m);
+    }
+    auto masked = [&](const ulonglong2 x, const ulonglong2 x2) {
+        if (RUNS) return make_ulonglong2(shoup_pair(x.x, m1, x2.x, m2, m.q), shoup_pair(x.y, m1, x2.y, m2, m.q));
+        u128_t t0 = mul64wide(m1.x, x.x), t1 = mul64wide(m1.y, x.y);
+        add128(t0, mul64wide(m2.x, x2.x));
+        add128(t1, mul64wide(m2.y, x2.y));
+        return make_ulonglong2(barrett3_u(t0, m), barrett3_u(t1, m));
+    };
     u128_t pb[2] = {{0, 0}, {0, 0}}, pa[2] = {{0, 0}, {0, 0}};
     for (int d = 0; d < beta; d++) {
         ulonglong2 x1 = load2(T.ext + ((size_t)d * E + j) * N + base);
         ulonglong2 x2 = load2(T.ext2 + ((size_t)d * E + j) * N + base);
-        if (swap) {
-            u64 tmp = x1.x;
-            x1.x = x1.y;
-            x1.y = tmp;
-            tmp = x2.x;
-            x2.x = x2.y;
-            x2.y = tmp;
-        }
-        u64 z0, z1;
-        if (RUNS) {
-            z0 = shoup_pair(x1.x, m1, x2.x, m2, m.q);
-            z1 = shoup_pair(x1.y, m1, x2.y, m2, m.q);
-        } else {
-            u128_t t0 = mul64wide(m1.x, x1.x), t1 = mul64wide(m1.y, x1.y);
-            add128(t0, mul64wide(m2.x, x2.x));
-            add128(t1, mul64wide(m2.y, x2.y));
-            z0 = barrett3_u(t0, m);
-            z1 = barrett3_u(t1, m);
-        }
+        swap_if(swap, x1);
+        swap_if(swap, x2);
+        const ulonglong2 z = masked(x1, x2);
         const ulonglong2 kb = key_pair_ptr(T, kl.of(d, 0), n);
         const ulonglong2 ka = key_pair_ptr(T, kl.of(d, 1), n);
-        add128(pb[0], mul64wide(z0, kb.x));
-        add128(pb[1], mul64wide(z1, kb.y));
-        add128(pa[0], mul64wide(z0, ka.x));
-        add128(pa[1], mul64wide(z1, ka.y));
+        add128(pb[0], mul64wide(z.x, kb.x));
+        add128(pb[1], mul64wide(z.y, kb.y));
+        add128(pa[0], mul64wide(z.x, ka.x));
+        add128(pa[1], mul64wide(z.y, ka.y));
     }
-    if (beta <= 3) {   // at most 3 q^2: the short reduction applies
-        rb[0] = barrett3_u(pb[0], m);
-        rb[1] = barrett3_u(pb[1], m);
-        ra[0] = barrett3_u(pa[0], m);
-        ra[1] = barrett3_u(pa[1], m);
-    } else {
-        rb[0] = barrett128_u(pb[0], m);
-        rb[1] = barrett128_u(pb[1], m);
-        ra[0] = barrett128_u(pa[0], m);
-        ra[1] = barrett128_u(pa[1], m);
+    for (int i = 0; i < 2; i++) {   // at most 3 q^2: the short reduction applies
+        rb[i] = beta <= 3 ? barrett3_u(pb[i], m) : barrett128_u(pb[i], m);
+        ra[i] = beta <= 3 ? barrett3_u(pa[i], m) : barrett128_u(pa[i], m);
     }
     if (j < nq) {
         ulonglong2 b1 = load2(T.b + (size_t)j * N + base);
         ulonglong2 b2 = load2(T.b2 + (size_t)j * N + base);
-        if (swap) {
-            u64 tmp = b1.x;
-            b1.x = b1.y;
-            b1.y = tmp;
-            tmp = b2.x;
-            b2.x = b2.y;
-            b2.y = tmp;
-        }
+        swap_if(swap, b1);
+        swap_if(swap, b2);
         if (!b_premultiplied) {
             b1.x = mul_shoup_u(b1.x, pmod[j].w, pmod[j].ws, m.q);
             b1.y = mul_shoup_u(b1.y, pmod[j].w, pmod[j].ws, m.q);
             b2.x = mul_shoup_u(b2.x, pmod[j].w, pmod[j].ws, m.q);
             b2.y = mul_shoup_u(b2.y, pmod[j].w, pmod[j].ws, m.q);
         }
-        if (RUNS) {
-            rb[0] = addmod_u(rb[0], shoup_pair(b1.x, m1, b2.x, m2, m.q), m.q);
-            rb[1] = addmod_u(rb[1], shoup_pair(b1.y, m1, b2.y, m2, m.q), m.q);
-        } else {
-            u128_t t0 = mul64wide(m1.x, b1.x), t1 = mul64wide(m1.y, b1.y);
-            add128(t0, mul64wide(m2.x, b2.x));
-            add128(t1, mul64wide(m2.y, b2.y));
-            rb[0] = addmod_u(rb[0], barrett3_u(t0, m), m.q);
-            rb[1] = addmod_u(rb[1], barrett3_u(t1, m), m.q);
-        }
+        const ulonglong2 z = masked(b1, b2);
+        rb[0] = addmod_u(rb[0], z.x, m.q);
+        rb[1] = addmod_u(rb[1], z.y, m.q);
     }
 }
 
-// Residues (n, n+1) of limb j of both polynomials of output o (integer path), canonical.
+// Residues (n, n+1) of limb j of both polynomials of output o (integers, any prime and any number of digits), canonical.
 template <bool COMPACT>
 __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ terms,
                                                  const u32 *__restrict__ group_off, const KeyLimb kl,
@@ -265,13 +418,9 @@ __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ 
         const u32 base = np & ~1u;
         const bool swap = (np & 1u) != 0;
         if (T.ext2 != nullptr) {
-            // two masked sources under one key: z_d = mask * x_d + mask2 * x2_d, then one pass over the key
             u64 rb[2], ra[2];
             if (T.mask_shift != 0) {
-                // run-table masks are constants: the plaintext factor of the term, if it has one, is common to both
-                // sources and multiplies the finished pair once (same residues as masks multiplied by it beforehand)
-                two_source_int<true>(T, kl, m, pmod, j, n, base, swap, nq, E, beta, logN,
-                                              b_premultiplied, rb, ra);
+                two_source_int<true>(T, kl, m, pmod, j, n, base, swap, nq, E, beta, logN, b_premultiplied, rb, ra);
                 if (T.pt != nullptr) {
                     const ulonglong2 pv = load_rotated2(T.pt, T.pt_galois, j, n, logN);
                     rb[0] = mulmod_u(rb[0], pv.x, m);
@@ -280,8 +429,7 @@ __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ 
                     ra[1] = mulmod_u(ra[1], pv.y, m);
                 }
             } else {
-                two_source_int<false>(T, kl, m, pmod, j, n, base, swap, nq, E, beta, logN,
-                                               b_premultiplied, rb, ra);
+                two_source_int<false>(T, kl, m, pmod, j, n, base, swap, nq, E, beta, logN, b_premultiplied, rb, ra);
             }
             acc_b[0] = addmod_u(acc_b[0], rb[0], m.q);
             acc_b[1] = addmod_u(acc_b[1], rb[1], m.q);

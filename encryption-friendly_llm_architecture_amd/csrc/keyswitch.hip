@@ -466,6 +466,14 @@ __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict_
         rb[1] = f.canonical(fb[1]);
         ra[0] = f.canonical(fa[0]);
         ra[1] = f.canonical(fa[1]);
+    } else if (beta <= 3 && modq[prime].mu3 != 0) {
+        const ModQ m = modq[prime];
+        if (beta == 1)
+            hoisted_pair_pieces<COMPACT, 1>(terms, group_off, kl, m, pmod, j, o, n, nq, E, logN, b_premultiplied, rb, ra);
+        else if (beta == 2)
+            hoisted_pair_pieces<COMPACT, 2>(terms, group_off, kl, m, pmod, j, o, n, nq, E, logN, b_premultiplied, rb, ra);
+        else
+            hoisted_pair_pieces<COMPACT, 3>(terms, group_off, kl, m, pmod, j, o, n, nq, E, logN, b_premultiplied, rb, ra);
     } else {
         hoisted_pair_int<COMPACT>(terms, group_off, kl, modq[prime], pmod, j, o, n, nq, E, beta, logN, b_premultiplied, rb, ra);
     }

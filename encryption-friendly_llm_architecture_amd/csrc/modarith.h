@@ -36,7 +36,7 @@ struct ModQ {
     u64 mu;    // floor(2^(2k) / q), k = bit length of q
     u32 k;     // bit length of q (q < 2^k, k <= 61)
     u32 mdot;  // floor(2^(k+31) / q) (dot_reduce_lazy)
-    u64 mu3;   // floor(2^(2k+3) / q) for k = 59 or 60, else 0 (barrett_tight)
+    u64 mu3;   // floor(2^(k+63) / q) for k <= 60, else 0 (barrett_tight)
 };
 
 // x * w mod q for a constant w with ws = floor(w * 2^64 / q); result in [0, 2q).
@@ -83,14 +83,14 @@ __device__ __forceinline__ u64 barrett128(u128_t t, const ModQ &m) {
     if (r >= q) r -= q;
     return r;
 }
-// Barrett reduction of T < 3 * 2^(2k) to [0, q) for primes of 59 or 60 bits (m.mu3 != 0) with the three bits longer
-// constant: qhat = floor(floor(T / 2^(k-2)) * mu3 / 2^(k+5)) misses floor(T / q) by less than
+// Barrett reduction of T < 3 * 2^(2k) to [0, q) for primes below 2^60 (m.mu3 != 0) with a constant of 64 bits:
+// qhat = floor(floor(T / 2^(k-2)) * mu3 / 2^65) misses floor(T / q) by less than
 // T / 2^(2k+3) + 2^(k-2) / q + 1 < 3/8 + 1/2 + 1, i.e. by at most 1: only the high half of one product and a single
 // correction, against a full product and three corrections in barrett128.
 __device__ __forceinline__ u64 barrett_tight(u128_t t, const ModQ &m) {
     const u32 k = m.k;
     const u64 t1 = (t.hi << (66 - k)) | (t.lo >> (k - 2));
-    const u64 qhat = __umul64hi(t1, m.mu3) >> (k - 59);
+    const u64 qhat = __umul64hi(t1, m.mu3) >> 1;
     const u64 r = t.lo - qhat * m.q;
     return r >= m.q ? r - m.q : r;
 }
@@ -187,7 +187,7 @@ __device__ __forceinline__ u64 barrett128_u(u128_t t, const ModQ &m) {
 __device__ __forceinline__ u64 barrett_tight_u(u128_t t, const ModQ &m) {
     const u32 k = m.k;
     const u64 t1 = (t.hi << (66 - k)) | (t.lo >> (k - 2));
-    const u64 qhat = __umul64hi(t1, m.mu3) >> (k - 59);
+    const u64 qhat = __umul64hi(t1, m.mu3) >> 1;
     return cond_sub_u(t.lo + qhat * neg_uniform(m.q), m.q);
 }
 __device__ __forceinline__ u64 barrett3_u(u128_t t, const ModQ &m) {
@@ -196,3 +196,30 @@ __device__ __forceinline__ u64 barrett3_u(u128_t t, const ModQ &m) {
 __device__ __forceinline__ u64 mulmod_u(u64 a, u64 b, const ModQ &m) { return barrett3_u(mul64wide(a, b), m); }
 __device__ __forceinline__ u64 addmod_u(u64 a, u64 b, u64 q) { return cond_sub_u(a + b, q); }
 __device__ __forceinline__ u64 negmod(u64 a, u64 q) { return a ? q - a : 0; }
+
+// ---- sums of products of residues below 2^60 in pieces of 30 bits -----------------------------------------------------------
+// A 128-bit product summed as such is 17 instructions (the compiler makes its two halves apart, and carries them).  Cut at bit 30
+// it is four multiply-adds into accumulators of weights 1, 2^30 and 2^60 that nothing is carried out of.
+struct Pieces {
+    u32 lo, hi;
+};
+__device__ __forceinline__ Pieces pieces(const u64 v) { return Pieces{(u32)v & 0x3fffffffu, (u32)(v >> 30)}; }
+struct Acc3 {
+    u64 s0, s1, s2;
+};
+// x < 2^62, y < 2^60: the hi pieces below 2^32 and 2^30, so s1 grows by less than 5 * 2^60 and s2 by less than 2^62
+__device__ __forceinline__ void acc_mul(Acc3 &a, const Pieces x, const Pieces y) {
+    a.s0 += (u64)x.lo * y.lo;
+    a.s1 += (u64)x.lo * y.hi;
+    a.s1 += (u64)x.hi * y.lo;
+    a.s2 += (u64)x.hi * y.hi;
+}
+// T = s0 + 2^30 s1 + 2^60 s2 < 4 * 2^(2k) modulo a prime of 32 <= k <= 60 bits, to [0, 3q).  The quotient is barrett_tight's, from the
+// accumulators' own parts above 2^(k-2) (which miss the carries between them: 2 at most) instead of T's: it misses
+// floor(T / q) by less than T / 2^(2k+3) + (2 + 1) 2^(k-2) / q + 1 < 1/2 + 3/2 + 1, i.e. by at most 2.
+__device__ __forceinline__ u64 acc_reduce(const Acc3 &a, const ModQ &m) {
+    const u32 k = m.k;
+    const u64 t1 = (a.s2 << (62 - k)) + (a.s1 >> (k - 32)) + (a.s0 >> (k - 2));
+    const u64 qhat = __umul64hi(t1, m.mu3) >> 1;
+    return (a.s0 + (a.s1 << 30) + (a.s2 << 60)) + qhat * neg_uniform(m.q);
+}
