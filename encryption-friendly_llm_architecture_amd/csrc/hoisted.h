@@ -281,15 +281,15 @@ __device__ __forceinline__ void pieces_keyless(const RotTermDev &T, const u64 q,
     rb[0] = b_premultiplied ? b.x : mul_shoup_lazy_u(b.x, pmod.w, pmod.ws, q);
     rb[1] = b_premultiplied ? b.y : mul_shoup_lazy_u(b.y, pmod.w, pmod.ws, q);
 }
-template <bool COMPACT, int B>
-__device__ __forceinline__ void hoisted_pair_pieces(const RotTermDev *__restrict__ terms, const u32 *__restrict__ group_off, const KeyLimb kl,
+template <bool COMPACT, int S, int B>
+__device__ __forceinline__ void hoisted_pair_pieces(const RotTermDev *__restrict__ terms, const u32 *__restrict__ group_off, const u32 part, const KeyLimb kl,
                                                     const ModQ m, const Cst *__restrict__ pmods, const int j, const int o, const u32 n,
                                                     int nq, int E, int logN, int b_premultiplied, u64 (&out_b)[2], u64 (&out_a)[2]) {
     const u64 q = m.q;
     u64 acc_b[2] = {0, 0}, acc_a[2] = {0, 0};
     Cst pmod{0, 0};
     if (j < nq) pmod = pmods[j];
-    for (u32 t = group_off[o]; t < group_off[o + 1]; t++) {
+    for (u32 t = group_off[o] + part; t < group_off[o + 1]; t += S) {
         const RotTermDev T = terms[t];
         // a term without a key lives on the chain limbs: its polynomials and its mask have nq limbs, nothing of it
         // is read for a special limb
@@ -397,10 +397,11 @@ __device__ __forceinline__ void two_source_int(const RotTermDev &T, const KeyLim
     }
 }
 
+// Of a sum dealt to S wavefront groups, `part` says which terms are this one's.
 // Residues (n, n+1) of limb j of both polynomials of output o (integers, any prime and any number of digits), canonical.
-template <bool COMPACT>
+template <bool COMPACT, int S>
 __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ terms,
-                                                 const u32 *__restrict__ group_off, const KeyLimb kl,
+                                                 const u32 *__restrict__ group_off, const u32 part, const KeyLimb kl,
                                                  const ModQ m, const Cst *__restrict__ pmod,
                                                  const int j, const int o, const u32 n, int nq, int E,
                                                  int beta, int logN, int b_premultiplied, u64 (&out_b)[2],
@@ -409,7 +410,7 @@ __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ 
     u64 acc_b[2] = {0, 0}, acc_a[2] = {0, 0};
     u128_t lazy_b[2] = {{0, 0}, {0, 0}}, lazy_a[2] = {{0, 0}, {0, 0}};
     int pending = 0;
-    for (u32 t = group_off[o]; t < group_off[o + 1]; t++) {
+    for (u32 t = group_off[o] + part; t < group_off[o + 1]; t += S) {
         const RotTermDev T = terms[t];
         // a term without a key lives on the chain limbs: its polynomials and its mask have nq limbs, nothing of it
         // is read for a special limb
@@ -566,9 +567,9 @@ __device__ __forceinline__ D2 key_pair_fp(const __amdgpu_buffer_rsrc_t key, cons
 }
 #pragma clang fp contract(off)
 // The same residues in double precision (primes below 2^44); out_* are unreduced centred doubles.
-template <bool COMPACT>
+template <bool COMPACT, int S>
 __device__ __forceinline__ void hoisted_pair_fp(const RotTermDev *__restrict__ terms,
-                                                const u32 *__restrict__ group_off, const KeyLimb kl,
+                                                const u32 *__restrict__ group_off, const u32 part, const KeyLimb kl,
                                                 const FpMod f, const double p_mod_q,
                                                 const int j, const int o, const u32 n, int nq, int E,
                                                 int beta, int logN, int b_premultiplied, double (&out_b)[2],
@@ -576,7 +577,7 @@ __device__ __forceinline__ void hoisted_pair_fp(const RotTermDev *__restrict__ t
     const size_t N = (size_t)1 << logN;
     double acc_b0 = 0, acc_b1 = 0, acc_a0 = 0, acc_a1 = 0;
     int since = 0;
-    for (u32 t = group_off[o]; t < group_off[o + 1]; t++) {
+    for (u32 t = group_off[o] + part; t < group_off[o + 1]; t += S) {
         const RotTermDev T = terms[t];
         if (T.evk == nullptr && j >= nq) continue;   // a term without a key: chain limbs only, mask included
         const __amdgpu_buffer_rsrc_t kr = key_rsrc(T);

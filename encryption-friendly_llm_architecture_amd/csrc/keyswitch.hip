@@ -391,6 +391,7 @@ __device__ __forceinline__ void rows_under_products(const F f, const u64 (&rb)[2
 struct SumRows {
     u64 inverse;       // bit j: limb j of the extended basis leaves as the first pass of its inverse transform; the others as they are
     const Tw *tw;      // stage-ordered twiddles of the inverse transforms, [prime][N]
+    __device__ __forceinline__ bool takes_rows(const u32 j) const { return (inverse >> j) & 1ull; }
 };
 struct SumTail {       // all limbs of the launch end in the ModDown's tail
     const u64 *conv;   // [n_out][2][nq_out][N]
@@ -400,8 +401,9 @@ struct SumTail {       // all limbs of the launch end in the ModDown's tail
     size_t out_stride;
     int nq_out, listed;
     ResultList list;
+    __device__ __forceinline__ bool takes_rows(u32) const { return true; }
 };
-template <int MODE, bool COMPACT, class ROWS>
+template <int MODE, bool COMPACT, int S, class ROWS>
 __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict__ terms,
                                                    const u32 *__restrict__ group_off, u64 *__restrict__ y,
                                                    const ModQ *__restrict__ modq, const double *__restrict__ fp,
@@ -452,7 +454,8 @@ __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict_
     j = __builtin_amdgcn_readfirstlane(j);
     chunk = __builtin_amdgcn_readfirstlane(chunk);
     const int prime = (int)table_byte(ll.idx, j);
-    const u32 n = (chunk * 256 + threadIdx.x) * 2;
+    const u32 part = S > 1 ? (u32)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8)) : 0u;
+    const u32 n = (chunk * 256 + (S > 1 ? threadIdx.x & 255u : threadIdx.x)) * 2;
     const double fq = fp[4 * prime];
     const KeyLimb kl = key_limb<COMPACT>(koff, prime, logN, n_full);
     const size_t N = (size_t)1 << logN;
@@ -460,7 +463,7 @@ __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict_
     if (MODE == 1 || (MODE == 0 && fq != 0.0 && beta <= 6)) {
         const FpMod f{fq, fp[4 * prime + 1]};
         double fb[2], fa[2];
-        hoisted_pair_fp<COMPACT>(terms, group_off, kl, f, j < nq ? (double)pmod[j].w : 0.0, j, o, n, nq, E, beta, logN, b_premultiplied,
+        hoisted_pair_fp<COMPACT, S>(terms, group_off, part, kl, f, j < nq ? (double)pmod[j].w : 0.0, j, o, n, nq, E, beta, logN, b_premultiplied,
                                  fb, fa);
         rb[0] = f.canonical(fb[0]);
         rb[1] = f.canonical(fb[1]);
@@ -469,13 +472,35 @@ __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict_
     } else if (beta <= 3 && modq[prime].mu3 != 0) {
         const ModQ m = modq[prime];
         if (beta == 1)
-            hoisted_pair_pieces<COMPACT, 1>(terms, group_off, kl, m, pmod, j, o, n, nq, E, logN, b_premultiplied, rb, ra);
+            hoisted_pair_pieces<COMPACT, S, 1>(terms, group_off, part, kl, m, pmod, j, o, n, nq, E, logN, b_premultiplied, rb, ra);
         else if (beta == 2)
-            hoisted_pair_pieces<COMPACT, 2>(terms, group_off, kl, m, pmod, j, o, n, nq, E, logN, b_premultiplied, rb, ra);
+            hoisted_pair_pieces<COMPACT, S, 2>(terms, group_off, part, kl, m, pmod, j, o, n, nq, E, logN, b_premultiplied, rb, ra);
         else
-            hoisted_pair_pieces<COMPACT, 3>(terms, group_off, kl, m, pmod, j, o, n, nq, E, logN, b_premultiplied, rb, ra);
+            hoisted_pair_pieces<COMPACT, S, 3>(terms, group_off, part, kl, m, pmod, j, o, n, nq, E, logN, b_premultiplied, rb, ra);
     } else {
-        hoisted_pair_int<COMPACT>(terms, group_off, kl, modq[prime], pmod, j, o, n, nq, E, beta, logN, b_premultiplied, rb, ra);
+        hoisted_pair_int<COMPACT, S>(terms, group_off, part, kl, modq[prime], pmod, j, o, n, nq, E, beta, logN, b_premultiplied, rb, ra);
+    }
+    if (S > 1) {   // the parts' sums meet in LDS, the first part goes on with the whole
+        __shared__ u64 sums[S > 1 ? S - 1 : 1][4][256];
+        const u32 t = threadIdx.x & 255u;
+        if (part != 0) {
+            for (int h = 0; h < 2; h++) {
+                sums[part - 1][h][t] = rb[h];
+                sums[part - 1][2 + h][t] = ra[h];
+            }
+        }
+        __syncthreads();
+        if (part != 0) {
+            if (rows.takes_rows(j)) __syncthreads();   // the one in the row pass
+            return;
+        }
+        const u64 q = modq[prime].q;
+        for (int h = 0; h < 2; h++) {
+            for (int p = 0; p < S - 1; p++) {
+                rb[h] = cond_sub_u(rb[h] + sums[p][h][t], q);
+                ra[h] = cond_sub_u(ra[h] + sums[p][2 + h][t], q);
+            }
+        }
     }
     __shared__ u64 lds[4 * ROWPAD];
     const u32 first = chunk * 512;
@@ -491,7 +516,7 @@ __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict_
             rows_under_products(IntFieldT<true>(modq, nullptr, nullptr, fp, prime), rb, ra, cb, ca, ob, oa, lds, tw, logN - 8, 2 * chunk, cst);
     } else {
         u64 *yb = y + (((size_t)o * 2 + 0) * E + j) * N, *ya = y + (((size_t)o * 2 + 1) * E + j) * N;
-        if ((rows.inverse >> j) & 1ull) {
+        if (rows.takes_rows(j)) {
             const Tw *tw = rows.tw + ((size_t)prime << logN);
             if (fp_limb)
                 rows_of_products(FpField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
@@ -515,22 +540,22 @@ struct HoistedArgs {
 // Register budget for five waves per SIMD (96 registers): the double-precision form needs 72, the integer and the mixed form
 // all 96.  The mixed form under a ModDown's tail spills three; with four waves and none a product at level 9 takes 122.1 instead of
 // 120.2 us, the projection of a 768-wide layer 10.46 instead of 10.33 ms.  COMPACT: the key layout of the launch (hoisted.h, key_limb).
-#define HOISTED_KERNEL __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void
-template <int MODE, bool COMPACT, class ROWS>
+#define HOISTED_KERNEL __global__ __launch_bounds__(256 * S) __attribute__((amdgpu_waves_per_eu(S == 4 ? 4 : 5))) void
+template <int MODE, bool COMPACT, int S, class ROWS>
 HOISTED_KERNEL hoisted_terms_kernel(const HoistedArgs args, u64 *__restrict__ y, const ModQ *__restrict__ modq,
                                     const double *__restrict__ fp, LimbList ll, const Cst *__restrict__ pmod, int nq, int E, int beta,
                                     int n_full, int logN, int b_premultiplied, int n_out, LimbList jmap, int n_j,
                                     const u32 *__restrict__ koff, const ROWS rows) {
-    hoisted_terms_body<MODE, COMPACT>(args.t, args.off, y, modq, fp, ll, pmod, nq, E, beta, n_full, logN,
+    hoisted_terms_body<MODE, COMPACT, S>(args.t, args.off, y, modq, fp, ll, pmod, nq, E, beta, n_full, logN,
                                       b_premultiplied, n_out, jmap, n_j, koff, rows);
 }
-template <int MODE, bool COMPACT, class ROWS>
+template <int MODE, bool COMPACT, int S, class ROWS>
 HOISTED_KERNEL hoisted_terms_list_kernel(const RotTermDev *__restrict__ terms, const u32 *__restrict__ group_off,
                                          u64 *__restrict__ y, const ModQ *__restrict__ modq,
                                          const double *__restrict__ fp, LimbList ll, const Cst *__restrict__ pmod, int nq, int E,
                                          int beta, int n_full, int logN, int b_premultiplied, int n_out, LimbList jmap,
                                          int n_j, const u32 *__restrict__ koff, const ROWS rows) {
-    hoisted_terms_body<MODE, COMPACT>(terms, group_off, y, modq, fp, ll, pmod, nq, E, beta, n_full, logN,
+    hoisted_terms_body<MODE, COMPACT, S>(terms, group_off, y, modq, fp, ll, pmod, nq, E, beta, n_full, logN,
                                       b_premultiplied, n_out, jmap, n_j, koff, rows);
 }
 #undef HOISTED_KERNEL
@@ -1524,28 +1549,45 @@ static void sum_limbs(hemm_context *c, const HoistedList &l, int first, int n_ou
         kind[k].idx[n_kind[k]++] = jl.idx[i];
     }
     const size_t per_limb = (size_t)n_out * (c->N / 512);
-#define SUM_FORM(MODE, COMPACT, JM, NJ)                                                                                        \
+    // Few workgroups with many terms each are a chain of trips to memory: such a sum is dealt term by term to the four or two groups of
+    // wavefronts of a larger workgroup.  One / two / four groups, us (13 limbs, masked terms):
+    //   104 workgroups, 7 terms 16.8/13.3/13.4, 15 terms 31.2/21.4/19.4     208, 7 terms 18.6/13.6/13.0, 15 terms 36.3/23.2/19.5
+    //   416, 7 terms 23.9/18.2/20.2, 15 terms 45.9/32.7/35.3                832, 3 terms 15.6/17.8/22.1, 15 terms 59.6/60.0/63.5
+    // (two outputs of 4 terms at 208: 14.0/13.9/13.5; product of two encrypted 32 x 32 tiles 561/536/520, the last with both lines)
+    const size_t wgs = per_limb * n_j;
+    const bool many = l.n_terms >= 3 * n_out;
+#define SUM_FORM(MODE, COMPACT, S, JM, NJ)                                                                                     \
     do {                                                                                                                       \
-        const dim3 grid((unsigned)(per_limb * (NJ)));                                                                          \
+        const dim3 grid((unsigned)(per_limb * (NJ))), block(256 * (S));                                                        \
         if (l.terms_dev != nullptr)                                                                                            \
-            hipLaunchKernelGGL((hoisted_terms_list_kernel<MODE, COMPACT, ROWS>), grid, dim3(256), 0, s,                        \
+            hipLaunchKernelGGL((hoisted_terms_list_kernel<MODE, COMPACT, S, ROWS>), grid, block, 0, s,                         \
                                (const RotTermDev *)l.terms_dev, l.offsets_dev + first, y, c->d_modq, c->d_fp, ll, pm, nq, E,   \
                                beta, n_full, c->logN, pre, n_out, JM, NJ, c->d_key_off, rows);                                 \
         else                                                                                                                   \
-            hipLaunchKernelGGL((hoisted_terms_kernel<MODE, COMPACT, ROWS>), grid, dim3(256), 0, s, a, y, c->d_modq, c->d_fp,   \
+            hipLaunchKernelGGL((hoisted_terms_kernel<MODE, COMPACT, S, ROWS>), grid, block, 0, s, a, y, c->d_modq, c->d_fp,    \
                                ll, pm, nq, E, beta, n_full, c->logN, pre, n_out, JM, NJ, c->d_key_off, rows);                  \
     } while (0)
-#define SUM_LIMBS(MODE, JM, NJ)                   \
-    do {                                          \
-        if (compact) SUM_FORM(MODE, true, JM, NJ); \
-        else SUM_FORM(MODE, false, JM, NJ);       \
+#define SUM_LIMBS(MODE, S, JM, NJ)                   \
+    do {                                             \
+        if (compact) SUM_FORM(MODE, true, S, JM, NJ); \
+        else SUM_FORM(MODE, false, S, JM, NJ);       \
     } while (0)
-    if (n_kind[0] == 0 || n_kind[1] == 0 || per_limb * n_j < 16384) {
-        SUM_LIMBS(0, jl, n_j);
-    } else {
-        SUM_LIMBS(1, kind[0], n_kind[0]);
-        SUM_LIMBS(2, kind[1], n_kind[1]);
+    if (n_kind[0] != 0 && n_kind[1] != 0 && wgs >= 16384) {
+        SUM_LIMBS(1, 1, kind[0], n_kind[0]);
+        SUM_LIMBS(2, 1, kind[1], n_kind[1]);
+        return;
     }
+    if constexpr (std::is_same<ROWS, SumRows>::value) {   // (a sum under a ModDown's tail has more workgroups)
+        if (many && wgs <= 256) {
+            SUM_LIMBS(0, 4, jl, n_j);
+            return;
+        }
+        if (many && wgs <= 640) {
+            SUM_LIMBS(0, 2, jl, n_j);
+            return;
+        }
+    }
+    SUM_LIMBS(0, 1, jl, n_j);
 #undef SUM_LIMBS
 #undef SUM_FORM
 }

@@ -72,6 +72,10 @@ def test_every_kind_of_term(bits, chain, dnum, largest):
     got = ctx.hoisted_terms(give, nq).cpu().numpy().view(np.uint64)
     for o in range(len(groups)):
         assert np.array_equal(got[o], want[o]), o
+    # the longest sum by itself and many times over: few enough workgroups for its terms to be dealt to four, resp. two, groups of wavefronts
+    for copies in (1, 520 // (2 * len(primes))):
+        got = ctx.hoisted_terms(give[-1:] * copies, nq).cpu().numpy().view(np.uint64)
+        assert all(np.array_equal(y, want[-1]) for y in got), copies
 
 
 def add(x, y, primes):
