@@ -685,6 +685,41 @@ int hemm_sum_parts(hemm_context *ctx, const uint64_t *parts, uint32_t n_parts, u
     HEMM_CATCH
 }
 
+int hemm_diagonal_table_words(hemm_context *ctx, uint32_t k, uint32_t w, uint32_t g, uint32_t nq, size_t *words) {
+    HEMM_TRY
+    int nl;
+    chain_limbs(ctx, nq, 1, &nl);
+    need(words, "null operand");
+    *words = diagonals_ok(ctx, k, w, g) ? diagonal_table_words(ctx, k, w, g, (int)nq) : 0;
+    HEMM_CATCH
+}
+
+int hemm_diagonal_tables(hemm_context *ctx, const double *block, uint32_t k, uint32_t w, uint32_t g, double scale, uint32_t nq,
+                         uint64_t *tables, void *stream) {
+    HEMM_TRY
+    int nl;
+    chain_limbs(ctx, nq, 1, &nl);
+    need(block && tables, "null operand");
+    need(diagonals_ok(ctx, k, w, g), "no diagonal form for this shape or these primes");
+    launch_diagonal_tables(ctx, block, k, w, g, scale, (int)nq, (u64 *)tables, on_stream(ctx, stream));
+    check_launch();
+    HEMM_CATCH
+}
+
+int hemm_diagonal_sums(hemm_context *ctx, const uint64_t *rotated, const uint64_t *a, size_t a_stride, uint32_t k, uint32_t w, uint32_t g,
+                       uint32_t nq, const uint64_t *tables, uint64_t *y, void *stream) {
+    HEMM_TRY
+    int nl;
+    chain_limbs(ctx, nq, 1, &nl);
+    need(rotated && a && tables && y, "null operand");
+    need(a_stride >= (size_t)nq * (size_t)ctx->N, "polynomial stride below one polynomial");
+    need(diagonals_ok(ctx, k, w, g), "no diagonal form for this shape or these primes");
+    launch_diagonal_sums(ctx, (const u64 *)rotated, (const u64 *)a, a_stride, k, w, g, (int)nq, (const u64 *)tables, (u64 *)y,
+                         on_stream(ctx, stream));
+    check_launch();
+    HEMM_CATCH
+}
+
 int hemm_compact_mask(hemm_context *ctx, const uint64_t *mask, uint32_t n_limbs, uint32_t shift, uint64_t *table,
                       int *is_constant, void *stream) {
     HEMM_TRY

@@ -329,6 +329,8 @@ CentreArgs centre_args(const hemm_context *c, int n_limbs, double scale) {
 }
 }  // namespace
 
+const void *encode_roots(const hemm_context *c) { return tables_of(c).enc; }
+
 void hemm_embedding_tables_free(const hemm_context *c) {
     std::lock_guard<std::mutex> lk(g_mu);
     auto it = g_tabs.find(c);

@@ -148,6 +148,15 @@ public:
         Plaintext tau;
         int layout;
     };
+    // The diagonals of a plaintext weight as tables for hemm_diagonal_sums, kept like tau(B): one more part of the key is the level
+    // whose scale the encrypted operand carries.  layout as in WeightTau; no tables where the layout did not call for them.
+    struct WeightDiagonals {
+        DeviceBuffer tables;
+        int layout;
+    };
+    typedef std::tuple<u64, u64, TileTensorShape, u64, u64> DiagonalKey;
+    std::map<DiagonalKey, WeightDiagonals> weight_diagonals_;
+    std::vector<DiagonalKey> weight_diagonals_order_;
     // complexPackingInplace (rows[q] false: adjacent columns -> a + i b) / complexPackingRowInplace (true: adjacent
     // rows of rows `w` slots wide -> a - i b) of n_jobs ciphertexts at `level` through one launch chain: both
     // rotations of every job from one ModUp, masks applied in the extended basis, ModDown merged with the rescale.
@@ -232,6 +241,11 @@ void multMatMatPreFused(const HomEvaluator &eval, const CtxtTensor &a, std::vect
 // plaintext x ciphertext product through the hoisted column shifts (see matrix_utils_fused.cpp for the layouts it takes)
 bool multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2,
                           u64 target_level, MatrixTransformer &transformer, u64 batch, CtxtTensor &res);
+// the same over the diagonals of the weight, in baby and giant steps; a_single: the first operand holds one tile block and nothing else.
+// false: not a product for it.  plainDiagonalRotations: the rotations it takes (none: no such form).
+std::vector<u64> plainDiagonalRotations(i64 k, u64 log_slots);
+bool multMatMatPlainDiagonals(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2,
+                              u64 target_level, MatrixTransformer &transformer, bool a_single, CtxtTensor &res);
 // the n/2 column shifts (by two columns each) of a packed sigma(A) at level T+2, as ciphertexts at level T+1
 // (multPackedMatMatPreRot through the hoisted launches)
 void multPackedMatMatPreRotFused(const HomEvaluator &eval, const CtxtTensor &a, std::vector<Ciphertext> &tmp, u64 target_level,

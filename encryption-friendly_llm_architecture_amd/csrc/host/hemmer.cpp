@@ -632,6 +632,14 @@ CtxtTensor HEMMer::singleCCMatMul(const CtxtTensor &a, const CtxtTensor &b, u64 
 CtxtTensor HEMMer::singleMatMul(const CtxtTensor &a, const PtxtTensor &b, u64 T) const {
     const u64 slots = u64(1) << log_slots_;
     const i64 w = a.getBlockWidth(), n = pow2ceil(a.getWidth());
+    if (fused_) {
+        CtxtTensor res(context_, a.getHeight(), b.getWidth(), w);
+        const bool a_single = single_tile_ || a.get().occupiedSlots() <= (u64)(n * w);
+        if (a.getHeight() == n && b.getHeight() == n) {
+            ensureRotationKeys(plainDiagonalRotations(n, log_slots_));
+            if (multMatMatPlainDiagonals(eval_, btp_, a, b, T, matrix_transformer, a_single, res)) return res;
+        }
+    }
     ensureRotationKeys(transformRotations(MaskKind::Horizontal, w));
     if (fused_) {
         ensureRotationKeys(fusedRotations(TileTensorShape(n, n, w), log_slots_, false, false));

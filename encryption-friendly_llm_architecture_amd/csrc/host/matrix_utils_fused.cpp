@@ -1830,6 +1830,29 @@ std::pair<u64, u64> hashResidues(const Context &c, const Plaintext &pt) {
     }
     return {x, y};
 }
+// whose digests a weight's preparation is kept under: the hash needs a device-to-host copy and with it a drained queue, so it is taken once
+// per plaintext object
+std::pair<u64, u64> weightHash(const Context &c, const Plaintext &weight) {
+    if (weight.hash_state_ == 1) return {weight.content_hash_, weight.content_hash2_};
+    const std::pair<u64, u64> h = hashResidues(c, weight);
+    if (weight.hash_state_ == 0) {
+        weight.content_hash_ = h.first;
+        weight.content_hash2_ = h.second;
+        weight.hash_state_ = 1;
+    }
+    return h;
+}
+// 1: all tile blocks of `block` slots are equal, 2: only the first is not zero, 0: anything else.  Decoded values carry the encoding's
+// rounding noise (about sqrt(N) / 2^43 at this scale): "zero" and "equal" are taken up to 2^-24.
+int weightLayout(const Message &src, i64 block, i64 slots) {
+    const double tol = std::ldexp(1.0, -24);
+    bool rest_zero = true, rest_equal = true;
+    for (i64 j = block; j < slots && (rest_zero || rest_equal); j++) {
+        if (std::abs(src[(u64)j]) >= tol) rest_zero = false;
+        if (std::abs(src[(u64)j] - src[(u64)(j % block)]) >= tol) rest_equal = false;
+    }
+    return !rest_zero && !rest_equal ? 0 : rest_zero && block < slots ? 2 : 1;
+}
 }  // namespace
 
 bool multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2,
@@ -1847,36 +1870,17 @@ bool multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, con
         throw std::invalid_argument("[multMatMat] level >= " + std::to_string(T + 3) + " is needed.");
     const TileTensorShape shape_a(rows, k, w), shape_b(k, cols, w);
     // ---- tau(B) over the extended basis at level T+2, scaled like a plaintext of level T+1
-    // the hash needs a device-to-host copy and with it a drained queue: taken once per plaintext object
-    const Plaintext &weight = op2.get();
-    std::pair<u64, u64> weight_hash;
-    if (weight.hash_state_ == 1) {
-        weight_hash = {weight.content_hash_, weight.content_hash2_};
-    } else {
-        weight_hash = hashResidues(c, weight);
-        if (weight.hash_state_ == 0) {
-            weight.content_hash_ = weight_hash.first;
-            weight.content_hash2_ = weight_hash.second;
-            weight.hash_state_ = 1;
-        }
-    }
+    const std::pair<u64, u64> weight_hash = weightHash(c, op2.get());
     tr.useChainOf(c);
     const auto key = std::make_tuple(weight_hash.first, weight_hash.second, shape_b, T);
     auto it = tr.weight_tau_.find(key);
     if (it == tr.weight_tau_.end()) {
         EnDecoder endec(c);
         const Message src = endec.decode(op2.get());
-        // decoded values carry the encoding's rounding noise (about sqrt(N) / 2^43 at this scale): "zero" and "equal"
-        // are taken up to 2^-24
-        const double tol = std::ldexp(1.0, -24);
-        bool rest_zero = true, rest_equal = true;
-        for (i64 j = block; j < slots && (rest_zero || rest_equal); j++) {
-            if (std::abs(src[(u64)j]) >= tol) rest_zero = false;
-            if (std::abs(src[(u64)j] - src[(u64)(j % block)]) >= tol) rest_equal = false;
-        }
+        const int layout = weightLayout(src, block, slots);
         MatrixTransformer::WeightTau entry{Plaintext(c), 0};
-        if (rest_zero || rest_equal) {
-            const bool first_only = rest_zero && block < slots;
+        if (layout != 0) {
+            const bool first_only = layout == 2;
             Message dst(src.getLogSlots(), 0);
             const i64 height = slots / w;
             for (i64 r = 0; r < height; r++)
@@ -1886,7 +1890,7 @@ bool multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, con
                     dst[(u64)(r * w + cc)] = src[(u64)((rb + (i + j) % k) * w + cb + j)];
                 }
             entry.tau = endec.encodeExtended(dst, T + 2, c->delta[T + 1]);
-            entry.layout = first_only ? 2 : 1;
+            entry.layout = layout;
         }
         if (tr.weight_tau_order_.size() >= 256) {   // bounded: the oldest weight is prepared again if it comes back
             tr.weight_tau_.erase(tr.weight_tau_order_.front());
@@ -1964,6 +1968,109 @@ bool multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, con
     res.get().allocate(2, T, 0);
     ck(hemm_rescale(c->dev, mid.data(), lo * N, res.get().buf_.data(), (lo - 1) * N, (uint32_t)lo, 2, nullptr));
     res_out = res;
+    return true;
+}
+
+// The same product over the diagonals of B, without sigma and tau: C[i][c] = sum_r A[i][c + r] B[c + r][c], a sum over the rotations of A
+// whose factors are the same in every row (hemm_diagonal_tables).  In baby and giant steps, 2 k / g of g,
+//     C = sum_t rho^(s_t)( sum_j rho^j(A) (.) Q_tj ),
+// g - 1 rotations of A from one ModUp stay in the extended basis, where the inner sums are taken (hemm_diagonal_sums); one ModDown merged
+// with the rescale leaves them at level T, and the giant rotations are terms of one sum with one ModDown.  g + 2 k / g - 2 key products of
+// few limbs instead of k - 1 after two transforms, and one level instead of three: A is only truncated to level T + 1, the
+// diagonals' scale takes it to that of level T.  128 x 128 tiles, pair layout, T = 4: 621 us, 1444 through the shifts above.
+// Takes what multMatMatPlainFused takes where rows and inside of the tiles are the same power of two; where only the first block of B is not
+// zero, the others of A have to be empty as well (the diagonals are the same in every block).
+// A baby step is one key product, a giant step also its share of a ModDown and a ModUp: twice as many baby steps as giant ones at least.  g = k / 8 /
+// k / 4, us: 128 x 128 tiles 672 / 621, 64 x 64 263 / 237, 32 x 32 (a quarter and half of k) 153 / 154.
+static i64 plainBabyCount(i64 k) { return std::min<i64>(32, 2 * bsgsBabyCount(k)); }
+std::vector<u64> plainDiagonalRotations(i64 k, u64 log_slots) {
+    std::vector<u64> r;
+    const i64 g = plainBabyCount(k), slots = i64(1) << log_slots;
+    if (g < 4) return r;
+    for (i64 j = 1; j < g; j++) r.push_back((u64)j);
+    for (i64 t = g; t < k; t += g) r.push_back((u64)t);
+    for (i64 t = g; t <= k; t += g) r.push_back((u64)(slots - t));
+    return r;
+}
+
+bool multMatMatPlainDiagonals(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2, u64 T,
+                              MatrixTransformer &tr, bool a_single, CtxtTensor &res_out) {
+    const Context &c = eval.getContext();
+    const i64 rows = op1.getHeight(), cols = op2.getWidth();
+    const i64 k = pow2ceil(commonInside(op1, op2)), w = commonBlockWidth(op1, op2), g = plainBabyCount(k), giants = 2 * k / g;
+    const i64 slots = (i64)(c->N / 2), block = k * w;
+    const Ciphertext &a = op1.get();
+    const u64 level = a.getLevel(), nq = T + 2, N = c->N, E = nq + c->nP, lo = nq - 1;
+    // what is refused is left to the general product to refuse
+    if (rows != k || block > slots || slots % block != 0 || level < T + 3 || level >= c->nQ || a.getRescaleCounter() != 0 || a.getNumPoly() != 2 ||
+        std::min(level, op2.getLevel()) < 1 + btp.getMinLevelForBootstrap() || level < 4 + btp.getMinLevelForBootstrap())
+        return false;
+    size_t words = 0;
+    ck(hemm_diagonal_table_words(c->dev, (uint32_t)k, (uint32_t)w, (uint32_t)g, (uint32_t)nq, &words));
+    if (words == 0) return false;
+    // ---- the diagonals, at the scale that takes the sums from level's to T's
+    tr.useChainOf(c);
+    const auto hash = weightHash(c, op2.get());
+    const auto key = std::make_tuple(hash.first, hash.second, TileTensorShape(k, cols, w), T, level);
+    auto it = tr.weight_diagonals_.find(key);
+    if (it == tr.weight_diagonals_.end() || (it->second.layout == 2 && a_single && it->second.tables.data() == nullptr)) {
+        const Message src = EnDecoder(c).decode(op2.get());
+        MatrixTransformer::WeightDiagonals entry{DeviceBuffer(), weightLayout(src, block, slots)};
+        if (entry.layout == 1 || (entry.layout == 2 && a_single)) {
+            DeviceBuffer first(c, 2 * (size_t)block);
+            if (hipMemcpy(first.data(), &src[0], (size_t)block * sizeof(Complex), hipMemcpyHostToDevice) != hipSuccess) throw RuntimeException("hipMemcpy");
+            entry.tables = DeviceBuffer(c, words);
+            ck(hemm_diagonal_tables(c->dev, (const double *)first.data(), (uint32_t)k, (uint32_t)w, (uint32_t)g,
+                                    c->delta[T] * (double)c->q[T + 1] / c->delta[level], (uint32_t)nq, entry.tables.data(), nullptr));
+        }
+        if (it == tr.weight_diagonals_.end()) {
+            if (tr.weight_diagonals_order_.size() >= 256) {   // bounded: the oldest weight is prepared again if it comes back
+                tr.weight_diagonals_.erase(tr.weight_diagonals_order_.front());
+                tr.weight_diagonals_order_.erase(tr.weight_diagonals_order_.begin());
+            }
+            tr.weight_diagonals_order_.push_back(key);
+            it = tr.weight_diagonals_.emplace(key, std::move(entry)).first;
+        } else {
+            it->second = std::move(entry);
+        }
+    }
+    if (it->second.tables.data() == nullptr) return false;
+    // ---- rotations of A in the extended basis
+    const KeyPack &pack = eval.getKeyPack();
+    const Rot rot(c);
+    DeviceBuffer cut(c, 2 * nq * N), y(c, (size_t)giants * 2 * E * N), v(c, (size_t)giants * 2 * lo * N);
+    ck(hemm_mul_scalar(c->dev, a.buf_.data(), a.polyStride(), std::vector<u64>(nq, 1).data(), cut.data(), nq * N, (uint32_t)nq, 0, 2, nullptr));
+    {
+        const Sources x = extendSources(c, cut.data(), 1, nq, nullptr, false);
+        DeviceBuffer rotated(c, (size_t)(g - 1) * 2 * E * N);
+        std::vector<hemm_rot_term> terms;
+        std::vector<uint32_t> off{0};
+        for (i64 j = 1; j < g; j++) {
+            terms.push_back(term(x.extOf(0), x.pbOf(0), pack, rot.galois(j), nullptr));
+            off.push_back((uint32_t)terms.size());
+        }
+        ck(hemm_hoisted_terms(c->dev, terms.data(), off.data(), (uint32_t)(g - 1), (uint32_t)nq, rotated.data(), x.premultiplied(), nullptr));
+        ck(hemm_diagonal_sums(c->dev, rotated.data(), cut.data(), nq * N, (uint32_t)k, (uint32_t)w, (uint32_t)g, (uint32_t)nq,
+                              it->second.tables.data(), y.data(), nullptr));
+    }
+    // ---- divided by P and rescaled, rotated and added up
+    {
+        DeviceBuffer ws(c, (size_t)giants * 2 * lo * N);
+        ck(hemm_moddown_batch(c->dev, y.data(), (uint32_t)nq, (uint32_t)(2 * giants), 1, v.data(), lo * N, ws.data(), nullptr));
+    }
+    const u64 *rotating = v.data() + 2 * lo * N;   // the first sum stays where it is
+    const Sources s = extendSources(c, rotating, (size_t)giants - 1, lo, nullptr, false);
+    std::vector<hemm_rot_term> terms;
+    for (i64 t = 1; t < giants; t++)
+        terms.push_back(term(s.extOf((size_t)t - 1), s.pbOf((size_t)t - 1), pack, rot.galois(t < giants / 2 ? t * g : (t - giants) * g), nullptr));
+    terms.push_back(keylessTerm(v.data(), v.data() + lo * N, nullptr));
+    const std::vector<uint32_t> off{0, (uint32_t)terms.size()};
+    CtxtTensor res(c, rows, cols, w);
+    res.get().allocate(2, T, 0);
+    DeviceBuffer ws(c, 2 * lo * N);
+    ck(hemm_hoisted_moddown(c->dev, terms.data(), off.data(), 1, (uint32_t)lo, s.premultiplied(), 0, y.data(), res.get().buf_.data(), lo * N,
+                            ws.data(), nullptr));
+    res_out = std::move(res);
     return true;
 }
 

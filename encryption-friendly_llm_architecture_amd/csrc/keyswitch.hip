@@ -993,6 +993,8 @@ static KsTables *g_tables_of(const hemm_context *c) {
     r.tabs[c] = t;
     return t;
 }
+const Cst *pmod_table(const hemm_context *c) { return g_tables_of(c)->dev + g_tables_of(c)->pmod_off; }
+
 void hemm_keyswitch_tables_free(const hemm_context *c) {
     KsRegistry &r = ks_registry();
     std::lock_guard<std::mutex> lk(r.mu);
@@ -1540,7 +1542,7 @@ static void sum_limbs(hemm_context *c, const HoistedList &l, int first, int n_ou
         memcpy(a.off, l.offsets, (size_t)(n_out + 1) * sizeof(u32));
     }
     const LimbList ll = limbs_default(c, nq, 1);
-    const Cst *pm = g_tables_of(c)->dev + g_tables_of(c)->pmod_off;
+    const Cst *pm = pmod_table(c);
     LimbList kind[2];   // double precision, integers
     int n_kind[2] = {0, 0};
     memset(kind, 0, sizeof(kind));

@@ -1160,7 +1160,7 @@ def mult_mat_mat_cc_reuse_fused(orc, tmp, b, step, rescale_after=False):
     return orc.rescale(res) if rescale_after else res
 
 
-def mult_mat_mat_pc_lazy(orc, a, b_pt, T, n, w):
+def mult_mat_mat_pc_shifts(orc, a, b_pt, T, n, w):
     """Plaintext x ciphertext product with ONE ModDown: every column shift of sigma(A) stays in the extended basis,
     is multiplied there by its column mask and by tau(B) rotated k w slots (a plaintext over the extended basis,
     encoded at the scale of level T+1), all n - 1 shifts are summed, the unshifted term P * (mask_0 tau(B)) sigma(A)
@@ -1208,6 +1208,72 @@ def mult_mat_mat_pc_lazy(orc, a, b_pt, T, n, w):
     res = orc.rescale(mid)
     res.scale = orc.delta[T]
     return res
+
+
+def _plain_tile(orc, b_pt, n, w):
+    """(slot values, whether only the first tile block is not zero) of a plaintext whose tile blocks are equal or zero but for the
+    first ("zero" and "equal" up to 2^-24: decoded values carry the encoding's rounding noise); None for any other."""
+    slots, block = orc.slots, n * w
+    if block > slots or slots % block:
+        return None
+    v = OracleEval(orc).pt_values(b_pt)
+    blocks = v.reshape(slots // block, block)
+    tol = 2.0 ** -24
+    rest_zero = bool(np.all(np.abs(blocks[1:]) < tol))
+    rest_equal = bool(np.all(np.abs(blocks[1:] - blocks[0]) < tol))
+    if not (rest_zero or rest_equal):
+        return None
+    return v, rest_zero and block < slots
+
+
+def plain_diagonal(v, n, w, r, back, slots):
+    """rho^-back of the diagonal r of a plaintext tile: B[c + r][c] in column c of every row, zero where c + r lies outside."""
+    c = np.arange(w)
+    row = c % n + r
+    inside = (row >= 0) & (row < n)
+    p = np.where(inside, v[np.where(inside, row, 0) * w + c], 0)
+    return np.tile(np.roll(p, back), slots // w)
+
+
+def mult_mat_mat_pc_lazy(orc, a, b_pt, T, n, w, a_known=True):
+    """Plaintext x ciphertext product over the diagonals of B, C = sum_t rho^(s_t)(sum_j rho^j(A) (.) Q_tj) with
+    Q_tj = rho^(-s_t)(diagonal s_t + j): g - 1 rotations of A, truncated to level T + 1, stay in the extended basis, where the
+    inner sums are taken; one ModDown merged with the rescale takes each to level T; the giant rotations are terms of one sum
+    with one ModDown.  a_known: nothing of A lies outside its first tile block; where it may and only the first block of B is not
+    zero, and for tiles of less than 8 columns, the product goes through the shifts of sigma(A).  None for plaintexts of other forms."""
+    from .oracle import Ct, Pt
+    tile = _plain_tile(orc, b_pt, n, w)
+    if tile is None:
+        return None
+    v, first_only = tile
+    slots, g = orc.slots, 1
+    while 4 * g * g <= 2 * n:
+        g *= 2
+    g = min(32, 2 * g)
+    if g < 4 or (first_only and not a_known):
+        return mult_mat_mat_pc_shifts(orc, a, b_pt, T, n, w)
+    giants, nq = 2 * n // g, T + 2
+    q = np.array([orc.mods[i] for i in orc.ext_primes(T + 1)], dtype=np.uint64)[:, None]
+    scale = orc.delta[T] * float(orc.q[T + 1]) / orc.delta[a.level]
+    x = [np.ascontiguousarray(p[:nq]) for p in a.data]
+    ext = orc.modup(x[1])
+    rotated = [np.zeros((2, nq + orc.nP, orc.N), dtype=np.uint64)]
+    for pol in range(2):
+        rotated[0][pol, :nq] = orc.mul_p_residues(x[pol])
+    rotated += [orc.hoisted_sum([(ext, x[0], j, None)], nq) for j in range(1, g)]
+    sums = []
+    for t in range(giants):
+        s = t * g if t < giants // 2 else (t - giants) * g
+        y = np.zeros_like(rotated[0])
+        for j in range(g):
+            d = orc.encode_ext(plain_diagonal(v, n, w, s + j, s, slots), T + 1, scale=scale)
+            for pol in range(2):
+                y[pol] = (y[pol] + orc.ext_plain_product(Pt(rotated[j][pol], 1.0), d, 1).data) % q
+        sums.append((s, Ct(orc.moddown_drop(y, nq, True), orc.delta[T])))
+    terms = [(orc.modup(u.data[1]), u.data[0], s % slots, None) for s, u in sums[1:]]
+    u = sums[0][1]
+    terms.append((u.data[1], u.data[0], ("none",), None))
+    return Ct(orc.moddown_drop(orc.hoisted_sum(terms, T + 1), T + 1, False), orc.delta[T])
 
 
 def weights_diagonal_to_row4(w1, w2, w3, w4, slots):
