@@ -690,7 +690,7 @@ int hemm_diagonal_table_words(hemm_context *ctx, uint32_t k, uint32_t w, uint32_
     int nl;
     chain_limbs(ctx, nq, 1, &nl);
     need(words, "null operand");
-    *words = diagonals_ok(ctx, k, w, g) ? diagonal_table_words(ctx, k, w, g, (int)nq) : 0;
+    *words = diagonals_ok(ctx, k, w, g, (int)nq) ? diagonal_table_words(ctx, k, w, g, (int)nq) : 0;
     HEMM_CATCH
 }
 
@@ -700,21 +700,27 @@ int hemm_diagonal_tables(hemm_context *ctx, const double *block, uint32_t k, uin
     int nl;
     chain_limbs(ctx, nq, 1, &nl);
     need(block && tables, "null operand");
-    need(diagonals_ok(ctx, k, w, g), "no diagonal form for this shape or these primes");
+    need(diagonals_ok(ctx, k, w, g, (int)nq), "no diagonal form for this shape or these primes");
     launch_diagonal_tables(ctx, block, k, w, g, scale, (int)nq, (u64 *)tables, on_stream(ctx, stream));
     check_launch();
     HEMM_CATCH
 }
 
-int hemm_diagonal_sums(hemm_context *ctx, const uint64_t *rotated, const uint64_t *a, size_t a_stride, uint32_t k, uint32_t w, uint32_t g,
-                       uint32_t nq, const uint64_t *tables, uint64_t *y, void *stream) {
+int hemm_diagonal_sums(hemm_context *ctx, const hemm_rot_term *rotations, const uint64_t *a, size_t a_stride, uint32_t k, uint32_t w,
+                       uint32_t g, uint32_t nq, int b_premultiplied, const uint64_t *tables, uint64_t *y, void *stream) {
     HEMM_TRY
     int nl;
     chain_limbs(ctx, nq, 1, &nl);
-    need(rotated && a && tables && y, "null operand");
+    need(rotations && a && tables && y, "null operand");
     need(a_stride >= (size_t)nq * (size_t)ctx->N, "polynomial stride below one polynomial");
-    need(diagonals_ok(ctx, k, w, g), "no diagonal form for this shape or these primes");
-    launch_diagonal_sums(ctx, (const u64 *)rotated, (const u64 *)a, a_stride, k, w, g, (int)nq, (const u64 *)tables, (u64 *)y,
+    need(diagonals_ok(ctx, k, w, g, (int)nq), "no diagonal form for this shape or these primes");
+    need(((uintptr_t)a | (uintptr_t)y) % 16 == 0 && a_stride % 2 == 0, "residue pairs need an alignment of 16 bytes");
+    std::vector<uint32_t> each(g);
+    for (uint32_t j = 0; j < g; j++) each[j] = j;
+    for (uint32_t j = 0; j + 1 < g; j++)
+        need(rotations[j].evk && rotations[j].b && !rotations[j].mask && !rotations[j].pt, "a rotation has a key, both polynomials and no factors");
+    const Terms t(ctx, rotations, each.data(), g - 1, on_stream(ctx, stream));
+    launch_diagonal_sums(ctx, t.list, (const u64 *)a, a_stride, k, w, g, (int)nq, b_premultiplied != 0, (const u64 *)tables, (u64 *)y,
                          on_stream(ctx, stream));
     check_launch();
     HEMM_CATCH

@@ -278,13 +278,13 @@ int masked_arg_capacity();
 // table[j][r] = mask[j][r << shift]; true when every aligned run of 2^shift residues of the mask is constant
 bool launch_compact_mask(hemm_context *c, const u64 *mask, int n_limbs, int shift, u64 *table, hipStream_t s);
 // Products with a plaintext matrix over its diagonals (diagonals.hip): k x k tiles, rows of w slots, g baby steps, 2k / g giant ones.
-bool diagonals_ok(const hemm_context *c, u32 k, u32 w, u32 g);
+bool diagonals_ok(const hemm_context *c, u32 k, u32 w, u32 g, int nq);
 size_t diagonal_table_words(const hemm_context *c, u32 k, u32 w, u32 g, int nq);
 // block: the first k rows of the matrix's slots, [k][w] complex doubles
 void launch_diagonal_tables(hemm_context *c, const double *block, u32 k, u32 w, u32 g, double scale, int nq, u64 *tables, hipStream_t s);
-// rotated: [g-1][2][nq+K][N], a: the ciphertext itself (chain limbs, polynomials a_stride apart), y: [2k/g][2][nq+K][N]
-void launch_diagonal_sums(hemm_context *c, const u64 *rotated, const u64 *a, size_t a_stride, u32 k, u32 w, u32 g, int nq, const u64 *tables,
-                          u64 *y, hipStream_t s);
+// l: the g - 1 rotations, one term each; a: the ciphertext itself (chain limbs, polynomials a_stride apart); y: [2k/g][2][nq+K][N]
+void launch_diagonal_sums(hemm_context *c, const HoistedList &l, const u64 *a, size_t a_stride, u32 k, u32 w, u32 g, int nq, bool b_premultiplied,
+                          const u64 *tables, u64 *y, hipStream_t s);
 const void *encode_roots(const hemm_context *c);     // complex roots of an encoding's butterflies (encode.hip)
 const Cst *pmod_table(const hemm_context *c);        // P mod q_j for the chain primes, on the device
 void launch_masked_sum_args(hemm_context *c, const void *terms_host, int n_terms, const u32 *group_off_host, int n_out,

@@ -29,6 +29,14 @@ struct RotTermDev {
 };
 #define ROT_TERM_COMPACT_KEY 1u
 #define ROT_TERM_EXT_ROTATED 2u
+// Term lists of up to HOISTED_ARG_TERMS terms and outputs travel in the kernel arguments (no staging copy before
+// the launch); longer lists are read from device memory.
+static_assert(sizeof(RotTermDev) == 80, "the C ABI builds these records on the host");
+#define HOISTED_ARG_TERMS 32
+struct HoistedArgs {
+    RotTermDev t[HOISTED_ARG_TERMS];
+    u32 off[HOISTED_ARG_TERMS + 1];
+};
 
 // Accesses to data that is touched once per launch (keys, masks, results): marked non-temporal so they do
 // not push the rotation sources, which every output gathers from, out of the L2.
@@ -555,15 +563,20 @@ __device__ __forceinline__ D2 gather_d2(const u64 *p, const bool swap) {
     }
     return to_d2(v);
 }
-// residues (n, n+1) of a key limb of a prime below 2^44 as doubles
-template <bool COMPACT>
-__device__ __forceinline__ D2 key_pair_fp(const __amdgpu_buffer_rsrc_t key, const u32 limb, const u32 n) {
-    if (!COMPACT) return to_d2(key_pair_u64(key, limb, n));
-    const u32x3 v = __builtin_amdgcn_raw_buffer_load_b96(key, n * 6u, limb, 2);   // one 12-byte load
+// residues (n, n+1) of a compact key's limb of a prime below 2^44: one 12-byte load, and the doubles in it
+__device__ __forceinline__ u32x3 key_record(const __amdgpu_buffer_rsrc_t key, const u32 limb, const u32 n) {
+    return __builtin_amdgcn_raw_buffer_load_b96(key, n * 6u, limb, 2);
+}
+__device__ __forceinline__ D2 key_record_fp(const u32x3 v) {
     D2 r;
     r.x = __hiloint2double((int)((v.z & 0xffffu) | 0x43300000u), (int)v.x) - 4503599627370496.0;
     r.y = __hiloint2double((int)((v.z >> 16) | 0x43300000u), (int)v.y) - 4503599627370496.0;
     return r;
+}
+template <bool COMPACT>
+__device__ __forceinline__ D2 key_pair_fp(const __amdgpu_buffer_rsrc_t key, const u32 limb, const u32 n) {
+    if (!COMPACT) return to_d2(key_pair_u64(key, limb, n));
+    return key_record_fp(key_record(key, limb, n));
 }
 #pragma clang fp contract(off)
 // The same residues in double precision (primes below 2^44); out_* are unreduced centred doubles.

@@ -1974,10 +1974,10 @@ bool multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, con
 // The same product over the diagonals of B, without sigma and tau: C[i][c] = sum_r A[i][c + r] B[c + r][c], a sum over the rotations of A
 // whose factors are the same in every row (hemm_diagonal_tables).  In baby and giant steps, 2 k / g of g,
 //     C = sum_t rho^(s_t)( sum_j rho^j(A) (.) Q_tj ),
-// g - 1 rotations of A from one ModUp stay in the extended basis, where the inner sums are taken (hemm_diagonal_sums); one ModDown merged
+// the inner sums are taken from g - 1 rotations of A in the extended basis, one ModUp for all (hemm_diagonal_sums); one ModDown merged
 // with the rescale leaves them at level T, and the giant rotations are terms of one sum with one ModDown.  g + 2 k / g - 2 key products of
 // few limbs instead of k - 1 after two transforms, and one level instead of three: A is only truncated to level T + 1, the
-// diagonals' scale takes it to that of level T.  128 x 128 tiles, pair layout, T = 4: 621 us, 1444 through the shifts above.
+// diagonals' scale takes it to that of level T.  128 x 128 tiles, pair layout, T = 4: 501 us, 1444 through the shifts above.
 // Takes what multMatMatPlainFused takes where rows and inside of the tiles are the same power of two; where only the first block of B is not
 // zero, the others of A have to be empty as well (the diagonals are the same in every block).
 // A baby step is one key product, a giant step also its share of a ModDown and a ModUp: twice as many baby steps as giant ones at least.  g = k / 8 /
@@ -2035,22 +2035,16 @@ bool multMatMatPlainDiagonals(const HomEvaluator &eval, const Bootstrapper &btp,
         }
     }
     if (it->second.tables.data() == nullptr) return false;
-    // ---- rotations of A in the extended basis
+    // ---- the inner sums, from rotations of A in the extended basis
     const KeyPack &pack = eval.getKeyPack();
     const Rot rot(c);
     DeviceBuffer cut(c, 2 * nq * N), y(c, (size_t)giants * 2 * E * N), v(c, (size_t)giants * 2 * lo * N);
     ck(hemm_mul_scalar(c->dev, a.buf_.data(), a.polyStride(), std::vector<u64>(nq, 1).data(), cut.data(), nq * N, (uint32_t)nq, 0, 2, nullptr));
     {
         const Sources x = extendSources(c, cut.data(), 1, nq, nullptr, false);
-        DeviceBuffer rotated(c, (size_t)(g - 1) * 2 * E * N);
         std::vector<hemm_rot_term> terms;
-        std::vector<uint32_t> off{0};
-        for (i64 j = 1; j < g; j++) {
-            terms.push_back(term(x.extOf(0), x.pbOf(0), pack, rot.galois(j), nullptr));
-            off.push_back((uint32_t)terms.size());
-        }
-        ck(hemm_hoisted_terms(c->dev, terms.data(), off.data(), (uint32_t)(g - 1), (uint32_t)nq, rotated.data(), x.premultiplied(), nullptr));
-        ck(hemm_diagonal_sums(c->dev, rotated.data(), cut.data(), nq * N, (uint32_t)k, (uint32_t)w, (uint32_t)g, (uint32_t)nq,
+        for (i64 j = 1; j < g; j++) terms.push_back(term(x.extOf(0), x.pbOf(0), pack, rot.galois(j), nullptr));
+        ck(hemm_diagonal_sums(c->dev, terms.data(), cut.data(), nq * N, (uint32_t)k, (uint32_t)w, (uint32_t)g, (uint32_t)nq, x.premultiplied(),
                               it->second.tables.data(), y.data(), nullptr));
     }
     // ---- divided by P and rescaled, rotated and added up

@@ -529,14 +529,6 @@ __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict_
     }
 }
 
-// Term lists of up to HOISTED_ARG_TERMS terms and outputs travel in the kernel arguments (no staging copy before
-// the launch); longer lists are read from device memory.
-static_assert(sizeof(RotTermDev) == 80, "the C ABI builds these records on the host");
-#define HOISTED_ARG_TERMS 32
-struct HoistedArgs {
-    RotTermDev t[HOISTED_ARG_TERMS];
-    u32 off[HOISTED_ARG_TERMS + 1];
-};
 // Register budget for five waves per SIMD (96 registers): the double-precision form needs 72, the integer and the mixed form
 // all 96.  The mixed form under a ModDown's tail spills three; with four waves and none a product at level 9 takes 122.1 instead of
 // 120.2 us, the projection of a 768-wide layer 10.46 instead of 10.33 ms.  COMPACT: the key layout of the launch (hoisted.h, key_limb).

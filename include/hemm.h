@@ -225,20 +225,22 @@ void hemm_abi_sizes(uint32_t *rot_term_bytes, uint32_t *lin_term_bytes);
 int hemm_sum_parts(hemm_context *ctx, const uint64_t *parts, uint32_t n_parts, uint32_t n_out, uint32_t nq, uint64_t *y,
                    void *stream);
 /* A plaintext matrix applied to every row of an encrypted one over its diagonals, in g baby and 2k / g giant steps: k x k tiles side by
- * side in rows of w slots (k, w, g powers of two, 4 <= g <= k <= w <= 512, 2w <= N; primes of 33 to 60 bits; N >= 1024).  With
- * rotations x_j = rho^j(A) in the extended basis (hemm_hoisted_terms, j = 1 .. g - 1, and x_0 = P A from `a` itself) and
+ * side in rows of w slots (k, w, g powers of two, 4 <= g <= k <= w <= 512, g <= 32, 2w <= N; primes of 33 to 60 bits; N >= 1024;
+ * nq limbs of at most three digits).  With
+ * rotations x_j = rho^j(A) in the extended basis (one term each as for hemm_hoisted_terms, without factors, j = 1 .. g - 1, and x_0 = P A from `a`
+ * itself) and
  * Q_tj = rho^(-s_t)(diagonal s_t + j) of the matrix, s_t = g t for t < k / g and g t - 2k above, the sums
  *     y[t] = sum_j x_j (.) Q_tj
  * are left in the extended basis, to be divided by P and rotated by s_t.  A B is the sum of the results.
  *   hemm_diagonal_table_words: words that the tables of the Q_tj take over nq + n_p limbs, 0 where there is no such form;
  *   hemm_diagonal_tables: from the first k rows of the matrix's slots, block [k][w] complex doubles on the device, encoded at `scale`;
- *   hemm_diagonal_sums: rotated [g-1][2][nq+n_p][N], a two polynomials of nq limbs a_stride words apart, y [2k/g][2][nq+n_p][N].
+ *   hemm_diagonal_sums: rotations[g-1], a two polynomials of nq limbs a_stride words apart, y [2k/g][2][nq+n_p][N].
  * Reference: MatrixUtils.cpp:1218-1305 (the same product through sigma, tau and k shifts). */
 int hemm_diagonal_table_words(hemm_context *ctx, uint32_t k, uint32_t w, uint32_t g, uint32_t nq, size_t *words);
 int hemm_diagonal_tables(hemm_context *ctx, const double *block, uint32_t k, uint32_t w, uint32_t g, double scale, uint32_t nq,
                          uint64_t *tables, void *stream);
-int hemm_diagonal_sums(hemm_context *ctx, const uint64_t *rotated, const uint64_t *a, size_t a_stride, uint32_t k, uint32_t w, uint32_t g,
-                       uint32_t nq, const uint64_t *tables, uint64_t *y, void *stream);
+int hemm_diagonal_sums(hemm_context *ctx, const hemm_rot_term *rotations, const uint64_t *a, size_t a_stride, uint32_t k, uint32_t w,
+                       uint32_t g, uint32_t nq, int b_premultiplied, const uint64_t *tables, uint64_t *y, void *stream);
 /* Run table of a mask over the extended basis (n_limbs = nq + n_p) that is constant over aligned runs of 2^shift
  * coefficients: table[j][r] = { v = mask[j][r << shift], floor(v * 2^64 / prime_j) } (2 * n_limbs * (N >> shift)
  * words; the second word lets the 60-bit limbs multiply by v as by a constant); *is_constant = 0 (and the table is
