@@ -256,8 +256,7 @@ __device__ __forceinline__ void cols_lifted_body(const __amdgpu_buffer_rsrc_t li
                                                  const ModQ m) {
     typedef Slab<LR, 8> S;
     typename F::E x[8];
-#pragma unroll
-    for (int k = 0; k < 8; k++) x[k] = f.from_canonical(lifted(ls, coef, ((u32)S::r_outer_s(k) << 8) + S::col(), m));
+    lifted_inputs(f, x, ls, coef, m, [](const int k) { return ((u32)S::r_outer_s(k) << 8) + S::col(); });
     cols_forward<LR>(limb, (const typename F::W *)tw_int, f, x, (typename F::E *)lds_raw);
 }
 template <int LR>

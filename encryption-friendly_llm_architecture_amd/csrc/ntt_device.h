@@ -145,6 +145,11 @@ struct IntFieldT {
     __device__ __forceinline__ u64 scale_to_canonical(E v) const {
         return csub(mul_shoup_lazy(v, ni, nis, q), q, nq1);
     }
+    // a signed integer as an input of a forward transform, where it is as small as from_signed takes it: below 2q
+    __device__ __forceinline__ bool takes_signed(long long v) const { return (u64)v + q < q2; }
+    __device__ __forceinline__ E from_signed(long long v) const { return (u64)v + q; }
+    // v - a s, canonical, for canonical a and s
+    __device__ __forceinline__ u64 minus_product(E v, u64 a, u64 s, const ModQ &m) const { return submod(to_canonical(v), mulmod(a, s, m), q); }
     // (y - v) * cst mod q for a transformed value v and a canonical minuend y
     __device__ __forceinline__ u64 sub_scale(E v, u64 y, const Tw cst) const {
         const u64 c = to_canonical(v);
@@ -212,6 +217,15 @@ struct FpField {
     }
     __device__ __forceinline__ u64 to_canonical(E v) const { return centred_to_canonical(reduce(v)); }
     __device__ __forceinline__ u64 scale_to_canonical(E v) const { return centred_to_canonical(mulmod(v, ni, niinv)); }
+    // integers of magnitude below 2^51 are exact, and so is what is left of them below q / 2
+    __device__ __forceinline__ bool takes_signed(long long v) const { return (u64)v + (1ull << 51) < 1ull << 52; }
+    __device__ __forceinline__ E from_signed(long long v) const {
+        return reduce(__longlong_as_double(v + 0x4338000000000000ll) - 6755399441055744.0);
+    }
+    __device__ __forceinline__ u64 minus_product(E v, u64 a, u64 s, const ModQ &) const {
+        const double w = from_canonical(s);
+        return to_canonical(v - mulmod(from_canonical(a), w, w * qinv));
+    }
     __device__ __forceinline__ u64 sub_scale(E v, u64 y, const Tw cst) const {
         const double w = (double)cst.w;
         return centred_to_canonical(mulmod(from_canonical(y) - v, w, w * qinv));
@@ -349,6 +363,29 @@ __device__ __forceinline__ u64 lifted(const LiftSource &ls, const long long *__r
     const int e = sample_error(ls.error_key, n);
     return addmod(r, e >= 0 ? (u64)e : m.q - (u64)(-e), m.q);
 }
+// The coefficients of a thread, number k of them at index(k), as inputs of a forward transform.  Nearly always they are small enough to be taken as
+// they are, in two instructions for primes of 44 bits and more and five for the others; a Barrett reduction of each (and a modular
+// addition of the error) is 45.
+template <int P, class F, class INDEX>
+__device__ __forceinline__ void lifted_inputs(const F &f, typename F::E (&x)[P], const LiftSource &ls, const long long *__restrict__ coef,
+                                              const ModQ &m, const INDEX index) {
+    long long v[P];
+    bool small = true;
+#pragma unroll
+    for (int k = 0; k < P; k++) v[k] = coef[index(k)];
+#pragma unroll
+    for (int k = 0; k < P; k++) {
+        if (ls.with_error) v[k] = (long long)((u64)v[k] + (u64)(long long)sample_error(ls.error_key, index(k)));
+        small = small && f.takes_signed(v[k]);
+    }
+    if (small) {
+#pragma unroll
+        for (int k = 0; k < P; k++) x[k] = f.from_signed(v[k]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < P; k++) x[k] = f.from_canonical(lifted(ls, coef, index(k), m));
+    }
+}
 // The eight coefficients of a thread as a basis conversion computed on the fly: coefficient k is sum_i v_i * hat_i mod q over
 // the n_src <= NS source limbs (pre-scaled, the same sums as the stand-alone conversion kernels), read at voff + off(k) inside a
 // limb; so[i]: byte offset of source limb i.
@@ -477,12 +514,15 @@ __device__ __forceinline__ void rows_body(u64 *__restrict__ row, const Tw *__res
 #pragma unroll
             for (int k = 0; k < P; k++) o[cm + step * k] = f.sub_scale(l[padc(cm + step * k)], mv[k], cst);
         } else if (TAIL == TAIL_ENCRYPT) {
-#pragma unroll 4
+            u64 s[P], a[P];
+#pragma unroll
+            for (int k = 0; k < P; k++) s[k] = sec.sk[cm + step * k];
+            sample_uniform(sec.key, (u64)((r << 8) + (u32)cm), (u64)step, sec.m, a);
+#pragma unroll
             for (int k = 0; k < P; k++) {
                 const int e = cm + step * k;
-                const u64 a = sample_uniform(sec.key, (r << 8) + (u32)e, sec.m);
-                o[e] = submod(f.to_canonical(l[padc(e)]), mulmod(a, sec.sk[e], sec.m), sec.m.q);
-                sec.out[e] = a;
+                o[e] = f.minus_product(l[padc(e)], a[k], s[k], sec.m);
+                sec.out[e] = a[k];
             }
         } else {
 #pragma unroll
@@ -490,7 +530,7 @@ __device__ __forceinline__ void rows_body(u64 *__restrict__ row, const Tw *__res
         }
     } else {
         if (LOAD == LOAD_DECRYPT) {
-#pragma unroll 4
+#pragma unroll
             for (int k = 0; k < P; k++) {
                 const int e = cm + step * k;
                 lc[padc(e)] = addmod(ld[e], mulmod(sec.in[e], sec.sk[e], sec.m), sec.m.q);

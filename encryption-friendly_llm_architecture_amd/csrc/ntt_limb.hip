@@ -62,8 +62,7 @@ __device__ __forceinline__ void limb_forward(u64 *__restrict__ limb, const Tw *_
         converted_inputs<NS>(f, x, src, S::voff(), so, h, n_src, m,
                              [](const int k) { return S::off(k); });
     } else if (NS == LIFTED) {
-#pragma unroll
-        for (int k = 0; k < P; k++) x[k] = f.from_canonical(lifted(ls, coef, (S::voff() + S::off(k)) >> 3, m));
+        lifted_inputs(f, x, ls, coef, m, [](const int k) { return (S::voff() + S::off(k)) >> 3; });
     } else {
 #pragma unroll
         for (int k = 0; k < P; k++) x[k] = f.from_canonical(buf_load<u64>(src, S::voff(), S::off(k)));

@@ -15,15 +15,27 @@ __device__ __forceinline__ u64 sm64(u64 x) {
     return z ^ (z >> 31);
 }
 __device__ __forceinline__ u64 draw(u64 key, u64 ctr) { return sm64(key + ctr * 0x9E3779B97F4A7C15ull); }
-__device__ __forceinline__ u64 sample_uniform(const u64 key, const u64 i, const ModQ &m) {
+// from attempt t on
+__device__ __forceinline__ u64 sample_uniform(const u64 key, const u64 i, const ModQ &m, u64 t = 0) {
     const u64 mask = (1ull << m.k) - 1;
     u64 x = 0;
     // acceptance is at least 1/2 per attempt; 4096 attempts cannot all fail in practice and bound the loop
-    for (u64 t = 0; t < 4096; t++) {
+    for (; t < 4096; t++) {
         x = draw(sm64(key + t), i) & mask;
         if (x < m.q) break;
     }
     return x;
+}
+// n of them, `step` apart: the first attempts of all are independent of each other, and for primes just below a power of two nearly
+// always the only ones (one after the other behind the loop's branch, eight of them were most of an encryption's last pass)
+template <int n>
+__device__ __forceinline__ void sample_uniform(const u64 key, const u64 i, const u64 step, const ModQ &m, u64 (&x)[n]) {
+    const u64 first = sm64(key), mask = (1ull << m.k) - 1;
+#pragma unroll
+    for (int k = 0; k < n; k++) x[k] = draw(first, i + step * (u64)k) & mask;
+#pragma unroll
+    for (int k = 0; k < n; k++)
+        if (x[k] >= m.q) x[k] = sample_uniform(key, i + step * (u64)k, m, 1);
 }
 __device__ __forceinline__ int sample_error(const u64 key, const u64 i) {
     const u64 x = draw(key, i), M21 = (1ull << 21) - 1;
