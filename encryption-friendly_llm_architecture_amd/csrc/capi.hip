@@ -534,7 +534,7 @@ struct Terms {
         build_rot_terms(ctx, terms, group_offsets, n_out, d, off);
         for (const RotDev &t : d)
             need(t.flags == d[0].flags, "all terms of a hoisted sum must use the same key layout");
-        list = HoistedList{d.data(), off.data(), nullptr, nullptr, (int)d.size()};
+        list = HoistedList{d.data(), off.data(), nullptr, nullptr, (int)d.size(), nullptr, 1};
         if ((int)d.size() <= hoisted_arg_capacity() && (int)n_out <= hoisted_arg_capacity()) return;
         void *off_dev = nullptr;
         list.terms_dev = upload_desc(ctx, d.data(), d.size() * sizeof(RotDev), off.data(), (n_out + 1) * sizeof(uint32_t), &off_dev,

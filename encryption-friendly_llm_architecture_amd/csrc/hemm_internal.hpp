@@ -258,6 +258,10 @@ struct HoistedList {
     const void *terms_dev;
     const u32 *offsets_dev;
     int n_terms;
+    // a single key switch whose ModUp is not finished: the first term's ext holds the column passes' results only, and the digits' own
+    // limbs are those of this polynomial [nq][N] (nullptr: none of that), of its automorphism switched_galois (1: none)
+    const u64 *switched;
+    u32 switched_galois;
 };
 int hoisted_arg_capacity();
 void launch_hoisted_terms(hemm_context *c, const HoistedList &l, int n_out, int nq, u64 *y, bool b_premultiplied, hipStream_t s);

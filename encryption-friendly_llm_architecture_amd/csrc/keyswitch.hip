@@ -403,6 +403,37 @@ struct SumTail {       // all limbs of the launch end in the ModDown's tail
     ResultList list;
     __device__ __forceinline__ bool takes_rows(u32) const { return true; }
 };
+// What becomes of residues (n, n + 1) of both polynomials of output o, n = 512 chunk + 2 i in the workgroup's thread i
+template <class ROWS>
+__device__ __forceinline__ void sum_done(const u64 (&rb)[2], const u64 (&ra)[2], u64 *__restrict__ y, const ModQ *__restrict__ modq,
+                                         const double *__restrict__ fp, const int prime, const bool fp_limb, const u32 o, const u32 j,
+                                         const u32 chunk, const u32 n, const int E, const int logN, const ROWS &rows) {
+    const size_t N = (size_t)1 << logN;
+    __shared__ u64 lds[4 * ROWPAD];
+    const u32 first = chunk * 512;
+    if constexpr (std::is_same<ROWS, SumTail>::value) {
+        const u64 *cb = rows.conv + ((size_t)o * 2 * rows.nq_out + j) * N + first, *ca = cb + (size_t)rows.nq_out * N;
+        u64 *ob = (rows.listed ? rows.list.at[o] : rows.out + (size_t)o * 2 * rows.out_stride) + (size_t)j * N + first;
+        u64 *oa = ob + rows.out_stride;
+        const Tw *tw = rows.tw + ((size_t)prime << logN), cst = rows.cst[j];
+        if (fp_limb)
+            rows_under_products(FpField(modq, nullptr, nullptr, fp, prime), rb, ra, cb, ca, ob, oa, lds, tw, logN - 8, 2 * chunk, cst);
+        else
+            rows_under_products(IntFieldT<true>(modq, nullptr, nullptr, fp, prime), rb, ra, cb, ca, ob, oa, lds, tw, logN - 8, 2 * chunk, cst);
+    } else {
+        u64 *yb = y + (((size_t)o * 2 + 0) * E + j) * N, *ya = y + (((size_t)o * 2 + 1) * E + j) * N;
+        if (rows.takes_rows(j)) {
+            const Tw *tw = rows.tw + ((size_t)prime << logN);
+            if (fp_limb)
+                rows_of_products(FpField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
+            else
+                rows_of_products(IntField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
+            return;
+        }
+        stream_store2(yb + n, rb[0], rb[1]);
+        stream_store2(ya + n, ra[0], ra[1]);
+    }
+}
 template <int MODE, bool COMPACT, int S, class ROWS>
 __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict__ terms,
                                                    const u32 *__restrict__ group_off, u64 *__restrict__ y,
@@ -502,31 +533,7 @@ __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict_
             }
         }
     }
-    __shared__ u64 lds[4 * ROWPAD];
-    const u32 first = chunk * 512;
-    const bool fp_limb = MODE == 1 || (MODE == 0 && fq != 0.0);
-    if constexpr (std::is_same<ROWS, SumTail>::value) {
-        const u64 *cb = rows.conv + ((size_t)o * 2 * rows.nq_out + j) * N + first, *ca = cb + (size_t)rows.nq_out * N;
-        u64 *ob = (rows.listed ? rows.list.at[o] : rows.out + (size_t)o * 2 * rows.out_stride) + (size_t)j * N + first;
-        u64 *oa = ob + rows.out_stride;
-        const Tw *tw = rows.tw + ((size_t)prime << logN), cst = rows.cst[j];
-        if (fp_limb)
-            rows_under_products(FpField(modq, nullptr, nullptr, fp, prime), rb, ra, cb, ca, ob, oa, lds, tw, logN - 8, 2 * chunk, cst);
-        else
-            rows_under_products(IntFieldT<true>(modq, nullptr, nullptr, fp, prime), rb, ra, cb, ca, ob, oa, lds, tw, logN - 8, 2 * chunk, cst);
-    } else {
-        u64 *yb = y + (((size_t)o * 2 + 0) * E + j) * N, *ya = y + (((size_t)o * 2 + 1) * E + j) * N;
-        if (rows.takes_rows(j)) {
-            const Tw *tw = rows.tw + ((size_t)prime << logN);
-            if (fp_limb)
-                rows_of_products(FpField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
-            else
-                rows_of_products(IntField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
-            return;
-        }
-        stream_store2(yb + n, rb[0], rb[1]);
-        stream_store2(ya + n, ra[0], ra[1]);
-    }
+    sum_done(rb, ra, y, modq, fp, prime, MODE == 1 || (MODE == 0 && fq != 0.0), o, j, chunk, n, E, logN, rows);
 }
 
 // Register budget for five waves per SIMD (96 registers): the double-precision form needs 72, the integer and the mixed form
@@ -551,6 +558,161 @@ HOISTED_KERNEL hoisted_terms_list_kernel(const RotTermDev *__restrict__ terms, c
                                       b_premultiplied, n_out, jmap, n_j, koff, rows);
 }
 #undef HOISTED_KERNEL
+
+// A single key switch with the last pass of its ModUp inside: the digits' converted limbs come as their column pass has left them, a
+// workgroup runs the row stages on the two rows of each that its 512 products read, a wavefront per row, and takes the limbs that
+// a digit has of its own from the polynomial itself -- no launch for the rows, no copies of those limbs, and the extended digits are neither
+// written in full nor read back.  (A hoisted sum, whose digits serve many rotations, reads finished rows.)  Bound by the number of launches and by
+// a part-filled round of each; three digits need 168 registers (four waves per SIMD would spill 24).
+// Rotation on 24 primes of 60 bits, level 20: rows 21 + sums 11 and 35 us in three launches, sums with the rows in them 14 and 44; 140.3 -> 129.4 us,
+// at N = 2^13 44.7 -> 41.0, product at level 9 119.4 -> 111.5.
+struct SwitchedPoly {
+    const u64 *in;     // [nq][N]
+    u32 galois;        // the switch is of this automorphism of it; 1: none
+    u32 alpha;         // limbs of a digit
+};
+// B digits; keyed: ext with the column passes' results [B][E][N], key (plain), b or nullptr with its own automorphism; own: a term without a
+// key as in a hoisted sum, ext == nullptr: none
+template <bool FP, int B, class F>
+__device__ __forceinline__ void switched_pair(const F f, const FpMod fm, const ModQ &m, const Cst pmod, const RotTermDev &keyed, const RotTermDev &own,
+                                              const SwitchedPoly &sw, const Tw *__restrict__ tw_int, u64 *lds_raw, const int prime, const u32 j,
+                                              const u32 chunk, const int nq, const int E, const int n_full, const int logN, u64 (&rb)[2],
+                                              u64 (&ra)[2]) {
+    typedef typename F::E T;
+    const typename F::W *tw = (const typename F::W *)tw_int;
+    const size_t N = (size_t)1 << logN;
+    const u32 t = threadIdx.x, lane = t & 63u, wave = (u32)__builtin_amdgcn_readfirstlane((int)(t >> 6));
+    const u32 n = chunk * 512 + 2 * t, own_digit = (int)j < nq ? j / sw.alpha : (u32)B;
+    const bool chain = (int)j < nq;
+    auto pair = [&](const u64 *limb, const u32 g) {
+        ulonglong2 v = load2(limb + (galois_index(n, g, logN) & ~1u));
+        swap_if((galois_index(n, g, logN) & 1u) != 0, v);
+        return v;
+    };
+    ulonglong2 kb[B], ka[B], x[B], mine = make_ulonglong2(0, 0), b = mine, pb = mine, pa = mine;
+#pragma unroll
+    for (int d = 0; d < B; d++) {
+        kb[d] = stream_load2(keyed.evk + ((size_t)(2 * d) * n_full + prime) * N + n);
+        ka[d] = stream_load2(keyed.evk + ((size_t)(2 * d + 1) * n_full + prime) * N + n);
+    }
+    if (chain) {
+        mine = pair(sw.in + j * N, sw.galois);
+        if (keyed.b != nullptr) b = pair(keyed.b + j * N, keyed.galois);
+        if (own.ext != nullptr) {
+            pa = load2(own.ext + j * N + n);
+            pb = load2(own.b + j * N + n);
+        }
+    }
+    const u32 r = wave & 1u, R = 1u << (logN - 8), X = R + 2 * chunk + r, rows = 2u * (own_digit < (u32)B ? B - 1 : B);
+    const TwoStages<F> s64(tw, X), s16(tw, 4u * X + (lane >> 4)), s4(tw, 16u * X + (lane >> 2)), s1(tw, 64u * X + lane);
+    const int at4 = (int)(16u * (lane >> 2) + (lane & 3u)), at16 = (int)(64u * (lane >> 4) + (lane & 15u));
+    for (u32 q = wave; q < rows; q += 4) {
+        const u32 i = q >> 1, d = i + (i >= own_digit ? 1u : 0u);
+        const T *from = (const T *)(keyed.ext + ((size_t)d * E + j) * N + chunk * 512 + 256u * r) + lane;
+        T *l = (T *)lds_raw + (2 * d + r) * ROWPAD;
+        T v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = from[64 * k];
+        s64.forward(f, v);
+#pragma unroll
+        for (int k = 0; k < 4; k++) l[padc((int)lane + 64 * k)] = v[k];
+        wave_sync();
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = l[padc(at16 + 16 * k)];
+        s16.forward(f, v);
+#pragma unroll
+        for (int k = 0; k < 4; k++) l[padc(at16 + 16 * k)] = v[k];
+        wave_sync();
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = l[padc(at4 + 4 * k)];
+        s4.forward(f, v);
+#pragma unroll
+        for (int k = 0; k < 4; k++) l[padc(at4 + 4 * k)] = v[k];
+        wave_sync();
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = l[padc(4 * (int)lane + k)];
+        s1.forward(f, v);
+#pragma unroll
+        for (int k = 0; k < 4; k++) lds_raw[(2 * d + r) * ROWPAD + padc(4 * (int)lane + k)] = f.to_canonical(v[k]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d < B; d++) {
+        const u64 *l = lds_raw + (2 * d + (t >> 7)) * ROWPAD;
+        x[d] = (u32)d == own_digit ? mine : make_ulonglong2(l[padc((int)((2 * t) & 255u))], l[padc((int)((2 * t + 1) & 255u))]);
+    }
+    if (FP) {
+        double sb0 = 0, sb1 = 0, sa0 = 0, sa1 = 0;
+#pragma unroll
+        for (int d = 0; d < B; d++) {
+            const D2 v = to_d2(x[d]), b0 = to_d2(kb[d]), a0 = to_d2(ka[d]);
+            sb0 += fm.mul(v.x, b0.x);
+            sb1 += fm.mul(v.y, b0.y);
+            sa0 += fm.mul(v.x, a0.x);
+            sa1 += fm.mul(v.y, a0.y);
+        }
+        if (chain) {
+            const double p = (double)pmod.w;
+            const D2 v = to_d2(b), vb = to_d2(pb), va = to_d2(pa);
+            sb0 += fm.mul(v.x + vb.x, p);
+            sb1 += fm.mul(v.y + vb.y, p);
+            sa0 += fm.mul(va.x, p);
+            sa1 += fm.mul(va.y, p);
+        }
+        rb[0] = fm.canonical(sb0);
+        rb[1] = fm.canonical(sb1);
+        ra[0] = fm.canonical(sa0);
+        ra[1] = fm.canonical(sa1);
+    } else {
+        const u64 q = m.q;
+        Acc3 sb[2] = {{0, 0, 0}, {0, 0, 0}}, sa[2] = {{0, 0, 0}, {0, 0, 0}};
+#pragma unroll
+        for (int d = 0; d < B; d++) {
+            const Pieces px = pieces(x[d].x), py = pieces(x[d].y);
+            acc_mul(sb[0], px, pieces(kb[d].x));
+            acc_mul(sb[1], py, pieces(kb[d].y));
+            acc_mul(sa[0], px, pieces(ka[d].x));
+            acc_mul(sa[1], py, pieces(ka[d].y));
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {   // below 3q, 5q with what the chain limbs add
+            rb[h] = acc_reduce(sb[h], m);
+            ra[h] = acc_reduce(sa[h], m);
+        }
+        if (chain) {
+            rb[0] += mul_shoup_lazy_u(cond_sub_u(b.x + pb.x, q), pmod.w, pmod.ws, q);
+            rb[1] += mul_shoup_lazy_u(cond_sub_u(b.y + pb.y, q), pmod.w, pmod.ws, q);
+            ra[0] += mul_shoup_lazy_u(pa.x, pmod.w, pmod.ws, q);
+            ra[1] += mul_shoup_lazy_u(pa.y, pmod.w, pmod.ws, q);
+        }
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            rb[h] = cond_sub_u(cond_sub_u(cond_sub_u(rb[h], 4 * q), 2 * q), q);
+            ra[h] = cond_sub_u(cond_sub_u(cond_sub_u(ra[h], 4 * q), 2 * q), q);
+        }
+    }
+}
+template <int B, class ROWS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(B == 3 ? 3 : 4))) void switched_sum_kernel(
+    const RotTermDev keyed, const RotTermDev own, const SwitchedPoly sw, const Tw *__restrict__ tw_all, u64 *__restrict__ y,
+    const ModQ *__restrict__ modq, const double *__restrict__ fp, LimbList ll, const Cst *__restrict__ pmods, int nq, int E, int n_full,
+    int logN, LimbList jmap, const ROWS rows) {
+    __shared__ u64 digits[2 * B * ROWPAD];
+    const u32 chunks = 1u << (logN - 9), chunk = blockIdx.x & (chunks - 1), j = table_byte(jmap.idx, blockIdx.x >> (logN - 9));
+    const int prime = (int)table_byte(ll.idx, j);
+    const ModQ m = modq[prime];
+    const FpMod fm{fp[4 * prime], fp[4 * prime + 1]};
+    const Cst pmod = (int)j < nq ? pmods[j] : Cst{0, 0};
+    const Tw *tw = tw_all + ((size_t)prime << logN);
+    u64 rb[2], ra[2];
+    if (fm.q != 0.0)
+        switched_pair<true, B>(FpField(modq, nullptr, nullptr, fp, prime), fm, m, pmod, keyed, own, sw, tw, digits, prime, j, chunk, nq, E, n_full,
+                               logN, rb, ra);
+    else
+        switched_pair<false, B>(IntFieldT<true>(modq, nullptr, nullptr, fp, prime), fm, m, pmod, keyed, own, sw, tw, digits, prime, j, chunk, nq, E,
+                                n_full, logN, rb, ra);
+    sum_done(rb, ra, y, modq, fp, prime, fm.q != 0.0, 0u, j, chunk, chunk * 512 + 2 * threadIdx.x, E, logN, rows);
+}
 
 struct LinTermDev {
     const u64 *ct;    // [n_polys][.][N]
@@ -1118,6 +1280,15 @@ void launch_moddown(hemm_context *c, u64 *acc, int nq, int n_polys, u64 *out, si
                        add_polys, out, out_stride, c->d_modq, cl, nq, c->logN);
 }
 
+// cols_only: the converted limbs are left after the first of two passes and the digits' own limbs are not copied
+// (modup_in_two_passes has to say that there is such a form)
+static bool modup_in_two_passes(const hemm_context *c, int nq) {
+    const int E = nq + c->nP, beta = (nq + c->alpha - 1) / c->alpha;
+    return c->logN >= 13 && modup_through_automorphism_ok(c, nq) && !one_launch(c, (size_t)(beta * E - nq), false);
+}
+static void modup(hemm_context *c, const u64 *in, size_t in_stride, int nq, int n_in, u64 *ext, u64 *coef, hipStream_t s, u32 galois,
+                  bool cols_only);
+
 // Full key switch of `in` ([nq][N], NTT) with `evk` ([dnum][2][nQ+K][N]):
 // out[0] = ks_b (+ add_b), out[1] = ks_a; out poly stride out_stride.
 void launch_keyswitch(hemm_context *c, const u64 *in, const u64 *evk, int nq, u64 *out, size_t out_stride,
@@ -1129,7 +1300,9 @@ void launch_keyswitch(hemm_context *c, const u64 *in, const u64 *evk, int nq, u6
     u64 *coef = sc;                              // [nq][N]   (reused as conv[2][nq] needs 2*nq)
     u64 *ext = coef + (size_t)2 * (c->nQ) * N;   // [beta][E][N]
     u64 *acc = ext + (size_t)beta * E * N;       // [2][E][N]
-    launch_modup_batch(c, in, (size_t)nq * N, nq, 1, ext, coef, s, galois);   // same arithmetic as launch_modup
+    // the ModUp ends inside the key product where that reads aligned pairs of all it needs and has the digits for it
+    const bool switched = modup_in_two_passes(c, nq) && beta <= 3 && (uintptr_t)in % 16 == 0 && (uintptr_t)evk % 16 == 0;
+    modup(c, in, (size_t)nq * N, nq, 1, ext, coef, s, galois, switched);   // same arithmetic as launch_modup
     if (b_rotates && (galois == 0 || N < 512)) throw std::invalid_argument("add_b rotates only with the key switch's input");
     if (add_a != nullptr && (N < 512 || add_b == nullptr || b_rotates))
         throw std::invalid_argument("an addend for the second polynomial needs N >= 512 and one for the first");
@@ -1158,8 +1331,12 @@ void launch_keyswitch(hemm_context *c, const u64 *in, const u64 *evk, int nq, u6
             n_terms = 2;
         }
         const u32 off[2] = {0, (u32)n_terms};
-        launch_hoisted_moddown(c, HoistedList{term, off, nullptr, nullptr, n_terms}, 1, nq, acc, false, 0, out, out_stride, nullptr,
-                               coef, s);
+        HoistedList list{term, off, nullptr, nullptr, n_terms, nullptr, 1};
+        if (switched) {
+            list.switched = in;
+            if (galois != 0) list.switched_galois = galois;
+        }
+        launch_hoisted_moddown(c, list, 1, nq, acc, false, 0, out, out_stride, nullptr, coef, s);
         return;
     }
     launch_inner_product(c, in, ext, evk, nq, acc, s);
@@ -1353,6 +1530,10 @@ bool modup_through_automorphism_ok(const hemm_context *c, int nq) {
 
 void launch_modup_batch(hemm_context *c, const u64 *in, size_t in_stride, int nq, int n_in, u64 *ext, u64 *coef,
                         hipStream_t s, u32 galois) {
+    modup(c, in, in_stride, nq, n_in, ext, coef, s, galois, false);
+}
+static void modup(hemm_context *c, const u64 *in, size_t in_stride, int nq, int n_in, u64 *ext, u64 *coef, hipStream_t s, u32 galois,
+                  bool cols_only) {
     KsTables *t = g_tables_of(c);
     const int K = c->nP, E = nq + K, alpha = c->alpha, beta = (nq + alpha - 1) / alpha;
     const size_t N = c->N;
@@ -1449,14 +1630,16 @@ void launch_modup_batch(hemm_context *c, const u64 *in, size_t in_stride, int nq
         }
         cs.copy_src = in;
         cs.copy_src_stride = in_stride;
-        cs.n_copy = nq;
+        cs.n_copy = cols_only ? 0 : nq;
         cs.copy_galois = galois;
-        for (int j = 0; j < nq; j++) {
+        for (int j = 0; j < cs.n_copy; j++) {
             cs.copy_src_slot[j] = (uint8_t)j;
             cs.copy_dst_slot[j] = (uint8_t)((j / alpha) * E + j);
         }
-        if (launch_ntt_converted(c, cs, ext, jp, js, n_joint, n_in, (size_t)beta * E * N, s)) return;
+        if (launch_ntt_converted(c, cs, ext, jp, js, n_joint, n_in, (size_t)beta * E * N, s, nullptr, 0, nullptr, 0, nullptr, nullptr, cols_only))
+            return;
     }
+    if (cols_only) throw std::invalid_argument("this ModUp's conversion has a pass of its own");
     if (galois != 0) throw std::invalid_argument("this ModUp shape has no form that reads through an automorphism");
     g.d[0].split = bconv_split((int)N, n_in * beta, E - alpha);
     const dim3 grid((unsigned)(N / 512), n_in * g.d[0].split, beta), block(256);
@@ -1535,6 +1718,19 @@ static void sum_limbs(hemm_context *c, const HoistedList &l, int first, int n_ou
     }
     const LimbList ll = limbs_default(c, nq, 1);
     const Cst *pm = pmod_table(c);
+    if (l.switched != nullptr) {
+        const RotTermDev *terms = (const RotTermDev *)l.terms, none{};
+        const SwitchedPoly sw{l.switched, l.switched_galois, (u32)c->alpha};
+        const dim3 grid((unsigned)n_j * (unsigned)(c->N >> 9));
+#define SWITCHED(B)                                                                                                                   \
+    hipLaunchKernelGGL((switched_sum_kernel<B, ROWS>), grid, dim3(256), 0, s, terms[0], l.n_terms > 1 ? terms[1] : none, sw,          \
+                       (const Tw *)c->d_w, y, c->d_modq, c->d_fp, ll, pm, nq, E, n_full, c->logN, jl, rows)
+        if (beta == 1) SWITCHED(1);
+        else if (beta == 2) SWITCHED(2);
+        else SWITCHED(3);
+#undef SWITCHED
+        return;
+    }
     LimbList kind[2];   // double precision, integers
     int n_kind[2] = {0, 0};
     memset(kind, 0, sizeof(kind));
@@ -1715,6 +1911,7 @@ static bool tail_may_sum(const HoistedList &l, int n_out, size_t N, int nq, int 
     };
     for (size_t i = 1; i < written.size(); i++)
         if (written[i].first < written[i - 1].second) return false;
+    if (!apart(l.switched, (size_t)nq * N)) return false;
     const RotTermDev *t = (const RotTermDev *)l.terms, none{};
     for (int i = 0; i < l.n_terms; i++) {
         const RotTermDev &last = i > 0 ? t[i - 1] : none;   // terms share most of what they read
