@@ -259,9 +259,11 @@ void complexPackingPair(const HomEvaluator &eval, MatrixTransformer &transformer
 // add_conj: returns x + conj(x) itself; where the schedule ends in a giant-step sum the conjugated terms join that sum
 // (keys of every giant rotation's Galois element times 2N - 1, plain and square, and the square key of 2N - 1:
 // KeyGenerator::genGaloisKey / genGaloisSquareKey), otherwise the result is conjugated and added.
+// halves: A's other tile block takes half of the shifts (both operands single tiles, two of which make the slot vector, A >= T+6 and B >= T+5;
+// the rotations of halvesRotations on top)
 CtxtTensor multMatMatComplexPackedFused(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &a,
                                         const CtxtTensor &b, u64 target_level, MatrixTransformer &transformer,
-                                        u64 batch = 16, bool single_tile = false, bool add_conj = false);
+                                        u64 batch = 16, bool single_tile = false, bool add_conj = false, bool halves = false);
 // sum_k tmp[k] (x) rho^(k step)(b), relinearised (and rescaled when rescale_after): the ciphertext x ciphertext re-use
 // forms (multMatMatCCReUse: step = block width; multPackedMatMatCCReuse: step = 2 block widths, rescale) with all
 // rotations of b taken from ONE ModUp through direct keys, in batches of hoisted sums
@@ -285,6 +287,7 @@ std::vector<u64> rotateSumRotations(i64 unit, u64 count, u64 log_slots);
 std::vector<u64> fusedRotations(const TileTensorShape &shape, u64 log_slots, bool packed, bool need_rows);
 // the same for multMatMatFused; square_rots receives the giant steps that also need KeyPack::galoisSquareKey
 std::vector<u64> fusedCcmmRotations(const TileTensorShape &shape, u64 log_slots, std::vector<u64> &square_rots,
-                                    bool packed = false, bool single_tile = false);
+                                    bool packed = false, bool single_tile = false, bool halves = false);
+std::vector<u64> halvesRotations(i64 n, i64 w, u64 log_slots);
 
 }  // namespace HELLM

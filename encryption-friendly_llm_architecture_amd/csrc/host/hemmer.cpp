@@ -593,7 +593,13 @@ CtxtTensor HEMMer::singleCCMatMul(const CtxtTensor &a, const CtxtTensor &b, u64 
             // stacked tiles / unknown content keep their per-block products: the packed cells then shift through
             // masked pairs (no baby-step / giant-step split, which needs exact row rotations)
             const bool spread = single && block < slots;
-            ensureRotationKeys(fusedCcmmRotations(TileTensorShape(n, n, w), log_slots_, sq, true, spread));
+            // Two single tiles that leave half of the slots empty, with a level more to spare: half of the shifts go there.  On small
+            // tiles what counts is launches, of which that takes more; without / with, us (target 4): 32 x 32 tiles 509/551, 64 x 64
+            // 868/870, 128 x 128 2484/2127 (target 3 2290/1918).
+            const bool halves = spread && a_single && slots == 2 * block && n >= 128 && a.getLevel() >= T + 6 && b.getLevel() >= T + 5 &&
+                                std::min(a.getLevel(), b.getLevel()) >= 4 + btp_.getMinLevelForBootstrap();
+            if (halves) ensureRotationKeys(halvesRotations(n, w, log_slots_));
+            ensureRotationKeys(fusedCcmmRotations(TileTensorShape(n, n, w), log_slots_, sq, true, spread, halves));
             KeyGenerator kg(context_, sk_, pack_);
             for (u64 r : sq) kg.genLeftRotSquareKey(r);
             // x + conj(x) inside the product: its giant-step sum (exact row rotations: the block fills the slot vector
@@ -614,7 +620,7 @@ CtxtTensor HEMMer::singleCCMatMul(const CtxtTensor &a, const CtxtTensor &b, u64 
                     kg.genGaloisSquareKey(gc);
                 }
             }
-            CtxtTensor res = multMatMatComplexPackedFused(eval_, btp_, a, b, T, matrix_transformer, batch_, spread, true);
+            CtxtTensor res = multMatMatComplexPackedFused(eval_, btp_, a, b, T, matrix_transformer, batch_, spread, true, halves);
             if (spread) res.get().occupied_ = a_single ? block : unknown;
             return res;
         }

@@ -873,7 +873,7 @@ def _assemble_shifts(orc, src, ext, back, shifts):
 
 def _bsgs_shift_product(orc, a, b_low, acc, cm, n, units, cu, w, spread_block=0, with_conj=False):
     """Baby-step / giant-step sum over the shift index i = i1 + g i2 (column shift cu * i slots, row rotation
-    i * cu * w slots); `acc` holds the i = 0 term, a = sigma(A) at T+2, b_low = tau(B) at T+1.
+    i * cu * w slots); `acc` holds the i = 0 term (None: a lowered times the copied tau(B)), a = sigma(A) at T+2, b_low = tau(B) at T+1.
     spread_block: tau(B) holds one tile block of that many slots and nothing else; every baby rotation then
     also gathers the copies rho^(-j spread_block) (further terms of the same hoisted sum), i.e. it is the
     rotation of tau(B) copied into every block.
@@ -896,7 +896,7 @@ def _bsgs_shift_product(orc, a, b_low, acc, cm, n, units, cu, w, spread_block=0,
     ta = _assemble_shifts(orc, a, ext_a, -n,
                           [((cu * i - g * (i // g) * ru) % orc.slots, cm[2 * cu * i + 1], cm[2 * cu * i])
                            for i in range(1, units)])
-    U = [acc] + [None] * (units // g - 1)
+    U = [orc.tensor(orc.level_down_one(a), bb[0]) if acc is None else acc] + [None] * (units // g - 1)
     for i in range(1, units):
         t = orc.tensor(ta[i - 1], bb[i % g])
         U[i // g] = t if U[i // g] is None else orc.add(U[i // g], t)
@@ -956,8 +956,9 @@ def mult_mat_mat_cc_fused(orc, a, b, T, n, w, single_tile=False):
 
 
 def mult_packed_mat_mat_fused(orc, a, b, T, n, w, single_tile=False, merge_packing=False, with_conj=False,
-                              own_levels=False, first_stage=1):
-    """single_tile: the operands hold one tile block and nothing else (see mult_mat_mat_cc_fused).
+                              own_levels=False, first_stage=1, halves=False):
+    """halves: half of the shifts only (mult_mat_mat_cc_packed_halves).
+    single_tile: the operands hold one tile block and nothing else (see mult_mat_mat_cc_fused).
     merge_packing: a and b are NOT packed yet; the packing and the packed transform run as one composite one-stage
     transform from T+3 (kinds PKH / PKV).
     with_conj: returns x + conj(x) of the product x -- inside the giant-step sum where the schedule has one, by a
@@ -1005,9 +1006,9 @@ def mult_packed_mat_mat_fused(orc, a, b, T, n, w, single_tile=False, merge_packi
     else:
         a = lower_and_transform_fused(orc, a, PH, n, w, T + 2)
         b = lower_and_transform_fused(orc, b, PV, n, w, T + 1)
-    # the k = 0 term joins the accumulator at the shifts' level
-    acc = orc.tensor(orc.level_down_one(a), b)
-    return _bsgs_shift_product(orc, a, b, acc, cm, n, n // 2, 2, w, n * w if spread else 0, with_conj)
+    # the k = 0 term joins the accumulator at the shifts' level (by halves: with the copied tau(B), which meets A in both blocks)
+    acc = None if halves else orc.tensor(orc.level_down_one(a), b)
+    return _bsgs_shift_product(orc, a, b, acc, cm, n, n // (4 if halves else 2), 2, w, n * w if spread else 0, with_conj)
 
 
 def packing_maps(slots, w, rows):
@@ -1087,12 +1088,44 @@ def mult_mat_mat_cc_packed(orc, a, b, T, n, w, single_tile):
     return mult_packed_mat_mat_fused(orc, pa, pb, T, n, w, single_tile=single_tile, with_conj=True)
 
 
+def _masked_rotations(orc, x, parts):
+    """sum of mask (.) rho^amount(x) over (amount, mask), one level down: one ModUp, one hoisted sum, one ModDown; masks encoded as in
+    complex_packing_hoisted."""
+    from .oracle import Ct
+    nq, lvl = x.nq, x.level
+    ms = orc.delta[lvl] if x.scale == orc.delta[lvl] else orc.delta[lvl - 1] * float(orc.q[lvl]) / x.scale
+    ext = orc.modup(x.data[1])
+    terms = [(ext, x.data[0], r % orc.slots, orc.encode_ext(m, lvl, ms)) if r else
+             (x.data[1], x.data[0], ("none",), orc.encode_ext(m, lvl, ms)) for r, m in parts]
+    return Ct(orc.moddown_drop(orc.hoisted_sum(terms, nq), nq, True), orc.delta[lvl - 1])
+
+
+def mult_mat_mat_cc_packed_halves(orc, a, b, T, n, w):
+    """mult_mat_mat_cc_packed_single where two tile blocks make the slot vector, A >= T+6 and B >= T+5: the packing also copies A with
+    its rows moved by n / 2 into the second block, where sigma and the shifts i < n / 4 of two columns are those of i + n / 4; two
+    rotations under masks add the halves of the product, computed for target T + 1."""
+    from .oracle import Ct
+    cut = lambda x, lvl: Ct(np.ascontiguousarray(x.data[:, : lvl + 1]), x.scale)
+    half, row = n // 2 * w, np.arange(orc.slots) // w
+    zmask, ((_, plus), (_, minus)) = packing_maps(orc.slots, w, rows=False)
+    here = [np.ones(orc.slots), (row >= n) & (row < n + n // 2), row >= n + n // 2]
+    parts = [(s + e, m * h) for s, h in zip((0, -half, half), here) for e, m in ((0, zmask), (1, plus), (-1, minus))]
+    pa = _masked_rotations(orc, cut(a, T + 6), parts)
+    pb = complex_packing_hoisted(orc, cut(b, T + 5), w, rows=True)
+    y = mult_packed_mat_mat_fused(orc, pa, pb, T + 1, n, w, single_tile=True, with_conj=True, own_levels=True, halves=True)
+    one = np.ones(orc.slots, dtype=np.complex128)
+    return _masked_rotations(orc, y, [(0, one * (row < n)), (-half, one * (row < n // 2)), (half, one * ((row >= n // 2) & (row < n)))])
+
+
 def mult_mat_mat_cc_packed_single(orc, a, b, T, n, w):
     """One product through the complex-packed route: adjacent columns of A and adjacent rows of B are fused into
     complex slots (complexPackingInplace / complexPackingRowInplace, one level), the packed product then needs n / 2
     shifts instead of n, and x + conj(x) returns the real product (repackCC).  For operands that hold a single tile.
     Operands above the packing level are only truncated to it (the packing masks absorb the change of scale);
-    operands three levels above the target take the packing and the packed transform as one composite transform."""
+    operands three levels above the target take the packing and the packed transform as one composite transform, operands with
+    a level more to spare than a separate packing needs the product by halves."""
+    if orc.slots == 2 * n * w and n >= 128 and a.level >= T + 6 and b.level >= T + 5:
+        return mult_mat_mat_cc_packed_halves(orc, a, b, T, n, w)
     return mult_mat_mat_cc_packed(orc, a, b, T, n, w, single_tile=True)
 
 
