@@ -71,14 +71,15 @@ __global__ __launch_bounds__(256) void ntt_small_kernel(u64 *__restrict__ data, 
 // ------------------------------------------------------------------------------------------
 // two-launch kernels (N = 2^13 .. 2^16)
 // ------------------------------------------------------------------------------------------
-// Column passes work on a slab of R = 2^LR rows and CW = 4096 / R columns (R = 256: 16 columns): the 16 residues of a thread or lane pair
+// Column passes work on a slab of R = 2^LR rows and CW = 4096 / R columns (R = 256: 16 columns), or of CW >> H in small launches
+// (narrower_slabs): the 16 residues of a thread or lane pair
 // are rows rh + (R / 16) k for the block of the four widest stages and rows 16 rh + k for the LR - 4 others.
-template <int LR, int P>
+template <int LR, int P, int H = 0>
 struct Slab {
     typedef Lanes<P> L;
-    static constexpr int R = 1 << LR, Q = R / 16, CW = 4096 / R, T = LR - 4;
+    static constexpr int R = 1 << LR, Q = R / 16, CW = (4096 >> H) / R, T = LR - 4, WORDS = 4096 >> H;
     static __device__ __forceinline__ u32 cc() { return L::t() & (CW - 1); }
-    static __device__ __forceinline__ u32 rh() { return L::t() >> (12 - LR); }
+    static __device__ __forceinline__ u32 rh() { return L::t() >> (12 - LR - H); }
     static __device__ __forceinline__ u32 col() { return blockIdx.x * CW + cc(); }
     // twiddle group of the second block: 16 / Q sub-blocks per thread
     static __device__ __forceinline__ u32 group() { return 16u + rh() * (16 / Q); }
@@ -87,7 +88,9 @@ struct Slab {
     // (forward only: an inverse pass, which writes those rows, loses more to the xor in each address than to the
     // conflicts: 9.7 against 8.8 us for 10 limbs of 42-bit primes)
     template <bool INV>
-    static __device__ __forceinline__ int at(const int r) { return (CW == 16 && !INV ? swz_row(r) : r) * CW + (int)cc(); }
+    static __device__ __forceinline__ int at(const int r) {
+        return (CW == 16 && !INV ? swz_row(r) : r) * CW + (int)cc();
+    }
     // rows of a thread's register k: of the four widest stages (split, whole), of the others (split, whole)
     static __device__ __forceinline__ int r_outer_s(const int k) { return (int)(rh() + Q * L::template h_split<4>()) + Q * L::template split<4>(k); }
     static __device__ __forceinline__ int r_outer_w(const int k) { return (int)(rh() + Q * L::h_whole()) + Q * k; }
@@ -101,11 +104,11 @@ struct Slab {
     static __device__ __forceinline__ constexpr u32 inner(const int k) { return (u32)k << 11; }
 };
 // the exchange and the second block of a forward column pass, results to memory
-template <int LR, int P, class F>
+template <int LR, int H = 0, int P, class F>
 __device__ __forceinline__ void cols_forward(const __amdgpu_buffer_rsrc_t limb, const typename F::W *__restrict__ tw,
                                              const F f, typename F::E (&x)[P], typename F::E *lds) {
     typedef typename F::E E;
-    typedef Slab<LR, P> S;
+    typedef Slab<LR, P, H> S;
     radix_fwd<4>(f, x, tw, 1u);
 #pragma unroll
     for (int k = 0; k < P; k++) lds[S::template at<false>(S::r_outer_w(k))] = x[k];
@@ -116,18 +119,18 @@ __device__ __forceinline__ void cols_forward(const __amdgpu_buffer_rsrc_t limb, 
 #pragma unroll
     for (int k = 0; k < P; k++) buf_store<E>(limb, S::v_inner(), S::inner(k), x[k]);
 }
-template <int LR, int P, bool INV, class F>
+template <int LR, int P, int H, bool INV, class F>
 __device__ __forceinline__ void cols_body(const __amdgpu_buffer_rsrc_t limb, const Tw *__restrict__ tw_int, const F f,
                                           u64 *lds_raw) {
     typedef typename F::E E;
-    typedef Slab<LR, P> S;
+    typedef Slab<LR, P, H> S;
     const typename F::W *tw = (const typename F::W *)tw_int;
     E *lds = (E *)lds_raw;
     E x[P];
     if (!INV) {
 #pragma unroll
         for (int k = 0; k < P; k++) x[k] = f.from_canonical(buf_load<u64>(limb, S::v_outer(), S::outer(k)));
-        cols_forward<LR>(limb, tw, f, x, lds);
+        cols_forward<LR, H>(limb, tw, f, x, lds);
     } else {
 #pragma unroll
         for (int k = 0; k < P; k++) x[k] = buf_load<E>(limb, S::v_inner(), S::inner(k));
@@ -144,13 +147,13 @@ __device__ __forceinline__ void cols_body(const __amdgpu_buffer_rsrc_t limb, con
     }
 }
 
-template <int LR, int P, bool INV>
-__global__ __launch_bounds__(4096 / P) void ntt16_cols_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
+template <int LR, int P, int H, bool INV>
+__global__ __launch_bounds__((4096 >> H) / P) void ntt16_cols_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
                                                          const ModQ *__restrict__ modq,
                                                          const u64 *__restrict__ ninv, const u64 *__restrict__ ninv_s,
                                                          const double *__restrict__ fp, LimbList ll, LimbList sl,
                                                          int n_limbs, size_t poly_stride, const Tw *__restrict__ final_scale) {
-    __shared__ u64 lds[256 * 16];
+    __shared__ u64 lds[4096 >> H];
     const int limb = blockIdx.y % n_limbs, poly = blockIdx.y / n_limbs;
     const int prime = (int)table_byte(ll.idx, limb);
     const Tw *tw = tw_all + ((size_t)prime << (8 + LR));
@@ -164,31 +167,31 @@ __global__ __launch_bounds__(4096 / P) void ntt16_cols_kernel(u64 *__restrict__ 
             f.ni = (double)final_scale[limb].w;
             f.niinv = f.ni * f.qinv;
         }
-        cols_body<LR, P, INV>(base, tw, f, lds);
+        cols_body<LR, P, H, INV>(base, tw, f, lds);
     } else if (INV || (modq[prime].q >> 60) != 0) {
         IntField f(modq, ninv, ninv_s, fp, prime);
         if (INV && final_scale != nullptr) {
             f.ni = final_scale[limb].w;
             f.nis = final_scale[limb].ws;
         }
-        cols_body<LR, P, INV>(base, tw, f, lds);
+        cols_body<LR, P, H, INV>(base, tw, f, lds);
     } else {
-        cols_body<LR, P, INV>(base, tw, IntFieldT<true>(modq, ninv, ninv_s, fp, prime), lds);
+        cols_body<LR, P, H, INV>(base, tw, IntFieldT<true>(modq, ninv, ninv_s, fp, prime), lds);
     }
 }
 
 // Forward pass 1 over a slab whose input is a basis conversion computed on the fly.  The workgroups
 // of the target limbs that share a (polynomial, slab) pair have consecutive blockIdx.y and the same blockIdx.x, so
 // they sit on one XCD at about the same time and all but the first find the source slabs in its L2.
-template <int LR, int NS, class F>
+template <int LR, int H, int NS, class F>
 __device__ __forceinline__ void cols_converted_body(const __amdgpu_buffer_rsrc_t limb, const Tw *__restrict__ tw_int,
                                                     const F f, u64 *lds_raw, const __amdgpu_buffer_rsrc_t src,
                                                     const u32 (&so)[NS], const DotCst (&h)[NS], const int n_src, const ModQ m) {
-    typedef Slab<LR, 8> S;
+    typedef Slab<LR, 8, H> S;
     typename F::E x[8];
     // the row step goes into the scalar offset
     converted_inputs<NS>(f, x, src, S::v_outer(), so, h, n_src, m, [](const int k) { return S::outer(k); });
-    cols_forward<LR>(limb, (const typename F::W *)tw_int, f, x, (typename F::E *)lds_raw);
+    cols_forward<LR, H>(limb, (const typename F::W *)tw_int, f, x, (typename F::E *)lds_raw);
 }
 
 // What bounds it is the work of a column pass and the trips to memory in front of it.  Eight points per thread and 20 source
@@ -196,15 +199,15 @@ __device__ __forceinline__ void cols_converted_body(const __amdgpu_buffer_rsrc_t
 // workgroups (16 polynomials x 6 limbs, 5 sources) 42 -> 37 us alone, 1002 -> 789 vector instructions per wave, with sums that carry
 // nothing (modarith.h, DotCst) and loads that wait once; rotation at 24 primes of 60 bits, level 20 161 -> 154 us, projection of a
 // 768-wide layer 2.5 % less.
-template <int LR, int NS>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) void ntt16_cols_converted_kernel(
+template <int LR, int H, int NS>
+__global__ __launch_bounds__(512 >> H) __attribute__((amdgpu_waves_per_eu(6, 6))) void ntt16_cols_converted_kernel(
     u64 *__restrict__ data, const Tw *__restrict__ tw_all, const ModQ *__restrict__ modq, const u64 *__restrict__ ninv,
     const u64 *__restrict__ ninv_s, const double *__restrict__ fp, LimbList ll, LimbList sl, int n_limbs,
     size_t poly_stride, ConvSources cs) {
-    __shared__ u64 lds[256 * 16];
+    __shared__ u64 lds[4096 >> H];
     const int per_poly = n_limbs + cs.n_copy;
     const int limb = blockIdx.y % per_poly, poly = blockIdx.y / per_poly;
-    typedef Slab<LR, 8> S;
+    typedef Slab<LR, 8, H> S;
     if (limb >= n_limbs) {   // a limb that is only copied into its slot
         const u64 *from = cs.copy_src + (size_t)poly * cs.copy_src_stride +
                           ((size_t)table_byte(cs.copy_src_slot, limb - n_limbs) << (8 + LR));
@@ -243,28 +246,28 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) voi
         h[i] = dot_cst(hg.w, hg.ws);
     }
     if (fp[4 * prime] != 0.0)
-        cols_converted_body<LR, NS>(base, tw, FpField(modq, ninv, ninv_s, fp, prime), lds, src, so, h, n_src, m);
+        cols_converted_body<LR, H, NS>(base, tw, FpField(modq, ninv, ninv_s, fp, prime), lds, src, so, h, n_src, m);
     else   // (the sums take primes below 2^60)
-        cols_converted_body<LR, NS>(base, tw, IntFieldT<true>(modq, ninv, ninv_s, fp, prime), lds, src, so, h, n_src, m);
+        cols_converted_body<LR, H, NS>(base, tw, IntFieldT<true>(modq, ninv, ninv_s, fp, prime), lds, src, so, h, n_src, m);
 }
 
 // Forward pass 1 whose input is the rounded coefficients of an encoding, the same for every limb of a polynomial: reduced
 // as they are loaded instead of being written limb by limb and read back.
-template <int LR, class F>
+template <int LR, int H, class F>
 __device__ __forceinline__ void cols_lifted_body(const __amdgpu_buffer_rsrc_t limb, const Tw *__restrict__ tw_int, const F f,
                                                  u64 *lds_raw, const LiftSource &ls, const long long *__restrict__ coef,
                                                  const ModQ m) {
-    typedef Slab<LR, 8> S;
+    typedef Slab<LR, 8, H> S;
     typename F::E x[8];
     lifted_inputs(f, x, ls, coef, m, [](const int k) { return ((u32)S::r_outer_s(k) << 8) + S::col(); });
-    cols_forward<LR>(limb, (const typename F::W *)tw_int, f, x, (typename F::E *)lds_raw);
+    cols_forward<LR, H>(limb, (const typename F::W *)tw_int, f, x, (typename F::E *)lds_raw);
 }
-template <int LR>
-__global__ __launch_bounds__(512) void ntt16_cols_lifted_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
+template <int LR, int H>
+__global__ __launch_bounds__(512 >> H) void ntt16_cols_lifted_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
                                                                 const ModQ *__restrict__ modq, const double *__restrict__ fp,
                                                                 LimbList ll, LimbList sl, int n_limbs, size_t poly_stride,
                                                                 LiftSource ls) {
-    __shared__ u64 lds[256 * 16];
+    __shared__ u64 lds[4096 >> H];
     const int limb = blockIdx.y % n_limbs, poly = blockIdx.y / n_limbs;
     const int prime = (int)table_byte(ll.idx, limb);
     const Tw *tw = tw_all + ((size_t)prime << (8 + LR));
@@ -273,11 +276,11 @@ __global__ __launch_bounds__(512) void ntt16_cols_lifted_kernel(u64 *__restrict_
     const long long *coef = ls.coef + (size_t)poly * ls.stride;
     const ModQ m = modq[prime];
     if (fp[4 * prime] != 0.0)
-        cols_lifted_body<LR>(base, tw, FpField(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
+        cols_lifted_body<LR, H>(base, tw, FpField(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
     else if ((m.q >> 60) != 0)
-        cols_lifted_body<LR>(base, tw, IntField(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
+        cols_lifted_body<LR, H>(base, tw, IntField(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
     else
-        cols_lifted_body<LR>(base, tw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
+        cols_lifted_body<LR, H>(base, tw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -526,27 +529,60 @@ void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, c
 static bool few_for_columns(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 512; }
 static bool few_for_rows(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 640; }
 
+// Column passes of few workgroups are bound by the instructions of the few CUs they are on, two wavefronts per SIMD: slabs of a half or a
+// quarter of the columns (1, 2: as powers of two) put them on as many more CUs.  Not below 16 columns, segments of 128 bytes: at 2^16 points,
+// half slabs take a rotation on 60-bit primes from 129.8 to 133.7 us where up to 512 workgroups have them, to 131.1 where up to 128 do.
+// Transforms (forward/inverse, us) with whole / with narrower slabs:
+//   limbs              1                 4                 16                32                48                64
+//   2^13 points        9.2/9.5 8.4/8.8   9.2/9.8 8.5/8.9   9.6/10.1 8.8/9.2  10.4/11.0 9.6/10.0   11.4/11.9 11.2/11.6  (one launch)
+//   2^14               9.4/10.0 8.5/8.9  9.6/10.2 8.6/9.2  10.8/11.2 10.1/10.4 12.6/13.3 12.7/13.0 15.9/16.4 15.7/16.2 17.9/18.5 17.8/18.2
+//   2^15               9.8/10.5 8.9/9.2  10.3/10.8 9.5/9.7 13.0/13.3 12.3/12.1 18.2/18.7 18.9/18.3 25.4/26.3 24.5/24.9 30.4/31.3 30.7/30.9
+// (plain forward passes of 2^15 points keep whole slabs above 128 workgroups.)  Rotations of 6 / 12 / 24 limbs, 42 bits: 2^13 41.2/43.6/98.7 ->
+// 35.6/38.4/92.9, 2^14 43.9/50.8/114.7 -> 38.5/47.2/112.0, 2^15 50.3/68.0/145.1 -> 46.3/62.8/142.3; products alike.
+static int narrower_slabs(const hemm_context *c, int limbs, bool plain_forward = false) {
+    const size_t wgs = (size_t)limbs * (c->N >> 12);
+    if (c->logN == 16 || (c->logN == 15 && plain_forward && wgs > 128)) return 0;
+    return c->logN <= 14 && wgs <= 128 ? 2 : wgs <= 512 ? 1 : 0;
+}
+
 static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbList &ll, const LimbList &sl, int n_limbs,
                       int n_polys, size_t poly_stride, hipStream_t s, const void *final_scale = nullptr) {
-    const dim3 grid((unsigned)(c->N >> 12), (unsigned)(n_limbs * n_polys));
     const bool few = few_for_columns(c, n_limbs * n_polys);
+    const int narrow = narrower_slabs(c, n_limbs * n_polys, !inverse);
+    const dim3 grid((unsigned)(c->N >> (12 - narrow)), (unsigned)(n_limbs * n_polys));
     const Tw *tw = (const Tw *)(inverse ? c->d_iw : c->d_w);
-#define COLS_FORM(LR, P, INV)                                                                                             \
-    hipLaunchKernelGGL((ntt16_cols_kernel<LR, P, INV>), grid, dim3(4096 / P), 0, s, d, tw, c->d_modq, c->d_ninv,          \
+#define COLS_FORM(LR, P, H, INV)                                                                                          \
+    hipLaunchKernelGGL((ntt16_cols_kernel<LR, P, H, INV>), grid, dim3((4096 >> H) / P), 0, s, d, tw, c->d_modq, c->d_ninv,          \
                        c->d_ninv_s, c->d_fp, ll, sl, n_limbs, poly_stride, (const Tw *)(INV ? final_scale : nullptr))
+#define COLS_SLAB(LR, INV)                          \
+    do {                                            \
+        if (narrow == 1) COLS_FORM(LR, 8, 1, INV);  \
+        else if (few) COLS_FORM(LR, 8, 0, INV);     \
+        else COLS_FORM(LR, 16, 0, INV);             \
+    } while (0)
 #define COLS(LR)                                    \
     do {                                            \
-        if (inverse && few) COLS_FORM(LR, 8, true); \
-        else if (inverse) COLS_FORM(LR, 16, true);  \
-        else if (few) COLS_FORM(LR, 8, false);      \
-        else COLS_FORM(LR, 16, false);              \
+        if (inverse) COLS_SLAB(LR, true);           \
+        else COLS_SLAB(LR, false);                  \
+    } while (0)
+#define COLS_SMALL(LR)                                      \
+    do {                                                    \
+        if (narrow == 2 && inverse) COLS_FORM(LR, 8, 2, true); \
+        else if (narrow == 2) COLS_FORM(LR, 8, 2, false);   \
+        else COLS(LR);                                      \
     } while (0)
     switch (c->logN) {
-        case 13: COLS(5); break;
-        case 14: COLS(6); break;
+        case 13: COLS_SMALL(5); break;
+        case 14: COLS_SMALL(6); break;
         case 15: COLS(7); break;
-        default: COLS(8); break;
+        default:
+            if (inverse && few) COLS_FORM(8, 8, 0, true);
+            else if (inverse) COLS_FORM(8, 16, 0, true);
+            else if (few) COLS_FORM(8, 8, 0, false);
+            else COLS_FORM(8, 16, 0, false);
     }
+#undef COLS_SMALL
+#undef COLS_SLAB
 #undef COLS
 #undef COLS_FORM
 }
@@ -686,24 +722,37 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
                             tail ? TAIL_SUB_SCALE : TAIL_NONE, ep_list);
         return true;
     }
-    const dim3 grid((unsigned)(c->N >> 12), (n_limbs + cs.n_copy) * n_polys);
-#define CONV_CASE(LR, K)                                                                                                     \
-    hipLaunchKernelGGL((ntt16_cols_converted_kernel<LR, K>), grid, dim3(512), 0, s, data, (const Tw *)c->d_w, c->d_modq, \
+    const int narrow = narrower_slabs(c, (n_limbs + cs.n_copy) * n_polys);
+    const dim3 grid((unsigned)(c->N >> (12 - narrow)), (n_limbs + cs.n_copy) * n_polys);
+#define CONV_FORM(LR, H, K)                                                                                                  \
+    hipLaunchKernelGGL((ntt16_cols_converted_kernel<LR, H, K>), grid, dim3(512 >> H), 0, s, data, (const Tw *)c->d_w, c->d_modq, \
                        c->d_ninv, c->d_ninv_s, c->d_fp, ll, sl, n_limbs, poly_stride, cs)
-#define CONV_RING(LR)                      \
-    do {                                   \
-        if (widest <= 2) CONV_CASE(LR, 2); \
-        else if (widest <= 5) CONV_CASE(LR, 5); \
-        else CONV_CASE(LR, 8);             \
+#define CONV_RING(LR, H)                        \
+    do {                                        \
+        if (widest <= 2) CONV_FORM(LR, H, 2);   \
+        else if (widest <= 5) CONV_FORM(LR, H, 5); \
+        else CONV_FORM(LR, H, 8);               \
+    } while (0)
+#define CONV_SLAB(LR)                    \
+    do {                                 \
+        if (narrow == 1) CONV_RING(LR, 1); \
+        else CONV_RING(LR, 0);           \
+    } while (0)
+#define CONV_SMALL(LR)                   \
+    do {                                 \
+        if (narrow == 2) CONV_RING(LR, 2); \
+        else CONV_SLAB(LR);              \
     } while (0)
     switch (c->logN) {
-        case 13: CONV_RING(5); break;
-        case 14: CONV_RING(6); break;
-        case 15: CONV_RING(7); break;
-        default: CONV_RING(8); break;
+        case 13: CONV_SMALL(5); break;
+        case 14: CONV_SMALL(6); break;
+        case 15: CONV_SLAB(7); break;
+        default: CONV_RING(8, 0); break;
     }
+#undef CONV_SMALL
+#undef CONV_SLAB
 #undef CONV_RING
-#undef CONV_CASE
+#undef CONV_FORM
     if (cols_only) return true;
     rows_pass(c, false, data, ll, sl, n_limbs, n_polys, poly_stride, s,
               sub_scale_tail(ep_minuend, ep_minuend_stride, ep_out, ep_out_stride, ep_cst_dev), tail ? TAIL_SUB_SCALE : TAIL_NONE,
@@ -832,17 +881,24 @@ bool launch_ntt_lifted(const hemm_context *c, const LiftSource &ls, u64 *data, c
         u64 *d = data + (size_t)p0 * poly_stride;
         LiftSource l = ls;
         l.coef += (size_t)p0 * ls.stride;
-        const dim3 grid((unsigned)(c->N >> 12), (unsigned)(n_limbs * np));
-#define LIFTED(LR)                                                                                                         \
-    hipLaunchKernelGGL(ntt16_cols_lifted_kernel<LR>, grid, dim3(512), 0, s, d, (const Tw *)c->d_w, c->d_modq, c->d_fp, ll, sl, \
+        const bool half = narrower_slabs(c, n_limbs * np) != 0;
+        const dim3 grid((unsigned)(c->N >> (half ? 11 : 12)), (unsigned)(n_limbs * np));
+#define LIFTED_FORM(LR, H)                                                                                                     \
+    hipLaunchKernelGGL((ntt16_cols_lifted_kernel<LR, H>), grid, dim3(512 >> H), 0, s, d, (const Tw *)c->d_w, c->d_modq, c->d_fp, ll, sl, \
                        n_limbs, poly_stride, l)
+#define LIFTED(LR)                    \
+    do {                              \
+        if (half) LIFTED_FORM(LR, 1); \
+        else LIFTED_FORM(LR, 0);      \
+    } while (0)
         switch (c->logN) {
             case 13: LIFTED(5); break;
             case 14: LIFTED(6); break;
             case 15: LIFTED(7); break;
-            default: LIFTED(8); break;
+            default: LIFTED_FORM(8, 0); break;
         }
 #undef LIFTED
+#undef LIFTED_FORM
         rows_pass(c, false, d, ll, sl, n_limbs, np, poly_stride, s, ep, tail);
         if (enc != nullptr) {
             ep.out += (size_t)np * poly_stride;
