@@ -235,7 +235,7 @@ int hemm_sum_parts(hemm_context *ctx, const uint64_t *parts, uint32_t n_parts, u
  *   hemm_diagonal_table_words: words that the tables of the Q_tj take over nq + n_p limbs, 0 where there is no such form;
  *   hemm_diagonal_tables: from the first k rows of the matrix's slots, block [k][w] complex doubles on the device, encoded at `scale`;
  *   hemm_diagonal_sums: rotations[g-1], a two polynomials of nq limbs a_stride words apart, y [2k/g][2][nq+n_p][N].
- * Reference: MatrixUtils.cpp:1218-1305 (the same product through sigma, tau and k shifts). */
+ * Reference: MatrixUtils.cpp:1448-1570 (the same product through sigma, tau and k shifts). */
 int hemm_diagonal_table_words(hemm_context *ctx, uint32_t k, uint32_t w, uint32_t g, uint32_t nq, size_t *words);
 int hemm_diagonal_tables(hemm_context *ctx, const double *block, uint32_t k, uint32_t w, uint32_t g, double scale, uint32_t nq,
                          uint64_t *tables, void *stream);
