@@ -238,14 +238,21 @@ CtxtTensor multPackedMatMatFused(const HomEvaluator &eval, const Bootstrapper &b
                                  u64 batch = 16, bool single_tile = false);
 void multMatMatPreFused(const HomEvaluator &eval, const CtxtTensor &a, std::vector<Ciphertext> &tmp, u64 target_level,
                         MatrixTransformer &transformer, u64 batch = 16, bool first_block_only = false);
-// plaintext x ciphertext product through the hoisted column shifts (see matrix_utils_fused.cpp for the layouts it takes)
-bool multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2,
-                          u64 target_level, MatrixTransformer &transformer, u64 batch, CtxtTensor &res);
-// the same over the diagonals of the weight, in baby and giant steps; a_single: the first operand holds one tile block and nothing else.
-// false: not a product for it.  plainDiagonalRotations: the rotations it takes (none: no such form).
+// Plaintext x ciphertext product through the hoisted column shifts.  plainShiftsTau: tau(B), made on first use and kept by the transformer,
+// or none where the weight's layout is not one for this form (see matrix_utils_fused.cpp); it needs no keys, and throws where
+// the operands' levels are too low.
+const MatrixTransformer::WeightTau *plainShiftsTau(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1,
+                                                   const PtxtTensor &op2, u64 target_level, MatrixTransformer &transformer);
+CtxtTensor multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2,
+                                u64 target_level, MatrixTransformer &transformer, const MatrixTransformer::WeightTau &weight);
+// The same over the diagonals of the weight, in baby and giant steps.  plainDiagonalTables: the tables of its diagonals, made on first use and
+// kept by the transformer, or none where the product is not one for this form (a_single: the first operand holds one tile block and
+// nothing else); it needs no keys.  plainDiagonalRotations: the rotations the product takes (none: no such form).
+const DeviceBuffer *plainDiagonalTables(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2,
+                                        u64 target_level, MatrixTransformer &transformer, bool a_single);
 std::vector<u64> plainDiagonalRotations(i64 k, u64 log_slots);
-bool multMatMatPlainDiagonals(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2,
-                              u64 target_level, MatrixTransformer &transformer, bool a_single, CtxtTensor &res);
+CtxtTensor multMatMatPlainDiagonals(const HomEvaluator &eval, const CtxtTensor &op1, const PtxtTensor &op2, u64 target_level,
+                                    const DeviceBuffer &tables);
 // the n/2 column shifts (by two columns each) of a packed sigma(A) at level T+2, as ciphertexts at level T+1
 // (multPackedMatMatPreRot through the hoisted launches)
 void multPackedMatMatPreRotFused(const HomEvaluator &eval, const CtxtTensor &a, std::vector<Ciphertext> &tmp, u64 target_level,

@@ -638,20 +638,21 @@ CtxtTensor HEMMer::singleCCMatMul(const CtxtTensor &a, const CtxtTensor &b, u64 
 CtxtTensor HEMMer::singleMatMul(const CtxtTensor &a, const PtxtTensor &b, u64 T) const {
     const u64 slots = u64(1) << log_slots_;
     const i64 w = a.getBlockWidth(), n = pow2ceil(a.getWidth());
-    if (fused_) {
-        CtxtTensor res(context_, a.getHeight(), b.getWidth(), w);
+    if (fused_) {   // the form is decided, and what is refused is refused, before any key is derived
         const bool a_single = single_tile_ || a.get().occupiedSlots() <= (u64)(n * w);
         if (a.getHeight() == n && b.getHeight() == n) {
-            ensureRotationKeys(plainDiagonalRotations(n, log_slots_));
-            if (multMatMatPlainDiagonals(eval_, btp_, a, b, T, matrix_transformer, a_single, res)) return res;
+            if (const DeviceBuffer *tables = plainDiagonalTables(eval_, btp_, a, b, T, matrix_transformer, a_single)) {
+                ensureRotationKeys(plainDiagonalRotations(n, log_slots_));
+                return multMatMatPlainDiagonals(eval_, a, b, T, *tables);
+            }
+        }
+        if (const MatrixTransformer::WeightTau *tau = plainShiftsTau(eval_, btp_, a, b, T, matrix_transformer)) {
+            ensureRotationKeys(transformRotations(MaskKind::Horizontal, w));
+            ensureRotationKeys(fusedRotations(TileTensorShape(n, n, w), log_slots_, false, false));
+            return multMatMatPlainFused(eval_, btp_, a, b, T, matrix_transformer, *tau);
         }
     }
     ensureRotationKeys(transformRotations(MaskKind::Horizontal, w));
-    if (fused_) {
-        ensureRotationKeys(fusedRotations(TileTensorShape(n, n, w), log_slots_, false, false));
-        CtxtTensor res(context_, a.getHeight(), b.getWidth(), w);
-        if (multMatMatPlainFused(eval_, btp_, a, b, T, matrix_transformer, batch_, res)) return res;
-    }
     ensureRotationKeys({1, slots - (u64)n});
     return multMatMat(eval_, btp_, a, b, T, matrix_transformer);
 }

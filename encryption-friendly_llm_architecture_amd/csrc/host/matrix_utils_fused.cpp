@@ -1929,20 +1929,18 @@ int weightLayout(const Message &src, i64 block, i64 slots) {
 }
 }  // namespace
 
-bool multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2,
-                          u64 T, MatrixTransformer &tr, u64 batch, CtxtTensor &res_out) {
+const MatrixTransformer::WeightTau *plainShiftsTau(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1,
+                                                   const PtxtTensor &op2, u64 T, MatrixTransformer &tr) {
     const Context &c = eval.getContext();
-    (void)batch;
-    const i64 rows = op1.getHeight(), cols = op2.getWidth();
     const i64 k = pow2ceil(commonInside(op1, op2)), w = commonBlockWidth(op1, op2);
     if (std::min(op1.getLevel(), op2.getLevel()) < 1 + btp.getMinLevelForBootstrap())
         throw std::invalid_argument("[multMatMat] level >= " + std::to_string(1 + btp.getMinLevelForBootstrap()) +
                                     " is needed.");
     const i64 slots = (i64)(c->N / 2), block = k * w;
-    if (block > slots || slots % block != 0) return false;
+    if (block > slots || slots % block != 0) return nullptr;
     if (op1.getLevel() < T + 3)
         throw std::invalid_argument("[multMatMat] level >= " + std::to_string(T + 3) + " is needed.");
-    const TileTensorShape shape_a(rows, k, w), shape_b(k, cols, w);
+    const TileTensorShape shape_b(k, op2.getWidth(), w);
     // ---- tau(B) over the extended basis at level T+2, scaled like a plaintext of level T+1
     const std::pair<u64, u64> weight_hash = weightHash(c, op2.get());
     tr.useChainOf(c);
@@ -1973,9 +1971,17 @@ bool multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, con
         tr.weight_tau_order_.push_back(key);
         it = tr.weight_tau_.emplace(key, std::move(entry)).first;
     }
-    if (it->second.layout == 0) return false;
-    const bool first_block_only = it->second.layout == 2;
-    const Plaintext &tau = it->second.tau;
+    return it->second.layout == 0 ? nullptr : &it->second;
+}
+
+CtxtTensor multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2, u64 T,
+                                MatrixTransformer &tr, const MatrixTransformer::WeightTau &weight) {
+    const Context &c = eval.getContext();
+    const i64 rows = op1.getHeight(), cols = op2.getWidth();
+    const i64 k = pow2ceil(commonInside(op1, op2)), w = commonBlockWidth(op1, op2);
+    const TileTensorShape shape_a(rows, k, w);
+    const bool first_block_only = weight.layout == 2;
+    const Plaintext &tau = weight.tau;
     std::vector<Plaintext> &cm = tr.getColMaskExt(eval, shape_a, T + 2, first_block_only);
     // ---- sigma(A) at level T+2 and its two rotation sources
     const u64 nq = T + 3, N = c->N, K = c->nP, E = nq + K, lo = nq - 1;
@@ -2041,8 +2047,7 @@ bool multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, con
     CtxtTensor res(c, rows, cols, w);
     res.get().allocate(2, T, 0);
     ck(hemm_rescale(c->dev, mid.data(), lo * N, res.get().buf_.data(), (lo - 1) * N, (uint32_t)lo, 2, nullptr));
-    res_out = res;
-    return true;
+    return res;
 }
 
 // The same product over the diagonals of B, without sigma and tau: C[i][c] = sum_r A[i][c + r] B[c + r][c], a sum over the rotations of A
@@ -2052,7 +2057,7 @@ bool multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, con
 // with the rescale leaves them at level T, and the giant rotations are terms of one sum with one ModDown.  g + 2 k / g - 2 key products of
 // few limbs instead of k - 1 after two transforms, and one level instead of three: A is only truncated to level T + 1, the
 // diagonals' scale takes it to that of level T.  128 x 128 tiles, pair layout, T = 4: 501 us, 1444 through the shifts above.
-// Takes what multMatMatPlainFused takes where rows and inside of the tiles are the same power of two; where only the first block of B is not
+// Takes what the form through the shifts takes where rows and inside of the tiles are the same power of two; where only the first block of B is not
 // zero, the others of A have to be empty as well (the diagonals are the same in every block).
 // A baby step is one key product, a giant step also its share of a ModDown and a ModUp: twice as many baby steps as giant ones at least.  g = k / 8 /
 // k / 4, us: 128 x 128 tiles 672 / 621, 64 x 64 263 / 237, 32 x 32 (a quarter and half of k) 153 / 154.
@@ -2067,21 +2072,21 @@ std::vector<u64> plainDiagonalRotations(i64 k, u64 log_slots) {
     return r;
 }
 
-bool multMatMatPlainDiagonals(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2, u64 T,
-                              MatrixTransformer &tr, bool a_single, CtxtTensor &res_out) {
+const DeviceBuffer *plainDiagonalTables(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2, u64 T,
+                                        MatrixTransformer &tr, bool a_single) {
     const Context &c = eval.getContext();
-    const i64 rows = op1.getHeight(), cols = op2.getWidth();
-    const i64 k = pow2ceil(commonInside(op1, op2)), w = commonBlockWidth(op1, op2), g = plainBabyCount(k), giants = 2 * k / g;
+    const i64 cols = op2.getWidth();
+    const i64 k = pow2ceil(commonInside(op1, op2)), w = commonBlockWidth(op1, op2), g = plainBabyCount(k);
     const i64 slots = (i64)(c->N / 2), block = k * w;
     const Ciphertext &a = op1.get();
-    const u64 level = a.getLevel(), nq = T + 2, N = c->N, E = nq + c->nP, lo = nq - 1;
+    const u64 level = a.getLevel(), nq = T + 2;
     // what is refused is left to the general product to refuse
-    if (rows != k || block > slots || slots % block != 0 || level < T + 3 || level >= c->nQ || a.getRescaleCounter() != 0 || a.getNumPoly() != 2 ||
-        std::min(level, op2.getLevel()) < 1 + btp.getMinLevelForBootstrap() || level < 4 + btp.getMinLevelForBootstrap())
-        return false;
+    if (op1.getHeight() != k || block > slots || slots % block != 0 || level < T + 3 || level >= c->nQ || a.getRescaleCounter() != 0 ||
+        a.getNumPoly() != 2 || std::min(level, op2.getLevel()) < 1 + btp.getMinLevelForBootstrap() || level < 4 + btp.getMinLevelForBootstrap())
+        return nullptr;
     size_t words = 0;
     ck(hemm_diagonal_table_words(c->dev, (uint32_t)k, (uint32_t)w, (uint32_t)g, (uint32_t)nq, &words));
-    if (words == 0) return false;
+    if (words == 0) return nullptr;
     // ---- the diagonals, at the scale that takes the sums from level's to T's
     tr.useChainOf(c);
     const auto hash = weightHash(c, op2.get());
@@ -2108,7 +2113,14 @@ bool multMatMatPlainDiagonals(const HomEvaluator &eval, const Bootstrapper &btp,
             it->second = std::move(entry);
         }
     }
-    if (it->second.tables.data() == nullptr) return false;
+    return it->second.tables.data() == nullptr ? nullptr : &it->second.tables;
+}
+
+CtxtTensor multMatMatPlainDiagonals(const HomEvaluator &eval, const CtxtTensor &op1, const PtxtTensor &op2, u64 T, const DeviceBuffer &tables) {
+    const Context &c = eval.getContext();
+    const i64 k = pow2ceil(commonInside(op1, op2)), w = commonBlockWidth(op1, op2), g = plainBabyCount(k), giants = 2 * k / g;
+    const Ciphertext &a = op1.get();
+    const u64 nq = T + 2, N = c->N, E = nq + c->nP, lo = nq - 1;
     // ---- the inner sums, from rotations of A in the extended basis
     const KeyPack &pack = eval.getKeyPack();
     const Rot rot(c);
@@ -2119,7 +2131,7 @@ bool multMatMatPlainDiagonals(const HomEvaluator &eval, const Bootstrapper &btp,
         std::vector<hemm_rot_term> terms;
         for (i64 j = 1; j < g; j++) terms.push_back(term(x.extOf(0), x.pbOf(0), pack, rot.galois(j), nullptr));
         ck(hemm_diagonal_sums(c->dev, terms.data(), cut.data(), nq * N, (uint32_t)k, (uint32_t)w, (uint32_t)g, (uint32_t)nq, x.premultiplied(),
-                              it->second.tables.data(), y.data(), nullptr));
+                              tables.data(), y.data(), nullptr));
     }
     // ---- divided by P and rescaled, rotated and added up
     {
@@ -2133,13 +2145,12 @@ bool multMatMatPlainDiagonals(const HomEvaluator &eval, const Bootstrapper &btp,
         terms.push_back(term(s.extOf((size_t)t - 1), s.pbOf((size_t)t - 1), pack, rot.galois(t < giants / 2 ? t * g : (t - giants) * g), nullptr));
     terms.push_back(keylessTerm(v.data(), v.data() + lo * N, nullptr));
     const std::vector<uint32_t> off{0, (uint32_t)terms.size()};
-    CtxtTensor res(c, rows, cols, w);
+    CtxtTensor res(c, op1.getHeight(), op2.getWidth(), w);
     res.get().allocate(2, T, 0);
     DeviceBuffer ws(c, 2 * lo * N);
     ck(hemm_hoisted_moddown(c->dev, terms.data(), off.data(), 1, (uint32_t)lo, s.premultiplied(), 0, y.data(), res.get().buf_.data(), lo * N,
                             ws.data(), nullptr));
-    res_out = std::move(res);
-    return true;
+    return res;
 }
 
 }  // namespace HELLM

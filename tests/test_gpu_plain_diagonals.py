@@ -73,3 +73,21 @@ def test_unknown_left_operand_of_a_single_tile_keeps_its_masks(rings):
     s = H.decrypt_slots(got)
     assert np.abs(s[:256].real.reshape(16, 16) - z[:256].real.reshape(16, 16) @ B).max() < 2.0 ** -18
     assert np.abs(s[256:]).max() < 2.0 ** -20
+
+
+@pytest.mark.parametrize("a_level, b_level", [(6, 7), (7, 3)])   # A not three levels above the target; B below what the products ask for
+def test_a_refused_product_derives_no_keys(rings, a_level, b_level):
+    from efla_amd import hellm
+    _, orc = rings(10)
+    H = hellm.HEMMer(10, orc.q, orc.p, dnum=3, min_bootstrap_level=3, seed=SEED)
+    rng = np.random.default_rng(3)
+    A, B = rng.uniform(-1, 1, (16, 16)), rng.uniform(-1, 1, (16, 16))
+    ct = H.encrypt(A)
+    ct, pt = H.level_down(ct, a_level) if a_level < 7 else ct, H.encode(B, b_level)
+    held = H.key_bytes()
+    with pytest.raises(Exception, match="level >= "):
+        H.single_matmul(ct, pt, 4)
+    after = H.key_bytes()
+    assert (after["plain"], after["compact"]) == (held["plain"], held["compact"])
+    assert np.abs(H.decrypt(H.single_matmul(H.encrypt(A), H.encode(B), 4)) - A @ B).max() < 2.0 ** -14
+    assert H.key_bytes()["compact"] > held["compact"]
