@@ -15,6 +15,7 @@
 #include <map>
 #include <vector>
 
+#include "HELLM/BoundedStore.hpp"
 #include "HELLM/HETensor.hpp"
 
 namespace HELLM {
@@ -141,21 +142,14 @@ private:
     std::map<std::pair<TileTensorShape, u64>, Plaintext> first_block_masks_;
 
 public:
-    // tau(B) of a plaintext weight over the extended basis, kept per weight: the key is a hash of the weight's
-    // residues, so a weight whose content changes is prepared again.  layout: 0 = not usable by the batched product,
-    // 1 = equal tile blocks, 2 = only the first block is non-zero.
-    struct WeightTau {
-        Plaintext tau;
-        int layout;
-    };
-    // The diagonals of a plaintext weight as tables for hemm_diagonal_sums, kept like tau(B): one more part of the key is the level
-    // whose scale the encrypted operand carries.  layout as in WeightTau; no tables where the layout did not call for them.
-    struct WeightDiagonals {
-        DeviceBuffer tables;
-        int layout;
-    };
+    // What is kept per plaintext weight, under digests of its residues (PlainWeight), so that a weight whose content changes is prepared again:
+    //   its layout in blocks of so many slots (PlainWeight::layout): nothing is kept of a weight beyond that where its layout does
+    //   not call for it;
+    //   tau(B) over the extended basis, by shape and target level;
+    //   its diagonals as tables for hemm_diagonal_sums, by shape, target level and the level whose scale the encrypted operand carries.
+    BoundedStore<std::tuple<u64, u64, i64>, int> weight_layouts_{4096};
     typedef std::tuple<u64, u64, TileTensorShape, u64, u64> DiagonalKey;
-    std::map<DiagonalKey, WeightDiagonals> weight_diagonals_;
+    std::map<DiagonalKey, DeviceBuffer> weight_diagonals_;
     std::vector<DiagonalKey> weight_diagonals_order_;
     // complexPackingInplace (rows[q] false: adjacent columns -> a + i b) / complexPackingRowInplace (true: adjacent
     // rows of rows `w` slots wide -> a - i b) of n_jobs ciphertexts at `level` through one launch chain: both
@@ -167,7 +161,7 @@ public:
                              u64 *const *out, const u64 *scale_levels = nullptr);
     // (rows, w, level, part 0 = Z / 1 = +step / 2 = -step, level of the input's scale)
     std::map<std::tuple<int, i64, u64, int, u64>, Plaintext> pack_masks_;
-    std::map<std::tuple<u64, u64, TileTensorShape, u64>, WeightTau> weight_tau_;
+    std::map<std::tuple<u64, u64, TileTensorShape, u64>, Plaintext> weight_tau_;
     std::vector<std::tuple<u64, u64, TileTensorShape, u64>> weight_tau_order_;
 
 private:
@@ -238,18 +232,38 @@ CtxtTensor multPackedMatMatFused(const HomEvaluator &eval, const Bootstrapper &b
                                  u64 batch = 16, bool single_tile = false);
 void multMatMatPreFused(const HomEvaluator &eval, const CtxtTensor &a, std::vector<Ciphertext> &tmp, u64 target_level,
                         MatrixTransformer &transformer, u64 batch = 16, bool first_block_only = false);
+// A plaintext weight as the batched products look at it, for the time of one call.  Its values are decoded at most once, by whoever needs them
+// first: to find its layout or to prepare it.
+class PlainWeight {
+public:
+    enum Layout {
+        OTHER = 0,         // not one for the batched products
+        EQUAL_BLOCKS = 1,  // all tile blocks hold the same (one block that fills the slot vector among them)
+        FIRST_BLOCK = 2    // only the first is not zero
+    };
+    PlainWeight(const Context &c, const Plaintext &pt) : c_(c), pt_(pt) {}
+    const Context &getContext() const { return c_; }
+    std::pair<u64, u64> digests() const;   // needs a device-to-host copy, and with it a drained queue, once per plaintext object
+    const Message &values();
+    Layout layout(MatrixTransformer &transformer, i64 block);
+
+private:
+    const Context c_;
+    const Plaintext &pt_;
+    Message values_;
+};
 // Plaintext x ciphertext product through the hoisted column shifts.  plainShiftsTau: tau(B), made on first use and kept by the transformer,
 // or none where the weight's layout is not one for this form (see matrix_utils_fused.cpp); it needs no keys, and throws where
 // the operands' levels are too low.
-const MatrixTransformer::WeightTau *plainShiftsTau(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1,
-                                                   const PtxtTensor &op2, u64 target_level, MatrixTransformer &transformer);
+const Plaintext *plainShiftsTau(const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2, u64 target_level,
+                                MatrixTransformer &transformer, PlainWeight &weight);
 CtxtTensor multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2,
-                                u64 target_level, MatrixTransformer &transformer, const MatrixTransformer::WeightTau &weight);
+                                u64 target_level, MatrixTransformer &transformer, const Plaintext &tau, bool first_block_only);
 // The same over the diagonals of the weight, in baby and giant steps.  plainDiagonalTables: the tables of its diagonals, made on first use and
 // kept by the transformer, or none where the product is not one for this form (a_single: the first operand holds one tile block and
 // nothing else); it needs no keys.  plainDiagonalRotations: the rotations the product takes (none: no such form).
-const DeviceBuffer *plainDiagonalTables(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2,
-                                        u64 target_level, MatrixTransformer &transformer, bool a_single);
+const DeviceBuffer *plainDiagonalTables(const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2, u64 target_level,
+                                        MatrixTransformer &transformer, bool a_single, PlainWeight &weight);
 std::vector<u64> plainDiagonalRotations(i64 k, u64 log_slots);
 CtxtTensor multMatMatPlainDiagonals(const HomEvaluator &eval, const CtxtTensor &op1, const PtxtTensor &op2, u64 target_level,
                                     const DeviceBuffer &tables);

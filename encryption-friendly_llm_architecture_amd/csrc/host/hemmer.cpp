@@ -640,16 +640,18 @@ CtxtTensor HEMMer::singleMatMul(const CtxtTensor &a, const PtxtTensor &b, u64 T)
     const i64 w = a.getBlockWidth(), n = pow2ceil(a.getWidth());
     if (fused_) {   // the form is decided, and what is refused is refused, before any key is derived
         const bool a_single = single_tile_ || a.get().occupiedSlots() <= (u64)(n * w);
+        PlainWeight weight(context_, b.get());
         if (a.getHeight() == n && b.getHeight() == n) {
-            if (const DeviceBuffer *tables = plainDiagonalTables(eval_, btp_, a, b, T, matrix_transformer, a_single)) {
+            if (const DeviceBuffer *tables = plainDiagonalTables(btp_, a, b, T, matrix_transformer, a_single, weight)) {
                 ensureRotationKeys(plainDiagonalRotations(n, log_slots_));
                 return multMatMatPlainDiagonals(eval_, a, b, T, *tables);
             }
         }
-        if (const MatrixTransformer::WeightTau *tau = plainShiftsTau(eval_, btp_, a, b, T, matrix_transformer)) {
+        if (const Plaintext *tau = plainShiftsTau(btp_, a, b, T, matrix_transformer, weight)) {
             ensureRotationKeys(transformRotations(MaskKind::Horizontal, w));
             ensureRotationKeys(fusedRotations(TileTensorShape(n, n, w), log_slots_, false, false));
-            return multMatMatPlainFused(eval_, btp_, a, b, T, matrix_transformer, *tau);
+            const bool first_block_only = weight.layout(matrix_transformer, n * w) == PlainWeight::FIRST_BLOCK;
+            return multMatMatPlainFused(eval_, btp_, a, b, T, matrix_transformer, *tau, first_block_only);
         }
     }
     ensureRotationKeys(transformRotations(MaskKind::Horizontal, w));

@@ -215,6 +215,7 @@ void MatrixTransformer::cleanUp() {
     two_stage_masks_.clear();
     packing_stage_one_masks_.clear();
     pack_masks_.clear();
+    weight_layouts_.clear();
     weight_tau_.clear();
     weight_tau_order_.clear();
     weight_diagonals_.clear();

@@ -1904,34 +1904,43 @@ std::pair<u64, u64> hashResidues(const Context &c, const Plaintext &pt) {
     }
     return {x, y};
 }
-// whose digests a weight's preparation is kept under: the hash needs a device-to-host copy and with it a drained queue, so it is taken once
-// per plaintext object
-std::pair<u64, u64> weightHash(const Context &c, const Plaintext &weight) {
-    if (weight.hash_state_ == 1) return {weight.content_hash_, weight.content_hash2_};
-    const std::pair<u64, u64> h = hashResidues(c, weight);
-    if (weight.hash_state_ == 0) {
-        weight.content_hash_ = h.first;
-        weight.content_hash2_ = h.second;
-        weight.hash_state_ = 1;
-    }
-    return h;
-}
-// 1: all tile blocks of `block` slots are equal, 2: only the first is not zero, 0: anything else.  Decoded values carry the encoding's
-// rounding noise (about sqrt(N) / 2^43 at this scale): "zero" and "equal" are taken up to 2^-24.
-int weightLayout(const Message &src, i64 block, i64 slots) {
+// Decoded values carry the encoding's rounding noise (about sqrt(N) / 2^43 at this scale): "zero" and "equal" are taken up to 2^-24.
+PlainWeight::Layout weightLayout(const Message &src, i64 block, i64 slots) {
     const double tol = std::ldexp(1.0, -24);
     bool rest_zero = true, rest_equal = true;
     for (i64 j = block; j < slots && (rest_zero || rest_equal); j++) {
         if (std::abs(src[(u64)j]) >= tol) rest_zero = false;
         if (std::abs(src[(u64)j] - src[(u64)(j % block)]) >= tol) rest_equal = false;
     }
-    return !rest_zero && !rest_equal ? 0 : rest_zero && block < slots ? 2 : 1;
+    return !rest_zero && !rest_equal ? PlainWeight::OTHER : rest_zero && block < slots ? PlainWeight::FIRST_BLOCK : PlainWeight::EQUAL_BLOCKS;
 }
 }  // namespace
 
-const MatrixTransformer::WeightTau *plainShiftsTau(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1,
-                                                   const PtxtTensor &op2, u64 T, MatrixTransformer &tr) {
-    const Context &c = eval.getContext();
+std::pair<u64, u64> PlainWeight::digests() const {
+    if (pt_.hash_state_ == 1) return {pt_.content_hash_, pt_.content_hash2_};
+    const std::pair<u64, u64> h = hashResidues(c_, pt_);
+    if (pt_.hash_state_ == 0) {
+        pt_.content_hash_ = h.first;
+        pt_.content_hash2_ = h.second;
+        pt_.hash_state_ = 1;
+    }
+    return h;
+}
+const Message &PlainWeight::values() {
+    if (values_.getLogSlots() == 0) values_ = EnDecoder(c_).decode(pt_);
+    return values_;
+}
+PlainWeight::Layout PlainWeight::layout(MatrixTransformer &tr, i64 block) {
+    tr.useChainOf(c_);
+    const std::pair<u64, u64> h = digests();
+    const auto key = std::make_tuple(h.first, h.second, block);
+    if (const int *known = tr.weight_layouts_.find(key)) return (Layout)*known;
+    return (Layout)tr.weight_layouts_.keep(key, (int)weightLayout(values(), block, (i64)(c_->N / 2)));
+}
+
+const Plaintext *plainShiftsTau(const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2, u64 T, MatrixTransformer &tr,
+                                PlainWeight &weight) {
+    const Context &c = weight.getContext();
     const i64 k = pow2ceil(commonInside(op1, op2)), w = commonBlockWidth(op1, op2);
     if (std::min(op1.getLevel(), op2.getLevel()) < 1 + btp.getMinLevelForBootstrap())
         throw std::invalid_argument("[multMatMat] level >= " + std::to_string(1 + btp.getMinLevelForBootstrap()) +
@@ -1940,48 +1949,40 @@ const MatrixTransformer::WeightTau *plainShiftsTau(const HomEvaluator &eval, con
     if (block > slots || slots % block != 0) return nullptr;
     if (op1.getLevel() < T + 3)
         throw std::invalid_argument("[multMatMat] level >= " + std::to_string(T + 3) + " is needed.");
-    const TileTensorShape shape_b(k, op2.getWidth(), w);
+    const PlainWeight::Layout layout = weight.layout(tr, block);
+    if (layout == PlainWeight::OTHER) return nullptr;
     // ---- tau(B) over the extended basis at level T+2, scaled like a plaintext of level T+1
-    const std::pair<u64, u64> weight_hash = weightHash(c, op2.get());
-    tr.useChainOf(c);
-    const auto key = std::make_tuple(weight_hash.first, weight_hash.second, shape_b, T);
+    const std::pair<u64, u64> h = weight.digests();
+    const auto key = std::make_tuple(h.first, h.second, TileTensorShape(k, op2.getWidth(), w), T);
     auto it = tr.weight_tau_.find(key);
     if (it == tr.weight_tau_.end()) {
-        EnDecoder endec(c);
-        const Message src = endec.decode(op2.get());
-        const int layout = weightLayout(src, block, slots);
-        MatrixTransformer::WeightTau entry{Plaintext(c), 0};
-        if (layout != 0) {
-            const bool first_only = layout == 2;
-            Message dst(src.getLogSlots(), 0);
-            const i64 height = slots / w;
-            for (i64 r = 0; r < height; r++)
-                for (i64 cc = 0; cc < w; cc++) {
-                    const i64 cb = cc - cc % k, i = r % k, j = cc % k;
-                    const i64 rb = first_only ? 0 : r - r % k;   // single matrix: every block takes the first one's tau
-                    dst[(u64)(r * w + cc)] = src[(u64)((rb + (i + j) % k) * w + cb + j)];
-                }
-            entry.tau = endec.encodeExtended(dst, T + 2, c->delta[T + 1]);
-            entry.layout = layout;
-        }
+        const Message &src = weight.values();
+        const bool first_only = layout == PlainWeight::FIRST_BLOCK;
+        Message dst(src.getLogSlots(), 0);
+        const i64 height = slots / w;
+        for (i64 r = 0; r < height; r++)
+            for (i64 cc = 0; cc < w; cc++) {
+                const i64 cb = cc - cc % k, i = r % k, j = cc % k;
+                const i64 rb = first_only ? 0 : r - r % k;   // single matrix: every block takes the first one's tau
+                dst[(u64)(r * w + cc)] = src[(u64)((rb + (i + j) % k) * w + cb + j)];
+            }
+        Plaintext tau = EnDecoder(c).encodeExtended(dst, T + 2, c->delta[T + 1]);
         if (tr.weight_tau_order_.size() >= 256) {   // bounded: the oldest weight is prepared again if it comes back
             tr.weight_tau_.erase(tr.weight_tau_order_.front());
             tr.weight_tau_order_.erase(tr.weight_tau_order_.begin());
         }
         tr.weight_tau_order_.push_back(key);
-        it = tr.weight_tau_.emplace(key, std::move(entry)).first;
+        it = tr.weight_tau_.emplace(key, std::move(tau)).first;
     }
-    return it->second.layout == 0 ? nullptr : &it->second;
+    return &it->second;
 }
 
 CtxtTensor multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2, u64 T,
-                                MatrixTransformer &tr, const MatrixTransformer::WeightTau &weight) {
+                                MatrixTransformer &tr, const Plaintext &tau, bool first_block_only) {
     const Context &c = eval.getContext();
     const i64 rows = op1.getHeight(), cols = op2.getWidth();
     const i64 k = pow2ceil(commonInside(op1, op2)), w = commonBlockWidth(op1, op2);
     const TileTensorShape shape_a(rows, k, w);
-    const bool first_block_only = weight.layout == 2;
-    const Plaintext &tau = weight.tau;
     std::vector<Plaintext> &cm = tr.getColMaskExt(eval, shape_a, T + 2, first_block_only);
     // ---- sigma(A) at level T+2 and its two rotation sources
     const u64 nq = T + 3, N = c->N, K = c->nP, E = nq + K, lo = nq - 1;
@@ -2072,10 +2073,9 @@ std::vector<u64> plainDiagonalRotations(i64 k, u64 log_slots) {
     return r;
 }
 
-const DeviceBuffer *plainDiagonalTables(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2, u64 T,
-                                        MatrixTransformer &tr, bool a_single) {
-    const Context &c = eval.getContext();
-    const i64 cols = op2.getWidth();
+const DeviceBuffer *plainDiagonalTables(const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2, u64 T, MatrixTransformer &tr,
+                                        bool a_single, PlainWeight &weight) {
+    const Context &c = weight.getContext();
     const i64 k = pow2ceil(commonInside(op1, op2)), w = commonBlockWidth(op1, op2), g = plainBabyCount(k);
     const i64 slots = (i64)(c->N / 2), block = k * w;
     const Ciphertext &a = op1.get();
@@ -2087,33 +2087,26 @@ const DeviceBuffer *plainDiagonalTables(const HomEvaluator &eval, const Bootstra
     size_t words = 0;
     ck(hemm_diagonal_table_words(c->dev, (uint32_t)k, (uint32_t)w, (uint32_t)g, (uint32_t)nq, &words));
     if (words == 0) return nullptr;
+    const PlainWeight::Layout layout = weight.layout(tr, block);
+    if (layout == PlainWeight::OTHER || (layout == PlainWeight::FIRST_BLOCK && !a_single)) return nullptr;
     // ---- the diagonals, at the scale that takes the sums from level's to T's
-    tr.useChainOf(c);
-    const auto hash = weightHash(c, op2.get());
-    const auto key = std::make_tuple(hash.first, hash.second, TileTensorShape(k, cols, w), T, level);
+    const std::pair<u64, u64> h = weight.digests();
+    const auto key = std::make_tuple(h.first, h.second, TileTensorShape(k, op2.getWidth(), w), T, level);
     auto it = tr.weight_diagonals_.find(key);
-    if (it == tr.weight_diagonals_.end() || (it->second.layout == 2 && a_single && it->second.tables.data() == nullptr)) {
-        const Message src = EnDecoder(c).decode(op2.get());
-        MatrixTransformer::WeightDiagonals entry{DeviceBuffer(), weightLayout(src, block, slots)};
-        if (entry.layout == 1 || (entry.layout == 2 && a_single)) {
-            DeviceBuffer first(c, 2 * (size_t)block);
-            if (hipMemcpy(first.data(), &src[0], (size_t)block * sizeof(Complex), hipMemcpyHostToDevice) != hipSuccess) throw RuntimeException("hipMemcpy");
-            entry.tables = DeviceBuffer(c, words);
-            ck(hemm_diagonal_tables(c->dev, (const double *)first.data(), (uint32_t)k, (uint32_t)w, (uint32_t)g,
-                                    c->delta[T] * (double)c->q[T + 1] / c->delta[level], (uint32_t)nq, entry.tables.data(), nullptr));
+    if (it == tr.weight_diagonals_.end()) {
+        DeviceBuffer first(c, 2 * (size_t)block), tables(c, words);
+        if (hipMemcpy(first.data(), &weight.values()[0], (size_t)block * sizeof(Complex), hipMemcpyHostToDevice) != hipSuccess)
+            throw RuntimeException("hipMemcpy");
+        ck(hemm_diagonal_tables(c->dev, (const double *)first.data(), (uint32_t)k, (uint32_t)w, (uint32_t)g,
+                                c->delta[T] * (double)c->q[T + 1] / c->delta[level], (uint32_t)nq, tables.data(), nullptr));
+        if (tr.weight_diagonals_order_.size() >= 256) {   // bounded: the oldest weight is prepared again if it comes back
+            tr.weight_diagonals_.erase(tr.weight_diagonals_order_.front());
+            tr.weight_diagonals_order_.erase(tr.weight_diagonals_order_.begin());
         }
-        if (it == tr.weight_diagonals_.end()) {
-            if (tr.weight_diagonals_order_.size() >= 256) {   // bounded: the oldest weight is prepared again if it comes back
-                tr.weight_diagonals_.erase(tr.weight_diagonals_order_.front());
-                tr.weight_diagonals_order_.erase(tr.weight_diagonals_order_.begin());
-            }
-            tr.weight_diagonals_order_.push_back(key);
-            it = tr.weight_diagonals_.emplace(key, std::move(entry)).first;
-        } else {
-            it->second = std::move(entry);
-        }
+        tr.weight_diagonals_order_.push_back(key);
+        it = tr.weight_diagonals_.emplace(key, std::move(tables)).first;
     }
-    return it->second.tables.data() == nullptr ? nullptr : &it->second.tables;
+    return &it->second;
 }
 
 CtxtTensor multMatMatPlainDiagonals(const HomEvaluator &eval, const CtxtTensor &op1, const PtxtTensor &op2, u64 T, const DeviceBuffer &tables) {

@@ -91,3 +91,24 @@ def test_a_refused_product_derives_no_keys(rings, a_level, b_level):
     assert (after["plain"], after["compact"]) == (held["plain"], held["compact"])
     assert np.abs(H.decrypt(H.single_matmul(H.encrypt(A), H.encode(B), 4)) - A @ B).max() < 2.0 ** -14
     assert H.key_bytes()["compact"] > held["compact"]
+
+
+def test_a_weight_is_decoded_once(rings):
+    """What a product with a new weight takes more than one with a known weight: its decoding, and one transform where tau(B) is encoded
+    (the diagonals' tables are made without one)."""
+    H, orc = rings(10)
+    rng = np.random.default_rng(8)
+    A = H.encrypt(rng.uniform(-1, 1, (16, 16)))
+    unknown = H.upload(A.residues(), 16, 16, 16)
+
+    def transforms(a, w):
+        H.traffic(reset=True)
+        H.single_matmul(a, w, 2)
+        return H.traffic(reset=True)[1]["transforms"]
+
+    for a, more in ((A, 1), (unknown, 2)):
+        first, second = (H.encode(rng.uniform(-1, 1, (16, 16))) for _ in range(2))
+        transforms(a, first)
+        known = transforms(a, first)
+        assert transforms(a, second) == known + more
+        assert transforms(a, second) == known
