@@ -11,15 +11,19 @@ template <class Key, class Entry>
 class BoundedStore {
 public:
     explicit BoundedStore(uint64_t limit) : limit_(limit) {}
-    // stays where it is until the next keep() or clear()
+    // stays where it is until the next makeRoom(), keep() or clear()
     const Entry *find(const Key &key) const {
         auto it = entries_.find(key);
         return it == entries_.end() ? nullptr : &it->second.first;
     }
+    // gives up what an entry of this cost has to replace: in front of an allocation, which then finds the memory
+    void makeRoom(uint64_t cost) {
+        while (!order_.empty() && cost_ + cost > limit_) drop(order_.front());
+    }
     // an entry that costs more than the limit is kept alone
     const Entry &keep(const Key &key, Entry entry, uint64_t cost = 1) {
         drop(key);
-        while (!order_.empty() && cost_ + cost > limit_) drop(order_.front());
+        makeRoom(cost);
         order_.push_back(key);
         cost_ += cost;
         return entries_.emplace(key, std::make_pair(std::move(entry), cost)).first->second.first;
@@ -30,7 +34,6 @@ public:
         cost_ = 0;
     }
     uint64_t cost() const { return cost_; }
-    size_t size() const { return entries_.size(); }
 
 private:
     void drop(const Key key) {   // (by value: the key may be one of order_)

@@ -147,10 +147,12 @@ public:
     //   not call for it;
     //   tau(B) over the extended basis, by shape and target level;
     //   its diagonals as tables for hemm_diagonal_sums, by shape, target level and the level whose scale the encrypted operand carries.
+    // The tables are bounded by their bytes, 10 to 40 MB a weight at N = 2^16: the 216 pair-layout weights of a layer that is 768 wide (3072 inside)
+    // take 4.5 GB at target level 4.
+    static constexpr u64 DIAGONAL_BYTES = u64(6) << 30;
     BoundedStore<std::tuple<u64, u64, i64>, int> weight_layouts_{4096};
-    typedef std::tuple<u64, u64, TileTensorShape, u64, u64> DiagonalKey;
-    std::map<DiagonalKey, DeviceBuffer> weight_diagonals_;
-    std::vector<DiagonalKey> weight_diagonals_order_;
+    BoundedStore<std::tuple<u64, u64, TileTensorShape, u64>, Plaintext> weight_tau_{256};
+    BoundedStore<std::tuple<u64, u64, TileTensorShape, u64, u64>, DeviceBuffer> weight_diagonals_{DIAGONAL_BYTES};
     // complexPackingInplace (rows[q] false: adjacent columns -> a + i b) / complexPackingRowInplace (true: adjacent
     // rows of rows `w` slots wide -> a - i b) of n_jobs ciphertexts at `level` through one launch chain: both
     // rotations of every job from one ModUp, masks applied in the extended basis, ModDown merged with the rescale.
@@ -161,8 +163,6 @@ public:
                              u64 *const *out, const u64 *scale_levels = nullptr);
     // (rows, w, level, part 0 = Z / 1 = +step / 2 = -step, level of the input's scale)
     std::map<std::tuple<int, i64, u64, int, u64>, Plaintext> pack_masks_;
-    std::map<std::tuple<u64, u64, TileTensorShape, u64>, Plaintext> weight_tau_;
-    std::vector<std::tuple<u64, u64, TileTensorShape, u64>> weight_tau_order_;
 
 private:
     // (kind, shape, level, (scale level * 4 + stage) * 4096 + r * 4 + part) -> mask of the two-stage transforms; part 0 is

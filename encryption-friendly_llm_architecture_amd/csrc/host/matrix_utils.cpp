@@ -217,9 +217,7 @@ void MatrixTransformer::cleanUp() {
     pack_masks_.clear();
     weight_layouts_.clear();
     weight_tau_.clear();
-    weight_tau_order_.clear();
     weight_diagonals_.clear();
-    weight_diagonals_order_.clear();
     chain_.clear();
     last_context_ = Context();
 }

@@ -1954,27 +1954,18 @@ const Plaintext *plainShiftsTau(const Bootstrapper &btp, const CtxtTensor &op1, 
     // ---- tau(B) over the extended basis at level T+2, scaled like a plaintext of level T+1
     const std::pair<u64, u64> h = weight.digests();
     const auto key = std::make_tuple(h.first, h.second, TileTensorShape(k, op2.getWidth(), w), T);
-    auto it = tr.weight_tau_.find(key);
-    if (it == tr.weight_tau_.end()) {
-        const Message &src = weight.values();
-        const bool first_only = layout == PlainWeight::FIRST_BLOCK;
-        Message dst(src.getLogSlots(), 0);
-        const i64 height = slots / w;
-        for (i64 r = 0; r < height; r++)
-            for (i64 cc = 0; cc < w; cc++) {
-                const i64 cb = cc - cc % k, i = r % k, j = cc % k;
-                const i64 rb = first_only ? 0 : r - r % k;   // single matrix: every block takes the first one's tau
-                dst[(u64)(r * w + cc)] = src[(u64)((rb + (i + j) % k) * w + cb + j)];
-            }
-        Plaintext tau = EnDecoder(c).encodeExtended(dst, T + 2, c->delta[T + 1]);
-        if (tr.weight_tau_order_.size() >= 256) {   // bounded: the oldest weight is prepared again if it comes back
-            tr.weight_tau_.erase(tr.weight_tau_order_.front());
-            tr.weight_tau_order_.erase(tr.weight_tau_order_.begin());
+    if (const Plaintext *tau = tr.weight_tau_.find(key)) return tau;
+    const Message &src = weight.values();
+    const bool first_only = layout == PlainWeight::FIRST_BLOCK;
+    Message dst(src.getLogSlots(), 0);
+    const i64 height = slots / w;
+    for (i64 r = 0; r < height; r++)
+        for (i64 cc = 0; cc < w; cc++) {
+            const i64 cb = cc - cc % k, i = r % k, j = cc % k;
+            const i64 rb = first_only ? 0 : r - r % k;   // single matrix: every block takes the first one's tau
+            dst[(u64)(r * w + cc)] = src[(u64)((rb + (i + j) % k) * w + cb + j)];
         }
-        tr.weight_tau_order_.push_back(key);
-        it = tr.weight_tau_.emplace(key, std::move(tau)).first;
-    }
-    return &it->second;
+    return &tr.weight_tau_.keep(key, EnDecoder(c).encodeExtended(dst, T + 2, c->delta[T + 1]));
 }
 
 CtxtTensor multMatMatPlainFused(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1, const PtxtTensor &op2, u64 T,
@@ -2092,21 +2083,15 @@ const DeviceBuffer *plainDiagonalTables(const Bootstrapper &btp, const CtxtTenso
     // ---- the diagonals, at the scale that takes the sums from level's to T's
     const std::pair<u64, u64> h = weight.digests();
     const auto key = std::make_tuple(h.first, h.second, TileTensorShape(k, op2.getWidth(), w), T, level);
-    auto it = tr.weight_diagonals_.find(key);
-    if (it == tr.weight_diagonals_.end()) {
-        DeviceBuffer first(c, 2 * (size_t)block), tables(c, words);
-        if (hipMemcpy(first.data(), &weight.values()[0], (size_t)block * sizeof(Complex), hipMemcpyHostToDevice) != hipSuccess)
-            throw RuntimeException("hipMemcpy");
-        ck(hemm_diagonal_tables(c->dev, (const double *)first.data(), (uint32_t)k, (uint32_t)w, (uint32_t)g,
-                                c->delta[T] * (double)c->q[T + 1] / c->delta[level], (uint32_t)nq, tables.data(), nullptr));
-        if (tr.weight_diagonals_order_.size() >= 256) {   // bounded: the oldest weight is prepared again if it comes back
-            tr.weight_diagonals_.erase(tr.weight_diagonals_order_.front());
-            tr.weight_diagonals_order_.erase(tr.weight_diagonals_order_.begin());
-        }
-        tr.weight_diagonals_order_.push_back(key);
-        it = tr.weight_diagonals_.emplace(key, std::move(tables)).first;
-    }
-    return &it->second;
+    if (const DeviceBuffer *tables = tr.weight_diagonals_.find(key)) return tables;
+    const Message &values = weight.values();
+    tr.weight_diagonals_.makeRoom(words * 8);
+    DeviceBuffer first(c, 2 * (size_t)block), tables(c, words);
+    if (hipMemcpy(first.data(), &values[0], (size_t)block * sizeof(Complex), hipMemcpyHostToDevice) != hipSuccess)
+        throw RuntimeException("hipMemcpy");
+    ck(hemm_diagonal_tables(c->dev, (const double *)first.data(), (uint32_t)k, (uint32_t)w, (uint32_t)g,
+                            c->delta[T] * (double)c->q[T + 1] / c->delta[level], (uint32_t)nq, tables.data(), nullptr));
+    return &tr.weight_diagonals_.keep(key, std::move(tables), words * 8);
 }
 
 CtxtTensor multMatMatPlainDiagonals(const HomEvaluator &eval, const CtxtTensor &op1, const PtxtTensor &op2, u64 T, const DeviceBuffer &tables) {

@@ -112,3 +112,31 @@ def test_a_weight_is_decoded_once(rings):
         known = transforms(a, first)
         assert transforms(a, second) == known + more
         assert transforms(a, second) == known
+
+
+def test_tables_are_bounded_by_their_bytes():
+    """Weights on the preset at target level 9, 31.5 MB of tables each: no more than 6 GiB of them are held, and the oldest is prepared again."""
+    load_package()
+    from efla_amd import hellm
+    H = hellm.HEMMer(preset=True, seed=SEED)
+    rng = np.random.default_rng(2)
+    B = rng.uniform(-1, 1, (128, 128))
+    a = H.encrypt2(B, B)
+    tables = 15 * 512 * 32 * 8 * 16
+    room = 6 * 1024 ** 3 // tables
+
+    def transforms(i):   # of the product with weight i
+        w = H.encode2(np.roll(B, i % 128, 1), np.roll(B, i // 128, 0), 10)
+        H.traffic(reset=True)
+        H.single_matmul(a, w, 9)
+        return H.traffic(reset=True)[1]["transforms"]
+
+    transforms(0)
+    known = transforms(0)
+    held = H.key_bytes()["pool"]
+    for i in range(1, room + 24):
+        assert transforms(i) == known + 2   # (decoding it is two launches)
+    grown = H.key_bytes()["pool"] - held
+    assert (room - 2) * tables < grown < 6 * 1024 ** 3
+    assert transforms(room + 23) == transforms(24) == known
+    assert transforms(23) == known + 2
