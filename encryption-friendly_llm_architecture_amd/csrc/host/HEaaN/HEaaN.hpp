@@ -73,7 +73,7 @@ u64 getEncryptionLevel(const Context &c);
 std::vector<u64> getPrimeList(const Context &c);
 std::vector<Real> getDefaultScaleFactorList(const Context &c);
 hemm_context *getDeviceContext(const Context &c);
-void setSeed(u64 seed);  // seeds the key / encryption samplers
+void setSeed(u64 seed);  // seeds the encryption samplers, and the secret keys made from now on with the evaluation keys derived from them
 
 // ---- device memory ---------------------------------------------------------------------------
 class DeviceBuffer {
@@ -191,10 +191,12 @@ public:
     const std::vector<int> &getCoefficients() const { return coeffs_; }
     const u64 *ntt() const { return ntt_.data(); }  // [nQ+nP][N]
     const Context &getContext() const { return ctx_; }
+    u64 seed() const { return seed_; }   // of the evaluation keys derived from this key, whenever they are
 
 private:
     void upload();
     Context ctx_;
+    u64 seed_;
     std::vector<int> coeffs_;
     DeviceBuffer ntt_;
 };

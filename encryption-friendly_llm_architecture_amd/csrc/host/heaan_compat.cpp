@@ -371,8 +371,8 @@ u64 galois_of_rotation(const Context &c, u64 rot) { return powmod(5, rot % (c->N
 }  // namespace
 
 // ---- keys ----------------------------------------------------------------------------------------
-SecretKey::SecretKey(const Context &c) : ctx_(c), coeffs_(c->N, 0) {
-    const u64 key = stream_key(g_seed, TAG_SK, 0, 0);
+SecretKey::SecretKey(const Context &c) : ctx_(c), seed_(g_seed), coeffs_(c->N, 0) {
+    const u64 key = stream_key(seed_, TAG_SK, 0, 0);
     const int hw = (int)std::min<u64>(192, c->N / 2);
     int placed = 0;
     for (u64 ctr = 0; placed < hw; ctr++) {
@@ -384,10 +384,10 @@ SecretKey::SecretKey(const Context &c) : ctx_(c), coeffs_(c->N, 0) {
     }
     upload();
 }
-SecretKey::SecretKey(const Context &c, const int *coefficients) : ctx_(c), coeffs_(coefficients, coefficients + c->N) {
+SecretKey::SecretKey(const Context &c, const int *coefficients) : ctx_(c), seed_(g_seed), coeffs_(coefficients, coefficients + c->N) {
     upload();
 }
-SecretKey::SecretKey(const Context &c, const std::string &path) : ctx_(c), coeffs_(c->N, 0) {
+SecretKey::SecretKey(const Context &c, const std::string &path) : ctx_(c), seed_(g_seed), coeffs_(c->N, 0) {
     std::ifstream f(path, std::ios::binary);
     if (!f) throw RuntimeException("cannot open " + path);
     u64 n = 0;
@@ -541,9 +541,9 @@ void KeyGenerator::genSwitchKey(u64 key_id, const u64 *s_from, DeviceBuffer &out
     for (u64 d = 0; d < c->dnum; d++) {
         u64 *b = out.data() + (d * 2 + 0) * T * N, *a = out.data() + (d * 2 + 1) * T * N;
         // error and uniform part are sampled on the device (same counter-based streams as the host samplers)
-        ck(hemm_sample_error(c->dev, stream_key(g_seed, TAG_EVK_E, key_id, d), primes.data(), (uint32_t)T, e.data(), nullptr));
+        ck(hemm_sample_error(c->dev, stream_key(sk_.seed(), TAG_EVK_E, key_id, d), primes.data(), (uint32_t)T, e.data(), nullptr));
         ck(hemm_ntt(c->dev, e.data(), primes.data(), (uint32_t)T, 1, 0, nullptr));
-        for (size_t i = 0; i < T; i++) keys[i] = stream_key(g_seed, TAG_EVK_A, key_id, d * T + i);
+        for (size_t i = 0; i < T; i++) keys[i] = stream_key(sk_.seed(), TAG_EVK_A, key_id, d * T + i);
         ck(hemm_sample_uniform(c->dev, keys.data(), primes.data(), (uint32_t)T, a, nullptr));
         // tmp = a*s ; b = e - tmp     (all T limbs: chain then special, i.e. nq = nQ with_p = 1)
         ck(hemm_pointwise(c->dev, HEMM_MUL, a, 0, sk_.ntt(), 0, tmp.data(), 0, (uint32_t)c->nQ, 1, 1, nullptr));

@@ -721,3 +721,17 @@ def test_two_parameter_sets_take_turns(small):
         w = H.encode(B)
         p = H.single_matmul(ca, w, 2)
         assert np.abs(H.decrypt(p) - A @ B).max() < 2 ** -18
+
+
+def test_keys_derived_later_keep_their_seed():
+    """Rotation keys are derived on first use: one derived after another HEMMer was made is still the key of its own seed."""
+    load_package()
+    from efla_amd import hellm
+    qs, ps = O.ckks_chain(10, 4, 2)
+    first = hellm.HEMMer(10, qs, ps, dnum=2, min_bootstrap_level=0, seed=4)
+    hellm.HEMMer(10, qs, ps, dnum=2, min_bootstrap_level=0, seed=9)
+    first.ensure_rotation_keys([3])
+    alone = hellm.HEMMer(10, qs, ps, dnum=2, min_bootstrap_level=0, seed=4)
+    alone.ensure_rotation_keys([3])
+    galois = pow(5, 3, 2 << 10)
+    assert np.array_equal(first.export_key(galois), alone.export_key(galois))
