@@ -94,6 +94,7 @@ private:
     Context ctx_;
     u64 *ptr_ = nullptr;
     size_t words_ = 0, cap_ = 0;
+    u64 born_ = 0;   // Recordings::now() when the memory was handed out
 };
 
 // ---- value types -----------------------------------------------------------------------------

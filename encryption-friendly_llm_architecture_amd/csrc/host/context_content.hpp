@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <condition_variable>
 #include <map>
 #include <mutex>
@@ -13,6 +14,74 @@
 #include "HEaaN/HEaaN.hpp"
 
 namespace HEaaN {
+
+// A device buffer that was given up, with the readings of Recordings::now() when it was handed out and when it was given up.
+struct Freed {
+    size_t words;
+    u64 *ptr, born, freed;
+};
+// Recorded sequences (hellm_graph_begin / _end) replay on the addresses they were recorded with: masks, tables and keys that were there
+// already, whoever holds them and on whichever context they were made.  A buffer that was there while a recording was open may be one
+// of its addresses; once given up it is kept from reuse for as long as that recording lives.
+class Recordings {
+public:
+    static Recordings &all() {
+        static Recordings *r = new Recordings;   // (outlives every buffer, static ones among them)
+        return *r;
+    }
+    u64 now() const { return now_; }   // counts openings and closings
+    u64 open() {
+        std::lock_guard<std::mutex> lk(mu_);
+        const u64 id = ++now_;
+        closed_[id] = ~u64(0);
+        living_ = closed_.size();
+        return id;
+    }
+    void close(u64 id) {
+        std::lock_guard<std::mutex> lk(mu_);
+        closed_[id] = ++now_;
+    }
+    void drop(u64 id) {
+        std::vector<Freed> rest;
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            closed_.erase(id);
+            living_ = closed_.size();
+            rest.swap(orphans_);
+            dropped_++;
+        }
+        for (const Freed &f : rest) leave(f);
+    }
+    u64 dropped() const { return dropped_; }
+    bool need(const Freed &f) {
+        if (living_ == 0) return false;
+        std::lock_guard<std::mutex> lk(mu_);
+        return needLocked(f);
+    }
+    // memory whose context is gone
+    void leave(const Freed &f) {
+        {
+            std::lock_guard<std::mutex> lk(mu_);
+            if (needLocked(f)) {
+                orphans_.push_back(f);
+                return;
+            }
+        }
+        (void)hipFree(f.ptr);
+    }
+
+private:
+    bool needLocked(const Freed &f) const {
+        for (const auto &r : closed_)
+            if (r.first <= f.freed && r.second > f.born) return true;
+        return false;
+    }
+    std::mutex mu_;
+    std::map<u64, u64> closed_;   // living recordings: when opened -> when closed
+    std::vector<Freed> orphans_;
+    std::atomic<u64> now_{0}, dropped_{0};
+    std::atomic<size_t> living_{0};
+};
 
 struct ContextContent {
     hemm_context *dev = nullptr;
@@ -25,7 +94,9 @@ struct ContextContent {
     // ordered after the last use without any synchronisation.  The one exception is a side chain (forkSide /
     // joinSide below): while it is open, freed buffers are parked and only return to the pool at the join.
     std::multimap<size_t, u64 *> pool;
-    std::vector<std::pair<size_t, u64 *>> parked;
+    std::vector<Freed> parked;
+    std::vector<Freed> held;   // released, but a recording may replay on them
+    u64 held_since = 0;        // Recordings::dropped() when they were last looked at
     std::mutex mu;
     size_t pool_bytes = 0;
     hipStream_t side = nullptr;
@@ -80,7 +151,7 @@ struct ContextContent {
         (void)hipStreamWaitEvent(stream(), ev_join, 0);
         std::lock_guard<std::mutex> lk(mu);
         side_open = false;
-        for (auto &kv : parked) pool.emplace(kv.first, kv.second);
+        for (const Freed &f : parked) reuse(f);
         parked.clear();
     }
 
@@ -155,6 +226,12 @@ struct ContextContent {
     u64 *alloc(size_t words) {
         {
             std::lock_guard<std::mutex> lk(mu);
+            if (!held.empty() && held_since != Recordings::all().dropped()) {
+                std::vector<Freed> all;
+                all.swap(held);
+                held_since = Recordings::all().dropped();
+                for (const Freed &f : all) reuse(f);
+            }
             auto it = pool.find(words);
             if (it != pool.end()) {
                 u64 *r = it->second;
@@ -172,22 +249,29 @@ struct ContextContent {
     // stays with the graph being recorded -- its replays write that memory -- and returns to the pool when the graph
     // is destroyed.
     bool capture_open = false;
-    std::vector<std::pair<size_t, u64 *>> captured;
-    void release(u64 *ptr, size_t words) {
+    std::vector<Freed> captured;
+    void release(u64 *ptr, size_t words, u64 born) {
         std::lock_guard<std::mutex> lk(mu);
+        const Freed f{words, ptr, born, Recordings::all().now()};
         if (capture_open)
-            captured.emplace_back(words, ptr);
+            captured.push_back(f);
         else if (side_open)
-            parked.emplace_back(words, ptr);
+            parked.push_back(f);
         else
-            pool.emplace(words, ptr);
+            reuse(f);
+    }
+    void reuse(const Freed &f) {   // (with mu held)
+        if (Recordings::all().need(f))
+            held.push_back(f);
+        else
+            pool.emplace(f.words, f.ptr);
     }
     ~ContextContent() {
         (void)hipDeviceSynchronize();
         traceClear();
         for (auto &kv : pool) (void)hipFree(kv.second);
-        for (auto &kv : parked) (void)hipFree(kv.second);
-        for (auto &kv : captured) (void)hipFree(kv.second);
+        for (const std::vector<Freed> *l : {&parked, &held, &captured})
+            for (const Freed &f : *l) Recordings::all().leave(f);
         for (auto &st : stages) (void)hipEventDestroy(st.done);
         if (stage_memory) (void)hipHostFree(stage_memory);
         if (side) (void)hipStreamDestroy(side);

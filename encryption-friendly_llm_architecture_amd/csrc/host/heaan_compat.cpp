@@ -216,13 +216,14 @@ DeviceBuffer &DeviceBuffer::operator=(DeviceBuffer &&o) noexcept {
     ptr_ = o.ptr_;
     words_ = o.words_;
     cap_ = o.cap_;
+    born_ = o.born_;
     o.ptr_ = nullptr;
     o.words_ = o.cap_ = 0;
     return *this;
 }
 DeviceBuffer::~DeviceBuffer() { release(); }
 void DeviceBuffer::release() {
-    if (ptr_ && ctx_) ctx_->release(ptr_, cap_);
+    if (ptr_ && ctx_) ctx_->release(ptr_, cap_, born_);
     ptr_ = nullptr;
     words_ = cap_ = 0;
     ctx_.reset();
@@ -234,6 +235,7 @@ void DeviceBuffer::resize(const Context &c, size_t words) {
     }
     release();
     ctx_ = c;
+    born_ = Recordings::all().now();
     ptr_ = c->alloc(words);
     words_ = cap_ = words;
 }

@@ -172,7 +172,8 @@ struct hellm_graph {
     hipStream_t stream = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    std::vector<std::pair<size_t, HEaaN::u64 *>> owned;   // intermediates of the recorded calls
+    std::vector<HEaaN::Freed> owned;   // intermediates of the recorded calls
+    HEaaN::u64 recording = 0;          // HEaaN::Recordings::open()
     size_t nodes = 0;
 };
 namespace {
@@ -180,6 +181,12 @@ void hipck(hipError_t e, const char *what) {
     if (e != hipSuccess) throw RuntimeException(std::string(what) + ": " + hipGetErrorString(e));
 }
 thread_local hellm_graph *g_recording = nullptr;
+// what the graph kept from reuse goes back, except what another recording needs too
+void giveBack(hellm_graph *g) {
+    HEaaN::Recordings::all().drop(g->recording);
+    std::lock_guard<std::mutex> lk(g->ctx->mu);
+    for (const auto &f : g->owned) g->ctx->reuse(f);
+}
 }  // namespace
 int hellm_graph_begin(hellm_hemmer *h) {
     FACADE_TRY
@@ -201,6 +208,7 @@ int hellm_graph_begin(hellm_hemmer *h) {
         delete g;
         throw;
     }
+    g->recording = HEaaN::Recordings::all().open();
     c->capture_open = true;
     g_recording = g;
     FACADE_CATCH
@@ -219,9 +227,9 @@ int hellm_graph_end(hellm_hemmer *h, hellm_graph **out) {
         c->capture_open = false;
         g->owned.swap(c->captured);
     }
+    HEaaN::Recordings::all().close(g->recording);
     auto drop = [&]() {
-        std::lock_guard<std::mutex> lk(c->mu);
-        for (auto &kv : g->owned) c->pool.emplace(kv.first, kv.second);
+        giveBack(g);
         if (g->graph) (void)hipGraphDestroy(g->graph);
         (void)hipStreamDestroy(g->stream);
         delete g;
@@ -263,10 +271,7 @@ void hellm_graph_destroy(hellm_graph *g) {
     if (g->exec) (void)hipGraphExecDestroy(g->exec);
     if (g->graph) (void)hipGraphDestroy(g->graph);
     (void)hipStreamDestroy(g->stream);
-    {
-        std::lock_guard<std::mutex> lk(g->ctx->mu);
-        for (auto &kv : g->owned) g->ctx->pool.emplace(kv.first, kv.second);
-    }
+    giveBack(g);
     delete g;
 }
 

@@ -80,3 +80,50 @@ def test_two_contexts_replay_side_by_side():
             assert np.abs(H.decrypt(res) - prod).max() < 2.0 ** -12
     for _, graph, _, _, _, _ in lanes:
         graph.free()
+
+
+def test_recorded_products_outlive_the_caches():
+    """A recorded product reads masks, tables and keys that were there when it was recorded.  Another parameter set empties the caches
+    of the first, whose memory the next eager products would then take for their own; and the evaluator on whose context the masks were
+    made may be gone by the time of a replay."""
+    load_package()
+    from efla_amd import hellm
+    qs, ps = O.ckks_chain(10, 8, 3)
+    qs2, ps2 = O.ckks_chain(10, 9, 3)
+    rng = np.random.default_rng(12)
+    A, B = rng.uniform(-1, 1, (16, 16)), rng.uniform(-1, 1, (16, 16))
+    maker = hellm.HEMMer(10, qs, ps, dnum=3, min_bootstrap_level=0, seed=7)
+    other = hellm.HEMMer(10, qs2, ps2, dnum=3, min_bootstrap_level=0, seed=8)
+    H = hellm.HEMMer(10, qs, ps, dnum=3, min_bootstrap_level=0, seed=7)
+
+    def operands(h):
+        return h.encrypt(A), h.encrypt(B), h.encode(B)
+
+    def products(h, a, b, w, target=2):
+        return [h.single_cc_matmul(a, b, target), h.single_matmul(a, w, target)]
+
+    products(maker, *operands(maker))   # the masks and tables that H's products will use are on this context
+    ops = operands(H)
+    pool = []
+    for cycle in range(3):
+        want = [c.residues() for c in products(H, *ops)]
+        H.sync()
+        graph, res = H.record(lambda: products(H, *ops))
+        products(other, *operands(other))   # empties the caches
+        if maker is not None:
+            maker.close()
+            maker = None
+        for replay in range(3):
+            for target in (1, 2, 3):
+                products(H, *operands(H), target)
+            for c in res:   # something else, for the replay to write over
+                H.assign(c, H.level_down(ops[0], 2))
+            H.sync()
+            graph.launch()
+            graph.sync()
+            assert [np.array_equal(c.residues(), r) for c, r in zip(res, want)] == [True, True], (cycle, replay)
+        del res
+        graph.free()
+        H.sync()
+        pool.append(H.key_bytes()["pool"])
+    assert pool[2] == pool[1]
