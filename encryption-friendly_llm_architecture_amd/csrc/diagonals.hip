@@ -324,7 +324,9 @@ bool diagonals_ok(const hemm_context *c, u32 k, u32 w, u32 g, int nq) {
     auto pow2 = [](u32 v) { return v != 0 && (v & (v - 1)) == 0; };
     for (u64 q : c->primes)   // what the lazy dot products and their reduction take
         if ((q >> 60) != 0 || (q >> 32) == 0) return false;
-    return ring_has_fused_forms(c) && c->nP >= 1 && nq <= 3 * c->alpha && pow2(k) && pow2(w) && pow2(g) && g >= 4 && g <= k && g <= HOISTED_ARG_TERMS && k <= w && w <= DIAG_MAX_W && 2 * (size_t)w <= c->N;
+    // 4w <= N: a thread's two residues lie in one run of N / 2w
+    return ring_has_fused_forms(c) && c->nP >= 1 && nq <= 3 * c->alpha && pow2(k) && pow2(w) && pow2(g) && g >= 4 && g <= k && g <= HOISTED_ARG_TERMS &&
+           k <= w && w <= DIAG_MAX_W && 4 * (size_t)w <= c->N;
 }
 static u32 diagonal_chunks(u32 k, u32 g) { return (2 * k / g + DIAG_OUT - 1) / DIAG_OUT; }
 size_t diagonal_table_words(const hemm_context *c, u32 k, u32 w, u32 g, int nq) {

@@ -225,7 +225,7 @@ void hemm_abi_sizes(uint32_t *rot_term_bytes, uint32_t *lin_term_bytes);
 int hemm_sum_parts(hemm_context *ctx, const uint64_t *parts, uint32_t n_parts, uint32_t n_out, uint32_t nq, uint64_t *y,
                    void *stream);
 /* A plaintext matrix applied to every row of an encrypted one over its diagonals, in g baby and 2k / g giant steps: k x k tiles side by
- * side in rows of w slots (k, w, g powers of two, 4 <= g <= k <= w <= 512, g <= 32, 2w <= N; primes of 33 to 60 bits; N >= 1024;
+ * side in rows of w slots (k, w, g powers of two, 4 <= g <= k <= w <= 512, g <= 32, 4w <= N; primes of 33 to 60 bits; N >= 1024;
  * nq limbs of at most three digits).  With
  * rotations x_j = rho^j(A) in the extended basis (one term each as for hemm_hoisted_terms, without factors, j = 1 .. g - 1, and x_0 = P A from `a`
  * itself) and
