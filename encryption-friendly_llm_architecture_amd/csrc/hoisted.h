@@ -384,9 +384,9 @@ __device__ __forceinline__ void two_source_int(const RotTermDev &T, const KeyLim
         add128(pa[0], mul64wide(z.x, ka.x));
         add128(pa[1], mul64wide(z.y, ka.y));
     }
-    for (int i = 0; i < 2; i++) {   // at most 3 q^2: the short reduction applies
-        rb[i] = beta <= 3 ? barrett3_u(pb[i], m) : barrett128_u(pb[i], m);
-        ra[i] = beta <= 3 ? barrett3_u(pa[i], m) : barrett128_u(pa[i], m);
+    for (int i = 0; i < 2; i++) {   // 3 q^2 and less: the short reduction applies
+        rb[i] = beta <= 3 ? barrett3_u(pb[i], m) : barrett128_u(cut_sum(pb[i], m), m);
+        ra[i] = beta <= 3 ? barrett3_u(pa[i], m) : barrett128_u(cut_sum(pa[i], m), m);
     }
     if (j < nq) {
         ulonglong2 b1 = load2(T.b + (size_t)j * N + base);
@@ -470,10 +470,10 @@ __device__ __forceinline__ void hoisted_pair_int(const RotTermDev *__restrict__ 
             ra[0] = barrett3_u(sa[0], m);
             ra[1] = barrett3_u(sa[1], m);
         } else {
-            rb[0] = barrett128_u(sb[0], m);
-            rb[1] = barrett128_u(sb[1], m);
-            ra[0] = barrett128_u(sa[0], m);
-            ra[1] = barrett128_u(sa[1], m);
+            rb[0] = barrett128_u(cut_sum(sb[0], m), m);
+            rb[1] = barrett128_u(cut_sum(sb[1], m), m);
+            ra[0] = barrett128_u(cut_sum(sa[0], m), m);
+            ra[1] = barrett128_u(cut_sum(sa[1], m), m);
         }
         if (j < nq && T.b != nullptr) {
             ulonglong2 bv = load2(T.b + (size_t)j * N + base);

@@ -203,8 +203,8 @@ __global__ __launch_bounds__(256) void inner_product_kernel(const u64 *__restric
         add128(sb, mul64wide(x, kb));
         add128(sa, mul64wide(x, ka));
     }
-    acc[(size_t)j * N + n] = barrett128(sb, m);
-    acc[((size_t)n_ext + j) * N + n] = barrett128(sa, m);
+    acc[(size_t)j * N + n] = barrett128(cut_sum(sb, m), m);
+    acc[((size_t)n_ext + j) * N + n] = barrett128(cut_sum(sa, m), m);
 }
 
 // out[p][j] = (a[p][j] - t[p][j]) * cst[j]  (+ add[p][j] when add != nullptr)

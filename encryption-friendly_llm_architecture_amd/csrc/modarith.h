@@ -70,7 +70,8 @@ __device__ __forceinline__ u64 reduce_below_32q(u64 v, const u64 q) {
         if (v >= (u64)m * q) v -= (u64)m * q;
     return v;
 }
-// Barrett reduction of a 128-bit value T < 6 * 2^(2k) to [0, q).
+// Barrett reduction of a 128-bit value T to [0, q): T < 6 * 2^(2k) for primes below 2^60, T < 4 * 2^(2k) for those of 61 bits, where
+// T / 2^(k-1) fills 64 bits.
 __device__ __forceinline__ u64 barrett128(u128_t t, const ModQ &m) {
     const u32 k = m.k;
     u64 t1 = (t.hi << (65 - k)) | (t.lo >> (k - 1));
@@ -93,6 +94,16 @@ __device__ __forceinline__ u64 barrett_tight(u128_t t, const ModQ &m) {
     const u64 qhat = __umul64hi(t1, m.mu3) >> 1;
     const u64 r = t.lo - qhat * m.q;
     return r >= m.q ? r - m.q : r;
+}
+// any T: a sum of as many products of residues as 128 bits hold.  Multiples of 2^(k+1) q are taken off first, in front of the reduction and not
+// in the loop that sums the products: there it costs every kernel registers, whatever number of digits it is run for.
+__device__ __forceinline__ u128_t cut_sum(u128_t t, const ModQ &m) {   // to below 2 * 2^(2k)
+    const u64 hi = m.q >> (63 - m.k), lo = m.q << (m.k + 1);
+    while (t.hi > hi || (t.hi == hi && t.lo >= lo)) {
+        t.hi -= hi + (t.lo < lo ? 1 : 0);
+        t.lo -= lo;
+    }
+    return t;
 }
 // T < 3 * 2^(2k)
 __device__ __forceinline__ u64 barrett3(u128_t t, const ModQ &m) {
