@@ -190,6 +190,9 @@ CtxtTensor multPackedMatMatPreRev(const HomEvaluator &eval, const CtxtTensor &b,
                                   MatrixTransformer &transformer);
 CtxtTensor multPackedMatMatCCReuse(const HomEvaluator &eval, const std::vector<Ciphertext> &tmp, const CtxtTensor &b,
                                    u64 target_level, MatrixTransformer &transformer);
+// The forms that keep the column shifts of an operand make one per row, under masks of which there are two per column: throws for a tile
+// that is higher than wide.
+void checkShifts(const CtxtTensor &a, const char *what);
 // hoisted form: all column shifts of sigma(A) once, then one accumulation per weight tile
 void multMatMatPre(const HomEvaluator &eval, const CtxtTensor &a, std::vector<Ciphertext> &tmp, u64 target_level,
                    MatrixTransformer &transformer);

@@ -422,6 +422,10 @@ void checkLevel(u64 level, const Bootstrapper &btp) {
 }
 }  // namespace
 
+void checkShifts(const CtxtTensor &a, const char *what) {
+    if (a.getHeight() > a.getWidth()) throw std::invalid_argument(std::string(what) + " tiles are not higher than wide.");
+}
+
 template <>
 CtxtTensor multMatMat<Ciphertext>(const HomEvaluator &eval, const Bootstrapper &btp, const CtxtTensor &op1,
                                   const CtxtTensor &op2, u64 T, MatrixTransformer &tr) {
@@ -715,6 +719,7 @@ void multPackedMatMatPreRot(const HomEvaluator &eval, const CtxtTensor &a_in, st
     const Context &ctx = eval.getContext();
     tmp.clear();
     const i64 n = a_in.getHeight();
+    checkShifts(a_in, "[multPackedMatMatPreRot]");
     CtxtTensor a(a_in);
     Ciphertext first(ctx);
     eval.levelDownOne(a.get(), first);
@@ -762,6 +767,7 @@ void multMatMatPre(const HomEvaluator &eval, const CtxtTensor &a_in, std::vector
     const Context &ctx = eval.getContext();
     tmp.clear();
     const i64 n = a_in.getHeight();
+    checkShifts(a_in, "[multMatMatPre]");
     CtxtTensor a(a_in);
     if (a.getLevel() < T + 3)
         throw std::invalid_argument("[multMatMatPre] level >= " + std::to_string(T + 3) + " is needed.");

@@ -1520,6 +1520,7 @@ void multMatMatPreFused(const HomEvaluator &eval, const CtxtTensor &a_in, std::v
     const Context &c = eval.getContext();
     tmp.clear();
     const i64 n = a_in.getHeight();
+    checkShifts(a_in, "[multMatMatPre]");
     if (a_in.getLevel() < T + 3)
         throw std::invalid_argument("[multMatMatPre] level >= " + std::to_string(T + 3) + " is needed.");
     std::vector<Plaintext> &cm = tr.getColMaskExt(eval, a_in.getShape(), T + 2, first_block_only);
@@ -1552,6 +1553,7 @@ void multPackedMatMatPreRotFused(const HomEvaluator &eval, const CtxtTensor &a_i
     const Context &c = eval.getContext();
     tmp.clear();
     const i64 n = a_in.getHeight();
+    checkShifts(a_in, "[multPackedMatMatPreRot]");
     if (a_in.getLevel() != T + 2 || a_in.get().getRescaleCounter() != 0)
         throw std::invalid_argument("[multPackedMatMatPreRot] operand must be at level " + std::to_string(T + 2) + ".");
     std::vector<Plaintext> &cm = tr.getColMaskExt(eval, a_in.getShape(), T + 2);

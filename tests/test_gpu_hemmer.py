@@ -735,3 +735,19 @@ def test_keys_derived_later_keep_their_seed():
     alone.ensure_rotation_keys([3])
     galois = pow(5, 3, 2 << 10)
     assert np.array_equal(first.export_key(galois), alone.export_key(galois))
+
+
+@pytest.mark.parametrize("fused", [True, False])
+def test_shifts_of_a_tall_tile_are_refused(fused):
+    """There are masks for as many shifts as a tile has columns: a tile of more rows than that would read past them."""
+    load_package()
+    from efla_amd import hellm
+    qs, ps = O.ckks_chain(10, 8, 3)
+    H = hellm.HEMMer(10, qs, ps, dnum=3, min_bootstrap_level=0, seed=4)
+    H.set_schedule(fused)
+    A = np.random.default_rng(1).uniform(-1, 1, (16, 8))
+    with pytest.raises(ValueError, match="higher than wide"):
+        H.matmul_pre(H.encrypt2(A, A), 2)
+    with pytest.raises(ValueError, match="higher than wide"):
+        H.packed_matmul_pre_rot(H.level_down(H.encrypt2(A, A), 4), 2)
+    assert len(H.matmul_pre(H.encrypt2(A[:8], A[8:]), 2)) == 8
