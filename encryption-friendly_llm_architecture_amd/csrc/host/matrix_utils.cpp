@@ -314,6 +314,8 @@ CtxtTensor MatrixTransformer::packedDiagonalToRow(const HomEvaluator &eval, cons
 }
 
 // plaintext operands are permuted on the host (decode -> permute -> encode)
+// where tiles do not fill the slot vector evenly, the last one goes on beyond it
+static Complex slotOrZero(const Message &m, i64 slot) { return slot < (i64)m.getSize() ? m[(u64)slot] : Complex(0); }
 template <>
 PtxtTensor MatrixTransformer::diagonalToRow<Plaintext>(const HomEvaluator &eval, const PtxtTensor &op) {
     const Context &ctx = eval.getContext();
@@ -324,7 +326,7 @@ PtxtTensor MatrixTransformer::diagonalToRow<Plaintext>(const HomEvaluator &eval,
     for (i64 r = 0; r < height; r++)
         for (i64 c = 0; c < w; c++) {
             const i64 rb = r - r % n, cb = c - c % n, i = r % n, j = c % n;
-            dst[(u64)(r * w + c)] = src[(u64)((rb + (i + j) % n) * w + cb + j)];
+            dst[(u64)(r * w + c)] = slotOrZero(src, (rb + (i + j) % n) * w + cb + j);
         }
     return PtxtTensor(op.getShape(), endec.encode(dst, op.getLevel()));
 }
@@ -338,7 +340,7 @@ PtxtTensor MatrixTransformer::diagonalToColumn<Plaintext>(const HomEvaluator &ev
     for (i64 r = 0; r < height; r++)
         for (i64 c = 0; c < w; c++) {
             const i64 cb = c - c % n, i = r % n, j = c % n;
-            dst[(u64)(r * w + c)] = src[(u64)(r * w + cb + (i + j) % n)];
+            dst[(u64)(r * w + c)] = slotOrZero(src, r * w + cb + (i + j) % n);
         }
     return PtxtTensor(op.getShape(), endec.encode(dst, op.getLevel()));
 }
