@@ -816,6 +816,7 @@ namespace {
 // ones on columns [block * low, (block + 1) * low) of the first tile (or of every tile of width `cols`) in `rows` rows
 Message lowColBlockMask(u64 log_slots, u64 rows, u64 cols, u64 w, u64 block, u64 low, bool every_tile) {
     Message m(log_slots, 0);
+    if (cols == 0 || block >= cols / low || rows * w > m.getSize()) throw std::invalid_argument("[lowColBlock] no such block of columns.");
     for (u64 i = 0; i < rows; i++)
         for (u64 k = 0; k < (every_tile ? w : 1); k += cols)
             for (u64 j = block * low; j < (block + 1) * low; j++) m[i * w + k + j] = 1;
@@ -824,6 +825,7 @@ Message lowColBlockMask(u64 log_slots, u64 rows, u64 cols, u64 w, u64 block, u64
 // ones on rows [block * low, (block + 1) * low), columns [0, width)
 Message lowRowBlockMask(u64 log_slots, u64 w, u64 block, u64 low, u64 width) {
     Message m(log_slots, 0);
+    if (width == 0 || width > w || block >= m.getSize() / (low * w)) throw std::invalid_argument("[lowRowBlock] no such block of rows.");
     for (u64 i = block * low; i < (block + 1) * low; i++)
         for (u64 j = 0; j < width; j++) m[i * w + j] = 1;
     return m;

@@ -1,0 +1,29 @@
+"""Calls that would read or write beyond a mask or a message on the host are refused."""
+import numpy as np
+import pytest
+
+from __graft_entry__ import load_package
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def H():
+    load_package()
+    from efla_amd import hellm
+    qs, ps = O.ckks_chain(10, 8, 3)
+    return hellm.HEMMer(10, qs, ps, dnum=3, min_bootstrap_level=0, seed=4)
+
+
+def tile(rows, cols):
+    return np.random.default_rng(rows * 100 + cols).uniform(-1, 1, (rows, cols))
+
+
+def test_blocks_beyond_the_tile(H):
+    a = H.encrypt2(tile(16, 16), tile(16, 16))
+    for call in (H.repack_to_one_col, H.repack_to_multi_col, H.get_low_col_block, H.repack_to_one_row, H.repack_to_multi_row, H.get_low_row_block):
+        call(a, 7)
+        for block in (8, 1 << 40):
+            with pytest.raises(ValueError, match="no such block"):
+                call(a, block)
