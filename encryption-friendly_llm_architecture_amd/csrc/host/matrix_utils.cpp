@@ -56,6 +56,7 @@ Geometry geometry(MaskKind kind, const TileTensorShape &s) {
     (void)packing;   // the composite kinds move by single columns / rows: the geometry of the plain transforms
     g.cell = packed ? 2 : 1;
     g.units = (vertical ? rows : cols) / g.cell;
+    if (g.units < 1) throw std::invalid_argument("[MatrixTransformer] packed transforms need two rows and columns");
     g.sub = std::min(rows, cols) / g.cell;
     g.bs = (i64)std::ceil(std::sqrt((double)(2 * g.sub - 1)));
     g.gs = (i64)std::ceil((double)(g.sub - 1) / (double)g.bs);
@@ -510,6 +511,8 @@ CtxtTensor lowRankTerms(const HomEvaluator &eval, Ciphertext &a, Ciphertext &b, 
                         const CtxtTensor &op2, i64 w, u64 T, i64 low_dim, MatrixTransformer &tr) {
     const Context &ctx = eval.getContext();
     const i64 num_rows = op1.getHeight();
+    if (op1.getWidth() < low_dim || op2.getHeight() < low_dim)
+        throw std::invalid_argument("[multMatMatLow] the operands need " + std::to_string(low_dim) + " columns / rows.");
     CtxtTensor res(ctx, op1.getHeight(), op2.getWidth(), op2.getBlockWidth());
     eval.mult(a, b, res.get());
     if (low_dim < 2) return res;

@@ -62,6 +62,7 @@ Geo geo(MaskKind kind, const TileTensorShape &s) {
     g.n = rows;
     g.cell = packed ? 2 : 1;
     g.units = (vertical ? rows : cols) / g.cell;
+    if (g.units < 1) throw std::invalid_argument("[MatrixTransformer] packed transforms need two rows and columns");
     g.sub = std::min(rows, cols) / g.cell;
     g.bs = (i64)std::ceil(std::sqrt((double)(2 * g.sub - 1)));
     g.gs = (i64)std::ceil((double)(g.sub - 1) / (double)g.bs);

@@ -27,3 +27,14 @@ def test_blocks_beyond_the_tile(H):
         for block in (8, 1 << 40):
             with pytest.raises(ValueError, match="no such block"):
                 call(a, block)
+
+
+def test_low_rank_products_of_thinner_tiles(H):
+    thin, a = H.encrypt2(tile(1, 1), tile(1, 1)), H.encrypt2(tile(16, 16), tile(16, 16))
+    for x, y in ((thin, thin), (a, thin)):
+        for call in (lambda: H.matmul_high_low(x, y, 0, 2), lambda: H.matmul_low_high(x, y, 0, 2), lambda: H.matmul_low_low(x, y, 0, 0, 2)):
+            with pytest.raises(Exception):
+                call()
+    for call in (H.packed_matmul_pre, H.packed_matmul_pre_rev):
+        with pytest.raises(ValueError, match="two rows and columns"):
+            call(thin, 2)
