@@ -84,7 +84,7 @@ void oddSetUp(const HomEvaluator &eval, const Ciphertext &ctxt, std::vector<Ciph
 void oddBabyStep(const HomEvaluator &eval, const std::vector<Ciphertext> &odd, const std::vector<double> &poly,
                  Ciphertext &res, int k) {
     Ciphertext r(eval.getContext()), t(eval.getContext());
-    eval.mult(odd[0], Complex(poly[1], 0.0), r);
+    eval.mult(odd[0], Complex(poly.size() > 1 ? poly[1] : 0.0, 0.0), r);   // (a quotient may be a constant)
     for (int i = 1; i < k / 2; i++) {
         if ((size_t)(2 * i + 1) >= poly.size()) continue;
         eval.mult(odd[(size_t)i], Complex(poly[(size_t)(2 * i + 1)], 0.0), t);

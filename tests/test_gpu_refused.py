@@ -38,3 +38,12 @@ def test_low_rank_products_of_thinner_tiles(H):
     for call in (H.packed_matmul_pre, H.packed_matmul_pre_rev):
         with pytest.raises(ValueError, match="two rows and columns"):
             call(thin, 2)
+
+
+def test_odd_polynomial_whose_quotient_is_a_constant(H):
+    """Degree 8 by blocks of two: the last quotient has a constant term only, of which an odd polynomial takes nothing"""
+    x = np.linspace(-1, 1, 256).reshape(16, 16)
+    c = [0, 0.5, 0, -0.25, 0, 0.125, 0, 0.0625, 0.75]
+    with np.errstate(all="ignore"):
+        got = H.decrypt(H.eval_odd_polynomial(H.encrypt(x), c, 2, 3))
+    assert np.abs(got - sum(c[i] * x ** i for i in (1, 3, 5, 7))).max() < 1e-6
