@@ -750,4 +750,5 @@ def test_shifts_of_a_tall_tile_are_refused(fused):
         H.matmul_pre(H.encrypt2(A, A), 2)
     with pytest.raises(ValueError, match="higher than wide"):
         H.packed_matmul_pre_rot(H.level_down(H.encrypt2(A, A), 4), 2)
-    assert len(H.matmul_pre(H.encrypt2(A[:8], A[8:]), 2)) == 8
+    B = np.hstack([A, A])
+    assert len(H.matmul_pre(H.encrypt2(B, B), 2)) == 16
