@@ -4,9 +4,8 @@
 Headline metric: ms per 128 x 128 ciphertext-ciphertext matrix product
 (HEMMer::singleCCMatMul, N = 2^16, 13 + 4 primes, dnum 3, scale 2^42, inputs fresh at level 12,
 target level 4), inputs and keys resident in HBM.  Also reported in the same JSON line: one
-key-switched rotation at levels 12 and 6, batched NTT limb-transforms/s, the roofline of the
-dominant kernel family (the ModDown chain of the main loop), of the hoisted key-switch sums and of the NTT
-launch pair, and the CPU oracle timed on the host cores.
+key-switched rotation at levels 12 and 6, batched NTT limb-transforms/s, the rooflines of one chain of the main loop (key-switch
+sums and the ModDown around which they run), of a transform stage, of a ModDown and of the NTT launch pair, and the CPU oracle timed on the host cores.
 
 A "step" is one full CCMM.  Everything runs on one GPU; --gpus above 1 is refused.
 --roofline-only runs just the roofline legs and --ccmm-only just the headline product loop (used for the committed
@@ -244,125 +243,86 @@ def gpu_ntt(args, out):
     }
 
 
-# HBM bytes per call of the hoisted sum at the shape below (its two launches together), from two rocprofv3 --pmc runs
-# of `bench.py --roofline-only` (FETCH_SIZE, WRITE_SIZE), each scaled by what the same counter reads for the
-# 1 GiB copy this mode also launches (FETCH_SIZE x 2.0, WRITE_SIZE x 1.0):
-# (2 x (159 700.4 + 172 140.0) + 196 608 + 163 840) KiB, see profiles/hoisted_terms_and_ntt_roofline_shapes.txt.
-HOISTED_TRAFFIC_BYTES = 1048707891
-
-
-# HBM bytes of the four launches of one ModDown chain at the shape below, same two counters and scale factors.
-MODDOWN_TRAFFIC_BYTES = 1654669312
+# HBM bytes of one chain of the main loop at the shape below (its launches together), from two rocprofv3 --pmc runs of
+# `bench.py --roofline-only` (FETCH_SIZE, WRITE_SIZE), each scaled by what the same counter reads for the 1 GiB copy this mode also launches
+# (FETCH_SIZE x 2.0, WRITE_SIZE x 1.0): see profiles/main_loop_and_ntt_roofline_shapes.txt.
+CHAIN_TRAFFIC_BYTES = 1161650176
 
 
 def gpu_hoisted(args, out):
-    """Roofline of the dominant kernels, the hoisted sum of the CCMM's main loop: one call produces 32 column shifts
-    of sigma(A) in the extended basis, each the sum of two masked hoisted rotations (of the operand and of its
-    copy rotated by -n) under one key (7 chain + 4 special limbs, 2 digits).  The column masks are run tables (their
-    NTT form is constant over runs of 256 residues), and a call of this size is two launches over disjoint limbs:
-    hoisted_terms_kernel<1, true> (the 6 limbs of primes below 2^44, double precision) and hoisted_terms_kernel<2, true>
-    (the 5 limbs of 60-bit primes, integer); the second template argument says that the keys are in the compact layout.  Timed together: the figure is per call."""
+    """Rooflines of the products' launches at the shapes that the products run them with.
+
+    roofline: one of the two chains of the encrypted product's main loop (operands fresh at level 12, target 4, by halves): 16 column shifts, each the
+    sum of two masked hoisted rotations (of sigma(A) and of its copy rotated by -n) under one key, 8 chain + 4 special limbs, 2 digits, column masks
+    as run tables, compact keys, divided by P and rescaled to 7 limbs.  Four launches: the sums of the five limbs that the ModDown drops, as the first
+    pass of their inverse transform; their column pass; the conversion inside the column pass of the seven kept limbs; the sums of those under
+    their last pass.
+    roofline_transform_stage: one stage of the transform of one operand: a sum of 14 masked rotations and a part that does not rotate, full masks,
+    9 + 4 limbs, divided and rescaled to 8 limbs.
+    roofline_moddown: the ModDown merged with the rescale of the plaintext product's eight inner sums, 16 polynomials of 6 + 4 limbs."""
     import torch
     from __graft_entry__ import load_package
     pkg = load_package()
-    nq, K, dnum, n_out = 7, 4, 3, 32
+    K, dnum = 4, 3
     big = pkg.primes_below(60, 16, 1 + K)
     qs = [big[0]] + pkg.primes_below(42, 16, 12)
     ps = big[1:]
     ctx = pkg.Context(16, qs, ps, dnum)
-    N, E, T, beta, shift = 1 << 16, nq + K, 13 + K, 2, 8
+    N, T, beta, shift = 1 << 16, 13 + K, 2, 8
     g = torch.Generator(device="cuda").manual_seed(11)
 
     def rnd(*shape):
-        # residues below 2^41 are valid for every prime of the set; the kernel's work does not depend on values
+        # residues below 2^41 are valid for every prime of the set; the kernels' work does not depend on values
         return torch.randint(0, 2 ** 41, shape, dtype=torch.int64, device="cuda", generator=g)
 
+    def timed(call, iters=10):
+        for _ in range(2):
+            call()
+        torch.cuda.synchronize()
+        timer = pkg.Timer()
+        timer.start()
+        for _ in range(iters):
+            call()
+        return timer.stop() / iters
+
+    def entry(kernel, ms, moved, **more):
+        return dict({"kernel": kernel, "bound": "hbm", "achieved": moved / (ms * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                     "frac": moved / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, "algorithmic_bytes_per_launch": moved, "avg_ms_per_launch": ms}, **more)
+
+    def key_words_bytes(nq):
+        # what a sum of nq + K limbs reads of one compact key: 6 bytes a residue of the primes below 2^44, 8 of the others
+        small = sum(1 for q in qs[:nq] if q < 2 ** 44)
+        return beta * 2 * (small * 6 + (nq + K - small) * 8) * N
+
+    # algorithmic bytes of the sums: every key, source and mask read once, every result written once
+    nq, n_out = 8, 16
+    E = nq + K
     src = [(rnd(beta, E, N), rnd(nq, N)) for _ in range(2)]
     groups = []
     for o in range(n_out):
-        # keys in the compact layout, as the product's schedule passes them (6 bytes per residue of a prime below 2^44)
         evk, gal = ctx.compact_key(rnd(dnum, 2, T, N)), pow(5, o + 1, 2 * N)
-        groups.append([(src[t][0], src[t][1], evk, rnd(E, N >> shift), gal, shift) for t in range(2)])
-    for _ in range(2):
-        ctx.hoisted_terms(groups, nq, b_premultiplied=True, compact_keys=True)
-    torch.cuda.synchronize()
-    timer = pkg.Timer()
-    iters = 10
-    timer.start()
-    for _ in range(iters):
-        ctx.hoisted_terms(groups, nq, b_premultiplied=True, compact_keys=True)
-    ms = timer.stop() / iters
-    # algorithmic bytes: per output beta x 2 x E key limbs read (6 of them 6 bytes per residue, 5 of them 8) + 2 x E
-    # limbs written (the mask tables are 2 x E x 4 KiB per output, a value and its Shoup companion per run: counted,
-    # negligible); the two rotation sources (beta x E + nq limbs each) read once
-    n_small = sum(1 for q in qs[:nq] if q < 2 ** 44)
-    key_bytes = beta * 2 * (n_small * 6 + (E - n_small) * 8) * N
-    limbs = n_out * 2 * E + 2 * (beta * E + nq)
-    alg_bytes = n_out * key_bytes + limbs * LIMB_BYTES + n_out * 2 * E * (N >> shift) * 16
-    achieved = alg_bytes / (ms * 1e-3) / 1e9
-    out["roofline_hoisted_sum"] = {
-        "kernel": "hoisted_terms_kernel<1, true> + hoisted_terms_kernel<2, true> (one hoisted sum of the CCMM main loop: 32 "
-                  "outputs x 2 masked sources under one compact key, 7+4 limbs, 2 digits, run-table masks; "
-                  "double-precision limbs and integer limbs in one launch each)",
-        "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-        "frac": achieved / HBM_PEAK_GBS, "traffic": HOISTED_TRAFFIC_BYTES,
-        "algorithmic_bytes_per_launch": alg_bytes, "avg_ms_per_launch": ms,
-    }
-    # (b) the hoisted sum of one sigma / tau transform stage, the largest single launch of the product
-    # (hoisted_terms_kernel<0, true>): 2 outputs (one per operand) at level T+4, each 7 rotations of two masked sources
-    # under one key, full masks over the extended basis (9 + 4 limbs, 2 digits)
-    nq2, E2 = 9, 9 + K
-    src2 = [[(rnd(beta, E2, N), rnd(nq2, N)) for _ in range(2)] for _ in range(2)]
-    groups2 = []
-    for o in range(2):
-        grp = []
-        for r in range(7):
-            evk, gal = ctx.compact_key(rnd(dnum, 2, T, N)), pow(5, 8 * o + r + 1, 2 * N)
-            grp += [(src2[o][t][0], src2[o][t][1], evk, rnd(E2, N), gal, 0) for t in range(2)]
-        groups2.append(grp)
-    ctx.traffic(reset=True)
-    ctx.hoisted_terms(groups2, nq2, b_premultiplied=True, compact_keys=True)
-    stage_bytes = sum(ctx.traffic(reset=True)[0].values())
-    torch.cuda.synchronize()
-    timer.start()
-    for _ in range(iters):
-        ctx.hoisted_terms(groups2, nq2, b_premultiplied=True, compact_keys=True)
-    ms2 = timer.stop() / iters
-    out["roofline_transform_stage"] = {
-        "kernel": "hoisted_terms_kernel<0, true> (hoisted sum of one sigma/tau transform stage: 2 outputs x 7 compact keys x 2 "
-                  "masked sources, full masks, 9+4 limbs, 2 digits)",
-        "bound": "hbm", "achieved": stage_bytes / (ms2 * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-        "frac": stage_bytes / (ms2 * 1e-3) / 1e9 / HBM_PEAK_GBS, "algorithmic_bytes_per_launch": stage_bytes,
-        "avg_ms_per_launch": ms2,
-    }
-    # (c) the ModDown merged with the rescale of one main-loop batch: 64 polynomials from 7+4 to 6 limbs in four
-    # launches (inverse transform of the 5 dropped limbs, forward transform whose first pass computes the basis
-    # conversion and whose second ends with the fused (y - conv) / (P q_6) tail)
-    y = rnd(64, E, N)
-    ctx.traffic(reset=True)
-    ctx.moddown_batch(y, nq, True)
-    md_by = ctx.traffic(reset=True)[0]
-    md_bytes = sum(md_by.values())
-    torch.cuda.synchronize()
-    timer.start()
-    for _ in range(iters):
-        ctx.moddown_batch(y, nq, True)
-    ms3 = timer.stop() / iters
-    # the same arithmetic with the two column passes and the conversion in one kernel per slab (three launches)
-    timer.start()
-    for _ in range(iters):
-        ctx.moddown_batch(y, nq, True, column_slab=True)
-    ms3_slab = timer.stop() / iters
-    out["roofline"] = {
-        "kernel": "ntt16_rows_kernel<8, 8, true, 0, 0> + ntt16_cols_kernel<8, 16, true> + ntt16_cols_converted_kernel<8, 5> + "
-                  "ntt16_rows_kernel<8, 16, false, 1, 0> (ModDown + rescale of one main-loop batch, 64 polynomials, 7+4 -> 6 limbs: "
-                  "the largest kernel family of the CCMM; the basis conversion runs inside the first forward pass)",
-        "bound": "hbm", "achieved": md_bytes / (ms3 * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-        "frac": md_bytes / (ms3 * 1e-3) / 1e9 / HBM_PEAK_GBS, "traffic": MODDOWN_TRAFFIC_BYTES,
-        "algorithmic_bytes_per_launch": md_bytes, "avg_ms_per_launch": ms3,
-        "algorithmic_bytes_by_kind": {k: v for k, v in md_by.items() if v},
-        "column_slab_form_ms": ms3_slab,
-    }
+        groups.append([(src[t][0], src[t][1], evk, rnd(E, N >> shift, 2), gal, shift) for t in range(2)])
+    ms = timed(lambda: ctx.hoisted_moddown(groups, nq, True, b_premultiplied=True, compact_keys=True))
+    moved = n_out * (key_words_bytes(nq) + 2 * E * (N >> shift) * 16 + 2 * (nq - 1) * LIMB_BYTES) + 2 * (beta * E + nq) * LIMB_BYTES
+    out["roofline"] = entry("hoisted_terms_kernel<0, true, 1, SumRows> + ntt16_cols_kernel<8, 16, 0, true> + ntt16_cols_converted_kernel<8, 0, 5> + "
+                            "hoisted_terms_kernel<0, true, 1, SumTail> (one chain of the CCMM main loop: 16 shifts of two masked sources under one compact key, "
+                            "8+4 limbs, 2 digits, run-table masks, divided by P and rescaled to 7 limbs)", ms, moved, traffic=CHAIN_TRAFFIC_BYTES)
+    nq = 9
+    E = nq + K
+    x, a = (rnd(beta, E, N), rnd(nq, N)), rnd(nq, N)
+    stage = [(x[0], x[1], ctx.compact_key(rnd(dnum, 2, T, N)), rnd(E, N), pow(5, r + 1, 2 * N), 0) for r in range(14)] + [(a, x[1], None, rnd(nq, N), 1, 0)]
+    ms = timed(lambda: ctx.hoisted_moddown([stage], nq, True, compact_keys=True))
+    moved = 14 * (key_words_bytes(nq) + E * LIMB_BYTES) + (beta * E + 3 * nq + 2 * (nq - 1)) * LIMB_BYTES
+    out["roofline_transform_stage"] = entry("hoisted_terms_kernel<0, true, 1, SumRows> and the ModDown behind it (one sigma/tau transform stage of one operand: 14 "
+                                            "rotations under compact keys with full masks and an unrotated part, 9+4 limbs, 2 digits, rescaled to 8 limbs)",
+                                            ms, moved)
+    nq = 6
+    y = rnd(16, nq + K, N)
+    ms = timed(lambda: ctx.moddown_batch(y, nq, True))
+    moved = 16 * (nq + K + nq - 1) * LIMB_BYTES
+    out["roofline_moddown"] = entry("ntt16_rows_kernel<8, 8, true, 0, 0> + ntt16_cols_kernel<8, 16, 0, true> + ntt16_cols_converted_kernel<8, 0, 5> + "
+                                    "ntt16_rows_kernel<8, 16, false, 1, 0> (ModDown and rescale of the plaintext product's eight inner sums: 16 "
+                                    "polynomials, 6+4 -> 5 limbs)", ms, moved)
     if args.roofline_only:
         # a plain copy of known size in the same process: the scale reference for the --pmc counters
         a = torch.empty(1 << 27, dtype=torch.int64, device="cuda").fill_(1)

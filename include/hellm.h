@@ -47,7 +47,8 @@ int hellm_phase_report(hellm_hemmer *h, char *text, size_t capacity);
  * that run the same products on operands rewritten in place).  Between begin and end the calls of this thread on h are
  * recorded instead of run: every buffer they use must exist already, so run the same sequence once before (keys,
  * masks and scratch are made on first use).  Operand and result ciphertexts of the recorded calls must stay alive and
- * in place while the graph is replayed; intermediates belong to the graph until it is destroyed.  A replay runs on
+ * in place while the graph is replayed; intermediates belong to the graph until it is destroyed, and the masks, tables and
+ * keys the calls read are kept from reuse as long.  A replay runs on
  * the graph's own stream and is asynchronous: hellm_graph_sync before anything else touches its operands or results,
  * and before other work on h (the context's scratch has one user at a time).  Term lists too long for the kernel
  * arguments (more than 32 merged terms per launch) are refused while recording. */
