@@ -255,10 +255,10 @@ struct TwoStages {
     typename F::W w0, w1, w;
     __device__ __forceinline__ TwoStages(const typename F::W *__restrict__ tw, const u32 group) : w0(tw[2 * group]), w1(tw[2 * group + 1]), w(tw[group]) {}
     __device__ __forceinline__ void inverse(const F &f, typename F::E (&x)[4]) const {
-        f.gs(x[0], x[1], w0);
-        f.gs(x[2], x[3], w1);
-        f.gs(x[0], x[2], w);
-        f.gs(x[1], x[3], w);
+        f.gs(x[0], x[1], w0, false, false);
+        f.gs(x[2], x[3], w1, false, false);
+        f.gs(x[0], x[2], w, true, true);
+        f.gs(x[1], x[3], w, true, true);
     }
     __device__ __forceinline__ void forward(const F &f, typename F::E (&x)[4]) const {
         f.ct(x[0], x[2], w, false);
@@ -426,6 +426,8 @@ __device__ __forceinline__ void sum_done(const u64 (&rb)[2], const u64 (&ra)[2],
             const Tw *tw = rows.tw + ((size_t)prime << logN);
             if (fp_limb)
                 rows_of_products(FpField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
+            else if ((modq[prime].q >> 60) == 0)
+                rows_of_products(IntFieldT<true>(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
             else
                 rows_of_products(IntField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
             return;

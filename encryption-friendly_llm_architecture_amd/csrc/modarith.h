@@ -48,19 +48,31 @@ __device__ __forceinline__ u64 mul_shoup(u64 x, u64 w, u64 ws, u64 q) {
     return r >= q ? r - q : r;
 }
 
-// x * w - hi' * q with the quotient estimate hi' taken from three of the four 32-bit partial products of x * ws:
-// hi' = xh wh + (xh wl >> 32) + (xl wh >> 32) is at most 2 below floor(x ws / 2^64), so the result lies in [0, 4q)
+// u + x * w - hi' * q with the quotient estimate hi' taken from three of the four 32-bit partial products of x * ws:
+// hi' = xh wh + (xh wl >> 32) + (xl wh >> 32) is at most 2 below floor(x ws / 2^64), so that x * w - hi' * q lies in [0, 4q)
 // instead of [0, 2q) for any 64-bit x.  One multiply-add and the carry chain of the exact high product are saved.
-__device__ __forceinline__ u64 mul_shoup_lazy4(u64 x, u64 w, u64 ws, u64 q) {
+// x * w - hi' * q = x * w + hi' * (2^64 - q) mod 2^64 as 32-bit multiply-adds: the two low products accumulate on u (a carry
+// out of bit 64 is dropped, as it should be), the four cross products, of which only the low word counts, in a register pair of their
+// own.  That pair and the high word are hidden from the compiler, which otherwise makes low products and additions of the
+// cross terms or takes some products twice: 31 vector instructions for an inverse butterfly where this is 17.
+__device__ __forceinline__ u64 add_mul_shoup_lazy4(u64 u, u64 x, u64 w, u64 ws, u64 q) {
     const u32 xl = (u32)x, xh = (u32)(x >> 32), sl = (u32)ws, sh = (u32)(ws >> 32);
     const u64 hi = ((u64)xh * sh + __umulhi(xh, sl)) + __umulhi(xl, sh);
-    // x * w - hi * q = x * w + hi * (2^64 - q) mod 2^64 as one chain of 32-bit multiply-adds: the two low products
-    // accumulate in one 64-bit register (a carry out of bit 64 is dropped, as it should be), the four cross products
-    // only feed the high word; no 64-bit subtraction and none of its carry hazards
     const u64 nq = 0 - q;
     const u32 hl = (u32)hi, hh = (u32)(hi >> 32), wl = (u32)w, wh = (u32)(w >> 32), nl = (u32)nq, nh = (u32)(nq >> 32);
-    const u64 t = (u64)hl * nl + (u64)xl * wl;
-    const u32 top = (u32)(t >> 32) + xl * wh + xh * wl + hl * nh + hh * nl;
+    const u64 t = (u64)hl * nl + ((u64)xl * wl + u);
+    u64 cross = (u64)xl * wh + (u64)xh * wl + (u64)hl * nh + (u64)hh * nl;
+    asm("" : "+v"(cross));
+    u32 top = (u32)(t >> 32) + (u32)cross;
+    asm("" : "+v"(top));
+    return ((u64)top << 32) | (u32)t;
+}
+__device__ __forceinline__ u64 mul_shoup_lazy4(u64 x, u64 w, u64 ws, u64 q) { return add_mul_shoup_lazy4(0, x, w, ws, q); }
+// v + e * (2^64 - q) for a quotient e of 32 bits
+__device__ __forceinline__ u64 sub_multiple(u64 v, u32 e, u64 q) {
+    const u64 nq = 0 - q, t = (u64)e * (u32)nq + v;
+    u32 top = (u32)(t >> 32) + e * (u32)(nq >> 32);
+    asm("" : "+v"(top));
     return ((u64)top << 32) | (u32)t;
 }
 // v < 32q (q < 2^59) to [0, q)

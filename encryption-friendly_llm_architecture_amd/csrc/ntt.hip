@@ -147,6 +147,17 @@ __device__ __forceinline__ void cols_body(const __amdgpu_buffer_rsrc_t limb, con
     }
 }
 
+template <class F, int LR, int P, int H, bool INV>
+__device__ __forceinline__ void cols_int(const __amdgpu_buffer_rsrc_t base, const Tw *__restrict__ tw, const ModQ *__restrict__ modq,
+                                         const u64 *__restrict__ ninv, const u64 *__restrict__ ninv_s, const double *__restrict__ fp,
+                                         const int prime, const Tw *__restrict__ final_scale, const int limb, u64 *lds) {
+    F f(modq, ninv, ninv_s, fp, prime);
+    if (INV && final_scale != nullptr) {
+        f.ni = final_scale[limb].w;
+        f.nis = final_scale[limb].ws;
+    }
+    cols_body<LR, P, H, INV>(base, tw, f, lds);
+}
 template <int LR, int P, int H, bool INV>
 __global__ __launch_bounds__((4096 >> H) / P) void ntt16_cols_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
                                                          const ModQ *__restrict__ modq,
@@ -168,15 +179,10 @@ __global__ __launch_bounds__((4096 >> H) / P) void ntt16_cols_kernel(u64 *__rest
             f.niinv = f.ni * f.qinv;
         }
         cols_body<LR, P, H, INV>(base, tw, f, lds);
-    } else if (INV || (modq[prime].q >> 60) != 0) {
-        IntField f(modq, ninv, ninv_s, fp, prime);
-        if (INV && final_scale != nullptr) {
-            f.ni = final_scale[limb].w;
-            f.nis = final_scale[limb].ws;
-        }
-        cols_body<LR, P, H, INV>(base, tw, f, lds);
+    } else if ((modq[prime].q >> 60) != 0) {
+        cols_int<IntField, LR, P, H, INV>(base, tw, modq, ninv, ninv_s, fp, prime, final_scale, limb, lds);
     } else {
-        cols_body<LR, P, H, INV>(base, tw, IntFieldT<true>(modq, ninv, ninv_s, fp, prime), lds);
+        cols_int<IntFieldT<true>, LR, P, H, INV>(base, tw, modq, ninv, ninv_s, fp, prime, final_scale, limb, lds);
     }
 }
 
@@ -491,7 +497,7 @@ __global__ __launch_bounds__(256) void ntt16_rows_kernel(u64 *__restrict__ data,
     if (fp[4 * prime] != 0.0)
         rows_body<P, INV, TAIL, LOAD, false>(row, tw, rtw, FpField(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld, gal,
                                             sec);
-    else if (INV || (modq[prime].q >> 60) != 0)
+    else if ((modq[prime].q >> 60) != 0)
         rows_body<P, INV, TAIL, LOAD, false>(row, tw, rtw, IntField(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld, gal,
                                             sec);
     else

@@ -193,6 +193,18 @@ __device__ __forceinline__ void limb_inverse(u64 *__restrict__ limb, const Tw *_
     for (int k = 0; k < P; k++) buf_store<u64>(to, S::voff(), S::off(k), f.scale_to_canonical(x[k]));
 }
 
+template <class F, int LR, int P, int LOAD>
+__device__ __forceinline__ void limb_inverse_int(u64 *__restrict__ base, const Tw *__restrict__ tw, const Tw *__restrict__ rtw,
+                                                 const ModQ *__restrict__ modq, const u64 *__restrict__ ninv, const u64 *__restrict__ ninv_s,
+                                                 const double *__restrict__ fp, const int prime, const Tw *__restrict__ final_scale,
+                                                 const int limb, u64 *lds, const u64 *__restrict__ ld, const u32 gal, const RowSecond &sec) {
+    F f(modq, ninv, ninv_s, fp, prime);
+    if (final_scale != nullptr) {
+        f.ni = final_scale[limb].w;
+        f.nis = final_scale[limb].ws;
+    }
+    limb_inverse<LR, P, LOAD>(base, tw, rtw, f, lds, ld, gal, sec);
+}
 template <int LR, int P, int LOAD>
 __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_inverse_kernel(
     u64 *__restrict__ data, const Tw *__restrict__ tw_all, const Tw *__restrict__ rtw_all, const ModQ *__restrict__ modq,
@@ -219,13 +231,10 @@ __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_inverse_kernel(
             f.niinv = f.ni * f.qinv;
         }
         limb_inverse<LR, P, LOAD>(base, tw, rtw, f, lds, ld, from.galois, sec);
+    } else if ((modq[prime].q >> 60) != 0) {
+        limb_inverse_int<IntField, LR, P, LOAD>(base, tw, rtw, modq, ninv, ninv_s, fp, prime, final_scale, limb, lds, ld, from.galois, sec);
     } else {
-        IntField f(modq, ninv, ninv_s, fp, prime);
-        if (final_scale != nullptr) {
-            f.ni = final_scale[limb].w;
-            f.nis = final_scale[limb].ws;
-        }
-        limb_inverse<LR, P, LOAD>(base, tw, rtw, f, lds, ld, from.galois, sec);
+        limb_inverse_int<IntFieldT<true>, LR, P, LOAD>(base, tw, rtw, modq, ninv, ninv_s, fp, prime, final_scale, limb, lds, ld, from.galois, sec);
     }
 }
 

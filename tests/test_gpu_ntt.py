@@ -74,6 +74,26 @@ def test_ntt_extreme_residues(log_n):
         assert np.array_equal(_to_host(d), want)
 
 
+@pytest.mark.parametrize("log_n", [10, 13, 15, 16])
+def test_ntt_quotients_from_the_high_word(log_n):
+    """The corrections that take a quotient from a value's high word, at both ends of the bit lengths they serve: primes just above
+    2^44 and 2^59 (a quotient constant of the most and of the fewest bits) and just below 2^45, 2^52 and 2^60."""
+    pkg = load_package()
+    step = 2 << log_n
+    above = lambda b: next(p for p in range(2**b + 1, 2**b + 4000 * step, step) if O.is_prime(p))
+    qs = [above(44), above(59)] + [O.primes_below(b, log_n, 1)[0] for b in (45, 52, 60)]
+    assert qs[0] > 2**44 and qs[1] > 2**59 and qs[-1] < 2**60
+    ctx, orc = pkg.Context(log_n, qs, [], 1), O.Oracle(log_n, qs, [], 1)
+    rng, N = np.random.default_rng(log_n), 1 << log_n
+    a = np.array([[np.full(N, q - 1, dtype=np.uint64) for q in qs], [rng.integers(0, q, N, dtype=np.uint64) for q in qs]])
+    idx = list(range(len(qs)))
+    for inverse in (False, True):
+        d, want = _to_dev(a.copy()), a.copy()
+        ctx.ntt(d, idx, inverse=inverse)
+        orc.ntt(want, idx, inverse=inverse)
+        assert np.array_equal(_to_host(d), want)
+
+
 def test_ntt_config2_roundtrip_full_batch():
     """32 polys x 24 limbs x 2^16 with the 24 largest 60-bit NTT primes: bit-exact round trip on
     the whole batch, forward output of every polynomial checked against the oracle."""
