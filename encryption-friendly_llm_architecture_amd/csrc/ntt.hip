@@ -8,8 +8,8 @@
 // points, 512 KiB, does not fit a CU's LDS, and a smaller one spread over R / 16 workgroups keeps more CUs busy):
 //   forward pass 1: stages 0 .. log2 R - 1  act down columns  (butterfly distance >= 256)
 //   forward pass 2: the last eight stages   act inside rows   (distance <= 128)
-// and mirrored for the inverse.  Each workgroup owns 4096 points, R rows of 4096 / R columns (or 16 rows, 8 with eight points
-// per thread); a thread keeps 16 residues in registers, or two lanes of a wavefront 8 each, runs a block of up to four
+// and mirrored for the inverse.  Each workgroup owns 4096 points, R rows of 4096 / R columns (or 16 rows, 8 or 4 with eight or four
+// points per thread); a thread keeps 16 residues in registers, or two or four lanes of a wavefront 8 or 4 each, runs a block of up to four
 // stages on them, swaps through LDS once and runs the second block.  All global accesses
 // are segments of at least 128 bytes shared by adjacent lanes.
 //
@@ -89,6 +89,8 @@ struct Slab {
     // conflicts: 9.7 against 8.8 us for 10 limbs of 42-bit primes)
     template <bool INV>
     static __device__ __forceinline__ int at(const int r) {
+        if (P == 4)   // its lanes 16 apart hold rows a whole or the fourth part of a block apart, in both passes: one bit of either goes in
+            return (r ^ (((LR >= 7 ? 0 : r >> 2) ^ (r >> (LR - 2))) & 1)) * CW + (int)cc();
         return (CW == 16 && !INV ? swz_row(r) : r) * CW + (int)cc();
     }
     // rows of a thread's register k: of the four widest stages (split, whole), of the others (split, whole)
@@ -189,12 +191,12 @@ __global__ __launch_bounds__((4096 >> H) / P) void ntt16_cols_kernel(u64 *__rest
 // Forward pass 1 over a slab whose input is a basis conversion computed on the fly.  The workgroups
 // of the target limbs that share a (polynomial, slab) pair have consecutive blockIdx.y and the same blockIdx.x, so
 // they sit on one XCD at about the same time and all but the first find the source slabs in its L2.
-template <int LR, int H, int NS, class F>
+template <int LR, int P, int H, int NS, class F>
 __device__ __forceinline__ void cols_converted_body(const __amdgpu_buffer_rsrc_t limb, const Tw *__restrict__ tw_int,
                                                     const F f, u64 *lds_raw, const __amdgpu_buffer_rsrc_t src,
                                                     const u32 (&so)[NS], const DotCst (&h)[NS], const int n_src, const ModQ m) {
-    typedef Slab<LR, 8, H> S;
-    typename F::E x[8];
+    typedef Slab<LR, P, H> S;
+    typename F::E x[P];
     // the row step goes into the scalar offset
     converted_inputs<NS>(f, x, src, S::v_outer(), so, h, n_src, m, [](const int k) { return S::outer(k); });
     cols_forward<LR, H>(limb, (const typename F::W *)tw_int, f, x, (typename F::E *)lds_raw);
@@ -205,30 +207,30 @@ __device__ __forceinline__ void cols_converted_body(const __amdgpu_buffer_rsrc_t
 // workgroups (16 polynomials x 6 limbs, 5 sources) 42 -> 37 us alone, 1002 -> 789 vector instructions per wave, with sums that carry
 // nothing (modarith.h, DotCst) and loads that wait once; rotation at 24 primes of 60 bits, level 20 161 -> 154 us, projection of a
 // 768-wide layer 2.5 % less.
-template <int LR, int H, int NS>
-__global__ __launch_bounds__(512 >> H) __attribute__((amdgpu_waves_per_eu(6, 6))) void ntt16_cols_converted_kernel(
+template <int LR, int P, int H, int NS>
+__global__ __launch_bounds__((4096 >> H) / P) __attribute__((amdgpu_waves_per_eu(P == 4 ? 4 : 6, P == 4 ? 8 : 6))) void ntt16_cols_converted_kernel(
     u64 *__restrict__ data, const Tw *__restrict__ tw_all, const ModQ *__restrict__ modq, const u64 *__restrict__ ninv,
     const u64 *__restrict__ ninv_s, const double *__restrict__ fp, LimbList ll, LimbList sl, int n_limbs,
     size_t poly_stride, ConvSources cs) {
     __shared__ u64 lds[4096 >> H];
     const int per_poly = n_limbs + cs.n_copy;
     const int limb = blockIdx.y % per_poly, poly = blockIdx.y / per_poly;
-    typedef Slab<LR, 8, H> S;
+    typedef Slab<LR, P, H> S;
     if (limb >= n_limbs) {   // a limb that is only copied into its slot
         const u64 *from = cs.copy_src + (size_t)poly * cs.copy_src_stride +
                           ((size_t)table_byte(cs.copy_src_slot, limb - n_limbs) << (8 + LR));
         u64 *base = data + (size_t)poly * poly_stride + ((size_t)table_byte(cs.copy_dst_slot, limb - n_limbs) << (8 + LR)) + S::col();
-        u64 t[8];
+        u64 t[P];
         if (cs.copy_galois != 0) {   // the copy of the source's automorphism
 #pragma unroll
-            for (int k = 0; k < 8; k++)
+            for (int k = 0; k < P; k++)
                 t[k] = from[galois_index(((u32)S::r_outer_w(k) << 8) + S::col(), cs.copy_galois, 8 + LR)];
         } else {
 #pragma unroll
-            for (int k = 0; k < 8; k++) t[k] = from[((u32)S::r_outer_w(k) << 8) + S::col()];
+            for (int k = 0; k < P; k++) t[k] = from[((u32)S::r_outer_w(k) << 8) + S::col()];
         }
 #pragma unroll
-        for (int k = 0; k < 8; k++) base[(u32)S::r_outer_w(k) << 8] = t[k];
+        for (int k = 0; k < P; k++) base[(u32)S::r_outer_w(k) << 8] = t[k];
         return;
     }
     const __amdgpu_buffer_rsrc_t base = limb_rsrc(
@@ -252,24 +254,24 @@ __global__ __launch_bounds__(512 >> H) __attribute__((amdgpu_waves_per_eu(6, 6))
         h[i] = dot_cst(hg.w, hg.ws);
     }
     if (fp[4 * prime] != 0.0)
-        cols_converted_body<LR, H, NS>(base, tw, FpField(modq, ninv, ninv_s, fp, prime), lds, src, so, h, n_src, m);
+        cols_converted_body<LR, P, H, NS>(base, tw, FpField(modq, ninv, ninv_s, fp, prime), lds, src, so, h, n_src, m);
     else   // (the sums take primes below 2^60)
-        cols_converted_body<LR, H, NS>(base, tw, IntFieldT<true>(modq, ninv, ninv_s, fp, prime), lds, src, so, h, n_src, m);
+        cols_converted_body<LR, P, H, NS>(base, tw, IntFieldT<true>(modq, ninv, ninv_s, fp, prime), lds, src, so, h, n_src, m);
 }
 
 // Forward pass 1 whose input is the rounded coefficients of an encoding, the same for every limb of a polynomial: reduced
 // as they are loaded instead of being written limb by limb and read back.
-template <int LR, int H, class F>
+template <int LR, int P, int H, class F>
 __device__ __forceinline__ void cols_lifted_body(const __amdgpu_buffer_rsrc_t limb, const Tw *__restrict__ tw_int, const F f,
                                                  u64 *lds_raw, const LiftSource &ls, const long long *__restrict__ coef,
                                                  const ModQ m) {
-    typedef Slab<LR, 8, H> S;
-    typename F::E x[8];
+    typedef Slab<LR, P, H> S;
+    typename F::E x[P];
     lifted_inputs(f, x, ls, coef, m, [](const int k) { return ((u32)S::r_outer_s(k) << 8) + S::col(); });
     cols_forward<LR, H>(limb, (const typename F::W *)tw_int, f, x, (typename F::E *)lds_raw);
 }
-template <int LR, int H>
-__global__ __launch_bounds__(512 >> H) void ntt16_cols_lifted_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
+template <int LR, int P, int H>
+__global__ __launch_bounds__((4096 >> H) / P) void ntt16_cols_lifted_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
                                                                 const ModQ *__restrict__ modq, const double *__restrict__ fp,
                                                                 LimbList ll, LimbList sl, int n_limbs, size_t poly_stride,
                                                                 LiftSource ls) {
@@ -282,11 +284,11 @@ __global__ __launch_bounds__(512 >> H) void ntt16_cols_lifted_kernel(u64 *__rest
     const long long *coef = ls.coef + (size_t)poly * ls.stride;
     const ModQ m = modq[prime];
     if (fp[4 * prime] != 0.0)
-        cols_lifted_body<LR, H>(base, tw, FpField(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
+        cols_lifted_body<LR, P, H>(base, tw, FpField(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
     else if ((m.q >> 60) != 0)
-        cols_lifted_body<LR, H>(base, tw, IntField(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
+        cols_lifted_body<LR, P, H>(base, tw, IntField(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
     else
-        cols_lifted_body<LR, H>(base, tw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
+        cols_lifted_body<LR, P, H>(base, tw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -445,7 +447,7 @@ __global__ __launch_bounds__(256) void ntt16_rows_kernel(u64 *__restrict__ data,
                                                          LimbList ll, LimbList sl, int n_limbs, size_t poly_stride,
                                                          typename EpilogueOf<KTAIL>::T ep, const int log_r_arg) {
     constexpr int TAIL = tail_of(KTAIL);
-    constexpr int RB = P == 16 ? 4 : 3;   // log2 of the rows of a workgroup
+    constexpr int RB = P == 16 ? 4 : P == 8 ? 3 : 2;   // log2 of the rows of a workgroup
     __shared__ u64 lds[ROWPAD << RB];
     const int log_r = LR != 0 ? LR : log_r_arg;
     // The second radix-16 block of a row pass walks 1/16 of the prime's twiddle table per 16-row slab (as
@@ -515,27 +517,31 @@ void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, c
                          size_t poly_stride, hipStream_t s, const void *final_scale, const NttEpilogue &from, int load);
 
 // ---- launches of single passes (rings of 2^13 points and more) -------------------------------------------------------
-// Which passes give a thread eight points instead of sixteen (ntt_device.h, Lanes).  Passes that begin in a basis conversion
-// or a lift, and inverse row passes, always do: they fit four waves per SIMD instead of three resp. eight instead of four.
-// The others only where the launch leaves the chip part empty, since in a full one the second twiddle and address of each
-// pair of lanes is work for nothing.  Transforms of 2^16 points, us with sixteen / with eight in that pass (workgroups of 4096
-// points); both arithmetics are level between 400 and 1500 workgroups, the lines lie where rows with 87 registers are all resident:
-//   workgroups                  64        256        384        640        768       1024       3072
-//   columns, forward, 60 bits   12.7/11.8  19.6/19.4  26.2/26.3  28.7/29.2  31.8/31.8  38.3/38.0  90.3/93.8
-//                     42 bits    9.6/ 9.4  16.5/16.2  21.6/21.5  23.4/23.6  23.3/22.9  27.3/27.0  70.1/68.4
-//            inverse, 60 bits   13.1/12.3  20.2/19.2  28.0/27.3  31.8/30.7  32.6/31.9  39.5/39.1  92.9/95.4
-//                     42 bits    9.7/ 9.5  16.5/16.1  22.1/21.9  24.0/24.0  23.8/23.7  27.4/28.3  68.2/66.7
-//   forward rows,     60 bits   13.4/11.7  19.6/18.7  26.5/25.4  29.8/27.5  30.0/29.2  35.8/35.4  88.6/91.3
-//                     42 bits   10.1/ 9.4  17.3/15.9  21.9/21.1  23.6/22.6  22.5/23.1  26.2/27.1  68.4/67.3
-//   in a rescale (the fused tail: 110 registers, four waves, with sixteen points, 87 and five with eight; whole rescale)
-//                     60 bits   27.6/25.1  33.6/32.5  42.6/40.7  53.0/50.2  53.7/53.9  61.6/62.6
-//                     42 bits   20.0/18.7  24.8/24.5  31.5/30.4  41.1/37.5  42.5/40.4  46.6/46.2
-// Together, with the conversions: rotation at 24 primes of 60 bits, level 20: 172 -> 162 us, level 7: 100 -> 81; product at level 9
-// 153 -> 134; rotation at N = 2^13 66 -> 53.
+// Which passes give a thread four or eight points instead of sixteen (ntt_device.h, Lanes): few points only where the launch leaves the
+// chip part empty, since in a full one the twiddles and addresses of each lane of a block are work for nothing.  Transforms of
+// 2^16 points, us with sixteen / eight / four points in that pass (workgroups of 4096 points):
+//   workgroups                  64              128        256              384              512              768             1024
+//   columns, forward, 60 bits   12.7/12.1/12.0  13.7/13.1  19.6/18.5/18.1   26.2/24.9/24.3   27.5/26.5/26.0   28.6/28.9/28.3  33.9/34.8/35.0
+//                     42 bits    9.6/10.3/10.8  11.9/12.2  16.5/16.4/16.0   21.6/21.7/21.4   24.4/24.3/23.9   22.6/23.1/23.5  26.9/27.4/28.5
+//            inverse, 60 bits   13.1/12.6/12.2  14.0/13.9  20.2/19.1/18.4   28.0/25.8/25.6   29.1/28.5/28.7   31.6/31.9/31.5  38.8/39.1/39.2
+//                     42 bits    9.7/10.7/11.0  11.8/12.1  16.5/16.6/16.4   22.1/21.9/22.1   25.5/25.4/25.4   24.0/24.2/25.0  27.5/28.4/30.4
+//   rows, forward,    60 bits   13.4/12.1/11.0  13.7/13.1  19.6/18.5/17.9   26.5/24.9/24.4   27.8/26.5/25.9   28.6/28.4/27.8  33.9/34.1/34.3
+//                     42 bits   10.1/10.3/10.3  11.9/11.9  17.3/16.4/16.2   21.9/21.7/21.1   24.6/24.3/23.9   22.6/23.1/22.8  26.9/27.8/27.1
+//         inverse,    60 bits       12.6/11.6   14.0/13.4       19.1/18.6        25.8/25.5        28.5/28.1        31.6/30.8       38.8/37.6
+//                     42 bits       10.7/10.1   11.8/12.1       16.6/16.4        21.9/21.7        25.4/24.8        24.0/23.8       27.5/27.9
+//         inverse, 2^15 points, 42  10.2/10.4   11.7/11.9       16.6/16.6        21.4/21.3        26.0/25.2        23.3/23.9       26.7/28.2
+// With the conversions (below): rotation on 2^13 points 34.1 -> 30.2 us, inverse transform of 35 limbs of 2^14 points 12.9 -> 12.2, product at
+// level 9 109.6 -> 106.1; the products of 128 x 128 matrices the same to 1 %.
 static bool few_for_columns(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 512; }
 static bool few_for_rows(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 640; }
 
-// Column passes of few workgroups are bound by the instructions of the few CUs they are on, two wavefronts per SIMD: slabs of a half or a
+// Passes that begin in a basis conversion or a lift: four points where every CU has one workgroup at most, eight otherwise (six waves per
+// SIMD).  Rotations with four points up to 0 / 256 / 400 / 1024 workgroups in a launch of conversions, us: 2^16 points, 42 bits, level 4 (160 and
+// fewer) 55.9/54.8/55.0/55.1, level 6 (224) 63.4/62.2/62.2/61.9, level 9 (288) 72.0/72.1/73.6/73.5; 60 bits, level 5 (192) 60.3/58.8/58.8/58.7, level 10 (384)
+// 83.7/83.2/82.8/82.6, level 15 (512) 93.8/94.0/96.2/97.1, level 20 (864) 128.2/127.7/128.0/136.0; 2^14 points, level 6 (48) 42.2/39.9/40.6/41.0.
+static bool few_for_conversions(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 256; }
+
+// Column passes of few workgroups are bound by the instructions of the few CUs they are on: slabs of a half or a
 // quarter of the columns (1, 2: as powers of two) put them on as many more CUs.  Not below 16 columns, segments of 128 bytes: at 2^16 points,
 // half slabs take a rotation on 60-bit primes from 129.8 to 133.7 us where up to 512 workgroups have them, to 131.1 where up to 128 do.
 // Transforms (forward/inverse, us) with whole / with narrower slabs:
@@ -562,8 +568,8 @@ static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
                        c->d_ninv_s, c->d_fp, ll, sl, n_limbs, poly_stride, (const Tw *)(INV ? final_scale : nullptr))
 #define COLS_SLAB(LR, INV)                          \
     do {                                            \
-        if (narrow == 1) COLS_FORM(LR, 8, 1, INV);  \
-        else if (few) COLS_FORM(LR, 8, 0, INV);     \
+        if (narrow == 1) COLS_FORM(LR, 4, 1, INV);  \
+        else if (few) COLS_FORM(LR, 4, 0, INV);     \
         else COLS_FORM(LR, 16, 0, INV);             \
     } while (0)
 #define COLS(LR)                                    \
@@ -573,8 +579,8 @@ static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
     } while (0)
 #define COLS_SMALL(LR)                                      \
     do {                                                    \
-        if (narrow == 2 && inverse) COLS_FORM(LR, 8, 2, true); \
-        else if (narrow == 2) COLS_FORM(LR, 8, 2, false);   \
+        if (narrow == 2 && inverse) COLS_FORM(LR, 4, 2, true); \
+        else if (narrow == 2) COLS_FORM(LR, 4, 2, false);   \
         else COLS(LR);                                      \
     } while (0)
     switch (c->logN) {
@@ -582,9 +588,9 @@ static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
         case 14: COLS_SMALL(6); break;
         case 15: COLS(7); break;
         default:
-            if (inverse && few) COLS_FORM(8, 8, 0, true);
+            if (inverse && few) COLS_FORM(8, 4, 0, true);
             else if (inverse) COLS_FORM(8, 16, 0, true);
-            else if (few) COLS_FORM(8, 8, 0, false);
+            else if (few) COLS_FORM(8, 4, 0, false);
             else COLS_FORM(8, 16, 0, false);
     }
 #undef COLS_SMALL
@@ -595,8 +601,8 @@ static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
 static void rows_pass(const hemm_context *c, bool inverse, u64 *d, const LimbList &ll, const LimbList &sl, int n_limbs,
                       int n_polys, size_t poly_stride, hipStream_t s, const NttEpilogue &ep, int tail = TAIL_NONE,
                       int load = LOAD_PLAIN, const ResultList *list = nullptr, int first = 0) {
-    const bool few = inverse || few_for_rows(c, n_limbs * n_polys);
-    const dim3 grid((unsigned)(c->N >> (few ? 11 : 12)) * (unsigned)(n_limbs * n_polys)), block(256);
+    const bool few = few_for_rows(c, n_limbs * n_polys);
+    const dim3 grid((unsigned)(c->N >> (few ? 10 : inverse ? 11 : 12)) * (unsigned)(n_limbs * n_polys)), block(256);
     const int log_r = c->logN - 8;
 #define ROWS(LR, P, INV, TAIL, LOAD, EP)                                                                                      \
     hipLaunchKernelGGL((ntt16_rows_kernel<LR, P, INV, TAIL, LOAD>), grid, block, 0, s, d, (const Tw *)(INV ? c->d_iw : c->d_w), \
@@ -606,17 +612,22 @@ static void rows_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
         if (log_r == 8) ROWS(8, P, INV, TAIL, LOAD, EP);   \
         else ROWS(0, P, INV, TAIL, LOAD, EP);              \
     } while (0)
+#define ROWS_INVERSE(LOAD)                                       \
+    do {                                                         \
+        if (few) ROWS_RING(4, true, TAIL_NONE, LOAD, ep);        \
+        else ROWS_RING(8, true, TAIL_NONE, LOAD, ep);            \
+    } while (0)
 #define ROWS_FORWARD(TAIL, EP)                                   \
     do {                                                         \
-        if (few) ROWS_RING(8, false, TAIL, LOAD_PLAIN, EP);      \
+        if (few) ROWS_RING(4, false, TAIL, LOAD_PLAIN, EP);      \
         else ROWS_RING(16, false, TAIL, LOAD_PLAIN, EP);         \
     } while (0)
     if (inverse && load == LOAD_ROTATED)
-        ROWS_RING(8, true, TAIL_NONE, LOAD_ROTATED, ep);
+        ROWS_INVERSE(LOAD_ROTATED);
     else if (inverse && load == LOAD_DECRYPT)
-        ROWS_RING(8, true, TAIL_NONE, LOAD_DECRYPT, ep);
+        ROWS_INVERSE(LOAD_DECRYPT);
     else if (inverse)
-        ROWS_RING(8, true, TAIL_NONE, LOAD_PLAIN, ep);
+        ROWS_INVERSE(LOAD_PLAIN);
     else if (tail == TAIL_SUB_SCALE && list != nullptr) {
         const NttEpilogueList epl{ep, (u32)first, *list};
         ROWS_FORWARD(TAIL_SUB_SCALE_LIST, epl);
@@ -627,6 +638,7 @@ static void rows_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
     else
         ROWS_FORWARD(TAIL_NONE, ep);
 #undef ROWS_FORWARD
+#undef ROWS_INVERSE
 #undef ROWS_RING
 #undef ROWS
 }
@@ -730,8 +742,14 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
     }
     const int narrow = narrower_slabs(c, (n_limbs + cs.n_copy) * n_polys);
     const dim3 grid((unsigned)(c->N >> (12 - narrow)), (n_limbs + cs.n_copy) * n_polys);
-#define CONV_FORM(LR, H, K)                                                                                                  \
-    hipLaunchKernelGGL((ntt16_cols_converted_kernel<LR, H, K>), grid, dim3(512 >> H), 0, s, data, (const Tw *)c->d_w, c->d_modq, \
+    const bool few = few_for_conversions(c, (n_limbs + cs.n_copy) * n_polys);
+#define CONV_FORM(LR, H, K)                       \
+    do {                                          \
+        if (few) CONV_POINTS(LR, 4, H, K);       \
+        else CONV_POINTS(LR, 8, H, K);            \
+    } while (0)
+#define CONV_POINTS(LR, P, H, K)                                                                                             \
+    hipLaunchKernelGGL((ntt16_cols_converted_kernel<LR, P, H, K>), grid, dim3((4096 >> H) / P), 0, s, data, (const Tw *)c->d_w, c->d_modq, \
                        c->d_ninv, c->d_ninv_s, c->d_fp, ll, sl, n_limbs, poly_stride, cs)
 #define CONV_RING(LR, H)                        \
     do {                                        \
@@ -759,6 +777,7 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
 #undef CONV_SLAB
 #undef CONV_RING
 #undef CONV_FORM
+#undef CONV_POINTS
     if (cols_only) return true;
     rows_pass(c, false, data, ll, sl, n_limbs, n_polys, poly_stride, s,
               sub_scale_tail(ep_minuend, ep_minuend_stride, ep_out, ep_out_stride, ep_cst_dev), tail ? TAIL_SUB_SCALE : TAIL_NONE,
@@ -889,8 +908,14 @@ bool launch_ntt_lifted(const hemm_context *c, const LiftSource &ls, u64 *data, c
         l.coef += (size_t)p0 * ls.stride;
         const bool half = narrower_slabs(c, n_limbs * np) != 0;
         const dim3 grid((unsigned)(c->N >> (half ? 11 : 12)), (unsigned)(n_limbs * np));
-#define LIFTED_FORM(LR, H)                                                                                                     \
-    hipLaunchKernelGGL((ntt16_cols_lifted_kernel<LR, H>), grid, dim3(512 >> H), 0, s, d, (const Tw *)c->d_w, c->d_modq, c->d_fp, ll, sl, \
+        const bool few = few_for_conversions(c, n_limbs * np);
+#define LIFTED_FORM(LR, H)                    \
+    do {                                      \
+        if (few) LIFTED_POINTS(LR, 4, H);     \
+        else LIFTED_POINTS(LR, 8, H);         \
+    } while (0)
+#define LIFTED_POINTS(LR, P, H)                                                                                                     \
+    hipLaunchKernelGGL((ntt16_cols_lifted_kernel<LR, P, H>), grid, dim3((4096 >> H) / P), 0, s, d, (const Tw *)c->d_w, c->d_modq, c->d_fp, ll, sl, \
                        n_limbs, poly_stride, l)
 #define LIFTED(LR)                    \
     do {                              \
@@ -905,6 +930,7 @@ bool launch_ntt_lifted(const hemm_context *c, const LiftSource &ls, u64 *data, c
         }
 #undef LIFTED
 #undef LIFTED_FORM
+#undef LIFTED_POINTS
         rows_pass(c, false, d, ll, sl, n_limbs, np, poly_stride, s, ep, tail);
         if (enc != nullptr) {
             ep.out += (size_t)np * poly_stride;

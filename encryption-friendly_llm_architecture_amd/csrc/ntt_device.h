@@ -222,12 +222,14 @@ struct FpField {
     // largest value it multiplies is 2^T B.  With element 0 of every sub-block (and element 1 where T = 4) reduced after
     // each block every block starts from B <= 4 r: r <= 0.8 q gives B <= 3.2 q and 16 B <= 51 q < 2^49.7 (q < 2^44), for
     // which r <= 0.8 q holds again; products of values below 2^50 are still exact.
-    // (Eight registers per thread: the upper half of a block of four stages has its elements 4 and 5 reduced as well.)
+    // (Eight registers per thread: the upper half of a block of four stages has its elements 4 and 5 reduced as well.  Four: register 0
+    // of a block of four stages holds its elements 0 .. 3, registers 0 and 2 of two sub-blocks of three theirs.)
     template <int T, int P>
     __device__ __forceinline__ void after_inverse_block(E (&x)[P]) const {
+        constexpr int step = P == 4 ? (T == 4 || T == 2 ? 4 : 2) : 1 << T;
 #pragma unroll
-        for (int k = 0; k < P; k += 1 << T) x[k] = reduce(x[k]);
-        if (T == 4) x[1] = reduce(x[1]);
+        for (int k = 0; k < P; k += step) x[k] = reduce(x[k]);
+        if (T == 4 && P > 4) x[1] = reduce(x[1]);
     }
     __device__ __forceinline__ u64 centred_to_canonical(E r) const {
         r += r < 0.0 ? q : 0.0;
@@ -251,46 +253,70 @@ struct FpField {
 };
 
 // How a block of up to four stages on 16 points lies in registers.  P = 16: one thread holds the block.  P = 8: two lanes of a
-// wavefront 32 apart hold eight points each, h = 0 and 1; the threads that share a block are otherwise numbered as with
-// P = 16 (t).  Two layouts: `whole`, lane h holds points 8h .. 8h + 7, in which every stage of a distance below 8 is local,
-// and `split`, lane h holds points 4h .. 4h + 3 and 8 + 4h .. 8 + 4h + 3, in which the stage of distance 8 is; one
-// v_permlane32_swap_b32 per register pair turns one into the other.  T < 4 stages only ever use `whole`.
+// wavefront 32 apart hold eight points each, h = 0 and 1; P = 4: four lanes 16 apart hold four each, h = 0 .. 3; the threads that
+// share a block are otherwise numbered as with P = 16 (t).  Two layouts: `whole`, lane h holds points P h .. P h + P - 1, in which every
+// stage of a distance below P is local, and `split`, in which the wider ones are: with P = 8 lane h holds points 4h .. 4h + 3 and
+// 8 + 4h .. 8 + 4h + 3, with P = 4 points h, h + 4, h + 8 and h + 12.  v_permlane32_swap_b32 and, P = 4, v_permlane16_swap_b32 between
+// registers turn one into the other.  Blocks without a wide stage only ever use `whole`.
 // A thread of 16 points is one wavefront per SIMD in a launch of up to 256 workgroups, and then its load latencies and the
-// dependences of 64-bit products are what the launch takes; eight points per thread put two wavefronts there with half
-// the instructions each.  The arithmetic of every point, and with it the residues, is the same.
+// dependences of 64-bit products are what the launch takes; eight and four points per thread put two and four wavefronts there with a half
+// and a quarter of the instructions each.  The arithmetic of every point, and with it the residues, is the same.
 template <int P>
 struct Lanes {
-    static __device__ __forceinline__ u32 t() { return P == 16 ? threadIdx.x : (threadIdx.x & 31u) | ((threadIdx.x >> 6) << 5); }
-    static __device__ __forceinline__ u32 h() { return P == 16 ? 0u : (threadIdx.x >> 5) & 1u; }
+    static constexpr int SHARE = 64 * P / 16;   // lanes of a wavefront with blocks of their own
+    static __device__ __forceinline__ u32 t() { return P == 16 ? threadIdx.x : (threadIdx.x & (SHARE - 1u)) | ((threadIdx.x >> 6) * SHARE); }
+    static __device__ __forceinline__ u32 h() { return P == 16 ? 0u : (threadIdx.x & 63u) / SHARE; }
+    template <int T>
+    static __device__ __forceinline__ constexpr bool wide() { return (1 << T) > P; }   // whether T stages begin in `split`
     // point of register k: a constant and the lane's part
     template <int T>
-    static __device__ __forceinline__ constexpr int split(const int k) { return P == 16 || T < 4 ? k : (k & 3) + 8 * (k >> 2); }
+    static __device__ __forceinline__ constexpr int split(const int k) { return !wide<T>() ? k : P == 4 ? 4 * k : (k & 3) + 8 * (k >> 2); }
     template <int T>
-    static __device__ __forceinline__ u32 h_split() { return (P == 16 || T < 4 ? 8u : 4u) * h(); }
-    static __device__ __forceinline__ u32 h_whole() { return 8u * h(); }
+    static __device__ __forceinline__ u32 h_split() { return !wide<T>() ? P * h() : P == 4 ? h() : 4u * h(); }
+    static __device__ __forceinline__ u32 h_whole() { return P * h(); }
 };
-// split <-> whole
-__device__ __forceinline__ void swap_halves(u64 &a, u64 &b) {
-    const u32x2 lo = __builtin_amdgcn_permlane32_swap((u32)a, (u32)b, false, false);
-    const u32x2 hi = __builtin_amdgcn_permlane32_swap((u32)(a >> 32), (u32)(b >> 32), false, false);
+// split <-> whole: register k and lane h change places
+template <int DISTANCE>
+__device__ __forceinline__ void swap_lanes(u64 &a, u64 &b) {
+    const u32x2 lo = DISTANCE == 32 ? __builtin_amdgcn_permlane32_swap((u32)a, (u32)b, false, false)
+                                    : __builtin_amdgcn_permlane16_swap((u32)a, (u32)b, false, false);
+    const u32x2 hi = DISTANCE == 32 ? __builtin_amdgcn_permlane32_swap((u32)(a >> 32), (u32)(b >> 32), false, false)
+                                    : __builtin_amdgcn_permlane16_swap((u32)(a >> 32), (u32)(b >> 32), false, false);
     a = ((u64)hi.x << 32) | lo.x;
     b = ((u64)hi.y << 32) | lo.y;
+}
+template <int DISTANCE, class E>
+__device__ __forceinline__ void swap_values(E &x, E &y) {
+    u64 a, b;
+    __builtin_memcpy(&a, &x, 8);
+    __builtin_memcpy(&b, &y, 8);
+    swap_lanes<DISTANCE>(a, b);
+    __builtin_memcpy(&x, &a, 8);
+    __builtin_memcpy(&y, &b, 8);
+}
+template <class E>
+__device__ __forceinline__ void swap_layout(E (&x)[4]) {
+    swap_values<32>(x[0], x[2]);
+    swap_values<32>(x[1], x[3]);
+    swap_values<16>(x[0], x[1]);
+    swap_values<16>(x[2], x[3]);
 }
 template <class E>
 __device__ __forceinline__ void swap_layout(E (&x)[8]) {
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-        u64 a, b;
-        __builtin_memcpy(&a, &x[k], 8);
-        __builtin_memcpy(&b, &x[k + 4], 8);
-        swap_halves(a, b);
-        __builtin_memcpy(&x[k], &a, 8);
-        __builtin_memcpy(&x[k + 4], &b, 8);
-    }
+    for (int k = 0; k < 4; k++) swap_values<32>(x[k], x[k + 4]);
 }
 template <class E>
 __device__ __forceinline__ void swap_layout(E (&)[16]) {}
 
+// The pairs of a stage of distance d in a lane's registers: blocks of 2 dist, one twiddle group each, the first number first_group
+template <int P>
+struct StagePairs {
+    int dist;            // of a pair's registers
+    u32 first_group;
+    __device__ __forceinline__ constexpr StagePairs(const int d, const bool split, const u32 h)
+        : dist(!split ? d : P == 4 ? d / 4 : 4), first_group(!split ? h * (u32)(P / 2 / d) : 0u) {}
+};
 // T Cooley-Tukey stages on 16 points that are 16 >> T sub-blocks of 2^T consecutive ones; stage s, group g uses twiddle
 // tw(s, g).  Points come in as `split` and leave as `whole`.
 template <int T, int P, class F, class TW>
@@ -299,19 +325,15 @@ __device__ __forceinline__ void stages_fwd(const F &f, typename F::E (&x)[P], co
 #pragma unroll
     for (int s = 0; s < T; s++) {
         const int d = 1 << (T - 1 - s);
-        if (P == 8 && d == 8) {   // the first stage of four, in the split layout
-            const typename F::W w = tw(0, 0u);
+        const bool split = d >= P;
+        const StagePairs<P> p(d, split, h);
 #pragma unroll
-            for (int j = 0; j < 4; j++) f.ct(x[j], x[j + 4], w, false);
-            swap_layout(x);
-        } else {
+        for (int g = 0; g < P / 2 / p.dist; g++) {
+            const typename F::W w = tw(s, p.first_group + (u32)g);
 #pragma unroll
-            for (int g = 0; g < P / 2 / d; g++) {
-                const typename F::W w = tw(s, h * (u32)(8 / 2 / d) + (u32)g);
-#pragma unroll
-                for (int j = 0; j < d; j++) f.ct(x[g * 2 * d + j], x[g * 2 * d + j + d], w, (s & 1) != 0);
-            }
+            for (int j = 0; j < p.dist; j++) f.ct(x[g * 2 * p.dist + j], x[g * 2 * p.dist + j + p.dist], w, (s & 1) != 0);
         }
+        if (split && d / 2 < P) swap_layout(x);
     }
 }
 // T Gentleman-Sande stages, the other way round: `whole` in, `split` out; stage s has distance 1 << s.
@@ -321,18 +343,14 @@ __device__ __forceinline__ void stages_inv(const F &f, typename F::E (&x)[P], co
 #pragma unroll
     for (int s = 0; s < T; s++) {
         const int d = 1 << s;
-        if (P == 8 && d == 8) {
-            swap_layout(x);
-            const typename F::W w = tw(3, 0u);
+        const bool split = d >= P;
+        if (split && d / 2 < P) swap_layout(x);
+        const StagePairs<P> p(d, split, h);
 #pragma unroll
-            for (int j = 0; j < 4; j++) f.gs(x[j], x[j + 4], w, true, true);
-        } else {
+        for (int g = 0; g < P / 2 / p.dist; g++) {
+            const typename F::W w = tw(s, p.first_group + (u32)g);
 #pragma unroll
-            for (int g = 0; g < P / 2 / d; g++) {
-                const typename F::W w = tw(s, h * (u32)(8 / 2 / d) + (u32)g);
-#pragma unroll
-                for (int j = 0; j < d; j++) f.gs(x[g * 2 * d + j], x[g * 2 * d + j + d], w, (s & 1) != 0, s == T - 1);
-            }
+            for (int j = 0; j < p.dist; j++) f.gs(x[g * 2 * p.dist + j], x[g * 2 * p.dist + j + p.dist], w, (s & 1) != 0, s == T - 1);
         }
     }
 }
@@ -411,11 +429,11 @@ __device__ __forceinline__ void lifted_inputs(const F &f, typename F::E (&x)[P],
 // wait for the first of them instead of one per source limb behind a branch of its own.  More in flight cost wavefronts: ModDown
 // of 64 / 16 polynomials of 7 + 4 limbs 389 / 108 us with 20 residues and six waves per SIMD, 400 / 110 with 40 and four.
 #define CONV_LOADS 20
-template <int N_SRC, int NS, class F, class OFF>
-__device__ __forceinline__ void converted_exact(const F &f, typename F::E (&x)[8], const __amdgpu_buffer_rsrc_t src, const u32 voff,
+template <int N_SRC, int NS, int P, class F, class OFF>
+__device__ __forceinline__ void converted_exact(const F &f, typename F::E (&x)[P], const __amdgpu_buffer_rsrc_t src, const u32 voff,
                                                 const u32 (&so)[NS], const DotCst (&h)[NS], const ModQ m, const OFF off) {
-    constexpr int AHEAD = CONV_LOADS / N_SRC < 8 ? CONV_LOADS / N_SRC : 8;   // coefficients whose sources are in flight together
-    u32x2 v[8][N_SRC];
+    constexpr int AHEAD = CONV_LOADS / N_SRC < P ? CONV_LOADS / N_SRC : P;   // coefficients whose sources are in flight together
+    u32x2 v[P][N_SRC];
     auto load = [&](const int k) {
 #pragma unroll
         for (int i = 0; i < N_SRC; i++) v[k][i] = __builtin_amdgcn_raw_buffer_load_b64(src, voff, so[i] + off(k), 0);
@@ -423,17 +441,17 @@ __device__ __forceinline__ void converted_exact(const F &f, typename F::E (&x)[8
 #pragma unroll
     for (int k = 0; k < AHEAD; k++) load(k);
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
+    for (int k = 0; k < P; k++) {
         Dot2 d;
         dot_clear(d);
 #pragma unroll
         for (int i = 0; i < N_SRC; i++) dot_add(d, ((u64)v[k][i].y << 32) | v[k][i].x, h[i]);
-        if (k + AHEAD < 8) load(k + AHEAD);
+        if (k + AHEAD < P) load(k + AHEAD);
         x[k] = f.from_dot(d, m);
     }
 }
-template <int K, int NS, class F, class OFF>
-__device__ __forceinline__ void converted_inputs(const F &f, typename F::E (&x)[8], const __amdgpu_buffer_rsrc_t src,
+template <int K, int NS, int P, class F, class OFF>
+__device__ __forceinline__ void converted_inputs(const F &f, typename F::E (&x)[P], const __amdgpu_buffer_rsrc_t src,
                                                  const u32 voff, const u32 (&so)[NS], const DotCst (&h)[NS], const int n_src,
                                                  const ModQ m, const OFF off) {
     if constexpr (K > 1)
@@ -441,7 +459,7 @@ __device__ __forceinline__ void converted_inputs(const F &f, typename F::E (&x)[
     converted_exact<K>(f, x, src, voff, so, h, m, off);
 }
 
-// A row's 16 threads (32 with eight points each) sit in one wavefront, so the LDS exchanges of
+// A row's 16 threads (32 with eight points each, 64 with four) sit in one wavefront, so the LDS exchanges of
 // the row kernel never cross a wavefront: ordering them needs no workgroup barrier, only a fence that
 // keeps the compiler from moving LDS accesses across it.
 __device__ __forceinline__ void wave_sync() {
@@ -511,7 +529,7 @@ __device__ __forceinline__ void rows_body(u64 *__restrict__ row, const Tw *__res
             x[k] = IN_LDS ? l[padc(e)] : mem[e];
         }
         radix_fwd<4>(f, x, tw, (1u << log_r) + r);
-        if (IN_LDS && P == 8) wave_sync();   // both lanes of a pair have read before either writes
+        if (IN_LDS && P < 16) wave_sync();   // both lanes of a pair have read before either writes
 #pragma unroll
         for (int k = 0; k < P; k++) l[padc(cw + 16 * k)] = x[k];
         wave_sync();
@@ -573,7 +591,7 @@ __device__ __forceinline__ void rows_body(u64 *__restrict__ row, const Tw *__res
         for (int k = 0; k < P; k++) x[k] = l[padc(cw + 16 * k)];
         radix_inv<4>(f, x, tw, (1u << log_r) + r);
         f.template after_inverse_block<4>(x);
-        if (IN_LDS && P == 8) wave_sync();
+        if (IN_LDS && P < 16) wave_sync();
 #pragma unroll
         for (int k = 0; k < P; k++) {   // IN_LDS: the places this thread, or the other one of its pair, has just read
             const int e = cs + 16 * L::template split<4>(k);

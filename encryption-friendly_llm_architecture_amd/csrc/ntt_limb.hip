@@ -4,7 +4,7 @@
 // (R = N / 256) meet in LDS instead of in memory, and a transform that the two-launch kernels would take as two dependent
 // launches is one.  What bounds a call on the small rings is the number of dependent launches, a few microseconds each
 // however little they do, not arithmetic or bytes: one transform of 2^12 points 7 us against 36 us with the butterflies
-// of every stage read from and written to LDS one by one, which these kernels replace.  A thread holds eight residues (16 at 2^14 points, where
+// of every stage read from and written to LDS one by one, which these kernels replace.  A thread holds four or eight residues (16 at 2^14 points, where
 // eight would take 2048 threads; with eight a CU has two wavefronts per SIMD on a limb of 2^12 points instead of one: product
 // of two encrypted 32 x 32 tiles 687 -> 595 us): the log2 R
 // column stages in one block (R <= 16) or two, one exchange through LDS after each, then the row pass of the two-launch
@@ -238,8 +238,12 @@ __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_inverse_kernel(
     }
 }
 
-// points per thread
+// points per thread: of 2^12 points four where every CU has one limb at most (sixteen wavefronts on it; forward with a conversion 11.5 -> 10.6 us,
+// product of two encrypted 32 x 32 tiles 497 -> 486), eight in larger launches, whose second twiddle and address cost more than that
+// (transforms of 256 / 512 / 4096 limbs of 42 bits 6.9/10.5/61.6 us with four, 6.7/9.9/56.2 with eight)
 #define POINTS(LR) ((LR) <= 5 ? 8 : 16)
+#define POINTS_FEW(LR) ((LR) == 4 ? 4 : POINTS(LR))
+static bool few_limbs(const size_t limbs) { return limbs <= 256; }
 }  // namespace
 
 void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
@@ -257,10 +261,16 @@ void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, c
     if (ls != nullptr) lift = *ls;
     NttEpilogueList epl{ep, 0, {}};
     if (list != nullptr) epl.list = *list;
-    const dim3 grid((unsigned)((n_limbs + conv.n_copy) * n_polys)), block((unsigned)((256 / POINTS(LR)) << LR));
-#define LIMB_FORWARD(L, K, TAIL, EP)                                                                                       \
-    hipLaunchKernelGGL((ntt_limb_forward_kernel<L, POINTS(L), K, TAIL>), grid, block, 0, s, data, (const Tw *)c->d_w,                 \
+    const dim3 grid((unsigned)((n_limbs + conv.n_copy) * n_polys));
+    const bool few = few_limbs(grid.x);
+#define LIMB_FORWARD_POINTS(L, P, K, TAIL, EP)                                                                             \
+    hipLaunchKernelGGL((ntt_limb_forward_kernel<L, P, K, TAIL>), grid, dim3((256 / (P)) << (L)), 0, s, data, (const Tw *)c->d_w,       \
                        (const Tw *)c->d_rw, c->d_modq, c->d_fp, ll, sl, n_limbs, poly_stride, conv, lift, EP)
+#define LIMB_FORWARD(L, K, TAIL, EP)                                       \
+    do {                                                                   \
+        if (few) LIMB_FORWARD_POINTS(L, POINTS_FEW(L), K, TAIL, EP);       \
+        else LIMB_FORWARD_POINTS(L, POINTS(L), K, TAIL, EP);               \
+    } while (0)
 #define LIMB_SOURCES(L, TAIL, EP)                          \
     do {                                                   \
         if (widest == 0) LIMB_FORWARD(L, 0, TAIL, EP);     \
@@ -293,14 +303,21 @@ void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, c
 #undef LIMB_RING
 #undef LIMB_SOURCES
 #undef LIMB_FORWARD
+#undef LIMB_FORWARD_POINTS
 }
 
 void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, const LimbList &sl, int n_limbs, int n_polys,
                          size_t poly_stride, hipStream_t s, const void *final_scale, const NttEpilogue &from, int load) {
     const int LR = c->logN - 8;
-    const dim3 grid((unsigned)(n_limbs * n_polys)), block((unsigned)((256 / POINTS(LR)) << LR));
-#define LIMB_INVERSE(L, LOAD)                                                                                         \
-    hipLaunchKernelGGL((ntt_limb_inverse_kernel<L, POINTS(L), LOAD>), grid, block, 0, s, data, (const Tw *)c->d_iw,              \
+    const dim3 grid((unsigned)(n_limbs * n_polys));
+    const bool few = few_limbs(grid.x);
+#define LIMB_INVERSE(L, LOAD)                                              \
+    do {                                                                   \
+        if (few) LIMB_INVERSE_POINTS(L, POINTS_FEW(L), LOAD);              \
+        else LIMB_INVERSE_POINTS(L, POINTS(L), LOAD);                      \
+    } while (0)
+#define LIMB_INVERSE_POINTS(L, P, LOAD)                                                                               \
+    hipLaunchKernelGGL((ntt_limb_inverse_kernel<L, P, LOAD>), grid, dim3((256 / (P)) << (L)), 0, s, data, (const Tw *)c->d_iw,              \
                        (const Tw *)c->d_irw, c->d_modq, c->d_ninv, c->d_ninv_s, c->d_fp, ll, sl, n_limbs, poly_stride, \
                        (const Tw *)final_scale, from)
 #define LIMB_RING(L)                                                   \
@@ -322,4 +339,5 @@ void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, c
     }
 #undef LIMB_RING
 #undef LIMB_INVERSE
+#undef LIMB_INVERSE_POINTS
 }

@@ -1,0 +1,49 @@
+"""Passes of four, eight and sixteen points per thread: both sides of the lines between them, against the oracle."""
+import numpy as np
+import pytest
+
+from __graft_entry__ import load_package
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _context(log_n):
+    pkg = load_package()
+    mods = [O.primes_below(61, log_n, 1)[0], O.primes_below(60, log_n, 1)[0], O.primes_below(42, log_n, 1)[0]]
+    return pkg.Context(log_n, mods, [], 1), O.Oracle(log_n, mods, [], 1, threads=8), mods
+
+
+# limbs at which a pass changes: columns at 512 workgroups of 4096 points, rows at 640, one-launch transforms at 256 limbs
+@pytest.mark.parametrize("log_n,limbs", [(10, 2), (11, 2), (12, 1), (12, 256), (12, 257), (13, 1), (14, 81), (15, 64), (15, 65), (15, 80), (15, 81),
+                                         (16, 1), (16, 32), (16, 33), (16, 40), (16, 41)])
+def test_transforms(log_n, limbs):
+    import torch
+    ctx, orc, mods = _context(log_n)
+    rng = np.random.default_rng(limbs)
+    for prime, q in enumerate(mods):
+        a = rng.integers(0, q, (limbs, 1, 1 << log_n), dtype=np.uint64)
+        a[0] = q - 1
+        d = torch.from_numpy(a.view(np.int64)).cuda()
+        ctx.ntt(d, [prime])
+        got = d.cpu().numpy().view(np.uint64)
+        for p in {0, limbs // 2, limbs - 1}:
+            want = a[p].copy()
+            orc.ntt(want, [prime])
+            assert np.array_equal(got[p], want), (prime, p)
+        ctx.ntt(d, [prime], inverse=True)
+        assert np.array_equal(d.cpu().numpy().view(np.uint64), a), prime
+
+
+# conversions at 256 workgroups of 4096 points: a rescale of `polys` polynomials of nq limbs launches polys (nq - 1) limbs
+@pytest.mark.parametrize("log_n,polys,nq", [(11, 2, 4), (12, 2, 18), (13, 2, 4), (14, 4, 17), (14, 4, 18), (15, 2, 17), (15, 2, 18), (16, 2, 9), (16, 2, 10)])
+def test_conversions(log_n, polys, nq):
+    import torch
+    pkg = load_package()
+    mods = O.primes_below(60, log_n, 9) + O.primes_below(42, log_n, 9)
+    ctx, orc = pkg.Context(log_n, mods, [], 1), O.Oracle(log_n, mods, [], 1, threads=8)
+    rng = np.random.default_rng(polys)
+    a = np.stack([rng.integers(0, q, (polys, 1 << log_n), dtype=np.uint64) for q in mods[:nq]], axis=1)
+    a[0, -1] = mods[nq - 1] - 1
+    got = ctx.rescale(torch.from_numpy(a.view(np.int64)).cuda(), nq).cpu().numpy().view(np.uint64)
+    assert np.array_equal(got, orc.rescale(O.Ct(a.copy(), 1.0)).data)
