@@ -80,7 +80,12 @@ struct Slab {
     static constexpr int R = 1 << LR, Q = R / 16, CW = (4096 >> H) / R, T = LR - 4, WORDS = 4096 >> H;
     static __device__ __forceinline__ u32 cc() { return L::t() & (CW - 1); }
     static __device__ __forceinline__ u32 rh() { return L::t() >> (12 - LR - H); }
-    static __device__ __forceinline__ u32 col() { return blockIdx.x * CW + cc(); }
+    // Slabs of eight columns: the two that share lines of 128 bytes lie on one XCD (workgroups go round the eight by their number),
+    // whose L2 then fetches a line once and writes it whole
+    static __device__ __forceinline__ u32 slab() {
+        return CW >= 16 ? blockIdx.x : ((blockIdx.x & 7u) << 1) + ((blockIdx.x >> 4) << 4) + ((blockIdx.x >> 3) & 1u);
+    }
+    static __device__ __forceinline__ u32 col() { return slab() * CW + cc(); }
     // twiddle group of the second block: 16 / Q sub-blocks per thread
     static __device__ __forceinline__ u32 group() { return 16u + rh() * (16 / Q); }
     // place of (row r, column cc) in the exchange buffer.  At 16 columns a wavefront reads rows 16 apart together: row r is
@@ -89,6 +94,8 @@ struct Slab {
     // conflicts: 9.7 against 8.8 us for 10 limbs of 42-bit primes)
     template <bool INV>
     static __device__ __forceinline__ int at(const int r) {
+        if (P == 4 && CW == 8)
+            return (r ^ ((((r >> 6) ^ (r >> 4)) & 1) << 1)) * CW + (int)cc();
         if (P == 4)   // its lanes 16 apart hold rows a whole or the fourth part of a block apart, in both passes: one bit of either goes in
             return (r ^ (((LR >= 7 ? 0 : r >> 2) ^ (r >> (LR - 2))) & 1)) * CW + (int)cc();
         return (CW == 16 && !INV ? swz_row(r) : r) * CW + (int)cc();
@@ -542,25 +549,32 @@ static bool few_for_rows(const hemm_context *c, int limbs) { return (size_t)limb
 static bool few_for_conversions(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 256; }
 
 // Column passes of few workgroups are bound by the instructions of the few CUs they are on: slabs of a half or a
-// quarter of the columns (1, 2: as powers of two) put them on as many more CUs.  Not below 16 columns, segments of 128 bytes: at 2^16 points,
-// half slabs take a rotation on 60-bit primes from 129.8 to 133.7 us where up to 512 workgroups have them, to 131.1 where up to 128 do.
-// Transforms (forward/inverse, us) with whole / with narrower slabs:
+// quarter of the columns (1, 2: as powers of two) put them on as many more CUs.  At 2^16 points a half slab is eight columns, segments of
+// 64 bytes, and pays where both halves of a line are on one XCD (Slab::slab); on two of them rotations lost 3 %, and quarters gain nothing
+// more.  Transforms of 2^16 points, us (forward, inverse) with whole / half slabs, 60 and 42 bits:
+//   workgroups   64                              128                               192                              384                               512
+//   60 bits      10.9/10.0 11.0/9.9   12.6/12.0 13.3/12.4   13.0/11.9 13.5/12.5   23.8/22.9 25.3/24.0   24.8/25.1 27.3/27.5
+//   42 bits       9.7/ 9.6  9.7/9.9   11.8/11.1 12.1/11.4   11.6/11.0 12.3/11.6   21.0/20.3 21.9/20.9   23.5/23.6 24.5/24.5
+// Rotations and products, with conversions up to 256 workgroups: 42 bits, level 1 48.0/44.1 and 74.0/67.8, level 4 54.6/50.0 and 85.2/79.5, level 9
+// 70.8/69.4 and 106.9/104.8; 60 bits, level 5 57.7/53.1 and 91.2/85.1, level 10 82.2/80.8 and 124.4/122.4, level 20 126.0/125.7.
+// Smaller rings, transforms (forward/inverse, us) with whole / with narrower slabs:
 //   limbs              1                 4                 16                32                48                64
 //   2^13 points        9.2/9.5 8.4/8.8   9.2/9.8 8.5/8.9   9.6/10.1 8.8/9.2  10.4/11.0 9.6/10.0   11.4/11.9 11.2/11.6  (one launch)
 //   2^14               9.4/10.0 8.5/8.9  9.6/10.2 8.6/9.2  10.8/11.2 10.1/10.4 12.6/13.3 12.7/13.0 15.9/16.4 15.7/16.2 17.9/18.5 17.8/18.2
 //   2^15               9.8/10.5 8.9/9.2  10.3/10.8 9.5/9.7 13.0/13.3 12.3/12.1 18.2/18.7 18.9/18.3 25.4/26.3 24.5/24.9 30.4/31.3 30.7/30.9
 // (plain forward passes of 2^15 points keep whole slabs above 128 workgroups.)  Rotations of 6 / 12 / 24 limbs, 42 bits: 2^13 41.2/43.6/98.7 ->
 // 35.6/38.4/92.9, 2^14 43.9/50.8/114.7 -> 38.5/47.2/112.0, 2^15 50.3/68.0/145.1 -> 46.3/62.8/142.3; products alike.
-static int narrower_slabs(const hemm_context *c, int limbs, bool plain_forward = false) {
+static int narrower_slabs(const hemm_context *c, int limbs, bool plain = false, bool inverse = false) {
     const size_t wgs = (size_t)limbs * (c->N >> 12);
-    if (c->logN == 16 || (c->logN == 15 && plain_forward && wgs > 128)) return 0;
+    if (c->logN == 16) return wgs <= (plain ? 384 : 256) ? 1 : 0;
+    if (c->logN == 15 && plain && !inverse && wgs > 128) return 0;
     return c->logN <= 14 && wgs <= 128 ? 2 : wgs <= 512 ? 1 : 0;
 }
 
 static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbList &ll, const LimbList &sl, int n_limbs,
                       int n_polys, size_t poly_stride, hipStream_t s, const void *final_scale = nullptr) {
     const bool few = few_for_columns(c, n_limbs * n_polys);
-    const int narrow = narrower_slabs(c, n_limbs * n_polys, !inverse);
+    const int narrow = narrower_slabs(c, n_limbs * n_polys, true, inverse);
     const dim3 grid((unsigned)(c->N >> (12 - narrow)), (unsigned)(n_limbs * n_polys));
     const Tw *tw = (const Tw *)(inverse ? c->d_iw : c->d_w);
 #define COLS_FORM(LR, P, H, INV)                                                                                          \
@@ -588,7 +602,9 @@ static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
         case 14: COLS_SMALL(6); break;
         case 15: COLS(7); break;
         default:
-            if (inverse && few) COLS_FORM(8, 4, 0, true);
+            if (inverse && narrow == 1) COLS_FORM(8, 4, 1, true);
+            else if (narrow == 1) COLS_FORM(8, 4, 1, false);
+            else if (inverse && few) COLS_FORM(8, 4, 0, true);
             else if (inverse) COLS_FORM(8, 16, 0, true);
             else if (few) COLS_FORM(8, 4, 0, false);
             else COLS_FORM(8, 16, 0, false);
@@ -771,7 +787,15 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
         case 13: CONV_SMALL(5); break;
         case 14: CONV_SMALL(6); break;
         case 15: CONV_SLAB(7); break;
-        default: CONV_RING(8, 0); break;
+        default:
+            if (narrow == 1) {   // never without `few`
+                if (widest <= 2) CONV_POINTS(8, 4, 1, 2);
+                else if (widest <= 5) CONV_POINTS(8, 4, 1, 5);
+                else CONV_POINTS(8, 4, 1, 8);
+            } else if (widest <= 2) CONV_POINTS(8, 8, 0, 2);
+            else if (widest <= 5) CONV_POINTS(8, 8, 0, 5);
+            else CONV_POINTS(8, 8, 0, 8);
+            break;
     }
 #undef CONV_SMALL
 #undef CONV_SLAB
@@ -926,7 +950,10 @@ bool launch_ntt_lifted(const hemm_context *c, const LiftSource &ls, u64 *data, c
             case 13: LIFTED(5); break;
             case 14: LIFTED(6); break;
             case 15: LIFTED(7); break;
-            default: LIFTED_FORM(8, 0); break;
+            default:
+                if (half) LIFTED_POINTS(8, 4, 1);
+                else LIFTED_POINTS(8, 8, 0);
+                break;
         }
 #undef LIFTED
 #undef LIFTED_FORM

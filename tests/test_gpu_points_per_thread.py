@@ -14,9 +14,10 @@ def _context(log_n):
     return pkg.Context(log_n, mods, [], 1), O.Oracle(log_n, mods, [], 1, threads=8), mods
 
 
-# limbs at which a pass changes: columns at 512 workgroups of 4096 points, rows at 640, one-launch transforms at 256 limbs
+# limbs at which a pass changes: columns at 512 workgroups of 4096 points (of 2^16 points half slabs at 384), rows at 640, one-launch
+# transforms at 256 limbs
 @pytest.mark.parametrize("log_n,limbs", [(10, 2), (11, 2), (12, 1), (12, 256), (12, 257), (13, 1), (14, 81), (15, 64), (15, 65), (15, 80), (15, 81),
-                                         (16, 1), (16, 32), (16, 33), (16, 40), (16, 41)])
+                                         (16, 1), (16, 24), (16, 25), (16, 32), (16, 33), (16, 40), (16, 41)])
 def test_transforms(log_n, limbs):
     import torch
     ctx, orc, mods = _context(log_n)
