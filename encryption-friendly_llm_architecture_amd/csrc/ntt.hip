@@ -537,10 +537,10 @@ void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, c
 //         inverse,    60 bits       12.6/11.6   14.0/13.4       19.1/18.6        25.8/25.5        28.5/28.1        31.6/30.8       38.8/37.6
 //                     42 bits       10.7/10.1   11.8/12.1       16.6/16.4        21.9/21.7        25.4/24.8        24.0/23.8       27.5/27.9
 //         inverse, 2^15 points, 42  10.2/10.4   11.7/11.9       16.6/16.6        21.4/21.3        26.0/25.2        23.3/23.9       26.7/28.2
-// With the conversions (below): rotation on 2^13 points 34.1 -> 30.2 us, inverse transform of 35 limbs of 2^14 points 12.9 -> 12.2, product at
+// (The rows' line was drawn at 864 workgroups, in encodings of nine messages: 40.4 -> 40.1 us.)  With the conversions (below): rotation on 2^13 points 34.1 -> 30.2 us, inverse transform of 35 limbs of 2^14 points 12.9 -> 12.2, product at
 // level 9 109.6 -> 106.1; the products of 128 x 128 matrices the same to 1 %.
 static bool few_for_columns(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 512; }
-static bool few_for_rows(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 640; }
+static bool few_for_rows(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 900; }
 
 // Passes that begin in a basis conversion or a lift: four points where every CU has one workgroup at most, eight otherwise (six waves per
 // SIMD).  Rotations with four points up to 0 / 256 / 400 / 1024 workgroups in a launch of conversions, us: 2^16 points, 42 bits, level 4 (160 and
@@ -930,7 +930,9 @@ bool launch_ntt_lifted(const hemm_context *c, const LiftSource &ls, u64 *data, c
         u64 *d = data + (size_t)p0 * poly_stride;
         LiftSource l = ls;
         l.coef += (size_t)p0 * ls.stride;
-        const bool half = narrower_slabs(c, n_limbs * np) != 0;
+        // (2^16 points: the loads of a lift are few and shared by the limbs of a message, so that half slabs of four points pay longer than
+        // in a conversion.  Encodings of 4 x 6 / 4 x 13 / 9 x 6 / 9 x 13 limbs, us: 28.8/39.3/41.5/56.2 -> 27.7/38.7/40.4/56.5)
+        const bool half = c->logN == 16 ? n_limbs * np <= 64 : narrower_slabs(c, n_limbs * np) != 0;
         const dim3 grid((unsigned)(c->N >> (half ? 11 : 12)), (unsigned)(n_limbs * np));
         const bool few = few_for_conversions(c, n_limbs * np);
 #define LIFTED_FORM(LR, H)                    \

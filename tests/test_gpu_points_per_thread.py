@@ -14,10 +14,10 @@ def _context(log_n):
     return pkg.Context(log_n, mods, [], 1), O.Oracle(log_n, mods, [], 1, threads=8), mods
 
 
-# limbs at which a pass changes: columns at 512 workgroups of 4096 points (of 2^16 points half slabs at 384), rows at 640, one-launch
+# limbs at which a pass changes: columns at 512 workgroups of 4096 points (of 2^16 points half slabs at 384), rows at 900, one-launch
 # transforms at 256 limbs
-@pytest.mark.parametrize("log_n,limbs", [(10, 2), (11, 2), (12, 1), (12, 256), (12, 257), (13, 1), (14, 81), (15, 64), (15, 65), (15, 80), (15, 81),
-                                         (16, 1), (16, 24), (16, 25), (16, 32), (16, 33), (16, 40), (16, 41)])
+@pytest.mark.parametrize("log_n,limbs", [(10, 2), (11, 2), (12, 1), (12, 256), (12, 257), (13, 1), (14, 81), (15, 64), (15, 65), (15, 112), (15, 113),
+                                         (16, 1), (16, 24), (16, 25), (16, 32), (16, 33), (16, 56), (16, 57)])
 def test_transforms(log_n, limbs):
     import torch
     ctx, orc, mods = _context(log_n)
@@ -48,3 +48,17 @@ def test_conversions(log_n, polys, nq):
     a[0, -1] = mods[nq - 1] - 1
     got = ctx.rescale(torch.from_numpy(a.view(np.int64)).cuda(), nq).cpu().numpy().view(np.uint64)
     assert np.array_equal(got, orc.rescale(O.Ct(a.copy(), 1.0)).data)
+
+
+# lifts of encodings at 1024 workgroups of 4096 points (2^16 points: half slabs of four points up to there)
+@pytest.mark.parametrize("log_n,messages", [(16, 1), (16, 21), (16, 22)])
+def test_lifts(log_n, messages):
+    import torch
+    pkg = load_package()
+    mods = O.primes_below(60, log_n, 1) + O.primes_below(42, log_n, 2)
+    ctx, orc = pkg.Context(log_n, mods, [], 1), O.Oracle(log_n, mods, [], 1, threads=8)
+    rng = np.random.default_rng(messages)
+    z = rng.uniform(-1, 1, (messages, 1 << (log_n - 1))) + 1j * rng.uniform(-1, 1, (messages, 1 << (log_n - 1)))
+    got = ctx.encode(torch.from_numpy(z).cuda(), float(2**40), 3).cpu().numpy().view(np.uint64)
+    for p in {0, messages // 2, messages - 1}:
+        assert np.array_equal(got[p], orc.encode(z[p], 2, 2.0**40).data), p
