@@ -115,9 +115,11 @@ struct Slots {
     u32 count;
 };
 // The column stages.  A workgroup owns R rows of CW columns, a thread one butterfly of each stage: rows i and i + d.
-template <int LR, bool DECODE>
-__global__ __launch_bounds__(512) void emb_cols_kernel(const Slots io, double2 *__restrict__ z, const double2 *__restrict__ roots) {
-    constexpr int R = 1 << LR, CW = R >= 4 ? 1024 / R : 256;
+// POINTS of a workgroup: 1024, or 2048 (2^16 points) where the slots are read from host memory: segments of 128 bytes are half the requests,
+// 11.2 -> 8.8 us for 128 x 128 values.  Writing there gains nothing from them (5.9 / 6.5).
+template <int LR, bool DECODE, int POINTS>
+__global__ __launch_bounds__(POINTS / 2) void emb_cols_kernel(const Slots io, double2 *__restrict__ z, const double2 *__restrict__ roots) {
+    constexpr int R = 1 << LR, CW = R >= 4 ? POINTS / R : 256;
     __shared__ double2 s[R * CW];
     const u32 cc = threadIdx.x % CW, q = threadIdx.x / CW, col = blockIdx.x * CW + cc, n = 256u << LR;
     double2 k[LR];
@@ -172,14 +174,18 @@ __global__ __launch_bounds__(512) void emb_cols_kernel(const Slots io, double2 *
 // The row stages and the integers.  Coefficient i sits at point brev(i): i = brev8(column) R + brev(row).  A workgroup owns
 // the W rows whose reversed index runs over W consecutive values, so that it touches the coefficients in runs of W.
 // Encode: z -> coef (coefficient order); decode: residues co[limb][N] -> z.
-template <int LR, bool DECODE>
-__global__ __launch_bounds__(1024) void emb_rows_kernel(double2 *__restrict__ z, const double2 *__restrict__ roots,
+// Eight rows, runs of 64 bytes; a message or two, which would leave most CUs without a workgroup (a decoding's integers and
+// divisions are 4 us of instructions on sixteen), two rows: those that share a run then lie on one XCD.
+// One message of 2^15 slots: decode 10.4 -> 6.8 us, encode 5.3 -> 3.9; nine messages keep eight rows.
+template <int LR, bool DECODE, int W>
+__global__ __launch_bounds__(128 * W) void emb_rows_kernel(double2 *__restrict__ z, const double2 *__restrict__ roots,
                                                         long long *__restrict__ coef, const double scale,
                                                         const u64 *__restrict__ co, const CentreArgs ca,
                                                         const ModQ *__restrict__ modq) {
-    constexpr int R = 1 << LR, W = R < 8 ? R : 8, LW = LR < 3 ? LR : 3, PITCH = 257, TH = 128 * W;
+    constexpr int R = 1 << LR, LW = W == 8 ? 3 : W == 4 ? 2 : W == 2 ? 1 : 0, PITCH = 257, TH = 128 * W, SHARE = R < 8 ? 1 : 8 / W;
     __shared__ double2 s[W * PITCH];
-    const u32 n = 256u << LR, w = threadIdx.x >> 7, q = threadIdx.x & 127u, i0 = blockIdx.x * W;
+    const u32 x = blockIdx.x, slot = R >= 64 ? ((x & 7u) + 8u * ((x >> 3) / SHARE)) * SHARE + (x >> 3) % SHARE : x;
+    const u32 n = 256u << LR, w = threadIdx.x >> 7, q = threadIdx.x & 127u, i0 = slot * W;
     const u32 r = __brev(i0 + w) >> (32 - LR);   // the row in this slot
     double2 k[8];
 #pragma unroll
@@ -285,7 +291,7 @@ void cols_stages(const hemm_context *c, const Slots &io, double2 *z, int n_msgs,
     const EmbTables &t = tables_of(c);
     const double2 *roots = DECODE ? t.dec : t.enc;
 #define EMB_COLS(LR)                                                                                                       \
-    hipLaunchKernelGGL((emb_cols_kernel<LR, DECODE>), dim3(pow2(LR - 2), n_msgs), dim3(LR >= 2 ? 512 : 256), \
+    hipLaunchKernelGGL((emb_cols_kernel<LR, DECODE, LR >= 2 ? 1024 : 512>), dim3(pow2(LR - 2), n_msgs), dim3(LR >= 2 ? 512 : 256), \
                        0, s, io, z, roots)
     switch (c->logN - 9) {
         case 1: EMB_COLS(1); break;
@@ -294,7 +300,11 @@ void cols_stages(const hemm_context *c, const Slots &io, double2 *z, int n_msgs,
         case 4: EMB_COLS(4); break;
         case 5: EMB_COLS(5); break;
         case 6: EMB_COLS(6); break;
-        default: EMB_COLS(7); break;
+        default:
+            if (!DECODE && io.z == nullptr)
+                hipLaunchKernelGGL((emb_cols_kernel<7, false, 2048>), dim3(16, n_msgs), dim3(1024), 0, s, io, z, roots);
+            else
+                EMB_COLS(7);
     }
 #undef EMB_COLS
 }
@@ -303,9 +313,14 @@ void rows_stages(const hemm_context *c, double2 *z, long long *coef, double scal
                  int n_msgs, hipStream_t s) {
     const EmbTables &t = tables_of(c);
     const double2 *roots = DECODE ? t.dec : t.enc;
-#define EMB_ROWS(LR)                                                                                                  \
-    hipLaunchKernelGGL((emb_rows_kernel<LR, DECODE>), dim3(pow2(LR - 3), n_msgs),                                     \
-                       dim3(LR >= 3 ? 1024 : 128u << LR), 0, s, z, roots, coef, scale, co, ca, c->d_modq)
+#define EMB_ROWS_OF(LR, W)                                                                                            \
+    hipLaunchKernelGGL((emb_rows_kernel<LR, DECODE, W>), dim3((1u << LR) / (W), n_msgs), dim3(128 * (W)), 0, s, z, roots, coef, scale, co, ca, \
+                       c->d_modq)
+#define EMB_ROWS(LR)                                                     \
+    do {                                                                 \
+        if (LR >= 3 && (n_msgs << LR) > 256) EMB_ROWS_OF(LR, LR >= 3 ? 8 : 2); \
+        else EMB_ROWS_OF(LR, 2);                                         \
+    } while (0)
     switch (c->logN - 9) {
         case 1: EMB_ROWS(1); break;
         case 2: EMB_ROWS(2); break;
@@ -316,6 +331,7 @@ void rows_stages(const hemm_context *c, double2 *z, long long *coef, double scal
         default: EMB_ROWS(7); break;
     }
 #undef EMB_ROWS
+#undef EMB_ROWS_OF
 }
 
 CentreArgs centre_args(const hemm_context *c, int n_limbs, double scale) {
