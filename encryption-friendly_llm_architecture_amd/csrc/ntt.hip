@@ -542,10 +542,9 @@ void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, c
 static bool few_for_columns(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 512; }
 static bool few_for_rows(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 900; }
 
-// Passes that begin in a basis conversion or a lift: four points where every CU has one workgroup at most, eight otherwise (six waves per
-// SIMD).  Rotations with four points up to 0 / 256 / 400 / 1024 workgroups in a launch of conversions, us: 2^16 points, 42 bits, level 4 (160 and
-// fewer) 55.9/54.8/55.0/55.1, level 6 (224) 63.4/62.2/62.2/61.9, level 9 (288) 72.0/72.1/73.6/73.5; 60 bits, level 5 (192) 60.3/58.8/58.8/58.7, level 10 (384)
-// 83.7/83.2/82.8/82.6, level 15 (512) 93.8/94.0/96.2/97.1, level 20 (864) 128.2/127.7/128.0/136.0; 2^14 points, level 6 (48) 42.2/39.9/40.6/41.0.
+// Passes that begin in a basis conversion or a lift, on rings below 2^16 points: four points where every CU has one workgroup at most, eight
+// otherwise (six waves per SIMD); rotations of 2^14 points at level 6 (48 workgroups in a launch of conversions) 42.2 -> 39.9 us, at level 12 51.6 ->
+// 50.4.  At 2^16 points four points go with the half slabs of narrower_slabs, eight with whole ones.
 static bool few_for_conversions(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 256; }
 
 // Column passes of few workgroups are bound by the instructions of the few CUs they are on: slabs of a half or a
@@ -555,8 +554,15 @@ static bool few_for_conversions(const hemm_context *c, int limbs) { return (size
 //   workgroups   64                              128                               192                              384                               512
 //   60 bits      10.9/10.0 11.0/9.9   12.6/12.0 13.3/12.4   13.0/11.9 13.5/12.5   23.8/22.9 25.3/24.0   24.8/25.1 27.3/27.5
 //   42 bits       9.7/ 9.6  9.7/9.9   11.8/11.1 12.1/11.4   11.6/11.0 12.3/11.6   21.0/20.3 21.9/20.9   23.5/23.6 24.5/24.5
-// Rotations and products, with conversions up to 256 workgroups: 42 bits, level 1 48.0/44.1 and 74.0/67.8, level 4 54.6/50.0 and 85.2/79.5, level 9
-// 70.8/69.4 and 106.9/104.8; 60 bits, level 5 57.7/53.1 and 91.2/85.1, level 10 82.2/80.8 and 124.4/122.4, level 20 126.0/125.7.
+// Conversions take half slabs further, their whole ones being bound by the three workgroups that a CU holds in step.  Rotations and products of
+// 2^16 points, us, with none / up to 256 / 400 / 700 / 1000 workgroups of conversions on half slabs of four points:
+//   42 bits, level  4 (160 and fewer)   54.6/50.0/50.0/50.0/50.0   85.2/ 79.5/ 79.5/ 79.5/ 79.5
+//                   8 (up to 256, 288)  67.8/67.8/64.3/64.0/64.1  100.3/100.3/ 96.8/ 96.6/ 95.9
+//                  10 (400, 528)        80.8/80.8/80.1/76.2/76.3  117.3/117.3/114.5/110.8/111.1
+//   60 bits, level 10 (384)             82.2/80.6/75.2/75.2/75.4  124.4/120.7/113.9/114.1/113.9
+//                  18 (608, 784)       117.3/117.3/117.0/114.9/113.9  170.3/170.3/170.4/168.2/167.4
+//                  23 (768, 960)       130.2/130.2/130.2/130.6/131.6  191.2/191.2/191.5/191.6/192.7
+// The products of matrices, whose large conversions run beside other chains, are 1 - 3 % slower with all of them on half slabs.
 // Smaller rings, transforms (forward/inverse, us) with whole / with narrower slabs:
 //   limbs              1                 4                 16                32                48                64
 //   2^13 points        9.2/9.5 8.4/8.8   9.2/9.8 8.5/8.9   9.6/10.1 8.8/9.2  10.4/11.0 9.6/10.0   11.4/11.9 11.2/11.6  (one launch)
@@ -566,7 +572,7 @@ static bool few_for_conversions(const hemm_context *c, int limbs) { return (size
 // 35.6/38.4/92.9, 2^14 43.9/50.8/114.7 -> 38.5/47.2/112.0, 2^15 50.3/68.0/145.1 -> 46.3/62.8/142.3; products alike.
 static int narrower_slabs(const hemm_context *c, int limbs, bool plain = false, bool inverse = false) {
     const size_t wgs = (size_t)limbs * (c->N >> 12);
-    if (c->logN == 16) return wgs <= (plain ? 384 : 256) ? 1 : 0;
+    if (c->logN == 16) return wgs <= (plain ? 384 : 768) ? 1 : 0;
     if (c->logN == 15 && plain && !inverse && wgs > 128) return 0;
     return c->logN <= 14 && wgs <= 128 ? 2 : wgs <= 512 ? 1 : 0;
 }

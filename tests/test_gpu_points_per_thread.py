@@ -36,8 +36,9 @@ def test_transforms(log_n, limbs):
         assert np.array_equal(d.cpu().numpy().view(np.uint64), a), prime
 
 
-# conversions at 256 workgroups of 4096 points: a rescale of `polys` polynomials of nq limbs launches polys (nq - 1) limbs
-@pytest.mark.parametrize("log_n,polys,nq", [(11, 2, 4), (12, 2, 18), (13, 2, 4), (14, 4, 17), (14, 4, 18), (15, 2, 17), (15, 2, 18), (16, 2, 9), (16, 2, 10)])
+# conversions at 256 workgroups of 4096 points (2^16 points: at 768): a rescale of `polys` polynomials of nq limbs launches polys (nq - 1) limbs
+@pytest.mark.parametrize("log_n,polys,nq", [(11, 2, 4), (12, 2, 18), (13, 2, 4), (14, 4, 17), (14, 4, 18), (15, 2, 17), (15, 2, 18), (16, 2, 9), (16, 3, 17),
+                                            (16, 3, 18)])
 def test_conversions(log_n, polys, nq):
     import torch
     pkg = load_package()
