@@ -304,7 +304,7 @@ def gpu_hoisted(args, out):
         groups.append([(src[t][0], src[t][1], evk, rnd(E, N >> shift, 2), gal, shift) for t in range(2)])
     ms = timed(lambda: ctx.hoisted_moddown(groups, nq, True, b_premultiplied=True, compact_keys=True))
     moved = n_out * (key_words_bytes(nq) + 2 * E * (N >> shift) * 16 + 2 * (nq - 1) * LIMB_BYTES) + 2 * (beta * E + nq) * LIMB_BYTES
-    out["roofline"] = entry("hoisted_terms_kernel<0, true, 1, SumRows> + ntt16_cols_kernel<8, 16, 0, true> + ntt16_cols_converted_kernel<8, 0, 5> + "
+    out["roofline"] = entry("hoisted_terms_kernel<0, true, 1, SumRows> + ntt16_cols_kernel<8, 16, 0, true> + ntt16_cols_converted_kernel<8, 8, 0, 5> + "
                             "hoisted_terms_kernel<0, true, 1, SumTail> (one chain of the CCMM main loop: 16 shifts of two masked sources under one compact key, "
                             "8+4 limbs, 2 digits, run-table masks, divided by P and rescaled to 7 limbs)", ms, moved, traffic=CHAIN_TRAFFIC_BYTES)
     nq = 9
@@ -320,7 +320,7 @@ def gpu_hoisted(args, out):
     y = rnd(16, nq + K, N)
     ms = timed(lambda: ctx.moddown_batch(y, nq, True))
     moved = 16 * (nq + K + nq - 1) * LIMB_BYTES
-    out["roofline_moddown"] = entry("ntt16_rows_kernel<8, 8, true, 0, 0> + ntt16_cols_kernel<8, 16, 0, true> + ntt16_cols_converted_kernel<8, 0, 5> + "
+    out["roofline_moddown"] = entry("ntt16_rows_kernel<8, 8, true, 0, 0> + ntt16_cols_kernel<8, 16, 0, true> + ntt16_cols_converted_kernel<8, 8, 0, 5> + "
                                     "ntt16_rows_kernel<8, 16, false, 1, 0> (ModDown and rescale of the plaintext product's eight inner sums: 16 "
                                     "polynomials, 6+4 -> 5 limbs)", ms, moved)
     if args.roofline_only:
