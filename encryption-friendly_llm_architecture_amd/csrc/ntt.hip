@@ -537,10 +537,26 @@ void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, c
 //         inverse,    60 bits       12.6/11.6   14.0/13.4       19.1/18.6        25.8/25.5        28.5/28.1        31.6/30.8       38.8/37.6
 //                     42 bits       10.7/10.1   11.8/12.1       16.6/16.4        21.9/21.7        25.4/24.8        24.0/23.8       27.5/27.9
 //         inverse, 2^15 points, 42  10.2/10.4   11.7/11.9       16.6/16.6        21.4/21.3        26.0/25.2        23.3/23.9       26.7/28.2
-// (The rows' line was drawn at 864 workgroups, in encodings of nine messages: 40.4 -> 40.1 us.)  With the conversions (below): rotation on 2^13 points 34.1 -> 30.2 us, inverse transform of 35 limbs of 2^14 points 12.9 -> 12.2, product at
+// With the conversions (below): rotation on 2^13 points 34.1 -> 30.2 us, inverse transform of 35 limbs of 2^14 points 12.9 -> 12.2, product at
 // level 9 109.6 -> 106.1; the products of 128 x 128 matrices the same to 1 %.
 static bool few_for_columns(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 512; }
-static bool few_for_rows(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 900; }
+// Row passes: eight points beyond the line of four, where four put more workgroups on a CU than are resident; encodings of 2^14 points
+// leave four earlier and eight for sixteen at 640.  us with sixteen / eight / four points, second figure of each pair 42 bits:
+//   workgroups                        544                              640                              768                              896
+//   forward, 2^16 points   33.3/32.8/31.5 28.5/28.1/27.2  28.5/27.3/27.0 24.4/23.2/23.5  30.1/29.7/29.5 23.9/23.6/24.0  34.5/33.6/33.6 26.8/25.5/26.7
+//            2^15          32.5/31.6/30.6 28.4/27.2/26.8  29.5/28.0/27.7 25.7/24.6/24.6  28.8/28.6/28.7 23.5/23.2/23.8  33.3/32.3/33.0 25.9/25.0/26.1
+//   inverse, 2^16          37.0/35.3/34.1 29.7/29.5/28.5  32.6/31.5/30.7 26.1/25.2/24.9  33.6/32.4/32.8 25.2/24.7/25.0  38.4/36.7/36.6 27.9/26.8/27.3
+//            2^15          37.4/34.3/33.2 31.0/28.6/28.2  34.0/30.9/31.2 27.3/25.6/26.1  32.5/30.9/31.8 25.0/24.1/25.0  36.6/35.2/35.9 27.1/26.5/27.5
+//   rescale, 2^16          44.3/41.0/40.4 37.6/34.3/34.0  44.0/42.1/42.8 38.2/34.9/35.6  47.0/45.8/47.5 39.7/37.6/38.7
+//            2^15          46.1/42.4/41.6 38.1/35.2/34.6  46.7/43.9/43.9 39.7/36.2/35.9  48.8/46.0/46.6 41.4/37.6/38.6
+//   encodings of 2^14 points, m messages x limbs: 11x12 34.8/34.5/34.9, 23x6 37.9/36.6/37.6, 26x6 38.6/37.2/38.2, 32x5 37.6/37.3/38.7, 32x6 38.5/38.1/39.4,
+//   64x3 39.9/39.9/41.1, 16x13 37.4/39.2/40.3; of 2^16 4x13 40.8/39.5/40.3, 9x6 42.4/41.3/42.2
+static int points_for_rows(const hemm_context *c, int limbs, bool inverse, int tail) {
+    const size_t wgs = (size_t)limbs * (c->N >> 12);
+    const bool encoding = c->logN == 14 && !inverse && tail == TAIL_NONE;   // longer plain transforms of this ring are one launch
+    if (wgs <= (encoding ? 512 : 640)) return 4;
+    return inverse || wgs <= (encoding ? 640 : 900) ? 8 : 16;
+}
 
 // Passes that begin in a basis conversion or a lift, on rings below 2^16 points: four points where every CU has one workgroup at most, eight
 // otherwise (six waves per SIMD); rotations of 2^14 points at level 6 (48 workgroups in a launch of conversions) 42.2 -> 39.9 us, at level 12 51.6 ->
@@ -623,8 +639,8 @@ static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
 static void rows_pass(const hemm_context *c, bool inverse, u64 *d, const LimbList &ll, const LimbList &sl, int n_limbs,
                       int n_polys, size_t poly_stride, hipStream_t s, const NttEpilogue &ep, int tail = TAIL_NONE,
                       int load = LOAD_PLAIN, const ResultList *list = nullptr, int first = 0) {
-    const bool few = few_for_rows(c, n_limbs * n_polys);
-    const dim3 grid((unsigned)(c->N >> (few ? 10 : inverse ? 11 : 12)) * (unsigned)(n_limbs * n_polys)), block(256);
+    const int points = points_for_rows(c, n_limbs * n_polys, inverse, tail);
+    const dim3 grid((unsigned)(c->N >> 8) / (unsigned)points * (unsigned)(n_limbs * n_polys)), block(256);
     const int log_r = c->logN - 8;
 #define ROWS(LR, P, INV, TAIL, LOAD, EP)                                                                                      \
     hipLaunchKernelGGL((ntt16_rows_kernel<LR, P, INV, TAIL, LOAD>), grid, block, 0, s, d, (const Tw *)(INV ? c->d_iw : c->d_w), \
@@ -636,12 +652,13 @@ static void rows_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
     } while (0)
 #define ROWS_INVERSE(LOAD)                                       \
     do {                                                         \
-        if (few) ROWS_RING(4, true, TAIL_NONE, LOAD, ep);        \
+        if (points == 4) ROWS_RING(4, true, TAIL_NONE, LOAD, ep); \
         else ROWS_RING(8, true, TAIL_NONE, LOAD, ep);            \
     } while (0)
 #define ROWS_FORWARD(TAIL, EP)                                   \
     do {                                                         \
-        if (few) ROWS_RING(4, false, TAIL, LOAD_PLAIN, EP);      \
+        if (points == 4) ROWS_RING(4, false, TAIL, LOAD_PLAIN, EP); \
+        else if (points == 8) ROWS_RING(8, false, TAIL, LOAD_PLAIN, EP); \
         else ROWS_RING(16, false, TAIL, LOAD_PLAIN, EP);         \
     } while (0)
     if (inverse && load == LOAD_ROTATED)

@@ -14,10 +14,11 @@ def _context(log_n):
     return pkg.Context(log_n, mods, [], 1), O.Oracle(log_n, mods, [], 1, threads=8), mods
 
 
-# limbs at which a pass changes: columns at 512 workgroups of 4096 points (of 2^16 points half slabs at 384), rows at 900, one-launch
-# transforms at 256 limbs
-@pytest.mark.parametrize("log_n,limbs", [(10, 2), (11, 2), (12, 1), (12, 256), (12, 257), (13, 1), (14, 81), (15, 64), (15, 65), (15, 112), (15, 113),
-                                         (16, 1), (16, 24), (16, 25), (16, 32), (16, 33), (16, 56), (16, 57)])
+# limbs at which a pass changes: columns at 512 workgroups of 4096 points (of 2^16 points half slabs at 384), rows at 640 and (forward) 900,
+# one-launch transforms at 256 limbs
+@pytest.mark.parametrize("log_n,limbs", [(10, 2), (11, 2), (12, 1), (12, 256), (12, 257), (13, 1), (14, 81), (15, 64), (15, 65), (15, 80), (15, 81),
+                                         (15, 112), (15, 113), (16, 1), (16, 24), (16, 25), (16, 32), (16, 33), (16, 40), (16, 41), (16, 56),
+                                         (16, 57)])
 def test_transforms(log_n, limbs):
     import torch
     ctx, orc, mods = _context(log_n)
@@ -36,9 +37,11 @@ def test_transforms(log_n, limbs):
         assert np.array_equal(d.cpu().numpy().view(np.uint64), a), prime
 
 
-# conversions at 256 workgroups of 4096 points (2^16 points: at 768): a rescale of `polys` polynomials of nq limbs launches polys (nq - 1) limbs
-@pytest.mark.parametrize("log_n,polys,nq", [(11, 2, 4), (12, 2, 18), (13, 2, 4), (14, 4, 17), (14, 4, 18), (15, 2, 17), (15, 2, 18), (16, 2, 9), (16, 3, 17),
-                                            (16, 3, 18)])
+# conversions at 256 workgroups of 4096 points (2^16 points: at 768), the row passes behind them at 640 and 900: a rescale of `polys` polynomials
+# of nq limbs launches polys (nq - 1) limbs
+@pytest.mark.parametrize("log_n,polys,nq", [(11, 2, 4), (12, 2, 18), (13, 2, 4), (14, 4, 17), (14, 4, 18), (15, 2, 17), (15, 2, 18), (15, 5, 17),
+                                            (15, 9, 10), (15, 7, 17), (15, 8, 16), (16, 2, 9), (16, 4, 11), (16, 3, 15), (16, 3, 17), (16, 3, 18),
+                                            (16, 7, 9), (16, 6, 11)])
 def test_conversions(log_n, polys, nq):
     import torch
     pkg = load_package()
@@ -51,8 +54,11 @@ def test_conversions(log_n, polys, nq):
     assert np.array_equal(got, orc.rescale(O.Ct(a.copy(), 1.0)).data)
 
 
-# lifts of encodings at 1024 workgroups of 4096 points (2^16 points: half slabs of four points up to there)
-@pytest.mark.parametrize("log_n,messages", [(16, 1), (16, 21), (16, 22)])
+# lifts of encodings, three limbs a message: slabs at 128 and 512 workgroups of 4096 points (2^16 points: at 1024), points per thread at 256,
+# the row passes behind them at 640 and 900 (2^14 points: at 512 and 640); 2^13 points take one launch from 64 limbs on
+@pytest.mark.parametrize("log_n,messages", [(13, 1), (13, 21), (13, 22), (14, 10), (14, 11), (14, 21), (14, 22), (14, 42), (14, 43), (14, 53), (14, 54),
+                                            (15, 5), (15, 6), (15, 10), (15, 11), (15, 21), (15, 22), (15, 26), (15, 27), (15, 37), (15, 38),
+                                            (16, 1), (16, 13), (16, 14), (16, 18), (16, 19), (16, 21), (16, 22)])
 def test_lifts(log_n, messages):
     import torch
     pkg = load_package()
