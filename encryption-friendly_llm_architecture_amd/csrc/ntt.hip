@@ -605,7 +605,6 @@ static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
 #define COLS_SLAB(LR, INV)                          \
     do {                                            \
         if (narrow == 1) COLS_FORM(LR, 4, 1, INV);  \
-        else if (few) COLS_FORM(LR, 4, 0, INV);     \
         else COLS_FORM(LR, 16, 0, INV);             \
     } while (0)
 #define COLS(LR)                                    \
@@ -622,14 +621,14 @@ static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
     switch (c->logN) {
         case 13: COLS_SMALL(5); break;
         case 14: COLS_SMALL(6); break;
-        case 15: COLS(7); break;
+        case 15:   // (inverse whole slabs are never few)
+            if (few && narrow == 0 && !inverse) COLS_FORM(7, 4, 0, false);
+            else COLS(7);
+            break;
         default:
-            if (inverse && narrow == 1) COLS_FORM(8, 4, 1, true);
-            else if (narrow == 1) COLS_FORM(8, 4, 1, false);
-            else if (inverse && few) COLS_FORM(8, 4, 0, true);
-            else if (inverse) COLS_FORM(8, 16, 0, true);
-            else if (few) COLS_FORM(8, 4, 0, false);
-            else COLS_FORM(8, 16, 0, false);
+            if (few && narrow == 0 && inverse) COLS_FORM(8, 4, 0, true);
+            else if (few && narrow == 0) COLS_FORM(8, 4, 0, false);
+            else COLS(8);
     }
 #undef COLS_SMALL
 #undef COLS_SLAB
@@ -782,49 +781,38 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
     const int narrow = narrower_slabs(c, (n_limbs + cs.n_copy) * n_polys);
     const dim3 grid((unsigned)(c->N >> (12 - narrow)), (n_limbs + cs.n_copy) * n_polys);
     const bool few = few_for_conversions(c, (n_limbs + cs.n_copy) * n_polys);
-#define CONV_FORM(LR, H, K)                       \
-    do {                                          \
-        if (few) CONV_POINTS(LR, 4, H, K);       \
-        else CONV_POINTS(LR, 8, H, K);            \
-    } while (0)
-#define CONV_POINTS(LR, P, H, K)                                                                                             \
+#define CONV_FORM(LR, P, H, K)                                                                                               \
     hipLaunchKernelGGL((ntt16_cols_converted_kernel<LR, P, H, K>), grid, dim3((4096 >> H) / P), 0, s, data, (const Tw *)c->d_w, c->d_modq, \
                        c->d_ninv, c->d_ninv_s, c->d_fp, ll, sl, n_limbs, poly_stride, cs)
-#define CONV_RING(LR, H)                        \
-    do {                                        \
-        if (widest <= 2) CONV_FORM(LR, H, 2);   \
-        else if (widest <= 5) CONV_FORM(LR, H, 5); \
-        else CONV_FORM(LR, H, 8);               \
+#define CONV_RING(LR, P, H)                        \
+    do {                                           \
+        if (widest <= 2) CONV_FORM(LR, P, H, 2);   \
+        else if (widest <= 5) CONV_FORM(LR, P, H, 5); \
+        else CONV_FORM(LR, P, H, 8);               \
     } while (0)
-#define CONV_SLAB(LR)                    \
-    do {                                 \
-        if (narrow == 1) CONV_RING(LR, 1); \
-        else CONV_RING(LR, 0);           \
+#define CONV_SLAB(LR)                          \
+    do {                                       \
+        if (narrow == 0) CONV_RING(LR, 8, 0);  \
+        else if (few) CONV_RING(LR, 4, 1);     \
+        else CONV_RING(LR, 8, 1);              \
     } while (0)
-#define CONV_SMALL(LR)                   \
-    do {                                 \
-        if (narrow == 2) CONV_RING(LR, 2); \
-        else CONV_SLAB(LR);              \
+#define CONV_SMALL(LR)                         \
+    do {                                       \
+        if (narrow == 2) CONV_RING(LR, 4, 2);  \
+        else CONV_SLAB(LR);                    \
     } while (0)
     switch (c->logN) {
         case 13: CONV_SMALL(5); break;
         case 14: CONV_SMALL(6); break;
         case 15: CONV_SLAB(7); break;
-        default:
-            if (narrow == 1) {   // never without `few`
-                if (widest <= 2) CONV_POINTS(8, 4, 1, 2);
-                else if (widest <= 5) CONV_POINTS(8, 4, 1, 5);
-                else CONV_POINTS(8, 4, 1, 8);
-            } else if (widest <= 2) CONV_POINTS(8, 8, 0, 2);
-            else if (widest <= 5) CONV_POINTS(8, 8, 0, 5);
-            else CONV_POINTS(8, 8, 0, 8);
-            break;
+        default:   // half slabs take four points whatever the line of the smaller rings says
+            if (narrow == 1) CONV_RING(8, 4, 1);
+            else CONV_RING(8, 8, 0);
     }
 #undef CONV_SMALL
 #undef CONV_SLAB
 #undef CONV_RING
 #undef CONV_FORM
-#undef CONV_POINTS
     if (cols_only) return true;
     rows_pass(c, false, data, ll, sl, n_limbs, n_polys, poly_stride, s,
               sub_scale_tail(ep_minuend, ep_minuend_stride, ep_out, ep_out_stride, ep_cst_dev), tail ? TAIL_SUB_SCALE : TAIL_NONE,
@@ -958,31 +946,25 @@ bool launch_ntt_lifted(const hemm_context *c, const LiftSource &ls, u64 *data, c
         const bool half = c->logN == 16 ? n_limbs * np <= 64 : narrower_slabs(c, n_limbs * np) != 0;
         const dim3 grid((unsigned)(c->N >> (half ? 11 : 12)), (unsigned)(n_limbs * np));
         const bool few = few_for_conversions(c, n_limbs * np);
-#define LIFTED_FORM(LR, H)                    \
-    do {                                      \
-        if (few) LIFTED_POINTS(LR, 4, H);     \
-        else LIFTED_POINTS(LR, 8, H);         \
-    } while (0)
-#define LIFTED_POINTS(LR, P, H)                                                                                                     \
+#define LIFTED_FORM(LR, P, H)                                                                                                       \
     hipLaunchKernelGGL((ntt16_cols_lifted_kernel<LR, P, H>), grid, dim3((4096 >> H) / P), 0, s, d, (const Tw *)c->d_w, c->d_modq, c->d_fp, ll, sl, \
                        n_limbs, poly_stride, l)
-#define LIFTED(LR)                    \
-    do {                              \
-        if (half) LIFTED_FORM(LR, 1); \
-        else LIFTED_FORM(LR, 0);      \
+#define LIFTED(LR)                            \
+    do {                                      \
+        if (!half) LIFTED_FORM(LR, 8, 0);     \
+        else if (few) LIFTED_FORM(LR, 4, 1);  \
+        else LIFTED_FORM(LR, 8, 1);           \
     } while (0)
         switch (c->logN) {
             case 13: LIFTED(5); break;
             case 14: LIFTED(6); break;
             case 15: LIFTED(7); break;
             default:
-                if (half) LIFTED_POINTS(8, 4, 1);
-                else LIFTED_POINTS(8, 8, 0);
-                break;
+                if (half) LIFTED_FORM(8, 4, 1);
+                else LIFTED_FORM(8, 8, 0);
         }
 #undef LIFTED
 #undef LIFTED_FORM
-#undef LIFTED_POINTS
         rows_pass(c, false, d, ll, sl, n_limbs, np, poly_stride, s, ep, tail);
         if (enc != nullptr) {
             ep.out += (size_t)np * poly_stride;

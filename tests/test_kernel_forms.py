@@ -17,3 +17,19 @@ def test_row_passes():
     """Log2 of the rows (0: from the argument), points per thread, inverse."""
     points = {(4, 0), (8, 0), (16, 0), (4, 1), (8, 1)}
     assert _forms("ntt16_rows_kernel", 3) == {(lr,) + p for lr in (0, 8) for p in points}
+
+
+def test_column_passes():
+    """Log2 of the rows, points per thread, slabs narrowed by two to this, inverse: whole slabs of few points only where they are fewer
+    than the line of four and more than that of half slabs."""
+    narrow = {(lr, 4, h, inv) for lr in (5, 6, 7, 8) for h in (1, 2) if h < 2 or lr < 7 for inv in (0, 1)}
+    whole = {(lr, 16, 0, inv) for lr in (5, 6, 7, 8) for inv in (0, 1)} | {(7, 4, 0, 0), (8, 4, 0, 0), (8, 4, 0, 1)}
+    assert _forms("ntt16_cols_kernel", 4) == narrow | whole
+
+
+def test_converted_and_lifted_column_passes():
+    """Log2 of the rows, points per thread, slabs narrowed by two to this (and the sources kept in registers)."""
+    half = {(lr, p, 1) for lr in (5, 6, 7) for p in (4, 8)} | {(8, 4, 1)}
+    whole = {(lr, 8, 0) for lr in (5, 6, 7, 8)}
+    assert _forms("ntt16_cols_lifted_kernel", 3) == half | whole
+    assert _forms("ntt16_cols_converted_kernel", 4) == {f + (k,) for f in half | whole | {(5, 4, 2), (6, 4, 2)} for k in (2, 5, 8)}
