@@ -174,15 +174,21 @@ __global__ __launch_bounds__(POINTS / 2) void emb_cols_kernel(const Slots io, do
 // The row stages and the integers.  Coefficient i sits at point brev(i): i = brev8(column) R + brev(row).  A workgroup owns
 // the W rows whose reversed index runs over W consecutive values, so that it touches the coefficients in runs of W.
 // Encode: z -> coef (coefficient order); decode: residues co[limb][N] -> z.
-// Eight rows, runs of 64 bytes; a message or two, which would leave most CUs without a workgroup (a decoding's integers and
-// divisions are 4 us of instructions on sixteen), two rows: those that share a run then lie on one XCD.
-// One message of 2^15 slots: decode 10.4 -> 6.8 us, encode 5.3 -> 3.9; nine messages keep eight rows.
+// Eight rows, runs of 64 bytes; up to 256 rows of all messages together, which would leave most CUs without a workgroup (a decoding's
+// integers and divisions are 4 us of instructions on sixteen), two rows, runs of 16.  From 2^15 points the four workgroups that touch
+// the same 64 bytes then lie on one XCD; smaller rings have too few workgroups for that and gain from the rows all the same.
+// Whole calls, us with eight / two rows; the line lies where both sides were measured, two rows still lead one message past it:
+//   points                                   2^12        2^13        2^14        2^15        2^16
+//   decode, two limbs                   18.5/15.4   19.5/16.6   20.1/17.3   21.5/18.1   22.2/19.0
+//   encode, three limbs, one message    14.3/12.8   15.7/13.9   16.3/14.5   17.1/15.2   17.7/15.8
+//           256 rows of messages        16.3/14.8   18.7/17.4   18.6/16.7   19.6/17.8   19.0/17.2
+//           one message more            16.3/14.9               19.0/17.9               21.3/19.6
 template <int LR, bool DECODE, int W>
 __global__ __launch_bounds__(128 * W) void emb_rows_kernel(double2 *__restrict__ z, const double2 *__restrict__ roots,
                                                         long long *__restrict__ coef, const double scale,
                                                         const u64 *__restrict__ co, const CentreArgs ca,
                                                         const ModQ *__restrict__ modq) {
-    constexpr int R = 1 << LR, LW = W == 8 ? 3 : W == 4 ? 2 : W == 2 ? 1 : 0, PITCH = 257, TH = 128 * W, SHARE = R < 8 ? 1 : 8 / W;
+    constexpr int R = 1 << LR, LW = W == 8 ? 3 : 1, PITCH = 257, TH = 128 * W, SHARE = R < 8 ? 1 : 8 / W;
     __shared__ double2 s[W * PITCH];
     const u32 x = blockIdx.x, slot = R >= 64 ? ((x & 7u) + 8u * ((x >> 3) / SHARE)) * SHARE + (x >> 3) % SHARE : x;
     const u32 n = 256u << LR, w = threadIdx.x >> 7, q = threadIdx.x & 127u, i0 = slot * W;
@@ -316,11 +322,15 @@ void rows_stages(const hemm_context *c, double2 *z, long long *coef, double scal
 #define EMB_ROWS_OF(LR, W)                                                                                            \
     hipLaunchKernelGGL((emb_rows_kernel<LR, DECODE, W>), dim3((1u << LR) / (W), n_msgs), dim3(128 * (W)), 0, s, z, roots, coef, scale, co, ca, \
                        c->d_modq)
-#define EMB_ROWS(LR)                                                     \
-    do {                                                                 \
-        if (LR >= 3 && (n_msgs << LR) > 256) EMB_ROWS_OF(LR, LR >= 3 ? 8 : 2); \
-        else EMB_ROWS_OF(LR, 2);                                         \
-    } while (0)
+#define EMB_ROWS(LR)                            \
+    do {                                        \
+        if constexpr (!DECODE && LR >= 3)       \
+            if ((n_msgs << LR) > 256) {         \
+                EMB_ROWS_OF(LR, 8);             \
+                break;                          \
+            }                                   \
+        EMB_ROWS_OF(LR, 2);                     \
+    } while (0)   // (a decoding is one message)
     switch (c->logN - 9) {
         case 1: EMB_ROWS(1); break;
         case 2: EMB_ROWS(2); break;

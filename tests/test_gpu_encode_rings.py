@@ -58,8 +58,11 @@ def test_encode_and_decode(log_n, log_scale):
         assert np.array_equal(d.view(np.float64), orc.decode(O.Pt(want[1].data[:limbs], scale)).view(np.float64)), limbs
 
 
-# limbs on both sides of the 64 from which a ring of 2^13 points takes one launch; a batch that is cut into runs (2^16: 448 limbs)
-@pytest.mark.parametrize("log_n,messages,limbs,check", [(13, 21, 3, (0, 20)), (13, 16, 4, (0, 7, 15)), (13, 13, 5, (0, 12)), (14, 20, 5, (0, 19)),
+# limbs on both sides of the 64 from which a ring of 2^13 points takes one launch; messages on both sides of the 256 rows up to which the
+# embedding has two to a workgroup; a batch that is cut into runs (2^16: 448 limbs)
+@pytest.mark.parametrize("log_n,messages,limbs,check", [(12, 32, 2, (0, 31)), (12, 33, 2, (0, 32)), (13, 17, 2, (0, 16)), (14, 8, 2, (0, 7)), (14, 9, 2, (0, 8)),
+                                                        (15, 4, 2, (0, 3)), (15, 5, 2, (0, 4)), (16, 2, 2, (0, 1)),
+                                                        (13, 21, 3, (0, 20)), (13, 16, 4, (0, 7, 15)), (13, 13, 5, (0, 12)), (14, 20, 5, (0, 19)),
                                                         (16, 90, 5, (0, 37, 38, 89))])
 def test_encode_of_batches(log_n, messages, limbs, check):
     import torch

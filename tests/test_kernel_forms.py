@@ -33,3 +33,9 @@ def test_converted_and_lifted_column_passes():
     whole = {(lr, 8, 0) for lr in (5, 6, 7, 8)}
     assert _forms("ntt16_cols_lifted_kernel", 3) == half | whole
     assert _forms("ntt16_cols_converted_kernel", 4) == {f + (k,) for f in half | whole | {(5, 4, 2), (6, 4, 2)} for k in (2, 5, 8)}
+
+
+def test_embedding_rows():
+    """Log2 of the rows, decoding, rows of a workgroup: eight for batches of messages, and a decoding is one."""
+    two = {(lr, decode, 2) for lr in range(1, 8) for decode in (0, 1)}
+    assert _forms("emb_rows_kernel", 3) == two | {(lr, 0, 8) for lr in range(3, 8)}
