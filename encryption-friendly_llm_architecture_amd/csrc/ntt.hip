@@ -663,7 +663,7 @@ static void rows_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
     if (inverse && load == LOAD_ROTATED)
         ROWS_INVERSE(LOAD_ROTATED);
     else if (inverse && load == LOAD_DECRYPT)
-        ROWS_INVERSE(LOAD_DECRYPT);
+        ROWS_RING(4, true, TAIL_NONE, LOAD_DECRYPT, ep);   // one or two limbs
     else if (inverse)
         ROWS_INVERSE(LOAD_PLAIN);
     else if (tail == TAIL_SUB_SCALE && list != nullptr) {

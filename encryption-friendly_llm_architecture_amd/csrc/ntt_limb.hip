@@ -280,7 +280,7 @@ void launch_limb_forward(const hemm_context *c, u64 *data, const LimbList &ll, c
     } while (0)
 #define LIMB_RING(L)                                                       \
     do {                                                                   \
-        if (ls != nullptr && tail == TAIL_ENCRYPT) LIMB_FORWARD(L, LIFTED, TAIL_ENCRYPT, ep); \
+        if (ls != nullptr && tail == TAIL_ENCRYPT) LIMB_FORWARD_POINTS(L, POINTS_FEW(L), LIFTED, TAIL_ENCRYPT, ep); /* one message */ \
         else if (ls != nullptr) LIMB_FORWARD(L, LIFTED, TAIL_NONE, ep);    \
         else if (tail == TAIL_SUB_SCALE && list != nullptr) LIMB_SOURCES(L, TAIL_SUB_SCALE_LIST, epl); \
         else if (tail == TAIL_SUB_SCALE) LIMB_SOURCES(L, TAIL_SUB_SCALE, ep);  \
@@ -323,7 +323,7 @@ void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, c
 #define LIMB_RING(L)                                                   \
     do {                                                               \
         if (load == LOAD_ROTATED) LIMB_INVERSE(L, LOAD_ROTATED);       \
-        else if (load == LOAD_DECRYPT) LIMB_INVERSE(L, LOAD_DECRYPT);  \
+        else if (load == LOAD_DECRYPT) LIMB_INVERSE_POINTS(L, POINTS_FEW(L), LOAD_DECRYPT); /* one or two limbs */ \
         else LIMB_INVERSE(L, LOAD_PLAIN);                              \
     } while (0)
     switch (LR) {

@@ -9,14 +9,24 @@ def _forms(kernel, ints):
     """Template arguments (the leading integers) of every instantiation of a kernel, from the library's symbol names."""
     with open(os.path.join(PKG_DIR, "libhemm.so"), "rb") as f:
         names = f.read()
-    mangled = re.compile(b"%d%sI%s" % (len(kernel), kernel.encode(), b"L[ib]([0-9]+)E" * ints))
-    return {tuple(int(x) for x in m) for m in mangled.findall(names)}
+    mangled = re.compile(b"%d%sI%s" % (len(kernel), kernel.encode(), b"L[ib](n?[0-9]+)E" * ints))
+    return {tuple(int(x.replace(b"n", b"-")) for x in m) for m in mangled.findall(names)}
 
 
 def test_row_passes():
     """Log2 of the rows (0: from the argument), points per thread, inverse."""
     points = {(4, 0), (8, 0), (16, 0), (4, 1), (8, 1)}
     assert _forms("ntt16_rows_kernel", 3) == {(lr,) + p for lr in (0, 8) for p in points}
+    # what a decryption reads (the last argument, 2) is one or two limbs
+    assert {f for f in _forms("ntt16_rows_kernel", 5) if f[4] == 2} == {(lr, 4, 1, 0, 2) for lr in (0, 8)}
+
+
+def test_one_launch_transforms():
+    """Log2 of the rows, points per thread, what is loaded resp. the tail: four points of 2^12 for few limbs, which an encryption's (tail 2)
+    and a decryption's (load 2) always are."""
+    assert {f[:2] for f in _forms("ntt_limb_inverse_kernel", 3)} == {(2, 8), (3, 8), (4, 4), (4, 8), (5, 8), (6, 16)}
+    assert {f[:2] for f in _forms("ntt_limb_inverse_kernel", 3) if f[2] == 2} == {(2, 8), (3, 8), (4, 4)}
+    assert {f[:2] for f in _forms("ntt_limb_forward_kernel", 4) if f[3] == 2} == {(2, 8), (3, 8), (4, 4)}
 
 
 def test_column_passes():
