@@ -11,7 +11,7 @@
 // and mirrored for the inverse.  Each workgroup owns 4096 points, R rows of 4096 / R columns (or 16 rows, 8 or 4 with eight or four
 // points per thread); a thread keeps 16 residues in registers, or two or four lanes of a wavefront 8 or 4 each, runs a block of up to four
 // stages on them, swaps through LDS once and runs the second block.  All global accesses
-// are segments of at least 128 bytes shared by adjacent lanes.
+// are segments of at least 128 bytes shared by adjacent lanes, 64 in the half slabs of 2^16 points.
 //
 // Rings of 2^10 .. 2^12 points, and large batches of 2^13 and 2^14, take one launch (ntt_limb.hip), the smallest rings
 // (2^6 .. 2^9, small-parameter tests) a plain LDS kernel; the butterfly network is the same for all, so residues are identical for every N.
@@ -246,7 +246,7 @@ __global__ __launch_bounds__((4096 >> H) / P) __attribute__((amdgpu_waves_per_eu
     const Tw *tw = tw_all + ((size_t)prime << (8 + LR));
     const int dg = (int)table_byte(cs.digit_of, limb), n_src = cs.d[dg].n_src;
     // The sources are read through a buffer resource: base (the polynomial's source limbs; far below 4 GiB), source slot
-    // and slab row sit in scalar registers, a thread supplies one 32-bit offset for all of its 8 n_src loads.
+    // and slab row sit in scalar registers, a thread supplies one 32-bit offset for all of its P n_src loads.
     const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(cs.d[dg].src + (size_t)poly * cs.d[dg].src_poly_stride), 0, -1, 0x00020000);
     const Cst *hat = cs.d[dg].hat + prime;
@@ -525,23 +525,22 @@ void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, c
 
 // ---- launches of single passes (rings of 2^13 points and more) -------------------------------------------------------
 // Which passes give a thread four or eight points instead of sixteen (ntt_device.h, Lanes): few points only where the launch leaves the
-// chip part empty, since in a full one the twiddles and addresses of each lane of a block are work for nothing.  Transforms of
-// 2^16 points, us with sixteen / eight / four points in that pass (workgroups of 4096 points):
-//   workgroups                  64              128        256              384              512              768             1024
-//   columns, forward, 60 bits   12.7/12.1/12.0  13.7/13.1  19.6/18.5/18.1   26.2/24.9/24.3   27.5/26.5/26.0   28.6/28.9/28.3  33.9/34.8/35.0
-//                     42 bits    9.6/10.3/10.8  11.9/12.2  16.5/16.4/16.0   21.6/21.7/21.4   24.4/24.3/23.9   22.6/23.1/23.5  26.9/27.4/28.5
-//            inverse, 60 bits   13.1/12.6/12.2  14.0/13.9  20.2/19.1/18.4   28.0/25.8/25.6   29.1/28.5/28.7   31.6/31.9/31.5  38.8/39.1/39.2
-//                     42 bits    9.7/10.7/11.0  11.8/12.1  16.5/16.6/16.4   22.1/21.9/22.1   25.5/25.4/25.4   24.0/24.2/25.0  27.5/28.4/30.4
-//   rows, forward,    60 bits   13.4/12.1/11.0  13.7/13.1  19.6/18.5/17.9   26.5/24.9/24.4   27.8/26.5/25.9   28.6/28.4/27.8  33.9/34.1/34.3
-//                     42 bits   10.1/10.3/10.3  11.9/11.9  17.3/16.4/16.2   21.9/21.7/21.1   24.6/24.3/23.9   22.6/23.1/22.8  26.9/27.8/27.1
-//         inverse,    60 bits       12.6/11.6   14.0/13.4       19.1/18.6        25.8/25.5        28.5/28.1        31.6/30.8       38.8/37.6
-//                     42 bits       10.7/10.1   11.8/12.1       16.6/16.4        21.9/21.7        25.4/24.8        24.0/23.8       27.5/27.9
-//         inverse, 2^15 points, 42  10.2/10.4   11.7/11.9       16.6/16.6        21.4/21.3        26.0/25.2        23.3/23.9       26.7/28.2
-// With the conversions (below): rotation on 2^13 points 34.1 -> 30.2 us, inverse transform of 35 limbs of 2^14 points 12.9 -> 12.2, product at
-// level 9 109.6 -> 106.1; the products of 128 x 128 matrices the same to 1 %.
+// chip part empty, since in a full one the twiddles and addresses of each lane of a block are work for nothing.  All figures down to
+// narrower_slabs but the one marked there: us of device time a call, calls queued, one build with its lines moved.
+// Transforms of 2^16 points with sixteen / eight / four points in that pass (workgroups of 4096 points, columns on whole slabs):
+//   workgroups                 64               128              256              384              512              768              1024
+//   columns, forward, 60 bits  11.1/10.6/10.4   13.7/13.2/13.1   19.3/18.9/18.5   25.6/25.6/25.2   27.1/27.1/26.6   29.9/29.7/29.9   35.6/35.6/36.3
+//                     42 bits   9.3/ 9.1/ 9.0   11.6/11.3/11.3   16.7/16.3/16.0   22.2/21.9/21.8   24.9/24.5/24.4   23.8/23.1/24.5   27.9/27.9/29.9
+//            inverse, 60 bits  11.9/11.2/11.0   14.6/14.0/13.8   20.2/19.6/19.1   27.2/26.8/26.9   29.7/28.9/28.8   32.4/31.9/32.4   39.2/39.1/40.2
+//                     42 bits   9.5/ 9.2/ 9.4   12.0/11.7/11.9   17.1/16.8/16.6   22.6/22.7/22.9   26.0/25.6/25.8   24.7/24.3/25.8   28.9/28.8/31.0
+//   rows,    forward, 60 bits  11.9/10.7/ 9.5   13.8/12.6/12.3   19.2/19.0/18.6   25.3/24.9/24.5   27.6/27.5/26.7   30.1/29.7/29.5   35.9/36.1/36.2
+//                     42 bits  10.0/ 9.1/ 8.3   11.8/10.9/10.7   17.9/16.3/16.1   22.4/21.3/21.4   25.2/24.5/24.5   23.9/23.6/24.0   28.0/27.5/28.5
+//            inverse, 60 bits  12.3/10.8/ 9.7   14.3/12.7/12.5   19.9/19.4/19.3   26.5/25.8/25.6   30.7/30.0/28.9   33.6/32.4/32.8   39.8/39.6/38.7
+//                     42 bits  10.2/ 9.3/ 8.5   12.0/11.0/11.1   17.0/16.7/16.5   22.8/22.1/21.9   26.6/26.2/25.7   25.2/24.7/25.0   29.0/29.1/29.5
 static bool few_for_columns(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 512; }
-// Row passes: eight points beyond the line of four, where four put more workgroups on a CU than are resident; encodings of 2^14 points
-// leave four earlier and eight for sixteen at 640.  us with sixteen / eight / four points, second figure of each pair 42 bits:
+// Row passes: four points have eight wavefronts per SIMD, all resident up to 512 workgroups of 4096 points, and lead up to 640; eight points
+// lead from there to about 1000.  Encodings of 2^14 points leave four at 512 and eight, for sixteen, at 640.  us with sixteen / eight /
+// four points, the second figure of each pair 42 bits:
 //   workgroups                        544                              640                              768                              896
 //   forward, 2^16 points   33.3/32.8/31.5 28.5/28.1/27.2  28.5/27.3/27.0 24.4/23.2/23.5  30.1/29.7/29.5 23.9/23.6/24.0  34.5/33.6/33.6 26.8/25.5/26.7
 //            2^15          32.5/31.6/30.6 28.4/27.2/26.8  29.5/28.0/27.7 25.7/24.6/24.6  28.8/28.6/28.7 23.5/23.2/23.8  33.3/32.3/33.0 25.9/25.0/26.1
@@ -559,19 +558,20 @@ static int points_for_rows(const hemm_context *c, int limbs, bool inverse, int t
 }
 
 // Passes that begin in a basis conversion or a lift, on rings below 2^16 points: four points where every CU has one workgroup at most, eight
-// otherwise (six waves per SIMD); rotations of 2^14 points at level 6 (48 workgroups in a launch of conversions) 42.2 -> 39.9 us, at level 12 51.6 ->
-// 50.4.  At 2^16 points four points go with the half slabs of narrower_slabs, eight with whole ones.
+// otherwise (six waves per SIMD).  Rotations of 2^13 / 2^14 / 2^15 points at level 6 of 42 bits with eight / four points 33.6/32.2, 36.7/35.1,
+// 45.9/45.6, at level 8 of 60 bits 37.8/36.0, 46.7/44.8, 61.8/61.2; encodings of nine messages of six limbs 17.0/16.7, 23.0/22.5, 31.6/31.7 (beyond
+// the line).  At 2^16 points four points go with the half slabs of narrower_slabs, eight with whole ones.
 static bool few_for_conversions(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 256; }
 
 // Column passes of few workgroups are bound by the instructions of the few CUs they are on: slabs of a half or a
 // quarter of the columns (1, 2: as powers of two) put them on as many more CUs.  At 2^16 points a half slab is eight columns, segments of
 // 64 bytes, and pays where both halves of a line are on one XCD (Slab::slab); on two of them rotations lost 3 %, and quarters gain nothing
-// more.  Transforms of 2^16 points, us (forward, inverse) with whole / half slabs, 60 and 42 bits:
-//   workgroups   64                              128                               192                              384                               512
-//   60 bits      10.9/10.0 11.0/9.9   12.6/12.0 13.3/12.4   13.0/11.9 13.5/12.5   23.8/22.9 25.3/24.0   24.8/25.1 27.3/27.5
-//   42 bits       9.7/ 9.6  9.7/9.9   11.8/11.1 12.1/11.4   11.6/11.0 12.3/11.6   21.0/20.3 21.9/20.9   23.5/23.6 24.5/24.5
+// more.  Transforms of 2^16 points (forward, inverse) with whole / half slabs of four points, 60 and 42 bits:
+//   workgroups   64                             128                             192                             256                             384                             448                             512
+//   60 bits      10.4/ 9.5 11.0/ 9.7   13.0/12.3 13.8/12.6   15.6/15.9 16.3/16.5   18.2/18.3 19.0/18.9   25.0/24.1 26.6/25.3   26.2/26.4 28.0/28.3   26.5/26.6 28.6/28.9
+//   42 bits       9.0/ 8.4  9.4/ 8.5   11.3/10.7 11.9/11.1   13.6/13.7 14.2/14.3   16.0/16.1 16.6/16.6   21.9/21.3 22.7/21.9   23.5/23.8 24.5/24.7   24.6/24.9 25.7/25.7
 // Conversions take half slabs further, their whole ones being bound by the three workgroups that a CU holds in step.  Rotations and products of
-// 2^16 points, us, with none / up to 256 / 400 / 700 / 1000 workgroups of conversions on half slabs of four points:
+// 2^16 points (whole calls with their host time, an earlier build), us, with none / up to 256 / 400 / 700 / 1000 workgroups of conversions on half slabs of four points:
 //   42 bits, level  4 (160 and fewer)   54.6/50.0/50.0/50.0/50.0   85.2/ 79.5/ 79.5/ 79.5/ 79.5
 //                   8 (up to 256, 288)  67.8/67.8/64.3/64.0/64.1  100.3/100.3/ 96.8/ 96.6/ 95.9
 //                  10 (400, 528)        80.8/80.8/80.1/76.2/76.3  117.3/117.3/114.5/110.8/111.1
@@ -579,13 +579,17 @@ static bool few_for_conversions(const hemm_context *c, int limbs) { return (size
 //                  18 (608, 784)       117.3/117.3/117.0/114.9/113.9  170.3/170.3/170.4/168.2/167.4
 //                  23 (768, 960)       130.2/130.2/130.2/130.6/131.6  191.2/191.2/191.5/191.6/192.7
 // The products of matrices, whose large conversions run beside other chains, are 1 - 3 % slower with all of them on half slabs.
-// Smaller rings, transforms (forward/inverse, us) with whole / with narrower slabs:
-//   limbs              1                 4                 16                32                48                64
-//   2^13 points        9.2/9.5 8.4/8.8   9.2/9.8 8.5/8.9   9.6/10.1 8.8/9.2  10.4/11.0 9.6/10.0   11.4/11.9 11.2/11.6  (one launch)
-//   2^14               9.4/10.0 8.5/8.9  9.6/10.2 8.6/9.2  10.8/11.2 10.1/10.4 12.6/13.3 12.7/13.0 15.9/16.4 15.7/16.2 17.9/18.5 17.8/18.2
-//   2^15               9.8/10.5 8.9/9.2  10.3/10.8 9.5/9.7 13.0/13.3 12.3/12.1 18.2/18.7 18.9/18.3 25.4/26.3 24.5/24.9 30.4/31.3 30.7/30.9
-// (plain forward passes of 2^15 points keep whole slabs above 128 workgroups.)  Rotations of 6 / 12 / 24 limbs, 42 bits: 2^13 41.2/43.6/98.7 ->
-// 35.6/38.4/92.9, 2^14 43.9/50.8/114.7 -> 38.5/47.2/112.0, 2^15 50.3/68.0/145.1 -> 46.3/62.8/142.3; products alike.
+// Smaller rings, transforms of 42 bits (forward, inverse) with whole slabs of sixteen points / half slabs / quarter slabs of four:
+//   limbs         1                             4                             16                            32                              48                                64
+//   2^13 points   7.5/6.8/6.6  7.8/6.9/6.7   7.8/7.0/6.7  8.1/7.1/6.7   8.1/7.4/7.2  8.5/7.5/7.3    8.9/ 8.3/ 7.9  9.2/ 8.5/ 8.0   10.2/ 9.8/ 9.5 10.8/10.1/ 9.7   (one launch)
+//   2^14          7.6/6.9/6.6  8.0/7.2/6.7   7.9/7.1/6.8  8.2/7.3/6.8   9.2/8.2/7.9  9.6/8.4/8.0   11.6/10.5/10.4 12.3/10.9/10.8   14.5/13.2/13.1 15.2/13.9/13.5   17.5/15.7/15.7 19.3/16.3/16.4
+//   (35 / 80 limbs 12.6/11.7/11.5 13.2/12.3/12.0, 20.2/18.6/18.2 22.2/19.5/18.9: the line of quarter slabs, drawn with eight points, lies below its place)
+// Transforms of 2^15 points, whole slabs of sixteen / of four points / half slabs of four:
+//   limbs      1                               16                                 32                                 40                                 48                                 64
+//   42 bits    7.9/7.7/7.0   8.3/8.2/7.3   11.3/11.1/10.5 11.9/11.8/11.0   16.6/16.0/15.9 17.1/16.7/16.5   19.7/19.5/18.9 20.3/20.5/19.6   22.0/21.8/21.1 22.5/22.6/22.0   25.7/25.4/25.1 26.7/26.4/26.4
+//   60 bits    9.5/9.0/8.1  10.5/9.7/8.4   13.2/12.8/12.0 14.5/13.7/12.4   18.8/18.2/18.2 20.1/18.9/18.8   22.6/22.4/21.6 24.4/24.1/22.8   24.9/24.9/24.0 26.8/26.4/25.0   28.0/27.8/27.9 30.5/29.9/29.6
+// (plain forward passes of 2^15 points keep whole slabs above 128 workgroups: 24 limbs of 60 bits 15.4 against 15.7; from 40 limbs on half slabs
+// would lead.)
 static int narrower_slabs(const hemm_context *c, int limbs, bool plain = false, bool inverse = false) {
     const size_t wgs = (size_t)limbs * (c->N >> 12);
     if (c->logN == 16) return wgs <= (plain ? 384 : 768) ? 1 : 0;

@@ -422,7 +422,7 @@ __device__ __forceinline__ void lifted_inputs(const F &f, typename F::E (&x)[P],
         for (int k = 0; k < P; k++) x[k] = f.from_canonical(lifted(ls, coef, index(k), m));
     }
 }
-// The eight coefficients of a thread as a basis conversion computed on the fly: coefficient k is sum_i v_i * hat_i mod q over
+// The P coefficients of a thread as a basis conversion computed on the fly: coefficient k is sum_i v_i * hat_i mod q over
 // the n_src <= NS source limbs (pre-scaled, the same sums as the stand-alone conversion kernels), read at voff + off(k) inside a
 // limb; so[i]: byte offset of source limb i.
 // The loads of the next coefficients, about CONV_LOADS residues, are in flight while the present one's products are taken: one

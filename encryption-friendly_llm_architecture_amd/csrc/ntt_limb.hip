@@ -238,9 +238,9 @@ __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_inverse_kernel(
     }
 }
 
-// points per thread: of 2^12 points four where every CU has one limb at most (sixteen wavefronts on it; forward with a conversion 11.5 -> 10.6 us,
-// product of two encrypted 32 x 32 tiles 497 -> 486), eight in larger launches, whose second twiddle and address cost more than that
-// (transforms of 256 / 512 / 4096 limbs of 42 bits 6.9/10.5/61.6 us with four, 6.7/9.9/56.2 with eight)
+// points per thread: of 2^12 points four where every CU has one limb at most (sixteen wavefronts on it), eight in larger launches, whose second
+// twiddle and address cost more than that.  Transforms, us of device time with eight / four: 64 limbs of 60 bits 7.2/6.9, 256 8.6/8.3, 264 11.6/11.9,
+// 1024 22.4/23.8, 4096 79.4/82.7; of 42 bits 5.5/5.6, 6.7/6.7, 8.7/9.2, 16.3/18.2, 56.5/61.1; rotations 42.2/41.1 (42 bits), 47.7/46.6 (60)
 #define POINTS(LR) ((LR) <= 5 ? 8 : 16)
 #define POINTS_FEW(LR) ((LR) == 4 ? 4 : POINTS(LR))
 static bool few_limbs(const size_t limbs) { return limbs <= 256; }
