@@ -229,7 +229,7 @@ def gpu_ntt(args, out):
     # launches moves that much, so the pair cannot exceed half of the HBM roofline on this figure)
     alg_bytes = limbs * 2 * LIMB_BYTES
     out["roofline_ntt"] = {
-        "kernel": "ntt16_cols_kernel<8, 16, false> + ntt16_rows_kernel<8, 16, false, 0, 0> (one forward transform of "
+        "kernel": "ntt16_cols_kernel<8, 16, 0, false> + ntt16_rows_kernel<8, 16, false, 0, 0> (one forward transform of "
                   "32x24 limbs = 2 launches), 60-bit primes / 42-bit primes",
         "bound": "hbm", "peak": HBM_PEAK_GBS, "unit": "GB/s",
         "achieved": alg_bytes / (fwd_ms * 1e-3) / 1e9, "frac": alg_bytes / (fwd_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
@@ -246,7 +246,7 @@ def gpu_ntt(args, out):
 # HBM bytes of one chain of the main loop at the shape below (its launches together), from two rocprofv3 --pmc runs of
 # `bench.py --roofline-only` (FETCH_SIZE, WRITE_SIZE), each scaled by what the same counter reads for the 1 GiB copy this mode also launches
 # (FETCH_SIZE x 2.0, WRITE_SIZE x 1.0): see profiles/main_loop_and_ntt_roofline_shapes.txt.
-CHAIN_TRAFFIC_BYTES = 1161650176
+CHAIN_TRAFFIC_BYTES = 1160764416
 
 
 def gpu_hoisted(args, out):

@@ -81,12 +81,12 @@ inline bool ring_has_fused_forms(const hemm_context *c) { return c->logN >= 10; 
 // what counts; one of 42 bits has fewer instructions to spread and gains earlier.  A launch may hold limbs of both, so the lines
 // lie where 60-bit ones have crossed over.  Forward, us in one launch / in two:
 //   2^13 points, limbs    1          8         48         64        128         768
-//     60 bits     11.2/ 9.3  11.6/ 9.8  12.2/12.3  12.2/13.1  12.9/19.0   36.9/46.7
-//     42 bits      8.0/ 8.1   8.1/ 9.7   8.2/10.4   8.6/11.3   9.0/16.8   24.5/37.6
+//     60 bits     10.7/ 7.3  10.9/ 7.5  11.3/10.6  11.5/11.5  12.4/18.5   36.2/45.4
+//     42 bits      8.0/ 6.6   8.2/ 6.7   8.5/ 9.5   8.8/10.3   9.4/16.6   27.2/38.0
 //   2^14 points, limbs    8         48         64         80         96        128        768
-//     60 bits     20.3/10.3  21.6/16.4  21.5/18.4  21.6/23.2  21.8/25.5  23.5/30.0  78.0/82.8
-//     42 bits     12.1/ 8.8  13.2/14.0  13.1/16.0  13.3/19.3  13.4/21.3  14.3/25.3  54.4/67.3
-// (inverse ones alike: 60 bits cross over at 48 to 64 resp. 64 to 96 limbs; 768 of 2^14 points and 60 bits 86.3/85.6).
+//     60 bits     18.2/ 7.8  19.1/15.2  19.4/17.9  19.6/21.0  19.9/23.7  22.3/28.9  73.5/81.6
+//     42 bits     12.4/ 7.0  13.2/13.3  13.6/15.7  13.8/18.5  14.0/20.9  15.1/25.7  55.0/68.6
+// (inverse ones of 60 bits cross over a little later: 64 limbs of 2^13 points 12.5/12.0, 80 of 2^14 22.2/22.3; 768 of those 82.7/88.1.)
 // plain: no conversion, tail or automorphism -- with them a workgroup of the 1024 threads a limb of 2^14 takes would spill.
 inline bool one_launch(const hemm_context *c, size_t limbs, bool plain) {
     return c->logN >= 10 && (c->logN <= 12 || (c->logN == 13 && limbs >= 64) || (c->logN == 14 && plain && limbs >= 96));
