@@ -92,9 +92,10 @@ public:
     // `level` from a higher one; the masks of the first stage are then encoded at Delta_(level-1) q_level /
     // Delta_(scale level), which lands the result on the fixed scale of level - 1 without a levelDown in front.
     // first_stage = 2: only the second stage; `in` is then what a first stage from `level` left at level - 1.
+    // last_stage = 1: only the first one, which leaves `out` at level - 1.
     void diagonalTransformTwoStage(const HomEvaluator &eval, const u64 *in, size_t n_jobs, u64 level, const MaskKind *kinds,
                                    const TileTensorShape *shapes, u64 *out, const u64 *scale_levels = nullptr,
-                                   int first_stage = 1);
+                                   int first_stage = 1, int last_stage = 2);
     // The complex packing (by rows for PackedVertical, by columns for PackedHorizontal) and the FIRST stage of the
     // two-stage transform of `kind` as one linear map on the slots -- one hoisted sum, one mask level: the term that
     // rotates by a slots carries sum over (stage rotation r, packing shift e) with r + e = a of

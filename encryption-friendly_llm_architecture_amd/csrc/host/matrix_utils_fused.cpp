@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <functional>
 #include <map>
 #include <set>
 
@@ -604,17 +605,17 @@ Ciphertext MatrixTransformer::lowerAndTransformFused(const HomEvaluator &eval, c
 
 void MatrixTransformer::diagonalTransformTwoStage(const HomEvaluator &eval, const u64 *in, size_t n_jobs, u64 level,
                                                   const MaskKind *kinds, const TileTensorShape *shapes, u64 *out,
-                                                  const u64 *scale_levels, int first_stage) {
+                                                  const u64 *scale_levels, int first_stage, int last_stage) {
     const Context &c = eval.getContext();
     if (level < 2) throw std::invalid_argument("[diagonalTransform] level >= 2 is needed.");
     const u64 N = c->N;
-    if (first_stage != 1 && first_stage != 2) throw std::invalid_argument("[diagonalTransform] stage 1 or 2");
+    if (first_stage < 1 || last_stage > 2 || first_stage > last_stage) throw std::invalid_argument("[diagonalTransform] stage 1 or 2");
     DeviceBuffer mid;   // after stage 1: level - 1
-    if (first_stage == 1) mid = DeviceBuffer(c, n_jobs * 2 * level * N);
-    for (int stage = first_stage; stage <= 2; stage++) {
+    if (first_stage < last_stage) mid = DeviceBuffer(c, n_jobs * 2 * level * N);
+    for (int stage = first_stage; stage <= last_stage; stage++) {
         const u64 lvl = stage == 1 ? level : level - 1, nq = lvl + 1, E = nq + c->nP, ctw = 2 * nq * N;
         const u64 *src = stage == first_stage ? in : mid.data();
-        u64 *dst = stage == 1 ? mid.data() : out;
+        u64 *dst = stage == last_stage ? out : mid.data();
         auto from_of = [&](size_t q) -> u64 { return stage == 1 && scale_levels ? scale_levels[q] : 0; };
         // One rotation source per job (a single ModUp).  A stage's rotation by r cells wraps inside the tile, so it is
         //   main_r * rho^(r step)(X) + wrap_r * rho^(r step - tile side)(X):
@@ -1636,34 +1637,43 @@ CtxtTensor multMatMatComplexPackedFused(const HomEvaluator &eval, const Bootstra
                 return t;
             };
             OwnWays ways(c);
-            ways.toSide();
-            {
-                const MaskKind kind = MaskKind::PackedVertical;
-                if (separate) {   // truncated to T+4, packed by rows (T+3), tau in two stages (T+1)
-                    const u64 Lb = T + 4;
-                    const DeviceBuffer jb = truncated(b.get(), Lb);
-                    DeviceBuffer pk(c, 2 * Lb * N);
+            const MaskKind kind_a = MaskKind::PackedHorizontal, kind_b = MaskKind::PackedVertical;
+            DeviceBuffer ja, jb, pa, pb, ma, mb;   // truncated, packed, after the first transform stage
+            std::vector<std::function<void()>> way_a, way_b;
+            if (separate) {   // truncated to T+4, packed by rows (T+3), tau in two stages (T+1)
+                const u64 Lb = T + 4;
+                way_b.push_back([&, Lb] {
+                    jb = truncated(b.get(), Lb);
+                    pb = DeviceBuffer(c, 2 * Lb * N);
                     const bool by_rows = true;
-                    u64 *const out = pk.data();
+                    u64 *const out = pb.data();
                     tr.complexPackingBatch(eval, jb.data(), 1, Lb, &by_rows, w, &out, &lb);
-                    tr.diagonalTransformTwoStage(eval, pk.data(), 1, Lb - 1, &kind, &shape_b, tb.data());
-                } else {          // truncated to T+3, packing + first stage (T+2), second stage (T+1)
-                    const u64 Lb = T + 3;
-                    const DeviceBuffer jb = truncated(b.get(), Lb);
-                    DeviceBuffer mid(c, 2 * Lb * N);
-                    tr.packingStageOne(eval, jb.data(), 1, Lb, &kind, &shape_b, mid.data(), &lb);
-                    tr.diagonalTransformTwoStage(eval, mid.data(), 1, Lb, &kind, &shape_b, tb.data(), nullptr, 2);
-                }
+                });
+                way_b.push_back([&, Lb] {
+                    mb = DeviceBuffer(c, 2 * (Lb - 1) * N);
+                    tr.diagonalTransformTwoStage(eval, pb.data(), 1, Lb - 1, &kind_b, &shape_b, mb.data(), nullptr, 1, 1);
+                });
+                way_b.push_back([&, Lb] { tr.diagonalTransformTwoStage(eval, mb.data(), 1, Lb - 1, &kind_b, &shape_b, tb.data(), nullptr, 2); });
+            } else {          // truncated to T+3, packing + first stage (T+2), second stage (T+1)
+                const u64 Lb = T + 3;
+                way_b.push_back([&, Lb] {
+                    jb = truncated(b.get(), Lb);
+                    mb = DeviceBuffer(c, 2 * Lb * N);
+                    tr.packingStageOne(eval, jb.data(), 1, Lb, &kind_b, &shape_b, mb.data(), &lb);
+                });
+                way_b.push_back([&, Lb] { tr.diagonalTransformTwoStage(eval, mb.data(), 1, Lb, &kind_b, &shape_b, tb.data(), nullptr, 2); });
             }
-            ways.toOwn();
             if (separate) {       // truncated to T+5, packed by columns (T+4), sigma in two stages (T+2)
                 const u64 La = T + 5;
-                const DeviceBuffer ja = truncated(a.get(), La);
-                DeviceBuffer pk(c, 2 * La * N);
-                const bool by_rows = false;
-                const MaskKind kind = MaskKind::PackedHorizontal;
-                u64 *const out = pk.data();
-                if (halves) {
+                way_a.push_back([&, La] {
+                    ja = truncated(a.get(), La);
+                    pa = DeviceBuffer(c, 2 * La * N);
+                    const bool by_rows = false;
+                    u64 *const out = pa.data();
+                    if (!halves) {
+                        tr.complexPackingBatch(eval, ja.data(), 1, La, &by_rows, w, &out, &la);
+                        return;
+                    }
                     tr.useChainOf(c);
                     const i64 half = k / 2 * w;
                     std::vector<std::pair<i64, const Plaintext *>> parts;
@@ -1672,21 +1682,35 @@ CtxtTensor multMatMatComplexPackedFused(const HomEvaluator &eval, const Bootstra
                             parts.push_back({(h == 0 ? 0 : h == 1 ? -half : half) + (e == 0 ? 0 : e == 1 ? 1 : -1),
                                              &packingMask(tr, c, false, w, La, 3 * h + e, la)});
                     maskedRotations(eval, ja.data(), La, parts, out);
-                } else {
-                    tr.complexPackingBatch(eval, ja.data(), 1, La, &by_rows, w, &out, &la);
-                }
-                tr.diagonalTransformTwoStage(eval, pk.data(), 1, La - 1, &kind, &shape_a, sa.data());
+                });
+                way_a.push_back([&, La] {
+                    ma = DeviceBuffer(c, 2 * (La - 1) * N);
+                    tr.diagonalTransformTwoStage(eval, pa.data(), 1, La - 1, &kind_a, &shape_a, ma.data(), nullptr, 1, 1);
+                });
+                way_a.push_back([&, La] { tr.diagonalTransformTwoStage(eval, ma.data(), 1, La - 1, &kind_a, &shape_a, sa.data(), nullptr, 2); });
             } else if (la >= T + 4) {   // truncated to T+4, packing + first stage (T+3), second stage (T+2)
                 const u64 La = T + 4;
-                const DeviceBuffer ja = truncated(a.get(), La);
-                DeviceBuffer mid(c, 2 * La * N);
-                const MaskKind kind = MaskKind::PackedHorizontal;
-                tr.packingStageOne(eval, ja.data(), 1, La, &kind, &shape_a, mid.data(), &la);
-                tr.diagonalTransformTwoStage(eval, mid.data(), 1, La, &kind, &shape_a, sa.data(), nullptr, 2);
+                way_a.push_back([&, La] {
+                    ja = truncated(a.get(), La);
+                    ma = DeviceBuffer(c, 2 * La * N);
+                    tr.packingStageOne(eval, ja.data(), 1, La, &kind_a, &shape_a, ma.data(), &la);
+                });
+                way_a.push_back([&, La] { tr.diagonalTransformTwoStage(eval, ma.data(), 1, La, &kind_a, &shape_a, sa.data(), nullptr, 2); });
             } else {              // at T+3: packing and sigma as one composite one-stage transform (T+2)
-                const MaskKind kind = MaskKind::PackingHorizontal;
-                tr.diagonalTransformBatch(eval, a.get().buf_.data(), 1, T + 3, &kind, &shape_a, sa.data());
+                way_a.push_back([&] {
+                    const MaskKind kind = MaskKind::PackingHorizontal;
+                    tr.diagonalTransformBatch(eval, a.get().buf_.data(), 1, T + 3, &kind, &shape_a, sa.data());
+                });
             }
+            // Queued step by step in turn, the longer way of A first: a product that finds the GPU idle runs as far as the
+            // host has come, and one way queued whole holds the other's first launch back by its thirty launches.
+            for (size_t i = 0; i < std::max(way_a.size(), way_b.size()); i++) {
+                ways.toOwn();
+                if (i < way_a.size()) way_a[i]();
+                ways.toSide();
+                if (i < way_b.size()) way_b[i]();
+            }
+            ways.toOwn();
             ways.marksOn();
             c->mark("packing and transforms of A");
             if (!halves)
