@@ -18,6 +18,8 @@ u64 h_powmod(u64 a, u64 e, u64 q) {
     return r;
 }
 u64 h_invmod(u64 a, u64 q) { return h_powmod(a % q, q - 2, q); }
+// a constant as near60_add_mul takes it: the value cut at bit 29, its low part in the low word
+static u64 near60_cut(u64 w) { return (w & ((1ull << 29) - 1)) | (w >> 29 << 32); }
 static u64 h_shoup(u64 w, u64 q) { return (u64)(((u128)w << 64) / q); }
 
 static bool h_is_prime(u64 n) {
@@ -128,6 +130,7 @@ hemm_context *hemm_context_build(int logN, int nQ, int nP, const u64 *primes, in
         // table is the N twiddles as doubles, packed into the first half of the prime's region (8 bytes per twiddle
         // instead of 16: the row passes read as many twiddle bytes as data, and the quotient w / q costs one multiply).
         const bool fp = ring_has_fused_forms(c) && (q >> 44) == 0;
+        const bool near = ring_has_fused_forms(c) && near_2_60(q);   // w and 2^32 w mod q (Near60Field)
         auto as_bits = [](double d) {
             u64 b;
             memcpy(&b, &d, 8);
@@ -139,6 +142,13 @@ hemm_context *hemm_context_build(int logN, int nQ, int nP, const u64 *primes, in
                 wt[j] = as_bits((double)pw[r]);
                 iwt[j] = as_bits((double)ipw[r]);
                 wt[N + j] = iwt[N + j] = 0;
+                continue;
+            }
+            if (near) {
+                wt[2 * j] = near60_cut(pw[r]);
+                wt[2 * j + 1] = near60_cut(h_mulmod(pw[r], 1ull << 32, q));
+                iwt[2 * j] = near60_cut(ipw[r]);
+                iwt[2 * j + 1] = near60_cut(h_mulmod(ipw[r], 1ull << 32, q));
                 continue;
             }
             wt[2 * j] = pw[r];

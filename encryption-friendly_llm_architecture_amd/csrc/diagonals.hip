@@ -81,7 +81,7 @@ __global__ __launch_bounds__(256) void diagonal_tables_kernel(const double2 *__r
     if (fp[4 * prime] != 0.0)
         transform_runs(FpField(modq, nullptr, nullptr, fp, prime), buf, tw, w, (int)log_w + 1);
     else
-        transform_runs(IntFieldT<true>(modq, nullptr, nullptr, fp, prime), buf, tw, w, (int)log_w + 1);
+        with_field_60(modq, nullptr, nullptr, fp, prime, [&](const auto f) { transform_runs(f, buf, tw, w, (int)log_w + 1); });
     // the rotation by nothing enters as P times the ciphertext, on the chain limbs: its diagonals carry the factor
     const bool own = j == 0, none = own && (int)e >= nq;
     for (u32 run = threadIdx.x; run < 2 * w; run += 256) {

@@ -34,7 +34,8 @@ struct hemm_context {
     std::vector<u64> psi;           // primitive 2N-th roots
     std::vector<ModQ> modq;         // host copy
     // device tables, all [prime][N] unless noted
-    u64 *d_w, *d_iw;                // (psi^bitrev(i), Shoup quotient), forward and inverse transform
+    u64 *d_w, *d_iw;                // (psi^bitrev(i), Shoup quotient), forward and inverse transform; N >= 2^10: doubles of primes below
+                                    // 2^44, of primes just below 2^60 (w, 2^32 w mod q), both cut at bit 29
     u64 *d_rw, *d_irw;              // N >= 2^10: the twiddles of the row passes' inner radix-16 blocks in the order their
                                     // threads read them, entry (r * 15 + 2^l - 1 + g) * 16 + c = entry
                                     // ((16 (N / 256 + r) + c) << l) + g of d_w / d_iw (nullptr for other ring sizes)

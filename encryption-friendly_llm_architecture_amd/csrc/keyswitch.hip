@@ -419,17 +419,17 @@ __device__ __forceinline__ void sum_done(const u64 (&rb)[2], const u64 (&ra)[2],
         if (fp_limb)
             rows_under_products(FpField(modq, nullptr, nullptr, fp, prime), rb, ra, cb, ca, ob, oa, lds, tw, logN - 8, 2 * chunk, cst);
         else
-            rows_under_products(IntFieldT<true>(modq, nullptr, nullptr, fp, prime), rb, ra, cb, ca, ob, oa, lds, tw, logN - 8, 2 * chunk, cst);
+            with_field_60(modq, nullptr, nullptr, fp, prime,
+                          [&](const auto f) { rows_under_products(f, rb, ra, cb, ca, ob, oa, lds, tw, logN - 8, 2 * chunk, cst); });
     } else {
         u64 *yb = y + (((size_t)o * 2 + 0) * E + j) * N, *ya = y + (((size_t)o * 2 + 1) * E + j) * N;
         if (rows.takes_rows(j)) {
             const Tw *tw = rows.tw + ((size_t)prime << logN);
             if (fp_limb)
                 rows_of_products(FpField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
-            else if ((modq[prime].q >> 60) == 0)
-                rows_of_products(IntFieldT<true>(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
             else
-                rows_of_products(IntField(modq, nullptr, nullptr, fp, prime), rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk);
+                with_int_field(modq, nullptr, nullptr, fp, prime,
+                               [&](const auto f) { rows_of_products(f, rb, ra, yb + first, ya + first, lds, tw, logN - 8, 2 * chunk); });
             return;
         }
         stream_store2(yb + n, rb[0], rb[1]);
@@ -711,8 +711,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(B == 3 ? 3 
         switched_pair<true, B>(FpField(modq, nullptr, nullptr, fp, prime), fm, m, pmod, keyed, own, sw, tw, digits, prime, j, chunk, nq, E, n_full,
                                logN, rb, ra);
     else
-        switched_pair<false, B>(IntFieldT<true>(modq, nullptr, nullptr, fp, prime), fm, m, pmod, keyed, own, sw, tw, digits, prime, j, chunk, nq, E,
-                                n_full, logN, rb, ra);
+        with_field_60(modq, nullptr, nullptr, fp, prime, [&](const auto f) {
+            switched_pair<false, B>(f, fm, m, pmod, keyed, own, sw, tw, digits, prime, j, chunk, nq, E, n_full, logN, rb, ra);
+        });
     sum_done(rb, ra, y, modq, fp, prime, fm.q != 0.0, 0u, j, chunk, chunk * 512 + 2 * threadIdx.x, E, logN, rows);
 }
 

@@ -75,6 +75,26 @@ __device__ __forceinline__ u64 sub_multiple(u64 v, u32 e, u64 q) {
     asm("" : "+v"(top));
     return ((u64)top << 32) | (u32)t;
 }
+// ---- primes just below 2^60: q = 2^60 - delta, delta < 2^27 ------------------------------------------------------------------
+// What lies above bit 60 of a value counts delta times, so no quotient is estimated.  A constant w is kept with v = 2^32 w mod q, both cut at
+// bit 29 (near60_constant), and y w for a 64-bit y is yl w + yh v: four multiply-adds into accumulators s0 and s1 of weights 1 and 2^29.
+// 2^29 s1 is 2^29 times its low word plus 2^61 = 2 delta times its high word, two multiply-adds more; y is never cut into pieces.
+#define NEAR60_DELTA (1ull << 27)
+__host__ __device__ __forceinline__ bool near_2_60(const u64 q) { return q < (1ull << 60) && (1ull << 60) - q < NEAR60_DELTA; }
+// u + y w, the product below 6.9q for y < 15.1q (5.8q for y < 8.1q): s0 < 2^29 (2^32 + yh), 2^29 sl < 2^61, 2 delta sh < 2^28 (2^31 + yh / 2)
+__device__ __forceinline__ u64 near60_add_mul(const u64 u, const u64 y, const u64 w, const u64 v, const u32 two_delta, const u32 two_29) {
+    const u32 yl = (u32)y, yh = (u32)(y >> 32);
+    const u64 s1 = (u64)yh * (u32)(v >> 32) + (u64)yl * (u32)(w >> 32);
+    u64 s0 = (u64)yl * (u32)w + u;
+    s0 += (u64)yh * (u32)v;
+    s0 += (u64)(u32)s1 * two_29;
+    return s0 + (u64)(u32)(s1 >> 32) * two_delta;
+}
+// any v to below q + 2^32: the four bits above 2^60 are taken off and count delta each
+__device__ __forceinline__ u64 near60_fold(const u64 v, const u32 delta) {
+    const u32 h = (u32)(v >> 32);
+    return (((u64)(h & 0x0fffffffu) << 32) | (u32)v) + (u64)(h >> 28) * delta;
+}
 // v < 32q (q < 2^59) to [0, q)
 __device__ __forceinline__ u64 reduce_below_32q(u64 v, const u64 q) {
 #pragma unroll

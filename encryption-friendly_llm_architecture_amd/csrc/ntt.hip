@@ -156,17 +156,6 @@ __device__ __forceinline__ void cols_body(const __amdgpu_buffer_rsrc_t limb, con
     }
 }
 
-template <class F, int LR, int P, int H, bool INV>
-__device__ __forceinline__ void cols_int(const __amdgpu_buffer_rsrc_t base, const Tw *__restrict__ tw, const ModQ *__restrict__ modq,
-                                         const u64 *__restrict__ ninv, const u64 *__restrict__ ninv_s, const double *__restrict__ fp,
-                                         const int prime, const Tw *__restrict__ final_scale, const int limb, u64 *lds) {
-    F f(modq, ninv, ninv_s, fp, prime);
-    if (INV && final_scale != nullptr) {
-        f.ni = final_scale[limb].w;
-        f.nis = final_scale[limb].ws;
-    }
-    cols_body<LR, P, H, INV>(base, tw, f, lds);
-}
 template <int LR, int P, int H, bool INV>
 __global__ __launch_bounds__((4096 >> H) / P) void ntt16_cols_kernel(u64 *__restrict__ data, const Tw *__restrict__ tw_all,
                                                          const ModQ *__restrict__ modq,
@@ -183,15 +172,13 @@ __global__ __launch_bounds__((4096 >> H) / P) void ntt16_cols_kernel(u64 *__rest
     // conversion folds its (S/q_i)^-1 factor in here (the caller supplies (1/N)(S/q_i)^-1), at no cost
     if (fp[4 * prime] != 0.0) {
         FpField f(modq, ninv, ninv_s, fp, prime);
-        if (INV && final_scale != nullptr) {
-            f.ni = (double)final_scale[limb].w;
-            f.niinv = f.ni * f.qinv;
-        }
+        if (INV && final_scale != nullptr) f.set_scale(final_scale[limb]);
         cols_body<LR, P, H, INV>(base, tw, f, lds);
-    } else if ((modq[prime].q >> 60) != 0) {
-        cols_int<IntField, LR, P, H, INV>(base, tw, modq, ninv, ninv_s, fp, prime, final_scale, limb, lds);
     } else {
-        cols_int<IntFieldT<true>, LR, P, H, INV>(base, tw, modq, ninv, ninv_s, fp, prime, final_scale, limb, lds);
+        with_int_field(modq, ninv, ninv_s, fp, prime, [&](auto f) {
+            if (INV && final_scale != nullptr) f.set_scale(final_scale[limb]);
+            cols_body<LR, P, H, INV>(base, tw, f, lds);
+        });
     }
 }
 
@@ -263,7 +250,7 @@ __global__ __launch_bounds__((4096 >> H) / P) __attribute__((amdgpu_waves_per_eu
     if (fp[4 * prime] != 0.0)
         cols_converted_body<LR, P, H, NS>(base, tw, FpField(modq, ninv, ninv_s, fp, prime), lds, src, so, h, n_src, m);
     else   // (the sums take primes below 2^60)
-        cols_converted_body<LR, P, H, NS>(base, tw, IntFieldT<true>(modq, ninv, ninv_s, fp, prime), lds, src, so, h, n_src, m);
+        with_field_60(modq, ninv, ninv_s, fp, prime, [&](const auto f) { cols_converted_body<LR, P, H, NS>(base, tw, f, lds, src, so, h, n_src, m); });
 }
 
 // Forward pass 1 whose input is the rounded coefficients of an encoding, the same for every limb of a polynomial: reduced
@@ -292,12 +279,9 @@ __global__ __launch_bounds__((4096 >> H) / P) void ntt16_cols_lifted_kernel(u64 
     const ModQ m = modq[prime];
     if (fp[4 * prime] != 0.0)
         cols_lifted_body<LR, P, H>(base, tw, FpField(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
-    else if ((m.q >> 60) != 0)
-        cols_lifted_body<LR, P, H>(base, tw, IntField(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
     else
-        cols_lifted_body<LR, P, H>(base, tw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, ls, coef, m);
+        with_int_field(modq, nullptr, nullptr, fp, prime, [&](const auto f) { cols_lifted_body<LR, P, H>(base, tw, f, lds, ls, coef, m); });
 }
-
 // ------------------------------------------------------------------------------------------
 // Column-slab kernel of a ModDown (or any conversion of a few source limbs): for one (polynomial, 16-column slab) a
 // workgroup runs the second pass of the inverse transform of every source limb, keeps the canonical coefficients on
@@ -408,14 +392,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
         if (fp[4 * prime] != 0.0) {
             FpField f(modq, ninv, ninv_s, fp, prime);
-            f.ni = (double)fs.w;
-            f.niinv = f.ni * f.qinv;
+            f.set_scale(fs);
             slab_inverse(limb, v_inner, tw, f, lds, c[3]);
         } else {
-            IntField f(modq, ninv, ninv_s, fp, prime);
-            f.ni = fs.w;
-            f.nis = fs.ws;
-            slab_inverse(limb, v_inner, tw, f, lds, c[3]);
+            with_field_60(modq, ninv, ninv_s, fp, prime, [&](auto f) {
+                f.set_scale(fs);
+                slab_inverse(limb, v_inner, tw, f, lds, c[3]);
+            });
         }
         if (i < n_lds) {
 #pragma unroll
@@ -441,7 +424,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (fp[4 * prime] != 0.0)
             slab_forward<NREG, LDS>(limb, v_inner, tw, FpField(modq, ninv, ninv_s, fp, prime), lds, lsrc, hl, c, h, m);
         else
-            slab_forward<NREG, LDS>(limb, v_inner, tw, IntFieldT<true>(modq, ninv, ninv_s, fp, prime), lds, lsrc, hl, c, h, m);
+            with_field_60(modq, ninv, ninv_s, fp, prime, [&](const auto f) { slab_forward<NREG, LDS>(limb, v_inner, tw, f, lds, lsrc, hl, c, h, m); });
     }
 }
 
@@ -506,12 +489,10 @@ __global__ __launch_bounds__(256) void ntt16_rows_kernel(u64 *__restrict__ data,
     if (fp[4 * prime] != 0.0)
         rows_body<P, INV, TAIL, LOAD, false>(row, tw, rtw, FpField(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld, gal,
                                             sec);
-    else if ((modq[prime].q >> 60) != 0)
-        rows_body<P, INV, TAIL, LOAD, false>(row, tw, rtw, IntField(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld, gal,
-                                            sec);
     else
-        rows_body<P, INV, TAIL, LOAD, false>(row, tw, rtw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, log_r, r, mn, o, cst, ld,
-                                            gal, sec);
+        with_int_field(modq, nullptr, nullptr, fp, prime, [&](const auto f) {
+            rows_body<P, INV, TAIL, LOAD, false>(row, tw, rtw, f, lds, log_r, r, mn, o, cst, ld, gal, sec);
+        });
 }
 
 }  // namespace
@@ -526,7 +507,8 @@ void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, c
 // ---- launches of single passes (rings of 2^13 points and more) -------------------------------------------------------
 // Which passes give a thread four or eight points instead of sixteen (ntt_device.h, Lanes): few points only where the launch leaves the
 // chip part empty, since in a full one the twiddles and addresses of each lane of a block are work for nothing.  All figures down to
-// narrower_slabs but the one marked there: us of device time a call, calls queued, one build with its lines moved.
+// narrower_slabs but the one marked there: us of device time a call, calls queued, one build with its lines moved; 60 bits in the arithmetic
+// of primes that are not just below 2^60 (those lie between these figures and the ones of 42 bits).
 // Transforms of 2^16 points with sixteen / eight / four points in that pass (workgroups of 4096 points, columns on whole slabs):
 //   workgroups                 64               128              256              384              512              768              1024
 //   columns, forward, 60 bits  11.1/10.6/10.4   13.7/13.2/13.1   19.3/18.9/18.5   25.6/25.6/25.2   27.1/27.1/26.6   29.9/29.7/29.9   35.6/35.6/36.3

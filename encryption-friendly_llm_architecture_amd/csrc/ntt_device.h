@@ -4,7 +4,7 @@
 #include "hemm_internal.hpp"
 #include "sampling.h"
 
-// a twiddle and its Shoup quotient
+// a twiddle and its Shoup quotient; of primes just below 2^60 the twiddle and 2^32 times it, both cut (modarith.h, near60_add_mul)
 struct __align__(16) Tw {
     u64 w, ws;
 };
@@ -85,6 +85,7 @@ __device__ __forceinline__ void gs_bfly(u64 &x, u64 &y, const Tw tw, const u64 q
 
 // Two arithmetic back ends share the kernels below.
 //
+// (and a third, Near60Field below, for primes just below 2^60.)
 // IntField: 64-bit Shoup butterflies with values kept in [0, 4q) (Harvey), for primes up to 2^61.
 //
 // FpField: primes below 2^44 in double precision.  gfx950 issues one FP64 FMA per lane per clock but
@@ -125,6 +126,10 @@ struct IntFieldT {
         // a pass that does not end an inverse transform has no use for them and brings no table
         ni = ninv != nullptr ? ninv[prime] : 0;
         nis = ninv_s != nullptr ? ninv_s[prime] : 0;
+    }
+    __device__ __forceinline__ void set_scale(const Tw c) {
+        ni = c.w;
+        nis = c.ws;
     }
     // v < 16q, 2^44 < q < 2^60, to below 3q: v / q exceeds (v >> 32) floor(2^64 / q) / 2^32 by less than v / 2^64 + 2^32 / q < 1 + 2^-12, and
     // the product's high word by less than 1 more
@@ -178,6 +183,82 @@ struct IntFieldT {
 
 typedef IntFieldT<false> IntField;
 
+// Primes just below 2^60 (near_2_60: what a chain of 60-bit primes is made of, and the special primes).  Forward values stay below 15.1q: a
+// stage of even number in its block folds its first operand to q and a little, sums and differences are then below 8.1q, and after the
+// odd stage behind it below 15.1q.  Inverse values lie below 6.9q in front of every stage, whose sums are folded.  A butterfly is 10.5
+// vector instructions forward and 13 inverse where LAZY16 takes 16.5 and 17 (a column pass of 16 points per thread 733 and 1140
+// instructions in all, 1088 and 1501).  Such passes were bound by these instructions: 32 x 24 limbs forward 337 -> 309 us (the trips
+// through memory take 303), rotation on 24 + 4 primes of 60 bits, level 20 125.8 -> 115.4, product of two encrypted 32 x 32 tiles
+// 432 -> 404, projection of a 768-wide layer 9770 -> 9587.  The line: a product stays below 6.9q as long as 2^28 (2^31 + yh / 2) is
+// below 0.97 * 2^60; the first 55 primes of rings of 2^16 points lie above 2^60 - 2^27, of smaller rings
+// more.
+struct Near60Field {
+    typedef u64 E;
+    typedef Tw W;
+    u64 q, q2, q7, nq1;
+    u32 delta, delta2, two_29;
+    Tw scale;   // what an inverse transform ends with, cut
+    __device__ __forceinline__ Near60Field(const ModQ *modq, const u64 *ninv, const u64 *ninv_s, const double *, int prime) {
+        q = modq[prime].q;
+        q2 = 2 * q;
+        q7 = 7 * q;
+        nq1 = opaque_neg(q);
+        delta = 0u - (u32)q;
+        delta2 = 2 * delta;
+        two_29 = 1u << 29;
+        asm("" : "+s"(two_29), "+s"(q7));   // multiply by the one and add the other, instead of making either from what it is made of
+        if (ninv != nullptr) set_scale(Tw{ninv[prime], ninv_s[prime]});
+    }
+    // a constant with its Shoup quotient, whose upper half is the quotient of 2^32 times the constant
+    __device__ __forceinline__ Tw cut(const Tw c) const {
+        const u64 v = (c.w << 32) - (c.ws >> 32) * q;
+        return Tw{(c.w >> 29 << 32) | (c.w & 0x1fffffffu), (v >> 29 << 32) | (v & 0x1fffffffu)};
+    }
+    // v c, canonical
+    __device__ __forceinline__ u64 times(const u64 v, const Tw c) const {
+        return csub(fold(near60_add_mul(0, v, c.w, c.ws, delta2, two_29)), q, nq1);
+    }
+    __device__ __forceinline__ void set_scale(const Tw c) { scale = cut(c); }
+    __device__ __forceinline__ u64 fold(u64 v) const { return near60_fold(v, delta); }
+    __device__ __forceinline__ E from_canonical(u64 v) const { return v; }
+    // up to 8 sources: either half of the sum may fill 64 bits; below 7.1q
+    __device__ __forceinline__ E from_dot(const Dot2 &d, const ModQ &) const {
+        return fold(d.s0) + (u64)(u32)d.s1 * (two_29 * 2) + (u64)(u32)(d.s1 >> 32) * (4 * delta);
+    }
+    __device__ __forceinline__ void ct(E &x, E &y, const W tw, const bool odd) const {
+        const u64 u = odd ? x : fold(x);
+        x = near60_add_mul(u, y, tw.w, tw.ws, delta2, two_29);
+        y = (2 * u + q7) - x;
+    }
+    __device__ __forceinline__ void gs(E &x, E &y, const W tw, const bool, const bool) const {
+        const u64 u = x, v = y;
+        x = fold(u + v);
+        y = near60_add_mul(0, (u + q7) - v, tw.w, tw.ws, delta2, two_29);
+    }
+    template <int T, int P>
+    __device__ __forceinline__ void after_inverse_block(E (&)[P]) const {}
+    __device__ __forceinline__ u64 to_canonical(E v) const { return csub(fold(v), q, nq1); }
+    __device__ __forceinline__ u64 scale_to_canonical(E v) const { return times(v, scale); }
+    __device__ __forceinline__ bool takes_signed(long long v) const { return (u64)v + q < q2; }
+    __device__ __forceinline__ E from_signed(long long v) const { return (u64)v + q; }
+    __device__ __forceinline__ u64 minus_product(E v, u64 a, u64 s, const ModQ &m) const { return submod(to_canonical(v), mulmod(a, s, m), q); }
+    __device__ __forceinline__ u64 sub_scale(E v, u64 y, const Tw cst) const { return times((y + q2) - fold(v), cut(cst)); }
+};
+// fn with the arithmetic of an integer prime below 2^60, resp. of any integer prime
+template <class FN>
+__device__ __forceinline__ void with_field_60(const ModQ *modq, const u64 *ninv, const u64 *ninv_s, const double *fp, const int prime, const FN fn) {
+    if (near_2_60(modq[prime].q))
+        fn(Near60Field(modq, ninv, ninv_s, fp, prime));
+    else
+        fn(IntFieldT<true>(modq, ninv, ninv_s, fp, prime));
+}
+template <class FN>
+__device__ __forceinline__ void with_int_field(const ModQ *modq, const u64 *ninv, const u64 *ninv_s, const double *fp, const int prime, const FN fn) {
+    if ((modq[prime].q >> 60) != 0)
+        fn(IntField(modq, ninv, ninv_s, fp, prime));
+    else
+        with_field_60(modq, ninv, ninv_s, fp, prime, fn);
+}
 
 struct FpField {
     typedef double E;
@@ -188,6 +269,10 @@ struct FpField {
         qinv = fp[4 * prime + 1];
         ni = fp[4 * prime + 2];
         niinv = fp[4 * prime + 3];
+    }
+    __device__ __forceinline__ void set_scale(const Tw c) {
+        ni = (double)c.w;
+        niinv = ni * qinv;
     }
     __device__ __forceinline__ E mulmod(E y, E w, E winv) const {
         const double c = __builtin_rint(y * winv);

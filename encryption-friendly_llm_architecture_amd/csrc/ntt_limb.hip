@@ -153,12 +153,15 @@ __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_forward_kernel(
     if (fp[4 * prime] != 0.0)
         limb_forward<LR, P, NS, TAIL>(base, tw, rtw, FpField(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, ls,
                                    coef, mn, o, cst, sec);
-    else if (NS <= 0 && (m.q >> 60) != 0)   // (the sums of a conversion take primes below 2^60)
-        limb_forward<LR, P, NS, TAIL>(base, tw, rtw, IntField(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, ls,
-                                   coef, mn, o, cst, sec);
-    else
-        limb_forward<LR, P, NS, TAIL>(base, tw, rtw, IntFieldT<true>(modq, nullptr, nullptr, fp, prime), lds, src, so, h, n_src, m, ls,
-                                   coef, mn, o, cst, sec);
+    else {
+        const auto transform = [&](const auto f) {
+            limb_forward<LR, P, NS, TAIL>(base, tw, rtw, f, lds, src, so, h, n_src, m, ls, coef, mn, o, cst, sec);
+        };
+        if constexpr (NS <= 0)
+            with_int_field(modq, nullptr, nullptr, fp, prime, transform);
+        else   // (the sums of a conversion take primes below 2^60)
+            with_field_60(modq, nullptr, nullptr, fp, prime, transform);
+    }
 }
 
 template <int LR, int P, int LOAD, class F>
@@ -193,18 +196,6 @@ __device__ __forceinline__ void limb_inverse(u64 *__restrict__ limb, const Tw *_
     for (int k = 0; k < P; k++) buf_store<u64>(to, S::voff(), S::off(k), f.scale_to_canonical(x[k]));
 }
 
-template <class F, int LR, int P, int LOAD>
-__device__ __forceinline__ void limb_inverse_int(u64 *__restrict__ base, const Tw *__restrict__ tw, const Tw *__restrict__ rtw,
-                                                 const ModQ *__restrict__ modq, const u64 *__restrict__ ninv, const u64 *__restrict__ ninv_s,
-                                                 const double *__restrict__ fp, const int prime, const Tw *__restrict__ final_scale,
-                                                 const int limb, u64 *lds, const u64 *__restrict__ ld, const u32 gal, const RowSecond &sec) {
-    F f(modq, ninv, ninv_s, fp, prime);
-    if (final_scale != nullptr) {
-        f.ni = final_scale[limb].w;
-        f.nis = final_scale[limb].ws;
-    }
-    limb_inverse<LR, P, LOAD>(base, tw, rtw, f, lds, ld, gal, sec);
-}
 template <int LR, int P, int LOAD>
 __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_inverse_kernel(
     u64 *__restrict__ data, const Tw *__restrict__ tw_all, const Tw *__restrict__ rtw_all, const ModQ *__restrict__ modq,
@@ -226,15 +217,13 @@ __global__ __launch_bounds__((256 / P) << LR) void ntt_limb_inverse_kernel(
     const Tw *tw = tw_all + ((size_t)prime << log_n), *rtw = rtw_all + ((size_t)prime << log_n);
     if (fp[4 * prime] != 0.0) {
         FpField f(modq, ninv, ninv_s, fp, prime);
-        if (final_scale != nullptr) {
-            f.ni = (double)final_scale[limb].w;
-            f.niinv = f.ni * f.qinv;
-        }
+        if (final_scale != nullptr) f.set_scale(final_scale[limb]);
         limb_inverse<LR, P, LOAD>(base, tw, rtw, f, lds, ld, from.galois, sec);
-    } else if ((modq[prime].q >> 60) != 0) {
-        limb_inverse_int<IntField, LR, P, LOAD>(base, tw, rtw, modq, ninv, ninv_s, fp, prime, final_scale, limb, lds, ld, from.galois, sec);
     } else {
-        limb_inverse_int<IntFieldT<true>, LR, P, LOAD>(base, tw, rtw, modq, ninv, ninv_s, fp, prime, final_scale, limb, lds, ld, from.galois, sec);
+        with_int_field(modq, ninv, ninv_s, fp, prime, [&](auto f) {
+            if (final_scale != nullptr) f.set_scale(final_scale[limb]);
+            limb_inverse<LR, P, LOAD>(base, tw, rtw, f, lds, ld, from.galois, sec);
+        });
     }
 }
 

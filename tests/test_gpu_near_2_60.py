@@ -1,0 +1,77 @@
+"""Primes on both sides of 2^60 - 2^27, where transforms and key switches change their arithmetic, against the oracle: operands at q - 1
+and random ones."""
+import numpy as np
+import pytest
+
+from __graft_entry__ import load_package
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+LINE = 2**60 - 2**27
+
+
+def dev(a):
+    import torch
+    return torch.from_numpy(np.array(a).view(np.int64)).cuda()
+
+
+def host(t):
+    return t.cpu().numpy().view(np.uint64)
+
+
+def around_the_line(log_n):
+    """The first primes above and at or below the line, and the first below 2^60."""
+    step = 2 << log_n
+    first = LINE // step * step + 1
+    above = next(p for p in range(first if first > LINE else first + step, 2**60, step) if O.is_prime(p))
+    below = next(p for p in range(first if first <= LINE else first - step, 0, -step) if O.is_prime(p))
+    assert 2**60 - above < 2**27 <= 2**60 - below
+    return [above, below, O.primes_below(60, log_n, 1)[0]]
+
+
+def residues(rng, primes, lead, n, largest):
+    out = np.empty(tuple(lead) + (len(primes), n), dtype=np.uint64)
+    for j, q in enumerate(primes):
+        out[..., j, :] = q - 1 if largest else rng.integers(0, q, tuple(lead) + (n,), dtype=np.uint64)
+    return out
+
+
+@pytest.mark.parametrize("log_n", [9, 10, 11, 12, 13, 14, 15, 16])
+@pytest.mark.parametrize("polys", [1, 40])
+def test_transforms(log_n, polys):
+    qs = around_the_line(log_n)
+    ctx, orc = load_package().Context(log_n, qs, [], 1), O.Oracle(log_n, qs, [], 1)
+    rng, n = np.random.default_rng(log_n), 1 << log_n
+    a = np.concatenate([residues(rng, qs, (1,), n, True), residues(rng, qs, (1,), n, False)])
+    a[0, :, 1::2] = 0
+    for inverse in (False, True):
+        want = a.copy()
+        orc.ntt(want, [0, 1, 2], inverse=inverse)
+        for i in (0, 1):
+            got = host(ctx.ntt(dev(np.broadcast_to(a[i], (polys,) + a[i].shape)), [0, 1, 2], inverse=inverse))
+            assert np.array_equal(got, np.broadcast_to(want[i], got.shape)), (inverse, i)
+
+
+@pytest.mark.parametrize("log_n", [10, 13, 16])
+@pytest.mark.parametrize("largest", [False, True])
+def test_key_switches_and_conversions(log_n, largest):
+    """Chain and special primes of either kind: key products between the passes of their transforms, conversions from and to both kinds, and
+    the tail of a ModDown."""
+    above, below, top = around_the_line(log_n)
+    others = [p for p in O.primes_below(60, log_n, 4) if p not in (above, top)]
+    small = O.primes_below(42, log_n, 1)
+    qs, ps, dnum = [above, others[0]] + small + [below], [top, others[1]], 2
+    orc, ctx = O.Oracle(log_n, qs, ps, dnum), load_package().Context(log_n, qs, ps, dnum)
+    rng, n = np.random.default_rng(log_n + 100 * largest), 1 << log_n
+    key = residues(rng, qs + ps, (dnum, 2), n, largest)
+    for nq in (4, 2):
+        p = residues(rng, qs[:nq], (), n, largest)
+        ob, oa = np.empty((nq, n), dtype=np.uint64), np.empty((nq, n), dtype=np.uint64)
+        orc.L.orc_keyswitch(orc.h, O._p(p), O._p(key), nq, O._p(ob), O._p(oa))
+        assert np.array_equal(host(ctx.keyswitch(dev(p), dev(key), nq)), np.stack([ob, oa])), nq
+        for polys in (2, 16):
+            y = np.broadcast_to(residues(rng, qs[:nq] + ps, (2,), n, largest), (polys // 2, 2, nq + 2, n)).reshape(polys, nq + 2, n)
+            for drop in (False, True):
+                want = orc.moddown_drop(np.ascontiguousarray(y[:2]), nq, drop)
+                got = host(ctx.moddown_batch(dev(y), nq, drop))
+                assert np.array_equal(got[:2], want) and np.array_equal(got[-2:], want), (nq, polys, drop)
