@@ -124,7 +124,8 @@ struct Rotation {
         }
         if ((int)e < nq) b = load2(T.b + from);
     }
-    // to [0, q)
+    // to [0, q); NEAR: of a prime just below 2^60 (modarith.h, Near60)
+    template <bool NEAR>
     __device__ __forceinline__ void finish(const ModQ &m, const FpMod f, const Cst pmod, const bool with_b, const int premultiplied, u64 (&rb)[2], u64 (&ra)[2]) {
         if (FP) {
             double sb0 = 0, sb1 = 0, sa0 = 0, sa1 = 0;
@@ -160,6 +161,23 @@ struct Rotation {
                 acc_mul(sa[0], px, pieces(ka[d].v.x));
                 acc_mul(sa[1], py, pieces(ka[d].v.y));
             }
+            if (NEAR) {
+                const Near60 near(q);
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    rb[h] = near.reduce(sb[h]);
+                    ra[h] = near.canonical(near.fold(near.reduce(sa[h])));
+                }
+                if (with_b) {
+                    swap_if(swap, b);
+                    const Cut p = near.cut(pmod.w, pmod.ws);
+                    rb[0] = premultiplied ? rb[0] + b.x : near.add_mul(rb[0], b.x, p);
+                    rb[1] = premultiplied ? rb[1] + b.y : near.add_mul(rb[1], b.y, p);
+                }
+#pragma unroll
+                for (int h = 0; h < 2; h++) rb[h] = near.canonical(near.fold(rb[h]));
+                return;
+            }
 #pragma unroll
             for (int h = 0; h < 2; h++) {   // below 3q
                 rb[h] = acc_reduce(sb[h], m);
@@ -186,14 +204,20 @@ struct DiagonalTile {
     ulonglong2 (*made)[2][2][128];   // [turn][rotation of the turn][polynomial]: residues n, n + 1
     u64 (*acc)[256];          // [DIAG_OUT / 2 * 4]: what the accumulators have been reduced to
 };
-template <bool FP, int B, bool COMPACT>
+template <bool FP, int B, bool COMPACT, bool NEAR>
 __device__ __forceinline__ void diagonal_sums(const HoistedArgs &args, const DiagonalTile &w, const u64 *__restrict__ a, const size_t a_stride,
                                               const ModQ m, const FpMod f, const Cst pmod, const KeyLimb kl, const int nq, const int E,
                                               const int logN, const int premultiplied, const u32 g) {
     constexpr int OUT = DIAG_OUT / 2;
     const u64 q = m.q, n8 = opaque_neg(8 * q), n4 = opaque_neg(4 * q), n2 = opaque_neg(2 * q), n1 = opaque_neg(q);
+    const Near60 near(q);
     const size_t N = (size_t)1 << logN;
     const bool chain = (int)w.e < nq;
+    // what the accumulators hold, added to acc < 8q, to below 8q
+    auto more = [&](const u64 acc, const Dot2 &s) {
+        if (NEAR) return near.fold(acc + near.reduce(s.s0, s.s1));
+        return csub(acc + csub(dot_reduce_lazy(s, m), 8 * q, n8), 8 * q, n8);   // 13q to 8q, and the sum of two to 8q
+    };
     Dot2 d[OUT][4];
 #pragma unroll
     for (int i = 0; i < OUT; i++)
@@ -208,7 +232,7 @@ __device__ __forceinline__ void diagonal_sums(const HoistedArgs &args, const Dia
         const u32 j = j0 + w.half, turn = (j0 >> 1) & 1u;
         u64 rb[2] = {0, 0}, ra[2] = {0, 0};
         if (j != 0) {
-            r.finish(m, f, pmod, chain, premultiplied, rb, ra);
+            r.template finish<NEAR>(m, f, pmod, chain, premultiplied, rb, ra);
         } else if (chain) {
             const ulonglong2 b0 = load2(a + w.e * N + w.n), a0 = load2(a + a_stride + w.e * N + w.n);
             rb[0] = b0.x;
@@ -236,9 +260,9 @@ __device__ __forceinline__ void diagonal_sums(const HoistedArgs &args, const Dia
 #pragma unroll
             for (int i = 0; i < OUT; i++)
 #pragma unroll
-                for (int v = 0; v < 4; v++) {   // 13q to 8q, and the sum of two to 8q
+                for (int v = 0; v < 4; v++) {
                     u64 &acc = w.acc[i * 4 + v][threadIdx.x];
-                    acc = csub(acc + csub(dot_reduce_lazy(d[i][v], m), 8 * q, n8), 8 * q, n8);
+                    acc = more(acc, d[i][v]);
                     dot_clear(d[i][v]);
                 }
         }
@@ -249,8 +273,8 @@ __device__ __forceinline__ void diagonal_sums(const HoistedArgs &args, const Dia
         u64 s[4];
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-            s[v] = csub(w.acc[i * 4 + v][threadIdx.x] + csub(dot_reduce_lazy(d[i][v], m), 8 * q, n8), 8 * q, n8);
-            s[v] = csub(csub(csub(s[v], 4 * q, n4), 2 * q, n2), q, n1);
+            s[v] = more(w.acc[i * 4 + v][threadIdx.x], d[i][v]);
+            s[v] = csub(NEAR ? s[v] : csub(csub(s[v], 4 * q, n4), 2 * q, n2), q, n1);
         }
         u64 *to = w.y + (size_t)i * 2 * w.pol;
         stream_store2(to, s[0], s[1]);
@@ -306,15 +330,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
     w.tab = tables + ((((size_t)w.e << (logN - log_run)) + run) * chunks + chunk) * g * DIAG_OUT + w.half * (DIAG_OUT / 2);
     const Cst pmod = (int)w.e < nq ? pmods[w.e] : Cst{0, 0};
     const FpMod f{fp[4 * prime], fp[4 * prime + 1]};
-#define SUMS(FP, B) diagonal_sums<FP, B, COMPACT>(args, w, a, a_stride, m, f, pmod, kl, nq, E, logN, premultiplied, g)
+#define SUMS(FP, B, NEAR) diagonal_sums<FP, B, COMPACT, NEAR>(args, w, a, a_stride, m, f, pmod, kl, nq, E, logN, premultiplied, g)
     if (f.q != 0.0) {
-        if (beta == 1) SUMS(true, 1);
-        else if (beta == 2) SUMS(true, 2);
-        else SUMS(true, 3);
+        if (beta == 1) SUMS(true, 1, false);
+        else if (beta == 2) SUMS(true, 2, false);
+        else SUMS(true, 3, false);
+    } else if (near_2_60(m.q) && beta <= 2) {   // (with three digits it would spill)
+        if (beta == 1) SUMS(false, 1, true);
+        else SUMS(false, 2, true);
     } else {
-        if (beta == 1) SUMS(false, 1);
-        else if (beta == 2) SUMS(false, 2);
-        else SUMS(false, 3);
+        if (beta == 1) SUMS(false, 1, false);
+        else if (beta == 2) SUMS(false, 2, false);
+        else SUMS(false, 3, false);
     }
 #undef SUMS
 }

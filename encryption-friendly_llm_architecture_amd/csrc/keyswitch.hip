@@ -504,12 +504,17 @@ __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict_
         ra[1] = f.canonical(fa[1]);
     } else if (beta <= 3 && modq[prime].mu3 != 0) {
         const ModQ m = modq[prime];
-        if (beta == 1)
-            hoisted_pair_pieces<COMPACT, S, 1>(terms, group_off, part, kl, m, pmod, j, o, n, nq, E, logN, b_premultiplied, rb, ra);
-        else if (beta == 2)
-            hoisted_pair_pieces<COMPACT, S, 2>(terms, group_off, part, kl, m, pmod, j, o, n, nq, E, logN, b_premultiplied, rb, ra);
-        else
-            hoisted_pair_pieces<COMPACT, S, 3>(terms, group_off, part, kl, m, pmod, j, o, n, nq, E, logN, b_premultiplied, rb, ra);
+#define PIECES(B, NEAR) hoisted_pair_pieces<COMPACT, S, B, NEAR>(terms, group_off, part, kl, m, pmod, j, o, n, nq, E, logN, b_premultiplied, rb, ra)
+        if (near_2_60(m.q)) {
+            if (beta == 1) PIECES(1, true);
+            else if (beta == 2) PIECES(2, true);
+            else PIECES(3, true);
+        } else {
+            if (beta == 1) PIECES(1, false);
+            else if (beta == 2) PIECES(2, false);
+            else PIECES(3, false);
+        }
+#undef PIECES
     } else {
         hoisted_pair_int<COMPACT, S>(terms, group_off, part, kl, modq[prime], pmod, j, o, n, nq, E, beta, logN, b_premultiplied, rb, ra);
     }
@@ -675,6 +680,26 @@ __device__ __forceinline__ void switched_pair(const F f, const FpMod fm, const M
             acc_mul(sb[1], py, pieces(kb[d].y));
             acc_mul(sa[0], px, pieces(ka[d].x));
             acc_mul(sa[1], py, pieces(ka[d].y));
+        }
+        if constexpr (std::is_same<F, Near60Field>::value) {
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                rb[h] = f.reduce(sb[h]);
+                ra[h] = f.reduce(sa[h]);
+            }
+            if (chain) {   // 8.4q and 4.9q
+                const Cut p = f.cut(pmod.w, pmod.ws);
+                rb[0] = f.add_mul(rb[0], b.x + pb.x, p);
+                rb[1] = f.add_mul(rb[1], b.y + pb.y, p);
+                ra[0] = f.add_mul(ra[0], pa.x, p);
+                ra[1] = f.add_mul(ra[1], pa.y, p);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                rb[h] = f.to_canonical(rb[h]);
+                ra[h] = f.to_canonical(ra[h]);
+            }
+            return;
         }
 #pragma unroll
         for (int h = 0; h < 2; h++) {   // below 3q, 5q with what the chain limbs add

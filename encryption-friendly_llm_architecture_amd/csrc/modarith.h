@@ -95,6 +95,9 @@ __device__ __forceinline__ u64 near60_fold(const u64 v, const u32 delta) {
     const u32 h = (u32)(v >> 32);
     return (((u64)(h & 0x0fffffffu) << 32) | (u32)v) + (u64)(h >> 28) * delta;
 }
+struct Cut {   // a constant and 2^32 times it, cut
+    u64 w, v;
+};
 // v < 32q (q < 2^59) to [0, q)
 __device__ __forceinline__ u64 reduce_below_32q(u64 v, const u64 q) {
 #pragma unroll
@@ -266,3 +269,34 @@ __device__ __forceinline__ u64 acc_reduce(const Acc3 &a, const ModQ &m) {
     const u64 qhat = __umul64hi(t1, m.mu3) >> 1;
     return (a.s0 + (a.s1 << 30) + (a.s2 << 60)) + qhat * neg_uniform(m.q);
 }
+
+// The arithmetic of a prime just below 2^60 that is uniform over the wavefront
+struct Near60 {
+    u64 q;
+    u32 delta, delta2, delta4, two_29;
+    __device__ __forceinline__ explicit Near60(const u64 prime) : q(prime), delta(0u - (u32)prime), delta2(2 * delta), delta4(4 * delta), two_29(1u << 29) {
+        asm("" : "+s"(two_29));   // multiplied by, not shifted by in three instructions
+    }
+    // a constant with its Shoup quotient, whose upper half is the quotient of 2^32 times the constant
+    __device__ __forceinline__ Cut cut(const u64 w, const u64 ws) const {
+        const u64 v = (w << 32) - (ws >> 32) * q;
+        return Cut{(w >> 29 << 32) | (w & 0x1fffffffu), (v >> 29 << 32) | (v & 0x1fffffffu)};
+    }
+    __device__ __forceinline__ u64 fold(const u64 v) const { return near60_fold(v, delta); }
+    // u + y c; the product is below 6.9q for y < 15.1q, 4.9q for y < 2q
+    __device__ __forceinline__ u64 add_mul(const u64 u, const u64 y, const Cut c) const { return near60_add_mul(u, y, c.w, c.v, delta2, two_29); }
+    // s0 + 2^30 s1 for any two sums, below 7.1q
+    __device__ __forceinline__ u64 reduce(const u64 s0, const u64 s1) const {
+        return fold(s0) + (u64)(u32)s1 * (2 * two_29) + (u64)(u32)(s1 >> 32) * delta4;
+    }
+    // s0 + 2^30 s1 + 2^60 s2 for s0 < 2^62, s1 < 14 * 2^60, s2 < 2^63 (three products of values below 2q): 2^60 counts delta, 2^92 2^30 times
+    // 4 delta.  Below 10.4q, 8.4q for three products of canonical values: multiply-adds alone where a Barrett step (acc_reduce) is 22 instructions.
+    __device__ __forceinline__ u64 reduce(const Acc3 &a) const {
+        const u64 s1 = a.s1 + (u64)(u32)(a.s2 >> 32) * delta4;
+        u64 s0 = a.s0 + (u64)(u32)a.s2 * delta;
+        s0 += (u64)(u32)s1 * (2 * two_29);
+        return s0 + (u64)(u32)(s1 >> 32) * delta4;
+    }
+    // v < 2q to [0, q)
+    __device__ __forceinline__ u64 canonical(const u64 v) const { return cond_sub_u(v, q); }
+};

@@ -192,48 +192,33 @@ typedef IntFieldT<false> IntField;
 // 432 -> 404, projection of a 768-wide layer 9770 -> 9587.  The line: a product stays below 6.9q as long as 2^28 (2^31 + yh / 2) is
 // below 0.97 * 2^60; the first 55 primes of rings of 2^16 points lie above 2^60 - 2^27, of smaller rings
 // more.
-struct Near60Field {
+struct Near60Field : Near60 {
     typedef u64 E;
     typedef Tw W;
-    u64 q, q2, q7, nq1;
-    u32 delta, delta2, two_29;
-    Tw scale;   // what an inverse transform ends with, cut
-    __device__ __forceinline__ Near60Field(const ModQ *modq, const u64 *ninv, const u64 *ninv_s, const double *, int prime) {
-        q = modq[prime].q;
+    u64 q2, q7, nq1;
+    Cut scale;   // what an inverse transform ends with
+    __device__ __forceinline__ Near60Field(const ModQ *modq, const u64 *ninv, const u64 *ninv_s, const double *, int prime) : Near60(modq[prime].q) {
         q2 = 2 * q;
         q7 = 7 * q;
+        asm("" : "+s"(q7));   // added, not made of q by a multiply-add
         nq1 = opaque_neg(q);
-        delta = 0u - (u32)q;
-        delta2 = 2 * delta;
-        two_29 = 1u << 29;
-        asm("" : "+s"(two_29), "+s"(q7));   // multiply by the one and add the other, instead of making either from what it is made of
         if (ninv != nullptr) set_scale(Tw{ninv[prime], ninv_s[prime]});
     }
-    // a constant with its Shoup quotient, whose upper half is the quotient of 2^32 times the constant
-    __device__ __forceinline__ Tw cut(const Tw c) const {
-        const u64 v = (c.w << 32) - (c.ws >> 32) * q;
-        return Tw{(c.w >> 29 << 32) | (c.w & 0x1fffffffu), (v >> 29 << 32) | (v & 0x1fffffffu)};
-    }
     // v c, canonical
-    __device__ __forceinline__ u64 times(const u64 v, const Tw c) const {
-        return csub(fold(near60_add_mul(0, v, c.w, c.ws, delta2, two_29)), q, nq1);
-    }
-    __device__ __forceinline__ void set_scale(const Tw c) { scale = cut(c); }
-    __device__ __forceinline__ u64 fold(u64 v) const { return near60_fold(v, delta); }
+    __device__ __forceinline__ u64 times(const u64 v, const Cut c) const { return csub(fold(add_mul(0, v, c)), q, nq1); }
+    __device__ __forceinline__ void set_scale(const Tw c) { scale = cut(c.w, c.ws); }
     __device__ __forceinline__ E from_canonical(u64 v) const { return v; }
     // up to 8 sources: either half of the sum may fill 64 bits; below 7.1q
-    __device__ __forceinline__ E from_dot(const Dot2 &d, const ModQ &) const {
-        return fold(d.s0) + (u64)(u32)d.s1 * (two_29 * 2) + (u64)(u32)(d.s1 >> 32) * (4 * delta);
-    }
+    __device__ __forceinline__ E from_dot(const Dot2 &d, const ModQ &) const { return reduce(d.s0, d.s1); }
     __device__ __forceinline__ void ct(E &x, E &y, const W tw, const bool odd) const {
         const u64 u = odd ? x : fold(x);
-        x = near60_add_mul(u, y, tw.w, tw.ws, delta2, two_29);
+        x = add_mul(u, y, Cut{tw.w, tw.ws});
         y = (2 * u + q7) - x;
     }
     __device__ __forceinline__ void gs(E &x, E &y, const W tw, const bool, const bool) const {
         const u64 u = x, v = y;
         x = fold(u + v);
-        y = near60_add_mul(0, (u + q7) - v, tw.w, tw.ws, delta2, two_29);
+        y = add_mul(0, (u + q7) - v, Cut{tw.w, tw.ws});
     }
     template <int T, int P>
     __device__ __forceinline__ void after_inverse_block(E (&)[P]) const {}
@@ -242,7 +227,7 @@ struct Near60Field {
     __device__ __forceinline__ bool takes_signed(long long v) const { return (u64)v + q < q2; }
     __device__ __forceinline__ E from_signed(long long v) const { return (u64)v + q; }
     __device__ __forceinline__ u64 minus_product(E v, u64 a, u64 s, const ModQ &m) const { return submod(to_canonical(v), mulmod(a, s, m), q); }
-    __device__ __forceinline__ u64 sub_scale(E v, u64 y, const Tw cst) const { return times((y + q2) - fold(v), cut(cst)); }
+    __device__ __forceinline__ u64 sub_scale(E v, u64 y, const Tw cst) const { return times((y + q2) - fold(v), cut(cst.w, cst.ws)); }
 };
 // fn with the arithmetic of an integer prime below 2^60, resp. of any integer prime
 template <class FN>

@@ -12,7 +12,7 @@ LINE = 2**60 - 2**27
 
 def dev(a):
     import torch
-    return torch.from_numpy(np.array(a).view(np.int64)).cuda()
+    return torch.from_numpy(np.array(a, order="C").view(np.int64)).cuda()
 
 
 def host(t):
@@ -75,3 +75,34 @@ def test_key_switches_and_conversions(log_n, largest):
                 want = orc.moddown_drop(np.ascontiguousarray(y[:2]), nq, drop)
                 got = host(ctx.moddown_batch(dev(y), nq, drop))
                 assert np.array_equal(got[:2], want) and np.array_equal(got[-2:], want), (nq, polys, drop)
+
+
+@pytest.mark.parametrize("digits", [1, 2, 3])
+@pytest.mark.parametrize("largest", [False, True])
+def test_hoisted_sums(digits, largest):
+    """One source, two masked ones under one key (whole masks and run tables), and a sum longer than the accumulators' corrections are apart."""
+    log_n, shift, n = 10, 3, 1 << 10
+    above, below, top = around_the_line(log_n)
+    qs, ps, nq = [above, below, O.primes_below(60, log_n, 5)[4]][:digits], [top, O.primes_below(60, log_n, 5)[3]], digits
+    orc, ctx = O.Oracle(log_n, qs, ps, digits), load_package().Context(log_n, qs, ps, digits)
+    rng, primes = np.random.default_rng(digits), qs + ps
+    ext, b = [residues(rng, primes, (digits,), n, largest) for _ in range(2)], [residues(rng, qs, (), n, largest) for _ in range(2)]
+    keys = [residues(rng, primes, (digits, 2), n, largest) for _ in range(2)]
+    full = [residues(rng, primes, (), n, largest) for _ in range(2)]
+    runs = [np.repeat(residues(rng, primes, (), n >> shift, largest), 1 << shift, axis=-1) for _ in range(2)]
+    g = [pow(5, 77, 2 * n), pow(5, 3, 2 * n)]
+    sums = [[(0, 0, None, 0)], [(0, 0, full[0], 0), (1, 0, full[1], 0)], [(0, 0, runs[0], 0), (1, 0, runs[1], 0)],
+            [(i & 1, i >> 1 & 1, full[i & 1], i >> 1 & 1) for i in range(20)]]
+    d_ext, d_b, d_keys, d_full = [[dev(x) for x in v] for v in (ext, b, keys, full)]
+    d_runs = [ctx.compact_mask(dev(m), shift) for m in runs]
+    groups, want = [], np.zeros((len(sums), 2, nq + 2, n), dtype=np.uint64)
+    for o, terms in enumerate(sums):
+        group = []
+        for i, (s, k, m, a) in enumerate(terms):
+            table = o == 2
+            mask = None if m is None else d_runs[s] if table else d_full[s]
+            group.append((d_ext[s], d_b[s], d_keys[k], mask, g[a], shift) if table else (d_ext[s], d_b[s], d_keys[k], mask, g[a]))
+            orc.L.orc_hoisted_term(orc.h, O._p(ext[s]), O._p(b[s]), O._p(keys[k]), O._p(m) if m is not None else None, g[a], nq, O._p(want[o]), int(i > 0))
+        groups.append(group)
+    for o, got in enumerate(host(ctx.hoisted_terms(groups, nq))):
+        assert np.array_equal(got, want[o]), o
