@@ -196,13 +196,17 @@ void launch_encode(const hemm_context *c, const double *slots, const double *re,
 // != nullptr: slots is a workspace and the real parts of the first `count` slots go to re.  a and re need N >= 2^10.
 void launch_decode(const hemm_context *c, const u64 *pt, const u64 *a, const u64 *sk, int n_limbs, double scale, u64 *work,
                    double *slots, double *re, size_t count, hipStream_t s);
-// out[p][j] = (y[p][j] - conversion of the n_src listed limbs of y[p] to prime j) * cst[j], j < nq_out, as inverse row
-// pass (in place on the listed limbs), one column-slab kernel (second inverse pass, conversion as lazy dot products, first
-// forward pass into conv[n_polys][nq_out][N]) and forward row pass with the fused tail.  final_scale / hat / cst: device
-// tables in source order, [n_src][hat_ld] by prime (as in ConvSources), by target limb.  false when the shape has no such form.
+// out[p][j] = (y[p][j] - conversion of the n_src listed limbs of y[p] to chain prime j) * cst[j], j < nq_out, as inverse row
+// pass (in place on the listed limbs; rows_done: it has run), one column-slab kernel (second inverse pass, conversion as lazy dot
+// products, first forward pass into conv[n_polys][nq_out][N]) and forward row pass with the fused tail (not with cols_only).  final_scale
+// / hat / cst: device tables in source order, [n_src][hat_ld] by prime (as in ConvSources), by target limb.  list: where the results
+// lie, for one run of polynomials.  Primes below 2^60.  false when the shape has no such form (nothing was launched).
 bool launch_moddown_slab(const hemm_context *c, u64 *y, size_t y_stride, const uint8_t *src_slot, const uint8_t *src_prime,
                          int n_src, const void *final_scale_dev, const void *hat_dev, int hat_ld, u64 *conv, int nq_out,
-                         int n_polys, u64 *out, size_t out_stride, const void *cst_dev, hipStream_t s);
+                         int n_polys, u64 *out, size_t out_stride, const void *cst_dev, hipStream_t s, const ResultList *list = nullptr,
+                         bool rows_done = false, bool cols_only = false);
+// whether that form is the faster one (N = 2^16, two to five sources)
+bool takes_moddown_slab(const hemm_context *c, int n_src, int nq_out, int n_polys);
 // inverse transform reading src (same slot numbering as data, polynomial stride src_poly_stride) and leaving the
 // coefficients in data; false when this ring size has no out-of-place form (the caller copies, then transforms)
 // galois != 0: src is read through that automorphism (the transform of the rotated polynomial, without a launch

@@ -1851,19 +1851,15 @@ void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop
         sl.idx[i] = a.src_slot[i];
     }
     const bool fold = ring_has_fused_forms(c);   // the inverse transform ends with (1/N)(S/q_i)^-1: no scaling pass in the conversion
-    // the three-launch form with one column-slab kernel in the middle, only on request: it moves a fifth less data but
-    // runs at two waves per SIMD and is slower on every batch size measured
-    if (slab && rows_done) throw std::invalid_argument("the column-slab ModDown begins with its own row pass");
-    if (slab && list != nullptr) throw std::invalid_argument("the column-slab ModDown leaves its results back to back");
     if (slab && !(c->logN == 16 && lazy_dot_ok(c))) throw std::invalid_argument("the column-slab ModDown needs N = 2^16 and primes below 2^60");
-    if (slab) {
-        if (!launch_moddown_slab(c, y, (size_t)E * N, a.src_slot, a.src_prime, ns,
+    if (slab && (ns < 4 || ns > 5)) throw std::invalid_argument("the column-slab ModDown takes 4 or 5 dropped limbs");
+    // inverse column pass, conversion and forward column pass as one kernel, where it is the faster form and on request
+    if ((slab || takes_moddown_slab(c, ns, nq_out, n_polys)) && lazy_dot_ok(c) &&
+        launch_moddown_slab(c, y, (size_t)E * N, a.src_slot, a.src_prime, ns,
                             t->dev + (drop_last ? t->drop_invn_off[nq] : t->p_invn_off),
                             t->dot + (drop_last ? t->drop_hat_off[nq] : t->p_hat_off), c->nQ + c->nP, conv, nq_out, n_polys,
-                            out, out_stride, t->dev + (drop_last ? t->dropinv_off[nq] : t->pinv_off), s))
-            throw std::invalid_argument("the column-slab ModDown takes 4 or 5 dropped limbs");
+                            out, out_stride, t->dev + (drop_last ? t->dropinv_off[nq] : t->pinv_off), s, list, rows_done, cols_only))
         return;
-    }
     if (rows_done)
         launch_intt_cols(c, y, pl, sl, ns, n_polys, (size_t)E * N, s, t->dev + (drop_last ? t->drop_invn_off[nq] : t->p_invn_off));
     else

@@ -158,6 +158,10 @@ __device__ __forceinline__ u64 reduce64(u64 a, const ModQ &m) {
 // conversion).  With v = v0 + 2^30 v1 and g = 2^30 h mod q kept beside h, the term is v0 h + v1 g: products of 30-bit
 // pieces of v with 30-bit pieces of h and g, four multiply-adds into two 64-bit accumulators of weights 1 and 2^30 that 16
 // products below 2^60 cannot overflow -- no carries, and a sum 34 bits longer than q instead of 64 to reduce.
+struct Pieces {
+    u32 lo, hi;
+};
+__device__ __forceinline__ Pieces pieces(const u64 v) { return Pieces{(u32)v & 0x3fffffffu, (u32)(v >> 30)}; }
 struct DotCst {
     u32 h0, h1, g0, g1;
 };
@@ -174,6 +178,13 @@ __device__ __forceinline__ void dot_add(Dot2 &d, const u64 v, const DotCst &c) {
     d.s0 += (u64)v1 * c.g0;
     d.s1 += (u64)v0 * c.h1;
     d.s1 += (u64)v1 * c.g1;
+}
+// the same of a residue that is kept in pieces
+__device__ __forceinline__ void dot_add(Dot2 &d, const Pieces v, const DotCst &c) {
+    d.s0 += (u64)v.lo * c.h0;
+    d.s0 += (u64)v.hi * c.g0;
+    d.s1 += (u64)v.lo * c.h1;
+    d.s1 += (u64)v.hi * c.g1;
 }
 // the sum as a 128-bit value, below 2^(k + 34) for constants below 2^k
 __device__ __forceinline__ u128_t dot_value(const Dot2 &d) {
@@ -246,10 +257,6 @@ __device__ __forceinline__ u64 negmod(u64 a, u64 q) { return a ? q - a : 0; }
 // ---- sums of products of residues below 2^60 in pieces of 30 bits -----------------------------------------------------------
 // A 128-bit product summed as such is 17 instructions (the compiler makes its two halves apart, and carries them).  Cut at bit 30
 // it is four multiply-adds into accumulators of weights 1, 2^30 and 2^60 that nothing is carried out of.
-struct Pieces {
-    u32 lo, hi;
-};
-__device__ __forceinline__ Pieces pieces(const u64 v) { return Pieces{(u32)v & 0x3fffffffu, (u32)(v >> 30)}; }
 struct Acc3 {
     u64 s0, s1, s2;
 };

@@ -283,148 +283,170 @@ __global__ __launch_bounds__((4096 >> H) / P) void ntt16_cols_lifted_kernel(u64 
         with_int_field(modq, nullptr, nullptr, fp, prime, [&](const auto f) { cols_lifted_body<LR, P, H>(base, tw, f, lds, ls, coef, m); });
 }
 // ------------------------------------------------------------------------------------------
-// Column-slab kernel of a ModDown (or any conversion of a few source limbs): for one (polynomial, 16-column slab) a
-// workgroup runs the second pass of the inverse transform of every source limb, keeps the canonical coefficients on
-// chip -- the last four sources in registers, one more in LDS -- and then, target limb by target limb, takes the
-// basis conversion as lazy dot products and runs the first pass of the forward transform.  The inverse result is
-// never written and the sources are never read back: the three steps are local to the slab, only the row passes on
-// either side need the other half of the 256 x 256 view.  Arithmetic, order of operations and stored values are those
-// of ntt16_cols_kernel<true> followed by ntt16_cols_converted_kernel.
-// 128 registers of sources per thread leave room for two waves per SIMD; LDS: 32 KiB exchange + 32 KiB source.
+// Column-slab kernel of a ModDown: for one (polynomial, half slab of eight columns) a workgroup runs the second pass of the inverse
+// transform of every source limb, keeps the canonical coefficients in registers and then, target limb by target limb, takes the basis
+// conversion as lazy dot products and runs the first pass of the forward transform.  The inverse result is never written and
+// the sources are never read back: the three steps are local to the slab, only the row passes on either side need the other half
+// of the 256 x 256 view.  Arithmetic, order of operations and stored values are those of ntt16_cols_kernel<true> followed by
+// ntt16_cols_converted_kernel.
+// Four points per thread: five sources are 40 registers (122 in all, four waves per SIMD, two workgroups on a CU), kept in the pieces that the
+// dot products take; a source's loads are in flight under the one before it.  Bound by issue: 3610 vector instructions per wave, VALUBusy 74 %,
+// 43.5 us for 16 polynomials of 5 sources and 6 targets where the two kernels take 16 + 37.  (Sixteen points per thread, 256 registers and
+// two waves per SIMD, was slower than the two kernels at any size.)
 // ------------------------------------------------------------------------------------------
-#define SLAB_REG_SOURCES 4
+#define SLAB_MAX_SOURCES 5
 struct SlabSources {
     const u64 *src;            // first-pass output of the inverse transform (raw field values), [n_polys][.][N]
     size_t src_poly_stride;
     const Cst *hat;            // [n_src][hat_ld]  (S/q_i) mod prime and 2^30 times that, indexed by prime
     const Tw *final_scale;     // [n_src]  (1/N)(S/q_i)^-1 mod q_i
-    int hat_ld, n_src, n_dst;
-    uint8_t src_slot[SLAB_REG_SOURCES + 1], src_prime[SLAB_REG_SOURCES + 1];
-    uint8_t dst_slot[HEMM_MAX_PRIMES], dst_prime[HEMM_MAX_PRIMES];
+    int hat_ld, n_src, n_dst;  // targets: chain primes 0 .. n_dst - 1, in the slots of these numbers
+    uint8_t src_slot[8], src_prime[8];   // SLAB_MAX_SOURCES of them, whole words (table_byte)
 };
 
+// Half slabs of 2^16 points, four points per thread.  What a thread keeps through all limbs: its place in the exchange buffer (rows 4 h + k
+// of the widest stages' block, k even and odd, and rows h + 4 k of the others': Slab::at written out) and the offset of its column.  The
+// rest of its place is made anew for every limb: kept as well, the offsets of the twelve twiddles of either arithmetic spill.
+struct SlabPlace {
+    typedef Slab<8, 4, 1> S;
+    u32 outer_even, outer_odd, inner, v_inner;
+    __device__ __forceinline__ SlabPlace() {
+        const u32 h = Lanes<4>::h(), rh = S::rh(), cc = S::cc(), flip = ((rh >> 2) ^ rh) & 1u;
+        outer_even = ((rh ^ ((h & 1u) << 1)) + 64u * h) * 8u + cc;
+        outer_odd = outer_even ^ 16u;
+        inner = (16u * rh + (h ^ (flip << 1))) * 8u + cc;
+        v_inner = S::v_inner();
+    }
+    __device__ __forceinline__ u32 outer(const int k) const { return (k & 1 ? outer_odd : outer_even) + 128u * (u32)k; }
+    __device__ __forceinline__ u32 within(const int k) const { return inner + 32u * (u32)k; }
+};
+struct SlabLane {   // lane of a block, twiddle group of the second block
+    u32 h, group;
+    __device__ __forceinline__ SlabLane() {
+        u32 t = threadIdx.x;
+        asm volatile("" : "+v"(t));
+        h = (t & 63u) >> 4;
+        group = 16u + (((t & 15u) | ((t >> 6) << 4)) >> 3);
+    }
+};
+
+// second pass of an inverse transform: x as loaded, r canonical coefficients in the layout a forward transform begins with
 template <class F>
-__device__ __forceinline__ void slab_inverse(const __amdgpu_buffer_rsrc_t limb, const u32 v_inner,
-                                             const Tw *__restrict__ tw_int, const F f, u64 *lds_raw, u64 (&r)[16]) {
+__device__ __forceinline__ void slab_inverse(const u64 (&raw)[4], const Tw *__restrict__ tw_int, const F f, u64 *lds_raw,
+                                             const SlabPlace &at, Pieces (&r)[4]) {
     typedef typename F::E E;
     const typename F::W *tw = (const typename F::W *)tw_int;
     E *lds = (E *)lds_raw;
-    const int cc = threadIdx.x & 15, rh = threadIdx.x >> 4;
-    E x[16];
+    const SlabLane lane;
+    E x[4];
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = buf_load<E>(limb, v_inner, (u32)k << 11);
-    radix_inv<4>(f, x, tw, 16u + rh);
+    for (int k = 0; k < 4; k++) __builtin_memcpy(&x[k], &raw[k], 8);
+    radix_inv<4>(f, x, tw, lane.group, lane.h);
     f.template after_inverse_block<4>(x);
-    __syncthreads();   // the previous exchange has been read by every wave
 #pragma unroll
-    for (int k = 0; k < 16; k++) lds[(16 * rh + k) * 16 + cc] = x[k];
+    for (int k = 0; k < 4; k++) lds[at.within(k)] = x[k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = lds[(rh + 16 * k) * 16 + cc];
-    radix_inv<4>(f, x, tw, 1u);
+    for (int k = 0; k < 4; k++) x[k] = lds[at.outer(k)];
+    radix_inv<4>(f, x, tw, 1u, lane.h);
 #pragma unroll
-    for (int k = 0; k < 16; k++) r[k] = f.scale_to_canonical(x[k]);
+    for (int k = 0; k < 4; k++) {
+        r[k] = pieces(f.scale_to_canonical(x[k]));
+        asm("" : "+v"(r[k].lo), "+v"(r[k].hi));   // kept as pieces, not as a residue that is cut again for every target
+    }
 }
 
-template <int NREG, bool LDS, class F>
-__device__ __forceinline__ void slab_forward(const __amdgpu_buffer_rsrc_t limb, const u32 v_inner,
-                                             const Tw *__restrict__ tw_int, const F f, u64 *lds_raw,
-                                             const u64 *__restrict__ lsrc, const DotCst &hl,
-                                             const u64 (&c)[SLAB_REG_SOURCES][16], const DotCst (&h)[SLAB_REG_SOURCES],
-                                             const ModQ m) {
+template <int NS, class F>
+__device__ __forceinline__ void slab_forward(const __amdgpu_buffer_rsrc_t limb, const Tw *__restrict__ tw_int, const F f, u64 *lds_raw,
+                                             const SlabPlace &at, const Pieces (&c)[NS][4], const DotCst (&h)[NS], const ModQ m) {
     typedef typename F::E E;
     const typename F::W *tw = (const typename F::W *)tw_int;
     E *lds = (E *)lds_raw;
-    const int cc = threadIdx.x & 15, rh = threadIdx.x >> 4;
-    E x[16];
+    const SlabLane lane;
+    E x[4];
 #pragma unroll
-    for (int k = 0; k < 16; k++) {
+    for (int k = 0; k < 4; k++) {
         Dot2 d;
         dot_clear(d);
-        if (LDS) dot_add(d, lsrc[k * 256 + threadIdx.x], hl);
 #pragma unroll
-        for (int j = SLAB_REG_SOURCES - NREG; j < SLAB_REG_SOURCES; j++) dot_add(d, c[j][k], h[j]);
+        for (int i = 0; i < NS; i++) dot_add(d, c[i][k], h[i]);
         x[k] = f.from_dot(d, m);
     }
-    radix_fwd<4>(f, x, tw, 1u);
+    radix_fwd<4>(f, x, tw, 1u, lane.h);
+#pragma unroll
+    for (int k = 0; k < 4; k++) lds[at.outer(k)] = x[k];
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 16; k++) lds[swz_row(rh + 16 * k) * 16 + cc] = x[k];
-    __syncthreads();
+    for (int k = 0; k < 4; k++) x[k] = lds[at.within(k)];
+    radix_fwd<4>(f, x, tw, lane.group, lane.h);
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = lds[swz_row(16 * rh + k) * 16 + cc];
-    radix_fwd<4>(f, x, tw, 16u + rh);
-#pragma unroll
-    for (int k = 0; k < 16; k++) buf_store<E>(limb, v_inner, (u32)k << 11, x[k]);
+    for (int k = 0; k < 4; k++) buf_store<E>(limb, at.v_inner, (u32)k << 11, x[k]);
 }
 
-template <int NREG, bool LDS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void ntt16_slab_convert_kernel(
-    u64 *__restrict__ data, const size_t poly_stride, const Tw *__restrict__ tw_all, const Tw *__restrict__ itw_all,
-    const ModQ *__restrict__ modq, const u64 *__restrict__ ninv, const u64 *__restrict__ ninv_s,
-    const double *__restrict__ fp, const SlabSources ss) {
-    __shared__ u64 lds[256 * 16];
-    __shared__ u64 lsrc[256 * 16];
-    const int poly = blockIdx.y;
-    const u32 col = blockIdx.x * 16 + (threadIdx.x & 15);
-    const u32 v_inner = (col + ((u32)(threadIdx.x >> 4) << 12)) * 8u;   // (row 16 rh, col); row k further: scalar offset
-    constexpr int n_lds = LDS ? 1 : 0, n_src = NREG + n_lds, first_reg = SLAB_REG_SOURCES - NREG;
-    u64 c[SLAB_REG_SOURCES][16];
+__device__ __forceinline__ void slab_load(const u64 *__restrict__ src, const SlabSources &ss, const SlabPlace &at, const int i, u64 (&next)[4]) {
+    const __amdgpu_buffer_rsrc_t limb = limb_rsrc(src + ((size_t)table_byte(ss.src_slot, i) << 16));
 #pragma unroll
-    for (int j = 0; j < SLAB_REG_SOURCES; j++)
-#pragma unroll
-        for (int k = 0; k < 16; k++) c[j][k] = 0;
-    // source i < n_lds goes to LDS, the others shift through the register sets: the last source ends in c[3]
-#pragma unroll 1
-    for (int i = 0; i < n_src; i++) {
-        const int prime = __builtin_amdgcn_readfirstlane((int)ss.src_prime[i]);
-        const __amdgpu_buffer_rsrc_t limb = limb_rsrc(
-            ss.src + (size_t)poly * ss.src_poly_stride + ((size_t)__builtin_amdgcn_readfirstlane((int)ss.src_slot[i]) << 16));
+    for (int k = 0; k < 4; k++) next[k] = buf_load<u64>(limb, at.v_inner, (u32)k << 11);
+}
+// sources I, I + 1, ... of NS; the next one's loads are in flight under a source's butterflies
+template <int I, int NS>
+__device__ __forceinline__ void slab_sources(const u64 *__restrict__ src, const SlabSources &ss, const Tw *__restrict__ itw_all,
+                                             const ModQ *__restrict__ modq, const u64 *__restrict__ ninv, const u64 *__restrict__ ninv_s,
+                                             const double *__restrict__ fp, u64 (&lds)[2][2048], const SlabPlace &at, u64 (&next)[4],
+                                             Pieces (&c)[NS][4]) {
+    if constexpr (I < NS) {
+        const int prime = (int)table_byte(ss.src_prime, I);
         const Tw *tw = itw_all + ((size_t)prime << 16);
-        const Tw fs = ss.final_scale[i];
-        if (i >= n_lds) {
+        const Tw fs = ss.final_scale[I];
+        u64 raw[4];
 #pragma unroll
-            for (int k = 0; k < 16; k++) {
-                c[0][k] = c[1][k];
-                c[1][k] = c[2][k];
-                c[2][k] = c[3][k];
-            }
-        }
+        for (int k = 0; k < 4; k++) raw[k] = next[k];
+        if (I + 1 < NS) slab_load(src, ss, at, I + 1, next);
         if (fp[4 * prime] != 0.0) {
             FpField f(modq, ninv, ninv_s, fp, prime);
             f.set_scale(fs);
-            slab_inverse(limb, v_inner, tw, f, lds, c[3]);
+            slab_inverse(raw, tw, f, lds[I & 1], at, c[I]);
         } else {
             with_field_60(modq, ninv, ninv_s, fp, prime, [&](auto f) {
                 f.set_scale(fs);
-                slab_inverse(limb, v_inner, tw, f, lds, c[3]);
+                slab_inverse(raw, tw, f, lds[I & 1], at, c[I]);
             });
         }
-        if (i < n_lds) {
-#pragma unroll
-            for (int k = 0; k < 16; k++) lsrc[k * 256 + threadIdx.x] = c[3][k];
-        }
+        slab_sources<I + 1>(src, ss, itw_all, modq, ninv, ninv_s, fp, lds, at, next, c);
     }
+}
+
+template <int NS>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 8))) void ntt16_slab_convert_kernel(
+    u64 *__restrict__ data, const size_t poly_stride, const Tw *__restrict__ tw_all, const Tw *__restrict__ itw_all,
+    const ModQ *__restrict__ modq, const u64 *__restrict__ ninv, const u64 *__restrict__ ninv_s,
+    const double *__restrict__ fp, const SlabSources ss) {
+    // Two exchange buffers in turn: a limb's exchange needs one barrier, since the one before the last is behind it for every wave
+    __shared__ u64 lds[2][2048];
+    const SlabPlace at;
+    const int poly = blockIdx.y;
+    const u64 *src = ss.src + (size_t)poly * ss.src_poly_stride;
+    Pieces c[NS][4];
+    u64 next[4];
+    slab_load(src, ss, at, 0, next);
+    slab_sources<0>(src, ss, itw_all, modq, ninv, ninv_s, fp, lds, at, next, c);
 #pragma unroll 1
     for (int t = 0; t < ss.n_dst; t++) {
-        const int prime = __builtin_amdgcn_readfirstlane((int)ss.dst_prime[t]);
-        const __amdgpu_buffer_rsrc_t limb = limb_rsrc(
-            data + (size_t)poly * poly_stride + ((size_t)__builtin_amdgcn_readfirstlane((int)ss.dst_slot[t]) << 16));
-        const Tw *tw = tw_all + ((size_t)prime << 16);
-        const ModQ m = modq[prime];
-        const Cst *hat = ss.hat + prime;
-        DotCst h[SLAB_REG_SOURCES];
+        const __amdgpu_buffer_rsrc_t limb = limb_rsrc(data + (size_t)poly * poly_stride + ((size_t)t << 16));
+        const Tw *tw = tw_all + ((size_t)t << 16);
+        const ModQ m = modq[t];
+        const Cst *hat = ss.hat + t;
+        DotCst h[NS];
 #pragma unroll
-        for (int j = 0; j < SLAB_REG_SOURCES; j++) {
-            const int i = n_lds + j - first_reg;
-            const Cst hg = j >= first_reg ? hat[(size_t)i * ss.hat_ld] : Cst{0, 0};
-            h[j] = dot_cst(hg.w, hg.ws);
+        for (int i = 0; i < NS; i++) {
+            const Cst hg = hat[(size_t)i * ss.hat_ld];
+            h[i] = dot_cst(hg.w, hg.ws);
         }
-        const DotCst hl = dot_cst(LDS ? hat[0].w : 0, LDS ? hat[0].ws : 0);
-        if (fp[4 * prime] != 0.0)
-            slab_forward<NREG, LDS>(limb, v_inner, tw, FpField(modq, ninv, ninv_s, fp, prime), lds, lsrc, hl, c, h, m);
+        u64 *buffer = lds[(NS + t) & 1];
+        if (fp[4 * t] != 0.0)
+            slab_forward<NS>(limb, tw, FpField(modq, nullptr, nullptr, fp, t), buffer, at, c, h, m);
         else
-            with_field_60(modq, ninv, ninv_s, fp, prime, [&](const auto f) { slab_forward<NREG, LDS>(limb, v_inner, tw, f, lds, lsrc, hl, c, h, m); });
+            with_field_60(modq, nullptr, nullptr, fp, t, [&](const auto f) { slab_forward<NS>(limb, tw, f, buffer, at, c, h, m); });
     }
 }
 
@@ -806,61 +828,80 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
     return true;
 }
 
-// out[p][j] = (y[p][j] - conversion of the n_src listed limbs of y[p] to prime j) * cst[j] for j < nq_out, in three
-// launches: first pass of the inverse transform of the listed limbs (in place), the column-slab kernel (second inverse
-// pass, conversion, first forward pass into conv), second forward pass with the fused tail.  Same residues as the
-// four-launch chain.  false when the shape has no such form (nothing was launched).
+// The slab kernel saves two trips of every source limb and a launch, and keeps few workgroups, 32 per polynomial of which 512 are
+// resident, busy for as long as there are targets.  Whole ModDowns in four launches / with it, us (sources -> targets; primes of 42 bits in the
+// chain, then 60):
+//   polynomials      4            6            8            12           16             20             32             64
+//   42 bits   5->3   35.7/ 34.2   43.3/ 39.2   49.0/ 44.3   65.0/ 60.6    76.6/ 68.6     89.7/ 86.6    126/118        268/241
+//             5->7   42.4/ 46.9   54.3/ 53.5   63.5/ 59.1   84.2/ 82.6   102.3/ 95.2    123.7/122.7    194/186        410/383
+//             4->8   41.4/ 48.0   52.1/ 53.5   64.1/ 61.1   81.2/ 82.5    99.4/ 95.0    120.7/124.1    193/188        398/408
+//             2->5   29.9/ 30.6   38.0/ 36.5   42.9/ 41.4   55.3/ 52.0    68.3/ 60.2     79.7/ 73.3    109/102        216/205
+//             5->12  51.9/ 63.0   69.4/ 73.1   82.0/ 82.1  109.3/112.6   142.6/133.4    173.8/180.5    283/281        586/592
+//   60 bits   5->7   44.0/ 51.6   57.2/ 59.2   66.9/ 64.8   89.2/ 89.5   106.2/100.4    132.0/132.4    202/196        426/399
+//             3->6   36.2/ 42.6   46.2/ 48.8   52.7/ 53.4   74.9/ 70.5    82.7/ 79.0     99.3/ 96.9    147/139        299/286
+//             5->12  54.7/ 72.2   74.8/ 84.5   86.9/ 92.8  115.2/122.1   149.9/145.5    185.6/197.7    299/297        612/626
+//             4->20  68.3/100     91.0/111      112/124      161/174       212/218                     439/491        874/975
+// So: eight polynomials and more and up to three targets more than sources; up to twelve where the workgroups are one nearly full round, and with
+// five sources from 28 polynomials on, which alone is even and in an attention block, beside another chain, 1.3 % of it.
+// Product of two encrypted matrices 2017 -> 1987 us, plaintext product 468 -> 456, projection of a 768-wide layer 9555 -> 9280, attention
+// block 19708 -> 19392.
+bool takes_moddown_slab(const hemm_context *c, int n_src, int nq_out, int n_polys) {
+    if (c->logN != 16 || n_src < 2 || n_src > SLAB_MAX_SOURCES) return false;
+    if (nq_out <= n_src + 3) return n_polys >= 8;
+    return nq_out <= 12 && ((n_polys > 12 && n_polys <= 16) || (n_src == 5 && n_polys >= 28));
+}
+
 bool launch_moddown_slab(const hemm_context *c, u64 *y, size_t y_stride, const uint8_t *src_slot, const uint8_t *src_prime,
                          int n_src, const void *final_scale_dev, const void *hat_dev, int hat_ld, u64 *conv, int nq_out,
-                         int n_polys, u64 *out, size_t out_stride, const void *cst_dev, hipStream_t s) {
-    if (c->logN != 16 || n_src < 4 || n_src > 5 || nq_out < 1 || nq_out > HEMM_MAX_PRIMES) return false;
+                         int n_polys, u64 *out, size_t out_stride, const void *cst_dev, hipStream_t s, const ResultList *list,
+                         bool rows_done, bool cols_only) {
+    if (c->logN != 16 || n_src < 2 || n_src > SLAB_MAX_SOURCES || nq_out < 1 || nq_out > c->nQ || n_polys > 65535) return false;
     if (n_polys <= 0) return true;
+    if (list != nullptr && n_polys > 2 * RESULT_PARTS) throw std::invalid_argument("too many results for one list");
     SlabSources ss;
     memset(&ss, 0, sizeof(ss));
-    LimbList sp, ssl, cl, ident;
+    LimbList sp, ssl, ident;
     memset(&sp, 0, sizeof(sp));
     memset(&ssl, 0, sizeof(ssl));
-    for (int j = 0; j < HEMM_MAX_PRIMES; j++) cl.idx[j] = ident.idx[j] = (uint8_t)j;
+    for (int j = 0; j < HEMM_MAX_PRIMES; j++) ident.idx[j] = (uint8_t)j;
     for (int i = 0; i < n_src; i++) {
         ss.src_slot[i] = ssl.idx[i] = src_slot[i];
         ss.src_prime[i] = sp.idx[i] = src_prime[i];
     }
-    for (int j = 0; j < nq_out; j++) {
-        ss.dst_slot[j] = (uint8_t)j;
-        ss.dst_prime[j] = (uint8_t)j;
-    }
+    ss.src_poly_stride = y_stride;
     ss.hat = (const Cst *)hat_dev;
     ss.final_scale = (const Tw *)final_scale_dev;
     ss.hat_ld = hat_ld;
     ss.n_src = n_src;
     ss.n_dst = nq_out;
-    ss.src_poly_stride = y_stride;
     // same algorithmic bytes as the separate launches: the dropped limbs in and out of the inverse transform, the
     // conversion's sources, the minuend in and the result out of the forward transform
-    account(c, TR_NTT, (size_t)2 * n_src * n_polys * c->N * 8, 1);
-    account(c, TR_BCONV, (size_t)n_src * n_polys * c->N * 8, 1);
-    account(c, TR_NTT, (size_t)2 * nq_out * n_polys * c->N * 8, 1);
-    const dim3 block(256);
+    account(c, TR_NTT, (size_t)2 * n_src * n_polys * c->N * 8, rows_done ? 1 : 2);
+    account(c, TR_BCONV, (size_t)n_src * n_polys * c->N * 8, 0);
+    account(c, TR_NTT, (size_t)(cols_only ? 1 : 2) * nq_out * n_polys * c->N * 8, cols_only ? 0 : 1);
     const size_t conv_stride = (size_t)nq_out << 16;
-    const int widest = n_src > nq_out ? n_src : nq_out;
-    int run = 448 / widest;
-    if (run < 1) run = 1;
+    // runs whose limbs the memory-side cache holds between the launches, as in polys_per_run
+    const int run = rows_done && cols_only ? n_polys : std::max(1, 448 / std::max(n_src, nq_out));
     for (int p0 = 0; p0 < n_polys; p0 += run) {
-        const int np = n_polys - p0 < run ? n_polys - p0 : run;
-        u64 *yp = y + (size_t)p0 * y_stride;
-        u64 *cp = conv + (size_t)p0 * conv_stride;
+        const int np = std::min(run, n_polys - p0);
+        u64 *yp = y + (size_t)p0 * y_stride, *cp = conv + (size_t)p0 * conv_stride;
         ss.src = yp;
-        rows_pass(c, true, yp, sp, ssl, n_src, np, y_stride, s, NttEpilogue{});
-#define SLAB_CASE(NREG, LDS)                                                                                             \
-    hipLaunchKernelGGL((ntt16_slab_convert_kernel<NREG, LDS>), dim3(16, np), block, 0, s, cp, conv_stride,             \
-                       (const Tw *)c->d_w, (const Tw *)c->d_iw, c->d_modq, c->d_ninv, c->d_ninv_s, c->d_fp, ss)
-        if (n_src == 5)
-            SLAB_CASE(4, true);
-        else
-            SLAB_CASE(4, false);
+        if (!rows_done) rows_pass(c, true, yp, sp, ssl, n_src, np, y_stride, s, NttEpilogue{});
+        const dim3 grid(32, (unsigned)np), block(512);
+#define SLAB_CASE(NS)                                                                                                         \
+    hipLaunchKernelGGL((ntt16_slab_convert_kernel<NS>), grid, block, 0, s, cp, conv_stride, (const Tw *)c->d_w,      \
+                       (const Tw *)c->d_iw, c->d_modq, c->d_ninv, c->d_ninv_s, c->d_fp, ss)
+        switch (n_src) {
+            case 2: SLAB_CASE(2); break;
+            case 3: SLAB_CASE(3); break;
+            case 4: SLAB_CASE(4); break;
+            default: SLAB_CASE(5);
+        }
 #undef SLAB_CASE
-        rows_pass(c, false, cp, cl, ident, nq_out, np, conv_stride, s,
-                  sub_scale_tail(yp, y_stride, out + (size_t)p0 * out_stride, out_stride, cst_dev), TAIL_SUB_SCALE);
+        if (cols_only) continue;
+        rows_pass(c, false, cp, ident, ident, nq_out, np, conv_stride, s,
+                  sub_scale_tail(yp, y_stride, list != nullptr ? nullptr : out + (size_t)p0 * out_stride, out_stride, cst_dev),
+                  TAIL_SUB_SCALE, LOAD_PLAIN, list, p0);
     }
     return true;
 }

@@ -390,8 +390,7 @@ struct StagePairs {
 // T Cooley-Tukey stages on 16 points that are 16 >> T sub-blocks of 2^T consecutive ones; stage s, group g uses twiddle
 // tw(s, g).  Points come in as `split` and leave as `whole`.
 template <int T, int P, class F, class TW>
-__device__ __forceinline__ void stages_fwd(const F &f, typename F::E (&x)[P], const TW tw) {
-    const u32 h = Lanes<P>::h();
+__device__ __forceinline__ void stages_fwd(const F &f, typename F::E (&x)[P], const TW tw, const u32 h = Lanes<P>::h()) {
 #pragma unroll
     for (int s = 0; s < T; s++) {
         const int d = 1 << (T - 1 - s);
@@ -408,8 +407,7 @@ __device__ __forceinline__ void stages_fwd(const F &f, typename F::E (&x)[P], co
 }
 // T Gentleman-Sande stages, the other way round: `whole` in, `split` out; stage s has distance 1 << s.
 template <int T, int P, class F, class TW>
-__device__ __forceinline__ void stages_inv(const F &f, typename F::E (&x)[P], const TW tw) {
-    const u32 h = Lanes<P>::h();
+__device__ __forceinline__ void stages_inv(const F &f, typename F::E (&x)[P], const TW tw, const u32 h = Lanes<P>::h()) {
 #pragma unroll
     for (int s = 0; s < T; s++) {
         const int d = 1 << s;
@@ -428,15 +426,15 @@ __device__ __forceinline__ void stages_inv(const F &f, typename F::E (&x)[P], co
 // sub-blocks are different columns of one block and share its twiddles.
 template <int T, bool SAME = false, int P, class F>
 __device__ __forceinline__ void radix_fwd(const F &f, typename F::E (&x)[P], const typename F::W *__restrict__ tw,
-                                          const u32 X) {
-    stages_fwd<T>(f, x, [&](const int s, const u32 g) { return tw[(X << s) + (SAME ? g & ((1u << s) - 1u) : g)]; });
+                                          const u32 X, const u32 h = Lanes<P>::h()) {
+    stages_fwd<T>(f, x, [&](const int s, const u32 g) { return tw[(X << s) + (SAME ? g & ((1u << s) - 1u) : g)]; }, h);
 }
 template <int T, bool SAME = false, int P, class F>
 __device__ __forceinline__ void radix_inv(const F &f, typename F::E (&x)[P], const typename F::W *__restrict__ tw,
-                                          const u32 X) {
+                                          const u32 X, const u32 h = Lanes<P>::h()) {
     stages_inv<T>(f, x, [&](const int s, const u32 g) {
         return tw[(X << (T - 1 - s)) + (SAME ? g & ((1u << (T - 1 - s)) - 1u) : g)];
-    });
+    }, h);
 }
 
 // The inner radix-16 block of a row pass (X = 16 (R + r) + c: a different X for every thread) reads its 15 twiddles

@@ -45,6 +45,12 @@ def test_converted_and_lifted_column_passes():
     assert _forms("ntt16_cols_converted_kernel", 4) == {f + (k,) for f in half | whole | {(5, 4, 2), (6, 4, 2)} for k in (2, 5, 8)}
 
 
+def test_column_slabs():
+    """Sources kept in registers."""
+    with open(os.path.join(PKG_DIR, "libhemm.so"), "rb") as f:
+        assert set(re.findall(rb"25ntt16_slab_convert_kernelILi([0-9]+)E", f.read())) == {b"2", b"3", b"4", b"5"}
+
+
 def test_embedding_rows():
     """Log2 of the rows, decoding, rows of a workgroup: eight for batches of messages, and a decoding is one."""
     two = {(lr, decode, 2) for lr in range(1, 8) for decode in (0, 1)}
