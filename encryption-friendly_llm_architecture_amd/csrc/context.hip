@@ -128,7 +128,7 @@ hemm_context *hemm_context_build(int logN, int nQ, int nP, const u64 *primes, in
         u64 *wt = w.data() + (size_t)i * N * 2, *iwt = iw.data() + (size_t)i * N * 2;
         // Primes below 2^44 run the register-blocked transforms in double precision (exact: see ntt.hip); their
         // table is the N twiddles as doubles, packed into the first half of the prime's region (8 bytes per twiddle
-        // instead of 16: the row passes read as many twiddle bytes as data, and the quotient w / q costs one multiply).
+        // instead of 16: the row passes read as many twiddle bytes as data, and a product needs no quotient of its own).
         const bool fp = ring_has_fused_forms(c) && (q >> 44) == 0;
         const bool near = ring_has_fused_forms(c) && near_2_60(q);   // w and 2^32 w mod q (Near60Field)
         auto as_bits = [](double d) {
