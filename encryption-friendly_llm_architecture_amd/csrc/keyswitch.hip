@@ -1968,9 +1968,11 @@ void launch_hoisted_moddown(hemm_context *c, const HoistedList &l, int n_out, in
     //                 46.3/63.8   55.5/54.6  79.8/82.0   98.3/103    128.5/127.5 158/162     225/217     435/418
     // (rotation at N = 2^13, 128 workgroups: 45.0/47.4; on 24 primes of 60 bits, level 20, 3200: 147.2/144.1)
     const size_t wgs = (size_t)n_out * E * (N / 512);
+    const bool compact = l.n_terms > 0 && (((const RotTermDev *)l.terms)[0].flags & ROT_TERM_COMPACT_KEY) != 0;
+    const size_t key_words = (size_t)c->dnum * 2 * (compact ? (size_t)c->key_off.back() * N / 4 : (size_t)(c->nQ + K) * N);
     const bool tail = rows && (wgs >= 4096 || (wgs >= 1024 && l.n_terms <= 2 * n_out)) && ns <= CONV_MAX_SOURCES && lazy_dot_ok(c) && !one_launch(c, (size_t)2 * group * nq_out, false) &&
                       (size_t)2 * group * nq_out <= 65535 &&
-                      tail_may_sum(l, n_out, N, nq, E, beta, (size_t)c->dnum * 2 * (c->nQ + K) * N, out, out_stride, outs, conv,
+                      tail_may_sum(l, n_out, N, nq, E, beta, key_words, out, out_stride, outs, conv,
                                    (size_t)n_out * 2 * nq_out * N, nq_out);
     account(c, TR_KEYPROD, hoisted_bytes(c, (const RotTermDev *)l.terms, l.n_terms, n_out, nq));
     LimbList all, dropped, kept;
