@@ -4,7 +4,7 @@
 // walks (poly, limb) so every wavefront streams one contiguous 4 KiB run.
 #include <algorithm>
 
-#include "hemm_internal.hpp"
+#include "hoisted.h"
 
 namespace {
 
@@ -88,20 +88,41 @@ __global__ __launch_bounds__(256) void scalar_add_kernel(Operand a, u64 *__restr
     *(ulonglong2 *)(out + e) = make_ulonglong2(addmod(x.x, c, q), addmod(x.y, c, q));
 }
 
-// (b1,a1) x (b2,a2) -> (b1 b2, a1 b2 + a2 b1, a1 a2); ACC adds into out.
+// (b1,a1) x (b2,a2) -> (b1 b2, a1 b2 + a2 b1, a1 a2); ACC adds into out.  In double precision for primes below 2^44, in pieces just below
+// 2^60: ten limbs of the 42-bit chain 7.3 us instead of 8.8 with 128-bit products and a Barrett step each, product at level 9 95.5 -> 94.5.
 template <bool ACC>
 __global__ __launch_bounds__(256) void tensor_kernel(Operand c1, Operand c2, u64 *__restrict__ out, size_t out_stride,
-                                                     const ModQ *__restrict__ modq, int logN) {
+                                                     const ModQ *__restrict__ modq, const double *__restrict__ fp, int logN) {
     const int limb = blockIdx.y;
     const ModQ m = modq[limb];
+    const FpMod f{fp[4 * limb], fp[4 * limb + 1]};
     const size_t e = ((size_t)limb << logN) + (size_t)blockIdx.x * 256 + threadIdx.x;
     const u64 b1 = c1.p[e], a1 = c1.p[c1.poly_stride + e];
     const u64 b2 = c2.p[e], a2 = c2.p[c2.poly_stride + e];
-    u64 d0 = mulmod(b1, b2, m);
-    u128_t t = mul64wide(a1, b2);
-    add128(t, mul64wide(a2, b1));
-    u64 d1 = barrett128(t, m);
-    u64 d2 = mulmod(a1, a2, m);
+    u64 d0, d1, d2;
+    if (f.q != 0.0) {
+        const double x1 = u64_to_double(b1), y1 = u64_to_double(a1), x2 = u64_to_double(b2), y2 = u64_to_double(a2);
+        d0 = f.canonical(f.mul(x1, x2));
+        d1 = f.canonical(f.mul(y1, x2) + f.mul(y2, x1));
+        d2 = f.canonical(f.mul(y1, y2));
+    } else if (near_2_60(m.q)) {
+        const Near60 near(m.q);
+        const Pieces x1 = pieces(b1), y1 = pieces(a1), x2 = pieces(b2), y2 = pieces(a2);
+        Acc3 t0{0, 0, 0}, t1{0, 0, 0}, t2{0, 0, 0};
+        acc_mul(t0, x1, x2);
+        acc_mul(t1, y1, x2);
+        acc_mul(t1, y2, x1);
+        acc_mul(t2, y1, y2);
+        d0 = near.canonical(near.fold(near.reduce(t0)));
+        d1 = near.canonical(near.fold(near.reduce(t1)));
+        d2 = near.canonical(near.fold(near.reduce(t2)));
+    } else {
+        d0 = mulmod(b1, b2, m);
+        u128_t t = mul64wide(a1, b2);
+        add128(t, mul64wide(a2, b1));
+        d1 = barrett128(t, m);
+        d2 = mulmod(a1, a2, m);
+    }
     if (ACC) {
         d0 = addmod(d0, out[e], m.q);
         d1 = addmod(d1, out[out_stride + e], m.q);
@@ -208,9 +229,9 @@ void launch_tensor(const hemm_context *c, const u64 *c1, size_t s1, const u64 *c
     Operand A{c1, s1}, B{c2, s2};
     account(c, TR_TENSOR, (size_t)(accumulate ? 10 : 7) * nq * c->N * 8);
     if (accumulate)
-        hipLaunchKernelGGL(tensor_kernel<true>, grid, block, 0, s, A, B, out, out_stride, c->d_modq, c->logN);
+        hipLaunchKernelGGL(tensor_kernel<true>, grid, block, 0, s, A, B, out, out_stride, c->d_modq, c->d_fp, c->logN);
     else
-        hipLaunchKernelGGL(tensor_kernel<false>, grid, block, 0, s, A, B, out, out_stride, c->d_modq, c->logN);
+        hipLaunchKernelGGL(tensor_kernel<false>, grid, block, 0, s, A, B, out, out_stride, c->d_modq, c->d_fp, c->logN);
 }
 
 void launch_galois(const hemm_context *c, const u64 *a, size_t a_stride, u64 *out, size_t out_stride, u64 g,
