@@ -582,6 +582,8 @@ static bool few_for_conversions(const hemm_context *c, int limbs) { return (size
 //   60 bits, level 10 (384)             82.2/80.6/75.2/75.2/75.4  124.4/120.7/113.9/114.1/113.9
 //                  18 (608, 784)       117.3/117.3/117.0/114.9/113.9  170.3/170.3/170.4/168.2/167.4
 //                  23 (768, 960)       130.2/130.2/130.2/130.6/131.6  191.2/191.2/191.5/191.6/192.7
+// In the arithmetic of primes just below 2^60, lines at 768 / 1024: 60 bits, level 16 (736) 98.6/98.8, 18 (800) 105.3/104.2, 20 (864) 113.5/111.9,
+// 22 (944) 117.8/118.8, 23 (976) 120.0/120.7; 24 + 6 primes of 42 bits, level 18 (800) 109.2/106.9.
 // The products of matrices, whose large conversions run beside other chains, are 1 - 3 % slower with all of them on half slabs.
 // Smaller rings, transforms of 42 bits (forward, inverse) with whole slabs of sixteen points / half slabs / quarter slabs of four:
 //   limbs         1                             4                             16                            32                              48                                64
@@ -596,7 +598,7 @@ static bool few_for_conversions(const hemm_context *c, int limbs) { return (size
 // would lead.)
 static int narrower_slabs(const hemm_context *c, int limbs, bool plain = false, bool inverse = false) {
     const size_t wgs = (size_t)limbs * (c->N >> 12);
-    if (c->logN == 16) return wgs <= (plain ? 384 : 768) ? 1 : 0;
+    if (c->logN == 16) return wgs <= (plain ? 384 : 880) ? 1 : 0;
     if (c->logN == 15 && plain && !inverse && wgs > 128) return 0;
     return c->logN <= 14 && wgs <= 128 ? 2 : wgs <= 512 ? 1 : 0;
 }
