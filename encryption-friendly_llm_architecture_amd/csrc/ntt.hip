@@ -543,7 +543,8 @@ void launch_limb_inverse(const hemm_context *c, u64 *data, const LimbList &ll, c
 //                     42 bits  10.2/ 9.3/ 8.5   12.0/11.0/11.1   17.0/16.7/16.5   22.8/22.1/21.9   26.6/26.2/25.7   25.2/24.7/25.0   29.0/29.1/29.5
 static bool few_for_columns(const hemm_context *c, int limbs) { return (size_t)limbs * (c->N >> 12) <= 512; }
 // Row passes: four points have eight wavefronts per SIMD, all resident up to 512 workgroups of 4096 points, and lead up to 640; eight points
-// lead from there to about 1000.  Encodings of 2^14 points leave four at 512 and eight, for sixteen, at 640.  us with sixteen / eight /
+// lead from there to about 1000 (figures below; further since the butterflies take fewer
+// instructions, table after it).  Encodings of 2^14 points leave four at 512 and eight, for sixteen, at 640.  us with sixteen / eight /
 // four points, the second figure of each pair 42 bits:
 //   workgroups                        544                              640                              768                              896
 //   forward, 2^16 points   33.3/32.8/31.5 28.5/28.1/27.2  28.5/27.3/27.0 24.4/23.2/23.5  30.1/29.7/29.5 23.9/23.6/24.0  34.5/33.6/33.6 26.8/25.5/26.7
@@ -554,11 +555,19 @@ static bool few_for_columns(const hemm_context *c, int limbs) { return (size_t)l
 //            2^15          46.1/42.4/41.6 38.1/35.2/34.6  46.7/43.9/43.9 39.7/36.2/35.9  48.8/46.0/46.6 41.4/37.6/38.6
 //   encodings of 2^14 points, m messages x limbs: 11x12 34.8/34.5/34.9, 23x6 37.9/36.6/37.6, 26x6 38.6/37.2/38.2, 32x5 37.6/37.3/38.7, 32x6 38.5/38.1/39.4,
 //   64x3 39.9/39.9/41.1, 16x13 37.4/39.2/40.3; of 2^16 4x13 40.8/39.5/40.3, 9x6 42.4/41.3/42.2
+// Forward passes beyond 900 workgroups, sixteen / eight points, with the present butterflies (60 bits: of primes just below 2^60):
+//   2^16 points, workgroups           960        1280       1536       1792       3072 (runs)  | ModDowns, tails of 960 / 1536 / 3072 / 5120
+//   60 bits                           29.9/28.8  37.7/35.9  42.1/41.0  46.3/46.1  293/297      | (42-bit chain) 70.4/68.5 88.3/86.6 167/164 301/301
+//   42 bits                           26.3/25.8  33.3/32.5  37.4/36.6  41.3/40.4  269/269      | encodings of 72 / 117 / 208 limbs 45.0/44.0 57.3/55.5 84.1/82.5
+//   2^15 points, 960 / 1280 / 1920 / 2560: 60 bits 30.0/29.1 38.5/38.2 53.0/51.4 63.2/63.2, 42 bits 25.8/25.3 34.0/33.4 46.3/45.3 57.8/56.0
+//   2^14 points: ModDowns of 16 / 32 polynomials 39.0/39.4 53.4/54.0 (its line stays at 900)
 static int points_for_rows(const hemm_context *c, int limbs, bool inverse, int tail) {
     const size_t wgs = (size_t)limbs * (c->N >> 12);
     const bool encoding = c->logN == 14 && !inverse && tail == TAIL_NONE;   // longer plain transforms of this ring are one launch
-    if (wgs <= (encoding ? 512 : 640)) return 4;
-    return inverse || wgs <= (encoding ? 640 : 900) ? 8 : 16;
+    if (wgs <= (encoding ? 512 : 640) || (tail == TAIL_ENCRYPT && c->logN < 16)) return 4;   // (an encryption's few limbs)
+    if (inverse) return 8;
+    if (c->logN >= 15) return tail == TAIL_NONE && wgs > 2560 ? 16 : 8;
+    return wgs <= (encoding ? 640 : 900) ? 8 : 16;
 }
 
 // Passes that begin in a basis conversion or a lift, on rings below 2^16 points: four points where every CU has one workgroup at most, eight
@@ -664,11 +673,11 @@ static void rows_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
         if (points == 4) ROWS_RING(4, true, TAIL_NONE, LOAD, ep); \
         else ROWS_RING(8, true, TAIL_NONE, LOAD, ep);            \
     } while (0)
-#define ROWS_FORWARD(TAIL, EP)                                   \
+#define ROWS_FORWARD(TAIL, EP, ROWS_16)                          \
     do {                                                         \
         if (points == 4) ROWS_RING(4, false, TAIL, LOAD_PLAIN, EP); \
         else if (points == 8) ROWS_RING(8, false, TAIL, LOAD_PLAIN, EP); \
-        else ROWS_RING(16, false, TAIL, LOAD_PLAIN, EP);         \
+        else ROWS_16;                                            \
     } while (0)
     if (inverse && load == LOAD_ROTATED)
         ROWS_INVERSE(LOAD_ROTATED);
@@ -678,13 +687,15 @@ static void rows_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
         ROWS_INVERSE(LOAD_PLAIN);
     else if (tail == TAIL_SUB_SCALE && list != nullptr) {
         const NttEpilogueList epl{ep, (u32)first, *list};
-        ROWS_FORWARD(TAIL_SUB_SCALE_LIST, epl);
+        ROWS_FORWARD(TAIL_SUB_SCALE_LIST, epl, ROWS(0, 16, false, TAIL_SUB_SCALE_LIST, LOAD_PLAIN, epl));
     } else if (tail == TAIL_SUB_SCALE)
-        ROWS_FORWARD(TAIL_SUB_SCALE, ep);
+        ROWS_FORWARD(TAIL_SUB_SCALE, ep, ROWS(0, 16, false, TAIL_SUB_SCALE, LOAD_PLAIN, ep));   // (2^14 points and fewer)
+    else if (tail == TAIL_ENCRYPT && points == 4)   // 64 limbs at most: eight points at 2^16 alone
+        ROWS_RING(4, false, TAIL_ENCRYPT, LOAD_PLAIN, ep);
     else if (tail == TAIL_ENCRYPT)
-        ROWS_FORWARD(TAIL_ENCRYPT, ep);
+        ROWS(8, 8, false, TAIL_ENCRYPT, LOAD_PLAIN, ep);
     else
-        ROWS_FORWARD(TAIL_NONE, ep);
+        ROWS_FORWARD(TAIL_NONE, ep, ROWS_RING(16, false, TAIL_NONE, LOAD_PLAIN, ep));
 #undef ROWS_FORWARD
 #undef ROWS_INVERSE
 #undef ROWS_RING

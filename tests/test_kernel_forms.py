@@ -17,6 +17,9 @@ def test_row_passes():
     """Log2 of the rows (0: from the argument), points per thread, inverse."""
     points = {(4, 0), (8, 0), (16, 0), (4, 1), (8, 1)}
     assert _forms("ntt16_rows_kernel", 3) == {(lr,) + p for lr in (0, 8) for p in points}
+    # ... tail: sixteen points at 2^16 in plain passes alone, an encryption's (2) few limbs eight there at most
+    assert {f for f in _forms("ntt16_rows_kernel", 4) if f[3] in (1, 3) and not f[2]} == {(lr, p, 0, t) for t in (1, 3) for lr, p in ((0, 4), (8, 4), (0, 8), (8, 8), (0, 16))}
+    assert {f for f in _forms("ntt16_rows_kernel", 4) if f[3] == 2} == {(0, 4, 0, 2), (8, 4, 0, 2), (8, 8, 0, 2)}
     # what a decryption reads (the last argument, 2) is one or two limbs
     assert {f for f in _forms("ntt16_rows_kernel", 5) if f[4] == 2} == {(lr, 4, 1, 0, 2) for lr in (0, 8)}
 
