@@ -246,7 +246,7 @@ def gpu_ntt(args, out):
 # HBM bytes of one chain of the main loop at the shape below (its launches together), from two rocprofv3 --pmc runs of
 # `bench.py --roofline-only` (FETCH_SIZE, WRITE_SIZE), each scaled by what the same counter reads for the 1 GiB copy this mode also launches
 # (FETCH_SIZE x 2.0, WRITE_SIZE x 1.0): see profiles/main_loop_and_ntt_roofline_shapes.txt.
-CHAIN_TRAFFIC_BYTES = 1160764416
+CHAIN_TRAFFIC_BYTES = 993712128
 
 
 def gpu_hoisted(args, out):
@@ -304,8 +304,7 @@ def gpu_hoisted(args, out):
         groups.append([(src[t][0], src[t][1], evk, rnd(E, N >> shift, 2), gal, shift) for t in range(2)])
     ms = timed(lambda: ctx.hoisted_moddown(groups, nq, True, b_premultiplied=True, compact_keys=True))
     moved = n_out * (key_words_bytes(nq) + 2 * E * (N >> shift) * 16 + 2 * (nq - 1) * LIMB_BYTES) + 2 * (beta * E + nq) * LIMB_BYTES
-    out["roofline"] = entry("hoisted_terms_kernel<0, true, 1, SumRows> + ntt16_cols_kernel<8, 16, 0, true> + ntt16_cols_converted_kernel<8, 8, 0, 5> + "
-                            "hoisted_terms_kernel<0, true, 1, SumTail> (one chain of the CCMM main loop: 16 shifts of two masked sources under one compact key, "
+    out["roofline"] = entry("hoisted_terms_kernel<0, true, 1, SumRows> + ntt16_slab_convert_kernel<5> + hoisted_terms_kernel<0, true, 1, SumTail> (one chain of the CCMM main loop: 16 shifts of two masked sources under one compact key, "
                             "8+4 limbs, 2 digits, run-table masks, divided by P and rescaled to 7 limbs)", ms, moved, traffic=CHAIN_TRAFFIC_BYTES)
     nq = 9
     E = nq + K
@@ -320,8 +319,7 @@ def gpu_hoisted(args, out):
     y = rnd(16, nq + K, N)
     ms = timed(lambda: ctx.moddown_batch(y, nq, True))
     moved = 16 * (nq + K + nq - 1) * LIMB_BYTES
-    out["roofline_moddown"] = entry("ntt16_rows_kernel<8, 8, true, 0, 0> + ntt16_cols_kernel<8, 16, 0, true> + ntt16_cols_converted_kernel<8, 8, 0, 5> + "
-                                    "ntt16_rows_kernel<8, 16, false, 1, 0> (ModDown and rescale of the plaintext product's eight inner sums: 16 "
+    out["roofline_moddown"] = entry("ntt16_rows_kernel<8, 8, true, 0, 0> + ntt16_slab_convert_kernel<5> + ntt16_rows_kernel<8, 8, false, 1, 0> (ModDown and rescale of the plaintext product's eight inner sums: 16 "
                                     "polynomials, 6+4 -> 5 limbs)", ms, moved)
     if args.roofline_only:
         # a plain copy of known size in the same process: the scale reference for the --pmc counters
