@@ -161,7 +161,7 @@ hemm_context *hemm_context_build(int logN, int nQ, int nP, const u64 *primes, in
         fpc[4 * i + 0] = small ? (double)q : 0.0;
         fpc[4 * i + 1] = small ? 1.0 / (double)q : 0.0;
         fpc[4 * i + 2] = (double)ninv[i];
-        fpc[4 * i + 3] = (double)ninv[i] / (double)q;
+        fpc[4 * i + 3] = 0.0;
         ninv_s[i] = h_shoup(ninv[i], q);
         im[i] = pw[N / 2];
         im_s[i] = h_shoup(im[i], q);

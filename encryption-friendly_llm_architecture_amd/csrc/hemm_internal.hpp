@@ -41,7 +41,7 @@ struct hemm_context {
                                     // ((16 (N / 256 + r) + c) << l) + g of d_w / d_iw (nullptr for other ring sizes)
     u64 *d_ninv, *d_ninv_s;         // [prime]
     ModQ *d_modq;                   // [prime]
-    double *d_fp;                   // [prime][4]: q, 1/q, 1/N mod q, that / q as doubles; q = 0 marks a prime of
+    double *d_fp;                   // [prime][4]: q, 1/q, 1/N mod q as doubles, 0; q = 0 marks a prime of
                                     // 44 bits or more, which only the integer code paths handle
     u64 *d_imag, *d_imag_s;         // [prime] psi^(N/2) and Shoup quotient
     // scratch owned by the context (single stream use)
