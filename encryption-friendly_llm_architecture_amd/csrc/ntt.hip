@@ -113,18 +113,18 @@ struct Slab {
     static __device__ __forceinline__ constexpr u32 inner(const int k) { return (u32)k << 11; }
 };
 // the exchange and the second block of a forward column pass, results to memory
-template <int LR, int H = 0, int P, class F>
+template <int LR, int H = 0, int P, class F, class LANE = KeptLane>
 __device__ __forceinline__ void cols_forward(const __amdgpu_buffer_rsrc_t limb, const typename F::W *__restrict__ tw,
-                                             const F f, typename F::E (&x)[P], typename F::E *lds) {
+                                             const F f, typename F::E (&x)[P], typename F::E *lds, const LANE lane = LANE{Lanes<P>::h()}) {
     typedef typename F::E E;
     typedef Slab<LR, P, H> S;
-    radix_fwd<4>(f, x, tw, 1u);
+    radix_fwd<4>(f, x, tw, 1u, lane);
 #pragma unroll
     for (int k = 0; k < P; k++) lds[S::template at<false>(S::r_outer_w(k))] = x[k];
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < P; k++) x[k] = lds[S::template at<false>(S::r_inner_s(k))];
-    radix_fwd<S::T>(f, x, tw, S::group());
+    radix_fwd<S::T>(f, x, tw, S::group(), lane);
 #pragma unroll
     for (int k = 0; k < P; k++) buf_store<E>(limb, S::v_inner(), S::inner(k), x[k]);
 }
@@ -193,7 +193,7 @@ __device__ __forceinline__ void cols_converted_body(const __amdgpu_buffer_rsrc_t
     typename F::E x[P];
     // the row step goes into the scalar offset
     converted_inputs<NS>(f, x, src, S::v_outer(), so, h, n_src, m, [](const int k) { return S::outer(k); });
-    cols_forward<LR, H>(limb, (const typename F::W *)tw_int, f, x, (typename F::E *)lds_raw);
+    cols_forward<LR, H>(limb, (const typename F::W *)tw_int, f, x, (typename F::E *)lds_raw, OwnLane<P>{});
 }
 
 // What bounds it is the work of a column pass and the trips to memory in front of it.  Eight points per thread and 20 source
@@ -341,14 +341,14 @@ __device__ __forceinline__ void slab_inverse(const u64 (&raw)[4], const Tw *__re
     E x[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) __builtin_memcpy(&x[k], &raw[k], 8);
-    radix_inv<4>(f, x, tw, lane.group, lane.h);
+    radix_inv<4>(f, x, tw, lane.group, KeptLane{lane.h});
     f.template after_inverse_block<4>(x);
 #pragma unroll
     for (int k = 0; k < 4; k++) lds[at.within(k)] = x[k];
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 4; k++) x[k] = lds[at.outer(k)];
-    radix_inv<4>(f, x, tw, 1u, lane.h);
+    radix_inv<4>(f, x, tw, 1u, KeptLane{lane.h});
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         r[k] = pieces(f.scale_to_canonical(x[k]));
@@ -372,13 +372,13 @@ __device__ __forceinline__ void slab_forward(const __amdgpu_buffer_rsrc_t limb, 
         for (int i = 0; i < NS; i++) dot_add(d, c[i][k], h[i]);
         x[k] = f.from_dot(d, m);
     }
-    radix_fwd<4>(f, x, tw, 1u, lane.h);
+    radix_fwd<4>(f, x, tw, 1u, KeptLane{lane.h});
 #pragma unroll
     for (int k = 0; k < 4; k++) lds[at.outer(k)] = x[k];
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 4; k++) x[k] = lds[at.within(k)];
-    radix_fwd<4>(f, x, tw, lane.group, lane.h);
+    radix_fwd<4>(f, x, tw, lane.group, KeptLane{lane.h});
 #pragma unroll
     for (int k = 0; k < 4; k++) buf_store<E>(limb, at.v_inner, (u32)k << 11, x[k]);
 }

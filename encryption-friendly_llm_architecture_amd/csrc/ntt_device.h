@@ -383,10 +383,23 @@ struct StagePairs {
     __device__ __forceinline__ constexpr StagePairs(const int d, const bool split, const u32 h)
         : dist(!split ? d : P == 4 ? d / 4 : 4), first_group(!split ? h * (u32)(P / 2 / d) : 0u) {}
 };
+// The lane of a block of stages.  KeptLane: a number that the caller has; the stages are then simplified before its bits are known.  OwnLane: made
+// where the stages begin.  Inverse transforms take the second, 72 registers instead of 78 in the row pass of 2^16 points and 64 instead of 72 where
+// a limb is one launch (32 x 24 limbs of 2^13 points 28.3 -> 25.3 us, of 60 bits 34.5 -> 31.5), and so do conversions, of which eight sources on
+// 2^15 points spill 20 registers with the first.  The other forward transforms take the first (the same limbs 24.0 -> 23.1).
+struct KeptLane {
+    u32 h;
+    __device__ __forceinline__ u32 operator()() const { return h; }
+};
+template <int P>
+struct OwnLane {
+    __device__ __forceinline__ u32 operator()() const { return Lanes<P>::h(); }
+};
 // T Cooley-Tukey stages on 16 points that are 16 >> T sub-blocks of 2^T consecutive ones; stage s, group g uses twiddle
 // tw(s, g).  Points come in as `split` and leave as `whole`.
-template <int T, int P, class F, class TW>
-__device__ __forceinline__ void stages_fwd(const F &f, typename F::E (&x)[P], const TW tw, const u32 h = Lanes<P>::h()) {
+template <int T, int P, class F, class TW, class LANE = KeptLane>
+__device__ __forceinline__ void stages_fwd(const F &f, typename F::E (&x)[P], const TW tw, const LANE lane = LANE{Lanes<P>::h()}) {
+    const u32 h = lane();
 #pragma unroll
     for (int s = 0; s < T; s++) {
         const int d = 1 << (T - 1 - s);
@@ -402,8 +415,9 @@ __device__ __forceinline__ void stages_fwd(const F &f, typename F::E (&x)[P], co
     }
 }
 // T Gentleman-Sande stages, the other way round: `whole` in, `split` out; stage s has distance 1 << s.
-template <int T, int P, class F, class TW>
-__device__ __forceinline__ void stages_inv(const F &f, typename F::E (&x)[P], const TW tw, const u32 h = Lanes<P>::h()) {
+template <int T, int P, class F, class TW, class LANE = OwnLane<P>>
+__device__ __forceinline__ void stages_inv(const F &f, typename F::E (&x)[P], const TW tw, const LANE lane = LANE()) {
+    const u32 h = lane();
 #pragma unroll
     for (int s = 0; s < T; s++) {
         const int d = 1 << s;
@@ -420,17 +434,17 @@ __device__ __forceinline__ void stages_inv(const F &f, typename F::E (&x)[P], co
 }
 // Blocks on the stage-ordered table: forward stage s, group g: entry (X << s) + g; inverse: (X << (T - 1 - s)) + g.  SAME: the
 // sub-blocks are different columns of one block and share its twiddles.
-template <int T, bool SAME = false, int P, class F>
+template <int T, bool SAME = false, int P, class F, class LANE = KeptLane>
 __device__ __forceinline__ void radix_fwd(const F &f, typename F::E (&x)[P], const typename F::W *__restrict__ tw,
-                                          const u32 X, const u32 h = Lanes<P>::h()) {
-    stages_fwd<T>(f, x, [&](const int s, const u32 g) { return tw[(X << s) + (SAME ? g & ((1u << s) - 1u) : g)]; }, h);
+                                          const u32 X, const LANE lane = LANE{Lanes<P>::h()}) {
+    stages_fwd<T>(f, x, [&](const int s, const u32 g) { return tw[(X << s) + (SAME ? g & ((1u << s) - 1u) : g)]; }, lane);
 }
-template <int T, bool SAME = false, int P, class F>
+template <int T, bool SAME = false, int P, class F, class LANE = OwnLane<P>>
 __device__ __forceinline__ void radix_inv(const F &f, typename F::E (&x)[P], const typename F::W *__restrict__ tw,
-                                          const u32 X, const u32 h = Lanes<P>::h()) {
+                                          const u32 X, const LANE lane = LANE()) {
     stages_inv<T>(f, x, [&](const int s, const u32 g) {
         return tw[(X << (T - 1 - s)) + (SAME ? g & ((1u << (T - 1 - s)) - 1u) : g)];
-    }, h);
+    }, lane);
 }
 
 // The inner radix-16 block of a row pass (X = 16 (R + r) + c: a different X for every thread) reads its 15 twiddles

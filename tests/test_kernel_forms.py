@@ -13,6 +13,22 @@ def _forms(kernel, ints):
     return {tuple(int(x.replace(b"n", b"-")) for x in m) for m in mangled.findall(names)}
 
 
+def _scratch():
+    """Kernel (mangled name) -> bytes of scratch per lane, from the metadata of the library's kernels (MessagePack: a name, then its scratch)."""
+    with open(os.path.join(PKG_DIR, "libhemm.so"), "rb") as f:
+        held = f.read()
+    entry = re.compile(b"\xa5\\.name(?:\xd9.|\xda..|[\xa0-\xbf])(_Z\\w+)\xbb\\.private_segment_fixed_size(\xcd..|\xcc.|[\x00-\x7f])", re.S)
+    return {name.decode(): int.from_bytes(size[1:] or size, "big") for name, size in entry.findall(held)}
+
+
+def test_scratch():
+    """Registers spill in the kernels where fewer wavefronts were measured to cost more than that, and in no other."""
+    scratch = _scratch()
+    assert len(scratch) > 300
+    may = re.compile("diagonal_sums_kernelI|hoisted_terms_(list_)?kernelILi2E")
+    assert [name for name, size in scratch.items() if size and not may.search(name)] == []
+
+
 def test_row_passes():
     """Log2 of the rows (0: from the argument), points per thread, inverse."""
     points = {(4, 0), (8, 0), (16, 0), (4, 1), (8, 1)}
