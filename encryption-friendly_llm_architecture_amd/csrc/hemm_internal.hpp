@@ -205,8 +205,8 @@ bool launch_moddown_slab(const hemm_context *c, u64 *y, size_t y_stride, const u
                          int n_src, const void *final_scale_dev, const void *hat_dev, int hat_ld, u64 *conv, int nq_out,
                          int n_polys, u64 *out, size_t out_stride, const void *cst_dev, hipStream_t s, const ResultList *list = nullptr,
                          bool rows_done = false, bool cols_only = false);
-// whether that form is the faster one (N = 2^16, two to five sources)
-bool takes_moddown_slab(const hemm_context *c, int n_src, int nq_out, int n_polys);
+// whether that form is the faster one (N = 2^16, two to five sources); uncut: with rows_done and cols_only
+bool takes_moddown_slab(const hemm_context *c, int n_src, int nq_out, int n_polys, bool uncut);
 // inverse transform reading src (same slot numbering as data, polynomial stride src_poly_stride) and leaving the
 // coefficients in data; false when this ring size has no out-of-place form (the caller copies, then transforms)
 // galois != 0: src is read through that automorphism (the transform of the rotated polynomial, without a launch

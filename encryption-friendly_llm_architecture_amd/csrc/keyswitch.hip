@@ -1854,7 +1854,7 @@ void launch_moddown_batch(hemm_context *c, u64 *y, int nq, int n_polys, int drop
     if (slab && !(c->logN == 16 && lazy_dot_ok(c))) throw std::invalid_argument("the column-slab ModDown needs N = 2^16 and primes below 2^60");
     if (slab && (ns < 4 || ns > 5)) throw std::invalid_argument("the column-slab ModDown takes 4 or 5 dropped limbs");
     // inverse column pass, conversion and forward column pass as one kernel, where it is the faster form and on request
-    if ((slab || takes_moddown_slab(c, ns, nq_out, n_polys)) && lazy_dot_ok(c) &&
+    if ((slab || takes_moddown_slab(c, ns, nq_out, n_polys, rows_done && cols_only)) && lazy_dot_ok(c) &&
         launch_moddown_slab(c, y, (size_t)E * N, a.src_slot, a.src_prime, ns,
                             t->dev + (drop_last ? t->drop_invn_off[nq] : t->p_invn_off),
                             t->dot + (drop_last ? t->drop_hat_off[nq] : t->p_hat_off), c->nQ + c->nP, conv, nq_out, n_polys,

@@ -841,27 +841,67 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
     return true;
 }
 
+// primes of 44 bits and more that are not just below 2^60 (IntFieldT), whose butterflies take the most instructions
+static bool has_far_primes(const hemm_context *c) {
+    for (const u64 q : c->primes)
+        if ((q >> 44) != 0 && !near_2_60(q)) return true;
+    return false;
+}
+// The polynomials of a ModDown that go through its launches together: as many as have limbs that the memory-side cache holds between the
+// launches, as in polys_per_run, or the whole rounds of the slab kernel (sixteen polynomials) in that where the kernel has fewer rounds then.  48 polynomials
+// of 5 -> 10 limbs, cut 44 + 4 / 32 + 16: 396/359 us of 42 bits, 468/428 of 50, 429/395 of 60.
+static int slab_run(int n_src, int nq_out, int n_polys) {
+    const int fit = std::max(1, 448 / std::max(n_src, nq_out)), whole = fit - fit % 16;
+    auto rounds = [&](int run) { return n_polys / run * ((run + 15) / 16) + (n_polys % run + 15) / 16; };
+    if (n_polys <= fit) return n_polys;
+    return whole != 0 && rounds(whole) < rounds(fit) ? whole : fit;
+}
 // The slab kernel saves two trips of every source limb and a launch, and keeps few workgroups, 32 per polynomial of which 512 are
-// resident, busy for as long as there are targets.  Whole ModDowns in four launches / with it, us (sources -> targets; primes of 42 bits in the
-// chain, then 60):
-//   polynomials      4            6            8            12           16             20             32             64
-//   42 bits   5->3   35.7/ 34.2   43.3/ 39.2   49.0/ 44.3   65.0/ 60.6    76.6/ 68.6     89.7/ 86.6    126/118        268/241
-//             5->7   42.4/ 46.9   54.3/ 53.5   63.5/ 59.1   84.2/ 82.6   102.3/ 95.2    123.7/122.7    194/186        410/383
-//             4->8   41.4/ 48.0   52.1/ 53.5   64.1/ 61.1   81.2/ 82.5    99.4/ 95.0    120.7/124.1    193/188        398/408
-//             2->5   29.9/ 30.6   38.0/ 36.5   42.9/ 41.4   55.3/ 52.0    68.3/ 60.2     79.7/ 73.3    109/102        216/205
-//             5->12  51.9/ 63.0   69.4/ 73.1   82.0/ 82.1  109.3/112.6   142.6/133.4    173.8/180.5    283/281        586/592
-//   60 bits   5->7   44.0/ 51.6   57.2/ 59.2   66.9/ 64.8   89.2/ 89.5   106.2/100.4    132.0/132.4    202/196        426/399
-//             3->6   36.2/ 42.6   46.2/ 48.8   52.7/ 53.4   74.9/ 70.5    82.7/ 79.0     99.3/ 96.9    147/139        299/286
-//             5->12  54.7/ 72.2   74.8/ 84.5   86.9/ 92.8  115.2/122.1   149.9/145.5    185.6/197.7    299/297        612/626
-//             4->20  68.3/100     91.0/111      112/124      161/174       212/218                     439/491        874/975
-// So: eight polynomials and more and up to three targets more than sources; up to twelve where the workgroups are one nearly full round, and with
-// five sources from 28 polynomials on, which alone is even and in an attention block, beside another chain, 1.3 % of it.
-// Product of two encrypted matrices 2017 -> 1987 us, plaintext product 468 -> 456, projection of a 768-wide layer 9555 -> 9280, attention
-// block 19708 -> 19392.
-bool takes_moddown_slab(const hemm_context *c, int n_src, int nq_out, int n_polys) {
-    if (c->logN != 16 || n_src < 2 || n_src > SLAB_MAX_SOURCES) return false;
-    if (nq_out <= n_src + 3) return n_polys >= 8;
-    return nq_out <= 12 && ((n_polys > 12 && n_polys <= 16) || (n_src == 5 && n_polys >= 28));
+// resident, busy for as long as there are targets: it leads by 2 - 10 % where its last round of sixteen polynomials is full, three quarters full or half
+// full (a workgroup on every CU), and loses where that round has few more than none or than half.  Whole ModDowns in four launches / with it, us, one build
+// with the line moved (sources -> targets; 42 bits in the chain; 50; 60):
+//   polynomials            8              10              12              18              20              24              40              64             100
+//   2->5  42 bits   41.1/ 38.8      47.8/ 46.7      52.4/ 48.8      70.6/ 64.9      76.0/ 68.4      84.3/ 75.5       127/119         211/201         334/330
+//   3->6  42 bits   49.3/ 45.9      58.4/ 57.1      67.4/ 61.8      85.3/ 83.3      90.7/ 86.9       104/ 95         169/156         281/266         450/417
+//         50 bits   60.3/ 59.9      71.0/ 74.2      83.8/ 79.3       105/105         114/111         129/120         207/196         330/320         520/501
+//   4->7  42 bits   58.3/ 53.2      68.3/ 67.1      74.9/ 72.1       100/102         108/107         128/121         213/203         371/355         580/540
+//         50 bits   69.9/ 67.8      82.9/ 85.7      91.9/ 92.3       124/133         133/138         156/152         255/248         417/407         648/637
+//   5->8  42 bits   66.8/ 61.9      77.2/ 79.7      86.1/ 85.2       120/120         129/126         156/145         266/255         444/415         747/669
+//         50 bits   80.7/ 80.0      94.6/101        106/108          143/154         157/161         185/181         309/302         493/488         812/784
+//         60 bits   73.8/ 71.9      85.3/ 87.5      95.7/ 94.2       132/137         143/143         171/165         286/279         469/449         782/723
+// and with more targets:
+//   polynomials           13              14              16              20              28              32              48              64             128
+//   2->12 50 bits    116/114         122/118         135/128
+//   3->12 50 bits    125/125         133/130         145/140
+//   4->12 50 bits    133/134         140/138         156/152
+//   5->9  42 bits    100/ 95         104/ 98         118/105         144/138         198/193         231/221         358/336         482/446        1029/888
+//   5->12 42 bits    118/112         123/116         139/127         174/175         246/245         287/280         439/410         599/549        1243/1103
+//         50 bits    144/144         150/148         168/159         209/219         295/297         333/327         494/492         663/644        1354/1292
+//         60 bits    129/126         136/131         153/143         190/196         270/272         306/299         465/454         628/598        1295/1196
+//   polynomials           26              28              34              36              50              68
+//   4->7  60 bits    151/150         162/159         197/201         209/210         295/300         398/415
+//         50 bits    165/169         177/175         214/218         227/227         318/323         429/450
+//   5->8  42 bits    164/165         177/175         218/218         234/231         332/332         468/448
+//         60 bits    182/186         195/196         237/242         252/252         353/356         492/489
+//         50 bits    196/206         212/216         256/265         272/275         378/384         518/528
+// The line lies where nothing in these tables loses more than 3 %, but for 68 polynomials, which are cut 64 + 4 either way (calls of one process differ by as
+// much from another's where neither form leads clearly, at 26 and 34 polynomials for instance).  uncut: never in runs.
+bool takes_moddown_slab(const hemm_context *c, int n_src, int nq_out, int n_polys, bool uncut) {
+    if (c->logN != 16 || n_src < 2 || n_src > SLAB_MAX_SOURCES || n_polys < 8) return false;
+    const bool far = has_far_primes(c);
+    const int run = uncut ? n_polys : slab_run(n_src, nq_out, n_polys), last = n_polys % 16;   // polynomials of the last round, 0: a full one
+    if (nq_out <= n_src + 3) {
+        if (n_src == 2) return n_polys != 9;
+        if (n_src == 3) return n_polys == 8 || n_polys >= 12 || !far;
+        if (last == 0 || last == 8 || last >= 13 || n_polys > 96 || (run == n_polys && n_polys >= 48)) return true;
+        return !far && (n_polys == 12 || n_polys >= 20 || (n_src == 4 && n_polys <= 11 && n_polys >= 10));
+    }
+    if (nq_out > 12) return false;
+    if (n_polys <= 16) return n_polys >= 13;
+    if (n_src != 5 || n_polys < 28) return false;
+    if (far) return last == 0 || last >= 14 || (run == n_polys && (last == 8 || (last >= 12 && n_polys > 32)));
+    const int rest = (n_polys - 1) % run + 1;   // the last of the runs
+    return rest % 16 == 0 || rest % 16 >= 12 || (rest > 16 && rest % 16 == 8);
 }
 
 bool launch_moddown_slab(const hemm_context *c, u64 *y, size_t y_stride, const uint8_t *src_slot, const uint8_t *src_prime,
@@ -893,8 +933,7 @@ bool launch_moddown_slab(const hemm_context *c, u64 *y, size_t y_stride, const u
     account(c, TR_BCONV, (size_t)n_src * n_polys * c->N * 8, 0);
     account(c, TR_NTT, (size_t)(cols_only ? 1 : 2) * nq_out * n_polys * c->N * 8, cols_only ? 0 : 1);
     const size_t conv_stride = (size_t)nq_out << 16;
-    // runs whose limbs the memory-side cache holds between the launches, as in polys_per_run
-    const int run = rows_done && cols_only ? n_polys : std::max(1, 448 / std::max(n_src, nq_out));
+    const int run = rows_done && cols_only ? n_polys : slab_run(n_src, nq_out, n_polys);
     for (int p0 = 0; p0 < n_polys; p0 += run) {
         const int np = std::min(run, n_polys - p0);
         u64 *yp = y + (size_t)p0 * y_stride, *cp = conv + (size_t)p0 * conv_stride;

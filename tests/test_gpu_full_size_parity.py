@@ -590,8 +590,8 @@ def test_conversions_with_every_source_residue_at_q_minus_1(bench):
 
 def test_moddown_column_slab_form_same_residues(bench, chain24):
     """HEMM_MODDOWN_COLUMN_SLAB: the three-launch ModDown (inverse column pass, conversion and forward column pass in
-    one kernel per slab) against the four-launch chain and the oracle; 4 and 5 dropped limbs, a 42-bit and a 60-bit
-    last limb (the fifth source goes through LDS in either arithmetic)."""
+    one kernel per slab) against the four-launch chain, which calls of four polynomials take, and the oracle; 4 and 5 dropped limbs, a 42-bit
+    and a 60-bit last limb."""
     import torch
     rng = np.random.default_rng(78)
     for orc, ctx, nq, n_polys in ((bench.orc, bench.ctx, 7, 64), (bench.orc, bench.ctx, 13, 3), (chain24[0], chain24[1], 21, 2)):
@@ -600,5 +600,5 @@ def test_moddown_column_slab_form_same_residues(bench, chain24):
         y = rand_limbs(rng, ext_mods, (n_polys,), N)
         for drop in (True, False):
             slab = ctx.moddown_batch(dev(y), nq, drop, column_slab=True)
-            assert torch.equal(slab, ctx.moddown_batch(dev(y), nq, drop))
+            assert torch.equal(slab, torch.cat([ctx.moddown_batch(dev(part), nq, drop) for part in np.split(y, range(4, n_polys, 4))]))
             assert np.array_equal(host(slab[-2:]), orc.moddown_drop(y[-2:], nq, drop))

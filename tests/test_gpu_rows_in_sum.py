@@ -46,7 +46,8 @@ def test_rows_in_sum(log_n, chain, special, dnum, bits, n_out, terms, drop, comp
     give = [ctx.compact_key(k) for k in keys] if compact else keys
     groups = [[(ext[(o + t) % 2], b[t % 2], give[t % 2], mask if t % 3 == 1 else None, pow(5, 3 * o + t, 2 * N)) for t in range(terms)]
               for o in range(n_out)]
-    want = ctx.moddown_batch(ctx.hoisted_terms(groups, nq, compact_keys=compact), nq, drop)
+    # (two results at a time: in more launches than a larger batch on 2^16 points takes)
+    want = torch.cat([ctx.moddown_batch(y, nq, drop) for y in ctx.hoisted_terms(groups, nq, compact_keys=compact).split(2)])
     assert torch.equal(ctx.hoisted_moddown(groups, nq, drop, compact_keys=compact), want)
     # results apart from each other, 16 bytes and 8 bytes aligned
     for pad in (2, 1):
