@@ -561,12 +561,18 @@ static bool few_for_columns(const hemm_context *c, int limbs) { return (size_t)l
 //   42 bits                           26.3/25.8  33.3/32.5  37.4/36.6  41.3/40.4  269/269      | encodings of 72 / 117 / 208 limbs 45.0/44.0 57.3/55.5 84.1/82.5
 //   2^15 points, 960 / 1280 / 1920 / 2560: 60 bits 30.0/29.1 38.5/38.2 53.0/51.4 63.2/63.2, 42 bits 25.8/25.3 34.0/33.4 46.3/45.3 57.8/56.0
 //   2^14 points: ModDowns of 16 / 32 polynomials 39.0/39.4 53.4/54.0 (its line stays at 900)
-static int points_for_rows(const hemm_context *c, int limbs, bool inverse, int tail) {
-    const size_t wgs = (size_t)limbs * (c->N >> 12);
+//   other primes, 50 / 59 / 61 bits: 2^15 points, 1920 55.5/55.4 56.2/56.2 59.9/59.9, 2560 69.1/71.0 69.4/72.0 74.3/78.1; 2^16, 2400 69.0/68.8 70.1/70.5 76.5/77.5
+// primes of 44 bits and more that are not just below 2^60 (IntFieldT), whose butterflies take the most instructions
+static bool is_far(const u64 q) { return (q >> 44) != 0 && !near_2_60(q); }
+static int points_for_rows(const hemm_context *c, const LimbList &ll, int n_limbs, int n_polys, bool inverse, int tail) {
+    const size_t wgs = (size_t)n_limbs * n_polys * (c->N >> 12);
     const bool encoding = c->logN == 14 && !inverse && tail == TAIL_NONE;   // longer plain transforms of this ring are one launch
     if (wgs <= (encoding ? 512 : 640) || (tail == TAIL_ENCRYPT && c->logN < 16)) return 4;   // (an encryption's few limbs)
     if (inverse) return 8;
-    if (c->logN >= 15) return tail == TAIL_NONE && wgs > 2560 ? 16 : 8;
+    if (c->logN >= 15) {
+        if (tail != TAIL_NONE || wgs <= 1920) return 8;
+        return wgs > 2560 || std::any_of(ll.idx, ll.idx + n_limbs, [&](const uint8_t i) { return is_far(c->primes[i]); }) ? 16 : 8;
+    }
     return wgs <= (encoding ? 640 : 900) ? 8 : 16;
 }
 
@@ -657,7 +663,7 @@ static void cols_pass(const hemm_context *c, bool inverse, u64 *d, const LimbLis
 static void rows_pass(const hemm_context *c, bool inverse, u64 *d, const LimbList &ll, const LimbList &sl, int n_limbs,
                       int n_polys, size_t poly_stride, hipStream_t s, const NttEpilogue &ep, int tail = TAIL_NONE,
                       int load = LOAD_PLAIN, const ResultList *list = nullptr, int first = 0) {
-    const int points = points_for_rows(c, n_limbs * n_polys, inverse, tail);
+    const int points = points_for_rows(c, ll, n_limbs, n_polys, inverse, tail);
     const dim3 grid((unsigned)(c->N >> 8) / (unsigned)points * (unsigned)(n_limbs * n_polys)), block(256);
     const int log_r = c->logN - 8;
 #define ROWS(LR, P, INV, TAIL, LOAD, EP)                                                                                      \
@@ -841,10 +847,9 @@ bool launch_ntt_converted(const hemm_context *c, const ConvSources &cs, u64 *dat
     return true;
 }
 
-// primes of 44 bits and more that are not just below 2^60 (IntFieldT), whose butterflies take the most instructions
 static bool has_far_primes(const hemm_context *c) {
     for (const u64 q : c->primes)
-        if ((q >> 44) != 0 && !near_2_60(q)) return true;
+        if (is_far(q)) return true;
     return false;
 }
 // The polynomials of a ModDown that go through its launches together: as many as have limbs that the memory-side cache holds between the

@@ -52,6 +52,24 @@ def test_transforms(log_n, polys):
             assert np.array_equal(got, np.broadcast_to(want[i], got.shape)), (inverse, i)
 
 
+# (2^15 points: 240 limbs have eight points per thread in the row pass, 255 and 320 sixteen where a prime is not just below 2^60)
+@pytest.mark.parametrize("bits,mixed", [(50, False), (61, False), (60, True)])
+def test_large_batches(bits, mixed):
+    import torch
+    log_n, pkg = 15, load_package()
+    for polys, limbs in ((15, 16), (15, 17), (16, 20)):
+        qs = pkg.primes_below(bits, log_n, limbs)
+        if mixed:
+            qs[-1] = around_the_line(log_n)[1]
+        ctx = pkg.Context(log_n, qs, [], 1)
+        q = torch.tensor(qs, dtype=torch.int64, device="cuda").view(-1, 1)
+        gen = torch.Generator(device="cuda").manual_seed(limbs)
+        a = torch.randint(0, 1 << 62, (polys, limbs, 1 << log_n), dtype=torch.int64, device="cuda", generator=gen).remainder_(q)
+        a[0] = q - 1
+        want = torch.cat([ctx.ntt(part.clone(), list(range(limbs))) for part in a.split(1)])   # four points: few limbs
+        assert torch.equal(ctx.ntt(a, list(range(limbs))), want), limbs
+
+
 @pytest.mark.parametrize("log_n", [10, 13, 16])
 @pytest.mark.parametrize("largest", [False, True])
 def test_key_switches_and_conversions(log_n, largest):
