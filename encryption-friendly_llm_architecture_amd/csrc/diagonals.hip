@@ -335,7 +335,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void d
         if (beta == 1) SUMS(true, 1, false);
         else if (beta == 2) SUMS(true, 2, false);
         else SUMS(true, 3, false);
-    } else if (near_2_60(m.q) && beta <= 2) {   // (with three digits it would spill)
+    } else if (near_2_60(m.q) && beta <= 2) {   // (with three digits it would spill more)
         if (beta == 1) SUMS(false, 1, true);
         else SUMS(false, 2, true);
     } else {

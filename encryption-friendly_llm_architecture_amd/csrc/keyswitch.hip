@@ -544,7 +544,8 @@ __device__ __forceinline__ void hoisted_terms_body(const RotTermDev *__restrict_
 }
 
 // Register budget for five waves per SIMD (96 registers): the double-precision form needs 72, the integer and the mixed form
-// all 96.  The mixed form under a ModDown's tail spills three; with four waves and none a product at level 9 takes 122.1 instead of
+// all 96; the integer form spills eight (four before it had the sums of primes just below 2^60; 32 and 48 outputs of two masked sources take 230 and 513 us
+// either way).  Four waves were slower even when the mixed form spilled three under a ModDown's tail: a product at level 9 122.1 instead of
 // 120.2 us, the projection of a 768-wide layer 10.46 instead of 10.33 ms.  COMPACT: the key layout of the launch (hoisted.h, key_limb).
 #define HOISTED_KERNEL __global__ __launch_bounds__(256 * S) __attribute__((amdgpu_waves_per_eu(S == 4 ? 4 : 5))) void
 template <int MODE, bool COMPACT, int S, class ROWS>

@@ -77,7 +77,7 @@ __device__ __forceinline__ u64 sub_multiple(u64 v, u32 e, u64 q) {
 }
 // ---- primes just below 2^60: q = 2^60 - delta, delta < 2^27 ------------------------------------------------------------------
 // What lies above bit 60 of a value counts delta times, so no quotient is estimated.  A constant w is kept with v = 2^32 w mod q, both cut at
-// bit 29 (near60_constant), and y w for a 64-bit y is yl w + yh v: four multiply-adds into accumulators s0 and s1 of weights 1 and 2^29.
+// bit 29 (near60_cut in context.hip, Near60::cut), and y w for a 64-bit y is yl w + yh v: four multiply-adds into accumulators s0 and s1 of weights 1 and 2^29.
 // 2^29 s1 is 2^29 times its low word plus 2^61 = 2 delta times its high word, two multiply-adds more; y is never cut into pieces.
 #define NEAR60_DELTA (1ull << 27)
 __host__ __device__ __forceinline__ bool near_2_60(const u64 q) { return q < (1ull << 60) && (1ull << 60) - q < NEAR60_DELTA; }

@@ -300,7 +300,7 @@ struct SlabSources {
     size_t src_poly_stride;
     const Cst *hat;            // [n_src][hat_ld]  (S/q_i) mod prime and 2^30 times that, indexed by prime
     const Tw *final_scale;     // [n_src]  (1/N)(S/q_i)^-1 mod q_i
-    int hat_ld, n_src, n_dst;  // targets: chain primes 0 .. n_dst - 1, in the slots of these numbers
+    int hat_ld, n_dst;         // targets: chain primes 0 .. n_dst - 1, in the slots of these numbers
     uint8_t src_slot[8], src_prime[8];   // SLAB_MAX_SOURCES of them, whole words (table_byte)
 };
 
@@ -604,7 +604,8 @@ static bool few_for_conversions(const hemm_context *c, int limbs) { return (size
 //   limbs         1                             4                             16                            32                              48                                64
 //   2^13 points   7.5/6.8/6.6  7.8/6.9/6.7   7.8/7.0/6.7  8.1/7.1/6.7   8.1/7.4/7.2  8.5/7.5/7.3    8.9/ 8.3/ 7.9  9.2/ 8.5/ 8.0   10.2/ 9.8/ 9.5 10.8/10.1/ 9.7   (one launch)
 //   2^14          7.6/6.9/6.6  8.0/7.2/6.7   7.9/7.1/6.8  8.2/7.3/6.8   9.2/8.2/7.9  9.6/8.4/8.0   11.6/10.5/10.4 12.3/10.9/10.8   14.5/13.2/13.1 15.2/13.9/13.5   17.5/15.7/15.7 19.3/16.3/16.4
-//   (35 / 80 limbs 12.6/11.7/11.5 13.2/12.3/12.0, 20.2/18.6/18.2 22.2/19.5/18.9: the line of quarter slabs, drawn with eight points, lies below its place)
+//   (35 / 80 limbs 12.6/11.7/11.5 13.2/12.3/12.0, 20.2/18.6/18.2 22.2/19.5/18.9: the line of quarter slabs, drawn with eight points, lies below its place
+//   and has not been moved)
 // Transforms of 2^15 points, whole slabs of sixteen / of four points / half slabs of four:
 //   limbs      1                               16                                 32                                 40                                 48                                 64
 //   42 bits    7.9/7.7/7.0   8.3/8.2/7.3   11.3/11.1/10.5 11.9/11.8/11.0   16.6/16.0/15.9 17.1/16.7/16.5   19.7/19.5/18.9 20.3/20.5/19.6   22.0/21.8/21.1 22.5/22.6/22.0   25.7/25.4/25.1 26.7/26.4/26.4
@@ -930,7 +931,6 @@ bool launch_moddown_slab(const hemm_context *c, u64 *y, size_t y_stride, const u
     ss.hat = (const Cst *)hat_dev;
     ss.final_scale = (const Tw *)final_scale_dev;
     ss.hat_ld = hat_ld;
-    ss.n_src = n_src;
     ss.n_dst = nq_out;
     // same algorithmic bytes as the separate launches: the dropped limbs in and out of the inverse transform, the
     // conversion's sources, the minuend in and the result out of the forward transform

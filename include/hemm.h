@@ -274,7 +274,7 @@ int hemm_hoisted_moddown_to(hemm_context *ctx, const hemm_rot_term *terms, const
  * drop_last | HEMM_MODDOWN_COLUMN_SLAB (N = 2^16, 4 or 5 dropped limbs, primes below 2^60) runs the same arithmetic
  * in three launches instead of four: the second pass of the inverse transform, the basis conversion and the first
  * pass of the forward transform in one kernel per slab of columns, so the dropped limbs are not written in
- * coefficient form and read back (identical residues).  Batches for which it is the faster form take it by themselves. */
+ * coefficient form and read back (identical residues).  Batches for which it is the faster form, with two or three dropped limbs too, take it by themselves. */
 #define HEMM_MODDOWN_COLUMN_SLAB 2
 int hemm_moddown_batch(hemm_context *ctx, uint64_t *y, uint32_t nq, uint32_t n_polys, int drop_last,
                        uint64_t *out, size_t out_stride, uint64_t *workspace, void *stream);

@@ -22,7 +22,7 @@ def _scratch():
 
 
 def test_scratch():
-    """Registers spill in the kernels where fewer wavefronts were measured to cost more than that, and in no other."""
+    """Registers spill in the sums whose launch bounds ask for more wavefronts than their registers allow, and in no other kernel."""
     scratch = _scratch()
     assert len(scratch) > 300
     may = re.compile("diagonal_sums_kernelI|hoisted_terms_(list_)?kernelILi2E")
