@@ -386,8 +386,8 @@ struct StagePairs {
         : dist(!split ? d : P == 4 ? d / 4 : 4), first_group(!split ? h * (u32)(P / 2 / d) : 0u) {}
 };
 // The lane of a block of stages.  KeptLane: a number that the caller has; the stages are then simplified before its bits are known.  OwnLane: made
-// where the stages begin.  Inverse transforms take the second, 72 registers instead of 78 in the row pass of 2^16 points and 64 instead of 72 where
-// a limb is one launch (32 x 24 limbs of 2^13 points 28.3 -> 25.3 us, of 60 bits 34.5 -> 31.5), and so do conversions, of which eight sources on
+// where the stages begin.  Inverse transforms take the second, 72 registers and 484 instructions instead of 78 and 452 in the row pass of 2^16 points
+// (even) and 64 registers instead of 72 where a limb is one launch (32 x 24 limbs of 2^13 points 28.3 -> 25.3 us, of 60 bits 34.5 -> 31.5), and so do conversions, of which eight sources on
 // 2^15 points spill 20 registers with the first.  The other forward transforms take the first (the same limbs 24.0 -> 23.1).
 struct KeptLane {
     u32 h;
