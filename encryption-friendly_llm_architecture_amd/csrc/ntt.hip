@@ -872,9 +872,9 @@ static int slab_run(int n_src, int nq_out, int n_polys) {
 //         50 bits   60.3/ 59.9      71.0/ 74.2      83.8/ 79.3       105/105         114/111         129/120         207/196         330/320         520/501
 //   4->7  42 bits   58.3/ 53.2      68.3/ 67.1      74.9/ 72.1       100/102         108/107         128/121         213/203         371/355         580/540
 //         50 bits   69.9/ 67.8      82.9/ 85.7      91.9/ 92.3       124/133         133/138         156/152         255/248         417/407         648/637
-//   5->8  42 bits   66.8/ 61.9      77.2/ 79.7      86.1/ 85.2       120/120         129/126         156/145         266/255         444/415         747/669
-//         50 bits   80.7/ 80.0      94.6/101        106/108          143/154         157/161         185/181         309/302         493/488         812/784
-//         60 bits   73.8/ 71.9      85.3/ 87.5      95.7/ 94.2       132/137         143/143         171/165         286/279         469/449         782/723
+//   5->8  42 bits   66.8/ 61.9      77.2/ 79.7      86.1/ 85.2       120/120         129/126         156/145         266/255         444/415         743/649
+//         50 bits   80.7/ 80.0      94.6/101        106/108          143/154         157/161         185/181         309/302         493/488         804/753
+//         60 bits   73.8/ 71.9      85.3/ 87.5      95.7/ 94.2       132/137         143/143         171/165         286/279         469/449         778/693
 // and with more targets:
 //   polynomials           13              14              16              20              28              32              48              64             128
 //   2->12 50 bits    116/114         122/118         135/128
